@@ -123,6 +123,9 @@ struct sgh_prof_kernel_scope {
       hipLaunchKernelGGL(kern, grid, block, lds, stream, __VA_ARGS__);                                           \
   } while (0)
 
+// Bias gradient (bgrad.hip); dtype 0 fp32, 1 binary16, 2 bfloat16.
+int sgh_conv_bgrad_run(const sgh_conv_geom *g, const void *dy, void *db, int dtype, hipStream_t s);
+
 // 3x3 (stride 1 or 2) weight gradient with a shared LDS input tile (wgrad3x3.hip).  *_run returns
 // SGH_EUNSUPPORTED for geometries it does not cover; *_workspace_bytes is 0 for those.
 size_t sgh_wgrad3x3_workspace_bytes(const sgh_conv_geom *g);

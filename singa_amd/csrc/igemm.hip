@@ -25,7 +25,6 @@
 #include <stdlib.h>
 
 #include "common.h"
-#include "storage.h"
 
 namespace {
 
@@ -677,22 +676,6 @@ __global__ __launch_bounds__(NT) void k_col2im_gather(const float *__restrict__ 
   }
 }
 
-// One thread per (k), summing dy over n, p, q is too serial; use one workgroup per k.
-template <class S>
-__global__ __launch_bounds__(NT) void k_conv_bgrad(const typename S::elem *__restrict__ dy,
-                                                  typename S::elem *__restrict__ db, int N, int K, int PQ) {
-  __shared__ float red[16];
-  const int k = blockIdx.x;
-  float s = 0.f;
-  const int total = N * PQ;
-  for (int i = threadIdx.x; i < total; i += NT) {
-    const int n = i / PQ, r = i - n * PQ;
-    s += S::ld(dy + (long(n) * K + k) * PQ + r);
-  }
-  s = sgh_block_sum(s, red);
-  if (threadIdx.x == 0) S::st(db + k, s);
-}
-
 inline int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
 inline ConvG to_g(const sgh_conv_geom *g) {
@@ -958,7 +941,7 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
 // [K, C/G, R, S] weight tensor.  Each group runs as a dense convolution of its own: its channel slices are
 // gathered into dense tensors in the workspace (strided device-to-device copies, one row per image), the
 // ordinary entry point runs on the sub-geometry, and the result is scattered back; a group's weight gradient
-// is a dense block of dW and needs no copy.  Workspace: [x slice | y slice | workspace of the sub-geometry].
+// is a dense block of dW and needs no copy.   Workspace: [x slice | y slice | workspace of the sub-geometry].
 namespace {
 
 struct GroupPlan {
@@ -1514,9 +1497,7 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
 }
 
 static int bgrad_launch(const sgh_conv_geom *g, const float *dy, float *db, hipStream_t s) {
-  hipLaunchKernelGGL(k_conv_bgrad<StF32>, dim3(g->K), dim3(NT), 0, s, dy, db, g->N, g->K, g->P * g->Q);
-  SGH_LAUNCH_CHECK();
-  return SGH_OK;
+  return sgh_conv_bgrad_run(g, dy, db, 0, s);
 }
 
 // `db` (may be null): the bias gradient as well.  In the generic kernel it rides along as one more column
@@ -1614,10 +1595,7 @@ int sgh_conv_wgrad_bias_f32(sgh_conv_geom *g, const float *dy, const float *x, f
 
 int sgh_conv_bgrad_f32(const sgh_conv_geom *g, const float *dy, float *db, void *stream) {
   if (!conv_ok(g) || !dy || !db) return SGH_EINVAL;
-  hipLaunchKernelGGL(k_conv_bgrad<StF32>, dim3(g->K), dim3(NT), 0, sgh_stream_of(stream), dy, db, g->N, g->K,
-                     g->P * g->Q);
-  SGH_LAUNCH_CHECK();
-  return SGH_OK;
+  return sgh_conv_bgrad_run(g, dy, db, 0, sgh_stream_of(stream));
 }
 
 int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B,
@@ -1744,17 +1722,11 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
 
 int sgh_conv_bgrad_f16(const sgh_conv_geom *g, const uint16_t *dy, uint16_t *db, void *stream) {
   if (!conv_ok(g) || !dy || !db) return SGH_EINVAL;
-  hipLaunchKernelGGL(k_conv_bgrad<StF16>, dim3(g->K), dim3(NT), 0, sgh_stream_of(stream), dy, db, g->N, g->K,
-                     g->P * g->Q);
-  SGH_LAUNCH_CHECK();
-  return SGH_OK;
+  return sgh_conv_bgrad_run(g, dy, db, 1, sgh_stream_of(stream));
 }
 int sgh_conv_bgrad_bf16(const sgh_conv_geom *g, const uint16_t *dy, uint16_t *db, void *stream) {
   if (!conv_ok(g) || !dy || !db) return SGH_EINVAL;
-  hipLaunchKernelGGL(k_conv_bgrad<StBF16>, dim3(g->K), dim3(NT), 0, sgh_stream_of(stream), dy, db, g->N, g->K,
-                     g->P * g->Q);
-  SGH_LAUNCH_CHECK();
-  return SGH_OK;
+  return sgh_conv_bgrad_run(g, dy, db, 2, sgh_stream_of(stream));
 }
 
 size_t sgh_conv_workspace_bytes_h(const sgh_conv_geom *g, int which) {

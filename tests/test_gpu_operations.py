@@ -725,3 +725,32 @@ def _shared_tile_cases(count, seed):
 @pytest.mark.parametrize("case", _shared_tile_cases(40, 777))
 def test_conv_shared_tile_sweep(singa, dev, case):
     test_conv_backward_vs_oracle(singa, dev, case)
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("shape", [
+    (64, 3, 56, 56),     # whole pieces, many images per step of the workgroup's walk
+    (5, 2, 111, 97),     # more pieces than threads in a plane, the last one partial
+    (300, 7, 5, 3),      # planes of two (fp32: four) pieces, the last one partial
+    (2000, 2, 1, 3),     # planes shorter than a piece
+    (1, 3, 2, 4),        # fewer pieces than threads
+    (3, 2, 96, 128),     # pieces an exact multiple of the workgroup
+])
+def test_conv_bias_gradient_vs_float64(singa, dev, kind, shape):
+    """The bias gradient's piece walk (planes shorter than, equal to and not a multiple of a piece).  Bound: every partial sum of
+    the tree is at most the sum of |dy|, at most 40 roundings of 2^-24 deep, plus one rounding of the storage type."""
+    print("bias gradient", kind, shape, flush=True)
+    N, K, P, Q = shape
+    r = rng(sum(shape))
+    dt = {"f32": singa.kFloat32, "f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+    t = singa.from_numpy(randn(r, *shape), dev)
+    t = t if kind == "f32" else t.AsType(dt)
+    dy = (t if kind == "f32" else t.AsType(singa.kFloat32)).to_numpy().astype(np.float64)
+    x = singa.Tensor((N, 1, P, Q), dev, dt)
+    h = singa.CudnnConvHandle(x, (1, 1), (1, 1), (0, 0), 1, K, True)
+    b = singa.Tensor((K,), dev, dt)
+    db = singa.GpuConvBackwardb(t, b, h)
+    got = (db if kind == "f32" else db.AsType(singa.kFloat32)).to_numpy().astype(np.float64)
+    want, mass = dy.sum(axis=(0, 2, 3)), np.abs(dy).sum(axis=(0, 2, 3))
+    ulp = {"f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[kind]
+    assert np.all(np.abs(got - want) <= 40 * 2.0 ** -24 * mass + ulp * np.abs(want))
