@@ -123,6 +123,13 @@ struct sgh_prof_kernel_scope {
       hipLaunchKernelGGL(kern, grid, block, lds, stream, __VA_ARGS__);                                           \
   } while (0)
 
+// Grouped convolutions with few channels per group (group_conv.hip), all three passes and types (dtype 0 fp32, 1 binary16,
+// 2 bfloat16): (a, b, out) = (x, W, y), (dy, W, dx), (dy, x, dW).  SGH_EUNSUPPORTED for every other geometry.
+bool sgh_group_conv_supported(const sgh_conv_geom *g, int which);
+size_t sgh_group_conv_workspace_bytes(const sgh_conv_geom *g, int which);
+int sgh_group_conv_run(const sgh_conv_geom *g, int which, int dtype, const void *a, const void *b, const void *bias, void *out,
+                       void *workspace, size_t ws_bytes, hipStream_t s);
+
 // Bias gradient (bgrad.hip); dtype 0 fp32, 1 binary16, 2 bfloat16.
 int sgh_conv_bgrad_run(const sgh_conv_geom *g, const void *dy, void *db, int dtype, hipStream_t s);
 

@@ -941,7 +941,8 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
 // [K, C/G, R, S] weight tensor.  Each group runs as a dense convolution of its own: its channel slices are
 // gathered into dense tensors in the workspace (strided device-to-device copies, one row per image), the
 // ordinary entry point runs on the sub-geometry, and the result is scattered back; a group's weight gradient
-// is a dense block of dW and needs no copy.   Workspace: [x slice | y slice | workspace of the sub-geometry].
+// is a dense block of dW and needs no copy.  Groups of few channels have kernels of their own (group_conv.hip).
+// Workspace: [x slice | y slice | workspace of the sub-geometry].
 namespace {
 
 struct GroupPlan {
@@ -1050,6 +1051,9 @@ int conv_dense_f32(sgh_conv_geom *sg, int which, const float *a, const float *b,
 
 int conv_grouped_f32(const sgh_conv_geom *g, int which, const float *a, const float *b, const float *bias, float *out,
                      void *workspace, size_t ws_bytes, void *stream) {
+  if (!a || !b || !out) return SGH_EINVAL;
+  const int rc = sgh_group_conv_run(g, which, 0, a, b, bias, out, workspace, ws_bytes, sgh_stream_of(stream));
+  if (rc != SGH_EUNSUPPORTED) return rc;
   GroupPlan p = group_plan(g, sizeof(float));
   const size_t sub_ws = sgh_conv_workspace_bytes(&p.sg, which);
   return conv_grouped<float>(g, which, a, b, bias, out, workspace, ws_bytes, sub_ws, sgh_stream_of(stream),
@@ -1065,6 +1069,7 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   if (!conv_ok(g)) return 0;
   if (g->groups > 1) {
     if (which < 0 || which > 2) return 0;
+    if (sgh_group_conv_supported(g, which)) return sgh_group_conv_workspace_bytes(g, which);
     const GroupPlan p = group_plan(g, sizeof(float));
     return p.x_bytes + p.y_bytes + sgh_conv_workspace_bytes(&p.sg, which);
   }
@@ -1658,6 +1663,9 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
               uint16_t *out, void *workspace, size_t ws_bytes, void *stream, cast_in_fn in, cast_out_fn outc) {
   if (!conv_ok(g) || !a || !b || !out) return SGH_EINVAL;
   if (g->groups > 1) {
+    const int rc = sgh_group_conv_run(g, which, in == sgh_cast_bf16_to_f32 ? 2 : 1, a, b, bias, out, workspace, ws_bytes,
+                                      sgh_stream_of(stream));
+    if (rc != SGH_EUNSUPPORTED) return rc;
     GroupPlan p = group_plan(g, sizeof(uint16_t));
     const size_t sub_ws = sgh_conv_workspace_bytes_h(&p.sg, which);
     return conv_grouped<uint16_t>(g, which, a, b, bias, out, workspace, ws_bytes, sub_ws, sgh_stream_of(stream),
@@ -1732,6 +1740,7 @@ int sgh_conv_bgrad_bf16(const sgh_conv_geom *g, const uint16_t *dy, uint16_t *db
 size_t sgh_conv_workspace_bytes_h(const sgh_conv_geom *g, int which) {
   if (!conv_ok(g) || which < 0 || which > 2) return 0;
   if (g->groups > 1) {
+    if (sgh_group_conv_supported(g, which)) return sgh_group_conv_workspace_bytes(g, which);
     const GroupPlan p = group_plan(g, sizeof(uint16_t));
     return p.x_bytes + p.y_bytes + sgh_conv_workspace_bytes_h(&p.sg, which);
   }

@@ -728,6 +728,45 @@ def test_conv_shared_tile_sweep(singa, dev, case):
 
 
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", [
+    (3, 8, 112, 112, 8, 3, 1, 1, 8),       # planes larger than a tile: several row tiles per plane
+    (37, 96, 7, 7, 96, 3, 1, 1, 96),       # planes smaller than a workgroup: many units per workgroup, the last one partial
+    (5, 12, 29, 31, 24, 3, 2, 1, 12),      # channel multiplier 2, stride 2 on odd planes (zeros between the rows of dy)
+    (2, 24, 19, 23, 16, 5, 2, 2, 8),       # 3 -> 2 channels per group, 5 x 5 stride 2
+    (9, 64, 14, 14, 64, 7, 1, 3, 8),       # the widest groups of these kernels: 8 -> 8, 7 x 7
+    (2, 72, 14, 9, 72, 3, 1, 1, 8),        # one channel per group more: one dense convolution per group
+    (4, 6, 9, 8, 12, 1, 1, 0, 6),          # 1 x 1
+    (2, 4, 10, 300, 4, 3, 1, 0, 4),        # rows wider than a workgroup, no padding
+])
+def test_narrow_groups_vs_oracle(singa, dev, kind, case):
+    """Grouped convolutions with at most eight channels per group (kernels of their own) against the per-group oracle at the
+    edges of their tiles: fp32 at the reduction bar, 16-bit tensors on the stored values."""
+    N, C, H, W, K, R, stride, pad, G = case
+    print("narrow groups", kind, case, flush=True)
+    r = rng(sum(case))
+    dt = {"f32": singa.kFloat32, "f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+    tol = TOL if kind == "f32" else 1e-2
+
+    def to(a):
+        t = singa.from_numpy(a.astype(np.float32), dev)
+        if kind != "f32":
+            t = t.AsType(dt)
+        return t, (t.AsType(singa.kFloat32) if kind != "f32" else t).to_numpy()
+    xt, x = to(randn(r, N, C, H, W))
+    wt, w = to(randn(r, K, C // G, R, R) * np.sqrt(2.0 * G / (C * R * R)))
+    bt, b = to(randn(r, K))
+    h = singa.CudnnConvHandle(xt, (R, R), (stride, stride), (pad, pad), C, K, True, G)
+    y_o = O.conv_fwd_grouped(x, w, b, (stride, stride), (pad, pad), G)
+    y = singa.GpuConvForward(xt, wt, bt, h)
+    dyt, dy = to(randn(r, *y_o.shape))
+    dx_o, dw_o = O.conv_bwd_grouped(dy, x, w, (stride, stride), (pad, pad), G)
+    dx = singa.GpuConvBackwardx(dyt, wt, xt, h)
+    dw = singa.GpuConvBackwardW(dyt, xt, wt, h)
+    assert nl2(y.to_numpy(), y_o) < tol and nl2(dx.to_numpy(), dx_o) < tol and nl2(dw.to_numpy(), dw_o) < tol
+    assert_bit_equal(singa.GpuConvBackwardW(dyt, xt, wt, h).to_numpy(), dw.to_numpy(), "dW again")
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("shape", [
     (64, 3, 56, 56),     # whole pieces, many images per step of the workgroup's walk
     (5, 2, 111, 97),     # more pieces than threads in a plane, the last one partial
