@@ -123,6 +123,11 @@ struct sgh_prof_kernel_scope {
       hipLaunchKernelGGL(kern, grid, block, lds, stream, __VA_ARGS__);                                           \
   } while (0)
 
+// fp32 GEMM with few output tiles, the reduction split over a workgroup's wavefronts (gemm_split.hip); arguments of
+// sgh_gemm_f32, checked by it, K > 0.  SGH_EUNSUPPORTED where the tiled kernel is the better one.
+int sgh_gemm_split_run(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+                       float beta, float *C, int ldc, hipStream_t s);
+
 // Grouped convolutions with few channels per group (group_conv.hip), all three passes and types (dtype 0 fp32, 1 binary16,
 // 2 bfloat16): (a, b, out) = (x, W, y), (dy, W, dx), (dy, x, dW).  SGH_EUNSUPPORTED for every other geometry.
 bool sgh_group_conv_supported(const sgh_conv_geom *g, int which);
