@@ -550,3 +550,30 @@ def test_int_float_casts(singa, dev):
     edge = np.array([3e9, -3e9, np.inf, -np.inf, np.nan], dtype=np.float32)
     got = singa.from_numpy(edge, dev).AsType(singa.kInt).to_numpy()
     assert got.tolist() == [2 ** 31 - 1, -2 ** 31, 2 ** 31 - 1, -2 ** 31, 0]
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 33, 7), (17, 15, 250), (33, 100, 257), (128, 10, 1031), (1, 300, 64),
+                                   (400, 333, 70), (415, 401, 255), (417, 349, 1033)])
+def test_gemm_split_reduction_edges(singa, dev, kind, M, N, K):
+    """Mult at the edges of the kernels that split the reduction over a workgroup's wavefronts: tiles of 16 and of 32 (from 128
+    tiles of 32 on), 4, 8 and 16 wavefronts, reductions that end inside a group or leave wavefronts without work, odd matrix
+    edges, all four transposes.  Bound: K products in fp32, |error| <= K 2^-24 sum |a b| (+ one rounding of the result)."""
+    print("gemm split", kind, M, N, K, flush=True)
+    r = rng(M + 3 * N + 7 * K)
+    dt = {"f32": singa.kFloat32, "f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+    ulp = {"f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[kind]
+
+    def to(a):
+        t = singa.from_numpy(a, dev)
+        t = t if kind == "f32" else t.AsType(dt)
+        return t, (t if kind == "f32" else t.AsType(singa.kFloat32)).to_numpy().astype(np.float64)
+    for tA in (False, True):
+        for tB in (False, True):
+            at, a = to(randn(r, K, M) if tA else randn(r, M, K))
+            bt, b = to(randn(r, N, K) if tB else randn(r, K, N))
+            a, b = (a.T if tA else a), (b.T if tB else b)
+            got = singa.Mult(at.T() if tA else at, bt.T() if tB else bt)
+            g = (got if kind == "f32" else got.AsType(singa.kFloat32)).to_numpy().astype(np.float64)
+            bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + ulp * np.abs(a @ b) + (1e-7 if kind == "f16" else 0.0)
+            assert np.all(np.abs(g - a @ b) <= bound), (tA, tB, float(np.max(np.abs(g - a @ b) - bound)))
