@@ -1,16 +1,19 @@
-"""Builds the gfx950 shared library (``singa_amd/lib/libsinga_hip.so``) with hipcc.
+"""Builds the gfx950 shared library (``singa_amd/lib/libsinga_hip.so``) with hipcc and the CPython extension that calls
+into it (``singa_amd/_native.so``) with the host compiler.
 
 Run as ``python -m singa_amd.build``.  The library is built in-tree; nothing is installed.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIBPATH = os.path.join(LIBDIR, "libsinga_hip.so")
+NATIVEPATH = os.path.join(HERE, "_native.so")
 
 SOURCES = ["runtime.hip", "eltwise.hip", "pool.hip", "batchnorm.hip", "igemm.hip", "wgrad3x3.hip", "conv16.hip",
     "wgrad_fewc.hip", "dgrad3x3.hip", "dgrad_fewc.hip", "half.hip", "tensor_fns.hip", "pointwise.hip", "fwd_fewc16.hip", "fwd_fewc.hip", "gemm16.hip", "bgrad.hip", "group_conv.hip", "gemm_split.hip"]
@@ -58,7 +61,19 @@ def build_library(verbose=True, jobs=4):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_native(verbose)
     return LIBPATH
+
+
+def build_native(verbose=True):
+    """The CPython extension on top of the library (host code only)."""
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-I", os.path.join(ROOT, "include"), "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "native.cc"),
+           "-o", NATIVEPATH, "-L", LIBDIR, "-lsinga_hip", "-Wl,-rpath,$ORIGIN/lib"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return NATIVEPATH
 
 
 def _drain(procs):

@@ -1,0 +1,380 @@
+// The host side of the singa_wrap mirror that every operation passes through, as a CPython extension
+// (singa_amd/_native.so): the memory block behind a tensor, the tensor's fields and accessors, and direct calls into the C ABI.
+//
+// A training step of a small network is bound by its host work: in Python with ctypes a Mult took 7 us around a launch of
+// 2.5 us (argument conversion 2.5, result tensor 2.5, shape checks 1.5).  Here a call converts its arguments from the ABI's
+// own prototypes at compile time, and a tensor is allocated in one call.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <tuple>
+#include <utility>
+
+#include "singa_hip.h"
+
+namespace {
+
+PyObject *g_check;   // singa_amd._lib.check(rc, what): raises the library's message
+PyObject *g_handle_name;
+
+bool failed(int rc, const char *what) {
+  if (rc == 0) return false;
+  PyObject *r = PyObject_CallFunction(g_check, "is", rc, what);
+  Py_XDECREF(r);
+  if (r) PyErr_SetString(PyExc_RuntimeError, what);   // (check always raises)
+  return true;
+}
+
+// ------------------------------------------------------------------------------------ direct calls
+
+template <class T>
+struct Arg;
+template <class T>
+struct Arg<T *> {
+  static T *from(PyObject *o) { return o == Py_None ? nullptr : static_cast<T *>(PyLong_AsVoidPtr(o)); }
+};
+template <>
+struct Arg<int> {
+  static int from(PyObject *o) {
+    const long v = PyLong_AsLong(o);
+    if (v != long(int(v))) PyErr_SetString(PyExc_OverflowError, "argument does not fit an int");
+    return int(v);
+  }
+};
+template <>
+struct Arg<size_t> {
+  static size_t from(PyObject *o) { return PyLong_AsSize_t(o); }
+};
+template <>
+struct Arg<float> {
+  static float from(PyObject *o) { return float(PyFloat_AsDouble(o)); }
+};
+
+template <auto F>
+struct Call;
+template <class... A, int (*F)(A...)>
+struct Call<F> {
+  template <size_t... I>
+  static PyObject *with(PyObject *const *args, std::integer_sequence<size_t, I...>) {
+    const std::tuple<A...> a{Arg<A>::from(args[I])...};
+    if (PyErr_Occurred()) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = F(std::get<I>(a)...);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(rc);
+  }
+  static PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != Py_ssize_t(sizeof...(A))) {
+      PyErr_Format(PyExc_TypeError, "%zd arguments given, %zd expected", n, Py_ssize_t(sizeof...(A)));
+      return nullptr;
+    }
+    return with(args, std::make_integer_sequence<size_t, sizeof...(A)>());
+  }
+};
+
+// ------------------------------------------------------------------------------------ Block
+
+struct Block {
+  PyObject_HEAD
+  PyObject *dev, *keepalive, *address;
+  sgh_device *handle;
+  void *ptr;
+  Py_ssize_t nbytes;
+  char owned;
+};
+extern PyTypeObject BlockType;
+
+// A block of the device's pool (ptr null), or around memory that someone else owns
+Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, void *ptr, PyObject *keepalive) {
+  sgh_device *h = nullptr;
+  if (!ptr) {
+    PyObject *ho = PyObject_GetAttr(dev, g_handle_name);
+    if (!ho) return nullptr;
+    h = static_cast<sgh_device *>(PyLong_AsVoidPtr(ho));
+    Py_DECREF(ho);
+    if (PyErr_Occurred()) return nullptr;
+    if (failed(sgh_malloc(h, &ptr, nbytes > 0 ? size_t(nbytes) : 1), "sgh_malloc")) return nullptr;
+  }
+  Block *b = reinterpret_cast<Block *>(type->tp_alloc(type, 0));
+  if (!b) {
+    if (h) sgh_free(h, ptr);
+    return nullptr;
+  }
+  b->handle = h, b->ptr = ptr, b->nbytes = nbytes, b->owned = h != nullptr;
+  Py_INCREF(dev);
+  b->dev = dev;
+  Py_XINCREF(keepalive);
+  b->keepalive = keepalive;
+  b->address = PyLong_FromVoidPtr(ptr);
+  return b;
+}
+
+PyObject *block_tp_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
+  static const char *names[] = {"dev", "nbytes", "ptr", "keepalive", nullptr};
+  PyObject *dev, *ptr = Py_None, *keepalive = nullptr;
+  Py_ssize_t nbytes;
+  if (!PyArg_ParseTupleAndKeywords(args, kw, "On|OO", const_cast<char **>(names), &dev, &nbytes, &ptr, &keepalive)) return nullptr;
+  void *p = ptr == Py_None ? nullptr : PyLong_AsVoidPtr(ptr);
+  if (PyErr_Occurred()) return nullptr;
+  return reinterpret_cast<PyObject *>(block_new(type, dev, nbytes, p, keepalive));
+}
+
+void block_dealloc(PyObject *self) {
+  Block *b = reinterpret_cast<Block *>(self);
+  if (b->owned && b->ptr) sgh_free(b->handle, b->ptr);
+  Py_XDECREF(b->dev);
+  Py_XDECREF(b->keepalive);
+  Py_XDECREF(b->address);
+  Py_TYPE(self)->tp_free(self);
+}
+
+PyMemberDef block_members[] = {
+    {"dev", T_OBJECT, offsetof(Block, dev), READONLY, "device"},
+    {"keepalive", T_OBJECT, offsetof(Block, keepalive), READONLY, "owner of memory that is not the pool's"},
+    {"ptr", T_OBJECT, offsetof(Block, address), READONLY, "device address"},
+    {"nbytes", T_PYSSIZET, offsetof(Block, nbytes), READONLY, "size"},
+    {"owned", T_BOOL, offsetof(Block, owned), READONLY, "whether the memory goes back to the pool"},
+    {nullptr, 0, 0, 0, nullptr}};
+
+PyTypeObject BlockType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ------------------------------------------------------------------------------------ Tensor
+
+struct Tensor {
+  PyObject_HEAD
+  PyObject *shape, *dev, *block;
+  int dtype;
+  char transposed;
+};
+extern PyTypeObject TensorType;
+
+inline Tensor *as_tensor(PyObject *o) { return reinterpret_cast<Tensor *>(o); }
+
+// product of the extents, -1 with an exception set when `shape` is not a tuple of whole numbers
+Py_ssize_t count_of(PyObject *shape) {
+  if (!shape || !PyTuple_Check(shape)) {
+    PyErr_SetString(PyExc_TypeError, "a tensor's shape is a tuple");
+    return -1;
+  }
+  Py_ssize_t n = 1;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(shape); ++i) {
+    n *= PyLong_AsSsize_t(PyTuple_GET_ITEM(shape, i));
+    if (PyErr_Occurred()) return -1;
+  }
+  return n;
+}
+
+inline Py_ssize_t elem_size(int dtype) { return dtype == 1 || dtype == 100 ? 2 : 4; }   // kFloat16, kBFloat16; kFloat32, kInt
+
+// a dense tensor of the pool
+PyObject *tensor_make(PyTypeObject *type, PyObject *shape, PyObject *dev, int dtype) {
+  const Py_ssize_t n = count_of(shape);
+  if (n < 0 && PyErr_Occurred()) return nullptr;
+  Block *b = block_new(&BlockType, dev, n * elem_size(dtype), nullptr, nullptr);
+  if (!b) return nullptr;
+  PyObject *o = type->tp_alloc(type, 0);
+  if (!o) {
+    Py_DECREF(b);
+    return nullptr;
+  }
+  Tensor *t = as_tensor(o);
+  Py_INCREF(shape);
+  t->shape = shape;
+  Py_INCREF(dev);
+  t->dev = dev;
+  t->block = reinterpret_cast<PyObject *>(b);
+  t->dtype = dtype, t->transposed = 0;
+  return o;
+}
+
+PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {   // empty(cls, shape, device, dtype)
+  if (n != 4 || !PyType_Check(args[0]) || !PyType_IsSubtype(reinterpret_cast<PyTypeObject *>(args[0]), &TensorType)) {
+    PyErr_SetString(PyExc_TypeError, "empty(cls, shape, device, dtype)");
+    return nullptr;
+  }
+  const long dtype = PyLong_AsLong(args[3]);
+  if (PyErr_Occurred()) return nullptr;
+  return tensor_make(reinterpret_cast<PyTypeObject *>(args[0]), args[1], args[2], int(dtype));
+}
+
+PyObject *empty_like(PyObject *, PyObject *o) {   // a dense tensor of o's shape, device and type
+  if (!PyObject_TypeCheck(o, &TensorType)) {
+    PyErr_SetString(PyExc_TypeError, "a Tensor is expected");
+    return nullptr;
+  }
+  Tensor *t = as_tensor(o);
+  if (!t->dev) {
+    PyErr_SetString(PyExc_AttributeError, "the tensor has no device");
+    return nullptr;
+  }
+  return tensor_make(Py_TYPE(o), t->shape, t->dev, t->dtype);
+}
+
+int tensor_traverse(PyObject *self, visitproc visit, void *arg) {
+  Tensor *t = as_tensor(self);
+  Py_VISIT(t->shape);
+  Py_VISIT(t->dev);
+  Py_VISIT(t->block);
+  return 0;
+}
+
+int tensor_clear(PyObject *self) {
+  Tensor *t = as_tensor(self);
+  Py_CLEAR(t->shape);
+  Py_CLEAR(t->dev);
+  Py_CLEAR(t->block);
+  return 0;
+}
+
+void tensor_dealloc(PyObject *self) {
+  PyObject_GC_UnTrack(self);
+  tensor_clear(self);
+  Py_TYPE(self)->tp_free(self);
+}
+
+PyObject *tensor_shape(PyObject *self, PyObject *const *args, Py_ssize_t n) {
+  PyObject *shape = as_tensor(self)->shape;
+  if (count_of(shape) < 0 && PyErr_Occurred()) return nullptr;
+  if (n == 0 || (n == 1 && args[0] == Py_None)) return PySequence_List(shape);
+  if (n != 1) {
+    PyErr_SetString(PyExc_TypeError, "shape(axis=None)");
+    return nullptr;
+  }
+  return PyObject_GetItem(shape, args[0]);
+}
+
+PyObject *tensor_size(PyObject *self, PyObject *) {
+  const Py_ssize_t n = count_of(as_tensor(self)->shape);
+  return n < 0 && PyErr_Occurred() ? nullptr : PyLong_FromSsize_t(n);
+}
+
+PyObject *tensor_memsize(PyObject *self, PyObject *) {
+  const Py_ssize_t n = count_of(as_tensor(self)->shape);
+  return n < 0 && PyErr_Occurred() ? nullptr : PyLong_FromSsize_t(n * elem_size(as_tensor(self)->dtype));
+}
+
+PyObject *tensor_ndim(PyObject *self, PyObject *) {
+  PyObject *shape = as_tensor(self)->shape;
+  return count_of(shape) < 0 && PyErr_Occurred() ? nullptr : PyLong_FromSsize_t(PyTuple_GET_SIZE(shape));
+}
+
+PyObject *tensor_data_type(PyObject *self, PyObject *) { return PyLong_FromLong(as_tensor(self)->dtype); }
+PyObject *tensor_transpose(PyObject *self, PyObject *) { return PyBool_FromLong(as_tensor(self)->transposed); }
+
+PyObject *tensor_device(PyObject *self, PyObject *) {
+  PyObject *d = as_tensor(self)->dev;
+  if (!d) d = Py_None;
+  Py_INCREF(d);
+  return d;
+}
+
+PyObject *tensor_ptr(PyObject *self, void *) {
+  PyObject *b = as_tensor(self)->block;
+  if (b && Py_TYPE(b) == &BlockType) {
+    PyObject *a = reinterpret_cast<Block *>(b)->address;
+    Py_INCREF(a);
+    return a;
+  }
+  PyErr_SetString(PyExc_AttributeError, "the tensor has no memory");
+  return nullptr;
+}
+
+PyMemberDef tensor_members[] = {{"_shape", T_OBJECT, offsetof(Tensor, shape), 0, "tuple of extents"},
+                                {"_dev", T_OBJECT, offsetof(Tensor, dev), 0, "device"},
+                                {"_block", T_OBJECT, offsetof(Tensor, block), 0, "memory"},
+                                {"_dtype", T_INT, offsetof(Tensor, dtype), 0, "data type"},
+                                {"_transposed", T_BOOL, offsetof(Tensor, transposed), 0, "view of the stored matrix transposed"},
+                                {nullptr, 0, 0, 0, nullptr}};
+PyGetSetDef tensor_getset[] = {{"ptr", tensor_ptr, nullptr, "device address", nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyMethodDef tensor_methods[] = {
+    {"shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(tensor_shape)), METH_FASTCALL, "extents, or one of them"},
+    {"Size", tensor_size, METH_NOARGS, "number of elements"},
+    {"MemSize", tensor_memsize, METH_NOARGS, "bytes"},
+    {"nDim", tensor_ndim, METH_NOARGS, "number of dimensions"},
+    {"data_type", tensor_data_type, METH_NOARGS, "data type"},
+    {"transpose", tensor_transpose, METH_NOARGS, "whether this is a transposed view"},
+    {"device", tensor_device, METH_NOARGS, "device"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyTypeObject TensorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ------------------------------------------------------------------------------------ module
+
+PyObject *set_check(PyObject *, PyObject *f) {
+  Py_INCREF(f);
+  Py_XSETREF(g_check, f);
+  Py_RETURN_NONE;
+}
+
+// fork(handle): the auxiliary stream's address
+PyObject *fork_(PyObject *, PyObject *h) {
+  void *aux = nullptr;
+  sgh_device *d = static_cast<sgh_device *>(PyLong_AsVoidPtr(h));
+  if (PyErr_Occurred() || failed(sgh_device_fork(d, &aux), "sgh_device_fork")) return nullptr;
+  return PyLong_FromVoidPtr(aux);
+}
+
+#define SGH_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call<&name>::call)), METH_FASTCALL, nullptr}
+#define SGH_CALL3(name) SGH_CALL(name##_f32), SGH_CALL(name##_f16), SGH_CALL(name##_bf16)
+
+PyMethodDef methods[] = {
+    {"set_check", set_check, METH_O, "the function that turns a return code into an exception"},
+    {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(empty)), METH_FASTCALL, "empty(cls, shape, device, dtype)"},
+    {"empty_like", empty_like, METH_O, "a dense tensor of the same shape, device and type"},
+    {"fork", fork_, METH_O, "sgh_device_fork: the auxiliary stream"},
+    SGH_CALL(sgh_device_join), SGH_CALL(sgh_block_used_on),
+    SGH_CALL3(sgh_memset), SGH_CALL3(sgh_relu_fwd), SGH_CALL3(sgh_relu_bwd), SGH_CALL3(sgh_relu_bwd_add), SGH_CALL3(sgh_add),
+    SGH_CALL3(sgh_add_relu), SGH_CALL3(sgh_eltwise_mult), SGH_CALL3(sgh_axpy), SGH_CALL(sgh_axpy_devalpha_f32),
+    SGH_CALL(sgh_sub_f32), SGH_CALL(sgh_div_f32), SGH_CALL(sgh_add_scalar_f32), SGH_CALL(sgh_mult_scalar_f32),
+    SGH_CALL(sgh_clamp_f32), SGH_CALL(sgh_cast_f32_to_f16), SGH_CALL(sgh_cast_f16_to_f32), SGH_CALL(sgh_cast_f32_to_bf16),
+    SGH_CALL(sgh_cast_bf16_to_f32), SGH_CALL(sgh_cast_f32_to_i32), SGH_CALL(sgh_cast_i32_to_f32),
+    SGH_CALL3(sgh_softmax_ce_bwd), SGH_CALL(sgh_softmax_fwd_f32), SGH_CALL(sgh_cross_entropy_fwd_f32),
+    SGH_CALL3(sgh_gemm), SGH_CALL(sgh_sum_rows_f32), SGH_CALL(sgh_add_row_f32), SGH_CALL(sgh_row_max_f32),
+    SGH_CALL(sgh_row_max_zero_seeded_f32), SGH_CALL(sgh_dot_f32), SGH_CALL(sgh_sum_all_f32),
+    SGH_CALL3(sgh_sgd_momentum), SGH_CALL(sgh_sgd_momentum_multi_f32), SGH_CALL(sgh_sgd_momentum_multi_mixed),
+    SGH_CALL(sgh_sgd_momentum_master_f16), SGH_CALL(sgh_sgd_momentum_master_bf16),
+    SGH_CALL3(sgh_conv_fwd), SGH_CALL3(sgh_conv_dgrad), SGH_CALL3(sgh_conv_wgrad), SGH_CALL3(sgh_conv_bgrad),
+    SGH_CALL(sgh_conv_dgrad_acc_f32), SGH_CALL(sgh_conv_wgrad_bias_f32),
+    SGH_CALL3(sgh_bn_fwd_train), SGH_CALL3(sgh_bn_relu_fwd_train), SGH_CALL3(sgh_bn_add_relu_fwd_train), SGH_CALL3(sgh_bn_fwd_infer),
+    SGH_CALL3(sgh_bn_bwd), SGH_CALL3(sgh_bn_relu_bwd), SGH_CALL3(sgh_pool_fwd), SGH_CALL3(sgh_pool_bwd),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "tensors, memory blocks and direct calls into libsinga_hip", -1, methods,
+                      nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native() {
+  BlockType.tp_name = "singa_amd._native.Block";
+  BlockType.tp_doc = "Block(dev, nbytes, ptr=None, keepalive=None): a pool allocation, or memory owned elsewhere";
+  BlockType.tp_basicsize = sizeof(Block);
+  BlockType.tp_flags = Py_TPFLAGS_DEFAULT;
+  BlockType.tp_new = block_tp_new;
+  BlockType.tp_dealloc = block_dealloc;
+  BlockType.tp_members = block_members;
+  TensorType.tp_name = "singa_amd._native.TensorBase";
+  TensorType.tp_doc = "the fields of a tensor and their accessors";
+  TensorType.tp_basicsize = sizeof(Tensor);
+  TensorType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC;
+  TensorType.tp_new = PyType_GenericNew;
+  TensorType.tp_dealloc = tensor_dealloc;
+  TensorType.tp_traverse = tensor_traverse;
+  TensorType.tp_clear = tensor_clear;
+  TensorType.tp_members = tensor_members;
+  TensorType.tp_getset = tensor_getset;
+  TensorType.tp_methods = tensor_methods;
+  if (PyType_Ready(&BlockType) < 0 || PyType_Ready(&TensorType) < 0) return nullptr;
+  g_handle_name = PyUnicode_InternFromString("_handle");
+  PyObject *m = PyModule_Create(&module);
+  if (!m) return nullptr;
+  Py_INCREF(&BlockType);
+  PyModule_AddObject(m, "Block", reinterpret_cast<PyObject *>(&BlockType));
+  Py_INCREF(&TensorType);
+  PyModule_AddObject(m, "TensorBase", reinterpret_cast<PyObject *>(&TensorType));
+  return m;
+}

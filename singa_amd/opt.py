@@ -7,13 +7,22 @@ single launch over all parameters (``apply_all``, the loop of ``Optimizer.call``
     g' = g + momentum * v   (nesterov)   |   v   (otherwise)
     p -= lr * g'
 """
-import ctypes as C
+import array
 
 import numpy as np
 
 from . import _lib
 from . import singa_wrap as singa
 from ._lib import check
+
+
+def _upload_table(dev, words):
+    """A table of 64-bit words on the device, uploaded in stream order without draining the stream."""
+    arr = array.array("Q", words)
+    address, count = arr.buffer_info()
+    table = singa.Tensor((2 * count,), dev, singa.kInt)
+    check(_lib.lib().sgh_upload_async(dev._h, table.ptr, address, 8 * count), "sgh_upload_async")
+    return table
 
 
 class SGD(object):
@@ -65,7 +74,7 @@ class SGD(object):
             return self._apply_op_by_op(param_name, param_value, param_grad)
         v = self._moment(param_name, param_value) if self.momentum != 0 else None
         name = "sgh_sgd_momentum_" + singa._SUFFIX[param_value.data_type()]   # f32 / f16 / bf16
-        check(getattr(_lib.lib(), name)(param_value.ptr, param_grad.ptr, v.ptr if v is not None else None,
+        check(getattr(singa._L(), name)(param_value.ptr, param_grad.ptr, v.ptr if v is not None else None,
                                         param_value.Size(), self.lr, self.momentum, self.dampening,
                                         self.weight_decay, int(self.nesterov), param_value.device().stream), name)
 
@@ -104,7 +113,7 @@ class SGD(object):
         master = self.masters[param_name]
         v = self._moment(param_name, master) if self.momentum != 0 else None
         name = "sgh_sgd_momentum_master_" + singa._SUFFIX[param_value.data_type()]
-        check(getattr(_lib.lib(), name)(master.ptr, param_grad.ptr, v.ptr if v is not None else None, param_value.ptr,
+        check(getattr(singa._L(), name)(master.ptr, param_grad.ptr, v.ptr if v is not None else None, param_value.ptr,
                                         param_value.Size(), self.lr, self.momentum, self.dampening,
                                         self.weight_decay, int(self.nesterov), param_value.device().stream), name)
 
@@ -125,21 +134,20 @@ class SGD(object):
             self._table, self._table_total = cached
             self._table_key = key
         if key != self._table_key:
-            arr = (_lib.SgdItem * len(items))()
+            words = []   # sgh_sgd_item {p, g, v, n} of every parameter, four 64-bit words each
             total = 0
-            for i, (n, p, g) in enumerate(items):
-                assert p.shape() == g.shape(), ("shape mismatch", n)
+            for n, p, g in items:
+                assert p._shape == g._shape, ("shape mismatch", n)
                 v = self._moment(n, p) if self.momentum != 0 else None
-                arr[i].p, arr[i].g, arr[i].v, arr[i].n = p.ptr, g.ptr, (v.ptr if v is not None else None), p.Size()
-                total += p.Size()
-            nbytes = C.sizeof(arr)
-            table = singa.Tensor(((nbytes + 3) // 4,), dev, singa.kInt)
-            check(_lib.lib().sgh_upload_async(dev._h, table.ptr, C.addressof(arr), nbytes), "sgh_upload_async")
+                size = p.Size()
+                words += (p.ptr, g.ptr, v.ptr if v is not None else 0, size)
+                total += size
+            table = _upload_table(dev, words)
             self._table, self._table_key, self._table_total = table, key, total
             if len(self._tables) >= 16:
                 self._tables.pop(next(iter(self._tables)))
             self._tables[key] = (table, total)
-        check(_lib.lib().sgh_sgd_momentum_multi_f32(self._table.ptr, len(items), self._table_total, self.lr,
+        check(singa._L().sgh_sgd_momentum_multi_f32(self._table.ptr, len(items), self._table_total, self.lr,
                                                     self.momentum, self.dampening, self.weight_decay,
                                                     int(self.nesterov), dev.stream), "sgh_sgd_momentum_multi_f32")
 
@@ -154,14 +162,14 @@ class SGD(object):
         key = ("mixed",) + tuple((n, p.ptr, g.ptr) for n, p, g in items)
         cached = self._tables.get(key)
         if cached is None:
-            arr = (_lib.SgdMixedItem * len(items))()
+            words = []   # sgh_sgd_mixed_item {p, g, v, p16, n} of every parameter
             total, half_type = 0, None
-            for i, (n, p, g) in enumerate(items):
-                assert p.shape() == g.shape(), ("shape mismatch", n)
+            for n, p, g in items:
+                assert p._shape == g._shape, ("shape mismatch", n)
                 if p.data_type() != g.data_type():
                     raise singa.SingaHipError("parameter and gradient differ in data type")
                 if p.data_type() == singa.kFloat32:
-                    tgt, p16 = p, None
+                    tgt, p16 = p, 0
                 else:
                     if half_type not in (None, p.data_type()):
                         raise singa.SingaHipError("one 16-bit type per update")
@@ -170,16 +178,15 @@ class SGD(object):
                         self.masters[n] = p.AsType(singa.kFloat32)
                     tgt, p16 = self.masters[n], p.ptr
                 v = self._moment(n, tgt) if self.momentum != 0 else None
-                arr[i].p, arr[i].g, arr[i].v, arr[i].p16, arr[i].n = tgt.ptr, g.ptr, (v.ptr if v is not None else None), p16, p.Size()
-                total += p.Size()
-            nbytes = C.sizeof(arr)
-            table = singa.Tensor(((nbytes + 3) // 4,), dev, singa.kInt)
-            check(_lib.lib().sgh_upload_async(dev._h, table.ptr, C.addressof(arr), nbytes), "sgh_upload_async")
+                size = p.Size()
+                words += (tgt.ptr, g.ptr, v.ptr if v is not None else 0, p16, size)
+                total += size
+            table = _upload_table(dev, words)
             if len(self._tables) >= 16:
                 self._tables.pop(next(iter(self._tables)))
             cached = self._tables[key] = (table, total, int(half_type == singa.kBFloat16))
         table, total, bf16 = cached
-        check(_lib.lib().sgh_sgd_momentum_multi_mixed(table.ptr, len(items), total, bf16, self.lr, self.momentum,
+        check(singa._L().sgh_sgd_momentum_multi_mixed(table.ptr, len(items), total, bf16, self.lr, self.momentum,
                                                       self.dampening, self.weight_decay, int(self.nesterov),
                                                       dev.stream), "sgh_sgd_momentum_multi_mixed")
 

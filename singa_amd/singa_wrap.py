@@ -22,7 +22,10 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
+from . import _native
 from ._lib import SingaHipError, check  # noqa: F401  (re-exported)
+
+_native.set_check(check)
 
 # core.proto DataType values (src/proto/core.proto:26-34)
 kFloat32, kFloat16, kInt = 0, 1, 2
@@ -36,13 +39,20 @@ _SIZE_OF = {kFloat32: 4, kInt: 4, kFloat16: 2, kBFloat16: 2}
 _SUFFIX = {kFloat32: "f32", kFloat16: "f16", kBFloat16: "bf16"}
 
 
+_entry = {}   # (operation, data type) -> (entry point, its name)
+
+
 def _fn(name, t):
     """The entry point of `name` for t's data type: sgh_<name>_<f32|f16|bf16>."""
-    sfx = _SUFFIX.get(t.data_type())
-    if sfx is None:
-        raise SingaHipError("%s: unsupported data type %r" % (name, t.data_type()))
-    full = "sgh_%s_%s" % (name, sfx)
-    return getattr(_L(), full), full
+    key = (name, t._dtype)
+    found = _entry.get(key)
+    if found is None:
+        sfx = _SUFFIX.get(t._dtype)
+        if sfx is None:
+            raise SingaHipError("%s: unsupported data type %r" % (name, t._dtype))
+        full = "sgh_%s_%s" % (name, sfx)
+        found = _entry[key] = (getattr(_L(), full), full)
+    return found
 
 
 def bf16_bits_to_float(bits):
@@ -61,8 +71,21 @@ def float_to_bf16_bits(a):
 USE_HIP = True
 
 
+class _Direct(object):
+    """The C ABI: calls made by the extension where it has them, ctypes for the rest (the functions that fill in structures
+    or host memory)."""
+
+    def __getattr__(self, name):
+        fn = getattr(_native, name, None) or getattr(_lib.lib(), name)
+        setattr(self, name, fn)
+        return fn
+
+
+_direct = _Direct()
+
+
 def _L():
-    return _lib.lib()
+    return _direct
 
 
 # ------------------------------------------------------------------------------------ device
@@ -75,6 +98,7 @@ class HipGPU(object):
         h = C.c_void_p()
         check(_L().sgh_device_open(int(gpu_id), C.byref(h)), "sgh_device_open")
         self._h = h
+        self._handle = h.value
         self._id = int(gpu_id)
         self.stream = _L().sgh_device_stream(h)
 
@@ -122,18 +146,16 @@ class HipGPU(object):
         return self._aux
 
     def Fork(self):
-        aux = C.c_void_p()
-        check(_L().sgh_device_fork(self._h, C.byref(aux)), "sgh_device_fork")
-        self._aux = aux.value
+        self._aux = _native.fork(self._handle)
         return self._aux
 
     def Join(self):
-        check(_L().sgh_device_join(self._h), "sgh_device_join")
+        check(_native.sgh_device_join(self._handle), "sgh_device_join")
 
     def UsedOn(self, stream, *tensors):
         for t in tensors:
             if t._block.owned:    # (memory the pool does not own is the caller's to keep alive)
-                check(_L().sgh_block_used_on(self._h, t.ptr, stream), "sgh_block_used_on")
+                check(_native.sgh_block_used_on(self._handle, t.ptr, stream), "sgh_block_used_on")
 
     def GetAllocatedMem(self):
         a, c, d = C.c_size_t(), C.c_size_t(), C.c_size_t()
@@ -175,15 +197,6 @@ class HipGPU(object):
             check(_L().sgh_graph_destroy(self._graph), "sgh_graph_destroy")
             self._graph = None
 
-    def _malloc(self, nbytes):
-        p = C.c_void_p()
-        check(_L().sgh_malloc(self._h, C.byref(p), nbytes), "sgh_malloc")
-        return p.value
-
-    def _free(self, ptr):
-        if self._h is not None and _lib._lib is not None:
-            _lib._lib.sgh_free(self._h, C.c_void_p(ptr))
-
 
 _devices = {}
 
@@ -202,29 +215,13 @@ create_cuda_gpu = create_hip_gpu_on
 
 # ------------------------------------------------------------------------------------ tensor
 
-class _Block(object):
-    """Counterpart of ``Block`` (include/singa/core/common.h:64-97): a pool allocation freed
-    when the last Tensor referring to it goes away."""
-
-    def __init__(self, dev, nbytes, ptr=None, keepalive=None):
-        self.dev = dev
-        self.nbytes = nbytes
-        self.owned = ptr is None
-        self.ptr = dev._malloc(max(nbytes, 1)) if ptr is None else ptr
-        self.keepalive = keepalive
-
-    def __del__(self):
-        try:
-            if self.owned and self.ptr:
-                self.dev._free(self.ptr)
-                self.ptr = None
-        except Exception:
-            pass
+_Block = _native.Block   # counterpart of ``Block`` (include/singa/core/common.h:64-97): freed with the last Tensor on it
 
 
-class Tensor(object):
-    """Counterpart of ``singa::Tensor`` as Python sees it (src/api/core_tensor.i:95-232):
-    dense row-major data on a HipGPU, plus a transpose flag for 2-D views."""
+class Tensor(_native.TensorBase):
+    """Counterpart of ``singa::Tensor`` as Python sees it (src/api/core_tensor.i:95-232): dense row-major data on a
+    HipGPU, plus a transpose flag for 2-D views.  The fields and their accessors (``shape``, ``nDim``, ``Size``,
+    ``MemSize``, ``data_type``, ``device``, ``transpose``, ``ptr``) live in the extension."""
 
     def __init__(self, shape=(), device=None, dtype=kFloat32, _block=None, _transposed=False):
         if device is None:
@@ -235,36 +232,7 @@ class Tensor(object):
         self._dev = device
         self._dtype = dtype
         self._transposed = _transposed
-        self._block = _block if _block is not None else _Block(device, self.Size() * _SIZE_OF[dtype])
-
-    # --- reference accessors
-    def shape(self, axis=None):
-        return list(self._shape) if axis is None else self._shape[axis]
-
-    def nDim(self):
-        return len(self._shape)
-
-    def Size(self):
-        n = 1
-        for s in self._shape:
-            n *= s
-        return n
-
-    def MemSize(self):
-        return self.Size() * _SIZE_OF[self._dtype]
-
-    def data_type(self):
-        return self._dtype
-
-    def device(self):
-        return self._dev
-
-    def transpose(self):
-        return self._transposed
-
-    @property
-    def ptr(self):
-        return self._block.ptr
+        self._block = _block if _block is not None else _Block(device, self.MemSize())
 
     # --- views
     def Reshape(self, shape):
@@ -377,7 +345,7 @@ def _need_f32(what, *tensors):
     """The fp32-only entry points read their operands as floats: refuse anything else, as the
     reference's TYPE_LANG_SWITCH does for a type it has no kernel for (tensor.cc:760-812)."""
     for t in tensors:
-        if t is not None and t.data_type() != kFloat32:
+        if t is not None and t._dtype != kFloat32:
             raise SingaHipError("%s: float32 tensors only, got data type %r" % (what, t.data_type()))
 
 
@@ -488,9 +456,9 @@ def Gaussian(mean, std, t):
 
 
 def _same(a, b):
-    if a.Size() != b.Size() or a.data_type() != b.data_type():
+    if a._dtype != b._dtype or (a._shape != b._shape and a.Size() != b.Size()):
         raise SingaHipError("shape/type mismatch: %s vs %s" % (a.shape(), b.shape()))
-    if a.transpose() or b.transpose():
+    if a._transposed or b._transposed:
         raise SingaHipError("elementwise ops need contiguous (non-transposed) tensors")
 
 
@@ -530,8 +498,8 @@ def Reshape(t, shape):
 
 # ------------------------------------------------------------------------------------ tensor math
 
-def _like(t):
-    return Tensor(t.shape(), t.device(), t.data_type())
+_like = _native.empty_like   # a dense tensor of t's shape, device and type
+_empty = _native.empty       # _empty(Tensor, shape tuple, device, dtype)
 
 
 def ReLU(x):
@@ -588,7 +556,7 @@ def _ce_dims(p, t, half_ok=False):
 
 def CrossEntropyFwd(p, t):
     batch, dim, int_target = _ce_dims(p, t)
-    loss = Tensor((batch,), p.device(), kFloat32)
+    loss = _empty(Tensor, (batch,), p.device(), kFloat32)
     check(_L().sgh_cross_entropy_fwd_f32(p.ptr, t.ptr, loss.ptr, batch, dim, int(int_target),
                                          p.device().stream), "sgh_cross_entropy_fwd_f32")
     return loss
@@ -708,17 +676,17 @@ def DivFloat(t, x):
 def Mult(A, B):
     """``singa.Mult(A, B)`` for 2-D tensors (src/core/tensor/tensor.cc:1633-1706): the transpose
     flags of the views select the GEMM variant, no data is moved."""
-    if A.nDim() != 2 or B.nDim() != 2 or A.shape(1) != B.shape(0):
+    sa, sb = A._shape, B._shape
+    if len(sa) != 2 or len(sb) != 2 or sa[1] != sb[0]:
         raise SingaHipError("Mult shape mismatch %s x %s" % (A.shape(), B.shape()))
-    if A.data_type() != B.data_type():
+    if A._dtype != B._dtype:
         raise SingaHipError("Mult: operands differ in data type")
     fn, name = _fn("gemm", A)   # 16-bit operands: the 16-bit matrix instructions, fp32 accumulation, one rounding
-    M, K, N = A.shape(0), A.shape(1), B.shape(1)
-    out = Tensor((M, N), A.device(), A.data_type())
-    tA, tB = A.transpose(), B.transpose()
-    lda = M if tA else K
-    ldb = K if tB else N
-    check(fn(int(tA), int(tB), M, N, K, 1.0, A.ptr, lda, B.ptr, ldb, 0.0, out.ptr, N, A.device().stream), name)
+    (M, K), N = sa, sb[1]
+    dev = A._dev
+    out = _empty(Tensor, (M, N), dev, A._dtype)
+    tA, tB = A._transposed, B._transposed
+    check(fn(int(tA), int(tB), M, N, K, 1.0, A.ptr, M if tA else K, B.ptr, K if tB else N, 0.0, out.ptr, N, dev.stream), name)
     return out
 
 
@@ -727,7 +695,7 @@ def Sum(t, axis):
     if t.nDim() != 2 or axis != 0 or t.transpose():
         raise SingaHipError("only Sum(2-D tensor, 0) is on the backward path")
     _need_f32("Sum", t)
-    out = Tensor((t.shape(1),), t.device(), kFloat32)
+    out = _empty(Tensor, (t.shape(1),), t.device(), kFloat32)
     check(_L().sgh_sum_rows_f32(t.ptr, out.ptr, t.shape(0), t.shape(1), t.device().stream), "sgh_sum_rows_f32")
     return out
 
@@ -763,8 +731,11 @@ class CudnnConvHandle(object):
                                               self.width, self.num_filters, self.kernel_h, self.kernel_w,
                                               self.stride_h, self.stride_w, self.pad_h, self.pad_w, groups),
               "sgh_conv_geom_init_grouped")
+        self.geom_ptr = C.addressof(self.geom)
         self.channels_per_filter = self.channels // groups   # (convolution.cc:461)
         self.conv_height, self.conv_width = self.geom.P, self.geom.Q
+        self.x_shape = (self.batchsize, self.channels, self.height, self.width)
+        self.dy_shape = (self.batchsize, self.num_filters, self.conv_height, self.conv_width)
         self.col_height = self.channels * self.kernel_h * self.kernel_w
         self.col_width = self.conv_height * self.conv_width
         self.imagesize = x.Size() // self.batchsize
@@ -779,20 +750,20 @@ class CudnnConvHandle(object):
         self.wgrad_workspace = None   # a second one, made when a weight gradient runs on the auxiliary stream
 
     def _check_x(self, x):
-        if x.shape() != [self.batchsize, self.channels, self.height, self.width]:
+        if x._shape != self.x_shape:
             raise SingaHipError("input sample shape should not change")
 
     def _check_dy(self, dy):
-        if dy.shape() != [self.batchsize, self.num_filters, self.conv_height, self.conv_width]:
+        if dy._shape != self.dy_shape:
             raise SingaHipError("dy shape does not match the handle")
 
 
 def GpuConvForward(x, W, b, h):
     h._check_x(x)
-    y = Tensor((h.batchsize, h.num_filters, h.conv_height, h.conv_width), x.device(), x.data_type())
+    y = _empty(Tensor, h.dy_shape, x.device(), x.data_type())
     bias = b.ptr if (h.bias_term and b is not None) else None
     fn, name = _fn("conv_fwd", x)
-    check(fn(C.byref(h.geom), x.ptr, W.ptr, bias, y.ptr, h.workspace.ptr, h.workspace.MemSize(),
+    check(fn(h.geom_ptr, x.ptr, W.ptr, bias, y.ptr, h.workspace.ptr, h.workspace.MemSize(),
              x.device().stream), name)
     return y
 
@@ -804,7 +775,7 @@ def GpuConvBackwardxAccumulate(dy, W, x, h, dx):
     h._check_dy(dy)
     _same(dx, x)
     if dy.data_type() == kFloat32:   # (on 16-bit tensors the kernel's read-modify-write loses to the separate add)
-        rc = _L().sgh_conv_dgrad_acc_f32(C.byref(h.geom), dy.ptr, W.ptr, dx.ptr, h.workspace.ptr,
+        rc = _L().sgh_conv_dgrad_acc_f32(h.geom_ptr, dy.ptr, W.ptr, dx.ptr, h.workspace.ptr,
                                          h.workspace.MemSize(), dy.device().stream)
         if rc != _lib.SGH_EUNSUPPORTED:
             check(rc, "sgh_conv_dgrad_acc_f32")
@@ -817,7 +788,7 @@ def GpuConvBackwardx(dy, W, x, h):
     h._check_dy(dy)
     dx = _like(x)
     fn, name = _fn("conv_dgrad", dy)
-    check(fn(C.byref(h.geom), dy.ptr, W.ptr, dx.ptr, h.workspace.ptr, h.workspace.MemSize(),
+    check(fn(h.geom_ptr, dy.ptr, W.ptr, dx.ptr, h.workspace.ptr, h.workspace.MemSize(),
              dy.device().stream), name)
     return dx
 
@@ -841,7 +812,7 @@ def GpuConvBackwardW(dy, x, W, h, stream=None, out=None):
             h.wgrad_workspace = Tensor(((max(need, 4) + 3) // 4,), dy.device(), kFloat32)
         ws = h.wgrad_workspace
         dy.device().UsedOn(stream, dy, x, dW, ws)
-    check(fn(C.byref(h.geom), dy.ptr, x.ptr, dW.ptr, ws.ptr, ws.MemSize(),
+    check(fn(h.geom_ptr, dy.ptr, x.ptr, dW.ptr, ws.ptr, ws.MemSize(),
              dy.device().stream if stream is None else stream), name)
     return dW
 
@@ -856,7 +827,7 @@ def GpuConvBackwardWb(dy, x, W, b, h):
     h._check_x(x)
     dW, db = _like(W), _like(b)
     ws = h.workspace
-    check(_L().sgh_conv_wgrad_bias_f32(C.byref(h.geom), dy.ptr, x.ptr, dW.ptr, db.ptr, ws.ptr, ws.MemSize(),
+    check(_L().sgh_conv_wgrad_bias_f32(h.geom_ptr, dy.ptr, x.ptr, dW.ptr, db.ptr, ws.ptr, ws.MemSize(),
                                        dy.device().stream), "sgh_conv_wgrad_bias_f32")
     return dW, db
 
@@ -892,7 +863,7 @@ def GpuConvBackwardb(dy, b, h):
     h._check_dy(dy)
     db = _like(b)
     fn, name = _fn("conv_bgrad", dy)
-    check(fn(C.byref(h.geom), dy.ptr, db.ptr, dy.device().stream), name)
+    check(fn(h.geom_ptr, dy.ptr, db.ptr, dy.device().stream), name)
     return db
 
 
@@ -909,6 +880,7 @@ class CudnnBatchNormHandle(object):
             self.batchsize, self.channels, self.height, self.width = x.shape()
         else:
             raise SingaHipError("BatchNorm expects a 2-D or 4-D input")
+        self.channel_shape = (self.channels,)
         hw = self.height * self.width
         nbytes = _L().sgh_bn_workspace_bytes(self.batchsize, self.channels, hw)
         self.workspace = Tensor((max(nbytes // 4, 1),), x.device(), kFloat32)
@@ -921,8 +893,8 @@ def GpuBatchNormForwardTraining(h, x, scale, bias, running_mean, running_var):
     """Returns ``[y, mean, var]`` where ``var`` holds the saved inverse standard deviation, and
     updates the running statistics in place (src/model/operation/batchnorm.cc:287-329)."""
     y = _like(x)
-    mean = Tensor((h.channels,), x.device(), kFloat32)
-    var = Tensor((h.channels,), x.device(), kFloat32)
+    mean = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
+    var = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
     fn, name = _fn("bn_fwd_train", x)  # 16-bit activations keep fp32 scale / bias / statistics
     check(fn(x.ptr, scale.ptr, bias.ptr,
              running_mean.ptr if running_mean is not None else None,
@@ -936,8 +908,8 @@ def GpuBatchNormReLUForwardTraining(h, x, scale, bias, running_mean, running_var
     """``GpuBatchNormForwardTraining`` with the ReLU that follows folded in: ``[relu(y), mean, var]``, the bits
     ``ReLU(GpuBatchNormForwardTraining(...)[0])`` stores (conv -> BatchNorm -> ReLU, examples/cnn/model/resnet.py:54-60)."""
     y = _like(x)
-    mean = Tensor((h.channels,), x.device(), kFloat32)
-    var = Tensor((h.channels,), x.device(), kFloat32)
+    mean = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
+    var = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
     fn, name = _fn("bn_relu_fwd_train", x)
     check(fn(x.ptr, scale.ptr, bias.ptr,
              running_mean.ptr if running_mean is not None else None,
@@ -952,8 +924,8 @@ def GpuBatchNormAddReLUForwardTraining(h, x, z, scale, bias, running_mean, runni
     (examples/cnn/model/resnet.py:70-77) in one call, the bits the three separate calls store."""
     _same(x, z)
     y = _like(x)
-    mean = Tensor((h.channels,), x.device(), kFloat32)
-    var = Tensor((h.channels,), x.device(), kFloat32)
+    mean = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
+    var = _empty(Tensor, h.channel_shape, x.device(), kFloat32)
     fn, name = _fn("bn_add_relu_fwd_train", x)
     check(fn(x.ptr, z.ptr, scale.ptr, bias.ptr,
              running_mean.ptr if running_mean is not None else None,
@@ -1017,22 +989,24 @@ class CudnnPoolingHandle(object):
         check(_L().sgh_pool_geom_init(C.byref(self.geom), self.batchsize, self.channels, self.height,
                                       self.width, self.kernel_h, self.kernel_w, self.stride_h, self.stride_w,
                                       self.pad_h, self.pad_w, int(self.is_max_pooling)), "sgh_pool_geom_init")
+        self.geom_ptr = C.addressof(self.geom)
         self.pooled_height, self.pooled_width = self.geom.P, self.geom.Q
+        self.dy_shape = (self.batchsize, self.channels, self.pooled_height, self.pooled_width)
 
 
 def GpuPoolingForward(h, x):
-    y = Tensor((h.batchsize, h.channels, h.pooled_height, h.pooled_width), x.device(), x.data_type())
+    y = _empty(Tensor, h.dy_shape, x.device(), x.data_type())
     fn, name = _fn("pool_fwd", x)
-    check(fn(C.byref(h.geom), x.ptr, y.ptr, x.device().stream), name)
+    check(fn(h.geom_ptr, x.ptr, y.ptr, x.device().stream), name)
     return y
 
 
 def GpuPoolingBackward(h, dy, x, y):
-    if dy.shape() != [h.batchsize, h.channels, h.pooled_height, h.pooled_width]:
+    if dy._shape != h.dy_shape:
         raise SingaHipError("dy shape does not match the handle")
     if dy.data_type() != x.data_type():
         raise SingaHipError("dy and x differ in data type")
     dx = _like(x)
     fn, name = _fn("pool_bwd", x)
-    check(fn(C.byref(h.geom), dy.ptr, x.ptr, y.ptr if y is not None else None, dx.ptr, dy.device().stream), name)
+    check(fn(h.geom_ptr, dy.ptr, x.ptr, y.ptr if y is not None else None, dx.ptr, dy.device().stream), name)
     return dx
