@@ -27,6 +27,7 @@ constexpr int kNT = 256, kRowsOut = 4, kFilters = 64, kR = 7, kChannels = 3;
 constexpr int kSteps = kChannels * kR * 2;        // 42 steps of four reduction indices
 constexpr int kWPitch = kSteps * 4 + 1;           // dwords per filter in LDS
 constexpr int kRowsIn = 2 * kRowsOut + 5;
+constexpr int kMaxBlocks = 8;   // blocks of 16 pixels in a row: 16 accumulator registers each
 
 struct FwArgs {
   const float *x, *wp, *bias;
@@ -141,8 +142,7 @@ bool sgh_fwd_fewc_supported(const sgh_conv_geom *g) {
     return false;
   if (g->C < 1 || g->C > kChannels || g->K != kFilters || g->H % 2 != 0 || g->W != 2 * g->Q || g->P % kRowsOut != 0)
     return false;
-  const int nb = g->Q / 16;
-  if (g->Q % 16 != 0 || !(nb == 1 || nb == 2 || nb == 4 || nb == 7)) return false;
+  if (g->Q % 16 != 0 || g->Q / 16 > kMaxBlocks) return false;
   return g->N <= 65535;
 }
 
@@ -163,8 +163,12 @@ int sgh_fwd_fewc_run(const sgh_conv_geom *g, const float *x, const float *W, con
   switch (g->Q / 16) {
     case 1: return launch<1>(a, s);
     case 2: return launch<2>(a, s);
+    case 3: return launch<3>(a, s);
     case 4: return launch<4>(a, s);
+    case 5: return launch<5>(a, s);
+    case 6: return launch<6>(a, s);
     case 7: return launch<7>(a, s);
+    case 8: return launch<8>(a, s);
   }
   return SGH_EUNSUPPORTED;
 }

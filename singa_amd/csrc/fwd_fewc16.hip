@@ -32,6 +32,7 @@ constexpr int kNT = 256, kRowsOut = 4, kFilters = 64, kR = 7;
 constexpr int kOctets = 24;                       // 3 channels x 7 window rows, padded to whole instructions
 constexpr int kWPitch = kOctets * 8 + 8;          // 16-bit elements per filter in LDS (the 8 keep 16-byte reads apart)
 constexpr int kRowsIn = 2 * kRowsOut + 5;
+constexpr int kMaxBlocks = 8;   // blocks of 16 pixels in a row: 16 accumulator registers each
 
 struct FwArgs {
   const uint16_t *x, *wp, *bias;
@@ -162,8 +163,12 @@ int launch_nb(const FwArgs &a, hipStream_t s) {
   switch (a.Q / 16) {
     case 1: return launch<1, BF16>(a, s);
     case 2: return launch<2, BF16>(a, s);
+    case 3: return launch<3, BF16>(a, s);
     case 4: return launch<4, BF16>(a, s);
+    case 5: return launch<5, BF16>(a, s);
+    case 6: return launch<6, BF16>(a, s);
     case 7: return launch<7, BF16>(a, s);
+    case 8: return launch<8, BF16>(a, s);
   }
   return SGH_EUNSUPPORTED;
 }
@@ -174,8 +179,7 @@ bool sgh_fwd_fewc16_supported(const sgh_conv_geom *g) {
   if (g->groups != 1 || g->R != kR || g->S != kR || g->stride_h != 2 || g->stride_w != 2 || g->pad_h != 3 || g->pad_w != 3)
     return false;
   if (g->C < 1 || g->C > 3 || g->K != kFilters || g->H % 2 != 0 || g->W != 2 * g->Q || g->P % kRowsOut != 0) return false;
-  const int nb = g->Q / 16;
-  if (g->Q % 16 != 0 || !(nb == 1 || nb == 2 || nb == 4 || nb == 7)) return false;
+  if (g->Q % 16 != 0 || g->Q / 16 > kMaxBlocks) return false;
   if (g->N > 65535) return false;
   return size_t(g->N) * g->K * g->P * g->Q < (size_t(1) << 31);
 }

@@ -864,3 +864,25 @@ def test_fp32_only_functions_refuse_16bit_tensors(singa, dev):
     for call in (lambda: singa.SoftMax(t), lambda: singa.Sum(t, 0), lambda: t.__imul__(2.0)):
         with pytest.raises(singa.SingaHipError):
             call()
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", [(1, 3, 96, True), (2, 2, 160, False), (1, 3, 192, False), (1, 1, 256, True)])
+def test_stem_forward_other_widths(singa, dev, kind, case):
+    """The stem's forward kernels at row lengths of 3, 5, 6 and 8 blocks of 16 pixels (the images of 96 .. 256 pixels), against
+    the oracle on the stored values."""
+    from oracle import cpu_oracle as O
+    from util import nl2
+    N, C, H, bias = case
+    print("stem forward", kind, case, flush=True)
+    r = rng(N + C + H)
+    x32 = r.standard_normal((N, C, H, H)).astype(np.float32)
+    w32 = (r.standard_normal((64, C, 7, 7)) * np.sqrt(2.0 / (C * 49))).astype(np.float32)
+    b32 = r.standard_normal(64).astype(np.float32)
+    if kind == "f32":
+        (xt, x), (wt, w), (bt, b) = ((singa.from_numpy(v, dev), v) for v in (x32, w32, b32))
+    else:
+        (xt, x), (wt, w), (bt, b) = (_to(singa, dev, v, kind) for v in (x32, w32, b32))
+    h = singa.CudnnConvHandle(xt, (7, 7), (2, 2), (3, 3), C, 64, bias)
+    y = singa.GpuConvForward(xt, wt, bt if bias else None, h)
+    assert nl2(y.to_numpy(), O.conv_fwd(x, w, b if bias else None, (2, 2), (3, 3))) < (1e-5 if kind == "f32" else 1e-2)
