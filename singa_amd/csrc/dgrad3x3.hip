@@ -1,23 +1,26 @@
-// Data gradient of 3x3, pad-1 convolutions (stride 1; stride 2 on even images) with an LDS gradient
-// tile shared by all nine taps.
+// Data gradient of 3x3 (stride 1; stride 2 on even images) and 5x5 (stride 1) convolutions with "same" padding, with an LDS
+// gradient tile shared by all taps; the stride-1 forward convolution runs through it as well (bias in the store).
 //
-//   dx[n][c][h][w] = sum_{k,r,s} dy[n][k][h + 1 - r][w + 1 - s] * W[k][c][r][s]
+//   dx[n][c][h][w] = sum_{k,r,s} dy[n][k][h + o - r][w + o - s] * W[k][c][r][s],   o = (R - 1) / 2
 //
-// GEMM view: M = C (128 per workgroup), N = 128 consecutive pixels of the flattened (n, h, w)
+// GEMM view: M = C (BM per workgroup), N = BN consecutive pixels of the flattened (n, h, w)
 // index, reduction = (k, tap).  The reduction runs in chunks of 16 output channels k; per chunk
 // the workgroup stages in LDS
-//   dyS[kc][vrow][col]   the dy rows its 128 pixels touch (one halo row above / below, halo
+//   dyS[kc][vrow][col]   the dy rows its BN pixels touch (o halo rows above / below, halo
 //                        columns, zero padding materialised).  Rows are addressed in a "virtual
-//                        row" space in which every image owns P + 2 rows (a zero row on top and
+//                        row" space in which every image owns P + 2 o rows (zero rows on top and
 //                        at the bottom), so a tile may straddle image boundaries;
-//   Ws[kc][m]            the 16 x 128 weight slice of ONE tap, double-buffered across taps.
-// Every tap reads its B operand from the same dy tile at a compile-time offset, so the inner loop
-// is nothing but LDS reads and MFMAs: no address arithmetic, no predicates, and each dy element is
-// fetched from global memory once per chunk instead of nine times.
-// 512 threads = 8 wavefronts in a 2 (M) x 4 (N) grid, 64 x 32 per wavefront
-// (v_mfma_f32_32x32x2_f32).  The LDS footprint is at most 80 KB and the kernel needs fewer than
-// 128 registers, so two workgroups (four wavefronts per SIMD) share a CU and one's staging work
-// and barriers overlap the other's MFMAs.
+//   Ws[kc][m]            the 16 x BM weight slice of ONE tap, double-buffered across taps.
+// Every tap reads its B operand from the same dy tile at a compile-time offset from one of R row
+// bases, so the inner loop is nothing but LDS reads and MFMAs: no address arithmetic, no predicates, and each dy
+// element is fetched from global memory once per chunk instead of once per tap.
+// 512 threads = 8 wavefronts in a 2 (M) x 4 (N) grid, 64 x 32 or 32 x 32 per wavefront, or (BM = 32) 1 x 8
+// (v_mfma_f32_32x32x2_f32).  With at most 80 KB of LDS and fewer than 128 registers two workgroups (four
+// wavefronts per SIMD) share a CU and one's staging work and barriers overlap the other's MFMAs.
+//
+// The row pitch of the slab is the row's own length, Q + 2 o, and a channel gets 256, 512 or 1024 floats, the smallest that
+// holds the rows a tile touches: any plane width up to about 140 fits, 7 x 7 planes take half the LDS that a pitch of 16
+// took, and a tile's reads step through the banks almost contiguously.
 #include <stdlib.h>
 
 #include "common.h"
@@ -29,11 +32,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int NT = 512;
-constexpr int BN = 128, KC = 16;
+constexpr int KC = 16;
 constexpr int kOOB = int(0x80000000u);
-#ifndef D3_LAT
-#define D3_LAT 2
-#endif
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
@@ -45,6 +45,7 @@ struct D3Args {
   int accumulate;         // dx += result instead of dx = result (gradient fan-in folded into the store)
   float *dx;
   int N, C, H, W, K, KP;  // dx is N x C x H x W
+  int pitch, rows;        // LDS row pitch, rows of the slab
   int P, Q;               // dy is N x K x P x Q (stride 1: P == H, Q == W; stride 2: H == 2P, W == 2Q)
   int total_pix;          // N * P * Q: pixels of the tile index space
   // Work assignment (1-D grid).  Tile t = (pixel tile t / ctiles, channel tile t % ctiles).  Workgroups
@@ -71,36 +72,44 @@ __device__ __forceinline__ int whole_tile_of(const D3Args &a, int w) {
   return (((j >> 3) << 3) + x) * 8 + (j & 7);
 }
 
-// LOGP: log2 of the LDS row pitch (>= W + 2); VR: virtual rows held per channel.
-// BM: output channels per workgroup (64 or 128; the wavefront tile is (BM/2) x 32).
+// BM: output channels per workgroup (the wavefront tile is (BM / 2) x 32, or 32 x 32 when BM is 32); CHS: floats of the slab
+// per gradient channel; R: filter height and width; RAGK: K is not a multiple of 16 (the slab rows of the channels beyond K
+// read as zero, like their weights).
 //
 // The reduction is a flat sequence of tap steps (chunk, tap).  Global loads run LAT steps ahead of
 // their LDS write: the data written at the end of step q (tap q+1's weights, a ninth of the next
 // chunk's dy slab) was requested at the start of step q - LAT and waits in registers, so a
 // request has LAT + 1 steps of MFMA time to return.  Every load address is "thread constant +
 // scalar term" (one vector add); the thread constant is out of range for elements that must read
-// as zero, and K is a multiple of 16, so no per-load predicate is left.
+// as zero.
 //
 // S2 (stride 2, pad 1, even H and W): the tile index space is the P x Q grid of one residue class
 // (h, w) = (2i + a, 2j + b); all four classes of a pixel block are accumulated by the same
 // workgroup (tap (r, s) belongs to class a = (r != 1), b = (s != 1) and reads dy[i + (r == 0)]
 // [j + (s == 0)]), so no MFMA is spent on the zeros of a dilated gradient, every tap is still a
 // compile-time LDS offset, and a lane stores its 2 x 2 output block as two 8-byte writes.
-template <int BM, int LOGP, int VR, bool S2>
+template <int BM>
+struct Tile {
+  static constexpr int WMN = BM == 32 ? 1 : 2, WNN = 8 / WMN;   // wavefront grid
+  static constexpr int BN = 32 * WNN;                           // pixels
+};
+
+template <int BM, int CHS, bool S2, int R, bool RAGK>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_dgrad3x3(D3Args a) {
   constexpr int NCLS = S2 ? 4 : 1;          // residue classes accumulated side by side
+  constexpr int BN = Tile<BM>::BN;
   constexpr int PA = BM;                    // weight tile pitch
-  constexpr int TM = BM / 64;               // 32-row MFMA tiles per wavefront
-  constexpr int PITCHP = 1 << LOGP;
-  constexpr int VRP = VR * PITCHP;          // floats per channel slab
-  constexpr int CHS = VRP;                   // channel stride in LDS (a wavefront's two 32-lane halves are served separately)
-  constexpr int DSLOTS = KC * VRP / NT;     // dy elements per thread per chunk
-  constexpr int SPT = (DSLOTS + 8) / 9;     // dy slots fetched per tap step
-  constexpr int SUB = VRP > NT ? VRP / NT : 1;   // passes of the 512 threads over one channel slab
-  constexpr int KPP = VRP > NT ? 1 : NT / VRP;   // channels covered by one pass
-  constexpr int LAT = D3_LAT;               // tap steps between a load and its LDS write
-  static_assert(KC * VRP % NT == 0 && (NT % VRP == 0 || VRP % NT == 0), "slab must tile over the threads");
-  static_assert(9 % (LAT + 1) == 0, "the staging registers rotate with the tap index");
+  constexpr int WROWS = BM / Tile<BM>::WMN; // rows of a wavefront's tile
+  constexpr int TM = WROWS / 32;            // 32-row MFMA tiles per wavefront
+  constexpr int TAPS = R * R, O = (R - 1) / 2;
+  constexpr int DSLOTS = KC * CHS / NT;     // dy elements per thread per chunk
+  constexpr int SPT = (DSLOTS + TAPS - 1) / TAPS;   // dy slots fetched per tap step
+  constexpr int SUB = CHS > NT ? CHS / NT : 1;   // passes of the 512 threads over one channel slab
+  constexpr int KPP = CHS > NT ? 1 : NT / CHS;   // channels covered by one pass
+  constexpr int LAT = R == 3 ? 2 : 4;       // tap steps between a load and its LDS write
+  static_assert(NT % CHS == 0 || CHS % NT == 0, "slab must tile over the threads");
+  static_assert(TAPS % (LAT + 1) == 0, "the staging registers rotate with the tap index");
+  static_assert(!S2 || (R == 3 && BM == 64), "strided layers: 3x3, 64 channels per workgroup");
 
   extern __shared__ float smem[];
   float *Ws = smem;                         // [2][KC][PA]
@@ -108,9 +117,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
 
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = wave >> 2, wn = wave & 3;  // 2 x 4 wavefronts, 64 x 32 each
+  const int wm = wave / Tile<BM>::WNN, wn = wave % Tile<BM>::WNN;
   const int HW = a.H * a.W, PQ = a.P * a.Q;
-  const int VH = S2 ? a.P + 1 : a.P + 2;    // virtual rows per image: its dy rows plus the zero rows a tap can reach
+  const int VH = S2 ? a.P + 1 : a.P + 2 * O;    // virtual rows per image: its dy rows plus the zero rows a tap can reach
   const rsrc_t rdy = make_rsrc(a.dy, a.dy_bytes), rw = make_rsrc(a.wt, a.wt_bytes);
   const int nchunks = a.KP / KC;
 
@@ -139,34 +148,35 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
   const int c0 = (tile % a.ctiles) * BM;
   const int pix0 = (tile / a.ctiles) * BN;
 
-  // first virtual row of the slab: the row above the tile's first pixel row
+  // first virtual row of the slab: O rows above the tile's first pixel row
   const int n_first = pix0 / PQ, h_first = (pix0 - n_first * PQ) / a.Q;
-  const int vbase = n_first * VH + h_first;  // stride 1: virtual row of dy row (h_first - 1); stride 2: of row h_first
+  const int vbase = n_first * VH + h_first;  // stride 1: virtual row of dy row (h_first - O); stride 2: of row h_first
 
   // ---- dy slab loader ------------------------------------------------------------------------
   // slot e covers channel kc = (e / SUB) * KPP + tkc and slab element within = (e % SUB) * NT + tw:
-  // virtual row vr = within >> LOGP, column col = within % PITCHP; dy row p = (vbase + vr) % VH - 1
-  // of image (vbase + vr) / VH, dy column q = col - 1.  The byte offset splits into a thread part
+  // virtual row vr = within / pitch, column col = within % pitch; dy row p = (vbase + vr) % VH - O
+  // of image (vbase + vr) / VH, dy column q = col - O.  The byte offset splits into a thread part
   // g0 (kOOB for halo / padding elements) and the scalar (k0 + (e / SUB) * KPP) * P * Q * 4.
   // (Stride 2: no halo row above or column to the left, p = (vbase + vr) % VH, q = col.)
-  const int tkc = VRP > NT ? 0 : t / VRP, tw = VRP > NT ? t : t % VRP;
+  const int tkc = CHS > NT ? 0 : t / CHS, tw = CHS > NT ? t : t % CHS;
   int g0[SUB];
 #pragma unroll
   for (int sub = 0; sub < SUB; ++sub) {
-    const int within = sub * NT + tw, vr = within >> LOGP, col = within & (PITCHP - 1);
-    const int v = vbase + vr, n = v / VH, p = v - n * VH - (S2 ? 0 : 1), q = col - (S2 ? 0 : 1);
-    const bool ok = n < a.N && unsigned(p) < unsigned(a.P) && unsigned(q) < unsigned(a.Q);
+    const int within = sub * NT + tw, vr = within / a.pitch, col = within - vr * a.pitch;
+    const int v = vbase + vr, n = v / VH, p = v - n * VH - (S2 ? 0 : O), q = col - (S2 ? 0 : O);
+    const bool ok = vr < a.rows && n < a.N && unsigned(p) < unsigned(a.P) && unsigned(q) < unsigned(a.Q);
     g0[sub] = ok ? (((n * a.K + tkc) * a.P + p) * a.Q + q) * 4 : kOOB;
   }
   const int l0 = tkc * CHS + tw;
   auto dy_get = [&](int e, int k0) -> float {
-    return __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(rdy, g0[e % SUB] + (k0 + (e / SUB) * KPP) * PQ * 4, 0, 0));
+    int off = g0[e % SUB] + (k0 + (e / SUB) * KPP) * PQ * 4;
+    if (RAGK) off = tkc < a.K - k0 - (e / SUB) * KPP ? off : kOOB;
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdy, off, 0, 0));
   };
   auto dy_loff = [&](int e) -> int { return l0 + (e / SUB) * KPP * CHS + (e % SUB) * NT; };
 
   // ---- weight tile loader: one 128-bit load per thread per tap step ------------------------
-  // (BM == 64: the upper half of the threads has no weight element to fetch)
+  // (BM < 128: the upper threads have no weight element to fetch)
   constexpr int WV = BM / 4;                     // float4 per weight row
   const int w_kc = t / WV, w_m = (t % WV) * 4;   // 16 rows x WV float4
   const int w0 = (c0 + w_m + 3 < a.C) && (w_kc < KC) ? (w_kc * a.C + c0 + w_m) * 4 : kOOB;
@@ -174,17 +184,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
     return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rw, w0 + (tap * a.KP + k0) * a.C * 4, 0, 0));
   };
   auto w_put = [&](v4f v, float *dst) {
-    if (BM == 128 || wave < 4) *reinterpret_cast<v4f *>(dst + w_kc * PA + w_m) = v;
+    if (BM == 128 || wave < BM / 16) *reinterpret_cast<v4f *>(dst + w_kc * PA + w_m) = v;
   };
 
   // ---- this lane's pixel (B operand column) ------------------------------------------------
   const int pix = pix0 + wn * 32 + (lane & 31);
   const int pixc = pix < a.total_pix ? pix : a.total_pix - 1;  // a tail lane computes a valid pixel, stores nothing
   const int pn = pixc / PQ, prem = pixc - pn * PQ, ph_ = prem / a.Q, pw_ = prem - ph_ * a.Q;
-  // LDS offset of tap (r = 2, s = 2); tap (r, s) adds (2 - r) * PITCHP + (2 - s):
-  //   dy row h + 1 - r  ->  virtual row pn*VH + h + 2 - r ; slab column of q = w + 1 - s is w + 2 - s
-  const int boff = (pn * VH + ph_ - vbase) * PITCHP + pw_ + (lane >> 5) * CHS;
-  const int aoff = (lane >> 5) * PA + wm * (BM / 2) + (lane & 31);
+  // LDS offset of tap (R - 1, R - 1); tap (r, s) adds (R - 1 - r) * pitch + (R - 1 - s):
+  //   dy row h + O - r  ->  virtual row pn*VH + h + 2 O - r ; slab column of q = w + O - s is w + 2 O - s
+  const int boff = (pn * VH + ph_ - vbase) * a.pitch + pw_ + (lane >> 5) * CHS;
+  const int aoff = (lane >> 5) * PA + wm * WROWS + (lane & 31);
 
   v16f acc[NCLS * TM];
 #pragma unroll
@@ -192,19 +202,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
 
-  // Staging registers.  Step q (tap q % 9 of chunk q / 9) requests what step q + LAT writes: the
+  // Staging registers.  Step q (tap q % TAPS of chunk q / TAPS) requests what step q + LAT writes: the
   // weights of step q + LAT + 1 and dy slots [td * SPT, (td + 1) * SPT) of the chunk after step
-  // q + LAT's, td = (q + LAT) % 9.  Requests past the last chunk land in buffers nobody reads.
+  // q + LAT's, td = (q + LAT) % TAPS.  Requests past the last chunk land in buffers nobody reads.
   v4f wst[LAT + 1];
   float dst[LAT + 1][SPT];
   auto request = [&](int tq, int ch) {  // tq: tap index relative to chunk ch (negative during warm-up)
     const int slot = ((tq % (LAT + 1)) + LAT + 1) % (LAT + 1);
     const int qw = tq + LAT + 1, qd = tq + LAT;
-    wst[slot] = w_get(qw % 9, (ch + qw / 9) * KC);
+    wst[slot] = w_get(qw % TAPS, (ch + qw / TAPS) * KC);
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
-      const int e = (qd % 9) * SPT + j;
-      if (e < DSLOTS) dst[slot][j] = dy_get(e, (ch + 1 + qd / 9) * KC);
+      const int e = (qd % TAPS) * SPT + j;
+      if (e < DSLOTS) dst[slot][j] = dy_get(e, (ch + 1 + qd / TAPS) * KC);
     }
   };
 
@@ -222,15 +232,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
     const float *dys = dyS + dcur * (KC * CHS) + boff;
     float *dyn = dyS + (dcur ^ 1) * (KC * CHS);
 #pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      const int r = tap / 3, s = tap - r * 3;
-      const int toff = S2 ? (r == 0) * PITCHP + (s == 0) : (2 - r) * PITCHP + (2 - s);
+    for (int tap = 0; tap < TAPS; ++tap) {
+      const int r = tap / R, s = tap - r * R;
+      const float *drow = S2 ? dys + (r == 0) * a.pitch + (s == 0) : dys + (R - 1 - r) * a.pitch + (R - 1 - s);
       const int cls = S2 ? 2 * (r != 1) + (s != 1) : 0;
       const float *ws = Ws + wcur * (KC * PA) + aoff;
       request(tap, ch);
 #pragma unroll
       for (int kk = 0; kk < KC; kk += 2) {
-        const float b = dys[kk * CHS + toff];
+        const float b = drow[kk * CHS];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
           acc[cls * TM + i] =
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
     dcur ^= 1;
   }
 
-  // epilogue.  A finished tile goes to dx[n][c][h][w] (this lane's pixel, rows c0 + wm*(BM/2) + i*32 +
+  // epilogue.  A finished tile goes to dx[n][c][h][w] (this lane's pixel, rows c0 + wm*WROWS + i*32 +
   // 8*(v/4) + 4*(lane/32) + v%4); an incomplete one to this workgroup's partial slot as
   // [class][row][pixel], to be summed by k_dgrad3x3_fixup.
   // (the lane term is laundered through an empty asm so that the epilogue's address arithmetic is
@@ -259,7 +269,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
   asm volatile("" : "+v"(lhalf));
   if (!whole) {
     float *ps = a.partials + (size_t(sk_g) * 2 + (tile_rel == first_tile ? 0 : 1)) * (NCLS * BM * BN) +
-                (wm * (BM / 2) + 4 * lhalf) * BN + wn * 32 + (lane & 31);
+                (wm * WROWS + 4 * lhalf) * BN + wn * 32 + (lane & 31);
 #pragma unroll
     for (int cl = 0; cl < NCLS; ++cl)
 #pragma unroll
@@ -274,7 +284,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int c = c0 + wm * (BM / 2) + i * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3);
+          const int c = c0 + wm * WROWS + i * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3);
           if (c < a.C) {
             const float bb = a.bias ? a.bias[c] : 0.f;
             float *oc = o + size_t(c) * HW;
@@ -291,7 +301,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int c = c0 + wm * (BM / 2) + i * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3);
+          const int c = c0 + wm * WROWS + i * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3);
           if (c < a.C) {
             float r = a.bias ? acc[i][v] + a.bias[c] : acc[i][v];
             if (a.accumulate) r += o[size_t(c) * HW];
@@ -312,7 +322,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 4))) void
 // instead of 11.3 us)
 template <int BM, bool S2, class I>
 __device__ __forceinline__ void dgrad3x3_fixup_body(const D3Args &a) {
-  constexpr int NCLS = S2 ? 4 : 1;
+  constexpr int NCLS = S2 ? 4 : 1, BN = Tile<BM>::BN, TPR = BN / 4;   // TPR: threads per row
   const int nchunks = a.KP / KC;
   const int r = blockIdx.x;
   const I x0 = I(r) * I(nchunks), x1 = x0 + I(nchunks) - 1;
@@ -329,10 +339,10 @@ __device__ __forceinline__ void dgrad3x3_fixup_body(const D3Args &a) {
   const int tile = a.dp_tiles + r;
   const int c0 = (tile % a.ctiles) * BM, pix0 = (tile / a.ctiles) * BN;
   const int HW = a.H * a.W, PQ = a.P * a.Q;
-  // a block covers 8 rows of the tile, a thread 4 consecutive pixels of one row
+  // a block covers 256 / TPR rows of the tile, a thread 4 consecutive pixels of one row
   typedef float v4f __attribute__((ext_vector_type(4)));
   typedef float v2f __attribute__((ext_vector_type(2)));
-  const int m = blockIdx.y * 8 + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 4;
+  const int m = blockIdx.y * (256 / TPR) + threadIdx.x / TPR, col = threadIdx.x % TPR * 4;
   const int c = c0 + m;
   if (c >= a.C) return;
   v4f s[NCLS];
@@ -378,8 +388,8 @@ __global__ __launch_bounds__(256) void k_dgrad3x3_fixup(D3Args a) {
 }
 
 struct D3Plan {
-  bool ok, s2;
-  int bm, logp, vr;
+  bool ok, s2, ragk;
+  int bm, bn, r, chs, pitch, rows;
   int ctiles, tiles, dp_tiles, sk_wgs;  // whole-tile workgroups, then sk_wgs workgroups sharing the rest
   long sk_units;
   size_t lds;
@@ -388,42 +398,36 @@ struct D3Plan {
 inline D3Plan plan(const sgh_conv_geom *g) {
   D3Plan p{};
   p.ok = false;
-  if (g->R != 3 || g->S != 3 || g->pad_h != 1 || g->pad_w != 1 || g->stride_h != g->stride_w) return p;
+  if ((g->R != 3 && g->R != 5) || g->S != g->R || g->stride_h != g->stride_w) return p;
+  const int o = (g->R - 1) / 2;
+  if (g->pad_h != o || g->pad_w != o) return p;
+  p.r = g->R;
   p.s2 = g->stride_h == 2;
   if (g->stride_h != 1 && !p.s2) return p;
-  if (p.s2 && (g->H != 2 * g->P || g->W != 2 * g->Q)) return p;  // even image: four residue classes of equal size
-  if (g->C < 64 || g->C % 4 != 0 || g->K % KC != 0 || g->Q < 2) return p;
+  if (p.s2 && (p.r != 3 || g->H != 2 * g->P || g->W != 2 * g->Q)) return p;  // even image: four residue classes of equal size
+  if (g->C < 16 || g->C % 4 != 0 || g->K < 8 || g->Q < 2) return p;
   if (sgh_env().dgrad3x3_off) return p;
-  // slab columns: stride 1 has a halo column on both sides, stride 2 one zero column on the right
-  const int cols = p.s2 ? g->Q + 1 : g->Q + 2;
-  if (cols > 64) return p;
-  p.logp = cols <= 8 ? 3 : (cols <= 16 ? 4 : (cols <= 32 ? 5 : 6));
-  if (!p.s2 && p.logp < 4) p.logp = 4;
-  // virtual rows a 128-pixel tile can touch: its pixel rows, the halo rows (stride 1: one each
-  // side; stride 2: one below), and the zero rows of every image boundary it crosses
-  const int rows = (BN + g->Q - 2) / g->Q + 1;
-  const int crossings = (BN - 1) / (g->P * g->Q) + 1;
-  const int need = p.s2 ? rows + 1 + crossings : rows + 2 + 2 * crossings;
-  if (p.s2) {
-    // instantiated: pitch 32 x 8 rows, pitch 16 x 16 rows, pitch 8 x 32 rows (256 floats per channel)
-    if (p.logp == 6) return p;
-    p.vr = 256 >> p.logp;
-    p.bm = 64;  // four classes x 16 accumulators per 32-row tile: the 64-row tile keeps two workgroups per CU
-  } else {
-    if (p.logp == 6) p.vr = 8;
-    else if (p.logp == 5) p.vr = 16;
-    else p.vr = need <= 16 ? 16 : 32;
-    p.bm = (g->C % 128 == 0 || g->C > 192) ? 128 : 64;
-    if (sgh_env().dgrad3x3_bm) p.bm = sgh_env().dgrad3x3_bm;
-  }
-  if (need > p.vr) return p;
-  const size_t chs = size_t(p.vr) * (1u << p.logp);
-  p.lds = (size_t(2) * KC * (p.bm) + size_t(2) * KC * chs) * sizeof(float);
+  p.ragk = g->K % KC != 0;
+  // four classes x 16 accumulators per 32-row tile: the 64-row tile keeps two workgroups per CU
+  p.bm = p.s2 ? 64 : g->C <= 32 ? 32 : (g->C % 128 == 0 || g->C > 192) && p.r == 3 ? 128 : 64;
+  if (!p.s2 && sgh_env().dgrad3x3_bm && p.r == 3) p.bm = sgh_env().dgrad3x3_bm;
+  p.bn = p.bm == 32 ? Tile<32>::BN : Tile<64>::BN;
+  // slab columns: stride 1 has halo columns on both sides, stride 2 one zero column on the right
+  p.pitch = p.s2 ? g->Q + 1 : g->Q + 2 * o;
+  // virtual rows a tile can touch: its pixel rows, the halo rows (stride 1: on both sides; stride 2: one below),
+  // and the zero rows of every image boundary it crosses
+  const int rows = (p.bn + g->Q - 2) / g->Q + 1;
+  const int crossings = (p.bn - 1) / (g->P * g->Q) + 1;
+  p.rows = p.s2 ? rows + 1 + crossings : rows + 2 * o + 2 * o * crossings;
+  const long floats = long(p.rows) * p.pitch;
+  p.chs = floats <= 256 ? 256 : floats <= 512 ? 512 : 1024;
+  if (floats > (p.s2 ? 512 : 1024)) return p;
+  p.lds = (size_t(2) * KC * p.bm + size_t(2) * KC * p.chs) * sizeof(float);
   if (p.lds > 160 * 1024) return p;
   const size_t lim = size_t(1) << 31;
   const size_t dx_elems = size_t(g->N) * g->C * g->H * g->W;
   if (size_t(g->N) * g->K * g->P * g->Q * 4 >= lim || dx_elems * 4 >= lim) return p;
-  if (size_t(g->N) * (g->P + 2) + p.vr >= lim / 64) return p;
+  if (size_t(g->N) * (g->P + 2 * o) + p.rows >= lim / 64) return p;
   // Work balance.  Whole multiples of the CU count of tiles run one tile per workgroup; the
   // remaining tiles (all of them when there are fewer tiles than CUs) are cut into (tile, chunk)
   // units and dealt evenly to one workgroup per CU (two per CU measured slower: twice the
@@ -432,7 +436,7 @@ inline D3Plan plan(const sgh_conv_geom *g) {
   const int cus = sgh_num_cus();
   const int nchunks = (g->K + KC - 1) / KC;
   p.ctiles = (g->C + p.bm - 1) / p.bm;
-  const long tiles = long(p.ctiles) * ((long(g->N) * g->P * g->Q + BN - 1) / BN);
+  const long tiles = long(p.ctiles) * ((long(g->N) * g->P * g->Q + p.bn - 1) / p.bn);
   if (tiles >= (long(1) << 30)) return p;
   p.tiles = int(tiles);
   p.dp_tiles = int(tiles / cus * cus);
@@ -442,9 +446,9 @@ inline D3Plan plan(const sgh_conv_geom *g) {
   return p;
 }
 
-template <int BM, int LOGP, int VR, bool S2>
+template <int BM, int CHS, bool S2, int R, bool RAGK>
 int launch(const D3Args &a, const D3Plan &p, dim3 grid, hipStream_t s) {
-  auto kern = k_dgrad3x3<BM, LOGP, VR, S2>;
+  auto kern = k_dgrad3x3<BM, CHS, S2, R, RAGK>;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -464,7 +468,7 @@ bool sgh_dgrad3x3_supported(const sgh_conv_geom *g) { return plan(g).ok; }
 size_t sgh_dgrad3x3_partial_bytes(const sgh_conv_geom *g) {
   const D3Plan p = plan(g);
   if (!p.ok || p.sk_wgs == 0) return 0;
-  return size_t(p.sk_wgs) * 2 * (p.s2 ? 4 : 1) * p.bm * BN * sizeof(float);
+  return size_t(p.sk_wgs) * 2 * (p.s2 ? 4 : 1) * p.bm * p.bn * sizeof(float);
 }
 
 // `wt` holds the weights re-laid as [tap][KP][C] (KP = K rounded up to 16, zero rows beyond K);
@@ -486,6 +490,8 @@ int sgh_dgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *wt, i
   a.W = g->W;
   a.K = g->K;
   a.KP = KP;
+  a.pitch = p.pitch;
+  a.rows = p.rows;
   a.P = g->P;
   a.Q = g->Q;
   a.total_pix = g->N * g->P * g->Q;
@@ -496,33 +502,31 @@ int sgh_dgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *wt, i
   a.sk_units = p.sk_units;
   a.partials = partials;
   a.dy_bytes = unsigned(size_t(g->N) * g->K * g->P * g->Q * 4);
-  a.wt_bytes = unsigned(size_t(9) * KP * g->C * 4);
+  a.wt_bytes = unsigned(size_t(p.r) * p.r * KP * g->C * 4);
   dim3 grid(unsigned(p.dp_tiles + p.sk_wgs), 1, 1);
   int rc = SGH_EUNSUPPORTED;
-  sgh_prof_kernel_begin(tag, 2.0 * g->N * g->K * g->P * g->Q * g->C * 9);
-#define D3_CASE(BM_, LOGP_, VR_) \
-  if (!p.s2 && p.bm == BM_ && p.logp == LOGP_ && p.vr == VR_) rc = launch<BM_, LOGP_, VR_, false>(a, p, grid, s);
-#define D3_CASE_S2(LOGP_, VR_) \
-  if (p.s2 && p.bm == 64 && p.logp == LOGP_ && p.vr == VR_) rc = launch<64, LOGP_, VR_, true>(a, p, grid, s);
-  D3_CASE(128, 6, 8)
-  D3_CASE(64, 6, 8)
-  D3_CASE(128, 5, 16)
-  D3_CASE(64, 5, 16)
-  D3_CASE(128, 4, 16)
-  D3_CASE(64, 4, 16)
-  D3_CASE(128, 4, 32)
-  D3_CASE(64, 4, 32)
-  D3_CASE_S2(5, 8)
-  D3_CASE_S2(4, 16)
-  D3_CASE_S2(3, 32)
+  sgh_prof_kernel_begin(tag, 2.0 * g->N * g->K * g->P * g->Q * g->C * p.r * p.r);
+#define D3_CASE(BM_, CHS_, S2_, R_)                                             \
+  if (p.bm == BM_ && p.chs == CHS_ && p.s2 == S2_ && p.r == R_)                 \
+    rc = p.ragk ? launch<BM_, CHS_, S2_, R_, true>(a, p, grid, s) : launch<BM_, CHS_, S2_, R_, false>(a, p, grid, s);
+#define D3_CASES(BM_, R_) \
+  D3_CASE(BM_, 256, false, R_) D3_CASE(BM_, 512, false, R_) D3_CASE(BM_, 1024, false, R_)
+  D3_CASES(32, 3)
+  D3_CASES(64, 3)
+  D3_CASES(128, 3)
+  D3_CASES(32, 5)
+  D3_CASES(64, 5)
+  D3_CASE(64, 256, true, 3)
+  D3_CASE(64, 512, true, 3)
+#undef D3_CASES
 #undef D3_CASE
-#undef D3_CASE_S2
   sgh_prof_kernel_end(s);
   if (rc != SGH_OK) return rc;
   if (p.sk_wgs > 0) {
     const int shared_tiles = p.tiles - p.dp_tiles;
-    const dim3 fgrid(shared_tiles, p.bm / 8);
+    const dim3 fgrid(shared_tiles, p.bm * p.bn / 1024);
     if (p.s2) hipLaunchKernelGGL((k_dgrad3x3_fixup<64, true>), fgrid, dim3(256), 0, s, a);
+    else if (p.bm == 32) hipLaunchKernelGGL((k_dgrad3x3_fixup<32, false>), fgrid, dim3(256), 0, s, a);
     else if (p.bm == 64) hipLaunchKernelGGL((k_dgrad3x3_fixup<64, false>), fgrid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((k_dgrad3x3_fixup<128, false>), fgrid, dim3(256), 0, s, a);
     if (hipGetLastError() != hipSuccess) return SGH_EINVAL;

@@ -836,21 +836,20 @@ inline DgradPath dgrad_path(const sgh_conv_geom *g) {
   // 1x1 without padding: a plain GEMM over the output pixels whose store dilates by the stride
   if (RS == 1 && g->pad_h == 0 && g->pad_w == 0 && g->C >= 32 && !sgh_env().dgrad_pointwise_off)
     return kDgradPointwise;
+  if (sgh_dgrad3x3_supported(g)) return kDgradTile3x3;
   // few input channels: the C x pixels output tile would waste most of a 64-row MFMA tile, so run
   // the dense GEMM dcol = W^T * dy (CRS rows) and fold the columns back with a gather
   if (g->C < 32 && RS * g->C * size_t(g->N) * g->P * g->Q * sizeof(float) < kMaxOperandBytes) return kDgradColumns;
-  if (sgh_dgrad3x3_supported(g)) return kDgradTile3x3;
   if (g->stride_h * g->stride_w <= kMaxClasses && RS <= size_t(kMaxTaps)) return kDgradClasses;
   return kDgradGather;
 }
 
 inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
-// A 3x3 stride-1 pad-1 forward convolution is the data gradient of the channel-swapped problem
+// A stride-1 forward convolution with "same" padding is the data gradient of the channel-swapped problem
 // with the filter taps reversed; `gt` receives that problem when the shared-tile kernel covers it.
 inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
-  if (g->R != 3 || g->S != 3 || g->stride_h != 1 || g->stride_w != 1 || g->pad_h != 1 || g->pad_w != 1) return false;
-  if (g->C % BK != 0) return false;  // the reduction (input channels) runs in whole chunks
+  if (g->stride_h != 1 || g->stride_w != 1) return false;
   *gt = *g;
   gt->C = g->K;
   gt->K = g->C;

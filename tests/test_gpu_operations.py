@@ -793,3 +793,43 @@ def test_conv_bias_gradient_vs_float64(singa, dev, kind, shape):
     want, mass = dy.sum(axis=(0, 2, 3)), np.abs(dy).sum(axis=(0, 2, 3))
     ulp = {"f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[kind]
     assert np.all(np.abs(got - want) <= 40 * 2.0 ** -24 * mass + ulp * np.abs(want))
+
+
+@pytest.mark.parametrize("case", [
+    # N, C, H, W, K, R, stride: dgrad on C output rows reduced over K, forward on K rows reduced over C
+    (2, 64, 40, 40, 64, 3, 1),       # planes wider than 32: 512 floats of slab per channel
+    (1, 64, 20, 110, 64, 3, 1),      # ... 1024 floats
+    (3, 128, 5, 5, 136, 3, 1),       # tiles over seven images; 136 = eight chunks and a half
+    (7, 64, 2, 2, 64, 3, 1),         # more image boundaries than pixel rows
+    (2, 32, 17, 19, 24, 3, 1),       # 32-row tiles, odd planes, 24 = a chunk and a half
+    (3, 20, 12, 9, 16, 3, 1),        # 20 of 32 rows
+    (2, 36, 16, 16, 72, 3, 1),       # 36 of 64 rows
+    (5, 32, 16, 16, 64, 5, 1),       # 5 x 5
+    (2, 16, 7, 9, 40, 5, 1),         # 5 x 5 on small odd planes, both sides ragged
+    (1, 64, 33, 47, 32, 5, 1),       # 5 x 5, 1024 floats
+    (2, 64, 80, 80, 64, 3, 2),       # stride 2: 512 floats
+    (3, 64, 10, 10, 72, 3, 2),       # stride 2, ragged reduction
+    (2, 20, 14, 6, 8, 3, 2),         # stride 2, 20 of 64 rows, half a chunk
+])
+def test_shared_tile_convolution_edges(singa, dev, case):
+    """The shared-tile data gradient / forward kernel at the edges of what it covers: slab sizes, row tiles, ragged reductions,
+    5 x 5 filters, strided layers; against the oracle, the sum into an existing gradient bit-identical to the separate add."""
+    N, C, H, W, K, R, stride = case
+    print("shared tile", case, flush=True)
+    r = rng(sum(case))
+    p = (R - 1) // 2
+    x = randn(r, N, C, H, W)
+    w = (randn(r, K, C, R, R) * np.sqrt(2.0 / (C * R * R))).astype(np.float32)
+    b = randn(r, K)
+    xd, wd, bd = (singa.from_numpy(v, dev) for v in (x, w, b))
+    h = singa.CudnnConvHandle(xd, (R, R), (stride, stride), (p, p), C, K, True)
+    y_o = O.conv_fwd(x, w, b, (stride, stride), (p, p))
+    assert nl2(singa.GpuConvForward(xd, wd, bd, h).to_numpy(), y_o) < 1e-5
+    dy = randn(r, *y_o.shape)
+    dyd = singa.from_numpy(dy, dev)
+    dx_o, _ = O.conv_bwd(dy, x, w, (stride, stride), (p, p))
+    dx = singa.GpuConvBackwardx(dyd, wd, xd, h)
+    assert nl2(dx.to_numpy(), dx_o) < 1e-5
+    into = singa.from_numpy(x, dev)
+    got = singa.GpuConvBackwardxAccumulate(dyd, wd, xd, h, into).to_numpy()
+    assert_bit_equal(got, (dx.to_numpy() + x).astype(np.float32), "dx += dgrad")
