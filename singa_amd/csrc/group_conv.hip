@@ -15,6 +15,7 @@
 // in registers and adds them over its threads; the chunks' sums are added in chunk order by a second kernel, so results
 // are the same on every run.
 #include "common.h"
+#include "fastdiv.h"
 #include "storage.h"
 
 namespace {
@@ -26,16 +27,6 @@ constexpr int kLdsMost = 64 * 1024;
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
-// n / d for 0 <= n < 2^31 with a multiplication: q = (mulhi(n, m) + n) >> s
-struct FastDiv {
-  unsigned d, m, s;
-  explicit FastDiv(unsigned d_ = 1) : d(d_), m(0), s(0) {
-    while ((1ull << s) < d) ++s;
-    m = unsigned(((1ull << 32) * ((1ull << s) - d)) / d + 1);
-  }
-  __device__ __forceinline__ int div(int n) const { return int((__umulhi(unsigned(n), m) + unsigned(n)) >> s); }
-};
-
 struct GroupArgs {
   int units, G;                 // N * G; groups
   int cs, cd;                   // channels per group of the source and of the destination
@@ -45,7 +36,7 @@ struct GroupArgs {
   int UB;                       // units per workgroup
   bool flip;                    // data gradient: reversed taps, filters indexed [source][destination]
   unsigned src_bytes;
-  FastDiv d_vc, d_vr, d_cs, d_dw, d_strips, d_cd, d_dil, d_G, d_taps;
+  sgh_fastdiv d_vc, d_vr, d_cs, d_dw, d_strips, d_cd, d_dil, d_G, d_taps;
 };
 
 template <class S>
@@ -256,9 +247,9 @@ bool plan_tile(GroupArgs *a, int R, int T, int channels, int out_channels, size_
   if (ub > fit) ub = fit;
   if (ub > most) ub = most;
   a->UB = ub < 1 ? 1 : int(ub);
-  a->d_vc = FastDiv(a->VC), a->d_vr = FastDiv(a->VR), a->d_cs = FastDiv(a->cs), a->d_dw = FastDiv(a->DW);
-  a->d_strips = FastDiv(strips), a->d_cd = FastDiv(a->cd), a->d_dil = FastDiv(a->dil), a->d_G = FastDiv(a->G);
-  a->d_taps = FastDiv(R * R);
+  a->d_vc = sgh_fastdiv(a->VC), a->d_vr = sgh_fastdiv(a->VR), a->d_cs = sgh_fastdiv(a->cs), a->d_dw = sgh_fastdiv(a->DW);
+  a->d_strips = sgh_fastdiv(strips), a->d_cd = sgh_fastdiv(a->cd), a->d_dil = sgh_fastdiv(a->dil), a->d_G = sgh_fastdiv(a->G);
+  a->d_taps = sgh_fastdiv(R * R);
   return true;
 }
 

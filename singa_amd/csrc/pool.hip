@@ -6,6 +6,7 @@
 // own element.  The additions therefore happen in exactly the order of the CPU scatter loop, so
 // dx is bit-identical to it and no atomics are needed.
 #include "common.h"
+#include "fastdiv.h"
 #include "storage.h"
 
 namespace {
@@ -113,6 +114,316 @@ __global__ __launch_bounds__(kBlock) void k_pool_max_bwd(const typename S::elem 
       for (int q = q_lo; q <= q_hi; ++q)
         if (window_argmax<S>(xb, g, p, q, nullptr) == r) s += S::ld(db + p * g.Q + q);
     S::st(dx + i, s);
+  }
+}
+
+// ---- 3 x 3 windows, stride 2, padding 1 (the residual networks' pooling layer) on planes of any size ------------------
+// One lane per window column, everything in registers: a lane loads the pair (2 q, 2 q + 1) of an x row -- four bytes of
+// 16-bit elements, eight of fp32, the lanes of a row contiguous, at whatever alignment the row has -- and takes element 2 q - 1
+// from the lane before it.  GROUP lanes form a strip of up to kStrip window rows of one plane (8, 16, 32 or 64 by the plane's
+// width, so that narrow planes do not leave lanes idle); the loads of a strip are all requested before the first is used.
+// Rows or columns outside the image read as -inf, which no comparison selects.  Planes wider than GROUP windows are cut
+// into chunks that overlap by one lane on either side.
+//
+// The kernels that the odd sizes ran before staged elements one by one in LDS (backward) or gave every output its own nine
+// loads (forward): bfloat16 50 x 72 x 57 x 43, 40.7 + 18.8 us; here 17.6 + 9.2.  Backward of the residual networks' stem (N x 64 x 112 x 112)
+// against rows staged in LDS as whole vectors: bfloat16 N = 64 65.8 -> 53.0, 128 125 -> 107, fp32 N = 64 82.3 -> 82.8.
+constexpr int kStrip = 7;
+constexpr float kLowest = -3.402823466e38f;
+
+struct RowBest {
+  float m;
+  int k;   // column within the window (0..2), 64 = none
+};
+
+__device__ __forceinline__ RowBest best_of(float a, float b, float c) {   // first maximum of a window's row
+  RowBest r{kLowest, 64};
+  if (a > r.m) r.m = a, r.k = 0;
+  if (b > r.m) r.m = b, r.k = 1;
+  if (c > r.m) r.m = c, r.k = 2;
+  return r;
+}
+
+struct StripG {
+  int H, W, P, Q;
+  int rows;               // window rows per strip
+  int strips, chunks;     // per plane
+  int units;              // planes * strips * chunks
+  unsigned x_bytes, y_bytes;
+  sgh_fastdiv d_chunks, d_strips;
+};
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+// Two neighbouring elements as stored; `ok` false: nothing is read
+template <class S>
+struct Pair {
+  typedef typename S::elem elem;
+  float lo, hi;
+  static __device__ __forceinline__ Pair load(rsrc_t r, int elem_index, bool ok) {
+    const int off = ok ? elem_index * int(sizeof(elem)) : int(0x80000000u);
+    if constexpr (sizeof(elem) == 4) {
+      typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+      const u2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+      const unsigned a = v[0], b = v[1];   // (copies: a bit cast of a vector's element takes element 0)
+      return Pair{__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
+    } else {
+      const unsigned v = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+      const elem a = elem(v & 0xffffu), b = elem(v >> 16);
+      return Pair{S::ld(&a), S::ld(&b)};
+    }
+  }
+};
+
+template <class S>
+__device__ __forceinline__ float ld_one(rsrc_t r, int elem_index, bool ok) {
+  typedef typename S::elem elem;
+  const int off = ok ? elem_index * int(sizeof(elem)) : int(0x80000000u);
+  if constexpr (sizeof(elem) == 4) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  else {
+    const elem e = __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
+    return S::ld(&e);
+  }
+}
+
+// What the lanes of a wavefront work on: strip of `rows` window rows from p0 of plane `plane`, window column q
+template <int GROUP>
+struct Strip {
+  int plane, p0, q;
+  bool live, inside, makes;   // a strip at all; the window exists; this lane produces its results (not a halo lane)
+  __device__ __forceinline__ Strip(const StripG &g) {
+    const int lane = threadIdx.x & 63, l = lane & (GROUP - 1);
+    const int unit = (int(blockIdx.x) * (kBlock / 64) + int(threadIdx.x >> 6)) * (64 / GROUP) + lane / GROUP;
+    live = unit < g.units;
+    const int u = live ? unit : 0;
+    const int t = g.d_chunks.div(u), chunk = u - t * g.chunks;
+    plane = g.d_strips.div(t);
+    p0 = (t - plane * g.strips) * g.rows;
+    const bool halo = g.chunks > 1;
+    q = halo ? chunk * (GROUP - 2) + l - 1 : l;
+    inside = live && q >= 0 && q < g.Q;
+    makes = inside && (!halo || (l > 0 && l < GROUP - 1));
+  }
+};
+
+// The three elements of x row h that window column q reads
+template <class S, int GROUP>
+struct Row3 {
+  float a, b, c;
+  // requested: the pair (2 q, 2 q + 1), or in a last column of an odd row the pair before it
+  static __device__ __forceinline__ Pair<S> request(rsrc_t x, const StripG &g, const Strip<GROUP> &s, int h) {
+    const bool ok = s.inside && h >= 0 && h < g.H;
+    const int w = 2 * s.q + 1 < g.W ? 2 * s.q : 2 * s.q - 1;
+    return Pair<S>::load(x, (s.plane * g.H + h) * g.W + w, ok);
+  }
+  __device__ __forceinline__ Row3(const Pair<S> &v, const StripG &g, const Strip<GROUP> &s, int h) {
+    const float none = -__builtin_inff();
+    const bool ok = s.inside && h >= 0 && h < g.H, whole = 2 * s.q + 1 < g.W;
+    b = !ok ? none : whole ? v.lo : v.hi;
+    c = ok && whole ? v.hi : none;
+    const float left = __shfl_up(c, 1, GROUP);
+    a = s.q > 0 && (threadIdx.x & (GROUP - 1)) != 0 ? left : none;
+    if (!ok) a = none;
+  }
+};
+
+// a 2 x 2 block of dx, two neighbouring elements per store; `below` / `right`: whether the second row / column exists
+template <class S>
+__device__ __forceinline__ void store_block(typename S::elem *o, int W, bool below, bool right, float o00, float o01, float o10,
+                                            float o11) {
+  typedef typename S::elem elem;
+  elem e[4];
+  S::st(e, o00), S::st(e + 1, o01), S::st(e + 2, o10), S::st(e + 3, o11);
+  if (right) {   // (at the alignment of an element)
+    if constexpr (sizeof(elem) == 4) {
+      typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
+      *reinterpret_cast<pair *>(o) = pair{e[0], e[1]};
+      if (below) *reinterpret_cast<pair *>(o + W) = pair{e[2], e[3]};
+    } else {
+      typedef unsigned pair __attribute__((aligned(2)));
+      *reinterpret_cast<pair *>(o) = unsigned(e[0]) | (unsigned(e[1]) << 16);
+      if (below) *reinterpret_cast<pair *>(o + W) = unsigned(e[2]) | (unsigned(e[3]) << 16);
+    }
+  } else {
+    o[0] = e[0];
+    if (below) o[W] = e[2];
+  }
+}
+
+template <class S, int GROUP>
+__global__ __launch_bounds__(kBlock) void k_pool_max_fwd_strip(const typename S::elem *__restrict__ x,
+                                                              typename S::elem *__restrict__ y, const StripG g) {
+  typedef typename S::elem elem;
+  const Strip<GROUP> s(g);
+  const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, g.x_bytes, 0x00020000);
+  constexpr int NR = 2 * kStrip + 1;
+  Pair<S> v[NR];
+  const int h0 = 2 * s.p0 - 1;
+#pragma unroll
+  for (int j = 0; j < NR; ++j) v[j] = Row3<S, GROUP>::request(xr, g, s, j <= 2 * g.rows ? h0 + j : -1);
+  elem *out = y + (size_t(s.plane) * g.P + s.p0) * g.Q + s.q;
+  const Row3<S, GROUP> r0(v[0], g, s, h0);
+  float top = best_of(r0.a, r0.b, r0.c).m;
+#pragma unroll
+  for (int k = 0; k < kStrip; ++k) {
+    const Row3<S, GROUP> rm(v[2 * k + 1], g, s, h0 + 2 * k + 1), rb(v[2 * k + 2], g, s, h0 + 2 * k + 2);
+    const float mid = best_of(rm.a, rm.b, rm.c).m, bot = best_of(rb.a, rb.b, rb.c).m;
+    float best = top;
+    if (mid > best) best = mid;
+    if (bot > best) best = bot;
+    top = bot;
+    if (s.makes && k < g.rows && s.p0 + k < g.P) S::st(out + size_t(k) * g.Q, best);
+  }
+}
+
+// The dx block (rows 2 i, 2 i + 1; columns 2 j, 2 j + 1) can only receive from windows (i, j), (i, j + 1), (i + 1, j),
+// (i + 1, j + 1), and only at fixed positions of those windows:
+//   * window p shares its top row with window p - 1's bottom row: the per-row first maximum (strict '>',
+//     left to right) is computed once per x row, and three of them combine top to bottom -- the same winner
+//     as the row-major scan of the CPU loop;
+//   * the winner is kept as a code 3 * dh + dw; the right-hand neighbour's code and dy come from lane + 1;
+//   * a block's four elements add the dy of the windows whose code names them, in ascending (p, q) order
+//     starting from +0.0, exactly the additions of the CPU's scatter loop.
+// A strip also computes the window row below it.
+template <class S, int GROUP>
+__global__ __launch_bounds__(kBlock) void k_pool_max_bwd_strip(const typename S::elem *__restrict__ dy,
+                                                              const typename S::elem *__restrict__ x,
+                                                              typename S::elem *__restrict__ dx, const StripG g) {
+  typedef typename S::elem elem;
+  const Strip<GROUP> s(g);
+  const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, g.x_bytes, 0x00020000);
+  const rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(dy), 0, g.y_bytes, 0x00020000);
+  constexpr int NR = 2 * kStrip + 3;
+  Pair<S> v[NR];
+  float d[kStrip + 1];
+  const int h0 = 2 * s.p0 - 1;
+#pragma unroll
+  for (int k = 0; k <= kStrip; ++k)
+    d[k] = ld_one<S>(yr, (s.plane * g.P + s.p0 + k) * g.Q + s.q, s.inside && k <= g.rows && s.p0 + k < g.P);
+#pragma unroll
+  for (int j = 0; j < NR; ++j) v[j] = Row3<S, GROUP>::request(xr, g, s, j <= 2 * g.rows + 2 ? h0 + j : -1);
+  const bool last = (threadIdx.x & (GROUP - 1)) == GROUP - 1;   // no lane to the right (a halo lane, or the plane's last window)
+  const Row3<S, GROUP> r0(v[0], g, s, h0);
+  RowBest top = best_of(r0.a, r0.b, r0.c);
+  int code_p = 64, ncode_p = 64;
+  float dy_p = 0.f, ndy_p = 0.f;
+#pragma unroll
+  for (int k = 0; k <= kStrip; ++k) {
+    const Row3<S, GROUP> rm(v[2 * k + 1], g, s, h0 + 2 * k + 1), rb(v[2 * k + 2], g, s, h0 + 2 * k + 2);
+    const RowBest mid = best_of(rm.a, rm.b, rm.c), bot = best_of(rb.a, rb.b, rb.c);
+    float best = top.m;
+    int code = top.k;
+    if (mid.m > best) best = mid.m, code = 3 + mid.k;
+    if (bot.m > best) code = 6 + bot.k;
+    if (!s.inside || s.p0 + k >= g.P || k > g.rows) code = 64;
+    top = bot;
+    const float dyv = d[k];
+    int ncode = __shfl_down(code, 1, GROUP);
+    const float ndy = __shfl_down(dyv, 1, GROUP);
+    if (last) ncode = 64;
+    if (k > 0 && k <= g.rows && s.makes && s.p0 + k - 1 < g.P) {
+      // block row p0 + k - 1: windows (.., q), (.., q + 1), then the two below, in that order
+      const float o00 = 0.f + (code_p == 4 ? dy_p : 0.f);
+      const float o01 = (0.f + (code_p == 5 ? dy_p : 0.f)) + (ncode_p == 3 ? ndy_p : 0.f);
+      const float o10 = (0.f + (code_p == 7 ? dy_p : 0.f)) + (code == 1 ? dyv : 0.f);
+      const float o11 = (((0.f + (code_p == 8 ? dy_p : 0.f)) + (ncode_p == 6 ? ndy_p : 0.f)) + (code == 2 ? dyv : 0.f)) +
+                        (ncode == 0 ? ndy : 0.f);
+      const int h = 2 * (s.p0 + k - 1);
+      store_block<S>(dx + (size_t(s.plane) * g.H + h) * g.W + 2 * s.q, g.W, h + 1 < g.H, 2 * s.q + 1 < g.W, o00, o01, o10, o11);
+    }
+    code_p = code, ncode_p = ncode, dy_p = dyv, ndy_p = ndy;
+  }
+}
+
+// ---- 2 x 2 windows, stride 2, no padding: the windows do not overlap, so both passes stream -----------------------------
+// One thread per 2 x 2 block of x: two pairs in; the maximum (or mean) out, or in the backward pass dy to the element of the
+// first maximum (a quarter of dy to each).  Blocks of a last odd row or column belong to no window and receive zero.
+// fp32 128 x 32 x 32 x 32, maximum: backward 19.4 -> 6.5 us (was: rows staged in LDS, a table of arg-max positions), forward
+// 6.9 -> 4.3 (one thread per output, four loads each); mean of 50 x 72 x 57 x 43 37.4 + 11.8 -> 9.7 + 7.1.
+struct QuadG {
+  int H, W, P, Q;
+  int BW;                 // blocks per row: ceil(W / 2) backward, Q forward
+  int total;              // blocks
+  unsigned x_bytes;
+  sgh_fastdiv d_bw, d_bh;
+};
+
+template <class S, bool MAX>
+__global__ __launch_bounds__(kBlock) void k_pool_quad_fwd(const typename S::elem *__restrict__ x, typename S::elem *__restrict__ y,
+                                                         const QuadG g) {
+  typedef typename S::elem elem;
+  const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, g.x_bytes, 0x00020000);
+  constexpr int U = 4;
+  for (int i0 = int(blockIdx.x) * kBlock * U + int(threadIdx.x); i0 < g.total; i0 += int(gridDim.x) * kBlock * U) {
+    Pair<S> t[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * kBlock, r = g.d_bw.div(i), q = i - r * g.BW, plane = g.d_bh.div(r), p = r - plane * g.P;
+      const int at = (plane * g.H + 2 * p) * g.W + 2 * q;
+      t[u] = Pair<S>::load(xr, at, i < g.total);
+      b[u] = Pair<S>::load(xr, at + g.W, i < g.total);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * kBlock;
+      if (i >= g.total) break;
+      float v;
+      if (MAX) {
+        v = kLowest;
+        if (t[u].lo > v) v = t[u].lo;
+        if (t[u].hi > v) v = t[u].hi;
+        if (b[u].lo > v) v = b[u].lo;
+        if (b[u].hi > v) v = b[u].hi;
+      } else {
+        v = ((((0.f + t[u].lo) + t[u].hi) + b[u].lo) + b[u].hi) / 4.f;
+      }
+      S::st(y + i, v);
+    }
+  }
+}
+
+template <class S, bool MAX>
+__global__ __launch_bounds__(kBlock) void k_pool_quad_bwd(const typename S::elem *__restrict__ dy, const typename S::elem *__restrict__ x,
+                                                         typename S::elem *__restrict__ dx, const QuadG g, int BH, unsigned y_bytes) {
+  typedef typename S::elem elem;
+  const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, MAX ? g.x_bytes : 0, 0x00020000);
+  const rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(dy), 0, y_bytes, 0x00020000);
+  constexpr int U = 4;
+  for (int i0 = int(blockIdx.x) * kBlock * U + int(threadIdx.x); i0 < g.total; i0 += int(gridDim.x) * kBlock * U) {
+    Pair<S> t[U], b[U];
+    float d[U];
+    int at[U], hr[U], q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * kBlock, r = g.d_bw.div(i), plane = g.d_bh.div(r), p = r - plane * BH;
+      q[u] = i - r * g.BW;
+      hr[u] = 2 * p;
+      at[u] = (plane * g.H + 2 * p) * g.W + 2 * q[u];
+      const bool window = i < g.total && p < g.P && q[u] < g.Q;
+      d[u] = ld_one<S>(yr, (plane * g.P + p) * g.Q + q[u], window);
+      if (MAX) {
+        t[u] = Pair<S>::load(xr, at[u], window);
+        b[u] = Pair<S>::load(xr, at[u] + g.W, window);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i0 + u * kBlock >= g.total) break;
+      float o[4];
+      if (MAX) {
+        float v = kLowest;
+        int k = -1;
+        if (t[u].lo > v) v = t[u].lo, k = 0;
+        if (t[u].hi > v) v = t[u].hi, k = 1;
+        if (b[u].lo > v) v = b[u].lo, k = 2;
+        if (b[u].hi > v) k = 3;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = 0.f + (k == e ? d[u] : 0.f);   // (a block without a window read d = 0)
+      } else {
+        o[0] = o[1] = o[2] = o[3] = 0.f + d[u] / 4.f;
+      }
+      store_block<S>(dx + at[u], g.W, hr[u] + 1 < g.H, 2 * q[u] + 1 < g.W, o[0], o[1], o[2], o[3]);
+    }
   }
 }
 
@@ -288,134 +599,6 @@ __global__ __launch_bounds__(kBlock) void k_pool_max_bwd_tiled(const typename S:
   }
 }
 
-// Max-pool backward for the residual networks' pooling layer: 3 x 3 windows, stride 2, padding 1, even H and W.
-// The dx block (rows 2i, 2i+1; columns 2j, 2j+1) can only receive from windows (i, j), (i, j+1), (i+1, j),
-// (i+1, j+1), and only at fixed positions of those windows, so instead of tables of arg-max positions and
-// dy values in LDS (the general kernel above: 67 vector instructions per dx element, which bound it) a lane
-// walks down one window column with everything in registers:
-//   * window p shares its top row with window p - 1's bottom row: the per-row first maximum (strict '>',
-//     left to right) is computed once per x row, and three of them combine top to bottom -- the same winner
-//     as the row-major scan of the CPU loop;
-//   * the winner is kept as a code 3 * dh + dw; the right-hand neighbour's code and dy come from lane + 1;
-//   * a block's four elements add the dy of the windows whose code names them, in ascending (p, q) order
-//     starting from +0.0, exactly the additions of the general kernel.
-// A workgroup owns kStripRows block rows per wavefront of one plane; x rows are staged in LDS as stored, behind
-// an element and (for the first band) a row of -inf, so no position needs a bounds check.
-constexpr int kStripRows = 7;   // block rows per wavefront (a wavefront also computes the window row below them)
-constexpr float kLowest = -3.402823466e38f;
-
-struct RowBest {
-  float m;
-  int k;   // column within the window (0..2), 64 = none
-};
-
-template <class S>
-__device__ __forceinline__ RowBest row_best(const typename S::elem *row) {   // row -> the window's middle element of one x row
-  typedef typename S::elem elem;
-  float a, b, c;
-  if constexpr (sizeof(elem) == 4) {
-    a = row[-1];
-    const float2 bc = *reinterpret_cast<const float2 *>(row);
-    b = bc.x, c = bc.y;
-  } else {
-    const unsigned pr = *reinterpret_cast<const unsigned *>(row);
-    const elem lo = elem(pr & 0xffffu), hi = elem(pr >> 16);
-    a = S::ld(row - 1), b = S::ld(&lo), c = S::ld(&hi);
-  }
-  RowBest r{kLowest, 64};
-  if (a > r.m) r.m = a, r.k = 0;
-  if (b > r.m) r.m = b, r.k = 1;
-  if (c > r.m) r.m = c, r.k = 2;
-  return r;
-}
-
-template <class S>
-__global__ __launch_bounds__(kBlock) void k_pool_max_bwd_3x3s2(const typename S::elem *__restrict__ dy,
-                                                               const typename S::elem *__restrict__ x,
-                                                               typename S::elem *__restrict__ dx, int H, int W, int bands) {
-  typedef typename S::elem elem;
-  constexpr int V = S::VEC;
-  typedef sgh_v4u raw;   // 16 bytes: V elements
-  // x rows as stored: element (r, w) at (r - r_lo) * pitch + V + w (rows start on 16-byte boundaries), the element
-  // before a row and the row above the image hold -inf, which no comparison selects
-  extern __shared__ __align__(16) unsigned char xs_raw[];
-  elem *xs = reinterpret_cast<elem *>(xs_raw);
-  const int P = H >> 1, Q = W >> 1, pitch = W + V;
-  const int plane = blockIdx.x / bands, band = blockIdx.x - plane * bands;
-  const int i0 = band * (4 * kStripRows), i1 = min(i0 + 4 * kStripRows, P);   // block rows (= window rows) of the band
-  const int r_lo = 2 * i0 - 1, r_hi = min(2 * i1 + 1, H - 1), rr0 = max(r_lo, 0);
-  const elem *xb = x + size_t(plane) * H * W;
-  const elem *db = dy + size_t(plane) * P * Q;
-  elem *ob = dx + size_t(plane) * H * W;
-  const int vpr = W / V;   // 16-byte (8-byte) vectors per row
-  for (int i = threadIdx.x; i < (r_hi - rr0 + 1) * vpr; i += kBlock) {
-    const int r = i / vpr, c = (i - r * vpr) * V;
-    *reinterpret_cast<raw *>(xs + (rr0 - r_lo + r) * pitch + V + c) =
-        __builtin_nontemporal_load(reinterpret_cast<const raw *>(xb + size_t(rr0 + r) * W + c));
-  }
-  for (int r = threadIdx.x; r <= r_hi - r_lo; r += kBlock) S::st(xs + r * pitch + V - 1, -__builtin_inff());
-  if (r_lo < 0)
-    for (int c = threadIdx.x; c < pitch; c += kBlock) S::st(xs + c, -__builtin_inff());
-  __syncthreads();
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ia = i0 + wave * kStripRows, ib = min(ia + kStripRows, i1);   // this wavefront's block rows [ia, ib)
-  if (ia >= ib) return;
-  for (int q0 = 0; q0 < Q; q0 += 63) {   // lanes 0..62 produce blocks, lane 63 only hands its window to lane 62
-    const int q = q0 + lane;
-    const bool col = q < Q;
-    const int qc = col ? q : Q - 1;   // (a lane without a window reads a valid address and discards it)
-    float dyr[kStripRows + 1];
-#pragma unroll
-    for (int k = 0; k <= kStripRows; ++k) {
-      const int p = ia + k;
-      dyr[k] = (p <= ib && p < P && col) ? S::ld(db + p * Q + q) : 0.f;
-    }
-    const elem *xq = xs + (2 * ia - r_lo) * pitch + V + 2 * qc;   // element (2 ia, 2 q)
-    RowBest top = row_best<S>(xq - pitch);
-    int code_p = 64, ncode_p = 64;
-    float dy_p = 0.f, ndy_p = 0.f;
-#pragma unroll
-    for (int k = 0; k <= kStripRows; ++k) {
-      const int p = ia + k;
-      if (p > ib) break;
-      int code = 64;
-      if (p < P) {
-        const RowBest mid = row_best<S>(xq + (2 * k) * pitch), bot = row_best<S>(xq + (2 * k + 1) * pitch);
-        float best = top.m;
-        code = top.k;
-        if (mid.m > best) best = mid.m, code = 3 + mid.k;
-        if (bot.m > best) code = 6 + bot.k;
-        if (!col) code = 64;
-        top = bot;
-      }
-      const float dyv = dyr[k];
-      const int ncode = __shfl_down(code, 1);
-      const float ndy = __shfl_down(dyv, 1);
-      if (k > 0 && lane < 63 && col) {
-        // block row p - 1: windows (p-1, q), (p-1, q+1), (p, q), (p, q+1) in that order
-        const float o00 = 0.f + (code_p == 4 ? dy_p : 0.f);
-        const float o01 = (0.f + (code_p == 5 ? dy_p : 0.f)) + (ncode_p == 3 ? ndy_p : 0.f);
-        const float o10 = (0.f + (code_p == 7 ? dy_p : 0.f)) + (code == 1 ? dyv : 0.f);
-        const float o11 = (((0.f + (code_p == 8 ? dy_p : 0.f)) + (ncode_p == 6 ? ndy_p : 0.f)) + (code == 2 ? dyv : 0.f)) +
-                          (ncode == 0 ? ndy : 0.f);
-        elem *o = ob + size_t(2 * (p - 1)) * W + 2 * q;
-        if constexpr (sizeof(elem) == 4) {
-          typedef float v2f __attribute__((ext_vector_type(2)));
-          __builtin_nontemporal_store(v2f{o00, o01}, reinterpret_cast<v2f *>(o));
-          __builtin_nontemporal_store(v2f{o10, o11}, reinterpret_cast<v2f *>(o + W));
-        } else {
-          elem t0[2], t1[2];
-          S::st(t0, o00), S::st(t0 + 1, o01), S::st(t1, o10), S::st(t1 + 1, o11);
-          *reinterpret_cast<unsigned *>(o) = unsigned(t0[0]) | (unsigned(t0[1]) << 16);
-          *reinterpret_cast<unsigned *>(o + W) = unsigned(t1[0]) | (unsigned(t1[1]) << 16);
-        }
-      }
-      code_p = code, ncode_p = ncode, dy_p = dyv, ndy_p = ndy;
-    }
-  }
-}
-
 __device__ __forceinline__ int window_count(const PoolG g, int p, int q, int *hs_, int *he_, int *ws_, int *we_) {
   int hs = p * g.sh - g.ph, ws = q * g.sw - g.pw;
   const int he = min(hs + g.kh, g.H), we = min(ws + g.kw, g.W);
@@ -550,15 +733,86 @@ inline bool geom_ok(const sgh_pool_geom *g) {
          size_t(g->H) * g->W < 0x7fffffffu;
 }
 
+// lanes per strip: the narrowest group that holds a row of windows
+inline int strip_group(int Q) { return Q <= 8 ? 8 : Q <= 16 ? 16 : Q <= 32 ? 32 : 64; }
+
+inline bool strip_plan(const sgh_pool_geom *g, int esize, StripG *s) {
+  if (g->kernel_h != 3 || g->kernel_w != 3 || g->stride_h != 2 || g->stride_w != 2 || g->pad_h != 1 || g->pad_w != 1 || g->W < 2)
+    return false;
+  const size_t x = size_t(g->N) * g->C * g->H * g->W * esize;
+  if (x >= (size_t(1) << 31)) return false;   // (32-bit byte offsets)
+  const int group = strip_group(g->Q);
+  s->H = g->H, s->W = g->W, s->P = g->P, s->Q = g->Q;
+  s->strips = (g->P + kStrip - 1) / kStrip;
+  s->rows = (g->P + s->strips - 1) / s->strips;
+  s->chunks = g->Q <= group ? 1 : (g->Q + group - 3) / (group - 2);
+  s->units = int(size_t(g->N) * g->C * s->strips * s->chunks);   // (fewer than dx elements)
+  s->x_bytes = unsigned(x);
+  s->y_bytes = unsigned(size_t(g->N) * g->C * g->P * g->Q * esize);
+  s->d_chunks = sgh_fastdiv(s->chunks), s->d_strips = sgh_fastdiv(s->strips);
+  return true;
+}
+
+inline unsigned strip_blocks(const StripG &s) {
+  const int per = kBlock / strip_group(s.Q);
+  return unsigned((s.units + per - 1) / per);
+}
+
+inline bool quad_plan(const sgh_pool_geom *g, int esize, bool bwd, QuadG *s) {
+  if (g->kernel_h != 2 || g->kernel_w != 2 || g->stride_h != 2 || g->stride_w != 2 || g->pad_h != 0 || g->pad_w != 0) return false;
+  const size_t x = size_t(g->N) * g->C * g->H * g->W * esize;
+  if (x >= (size_t(1) << 31)) return false;
+  s->H = g->H, s->W = g->W, s->P = g->P, s->Q = g->Q;
+  s->BW = bwd ? (g->W + 1) / 2 : g->Q;
+  const int bh = bwd ? (g->H + 1) / 2 : g->P;
+  s->total = int(size_t(g->N) * g->C * bh * s->BW);
+  s->x_bytes = unsigned(x);
+  s->d_bw = sgh_fastdiv(s->BW), s->d_bh = sgh_fastdiv(bh);
+  return true;
+}
+
+// Tensors of 2 GiB and more, where the kernels with 32-bit offsets apply otherwise: by groups of images
+inline int images_per_call(const sgh_pool_geom *g, int esize) {
+  const bool strip = g->is_max && g->kernel_h == 3 && g->kernel_w == 3 && g->pad_h == 1 && g->pad_w == 1;
+  const bool quad = g->kernel_h == 2 && g->kernel_w == 2 && g->pad_h == 0 && g->pad_w == 0;
+  const size_t image = size_t(g->C) * g->H * g->W * esize, most = (size_t(1) << 31) - 1;
+  if (!(strip || quad) || g->stride_h != 2 || g->stride_w != 2 || image > most || image * g->N <= most) return g->N;
+  return int(most / image);
+}
+
+// fp32 forward: outputs from which the strip kernel is the faster one (with 64 planes per image, 13 x 80 x 80 5.6 us before
+// and 7.0 with it, 21 x 96 x 96 12.5 and 11.9, 64 x 112 x 112 39.2 and 37.6, 128 x 112 x 112 105 and 93).  In 16 bits the
+// whole vectors of k_pool_max_fwd_3x3s2 win throughout: 7.0 us against 11.1, 26.9 against 26.5, 49 against 54.
+constexpr size_t kStripFwdMin = size_t(2) << 20;
+
 template <class S>
 int pool_fwd(const sgh_pool_geom *g, const typename S::elem *x, typename S::elem *y, void *stream) {
   if (!geom_ok(g) || !x || !y) return SGH_EINVAL;
+  const int esize = int(sizeof(typename S::elem)), images = images_per_call(g, esize);
+  if (images < g->N) {
+    sgh_pool_geom part = *g;
+    for (int n = 0; n < g->N; n += images) {
+      part.N = g->N - n < images ? g->N - n : images;
+      const int rc = pool_fwd<S>(&part, x + size_t(n) * g->C * g->H * g->W, y + size_t(n) * g->C * g->P * g->Q, stream);
+      if (rc != SGH_OK) return rc;
+    }
+    return SGH_OK;
+  }
   const size_t total = size_t(g->N) * g->C * g->P * g->Q;
+  StripG sg;
+  QuadG qg;
   if (g->is_max && g->kernel_h == 3 && g->kernel_w == 3 && g->stride_h == 2 && g->stride_w == 2 && g->pad_h == 1 &&
-      g->pad_w == 1 && g->H % 2 == 0 && g->W % 2 == 0 && g->Q % S::VEC == 0 && sgh_aligned16(x) && sgh_aligned16(y))
+      g->pad_w == 1 && g->H % 2 == 0 && g->W % 2 == 0 && g->Q % S::VEC == 0 && sgh_aligned16(x) && sgh_aligned16(y) && (esize == 2 || total <= kStripFwdMin))
     hipLaunchKernelGGL(k_pool_max_fwd_3x3s2<S>, dim3(grid_for(total / S::VEC)), dim3(kBlock), 0, sgh_stream_of(stream), x, y,
                        g->H, g->W, total / S::VEC);
-  else if (g->is_max)
+  else if (g->is_max && strip_plan(g, esize, &sg)) {
+    const int group = strip_group(g->Q);
+    auto kern = group == 8 ? k_pool_max_fwd_strip<S, 8> : group == 16 ? k_pool_max_fwd_strip<S, 16> : group == 32 ? k_pool_max_fwd_strip<S, 32> : k_pool_max_fwd_strip<S, 64>;
+    hipLaunchKernelGGL(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, sg);
+  } else if (quad_plan(g, esize, false, &qg)) {
+    auto kern = g->is_max ? k_pool_quad_fwd<S, true> : k_pool_quad_fwd<S, false>;
+    hipLaunchKernelGGL(kern, dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, qg);
+  } else if (g->is_max)
     hipLaunchKernelGGL(k_pool_max_fwd<S>, dim3(grid_for(total)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, to_g(g),
                        total);
   else if (g->P == 1 && g->Q == 1 && g->pad_h == 0 && g->pad_w == 0 && g->kernel_h >= g->H && g->kernel_w >= g->W &&
@@ -578,20 +832,33 @@ int pool_bwd(const sgh_pool_geom *g, const typename S::elem *dy, const typename 
   (void)y;
   if (!geom_ok(g) || !dy || !dx) return SGH_EINVAL;
   if (g->is_max && !x) return SGH_EINVAL;
+  const int esize = int(sizeof(typename S::elem)), images = images_per_call(g, esize);
+  if (images < g->N) {
+    sgh_pool_geom part = *g;
+    for (int n = 0; n < g->N; n += images) {
+      part.N = g->N - n < images ? g->N - n : images;
+      const size_t at = size_t(n) * g->C * g->H * g->W;
+      const int rc = pool_bwd<S>(&part, dy + size_t(n) * g->C * g->P * g->Q, x ? x + at : x, y, dx + at, stream);
+      if (rc != SGH_OK) return rc;
+    }
+    return SGH_OK;
+  }
   const size_t total = size_t(g->N) * g->C * g->H * g->W;
   // algorithmic bytes: dy and (max pooling) x in, dx out
   sgh_prof_kernel_scope prof(g->is_max ? "pool_bwd/k_pool_max_bwd" : "pool_bwd/k_pool_avg_bwd",
                       double(sizeof(typename S::elem)) *
                           (double(total) * (g->is_max ? 2 : 1) + double(g->N) * g->C * g->P * g->Q),
                       sgh_stream_of(stream));
-  if (g->is_max && g->kernel_h == 3 && g->kernel_w == 3 && g->stride_h == 2 && g->stride_w == 2 && g->pad_h == 1 &&
-      g->pad_w == 1 && g->H % 2 == 0 && g->W % S::VEC == 0 && g->W <= 256 &&
-      size_t(g->N) * g->C * ((g->H / 2 + 4 * kStripRows - 1) / (4 * kStripRows)) < 0x7fffffffu && sgh_aligned16(x) &&
-      sgh_aligned16(dx)) {
-    const int bands = (g->H / 2 + 4 * kStripRows - 1) / (4 * kStripRows);
-    const size_t lds = size_t(8 * kStripRows + 3) * (g->W + S::VEC) * sizeof(typename S::elem);   // <= 61 KB
-    SGH_LAUNCH_TIMED(k_pool_max_bwd_3x3s2<S>, dim3(unsigned(size_t(g->N) * g->C * bands)), dim3(kBlock), lds,
-                       sgh_stream_of(stream), dy, x, dx, g->H, g->W, bands);
+  StripG sg;
+  QuadG qg;
+  if (g->is_max && strip_plan(g, esize, &sg)) {
+    const int group = strip_group(g->Q);
+    auto kern = group == 8 ? k_pool_max_bwd_strip<S, 8> : group == 16 ? k_pool_max_bwd_strip<S, 16> : group == 32 ? k_pool_max_bwd_strip<S, 32> : k_pool_max_bwd_strip<S, 64>;
+    SGH_LAUNCH_TIMED(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), dy, x, dx, sg);
+  } else if (quad_plan(g, esize, true, &qg)) {
+    auto kern = g->is_max ? k_pool_quad_bwd<S, true> : k_pool_quad_bwd<S, false>;
+    SGH_LAUNCH_TIMED(kern, dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0, sgh_stream_of(stream), dy, x, dx, qg,
+                     (g->H + 1) / 2, unsigned(size_t(g->N) * g->C * g->P * g->Q * esize));
   } else if (g->is_max) {
     // band height: about 12 KB of x rows per workgroup (measured optimum: enough workgroups per CU to
     // overlap one's staging with another's scans), bands of equal height

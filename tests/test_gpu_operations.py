@@ -833,3 +833,64 @@ def test_shared_tile_convolution_edges(singa, dev, case):
     into = singa.from_numpy(x, dev)
     got = singa.GpuConvBackwardxAccumulate(dyd, wd, xd, h, into).to_numpy()
     assert_bit_equal(got, (dx.to_numpy() + x).astype(np.float32), "dx += dgrad")
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", [
+    # strips of 16, 32 and 64 lanes at and around the width they hold, odd rows and columns, several chunks per row
+    (2, 3, 15, 31, 3), (3, 2, 9, 32, 3), (2, 2, 16, 33, 3), (1, 3, 29, 63, 3), (2, 1, 14, 66, 3), (1, 2, 31, 127, 3),
+    (1, 1, 17, 129, 3), (1, 2, 7, 251, 3), (5, 7, 1, 2, 3), (4, 3, 2, 3, 3), (50, 9, 5, 7, 3), (1, 1, 43, 5, 3),
+    # 2 x 2: odd last rows and columns belong to no window, more blocks than one step of the grid covers, one window
+    (3, 5, 8, 8, 2), (2, 3, 7, 9, 2), (2, 2, 6, 5, 2), (1, 2, 2, 2, 2), (1, 1, 3, 2, 2), (3, 100, 45, 37, 2),
+])
+def test_strip_and_quad_pooling_bit_exact(singa, dev, kind, case):
+    """The pooling kernels for 3 x 3 / stride 2 / padding 1 and 2 x 2 / stride 2 windows on planes of any size: the oracle's bits
+    (heavy ties; sums in fp32, one rounding of the storage type), no element outside the windows left unwritten."""
+    N, C, H, W, kk = case
+    print("pooling", kind, case, flush=True)
+    kernel, stride, pad = (kk, kk), (2, 2), (kk // 2,) * 2 if kk == 3 else (0, 0)
+    r = rng(sum(case))
+    dt = {"f32": singa.kFloat32, "f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+
+    def to(a):
+        t = singa.from_numpy(a.astype(np.float32), dev)
+        return t if kind == "f32" else t.AsType(dt)
+
+    def rounded(a):
+        return a if kind == "f32" else to(a).AsType(singa.kFloat32).to_numpy()
+    back = lambda t: (t if kind == "f32" else t.AsType(singa.kFloat32)).to_numpy()
+    xt = to(np.round(randn(r, N, C, H, W) * 2) / 2)
+    x = back(xt)
+    for is_max in (True, False):
+        h = singa.CudnnPoolingHandle(xt, kernel, stride, pad, is_max)
+        y = singa.GpuPoolingForward(h, xt)
+        if is_max:
+            y_o, mask = O.pool_max_fwd(x, kernel, stride, pad)
+        else:
+            y_o = O.pool_avg_fwd(x, kernel, stride, pad, include_pad=False)
+        assert_bit_equal(back(y), rounded(y_o), "forward")
+        dyt = to(randn(r, *y_o.shape))
+        dy = back(dyt)
+        dx_o = O.pool_max_bwd(dy, mask, x.shape) if is_max else O.pool_avg_bwd(dy, x.shape, kernel, stride, pad, include_pad=False)
+        assert_bit_equal(back(singa.GpuPoolingBackward(h, dyt, xt, y)), rounded(dx_o), "backward")
+
+
+def test_pooling_by_groups_of_images(singa, dev):
+    """Tensors beyond 32-bit byte offsets go through the same kernels in groups of images: the bits of the images alone."""
+    N, C, H, W = 9, 64, 1030, 1030          # 2.4 GB, seven images per group
+    r = rng(5)
+    image, grad = r.standard_normal((C, H, W), dtype=np.float32), r.standard_normal((C, 515, 515), dtype=np.float32)
+    x = np.stack([np.roll(image, n) for n in range(N)])
+    dy = np.stack([np.roll(grad, n) for n in range(N)])
+    xd, dyd = singa.from_numpy(x, dev), singa.from_numpy(dy, dev)
+    for k, pad in ((3, 1), (2, 0)):
+        h = singa.CudnnPoolingHandle(xd, (k, k), (2, 2), (pad, pad), True)
+        y = singa.GpuPoolingForward(h, xd)
+        got_y, got_dx = y.to_numpy(), singa.GpuPoolingBackward(h, dyd, xd, y).to_numpy()
+        for n in (0, 6, 7, 8):
+            x1 = singa.from_numpy(x[n:n + 1], dev)
+            h1 = singa.CudnnPoolingHandle(x1, (k, k), (2, 2), (pad, pad), True)
+            y1 = singa.GpuPoolingForward(h1, x1)
+            assert np.array_equal(got_y[n:n + 1], y1.to_numpy()), ("forward", k, n)
+            dx1 = singa.GpuPoolingBackward(h1, singa.from_numpy(dy[n:n + 1], dev), x1, y1)
+            assert np.array_equal(got_dx[n:n + 1], dx1.to_numpy()), ("backward", k, n)
