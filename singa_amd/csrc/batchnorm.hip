@@ -554,12 +554,12 @@ inline ChipPlan chip_plan(int N, int C, int HW) {
     p.nt = 1024;
     G = 1;
   }
-  // few channels: thinner slices, so that there are two workgroups for every CU (at least one wavefront of vectors
-  // each) -- unless a channel fits one workgroup and there is a channel for every CU: then nothing is exchanged
+  // a channel that fits one workgroup and a channel for every CU: nothing is exchanged
   const bool whole_channels = G == 1 && C >= sgh_num_cus();
-  const long want = whole_channels ? 1 : (2L * sgh_num_cus() + C - 1) / C;
-  if (G < want) G = want;
-  // whole rounds: as many slices as still fit into the rounds of (2 workgroups x CUs) that this many need
+  // whole rounds: as many slices as still fit into the rounds of (2 workgroups x CUs) that this many need.  (A round more
+  // costs more than the thinner slices save -- the workgroups of a channel wait for each other: two workgroups for every CU
+  // rounded up, as it was, made 600 of 100 channels.  bfloat16 30 x 100 x 32 x 32 17.6 -> 10.6 us, 50 x 72 x 57 x 43
+  // 22.9 -> 14.9, fp32 32 x 48 x 56 x 56 16.5 -> 11.8)
   const long slots = 2L * sgh_num_cus(), rounds = (long(C) * G + slots - 1) / slots;
   long fill = rounds * slots / C;
   if (fill > kChipMaxG) fill = kChipMaxG;
@@ -853,14 +853,17 @@ constexpr int chip_fwd_nv(bool two) {
 template <class S>
 inline ChipPlan chip_fwd_plan(int N, int C, int HW, bool two) {
   ChipPlan p{false, 0, 0, 512, 0, false};
-  if (HW % S::VEC != 0 || size_t(N) * C * HW * sizeof(typename S::elem) >= (size_t(1) << 32)) return p;
-  const long TV = long(N) * (HW / S::VEC);
+  p.ragged = HW % S::VEC != 0;
+  if (p.ragged && (S::VEC * sizeof(typename S::elem) != 16 || HW < S::VEC || sgh_env().bn_ragged_off ||
+                   size_t(N) * C * HW * sizeof(typename S::elem) >= (size_t(1) << 31)))
+    return p;
+  if (size_t(N) * C * HW * sizeof(typename S::elem) >= (size_t(1) << 32)) return p;
+  const long TV = long(N) * ((HW + S::VEC - 1) / S::VEC);
   const long per_wg = 512L * chip_fwd_nv<S>(two);
   long G = (TV + per_wg - 1) / per_wg;
-  const long want = (2L * sgh_num_cus() + C - 1) / C;   // few channels: thinner slices, two workgroups for every CU
-  if (G < want) G = want;
   const long slots = 2L * sgh_num_cus(), rounds = (long(C) * G + slots - 1) / slots;
-  long fill = rounds * slots / C;                       // whole rounds
+  // whole rounds, as in chip_plan (50 x 72 x 57 x 43 22.1 -> 12.7 us, 64 x 300 x 8 x 8 in one workgroup per channel 11.6 -> 5.6)
+  long fill = rounds * slots / C;
   if (fill > kChipMaxG) fill = kChipMaxG;
   if (fill > G) G = fill;
   while (G > 1 && (TV + G - 1) / G < 64) --G;
@@ -871,7 +874,10 @@ inline ChipPlan chip_fwd_plan(int N, int C, int HW, bool two) {
   return p;
 }
 
-template <class S, int ACT>
+// RAGGED: pieces of 16 bytes at element alignment, the last one of a plane overlapping, as in k_bn_bwd_onchip; before, planes
+// that are no multiple of the vector ran the two passes below element by element (bfloat16 128 x 2048 x 7 x 7 43.1 -> 21.1 us,
+// 100 x 32 x 99 x 97 91.5 -> 32.0, 50 x 72 x 57 x 43 37.2 -> 12.7; fp32 128 x 2048 x 7 x 7 48.2 -> 25.5 us).
+template <class S, int ACT, bool RAGGED = false>
 __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem *__restrict__ x,
                                                            const typename S::elem *__restrict__ z,
                                                            const float *__restrict__ gamma, const float *__restrict__ beta,
@@ -898,7 +904,9 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
     ticket_s = (unsigned(wa) == unsigned(ticket1) && unsigned(wb) == unsigned(ticket1 >> 32)) ? ticket2 : ticket1;
     gave_up = 0;
   }
-  const int PV = s.HW / V, TV = s.N * PV;
+  static_assert(!RAGGED || V * sizeof(elem) == 16, "ragged planes: 16-byte pieces");
+  const int PV = RAGGED ? (s.HW + V - 1) / V : s.HW / V, TV = s.N * PV;
+  const int tail_skip = RAGGED ? PV * V - s.HW : 0;   // elements of a plane's last piece that are not its own
   const int lo = g * vpg, hi = min(lo + vpg, TV);
   const float pivot = S::ld(x + size_t(c) * s.HW);
   // the vectors of a thread are walked in steps of NT (ChipWalk), byte offsets are 32 bits from a uniform base
@@ -908,21 +916,38 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
   ChipWalk first;
   first.n = (lo + t) / PV, first.r = (lo + t) - first.n * PV;
   auto vec_bytes = [&](const ChipWalk &w) { return (unsigned(w.n) * CPV + cPV + unsigned(w.r)) * unsigned(sizeof(raw)); };
+  const int tensor_bytes = RAGGED ? int(size_t(s.N) * s.C * s.HW * sizeof(elem)) : 0;
+  const __amdgpu_buffer_rsrc_t rxb = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, tensor_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rzb = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(z), 0, tensor_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rob = __builtin_amdgcn_make_buffer_rsrc(y, 0, tensor_bytes, 0x00020000);
+  auto piece = [&](const ChipWalk &w) {   // byte offset of piece r of plane (n, c)
+    return int(((unsigned(w.n) * unsigned(s.C) + unsigned(c)) * unsigned(s.HW) + unsigned(w.r == PV - 1 ? s.HW - V : w.r * V)) *
+               unsigned(sizeof(elem)));
+  };
   raw xv[NV];
   {
     ChipWalk w = first;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if (lo + i * NT + t < hi) xv[i] = __builtin_nontemporal_load(reinterpret_cast<const raw *>(xb + vec_bytes(w)));
+      if (lo + i * NT + t < hi) {
+        if constexpr (RAGGED) xv[i] = __builtin_bit_cast(raw, __builtin_amdgcn_raw_buffer_load_b128(rxb, piece(w), 0, 0));
+        else xv[i] = __builtin_nontemporal_load(reinterpret_cast<const raw *>(xb + vec_bytes(w)));
+      }
       w.step(dn, dr, PV);
     }
   }
   float a = 0.f, b = 0.f;
+  ChipWalk wsum = first;
 #pragma unroll
-  for (int i = 0; i < NV; ++i)
+  for (int i = 0; i < NV; ++i) {
     if (lo + i * NT + t < hi) {
       float v[V];
       S::template load16<false>(reinterpret_cast<const elem *>(&xv[i]), v);
+      if constexpr (RAGGED) {
+        const int skip = wsum.r == PV - 1 ? tail_skip : 0;
+#pragma unroll
+        for (int q = 0; q < V; ++q) v[q] = q < skip ? pivot : v[q];   // (adds nothing to either sum)
+      }
 #pragma unroll
       for (int q = 0; q < V; q += 4) {
         const float d0 = v[q] - pivot, d1 = v[q + 1] - pivot, d2 = v[q + 2] - pivot, d3 = v[q + 3] - pivot;
@@ -930,6 +955,8 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
         b += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
       }
     }
+    if constexpr (RAGGED) wsum.step(dn, dr, PV);
+  }
   // the second tensor's slice is requested now and arrives during the block sums and the exchange
   raw zr[ACT == 2 ? NV : 1];
   if constexpr (ACT == 2) {
@@ -937,7 +964,10 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
     ChipWalk w = first;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if (lo + i * NT + t < hi) zr[i] = __builtin_nontemporal_load(reinterpret_cast<const raw *>(zb + vec_bytes(w)));
+      if (lo + i * NT + t < hi) {
+        if constexpr (RAGGED) zr[i] = __builtin_bit_cast(raw, __builtin_amdgcn_raw_buffer_load_b128(rzb, piece(w), 0, 0));
+        else zr[i] = __builtin_nontemporal_load(reinterpret_cast<const raw *>(zb + vec_bytes(w)));
+      }
       w.step(dn, dr, PV);
     }
   }
@@ -1014,7 +1044,8 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
         o[q] = bn_fwd_value<S, ACT>(bn_out_rounded(v[q], mean, invstd, gm, be), ACT == 2 ? zv[q] : 0.f);
       raw ov;
       S::store16(reinterpret_cast<elem *>(&ov), o);
-      *reinterpret_cast<raw *>(ob + vec_bytes(w)) = ov;
+      if constexpr (RAGGED) __builtin_amdgcn_raw_buffer_store_b128(ov, rob, piece(w), 0, 0);
+      else *reinterpret_cast<raw *>(ob + vec_bytes(w)) = ov;
     }
   }
 }
@@ -1041,7 +1072,11 @@ int launch_fwd_onchip(const typename S::elem *x, const typename S::elem *z, cons
   const dim3 grid(xcd_runs ? unsigned((s.C + 7) / 8) * 8u * p.G : unsigned(s.C) * p.G);
   const unsigned long long t1 = next_ticket(), t2 = next_ticket();
   if (p.G > 1) g_exchange_ran.store(true, std::memory_order_relaxed);
-  hipLaunchKernelGGL((k_bn_fwd_onchip<S, ACT>), grid, dim3(512), 0, st, x, z, gamma, beta, running_mean, running_var, factor,
+  auto kern = k_bn_fwd_onchip<S, ACT>;
+  if constexpr (S::VEC * sizeof(typename S::elem) == 16) {
+    if (p.ragged) kern = k_bn_fwd_onchip<S, ACT, true>;
+  }
+  hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, x, z, gamma, beta, running_mean, running_var, factor,
                      eps, y, save_mean, save_invstd, static_cast<unsigned long long *>(workspace), s, p.G, p.vpg, t1, t2,
                      g_spin_limit.load(std::memory_order_relaxed), xcd_runs);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
@@ -1394,7 +1429,14 @@ size_t sgh_bn_workspace_bytes(int N, int C, int HW) {
   return shared_workspace_bytes(N, C, HW) + fwd;
 }
 
-// 16-bit planes that are a multiple of 4 but not of 8 elements (14 x 14) use the 8-byte vector class
+// 16-bit planes that are a multiple of 4 but not of 8 elements (14 x 14): in training the 16-byte pieces where the one-pass
+// kernel runs (RAGGED in k_bn_fwd_onchip: 128 x 1024 x 14 x 14 33.8 -> 21.9 us, with the second tensor 40.6 -> 34.8), the
+// 8-byte vector class otherwise
+inline bool fwd_pieces16(int N, int C, int HW, bool two) {
+  return HW % 8 == 0 || HW % 4 != 0 || (!sgh_env().bn_fwd_onchip_off && chip_fwd_plan<StF16>(N, C, HW, two).ok);
+}
+#define SGH_BN_DISPATCH16_TRAIN(two, F16X8, F16X4, ...) \
+  (fwd_pieces16(N, C, HW, two) ? bn_fwd_train<F16X8>(__VA_ARGS__) : bn_fwd_train<F16X4>(__VA_ARGS__))
 #define SGH_BN_DISPATCH16(fn, F16X8, F16X4, ...) \
   (HW % 8 != 0 && HW % 4 == 0 ? fn<F16X4>(__VA_ARGS__) : fn<F16X8>(__VA_ARGS__))
 // (the backward pass takes such planes in 16-byte pieces, the last one overlapping -- RAGGED in k_bn_bwd_onchip:
@@ -1411,13 +1453,13 @@ int sgh_bn_fwd_train_f32(const float *x, const float *gamma, const float *beta, 
 int sgh_bn_fwd_train_f16(const uint16_t *x, const float *gamma, const float *beta, float *running_mean,
                          float *running_var, float factor, float eps, uint16_t *y, float *save_mean,
                          float *save_invstd, int N, int C, int HW, void *workspace, size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(false, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream);
 }
 int sgh_bn_fwd_train_bf16(const uint16_t *x, const float *gamma, const float *beta, float *running_mean,
                           float *running_var, float factor, float eps, uint16_t *y, float *save_mean,
                           float *save_invstd, int N, int C, int HW, void *workspace, size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(false, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream);
 }
 
@@ -1430,13 +1472,13 @@ int sgh_bn_relu_fwd_train_f32(const float *x, const float *gamma, const float *b
 int sgh_bn_relu_fwd_train_f16(const uint16_t *x, const float *gamma, const float *beta, float *running_mean,
                               float *running_var, float factor, float eps, uint16_t *y, float *save_mean,
                               float *save_invstd, int N, int C, int HW, void *workspace, size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(false, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream, 1);
 }
 int sgh_bn_relu_fwd_train_bf16(const uint16_t *x, const float *gamma, const float *beta, float *running_mean,
                                float *running_var, float factor, float eps, uint16_t *y, float *save_mean,
                                float *save_invstd, int N, int C, int HW, void *workspace, size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(false, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream, 1);
 }
 int sgh_bn_add_relu_fwd_train_f32(const float *x, const float *z, const float *gamma, const float *beta,
@@ -1450,14 +1492,14 @@ int sgh_bn_add_relu_fwd_train_f16(const uint16_t *x, const uint16_t *z, const fl
                                   float *running_mean, float *running_var, float factor, float eps, uint16_t *y,
                                   float *save_mean, float *save_invstd, int N, int C, int HW, void *workspace,
                                   size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(true, StF16, StF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream, 2, z);
 }
 int sgh_bn_add_relu_fwd_train_bf16(const uint16_t *x, const uint16_t *z, const float *gamma, const float *beta,
                                    float *running_mean, float *running_var, float factor, float eps, uint16_t *y,
                                    float *save_mean, float *save_invstd, int N, int C, int HW, void *workspace,
                                    size_t ws_bytes, void *stream) {
-  return SGH_BN_DISPATCH16(bn_fwd_train, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
+  return SGH_BN_DISPATCH16_TRAIN(true, StBF16, StBF16x4, x, gamma, beta, running_mean, running_var, factor, eps, y,
                            save_mean, save_invstd, N, C, HW, workspace, ws_bytes, stream, 2, z);
 }
 
@@ -1541,6 +1583,7 @@ int sgh_bn_relu_bwd_bf16(const uint16_t *dy, const uint16_t *x, const float *gam
   return SGH_BN_DISPATCH16_BWD(bn_bwd, StBF16, StBF16x4, dy, x, gamma, beta, save_mean, save_invstd, dx, dgamma, dbeta, N, C,
                            HW, workspace, ws_bytes, stream);
 }
+#undef SGH_BN_DISPATCH16_TRAIN
 #undef SGH_BN_DISPATCH16
 #undef SGH_BN_DISPATCH16_BWD
 

@@ -875,6 +875,38 @@ def test_strip_and_quad_pooling_bit_exact(singa, dev, kind, case):
         assert_bit_equal(back(singa.GpuPoolingBackward(h, dyt, xt, y)), rounded(dx_o), "backward")
 
 
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+@pytest.mark.parametrize("shape", [(2, 7, 2, 2), (3, 5, 3, 3), (5, 300, 1, 9), (40, 72, 23, 19), (32, 600, 6, 6), (2, 3, 127, 65)])
+def test_bn_forward_planes_of_any_size(singa, dev, kind, shape):
+    """One-pass forward on planes that are no whole 16-byte vectors, every element against float64 (half an ulp of the storage
+    type, the fp32 chain of y = (x - mean) * invstd * gamma + beta beside it), and the fused forms against the plain one."""
+    print("bn forward", kind, shape, flush=True)
+    r = rng(sum(shape))
+    half = kind == "bf16"
+    xt, zt = (singa.from_numpy((randn(r, *shape) * 2 + 0.5).astype(np.float32), dev) for _ in range(2))
+    if half:
+        xt, zt = xt.AsType(singa.kBFloat16), zt.AsType(singa.kBFloat16)
+    back = lambda t: (t.AsType(singa.kFloat32) if half else t).to_numpy()
+    x, z = back(xt).astype(np.float64), back(zt)
+    C = shape[1]
+    gamma, beta = (randn(r, C) * 0.2 + 1).astype(np.float32), randn(r, C)
+    h = singa.CudnnBatchNormHandle(0.9, xt)
+    new = lambda: [singa.from_numpy(a, dev) for a in (gamma, beta, np.zeros(C, np.float32), np.ones(C, np.float32))]
+    y, mean, inv = singa.GpuBatchNormForwardTraining(h, xt, *new())
+    m, v = x.mean((0, 2, 3)), x.var((0, 2, 3))
+    s = (gamma / np.sqrt(v + 1e-5))[:, None, None]
+    want = (x - m[:, None, None]) * s + beta[:, None, None]
+    # 16 fp32 roundings of values up to |x| + |mean|, scaled, and one of the storage type
+    bound = 16 * 2.0 ** -24 * ((np.abs(x) + np.abs(m)[:, None, None]) * np.abs(s) + np.abs(beta)[:, None, None] + np.abs(want))
+    bound += (2.0 ** -8 if half else 0.0) * np.abs(want)   # (8 significant bits: half an ulp is up to 2^-8 of the value)
+    err = np.abs(back(y) - want) - bound
+    assert err.max() <= 0, np.unravel_index(err.argmax(), err.shape)
+    assert_bit_equal(back(singa.GpuBatchNormReLUForwardTraining(h, xt, *new())[0]), np.maximum(back(y), 0), "ReLU")
+    total = singa.from_numpy(back(y) + z, dev)
+    total = back(total.AsType(singa.kBFloat16)) if half else back(total)
+    assert_bit_equal(back(singa.GpuBatchNormAddReLUForwardTraining(h, xt, zt, *new())[0]), np.maximum(total, 0), "sum and ReLU")
+
+
 def test_pooling_by_groups_of_images(singa, dev):
     """Tensors beyond 32-bit byte offsets go through the same kernels in groups of images: the bits of the images alone."""
     N, C, H, W = 9, 64, 1030, 1030          # 2.4 GB, seven images per group
