@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "pw16.h"
 #include "storage.h"
 
 namespace {
@@ -1076,6 +1077,7 @@ struct D16Plan {
   int slab_sp;        // slab entries
   int slab_ev;        // pixels per staging group: 8 or 4
   bool dilate;        // 1x1, stride 2, no padding, even image: see D16Args::dilate
+  bool pw;            // 1x1, stride 1, no padding: k_pw16 (tiles counts octets of planes, 16 a tile)
   sgh_conv_geom kg;   // the geometry the kernel sees (the stride-1 problem on the P x Q grid when `dilate`)
 };
 
@@ -1128,6 +1130,18 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
       p.ok = true;
       return p;
     }
+  }
+  if (fs == 1 && !p.dilate && g->R == 1 && g->S == 1 && st == 1 && g->pad_h == 0 && g->pad_w == 0 && g->H * g->W >= 8) {
+    const long octets = long(g->N) * ((g->H * g->W + 7) / 8);
+    p.pw = true;
+    p.tiles = int((octets + 15) / 16);
+    p.bm = sgh_pw16_tile(g->C, p.tiles);
+    p.mtiles = (g->C + p.bm - 1) / p.bm;
+    p.CP = p.mtiles * p.bm, p.KP = (g->K + KC - 1) / KC * KC;
+    if (octets >= (long(1) << 30) || long(p.tiles) * p.mtiles >= (long(1) << 30) || size_t(p.CP) * p.KP >= lim) return p;
+    p.wt_bytes = align256(size_t(p.CP) * p.KP * sizeof(uint16_t));
+    p.ok = true;
+    return p;
   }
   // 64-row channel tiles when 128-row ones would leave CUs without a workgroup
   p.bm = (g->C <= 64 || tiles * ((g->C + 127) / 128) < sgh_num_cus() * 5 / 4) ? 64 : 128;
@@ -1300,7 +1314,10 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     else hipLaunchKernelGGL(k_pixel_major16<false>, grid, dim3(256), 0, s, dy, dyT, g->K, PQ);
     if (hipGetLastError() != hipSuccess) return SGH_EINVAL;
   }
-  if (!fwd_of && prelaid) {
+  // 1x1 forward passes over whole chunks read the weight tensor as it is
+  const bool as_is = fwd_of && p.pw && g->K % KC == 0 && (reinterpret_cast<uintptr_t>(W) & 3u) == 0;
+  if (as_is) {
+  } else if (!fwd_of && prelaid) {
     // re-laid by sgh_conv_dgrad_prepare_multi
   } else if (fwd_of)
     hipLaunchKernelGGL(k_relayout16_fwd, dim3(unsigned((nw + 255) / 256)), dim3(256), 0, s, W, wt, fwd_of->K, fwd_of->C,
@@ -1322,6 +1339,18 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     if (p.slab == 1) rc = launch_slab<2, 2, 1, 4>(b, p, bf16, s);
     else if (p.slab == 2) rc = launch_slab<2, 2, 2, 4>(b, p, bf16, s);
     else rc = launch_slab<2, 2, 2, 2>(b, p, bf16, s);
+    sgh_prof_kernel_end(s);
+    return rc;
+  }
+  if (p.pw) {
+    sgh_pw16_args b{};
+    b.A = as_is ? W : wt, b.src = dy, b.out = dx, b.bias = bias;
+    b.M = g->C, b.K = g->K, b.HW = g->H * g->W, b.lda = p.KP;
+    b.QO = (b.HW + 7) / 8, b.octets = g->N * b.QO, b.mtiles = p.mtiles, b.ptiles = p.tiles;
+    b.a_bytes = unsigned((as_is ? size_t(g->C) * g->K : nw) * 2);
+    b.src_bytes = unsigned(size_t(g->N) * g->K * b.HW * 2);
+    sgh_prof_kernel_begin(fwd_of ? "conv_fwd16/k_pw16" : "conv_dgrad16/k_pw16", 2.0 * g->N * g->K * b.HW * double(g->C));
+    const int rc = sgh_pw16_launch(b, p.bm, bf16, s);
     sgh_prof_kernel_end(s);
     return rc;
   }

@@ -886,3 +886,44 @@ def test_stem_forward_other_widths(singa, dev, kind, case):
     h = singa.CudnnConvHandle(xt, (7, 7), (2, 2), (3, 3), C, 64, bias)
     y = singa.GpuConvForward(xt, wt, bt if bias else None, h)
     assert nl2(y.to_numpy(), O.conv_fwd(x, w, b if bias else None, (2, 2), (3, 3))) < (1e-5 if kind == "f32" else 1e-2)
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("case", [
+    # N, C, H, W, K: forward (K filters over C) and data gradient (C over K) of 1x1 layers
+    (1, 16, 2, 4, 8),       # one octet, less than one chunk
+    (3, 72, 3, 3, 136),     # planes of 9 pixels: two octets that overlap in seven, channels that fill no tile
+    (5, 40, 3, 6, 24),      # 18 pixels: even, no whole octets
+    (37, 136, 7, 7, 72),    # odd planes, tiles across images
+    (16, 256, 32, 48, 72),  # 256 filters per workgroup
+    (16, 64, 32, 48, 264),  # ... the second tile of them nearly empty; whole chunks, so the weight tensor is read as it is
+    (17, 128, 31, 49, 24),  # 128 per workgroup on odd planes
+    (17, 200, 31, 49, 40),  # ... where an even plane would take 256
+])
+def test_conv_1x1_16bit(singa, dev, kind, case):
+    """The pointwise kernels at the edges of their tiles, against the oracle: one rounding of a result is at most 2^-11 (binary16)
+    or 2^-8 / 2 (bfloat16) of it.  Operands that are not dword aligned take the register path: the same bits."""
+    from oracle import cpu_oracle as O
+    from util import nl2
+    N, C, H, W, K = case
+    print("1x1", kind, case, flush=True)
+    bound = 5e-4 if kind == "f16" else 4e-3
+    r = rng(sum(case) + 3)
+    xt, x = _to(singa, dev, r.standard_normal((N, C, H, W)).astype(np.float32), kind)
+    wt, w = _to(singa, dev, (r.standard_normal((K, C, 1, 1)) * np.sqrt(2.0 / C)).astype(np.float32), kind)
+    bt, b = _to(singa, dev, r.standard_normal(K).astype(np.float32), kind)
+    dyt, dy = _to(singa, dev, r.standard_normal((N, K, H, W)).astype(np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (1, 1), (1, 1), (0, 0), C, K, True)
+    y, dx = singa.GpuConvForward(xt, wt, bt, h).to_numpy(), singa.GpuConvBackwardx(dyt, wt, xt, h).to_numpy()
+    assert nl2(y, O.conv_fwd(x, w, b, (1, 1), (0, 0))) < bound
+    assert nl2(dx, O.conv_bwd(dy, x, w, (1, 1), (0, 0))[0]) < bound
+
+    def shifted(t):   # the same values one element behind an aligned address
+        room, _ = _to(singa, dev, np.concatenate([[0.0], t.to_numpy().ravel()]).astype(np.float32), kind)
+        return singa.from_device_pointer(room.ptr + 2, t.shape(), dev, t.data_type(), keepalive=room)
+
+    xs, ws, dys = shifted(xt), shifted(wt), shifted(dyt)
+    for got in (singa.GpuConvForward(xs, wt, bt, h), singa.GpuConvForward(xt, ws, bt, h)):
+        _same_bits(got.to_numpy(), y, "forward, one element behind an aligned address")
+    for got in (singa.GpuConvBackwardx(dys, wt, xt, h), singa.GpuConvBackwardx(dyt, ws, xt, h)):
+        _same_bits(got.to_numpy(), dx, "data gradient, one element behind an aligned address")
