@@ -742,7 +742,7 @@ __global__ __launch_bounds__(256) void k_relayout16_fwd(const uint16_t *W, uint1
 //   Staging: a thread owns EV (8 or 4) consecutive pixels of the NCHW tensor and 8 consecutive k (the lanes that
 // share a pixel group take different k octets): it
 // loads the 8 rows with 16- (8-) byte loads, transposes the 8 x EV block in registers (v_perm_b32) and
-// writes one 16-byte octet per pixel to that pixel's slab row (planes are whole groups of EV pixels, so
+// writes one 16-byte octet per pixel to that pixel's slab row (the last group of a plane ends with it, so
 // a group never straddles two images; it may straddle two rows, where the slab row skips the zero
 // position).  Zero positions are written once, at the start.  (2-byte loads, one per element, kept the
 // vector memory path busy for 10 us per slab: 47 cycles per wavefront instruction.)
@@ -803,10 +803,11 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
   const int c0 = (slot % a.mtiles) * BMC, m0 = pt * MT, HW = a.H * a.W;
   const rsrc_t rdy = make_rsrc(a.dy, a.dy_bytes), rwt = make_rsrc(a.wt, a.wt_bytes);
 
-  // This thread's pixel group: number gi among the groups of EV pixels (in tensor order, all images on one
-  // line) from the one that holds the first pixel of the slab; its blocks are k octets ko[j] of a chunk.
+  // This thread's pixel group, counted from the one that holds the first pixel of the slab.  A plane is QO groups of
+  // EV pixels, the last of which ends with the plane and overlaps the one before it (both write the same values to the
+  // slab); its blocks are k octets ko[j] of a chunk.
   const int g_lo = m0 - a.Wp - 1;
-  int voff = kOOB, row0 = a.SP, wrapat = EV, wrapinc = 0;
+  int voff = kOOB, row0 = a.SP, wrapat = EV;
   {
     int n, h, w;
     {
@@ -820,14 +821,13 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
         if (++h == a.H) h = 0, ++n;
       }
     }
-    const long f_lo = long(n) * HW + h * a.W + w;
-    const long f0 = (f_lo / EV + wave * (8 * NB) + lane / KOL) * EV;
-    if (f0 < long(a.N) * HW) {
-      const int n0 = int(f0 / HW), pix = int(f0 - long(n0) * HW), h0 = pix / a.W, w0 = pix - h0 * a.W;
+    const int QO = (HW + EV - 1) / EV;
+    const int gi = (h * a.W + w) / EV + wave * (8 * NB) + lane / KOL, dn = gi / QO, n0 = n + dn;
+    if (n0 < a.N) {
+      const int pix = min((gi - dn * QO) * EV, HW - EV), h0 = pix / a.W, w0 = pix - h0 * a.W;
       row0 = n0 * a.HpWp + h0 * a.Wp + w0 - g_lo;
       wrapat = a.W - w0;
-      wrapinc = 1 + (h0 + 1 == a.H ? a.Wp : 0);
-      const int last = row0 + EV - 1 + (EV - 1 >= wrapat ? wrapinc : 0);
+      const int last = row0 + EV - 1 + (EV - 1 >= wrapat ? 1 : 0);
       if (last >= 0 && row0 < a.SP) voff = (n0 * a.K * HW + pix) * 2;
     }
   }
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
 #pragma unroll
           for (int d = 0; d < 4; ++d)
             v[d] = __builtin_amdgcn_perm(blk[j][2 * d + 1][p >> 1], blk[j][2 * d][p >> 1], (p & 1) ? kSelHi : kSelLo);
-          int row = row0 + p + (p >= wrapat ? wrapinc : 0);
+          int row = row0 + p + (p >= wrapat ? 1 : 0);
           row = unsigned(row) < unsigned(a.SP) ? row : a.SP;
           *reinterpret_cast<u32x4 *>(slab + row * PITCH + ko[j] * 8) = v;
         }
@@ -1073,7 +1073,7 @@ struct D16Plan {
   int cls_tile0[5];
   size_t wt_bytes, dyT_bytes;   // workspace: re-laid weights, then the pixel-major copy
   int fs;             // see D16Args::fs
-  int slab;           // k_dgrad16_slab: 0 no, else the tile: 1 = 64 channels x 256 positions, 2 = 128 x 256, 3 = 128 x 128
+  int slab;           // k_dgrad16_slab: 0 no, else the tile: 1 = 64 channels x 256 positions, 2 = 128 x 256, 3 = 128 x 128, 4 = 64 x 128
   int slab_sp;        // slab entries
   int slab_ev;        // pixels per staging group: 8 or 4
   bool dilate;        // 1x1, stride 2, no padding, even image: see D16Args::dilate
@@ -1106,21 +1106,27 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
     tiles += (long(g->N) * Hc * Wc + BN - 1) / BN;
   }
   for (int cls = st * st; cls < 5; ++cls) p.cls_tile0[cls] = int(tiles);
-  // 3x3 / stride 1 / padding 1 on planes of whole 4- or 8-pixel groups: the slab kernel, when its slab fits beside
-  // the weight tiles in the 160 KB of LDS and a thread per pixel group (two per group of 4) covers it
+  // 3x3 / stride 1 / padding 1: the slab kernel, when its slab fits beside the weight tiles in the 160 KB of LDS and its
+  // threads cover the slab's pixel groups.  Groups of 8 pixels at element alignment, of 4 on rows of 3 to 6 (a group
+  // may end one row and start the next, no more).
   if (fs == 1 && g->R == 3 && g->S == 3 && st == 1 && g->pad_h == 1 && g->pad_w == 1 && !sgh_env().slab16_off &&
-      (g->H * g->W) % 4 == 0 && g->W >= 8) {
-    const long G = long(g->N) * (g->H + 1) * (g->W + 1);
-    const int ev = (g->H * g->W) % 8 == 0 ? 8 : 4;
-    const int bmc = g->C <= 64 ? 64 : 128, mt_c = (g->C + bmc - 1) / bmc;
+      g->W >= 3 && g->H * g->W >= (g->W >= 7 ? 8 : 4)) {
+    static const int tiles[4][3] = {{2, 128, 256}, {3, 128, 128}, {1, 64, 256}, {4, 64, 128}};
+    const long HpWp = long(g->H + 1) * (g->W + 1), G = long(g->N) * HpWp;
+    const int ev = g->W >= 7 ? 8 : 4, QO = (g->H * g->W + ev - 1) / ev;
     const int KP = (g->K + KC - 1) / KC * KC;
-    int mt = 256;
-    if (bmc == 128 && ((G + 255) / 256) * mt_c < sgh_num_cus() * 3 / 4) mt = 128;
-    for (; mt >= (bmc == 128 ? 128 : 256); mt /= 2) {
+    // The largest tile that gives three quarters of the CUs a workgroup, else the smallest one.  us, forward, against the
+    // tap-by-tap kernel (odd planes: on a pixel-major copy): 128 x 512 x 7 x 7 73.3 -> 51.3, 37 x 72 x 31 x 45 -> 136 60.7 ->
+    // 42.9; against 128 x 128 tiles of groups of four: 21 x 256 x 12 x 12 24.5 -> 21.0, 21 x 128 x 24 x 24 16.5 -> 13.7.
+    for (int i = g->C <= 64 ? 2 : 0; i < 4; ++i) {
+      const int bmc = tiles[i][1], mt = tiles[i][2], mt_c = (g->C + bmc - 1) / bmc;
       const int sp = mt + 2 * (g->W + 1) + 2;
       const size_t lds = (size_t(KP > KC ? 2 : 1) * (sp + 1) + 2 * bmc) * PITCH * 2;
-      if (G + 1024 >= (long(1) << 31) || sp / ev + 3 > (ev == 8 ? 64 : 128) || lds > size_t(160) * 1024) continue;
-      p.slab = bmc == 64 ? 1 : (mt == 256 ? 2 : 3);
+      const long images = (sp - 1) / HpWp + 2;   // images a slab can touch; each may add a group at either end
+      const long groups = images * QO < sp / ev + 2 * images ? images * QO : sp / ev + 2 * images;
+      if (G + 1024 >= (long(1) << 31) || groups > (ev == 8 ? 64 : 128) || lds > size_t(160) * 1024) continue;
+      if (i != 3 && (G + mt - 1) / mt * mt_c < sgh_num_cus() * 3 / 4) continue;
+      p.slab = tiles[i][0];
       p.slab_sp = sp, p.slab_ev = ev;
       p.bm = bmc, p.mtiles = mt_c, p.CP = mt_c * bmc, p.KP = KP;
       p.tiles = int((G + mt - 1) / mt);
@@ -1338,7 +1344,8 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     int rc;
     if (p.slab == 1) rc = launch_slab<2, 2, 1, 4>(b, p, bf16, s);
     else if (p.slab == 2) rc = launch_slab<2, 2, 2, 4>(b, p, bf16, s);
-    else rc = launch_slab<2, 2, 2, 2>(b, p, bf16, s);
+    else if (p.slab == 3) rc = launch_slab<2, 2, 2, 2>(b, p, bf16, s);
+    else rc = launch_slab<1, 2, 2, 2>(b, p, bf16, s);
     sgh_prof_kernel_end(s);
     return rc;
   }

@@ -927,3 +927,35 @@ def test_conv_1x1_16bit(singa, dev, kind, case):
         _same_bits(got.to_numpy(), y, "forward, one element behind an aligned address")
     for got in (singa.GpuConvBackwardx(dys, wt, xt, h), singa.GpuConvBackwardx(dyt, ws, xt, h)):
         _same_bits(got.to_numpy(), dx, "data gradient, one element behind an aligned address")
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("case", [
+    # N, C, H, W, K: 3x3 / stride 1 / padding 1 on planes that are no whole groups of pixels
+    (5, 72, 3, 3, 136),     # rows of 3: groups of four that overlap in three, many images in a slab
+    (30, 16, 2, 5, 8),      # 10 pixels, one chunk
+    (9, 256, 6, 6, 64),     # rows of 6: the widest that take groups of four
+    (11, 136, 7, 7, 72),    # rows of 7: groups of eight
+    (3, 64, 2, 7, 40),      # two rows: groups that wrap in every place
+    (40, 128, 9, 31, 24),   # odd planes, 128 x 128 tiles
+    (7, 40, 31, 45, 136),   # ... one tile of channels, mostly empty
+    (1, 16, 5, 109, 16),    # rows longer than a tile's half
+])
+def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
+    """The slab kernel (forward and data gradient) against the oracle: one rounding of a result is at most 2^-11 (binary16) or
+    2^-8 / 2 (bfloat16) of it; the border rows and columns and the last image by themselves."""
+    from oracle import cpu_oracle as O
+    from util import nl2
+    N, C, H, W, K = case
+    print("3x3", kind, case, flush=True)
+    bound = 5e-4 if kind == "f16" else 4e-3
+    r = rng(sum(case) + 4)
+    xt, x = _to(singa, dev, r.standard_normal((N, C, H, W)).astype(np.float32), kind)
+    wt, w = _to(singa, dev, (r.standard_normal((K, C, 3, 3)) * np.sqrt(2.0 / (9 * C))).astype(np.float32), kind)
+    dyt, dy = _to(singa, dev, r.standard_normal((N, K, H, W)).astype(np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (3, 3), (1, 1), (1, 1), C, K, False)
+    for got, want in ((singa.GpuConvForward(xt, wt, None, h).to_numpy(), O.conv_fwd(x, w, None, (1, 1), (1, 1))),
+                      (singa.GpuConvBackwardx(dyt, wt, xt, h).to_numpy(), O.conv_bwd(dy, x, w, (1, 1), (1, 1))[0])):
+        assert nl2(got, want) < bound
+        for part in (np.s_[:, :, 0], np.s_[:, :, -1], np.s_[:, :, :, 0], np.s_[:, :, :, -1], np.s_[-1]):
+            assert nl2(got[part], want[part]) < bound
