@@ -710,6 +710,29 @@ __global__ __launch_bounds__(256) void k_pixel_major16(const uint16_t *__restric
   }
 }
 
+// dst[row][i][j] = src[row][2 i][2 j]: the pixels that a 1x1 forward pass of stride 2 reads (row = (n, c); planes of H x W,
+// copies of P x Q).  V outputs per thread; V > 1: V divides Q and W = 2 Q, so their 2 V elements lie in one row.
+// Bound by bytes (every line of the even rows is fetched).  Copy + k_pw16 against the pixel-major copy of the whole input
+// that the tap-by-tap kernel reads: 128 x 256 x 56 x 56 -> 512 170 -> 98 us, 21 x 256 x 48 x 48 -> 512 24.7 -> 15.4.
+template <int V>
+__global__ __launch_bounds__(256) void k_every_second16(const uint16_t *__restrict__ src, uint16_t *__restrict__ dst, int H, int W,
+                                                       int P, int Q, unsigned groups) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= groups) return;
+  const unsigned QV = unsigned(Q) / V, line = i / QV, j = (i - line * QV) * V, row = line / unsigned(P), p = line - row * unsigned(P);
+  const uint16_t *from = src + (size_t(row) * H + 2 * p) * W + 2 * j;
+  uint16_t *to = dst + size_t(i) * V;
+  if constexpr (V == 1) {
+    *to = *from;
+  } else {
+    unsigned in[V], out[V / 2];
+    __builtin_memcpy(in, from, 4 * V);
+#pragma unroll
+    for (int e = 0; e < V / 2; ++e) out[e] = __builtin_amdgcn_perm(in[2 * e + 1], in[2 * e], kSelLo);
+    __builtin_memcpy(to, out, 2 * V);
+  }
+}
+
 // wt[tap][c][k] (c < CP, k < KP; zero beyond C / K) from W[k][c][r][s]
 __global__ __launch_bounds__(256) void k_relayout16(const uint16_t *W, uint16_t *wt, int K, int C, int RS, int KP, int CP) {
   const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x, n = size_t(RS) * CP * KP;
@@ -1071,13 +1094,14 @@ struct D16Plan {
   bool pixk;   // several taps: the kernel reads a pixel-major copy of the gradient (k_pixel_major16)
   int bm, mtiles, KP, CP, tiles;
   int cls_tile0[5];
-  size_t wt_bytes, dyT_bytes;   // workspace: re-laid weights, then the pixel-major copy
+  size_t wt_bytes, dyT_bytes;   // workspace: re-laid weights, then the pixel-major copy (pw: the copied pixels)
   int fs;             // see D16Args::fs
   int slab;           // k_dgrad16_slab: 0 no, else the tile: 1 = 64 channels x 256 positions, 2 = 128 x 256, 3 = 128 x 128, 4 = 64 x 128
   int slab_sp;        // slab entries
   int slab_ev;        // pixels per staging group: 8 or 4
   bool dilate;        // 1x1, stride 2, no padding, even image: see D16Args::dilate
-  bool pw;            // 1x1, stride 1, no padding: k_pw16 (tiles counts octets of planes, 16 a tile)
+  bool pw;            // 1x1, no padding: k_pw16 (tiles counts octets of planes, 16 a tile); a forward pass of stride 2
+                      // runs on a copy of the pixels that it reads (k_every_second16)
   sgh_conv_geom kg;   // the geometry the kernel sees (the stride-1 problem on the P x Q grid when `dilate`)
 };
 
@@ -1118,7 +1142,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
     // The largest tile that gives three quarters of the CUs a workgroup, else the smallest one.  us, forward, against the
     // tap-by-tap kernel (odd planes: on a pixel-major copy): 128 x 512 x 7 x 7 73.3 -> 51.3, 37 x 72 x 31 x 45 -> 136 60.7 ->
     // 42.9; against 128 x 128 tiles of groups of four: 21 x 256 x 12 x 12 24.5 -> 21.0, 21 x 128 x 24 x 24 16.5 -> 13.7.
-    for (int i = g->C <= 64 ? 2 : 0; i < 4; ++i) {
+    for (int i = g->C <= 64 ? 2 : 0; i < 4; ++i) {   // (129 to 192 channels on three tiles of 64 instead: 42.9 -> 44.6)
       const int bmc = tiles[i][1], mt = tiles[i][2], mt_c = (g->C + bmc - 1) / bmc;
       const int sp = mt + 2 * (g->W + 1) + 2;
       const size_t lds = (size_t(KP > KC ? 2 : 1) * (sp + 1) + 2 * bmc) * PITCH * 2;
@@ -1137,7 +1161,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
       return p;
     }
   }
-  if (fs == 1 && !p.dilate && g->R == 1 && g->S == 1 && st == 1 && g->pad_h == 0 && g->pad_w == 0 && g->H * g->W >= 8) {
+  if (!p.dilate && g->R == 1 && g->S == 1 && st == 1 && g->pad_h == 0 && g->pad_w == 0 && g->H * g->W >= 8) {
     const long octets = long(g->N) * ((g->H * g->W + 7) / 8);
     p.pw = true;
     p.tiles = int((octets + 15) / 16);
@@ -1146,6 +1170,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
     p.CP = p.mtiles * p.bm, p.KP = (g->K + KC - 1) / KC * KC;
     if (octets >= (long(1) << 30) || long(p.tiles) * p.mtiles >= (long(1) << 30) || size_t(p.CP) * p.KP >= lim) return p;
     p.wt_bytes = align256(size_t(p.CP) * p.KP * sizeof(uint16_t));
+    p.dyT_bytes = fs == 1 ? 0 : align256(size_t(g->N) * g->K * g->H * g->W * sizeof(uint16_t));
     p.ok = true;
     return p;
   }
@@ -1350,6 +1375,17 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     return rc;
   }
   if (p.pw) {
+    if (p.fs == 2) {
+      uint16_t *to = reinterpret_cast<uint16_t *>(static_cast<char *>(workspace) + p.wt_bytes);
+      const size_t n = size_t(g->N) * g->K * g->H * g->W;
+      const int v = g->Q != 2 * g->W || g->W % 2 ? 1 : (g->W % 4 ? 2 : 4);
+      const dim3 grid(unsigned((n / v + 255) / 256));
+      if (v == 4) hipLaunchKernelGGL(k_every_second16<4>, grid, dim3(256), 0, s, dy, to, g->P, g->Q, g->H, g->W, unsigned(n / 4));
+      else if (v == 2) hipLaunchKernelGGL(k_every_second16<2>, grid, dim3(256), 0, s, dy, to, g->P, g->Q, g->H, g->W, unsigned(n / 2));
+      else hipLaunchKernelGGL(k_every_second16<1>, grid, dim3(256), 0, s, dy, to, g->P, g->Q, g->H, g->W, unsigned(n));
+      if (hipGetLastError() != hipSuccess) return SGH_EINVAL;
+      dy = to;
+    }
     sgh_pw16_args b{};
     b.A = as_is ? W : wt, b.src = dy, b.out = dx, b.bias = bias;
     b.M = g->C, b.K = g->K, b.HW = g->H * g->W, b.lda = p.KP;

@@ -959,3 +959,21 @@ def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
         assert nl2(got, want) < bound
         for part in (np.s_[:, :, 0], np.s_[:, :, -1], np.s_[:, :, :, 0], np.s_[:, :, :, -1], np.s_[-1]):
             assert nl2(got[part], want[part]) < bound
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("case", [(2, 64, 16, 24, 40), (3, 40, 12, 20, 24), (2, 72, 14, 14, 136), (2, 16, 9, 11, 8), (1, 16, 4, 10, 64),
+                                  (1, 64, 7, 4, 16)])
+def test_conv_1x1_stride2_forward_16bit(singa, dev, kind, case):
+    """1x1 of stride 2 (a copy of the pixels that are read, by four, two and one; then the pointwise kernel) against the oracle:
+    one rounding of a result is at most 2^-11 (binary16) or 2^-8 / 2 (bfloat16) of it."""
+    from oracle import cpu_oracle as O
+    from util import nl2
+    N, C, H, W, K = case
+    print("1x1 stride 2", kind, case, flush=True)
+    r = rng(sum(case) + 6)
+    xt, x = _to(singa, dev, r.standard_normal((N, C, H, W)).astype(np.float32), kind)
+    wt, w = _to(singa, dev, (r.standard_normal((K, C, 1, 1)) * np.sqrt(2.0 / C)).astype(np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (1, 1), (2, 2), (0, 0), C, K, False)
+    y = singa.GpuConvForward(xt, wt, None, h).to_numpy()
+    assert nl2(y, O.conv_fwd(x, w, None, (2, 2), (0, 0))) < (5e-4 if kind == "f16" else 4e-3)
