@@ -35,7 +35,15 @@ template <class T>
 struct Arg;
 template <class T>
 struct Arg<T *> {
-  static T *from(PyObject *o) { return o == Py_None ? nullptr : static_cast<T *>(PyLong_AsVoidPtr(o)); }
+  static T *from(PyObject *o) {
+    if (o == Py_None) return nullptr;
+    if (PyLong_Check(o)) return static_cast<T *>(PyLong_AsVoidPtr(o));
+    PyObject *v = PyObject_GetAttrString(o, "value");   // a ctypes.c_void_p, as a caller's own stream may come
+    if (!v) return nullptr;
+    T *p = v == Py_None ? nullptr : static_cast<T *>(PyLong_AsVoidPtr(v));
+    Py_DECREF(v);
+    return p;
+  }
 };
 template <>
 struct Arg<int> {

@@ -234,6 +234,11 @@ class Tensor(_native.TensorBase):
         self._transposed = _transposed
         self._block = _block if _block is not None else _Block(device, self.MemSize())
 
+    def __copy__(self):   # (the fields are not in __dict__)
+        t = Tensor(self._shape, self._dev, self._dtype, _block=self._block, _transposed=self._transposed)
+        t.__dict__.update(self.__dict__)
+        return t
+
     # --- views
     def Reshape(self, shape):
         shape = tuple(int(s) for s in shape)

@@ -263,3 +263,19 @@ int main(int argc, char **argv) {
     assert int(out[1]) == lib.sgh_conv_workspace_bytes(C.byref(g), _lib.SGH_CONV_DGRAD)
     assert int(out[2]) == lib.sgh_bn_workspace_bytes(64, 64, 3136)
     assert "workspace" in out[3] and "non-allocating" in out[3]
+
+
+def test_tensors_and_pointer_arguments_keep_the_python_protocols():
+    """A shallow copy is a view of the same block, and addresses may come as ctypes.c_void_p (no GPU call: an empty operation
+    returns before any launch, a null pointer is refused)."""
+    import copy
+
+    from singa_amd import _native, singa_wrap as singa
+    dev = object()
+    t = singa.Tensor((3, 5), dev, singa.kFloat16, _block=_native.Block(dev, 30, 4096, None), _transposed=True)
+    c = copy.copy(t)
+    assert c.shape() == [3, 5] and c.data_type() == singa.kFloat16 and c.transpose() and c.ptr == 4096 and c.device() is dev
+    for null in (None, 0, C.c_void_p()):
+        assert _native.sgh_relu_fwd_f32(null, null, 4, None) == _lib.lib().sgh_relu_fwd_f32(None, None, 4, None) < 0
+    with pytest.raises((TypeError, AttributeError)):
+        _native.sgh_relu_fwd_f32("x", None, 4, None)
