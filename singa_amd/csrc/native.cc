@@ -132,11 +132,24 @@ PyObject *block_tp_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
   return reinterpret_cast<PyObject *>(block_new(type, dev, nbytes, p, keepalive));
 }
 
+// (the owner of wrapped memory may hold the tensor that keeps it alive)
+int block_traverse(PyObject *self, visitproc visit, void *arg) {
+  Py_VISIT(reinterpret_cast<Block *>(self)->dev);
+  Py_VISIT(reinterpret_cast<Block *>(self)->keepalive);
+  return 0;
+}
+
+int block_clear(PyObject *self) {
+  Py_CLEAR(reinterpret_cast<Block *>(self)->dev);
+  Py_CLEAR(reinterpret_cast<Block *>(self)->keepalive);
+  return 0;
+}
+
 void block_dealloc(PyObject *self) {
+  PyObject_GC_UnTrack(self);
   Block *b = reinterpret_cast<Block *>(self);
   if (b->owned && b->ptr) sgh_free(b->handle, b->ptr);
-  Py_XDECREF(b->dev);
-  Py_XDECREF(b->keepalive);
+  block_clear(self);
   Py_XDECREF(b->address);
   Py_TYPE(self)->tp_free(self);
 }
@@ -361,9 +374,11 @@ PyMODINIT_FUNC PyInit__native() {
   BlockType.tp_name = "singa_amd._native.Block";
   BlockType.tp_doc = "Block(dev, nbytes, ptr=None, keepalive=None): a pool allocation, or memory owned elsewhere";
   BlockType.tp_basicsize = sizeof(Block);
-  BlockType.tp_flags = Py_TPFLAGS_DEFAULT;
+  BlockType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
   BlockType.tp_new = block_tp_new;
   BlockType.tp_dealloc = block_dealloc;
+  BlockType.tp_traverse = block_traverse;
+  BlockType.tp_clear = block_clear;
   BlockType.tp_members = block_members;
   TensorType.tp_name = "singa_amd._native.TensorBase";
   TensorType.tp_doc = "the fields of a tensor and their accessors";

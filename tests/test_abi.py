@@ -279,3 +279,21 @@ def test_tensors_and_pointer_arguments_keep_the_python_protocols():
         assert _native.sgh_relu_fwd_f32(null, null, 4, None) == _lib.lib().sgh_relu_fwd_f32(None, None, 4, None) < 0
     with pytest.raises((TypeError, AttributeError)):
         _native.sgh_relu_fwd_f32("x", None, 4, None)
+
+
+def test_a_cycle_through_a_tensors_owner_is_collected():
+    """An object that keeps a tensor over its own memory, `keepalive` being the object itself, goes away."""
+    import gc
+    import weakref
+
+    from singa_amd import singa_wrap as singa
+
+    class Owner(object):
+        pass
+
+    owner = Owner()
+    owner.tensor = singa.from_device_pointer(4096, (3,), object(), singa.kFloat32, keepalive=owner)
+    alive = weakref.ref(owner)
+    del owner
+    gc.collect()
+    assert alive() is None
