@@ -97,10 +97,10 @@ struct Block {
 };
 extern PyTypeObject BlockType;
 
-// A block of the device's pool (ptr null), or around memory that someone else owns
-Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, void *ptr, PyObject *keepalive) {
+// A block of the device's pool, or (`external`) around memory that someone else owns, at any address: null as well
+Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, bool external, void *ptr, PyObject *keepalive) {
   sgh_device *h = nullptr;
-  if (!ptr) {
+  if (!external) {
     PyObject *ho = PyObject_GetAttr(dev, g_handle_name);
     if (!ho) return nullptr;
     h = static_cast<sgh_device *>(PyLong_AsVoidPtr(ho));
@@ -113,7 +113,7 @@ Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, void *ptr
     if (h) sgh_free(h, ptr);
     return nullptr;
   }
-  b->handle = h, b->ptr = ptr, b->nbytes = nbytes, b->owned = h != nullptr;
+  b->handle = h, b->ptr = ptr, b->nbytes = nbytes, b->owned = !external;
   Py_INCREF(dev);
   b->dev = dev;
   Py_XINCREF(keepalive);
@@ -129,7 +129,7 @@ PyObject *block_tp_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
   if (!PyArg_ParseTupleAndKeywords(args, kw, "On|OO", const_cast<char **>(names), &dev, &nbytes, &ptr, &keepalive)) return nullptr;
   void *p = ptr == Py_None ? nullptr : PyLong_AsVoidPtr(ptr);
   if (PyErr_Occurred()) return nullptr;
-  return reinterpret_cast<PyObject *>(block_new(type, dev, nbytes, p, keepalive));
+  return reinterpret_cast<PyObject *>(block_new(type, dev, nbytes, ptr != Py_None, p, keepalive));
 }
 
 // (the owner of wrapped memory may hold the tensor that keeps it alive)
@@ -196,7 +196,7 @@ inline Py_ssize_t elem_size(int dtype) { return dtype == 1 || dtype == 100 ? 2 :
 PyObject *tensor_make(PyTypeObject *type, PyObject *shape, PyObject *dev, int dtype) {
   const Py_ssize_t n = count_of(shape);
   if (n < 0 && PyErr_Occurred()) return nullptr;
-  Block *b = block_new(&BlockType, dev, n * elem_size(dtype), nullptr, nullptr);
+  Block *b = block_new(&BlockType, dev, n * elem_size(dtype), false, nullptr, nullptr);
   if (!b) return nullptr;
   PyObject *o = type->tp_alloc(type, 0);
   if (!o) {

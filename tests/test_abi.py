@@ -297,3 +297,13 @@ def test_a_cycle_through_a_tensors_owner_is_collected():
     del owner
     gc.collect()
     assert alive() is None
+
+
+def test_memory_wrapped_at_a_null_address_stays_external():
+    """An address of 0 (an empty or unallocated foreign buffer) is not a request for pool memory: the entry points see the null
+    pointer and refuse it."""
+    from singa_amd import _native, singa_wrap as singa
+    t = singa.from_device_pointer(0, (4,), object(), singa.kFloat32)   # (an object without a device handle has no pool)
+    assert t.ptr == 0 and not t._block.owned and t._block.nbytes == 16
+    assert _native.sgh_relu_fwd_f32(t.ptr, t.ptr, t.Size(), None) < 0
+    assert singa.from_device_pointer(0, (0,), object(), singa.kFloat32).Size() == 0
