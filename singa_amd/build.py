@@ -70,7 +70,7 @@ def build_native(verbose=True):
     """The CPython extension on top of the library (host code only)."""
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
            "-I", os.path.join(ROOT, "include"), "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "native.cc"),
-           "-o", NATIVEPATH, "-L", LIBDIR, "-lsinga_hip", "-Wl,-rpath,$ORIGIN/lib"]
+           "-o", NATIVEPATH, "-ldl"]   # (not linked against the library: the first call opens it)
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)

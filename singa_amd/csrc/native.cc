@@ -8,6 +8,7 @@
 #include <Python.h>
 #include <structmember.h>
 
+#include <dlfcn.h>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -19,7 +20,63 @@
 namespace {
 
 PyObject *g_check;   // singa_amd._lib.check(rc, what): raises the library's message
+PyObject *g_open;    // opens the library and returns its dlopen handle
 PyObject *g_handle_name;
+
+// The library is opened by the first call into it, not by loading this module: a program may import torch after this
+// package, and the library has to find the HIP runtime that torch brought, not put a second one into the process.
+void *g_library;
+
+void *entry_point(const char *name) {   // null with an exception set
+  if (!g_library) {
+    PyObject *h = PyObject_CallFunction(g_open, nullptr);
+    if (!h) return nullptr;
+    g_library = PyLong_AsVoidPtr(h);
+    Py_DECREF(h);
+    if (!g_library) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the library has no handle");
+      return nullptr;
+    }
+  }
+  void *p = dlsym(g_library, name);
+  if (!p) PyErr_Format(PyExc_AttributeError, "%s is not in the library", name);
+  return p;
+}
+
+// The address of an entry point with the type that the header declares; SGH_ENTRY(name)::get() is null with an exception
+// set when the library cannot be opened
+template <class F>
+struct EntryOf {
+  template <class N>
+  static F get() {
+    static F found = nullptr;
+    if (!found) found = reinterpret_cast<F>(entry_point(N::text));
+    return found;
+  }
+};
+#define SGH_ENTRY(name)                                                          \
+  struct Entry_##name {                                                          \
+    typedef decltype(&::name) type;                                              \
+    static constexpr const char *text = #name;                                   \
+    static type get() { return EntryOf<type>::template get<Entry_##name>(); }    \
+  };
+#define SGH_ENTRY3(name) SGH_ENTRY(name##_f32) SGH_ENTRY(name##_f16) SGH_ENTRY(name##_bf16)
+// what the methods below call by name
+#define SGH_CALLS(ONE, ALL)                                                                                                     \
+  ONE(sgh_device_join) ONE(sgh_block_used_on) ALL(sgh_memset) ALL(sgh_relu_fwd) ALL(sgh_relu_bwd) ALL(sgh_relu_bwd_add)         \
+  ALL(sgh_add) ALL(sgh_add_relu) ALL(sgh_eltwise_mult) ALL(sgh_axpy) ONE(sgh_axpy_devalpha_f32) ONE(sgh_sub_f32)                \
+  ONE(sgh_div_f32) ONE(sgh_add_scalar_f32) ONE(sgh_mult_scalar_f32) ONE(sgh_clamp_f32) ONE(sgh_cast_f32_to_f16)                 \
+  ONE(sgh_cast_f16_to_f32) ONE(sgh_cast_f32_to_bf16) ONE(sgh_cast_bf16_to_f32) ONE(sgh_cast_f32_to_i32)                         \
+  ONE(sgh_cast_i32_to_f32) ALL(sgh_softmax_ce_bwd) ONE(sgh_softmax_fwd_f32) ONE(sgh_cross_entropy_fwd_f32) ALL(sgh_gemm)        \
+  ONE(sgh_sum_rows_f32) ONE(sgh_add_row_f32) ONE(sgh_row_max_f32) ONE(sgh_row_max_zero_seeded_f32) ONE(sgh_dot_f32)             \
+  ONE(sgh_sum_all_f32) ALL(sgh_sgd_momentum) ONE(sgh_sgd_momentum_multi_f32) ONE(sgh_sgd_momentum_multi_mixed)                  \
+  ONE(sgh_sgd_momentum_master_f16) ONE(sgh_sgd_momentum_master_bf16) ALL(sgh_conv_fwd) ALL(sgh_conv_dgrad) ALL(sgh_conv_wgrad)  \
+  ALL(sgh_conv_bgrad) ONE(sgh_conv_dgrad_acc_f32) ONE(sgh_conv_wgrad_bias_f32) ALL(sgh_bn_fwd_train) ALL(sgh_bn_relu_fwd_train) \
+  ALL(sgh_bn_add_relu_fwd_train) ALL(sgh_bn_fwd_infer) ALL(sgh_bn_bwd) ALL(sgh_bn_relu_bwd) ALL(sgh_pool_fwd) ALL(sgh_pool_bwd)
+SGH_CALLS(SGH_ENTRY, SGH_ENTRY3)
+SGH_ENTRY(sgh_malloc)
+SGH_ENTRY(sgh_free)
+SGH_ENTRY(sgh_device_fork)
 
 bool failed(int rc, const char *what) {
   if (rc == 0) return false;
@@ -62,17 +119,19 @@ struct Arg<float> {
   static float from(PyObject *o) { return float(PyFloat_AsDouble(o)); }
 };
 
-template <auto F>
+template <class E, class F = typename E::type>
 struct Call;
-template <class... A, int (*F)(A...)>
-struct Call<F> {
+template <class E, class... A>
+struct Call<E, int (*)(A...)> {
   template <size_t... I>
   static PyObject *with(PyObject *const *args, std::integer_sequence<size_t, I...>) {
     const std::tuple<A...> a{Arg<A>::from(args[I])...};
     if (PyErr_Occurred()) return nullptr;
+    const typename E::type f = E::get();
+    if (!f) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = F(std::get<I>(a)...);
+    rc = f(std::get<I>(a)...);
     Py_END_ALLOW_THREADS
     return PyLong_FromLong(rc);
   }
@@ -106,11 +165,12 @@ Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, bool exte
     h = static_cast<sgh_device *>(PyLong_AsVoidPtr(ho));
     Py_DECREF(ho);
     if (PyErr_Occurred()) return nullptr;
-    if (failed(sgh_malloc(h, &ptr, nbytes > 0 ? size_t(nbytes) : 1), "sgh_malloc")) return nullptr;
+    const Entry_sgh_malloc::type take = Entry_sgh_malloc::get();
+    if (!take || !Entry_sgh_free::get() || failed(take(h, &ptr, nbytes > 0 ? size_t(nbytes) : 1), "sgh_malloc")) return nullptr;
   }
   Block *b = reinterpret_cast<Block *>(type->tp_alloc(type, 0));
   if (!b) {
-    if (h) sgh_free(h, ptr);
+    if (h) Entry_sgh_free::get()(h, ptr);
     return nullptr;
   }
   b->handle = h, b->ptr = ptr, b->nbytes = nbytes, b->owned = !external;
@@ -148,7 +208,7 @@ int block_clear(PyObject *self) {
 void block_dealloc(PyObject *self) {
   PyObject_GC_UnTrack(self);
   Block *b = reinterpret_cast<Block *>(self);
-  if (b->owned && b->ptr) sgh_free(b->handle, b->ptr);
+  if (b->owned && b->ptr) Entry_sgh_free::get()(b->handle, b->ptr);
   block_clear(self);
   Py_XDECREF(b->address);
   Py_TYPE(self)->tp_free(self);
@@ -332,37 +392,32 @@ PyObject *set_check(PyObject *, PyObject *f) {
   Py_RETURN_NONE;
 }
 
+PyObject *set_open(PyObject *, PyObject *f) {
+  Py_INCREF(f);
+  Py_XSETREF(g_open, f);
+  Py_RETURN_NONE;
+}
+
 // fork(handle): the auxiliary stream's address
 PyObject *fork_(PyObject *, PyObject *h) {
   void *aux = nullptr;
   sgh_device *d = static_cast<sgh_device *>(PyLong_AsVoidPtr(h));
-  if (PyErr_Occurred() || failed(sgh_device_fork(d, &aux), "sgh_device_fork")) return nullptr;
+  if (PyErr_Occurred()) return nullptr;
+  const Entry_sgh_device_fork::type split = Entry_sgh_device_fork::get();
+  if (!split || failed(split(d, &aux), "sgh_device_fork")) return nullptr;
   return PyLong_FromVoidPtr(aux);
 }
 
-#define SGH_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call<&name>::call)), METH_FASTCALL, nullptr}
-#define SGH_CALL3(name) SGH_CALL(name##_f32), SGH_CALL(name##_f16), SGH_CALL(name##_bf16)
+#define SGH_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call<Entry_##name>::call)), METH_FASTCALL, nullptr},
+#define SGH_CALL3(name) SGH_CALL(name##_f32) SGH_CALL(name##_f16) SGH_CALL(name##_bf16)
 
 PyMethodDef methods[] = {
     {"set_check", set_check, METH_O, "the function that turns a return code into an exception"},
+    {"set_open", set_open, METH_O, "the function that opens the library and returns its handle"},
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(empty)), METH_FASTCALL, "empty(cls, shape, device, dtype)"},
     {"empty_like", empty_like, METH_O, "a dense tensor of the same shape, device and type"},
     {"fork", fork_, METH_O, "sgh_device_fork: the auxiliary stream"},
-    SGH_CALL(sgh_device_join), SGH_CALL(sgh_block_used_on),
-    SGH_CALL3(sgh_memset), SGH_CALL3(sgh_relu_fwd), SGH_CALL3(sgh_relu_bwd), SGH_CALL3(sgh_relu_bwd_add), SGH_CALL3(sgh_add),
-    SGH_CALL3(sgh_add_relu), SGH_CALL3(sgh_eltwise_mult), SGH_CALL3(sgh_axpy), SGH_CALL(sgh_axpy_devalpha_f32),
-    SGH_CALL(sgh_sub_f32), SGH_CALL(sgh_div_f32), SGH_CALL(sgh_add_scalar_f32), SGH_CALL(sgh_mult_scalar_f32),
-    SGH_CALL(sgh_clamp_f32), SGH_CALL(sgh_cast_f32_to_f16), SGH_CALL(sgh_cast_f16_to_f32), SGH_CALL(sgh_cast_f32_to_bf16),
-    SGH_CALL(sgh_cast_bf16_to_f32), SGH_CALL(sgh_cast_f32_to_i32), SGH_CALL(sgh_cast_i32_to_f32),
-    SGH_CALL3(sgh_softmax_ce_bwd), SGH_CALL(sgh_softmax_fwd_f32), SGH_CALL(sgh_cross_entropy_fwd_f32),
-    SGH_CALL3(sgh_gemm), SGH_CALL(sgh_sum_rows_f32), SGH_CALL(sgh_add_row_f32), SGH_CALL(sgh_row_max_f32),
-    SGH_CALL(sgh_row_max_zero_seeded_f32), SGH_CALL(sgh_dot_f32), SGH_CALL(sgh_sum_all_f32),
-    SGH_CALL3(sgh_sgd_momentum), SGH_CALL(sgh_sgd_momentum_multi_f32), SGH_CALL(sgh_sgd_momentum_multi_mixed),
-    SGH_CALL(sgh_sgd_momentum_master_f16), SGH_CALL(sgh_sgd_momentum_master_bf16),
-    SGH_CALL3(sgh_conv_fwd), SGH_CALL3(sgh_conv_dgrad), SGH_CALL3(sgh_conv_wgrad), SGH_CALL3(sgh_conv_bgrad),
-    SGH_CALL(sgh_conv_dgrad_acc_f32), SGH_CALL(sgh_conv_wgrad_bias_f32),
-    SGH_CALL3(sgh_bn_fwd_train), SGH_CALL3(sgh_bn_relu_fwd_train), SGH_CALL3(sgh_bn_add_relu_fwd_train), SGH_CALL3(sgh_bn_fwd_infer),
-    SGH_CALL3(sgh_bn_bwd), SGH_CALL3(sgh_bn_relu_bwd), SGH_CALL3(sgh_pool_fwd), SGH_CALL3(sgh_pool_bwd),
+    SGH_CALLS(SGH_CALL, SGH_CALL3)
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "tensors, memory blocks and direct calls into libsinga_hip", -1, methods,

@@ -26,6 +26,7 @@ from . import _native
 from ._lib import SingaHipError, check  # noqa: F401  (re-exported)
 
 _native.set_check(check)
+_native.set_open(lambda: _lib.lib()._handle)
 
 # core.proto DataType values (src/proto/core.proto:26-34)
 kFloat32, kFloat16, kInt = 0, 1, 2

@@ -4,6 +4,7 @@ import ctypes as C
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -307,3 +308,18 @@ def test_memory_wrapped_at_a_null_address_stays_external():
     assert t.ptr == 0 and not t._block.owned and t._block.nbytes == 16
     assert _native.sgh_relu_fwd_f32(t.ptr, t.ptr, t.Size(), None) < 0
     assert singa.from_device_pointer(0, (0,), object(), singa.kFloat32).Size() == 0
+
+
+def test_importing_the_package_loads_no_hip_runtime():
+    """The library is opened by the first call, so that a torch imported after this package still brings the only HIP runtime
+    of the process."""
+    program = """
+import singa_amd.singa_wrap, singa_amd.opt, singa_amd.workloads
+loaded = lambda: {l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l or "libsinga_hip" in l}
+assert not loaded(), loaded()
+import torch
+from singa_amd import _native
+assert _native.sgh_relu_fwd_f32(None, None, 4, None) < 0     # opens the library; a null pointer is refused
+assert sum("libamdhip64" in l for l in loaded()) == 1 and sum("libsinga_hip" in l for l in loaded()) == 1, loaded()
+"""
+    subprocess.run([sys.executable, "-c", program], check=True, cwd=ROOT, timeout=300)
