@@ -166,7 +166,12 @@ Block *block_new(PyTypeObject *type, PyObject *dev, Py_ssize_t nbytes, bool exte
     Py_DECREF(ho);
     if (PyErr_Occurred()) return nullptr;
     const Entry_sgh_malloc::type take = Entry_sgh_malloc::get();
-    if (!take || !Entry_sgh_free::get() || failed(take(h, &ptr, nbytes > 0 ? size_t(nbytes) : 1), "sgh_malloc")) return nullptr;
+    if (!take || !Entry_sgh_free::get()) return nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS   // (a miss of the pool waits for the driver)
+    rc = take(h, &ptr, nbytes > 0 ? size_t(nbytes) : 1);
+    Py_END_ALLOW_THREADS
+    if (failed(rc, "sgh_malloc")) return nullptr;
   }
   Block *b = reinterpret_cast<Block *>(type->tp_alloc(type, 0));
   if (!b) {
@@ -208,7 +213,12 @@ int block_clear(PyObject *self) {
 void block_dealloc(PyObject *self) {
   PyObject_GC_UnTrack(self);
   Block *b = reinterpret_cast<Block *>(self);
-  if (b->owned && b->ptr) Entry_sgh_free::get()(b->handle, b->ptr);
+  if (b->owned && b->ptr) {
+    const Entry_sgh_free::type give = Entry_sgh_free::get();   // (found before the block was made)
+    Py_BEGIN_ALLOW_THREADS
+    give(b->handle, b->ptr);
+    Py_END_ALLOW_THREADS
+  }
   block_clear(self);
   Py_XDECREF(b->address);
   Py_TYPE(self)->tp_free(self);
@@ -404,7 +414,12 @@ PyObject *fork_(PyObject *, PyObject *h) {
   sgh_device *d = static_cast<sgh_device *>(PyLong_AsVoidPtr(h));
   if (PyErr_Occurred()) return nullptr;
   const Entry_sgh_device_fork::type split = Entry_sgh_device_fork::get();
-  if (!split || failed(split(d, &aux), "sgh_device_fork")) return nullptr;
+  if (!split) return nullptr;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = split(d, &aux);
+  Py_END_ALLOW_THREADS
+  if (failed(rc, "sgh_device_fork")) return nullptr;
   return PyLong_FromVoidPtr(aux);
 }
 

@@ -323,3 +323,47 @@ assert _native.sgh_relu_fwd_f32(None, None, 4, None) < 0     # opens the library
 assert sum("libamdhip64" in l for l in loaded()) == 1 and sum("libsinga_hip" in l for l in loaded()) == 1, loaded()
 """
     subprocess.run([sys.executable, "-c", program], check=True, cwd=ROOT, timeout=300)
+
+
+def test_pool_calls_let_other_threads_run(tmp_path):
+    """Taking and returning pool memory releases the interpreter lock: a stand-in for the library waits in both calls until
+    another thread has called into it (at most three seconds, then it refuses)."""
+    source = tmp_path / "stub.cc"
+    source.write_text("""
+#include <stddef.h>
+#include <atomic>
+#include <chrono>
+#include <thread>
+static std::atomic<int> calls{0}, late{0};
+static int wait_for(int n) {
+  for (int i = 0; i < 3000; ++i) {
+    if (calls >= n) return 0;
+    std::this_thread::sleep_for(std::chrono::milliseconds(1));
+  }
+  ++late;
+  return 0;
+}
+extern "C" {
+int sgh_malloc(void *, void **p, size_t) { *p = reinterpret_cast<void *>(4096); return wait_for(1); }
+int sgh_free(void *, void *) { return wait_for(2); }
+void other_thread() { ++calls; }
+int waits_in_vain() { return late; }
+}
+""")
+    stub = str(tmp_path / "libstub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", str(source), "-o", stub], check=True)
+    program = """
+import ctypes, sys, threading, time
+from singa_amd import _native
+stub = ctypes.CDLL(sys.argv[1])
+_native.set_open(lambda: stub._handle)
+class Device(object):
+    _handle = 1
+for step in (lambda: globals().__setitem__("block", _native.Block(Device(), 64)), lambda: globals().__delitem__("block")):
+    other = threading.Timer(0.1, stub.other_thread)
+    other.start()
+    step()
+    other.join()
+assert stub.waits_in_vain() == 0, stub.waits_in_vain()
+"""
+    subprocess.run([sys.executable, "-c", program, stub], check=True, cwd=ROOT, timeout=60)
