@@ -21,6 +21,7 @@ namespace {
 
 PyObject *g_check;   // singa_amd._lib.check(rc, what): raises the library's message
 PyObject *g_open;    // opens the library and returns its dlopen handle
+PyObject *g_tensor;  // singa_amd.singa_wrap.Tensor: the class of results
 PyObject *g_handle_name;
 
 // The library is opened by the first call into it, not by loading this module: a program may import torch after this
@@ -112,7 +113,13 @@ struct Arg<int> {
 };
 template <>
 struct Arg<size_t> {
-  static size_t from(PyObject *o) { return PyLong_AsSize_t(o); }
+  static size_t from(PyObject *o) {
+    PyObject *i = PyNumber_Index(o);   // (whole numbers of numpy as well)
+    if (!i) return 0;
+    const size_t v = PyLong_AsSize_t(i);
+    Py_DECREF(i);
+    return v;
+  }
 };
 template <>
 struct Arg<float> {
@@ -246,7 +253,8 @@ extern PyTypeObject TensorType;
 
 inline Tensor *as_tensor(PyObject *o) { return reinterpret_cast<Tensor *>(o); }
 
-// product of the extents, -1 with an exception set when `shape` is not a tuple of whole numbers
+// product of the extents, -1 with an exception set when `shape` is not a tuple of whole numbers or the product leaves no room
+// for an element's size
 Py_ssize_t count_of(PyObject *shape) {
   if (!shape || !PyTuple_Check(shape)) {
     PyErr_SetString(PyExc_TypeError, "a tensor's shape is a tuple");
@@ -254,8 +262,12 @@ Py_ssize_t count_of(PyObject *shape) {
   }
   Py_ssize_t n = 1;
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(shape); ++i) {
-    n *= PyLong_AsSsize_t(PyTuple_GET_ITEM(shape, i));
+    const Py_ssize_t e = PyLong_AsSsize_t(PyTuple_GET_ITEM(shape, i));
     if (PyErr_Occurred()) return -1;
+    if (__builtin_mul_overflow(n, e, &n) || n > PY_SSIZE_T_MAX / 4) {
+      PyErr_SetString(PyExc_OverflowError, "a tensor of this shape cannot be addressed");
+      return -1;
+    }
   }
   return n;
 }
@@ -303,7 +315,11 @@ PyObject *empty_like(PyObject *, PyObject *o) {   // a dense tensor of o's shape
     PyErr_SetString(PyExc_AttributeError, "the tensor has no device");
     return nullptr;
   }
-  return tensor_make(Py_TYPE(o), t->shape, t->dev, t->dtype);
+  if (!g_tensor) {
+    PyErr_SetString(PyExc_RuntimeError, "no tensor class has been set");
+    return nullptr;
+  }
+  return tensor_make(reinterpret_cast<PyTypeObject *>(g_tensor), t->shape, t->dev, t->dtype);
 }
 
 int tensor_traverse(PyObject *self, visitproc visit, void *arg) {
@@ -328,11 +344,14 @@ void tensor_dealloc(PyObject *self) {
   Py_TYPE(self)->tp_free(self);
 }
 
-PyObject *tensor_shape(PyObject *self, PyObject *const *args, Py_ssize_t n) {
+PyObject *tensor_shape(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *names) {
   PyObject *shape = as_tensor(self)->shape;
   if (count_of(shape) < 0 && PyErr_Occurred()) return nullptr;
-  if (n == 0 || (n == 1 && args[0] == Py_None)) return PySequence_List(shape);
-  if (n != 1) {
+  const Py_ssize_t named = names ? PyTuple_GET_SIZE(names) : 0;   // (their values follow the positional ones)
+  const bool known = named == 0 || (named == 1 && PyUnicode_CompareWithASCIIString(PyTuple_GET_ITEM(names, 0), "axis") == 0);
+  n += named;
+  if (known && (n == 0 || (n == 1 && args[0] == Py_None))) return PySequence_List(shape);
+  if (!known || n != 1) {
     PyErr_SetString(PyExc_TypeError, "shape(axis=None)");
     return nullptr;
   }
@@ -383,7 +402,7 @@ PyMemberDef tensor_members[] = {{"_shape", T_OBJECT, offsetof(Tensor, shape), 0,
                                 {nullptr, 0, 0, 0, nullptr}};
 PyGetSetDef tensor_getset[] = {{"ptr", tensor_ptr, nullptr, "device address", nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMethodDef tensor_methods[] = {
-    {"shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(tensor_shape)), METH_FASTCALL, "extents, or one of them"},
+    {"shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(tensor_shape)), METH_FASTCALL | METH_KEYWORDS, "extents, or one of them"},
     {"Size", tensor_size, METH_NOARGS, "number of elements"},
     {"MemSize", tensor_memsize, METH_NOARGS, "bytes"},
     {"nDim", tensor_ndim, METH_NOARGS, "number of dimensions"},
@@ -399,6 +418,16 @@ PyTypeObject TensorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 PyObject *set_check(PyObject *, PyObject *f) {
   Py_INCREF(f);
   Py_XSETREF(g_check, f);
+  Py_RETURN_NONE;
+}
+
+PyObject *set_tensor(PyObject *, PyObject *c) {
+  if (!PyType_Check(c) || !PyType_IsSubtype(reinterpret_cast<PyTypeObject *>(c), &TensorType)) {
+    PyErr_SetString(PyExc_TypeError, "a class derived from TensorBase is expected");
+    return nullptr;
+  }
+  Py_INCREF(c);
+  Py_XSETREF(g_tensor, c);
   Py_RETURN_NONE;
 }
 
@@ -429,6 +458,7 @@ PyObject *fork_(PyObject *, PyObject *h) {
 PyMethodDef methods[] = {
     {"set_check", set_check, METH_O, "the function that turns a return code into an exception"},
     {"set_open", set_open, METH_O, "the function that opens the library and returns its handle"},
+    {"set_tensor", set_tensor, METH_O, "the class of the tensors that empty_like makes"},
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(empty)), METH_FASTCALL, "empty(cls, shape, device, dtype)"},
     {"empty_like", empty_like, METH_O, "a dense tensor of the same shape, device and type"},
     {"fork", fork_, METH_O, "sgh_device_fork: the auxiliary stream"},

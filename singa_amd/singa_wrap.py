@@ -236,7 +236,9 @@ class Tensor(_native.TensorBase):
         self._block = _block if _block is not None else _Block(device, self.MemSize())
 
     def __copy__(self):   # (the fields are not in __dict__)
-        t = Tensor(self._shape, self._dev, self._dtype, _block=self._block, _transposed=self._transposed)
+        t = type(self).__new__(type(self))
+        t._shape, t._dev, t._dtype = self._shape, self._dev, self._dtype
+        t._block, t._transposed = self._block, self._transposed
         t.__dict__.update(self.__dict__)
         return t
 
@@ -504,7 +506,8 @@ def Reshape(t, shape):
 
 # ------------------------------------------------------------------------------------ tensor math
 
-_like = _native.empty_like   # a dense tensor of t's shape, device and type
+_native.set_tensor(Tensor)
+_like = _native.empty_like   # a dense Tensor of t's shape, device and type
 _empty = _native.empty       # _empty(Tensor, shape tuple, device, dtype)
 
 

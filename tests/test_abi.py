@@ -367,3 +367,56 @@ for step in (lambda: globals().__setitem__("block", _native.Block(Device(), 64))
 assert stub.waits_in_vain() == 0, stub.waits_in_vain()
 """
     subprocess.run([sys.executable, "-c", program, stub], check=True, cwd=ROOT, timeout=60)
+
+
+def test_tensor_accessors_and_results_behave_like_a_python_class(tmp_path):
+    """What the Python class offered: shape(axis=...), results that are plain Tensors whatever class the operand has, copies of the
+    operand's class, whole numbers of numpy as sizes; a shape beyond the address space is refused, not wrapped around."""
+    import copy
+
+    import numpy as np
+
+    from singa_amd import _native, singa_wrap as singa
+
+    class Named(singa.Tensor):
+        def __init__(self, name, *args, **kw):
+            super(Named, self).__init__(*args, **kw)
+            self.name = name
+
+    dev = object()
+    t = Named("weights", (3, 5), dev, singa.kFloat32, _block=_native.Block(dev, 60, 4096, None))
+    assert t.shape(axis=1) == 5 and t.shape(1) == 5 and t.shape(axis=None) == [3, 5] and t.shape(-1) == 5
+    for wrong in (lambda: t.shape(0, axis=1), lambda: t.shape(dim=1), lambda: t.shape(0, 1)):
+        with pytest.raises(TypeError):
+            wrong()
+    c = copy.copy(t)
+    assert type(c) is Named and c.name == "weights" and c.ptr == 4096
+    assert _native.sgh_relu_fwd_f32(None, None, np.int64(4), None) < 0
+    big = singa.Tensor.__new__(singa.Tensor)
+    big._shape, big._dtype = (1 << 33, 1 << 33), singa.kFloat32
+    for count in (big.Size, big.MemSize):
+        with pytest.raises(OverflowError):
+            count()
+    source = tmp_path / "stub.cc"
+    source.write_text("""
+#include <stddef.h>
+extern "C" {
+int sgh_malloc(void *, void **p, size_t n) { *p = reinterpret_cast<void *>(n); return 0; }
+int sgh_free(void *, void *) { return 0; }
+}
+""")
+    stub = str(tmp_path / "libstub.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(source), "-o", stub], check=True)
+    program = """
+import ctypes, sys
+from singa_amd import _native, singa_wrap as singa
+stub = ctypes.CDLL(sys.argv[1])
+_native.set_open(lambda: stub._handle)
+class Device(object):
+    _handle = 1
+class Derived(singa.Tensor):
+    pass
+like = singa._like(Derived((3, 5), Device(), singa.kFloat16))
+assert type(like) is singa.Tensor and like.shape() == [3, 5] and like.ptr == 30, (type(like), like.ptr)
+"""
+    subprocess.run([sys.executable, "-c", program, stub], check=True, cwd=ROOT, timeout=60)
