@@ -716,7 +716,16 @@ def AddRow(v, m):
 
 # ------------------------------------------------------------------------------------ operations
 
-class CudnnConvHandle(object):
+class _HasGeometry(object):
+    """A handle with a geometry structure, `geom`, that calls get the address of: asked for each time, because a copied or
+    unpickled handle and one whose `geom` was replaced have a structure of their own."""
+
+    @property
+    def geom_ptr(self):
+        return C.addressof(self.geom)
+
+
+class CudnnConvHandle(_HasGeometry):
     """Geometry + workspace of a convolution on the GPU device.  Same constructor arguments and
     public fields as the reference's handle (src/model/operation/convolution.h:43-129; fields read
     from Python: src/api/model_operation.i:37-54)."""
@@ -740,7 +749,6 @@ class CudnnConvHandle(object):
                                               self.width, self.num_filters, self.kernel_h, self.kernel_w,
                                               self.stride_h, self.stride_w, self.pad_h, self.pad_w, groups),
               "sgh_conv_geom_init_grouped")
-        self.geom_ptr = C.addressof(self.geom)
         self.channels_per_filter = self.channels // groups   # (convolution.cc:461)
         self.conv_height, self.conv_width = self.geom.P, self.geom.Q
         self.x_shape = (self.batchsize, self.channels, self.height, self.width)
@@ -982,7 +990,7 @@ def GpuBatchNormReLUBackward(h, dy, x, scale, bias, mean, var):
     return [dx, ds, db]
 
 
-class CudnnPoolingHandle(object):
+class CudnnPoolingHandle(_HasGeometry):
     """``CudnnPoolingHandle(x, kernel, stride, padding, is_max)``
     (src/model/operation/pooling.h:40-91)."""
 
@@ -998,7 +1006,6 @@ class CudnnPoolingHandle(object):
         check(_L().sgh_pool_geom_init(C.byref(self.geom), self.batchsize, self.channels, self.height,
                                       self.width, self.kernel_h, self.kernel_w, self.stride_h, self.stride_w,
                                       self.pad_h, self.pad_w, int(self.is_max_pooling)), "sgh_pool_geom_init")
-        self.geom_ptr = C.addressof(self.geom)
         self.pooled_height, self.pooled_width = self.geom.P, self.geom.Q
         self.dy_shape = (self.batchsize, self.channels, self.pooled_height, self.pooled_width)
 

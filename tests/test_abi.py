@@ -420,3 +420,20 @@ like = singa._like(Derived((3, 5), Device(), singa.kFloat16))
 assert type(like) is singa.Tensor and like.shape() == [3, 5] and like.ptr == 30, (type(like), like.ptr)
 """
     subprocess.run([sys.executable, "-c", program, stub], check=True, cwd=ROOT, timeout=60)
+
+
+def test_copied_handles_pass_their_own_geometry():
+    """A pooling handle that was copied, pickled or given another geometry structure calls with the structure it holds."""
+    import copy
+    import pickle
+
+    from singa_amd import _native, singa_wrap as singa
+    x = singa.from_device_pointer(4096, (2, 3, 8, 8), object(), singa.kFloat32)
+    h = singa.CudnnPoolingHandle(x, (3, 3), (2, 2), (1, 1), True)
+    other = copy.deepcopy(h)
+    assert other.geom_ptr == C.addressof(other.geom) != h.geom_ptr
+    loaded = pickle.loads(pickle.dumps(h))
+    assert loaded.geom_ptr == C.addressof(loaded.geom) and loaded.geom.P == h.geom.P
+    h.geom = other.geom
+    assert h.geom_ptr == other.geom_ptr
+    assert _native.sgh_pool_fwd_f32(loaded.geom_ptr, None, None, None) < 0   # (null tensors are refused)
