@@ -56,12 +56,13 @@ __device__ __forceinline__ rsrc_t buffer_of(const typename S::elem *p, unsigned 
 }
 
 // Source rows of `planes` consecutive planes (first plane `plane0`, those from `planes_end` on are zero) into LDS as
-// [plane][VR][VC]; row 0 of the virtual image is virtual row `vrow0`.
+// [plane][VR][VC]; row 0 of the virtual image is virtual row `vrow0`.  Returns whether this thread met an infinity or a NaN.
 template <class S>
-__device__ __forceinline__ void stage_planes(float *lds, const GroupArgs &a, rsrc_t src, int plane0, int planes, int plane_step,
+__device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsrc_t src, int plane0, int planes, int plane_step,
                                              int planes_end, int vrow0) {
   const int total = planes * a.VR * a.VC;
   constexpr int U = 4;
+  bool odd = false;
   for (int i0 = threadIdx.x; i0 < total; i0 += GT * U) {
     float v[U];
 #pragma unroll
@@ -80,10 +81,18 @@ __device__ __forceinline__ void stage_planes(float *lds, const GroupArgs &a, rsr
       v[u] = ld_elem<S>(src, ((plane0 + pl * plane_step) * a.SH + y) * a.SW + x, ok);
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      odd = odd || !isfinite(v[u]);
       if (i0 + u * GT < total) lds[i0 + u * GT] = v[u];
+    }
   }
+  return odd;
 }
+
+// The zeros that pad the image, and in the data gradient those between its rows, are multiplied like everything else; that
+// is the same sum unless the other factor is an infinity or a NaN.  Forward, such a filter gives NaN at the borders, as a
+// zero-padded image does; the data gradient has no padding in its definition, and with such a filter in LDS (`odd`) the
+// positions that hold no gradient are left out one by one.
 
 // R: filter height and width; T: output stride
 template <class S, int R, int T>
@@ -91,7 +100,12 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
                                                    const typename S::elem *__restrict__ bias, typename S::elem *__restrict__ dst,
                                                    const GroupArgs a) {
   extern __shared__ float lds[];
+  __shared__ int odd;
   constexpr int RS = R * R;
+  if (a.flip) {
+    if (threadIdx.x == 0) odd = 0;
+    __syncthreads();
+  }
   const int u0 = int(blockIdx.x) * a.UB, p0 = int(blockIdx.y) * a.TP;
   const int ub = a.units - u0 < a.UB ? a.units - u0 : a.UB;
   float *image = lds, *filt = lds + a.UB * a.cs * a.VR * a.VC;
@@ -103,10 +117,13 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
     const int q2 = a.d_cs.div(q), cl = q - q2 * a.cs;
     const int ul = a.d_cd.div(q2), m = q2 - ul * a.cd;
     const int unit = u0 + ul, g = unit - a.d_G.div(unit) * a.G;
-    filt[i] = S::ld(W + (a.flip ? (long(g * a.cs + cl) * a.cd + m) * RS + (RS - 1 - tap)
-                                : (long(g * a.cd + m) * a.cs + cl) * RS + tap));
+    const float f = S::ld(W + (a.flip ? (long(g * a.cs + cl) * a.cd + m) * RS + (RS - 1 - tap)
+                                      : (long(g * a.cd + m) * a.cs + cl) * RS + tap));
+    filt[i] = f;
+    if (a.flip && !isfinite(f)) odd = 1;
   }
   __syncthreads();
+  const bool select = a.flip && odd != 0;
   const int strips = (a.TP + STRIP - 1) / STRIP;
   const int items = ub * a.cd * strips * a.DW;
   for (int it = threadIdx.x; it < items; it += GT) {
@@ -125,14 +142,32 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
       float w[RS];
 #pragma unroll
       for (int k = 0; k < RS; ++k) w[k] = wf[k];
+      if (T > 1 || !select) {   // (T > 1: forward passes only)
 #pragma unroll
-      for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
+        for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
 #pragma unroll
-        for (int s = 0; s < R; ++s) {
-          const float v = im[i * a.VC + s];
+          for (int s = 0; s < R; ++s) {
+            const float v = im[i * a.VC + s];
 #pragma unroll
-          for (int r = 0; r < R; ++r)
-            if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP) acc[(i - r) / T] = fmaf(w[r * R + s], v, acc[(i - r) / T]);
+            for (int r = 0; r < R; ++r)
+              if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP) acc[(i - r) / T] = fmaf(w[r * R + s], v, acc[(i - r) / T]);
+          }
+        }
+      } else {
+        const int y0 = p0 + st * STRIP - a.padh, x0 = q - a.padw;
+#pragma unroll
+        for (int i = 0; i < STRIP - 1 + R; ++i) {
+          const int yy = y0 + i, y = a.d_dil.div(yy < 0 ? 0 : yy);
+          const bool row = yy >= 0 && y < a.SH && y * a.dil == yy;
+#pragma unroll
+          for (int s = 0; s < R; ++s) {
+            const int xx = x0 + s, x = a.d_dil.div(xx < 0 ? 0 : xx);
+            const bool there = row && xx >= 0 && x < a.SW && x * a.dil == xx;
+            const float v = im[i * a.VC + s];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+              if (i >= r && i - r < STRIP) acc[i - r] = there ? fmaf(w[r * R + s], v, acc[i - r]) : acc[i - r];
+          }
         }
       }
       im += a.VR * a.VC, wf += RS;
@@ -148,6 +183,8 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
 
 // One (filter k, channel c of its group) pair per blockIdx.x, a chunk of the images per blockIdx.y.  `a` describes the
 // staging of x (source) against the pixels of dy (destination); a.UB images are staged together, one channel of each.
+// The rows of a strip that lie beyond the last row of dy count as zeros of dy; from the first infinity or NaN that the
+// workgroup meets in x on (`odd`), their products are left out instead.
 template <class S, int R, int T>
 __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__restrict__ x, const typename S::elem *__restrict__ dy,
                                                     float *__restrict__ part, typename S::elem *__restrict__ dW,
@@ -155,6 +192,8 @@ __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__re
   extern __shared__ float lds[];
   constexpr int RS = R * R;
   __shared__ float red[GT / SGH_WAVE][RS];
+  __shared__ int odd;
+  if (threadIdx.x == 0) odd = 0;
   const int pair = blockIdx.x, k = a.d_cs.div(pair), cl = pair - k * a.cs, g = a.d_cd.div(k);
   const int C = a.G * a.cs, K = a.G * a.cd;
   const int n_end = (int(blockIdx.y) + 1) * images < N ? (int(blockIdx.y) + 1) * images : N;
@@ -167,8 +206,9 @@ __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__re
     const int ub = n_end - n0 < a.UB ? n_end - n0 : a.UB;
     for (int p0 = 0; p0 < a.DH; p0 += a.TP) {
       __syncthreads();   // (the previous tile has been read)
-      stage_planes<S>(lds, a, xs, n0 * C + g * a.cs + cl, a.UB, C, ub, p0 * T);
+      if (stage_planes<S>(lds, a, xs, n0 * C + g * a.cs + cl, a.UB, C, ub, p0 * T)) odd = 1;
       __syncthreads();
+      const bool select = odd != 0;
       const int items = ub * strips * a.DW;
       for (int it = threadIdx.x; it < items; it += GT) {
         const int r1 = a.d_dw.div(it), q = it - r1 * a.DW;
@@ -179,14 +219,28 @@ __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__re
         for (int o = 0; o < STRIP; ++o)
           d[o] = ld_elem<S>(ys, (((n0 + ul) * K + k) * a.DH + p + o) * a.DW + q, p + o < pe);
         const float *im = lds + (ul * a.VR + st * STRIP * T) * a.VC + q * T;
+        if (!select) {
 #pragma unroll
-        for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
+          for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
 #pragma unroll
-          for (int s = 0; s < R; ++s) {
-            const float v = im[i * a.VC + s];
+            for (int s = 0; s < R; ++s) {
+              const float v = im[i * a.VC + s];
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-              if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP) acc[r * R + s] = fmaf(d[(i - r) / T], v, acc[r * R + s]);
+              for (int r = 0; r < R; ++r)
+                if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP) acc[r * R + s] = fmaf(d[(i - r) / T], v, acc[r * R + s]);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              const float v = im[i * a.VC + s];
+#pragma unroll
+              for (int r = 0; r < R; ++r)
+                if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP)
+                  acc[r * R + s] = p + (i - r) / T < pe ? fmaf(d[(i - r) / T], v, acc[r * R + s]) : acc[r * R + s];
+            }
           }
         }
       }

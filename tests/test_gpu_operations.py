@@ -926,3 +926,55 @@ def test_pooling_by_groups_of_images(singa, dev):
             assert np.array_equal(got_y[n:n + 1], y1.to_numpy()), ("forward", k, n)
             dx1 = singa.GpuPoolingBackward(h1, singa.from_numpy(dy[n:n + 1], dev), x1, y1)
             assert np.array_equal(got_dx[n:n + 1], dx1.to_numpy()), ("backward", k, n)
+
+
+def _windows(x, R, stride, pad, P, Q):
+    """(r, s, output rows, output columns, x rows, x columns) of every filter tap: the products that exist, nothing padded."""
+    H, W = x.shape[2:]
+    for r in range(R):
+        p = [i for i in range(P) if 0 <= i * stride + r - pad < H]
+        for s in range(R):
+            q = [j for j in range(Q) if 0 <= j * stride + s - pad < W]
+            if p and q:
+                yield r, s, slice(p[0], p[-1] + 1), slice(q[0], q[-1] + 1), np.array(p) * stride + r - pad, np.array(q) * stride + s - pad
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+@pytest.mark.parametrize("case", [
+    # N, C, H, W, R, stride, pad: depthwise; output rows that are no whole strips of four
+    (3, 4, 7, 7, 3, 1, 1),
+    (2, 3, 8, 6, 3, 2, 0),       # the last row and column of x belong to no window
+    (5, 2, 14, 9, 5, 2, 2),
+    (2, 2, 30, 150, 3, 1, 1),    # several row tiles per plane
+])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_narrow_groups_keep_infinities_where_they_belong(singa, dev, kind, case, bad):
+    """An infinity or NaN in x (in a filter) reaches the filter taps (the pixels) that it is multiplied with and no others."""
+    N, C, H, W, R, stride, pad = case
+    print("narrow groups", kind, case, bad, flush=True)
+    r = rng(sum(case))
+    dt, tol = (singa.kFloat32, 1e-5) if kind == "f32" else (singa.kBFloat16, 1e-2)
+    to = lambda a: singa.from_numpy(a.astype(np.float32), dev).AsType(dt)
+    back = lambda t: t.AsType(singa.kFloat32).to_numpy()
+    x, w = randn(r, N, C, H, W), randn(r, C, 1, R, R)
+    x[N - 1, 0, H - 1, :] = bad
+    x[0, C - 1, :, 0] = bad
+    w[0, 0, R - 1, 0] = w[C - 1, 0, 0, R - 1] = bad
+    xt, wt = to(x), to(w)
+    x, w = back(xt), back(wt)
+    h = singa.CudnnConvHandle(xt, (R, R), (stride, stride), (pad, pad), C, C, False, C)
+    P, Q = h.conv_height, h.conv_width
+    dyt = to(randn(r, N, C, P, Q))
+    dy = back(dyt)
+    dw_want, dx_want = np.zeros((C, 1, R, R)), np.zeros((N, C, H, W))
+    with np.errstate(invalid="ignore"):
+        for i, j, p, q, rows, cols in _windows(x, R, stride, pad, P, Q):
+            at = np.s_[:, :, rows[:, None], cols[None, :]]
+            d = dy[:, :, p, q].astype(np.float64)
+            dw_want[:, 0, i, j] = (d * x[at]).sum((0, 2, 3))
+            dx_want[at] += d * w[:, 0, i, j].astype(np.float64)[None, :, None, None]
+    for got, want in ((back(singa.GpuConvBackwardW(dyt, xt, wt, h)), dw_want), (back(singa.GpuConvBackwardx(dyt, wt, xt, h)), dx_want)):
+        fine = np.isfinite(want)
+        assert fine.any() and not fine.all()
+        assert np.array_equal(np.isfinite(got), fine)
+        assert nl2(got[fine], want[fine]) < tol
