@@ -503,6 +503,46 @@ struct ChipSlot {   // one per (channel, slice): {bits(a) : ticket low half}, {b
   unsigned long long wa, wb;
 };
 inline size_t chip_workspace_bytes(int C, int G) { return size_t(C) * size_t(G) * sizeof(ChipSlot); }
+// the forward kernel's slot carries what a and b leave of the sums' double values as well: {.. a, b, rest of a, rest of b}
+constexpr int kFwdWords = 4;
+inline size_t chip_fwd_workspace_bytes(int C, int G) { return size_t(C) * size_t(G) * kFwdWords * sizeof(unsigned long long); }
+
+// Sums of two values over the NT threads of a workgroup.  The rounding errors of the first levels of the tree average out
+// over its many sums, those of the last ones do not: from sums of eight lanes on it is in double.  With fp32 throughout and one
+// slice where there were two to eight, a channel's mean came out up to 2.7 times as far from the exact one.
+// `red`: 2 * NT / 64 doubles that nothing has used before; one barrier.
+template <int NT>
+__device__ __forceinline__ void chip_block_sums(float a, float b, double *red, double *A, double *B) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 32; o >= 8; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+  double da = a, db = b;
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1) da += __shfl_xor(da, o, 64), db += __shfl_xor(db, o, 64);
+  if (lane == 0) red[2 * wave] = da, red[2 * wave + 1] = db;
+  __syncthreads();
+  da = 0, db = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) da += red[2 * w], db += red[2 * w + 1];
+  *A = da, *B = db;
+}
+
+// Adds the slices' values that the lanes of the first kChipMaxG / 64 wavefronts hold (zero in lanes without a slice), for all
+// threads; the order is the same in every workgroup of the channel.  (All threads adding all values from LDS took 2 us for 128
+// slices.)  `total`: 2 * kChipMaxG / 64 doubles; one barrier, `a` and `b` are read by those wavefronts alone.
+__device__ __forceinline__ void chip_totals(double a, double b, double *total, double *A, double *B) {
+  const int t = threadIdx.x;
+  if (t < kChipMaxG) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+    if ((t & 63) == 0) total[t >> 5] = a, total[(t >> 5) + 1] = b;
+  }
+  __syncthreads();
+  a = total[0], b = total[1];
+#pragma unroll
+  for (int w = 1; w < kChipMaxG / 64; ++w) a += total[2 * w], b += total[2 * w + 1];
+  *A = a, *B = b;
+}
 
 struct ChipPlan {
   bool ok;
@@ -603,8 +643,8 @@ __global__ __launch_bounds__(NT, 4) void k_bn_bwd_onchip(const typename S::elem 
   typedef typename S::elem elem;
   constexpr int V = S::VEC, NV = chip_nv<S>();
   typedef typename RawVec<V * sizeof(elem)>::type raw;
-  __shared__ float red[16];
-  __shared__ float part_a[kChipMaxG], part_b[kChipMaxG];
+  __shared__ double red[2 * NT / 64];
+  __shared__ double total[2 * kChipMaxG / 64];
   __shared__ int gave_up;
   __shared__ unsigned long long ticket_s;
   // Channels of few slices: each XCD (workgroup w runs on XCD w % 8) takes a run of consecutive channels, see
@@ -747,9 +787,11 @@ __global__ __launch_bounds__(NT, 4) void k_bn_bwd_onchip(const typename S::elem 
   }
 #undef BN_CHIP_ACCUMULATE
   b += b1;
-  float db = sgh_block_sum(a, red), dg = sgh_block_sum(b, red);
+  double sum_d, sum_dx;
+  chip_block_sums<NT>(a, b, red, &sum_d, &sum_dx);
+  float db = float(sum_d), dg = float(sum_dx);
   if (G > 1) {
-    // (the block sums above contain barriers: ticket_s and gave_up are visible to every thread)
+    // (the block sums above contain a barrier: ticket_s and gave_up are visible to every thread)
     const unsigned long long ticket = ticket_s;
     const unsigned lo32 = unsigned(ticket), hi32 = unsigned(ticket >> 32);   // (both halves are nonzero)
     if (t == 0) {
@@ -758,6 +800,7 @@ __global__ __launch_bounds__(NT, 4) void k_bn_bwd_onchip(const typename S::elem 
       __hip_atomic_store(words + 2 * g + 1, (static_cast<unsigned long long>(__float_as_uint(dg)) << 32) | hi32,
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    double slice_d = 0, slice_dx = 0;
     if (t < G) {   // one lane per slice of the channel polls that slice's words (the second one until it is
                    // there, then the first one: one load per poll)
       unsigned long long wa = 0, wb = 0;
@@ -778,13 +821,11 @@ __global__ __launch_bounds__(NT, 4) void k_bn_bwd_onchip(const typename S::elem 
         }
         __builtin_amdgcn_s_sleep(4);
       }
-      part_a[t] = __uint_as_float(unsigned(wa >> 32));
-      part_b[t] = __uint_as_float(unsigned(wb >> 32));
+      slice_d = __uint_as_float(unsigned(wa >> 32));
+      slice_dx = __uint_as_float(unsigned(wb >> 32));
     }
-    __syncthreads();
-    // the same G numbers in the same order in every workgroup of the channel
-    db = 0.f, dg = 0.f;
-    for (int i = 0; i < G; ++i) db += part_a[i], dg += part_b[i];
+    chip_totals(slice_d, slice_dx, total, &sum_d, &sum_dx);
+    db = float(sum_d), dg = float(sum_dx);
     if (gave_up) {
       db = dg = __builtin_nanf("");
       if (t == 0) atomicAdd(&g_bn_gave_up, 1);
@@ -890,17 +931,17 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
   typedef typename S::elem elem;
   constexpr int V = S::VEC, NV = chip_fwd_nv<S>(ACT == 2), NT = 512;
   typedef typename RawVec<V * sizeof(elem)>::type raw;
-  __shared__ float red[16];
-  __shared__ float part_a[kChipMaxG], part_b[kChipMaxG];
+  __shared__ double red[2 * NT / 64];
+  __shared__ double total[2 * kChipMaxG / 64];
   __shared__ int gave_up;
   __shared__ unsigned long long ticket_s;
   const int unit = xcd_runs ? int(blockIdx.x & 7) * int(gridDim.x >> 3) + int(blockIdx.x >> 3) : int(blockIdx.x);
   const int c = unit / G, g = unit - c * G, t = threadIdx.x;
   if (c >= s.C) return;
-  unsigned long long *words = ws + size_t(c) * 2 * size_t(G);   // the channel's G slots
+  unsigned long long *words = ws + size_t(c) * kFwdWords * size_t(G);   // the channel's G slots
   if (G > 1 && t == 0) {
-    const unsigned long long wa = __hip_atomic_load(words + 2 * g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long wb = __hip_atomic_load(words + 2 * g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long wa = __hip_atomic_load(words + kFwdWords * g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long wb = __hip_atomic_load(words + kFwdWords * g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     ticket_s = (unsigned(wa) == unsigned(ticket1) && unsigned(wb) == unsigned(ticket1 >> 32)) ? ticket2 : ticket1;
     gave_up = 0;
   }
@@ -971,31 +1012,37 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
       w.step(dn, dr, PV);
     }
   }
-  a = sgh_block_sum(a, red);
-  b = sgh_block_sum(b, red);
-  double A = a, B = b;
+  double A, B;
+  chip_block_sums<NT>(a, b, red, &A, &B);
   if (G > 1) {
-    // (the block sums above contain barriers: ticket_s and gave_up are visible to every thread)
+    // (the block sums above contain a barrier: ticket_s and gave_up are visible to every thread)
     const unsigned long long ticket = ticket_s;
     const unsigned lo32 = unsigned(ticket), hi32 = unsigned(ticket >> 32);   // (both halves are nonzero)
     if (t == 0) {
-      __hip_atomic_store(words + 2 * g, (static_cast<unsigned long long>(__float_as_uint(a)) << 32) | lo32,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(words + 2 * g + 1, (static_cast<unsigned long long>(__float_as_uint(b)) << 32) | hi32,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const float ah = float(A), bh = float(B);
+      const float al = isfinite(ah) ? float(A - ah) : 0.f, bl = isfinite(bh) ? float(B - bh) : 0.f;
+      auto put = [&](int word, float v, unsigned tag) {
+        __hip_atomic_store(words + kFwdWords * g + word, (static_cast<unsigned long long>(__float_as_uint(v)) << 32) | tag,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      put(0, ah, lo32), put(1, bh, hi32), put(2, al, lo32), put(3, bl, hi32);
     }
-    if (t < G) {   // one lane per slice of the channel polls that slice's words
-      unsigned long long wa = 0, wb = 0;
+    double slice_a = 0, slice_b = 0;
+    if (t < G) {   // one lane per slice of the channel polls that slice's words: the last one until it is there, then all
+      const unsigned long long *slot = words + kFwdWords * t;
+      auto get = [&](int word) { return __hip_atomic_load(slot + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+      auto value = [](unsigned long long w) { return double(__uint_as_float(unsigned(w >> 32))); };
+      unsigned long long wa = 0, wb = 0, ra = 0, rb = 0;
       int spins = 0;
-      bool have_b = false;
+      bool have_last = false;
       for (;;) {
-        if (!have_b) {
-          wb = __hip_atomic_load(words + 2 * t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          have_b = unsigned(wb) == hi32;
+        if (!have_last) {
+          rb = get(3);
+          have_last = unsigned(rb) == hi32;
         }
-        if (have_b) {
-          wa = __hip_atomic_load(words + 2 * t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (unsigned(wa) == lo32) break;
+        if (have_last) {
+          wa = get(0), wb = get(1), ra = get(2);
+          if (unsigned(wa) == lo32 && unsigned(wb) == hi32 && unsigned(ra) == lo32) break;
         }
         if (++spins >= spin_limit) {
           gave_up = 1;
@@ -1003,12 +1050,10 @@ __global__ __launch_bounds__(512, 4) void k_bn_fwd_onchip(const typename S::elem
         }
         __builtin_amdgcn_s_sleep(4);
       }
-      part_a[t] = __uint_as_float(unsigned(wa >> 32));
-      part_b[t] = __uint_as_float(unsigned(wb >> 32));
+      slice_a = value(wa) + value(ra);
+      slice_b = value(wb) + value(rb);
     }
-    __syncthreads();
-    A = 0, B = 0;
-    for (int i = 0; i < G; ++i) A += part_a[i], B += part_b[i];   // the same numbers in the same order in every slice
+    chip_totals(slice_a, slice_b, total, &A, &B);
   }
   const double M = double(s.N) * s.HW;
   const double dm = A / M;
@@ -1254,7 +1299,7 @@ int bn_fwd_train_act(const typename S::elem *x, const typename S::elem *z, const
   // may write some of a channel's words between two replays
   const size_t slots_at = shared_workspace_bytes(N, C, HW);
   if (fp.ok && !sgh_env().bn_onchip_off && !sgh_env().bn_fwd_onchip_off && sgh_aligned16(workspace) &&
-      ws_bytes >= slots_at + chip_workspace_bytes(C, fp.G))
+      ws_bytes >= slots_at + chip_fwd_workspace_bytes(C, fp.G))
     return launch_fwd_onchip<S, ACT>(x, z, gamma, beta, running_mean, running_var, factor, eps, y, save_mean, save_invstd,
                                      static_cast<char *>(workspace) + slots_at, s, fp, sgh_stream_of(stream));
   float *scratch = static_cast<float *>(workspace);
@@ -1425,7 +1470,7 @@ size_t sgh_bn_workspace_bytes(int N, int C, int HW) {
                          chip_fwd_plan<StF16x4>(N, C, HW, false), chip_fwd_plan<StF32>(N, C, HW, true),
                          chip_fwd_plan<StF16>(N, C, HW, true), chip_fwd_plan<StF16x4>(N, C, HW, true)};
   for (const ChipPlan &p : f)
-    if (p.ok && chip_workspace_bytes(C, p.G) > fwd) fwd = chip_workspace_bytes(C, p.G);
+    if (p.ok && chip_fwd_workspace_bytes(C, p.G) > fwd) fwd = chip_fwd_workspace_bytes(C, p.G);
   return shared_workspace_bytes(N, C, HW) + fwd;
 }
 

@@ -978,3 +978,25 @@ def test_narrow_groups_keep_infinities_where_they_belong(singa, dev, kind, case,
         assert fine.any() and not fine.all()
         assert np.array_equal(np.isfinite(got), fine)
         assert nl2(got[fine], want[fine]) < tol
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+@pytest.mark.parametrize("shape", [(124, 485, 9, 11), (17, 504, 23, 30), (20, 586, 19, 22), (5, 390, 54, 47)])
+def test_bn_statistics_to_the_last_bits(singa, dev, kind, shape):
+    """Saved mean and inverse standard deviation of channels that one or two workgroups hold, root mean square over the channels
+    against float64.  Their own rounding: 2^-24 / sqrt(3) of the value (the mean lies below 1/2: 2^-26 / sqrt(3)).  The sums: 64
+    values per workgroup rounded to 2^-24 at random and the levels below them, together 2^-24 sqrt(2 / 64) of the distance
+    between mean and pivot (one standard deviation) or of the variance: less than 2^-26."""
+    print("bn statistics", kind, shape, flush=True)
+    r = rng(sum(shape))
+    N, C, H, W = shape
+    xt = singa.from_numpy((randn(r, *shape) * 1.5 + 0.3).astype(np.float32), dev)
+    xt = xt if kind == "f32" else xt.AsType(singa.kBFloat16)
+    x = xt.AsType(singa.kFloat32).to_numpy().astype(np.float64)
+    h = singa.CudnnBatchNormHandle(0.9, xt)
+    ones, zeros = np.ones(C, np.float32), np.zeros(C, np.float32)
+    _, mean, inv = singa.GpuBatchNormForwardTraining(h, xt, *(singa.from_numpy(a, dev) for a in (ones, zeros, zeros, ones)))
+    m, v = x.mean((0, 2, 3)), x.var((0, 2, 3))
+    rms = lambda a: float(np.sqrt(np.mean(a * a)))
+    assert rms((mean.to_numpy() - m) / np.sqrt(v)) < 2.0 ** -26 / np.sqrt(3) / 1.5 + 2.0 ** -26
+    assert rms(inv.to_numpy() * np.sqrt(v + 1e-5) - 1) < 2.0 ** -24 / np.sqrt(3) + 2.0 ** -26
