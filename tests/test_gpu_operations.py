@@ -1000,3 +1000,23 @@ def test_bn_statistics_to_the_last_bits(singa, dev, kind, shape):
     rms = lambda a: float(np.sqrt(np.mean(a * a)))
     assert rms((mean.to_numpy() - m) / np.sqrt(v)) < 2.0 ** -26 / np.sqrt(3) / 1.5 + 2.0 ** -26
     assert rms(inv.to_numpy() * np.sqrt(v + 1e-5) - 1) < 2.0 ** -24 / np.sqrt(3) + 2.0 ** -26
+
+
+@pytest.mark.parametrize("case", [(5, 20, 42, 46, 18, 3, 1), (3, 24, 20, 31, 35, 5, 1), (4, 28, 40, 32, 12, 3, 2)])
+def test_few_channel_data_gradient_rounding(singa, dev, case):
+    """The data gradient of 16 to 31 channels adds K products and then at most R^2 taps: 2^-24 / sqrt(3) per rounding, partial
+    sums growing evenly, so sqrt((K + R^2) / 2) of it against float64 (one chain of K R^2 products would show sqrt(K R^2 / 2))."""
+    N, C, H, W, K, R, stride = case
+    print("few channels", case, flush=True)
+    r = rng(sum(case))
+    x, w = randn(r, N, C, H, W), (randn(r, K, C, R, R) * np.sqrt(2.0 / (C * R * R))).astype(np.float32)
+    xd, wd = singa.from_numpy(x, dev), singa.from_numpy(w, dev)
+    p = R // 2
+    h = singa.CudnnConvHandle(xd, (R, R), (stride, stride), (p, p), C, K, False)
+    P, Q = h.conv_height, h.conv_width
+    dy = randn(r, N, K, P, Q)
+    want = np.zeros((N, C, H, W))
+    for i, j, prow, qcol, rows, cols in _windows(x, R, stride, p, P, Q):
+        want[:, :, rows[:, None], cols[None, :]] += np.einsum("nkpq,kc->ncpq", dy[:, :, prow, qcol].astype(np.float64), w[:, :, i, j].astype(np.float64))
+    got = singa.GpuConvBackwardx(singa.from_numpy(dy, dev), wd, xd, h).to_numpy()
+    assert nl2(got, want) < 2.0 ** -24 / np.sqrt(3) * np.sqrt((K + R * R) / 2)
