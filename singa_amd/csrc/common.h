@@ -153,6 +153,7 @@ int sgh_wgrad_fewc_run(const sgh_conv_geom *g, const float *dy, const float *x, 
 // 3x3 stride-1 pad-1 data gradient with a shared LDS gradient tile (dgrad3x3.hip).
 // `wt` = weights re-laid as [tap][KP][C], KP = K rounded up to 16.
 bool sgh_dgrad3x3_supported(const sgh_conv_geom *g);
+bool sgh_dgrad3x3_forward_pays(const sgh_conv_geom *g);
 size_t sgh_dgrad3x3_partial_bytes(const sgh_conv_geom *g);  // scratch for split-reduction partial images
 // `tag` names the profiling record; `bias` (may be NULL) is added per output channel -- the forward
 // convolution runs through this kernel as the data gradient of the channel-swapped problem.

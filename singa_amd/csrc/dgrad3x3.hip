@@ -410,6 +410,11 @@ inline D3Plan plan(const sgh_conv_geom *g) {
   p.ragk = g->K % KC != 0;
   // four classes x 16 accumulators per 32-row tile: the 64-row tile keeps two workgroups per CU
   p.bm = p.s2 ? 64 : g->C <= 32 ? 32 : (g->C % 128 == 0 || g->C > 192) && p.r == 3 ? 128 : 64;
+  const int nchunks = (g->K + KC - 1) / KC;
+  // a chunk and a half of reduction or less: the 128-row tile's weights and stores outweigh its products (228 rows over 14
+  // channels, 85 planes of 5 x 5, forward: generic
+  // kernel 13.8 us, 20.0 with 128 rows, 12.7 with 64)
+  if (p.bm == 128 && p.ragk && nchunks <= 2) p.bm = 64;
   if (!p.s2 && sgh_env().dgrad3x3_bm && p.r == 3) p.bm = sgh_env().dgrad3x3_bm;
   p.bn = p.bm == 32 ? Tile<32>::BN : Tile<64>::BN;
   // slab columns: stride 1 has halo columns on both sides, stride 2 one zero column on the right
@@ -434,12 +439,19 @@ inline D3Plan plan(const sgh_conv_geom *g) {
   // partial tiles to write and sum), so that no CU is left with a whole extra tile while others idle.  Tiles shared between workgroups are finished by
   // k_dgrad3x3_fixup in a fixed order: results stay run-to-run identical.
   const int cus = sgh_num_cus();
-  const int nchunks = (g->K + KC - 1) / KC;
   p.ctiles = (g->C + p.bm - 1) / p.bm;
   const long tiles = long(p.ctiles) * ((long(g->N) * g->P * g->Q + p.bn - 1) / p.bn);
   if (tiles >= (long(1) << 30)) return p;
   p.tiles = int(tiles);
-  p.dp_tiles = int(tiles / cus * cus);
+  // (a reduction of one chunk cannot be cut: no shared tiles, no fix-up launch.  16 channels, 32 to 127 tiles: 4 us of 15.
+  // With a slab of 1024 floats a workgroup fills its CU, and up to three chunks are not worth cutting once two fifths of the
+  // CUs have a tile: 3x3, 102 to 255 tiles of 64 rows against the generic kernel 0.90 to 1.24 times cut, 1.04 to 1.71 whole)
+  const bool whole = nchunks == 1 || (p.r == 3 && p.chs == 1024 && nchunks <= 3 && 5 * tiles > 2 * cus);
+  p.dp_tiles = whole ? p.tiles : int(tiles / cus * cus);
+  // Strided layers other than those of whole chunks, 64 channels and short rows: four classes of partial tiles to write and sum
+  // cost more than the class-by-class kernel loses, unless the tiles fill the chip (from one per CU on 1.2 to 2 times faster)
+  // or the reduction is long (97 channels and more: 1.1 to 3 times; 17 to 64 channels on 16 to 127 tiles: 0.7 to 0.95 times)
+  if (p.s2 && (p.ragk || g->C < 64 || g->Q > 31) && tiles < cus && nchunks <= 6) return p;
   p.sk_units = long(p.tiles - p.dp_tiles) * nchunks;
   p.sk_wgs = int(p.sk_units < cus ? p.sk_units : cus);
   p.ok = true;
@@ -463,6 +475,15 @@ int launch(const D3Args &a, const D3Plan &p, dim3 grid, hipStream_t s) {
 }  // namespace
 
 bool sgh_dgrad3x3_supported(const sgh_conv_geom *g) { return plan(g).ok; }
+
+// As a forward pass: also the faster one?  On wide rows (a slab of 1024 floats: one workgroup per CU) with up to three chunks of
+// reduction there is too little to multiply per staged row once the launch is long, and the generic kernel's 64- or 128-row
+// tiles fill as well as these.  3x3, from three tiles per CU on, 36 to 128 filters over 8 to 46 channels: 0.84 to 1.04 times;
+// with fewer tiles 0.97 to 1.31, with 132 to 164 filters (which leave the generic kernel's second tile nearly empty) 1.2 to 1.3.
+bool sgh_dgrad3x3_forward_pays(const sgh_conv_geom *g) {
+  const D3Plan p = plan(g);
+  return p.ok && !(p.r == 3 && p.bm == 64 && p.chs == 1024 && g->K <= 3 * KC && g->C <= 128 && p.tiles > 3 * sgh_num_cus());
+}
 
 // Extra workspace (bytes, after the re-laid weights) for split-reduction partial images.
 size_t sgh_dgrad3x3_partial_bytes(const sgh_conv_geom *g) {

@@ -855,7 +855,7 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
   *gt = *g;
   gt->C = g->K;
   gt->K = g->C;
-  return sgh_dgrad3x3_supported(gt);
+  return sgh_dgrad3x3_forward_pays(gt);
 }
 
 }  // namespace

@@ -437,3 +437,21 @@ def test_copied_handles_pass_their_own_geometry():
     h.geom = other.geom
     assert h.geom_ptr == other.geom_ptr
     assert _native.sgh_pool_fwd_f32(loaded.geom_ptr, None, None, None) < 0   # (null tensors are refused)
+
+
+def test_shared_tile_data_gradient_is_chosen_by_size():
+    """Which fp32 layers the shared-tile data gradient takes (only it can add into dx): not those of few channels, not strided ones
+    outside its first range with few tiles and a short reduction."""
+    L = _lib.lib()
+
+    def takes(n, c, h, w, k, r, stride):
+        g = _lib.ConvGeom()
+        assert L.sgh_conv_geom_init(C.byref(g), n, c, h, w, k, r, r, stride, stride, r // 2, r // 2) == 0
+        return bool(L.sgh_conv_dgrad_acc_supported(C.byref(g)))
+
+    assert not takes(64, 24, 32, 32, 64, 3, 1) and not takes(64, 24, 32, 32, 64, 5, 1) and not takes(64, 28, 32, 32, 128, 3, 2)
+    assert takes(64, 32, 16, 16, 64, 5, 1) and takes(2, 36, 16, 16, 72, 3, 1)
+    assert takes(2, 64, 14, 14, 64, 3, 2)           # whole chunks, 64 channels, short rows
+    assert not takes(2, 64, 14, 14, 72, 3, 2) and not takes(2, 48, 14, 14, 64, 3, 2) and not takes(2, 64, 80, 80, 64, 3, 2)
+    assert takes(2, 64, 14, 14, 104, 3, 2)          # a longer reduction
+    assert takes(32, 48, 64, 64, 24, 3, 2)          # a tile for every CU

@@ -802,14 +802,21 @@ def test_conv_bias_gradient_vs_float64(singa, dev, kind, shape):
     (3, 128, 5, 5, 136, 3, 1),       # tiles over seven images; 136 = eight chunks and a half
     (7, 64, 2, 2, 64, 3, 1),         # more image boundaries than pixel rows
     (2, 32, 17, 19, 24, 3, 1),       # 32-row tiles, odd planes, 24 = a chunk and a half
-    (3, 20, 12, 9, 16, 3, 1),        # 20 of 32 rows
+    (3, 20, 12, 9, 16, 3, 1),        # 16 of 32 rows (forward; the data gradient of 16 to 31 channels takes the column kernel)
+    (3, 36, 12, 9, 20, 3, 1),        # 20 of 32 rows
     (2, 36, 16, 16, 72, 3, 1),       # 36 of 64 rows
     (5, 32, 16, 16, 64, 5, 1),       # 5 x 5
     (2, 16, 7, 9, 40, 5, 1),         # 5 x 5 on small odd planes, both sides ragged
     (1, 64, 33, 47, 32, 5, 1),       # 5 x 5, 1024 floats
-    (2, 64, 80, 80, 64, 3, 2),       # stride 2: 512 floats
-    (3, 64, 10, 10, 72, 3, 2),       # stride 2, ragged reduction
-    (2, 20, 14, 6, 8, 3, 2),         # stride 2, 20 of 64 rows, half a chunk
+    (2, 64, 80, 80, 64, 3, 2),       # stride 2 on wide rows: few tiles and a short reduction stay with the classes
+    (3, 64, 10, 10, 72, 3, 2),       # ... a ragged reduction likewise
+    (2, 20, 14, 6, 8, 3, 2),         # ... and few channels with the columns
+    (2, 64, 80, 80, 112, 3, 2),      # stride 2: 512 floats
+    (3, 64, 10, 10, 104, 3, 2),      # stride 2, ragged reduction
+    (2, 36, 14, 6, 97, 3, 2),        # stride 2, 36 of 64 rows, a chunk of one
+    (32, 32, 64, 64, 8, 3, 2),       # stride 2, a tile for every CU, half a chunk
+    (2, 128, 9, 7, 24, 3, 1),        # 128 rows over a chunk and a half: 64-row tiles
+    (5, 64, 60, 72, 40, 3, 1),       # wide rows, three chunks: whole tiles
 ])
 def test_shared_tile_convolution_edges(singa, dev, case):
     """The shared-tile data gradient / forward kernel at the edges of what it covers: slab sizes, row tiles, ragged reductions,
