@@ -1135,13 +1135,19 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
   // may end one row and start the next, no more).
   if (fs == 1 && g->R == 3 && g->S == 3 && st == 1 && g->pad_h == 1 && g->pad_w == 1 && !sgh_env().slab16_off &&
       g->W >= 3 && g->H * g->W >= (g->W >= 7 ? 8 : 4)) {
-    static const int tiles[4][3] = {{2, 128, 256}, {3, 128, 128}, {1, 64, 256}, {4, 64, 128}};
+    // tiles of channels x positions, and what one costs in fifths of the products of the smallest
+    static const int tiles[4][4] = {{2, 128, 256, 21}, {3, 128, 128, 11}, {1, 64, 256, 10}, {4, 64, 128, 6}};
     const long HpWp = long(g->H + 1) * (g->W + 1), G = long(g->N) * HpWp;
     const int ev = g->W >= 7 ? 8 : 4, QO = (g->H * g->W + ev - 1) / ev;
     const int KP = (g->K + KC - 1) / KC * KC;
-    // The largest tile that gives three quarters of the CUs a workgroup, else the smallest one.  us, forward, against the
-    // tap-by-tap kernel (odd planes: on a pixel-major copy): 128 x 512 x 7 x 7 73.3 -> 51.3, 37 x 72 x 31 x 45 -> 136 60.7 ->
-    // 42.9; against 128 x 128 tiles of groups of four: 21 x 256 x 12 x 12 24.5 -> 21.0, 21 x 128 x 24 x 24 16.5 -> 13.7.
+    // The tile with the least work for a CU: the tiles that fall to it, one after the other or two at a time where their LDS
+    // fits twice, and twice the smallest tile's products (ten fifths) per such turn for staging and stores.  Over 1000 layers
+    // of 8 to 640 channels the choice is 1.317 times as fast as the tap-by-tap kernel and the tiles before this one, two
+    // layers slower than 0.95; the largest tile that gives three quarters of the CUs a workgroup made 1.29, 13 slower, down to
+    // 0.63 where the smallest tile just missed a single turn: bfloat16 12 x 208 x 56 x 63 -> 62 25.2 us with 171 tiles of
+    // 64 x 256, 36.2 with 342 of 64 x 128.  (Against the tap-by-tap kernel alone, forward: 128 x 512 x 7 x 7 73.3 -> 51.3 us,
+    // 37 x 72 x 31 x 45 -> 136 60.7 -> 42.9.)
+    long least = 0;
     for (int i = g->C <= 64 ? 2 : 0; i < 4; ++i) {   // (129 to 192 channels on three tiles of 64 instead: 42.9 -> 44.6)
       const int bmc = tiles[i][1], mt = tiles[i][2], mt_c = (g->C + bmc - 1) / bmc;
       const int sp = mt + 2 * (g->W + 1) + 2;
@@ -1149,11 +1155,16 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
       const long images = (sp - 1) / HpWp + 2;   // images a slab can touch; each may add a group at either end
       const long groups = images * QO < sp / ev + 2 * images ? images * QO : sp / ev + 2 * images;
       if (G + 1024 >= (long(1) << 31) || groups > (ev == 8 ? 64 : 128) || lds > size_t(160) * 1024) continue;
-      if (i != 3 && (G + mt - 1) / mt * mt_c < sgh_num_cus() * 3 / 4) continue;
+      const long load = ((G + mt - 1) / mt * mt_c + sgh_num_cus() - 1) / sgh_num_cus();
+      const long turns = lds <= size_t(80) * 1024 ? (load + 1) / 2 : load, cost = load * tiles[i][3] + 10 * turns;
+      if (p.slab != 0 && cost >= least) continue;
+      least = cost;
       p.slab = tiles[i][0];
       p.slab_sp = sp, p.slab_ev = ev;
       p.bm = bmc, p.mtiles = mt_c, p.CP = mt_c * bmc, p.KP = KP;
       p.tiles = int((G + mt - 1) / mt);
+    }
+    if (p.slab != 0) {
       p.pixk = false;
       p.wt_bytes = align256(size_t(9) * p.CP * p.KP * sizeof(uint16_t));
       p.dyT_bytes = 0;

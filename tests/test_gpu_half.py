@@ -937,9 +937,16 @@ def test_conv_1x1_16bit(singa, dev, kind, case):
     (9, 256, 6, 6, 64),     # rows of 6: the widest that take groups of four
     (11, 136, 7, 7, 72),    # rows of 7: groups of eight
     (3, 64, 2, 7, 40),      # two rows: groups that wrap in every place
-    (40, 128, 9, 31, 24),   # odd planes, 128 x 128 tiles
-    (7, 40, 31, 45, 136),   # ... one tile of channels, mostly empty
+    (40, 128, 9, 31, 24),   # odd planes
+    (7, 40, 31, 45, 136),   # ... a last tile of channels that is mostly empty
     (1, 16, 5, 109, 16),    # rows longer than a tile's half
+    # the tiles of launches that fill the chip (forward; the smaller ones take 64 x 128): 64 channels x 256 positions,
+    (90, 8, 13, 14, 72),    # one chunk of reduction,
+    (90, 72, 13, 14, 72),   # two;
+    (60, 8, 5, 109, 72),    # 128 x 256, one
+    (40, 72, 28, 30, 72),   # and two;
+    (48, 8, 14, 14, 384),   # 128 x 128, one
+    (48, 72, 14, 14, 384),  # and two
 ])
 def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
     """The slab kernel (forward and data gradient) against the oracle: one rounding of a result is at most 2^-11 (binary16) or
