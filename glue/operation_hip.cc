@@ -9,6 +9,8 @@
 // to the Python layer and outlive the graph.
 #include "./operation_hip.h"
 
+#include <algorithm>
+
 #ifdef USE_HIP
 
 #include "singa/core/hip_gpu.h"
@@ -60,12 +62,14 @@ CudnnConvHandle::CudnnConvHandle(const Tensor &input, const std::vector<size_t> 
   CHECK_EQ(static_cast<size_t>(geom.P), conv_height);
   CHECK_EQ(static_cast<size_t>(geom.Q), conv_width);
   channels_per_filter = channels / groups;
-  size_t need = 0;
+  size_t need = 0, least = 0;
   for (int which : {SGH_CONV_FWD, SGH_CONV_DGRAD, SGH_CONV_WGRAD}) {
     const size_t b = dtype == kFloat32 ? sgh_conv_workspace_bytes(&geom, which) : sgh_conv_workspace_bytes_h(&geom, which);
-    if (b > need) need = b;
+    need = std::max(need, b);
+    least = std::max(least, sgh_conv_workspace_least_bytes(&geom, which, dtype == kFloat32 ? 0 : 1));
   }
-  CHECK_LE(need, workspace_byte_limit) << "convolution workspace exceeds the handle's limit";
+  CHECK_LE(least, workspace_byte_limit) << "convolution workspace exceeds the handle's limit";
+  need = std::min(need, workspace_byte_limit);
   workspace = scratch_tensor(need, input.device());
   workspace_count = workspace.Size();
 }

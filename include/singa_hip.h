@@ -434,9 +434,9 @@ SGH_API int sgh_conv_geom_init(sgh_conv_geom *g, int N, int C, int H, int W, int
  * src/model/operation/convolution.cc:446-461 and :486-495: cudnnSetConvolutionGroupCount, filter descriptor
  * [K, C / groups, R, S]; python/singa/layer.py:668-718 and the depthwise layer of SeparableConv2d, :780-795).
  * C and K must be multiples of `groups`.  Group i convolves input channels [i C/groups, (i+1) C/groups) with
- * filters [i K/groups, (i+1) K/groups).  Every convolution entry point below takes such a geometry: each group
- * runs as a dense convolution on slices gathered in the workspace (sgh_conv_workspace_bytes[_h] account for
- * them); sgh_conv_dgrad_acc_f32 returns SGH_EUNSUPPORTED and sgh_conv_dgrad_prepare_multi skips it. */
+ * filters [i K/groups, (i+1) K/groups).  Every convolution entry point below takes such a geometry: groups of
+ * at most eight channels on either side run on kernels of their own, others each as a dense convolution on slices
+ * gathered in the workspace (sgh_conv_workspace_bytes[_h] account for them); sgh_conv_dgrad_acc_f32 returns SGH_EUNSUPPORTED and sgh_conv_dgrad_prepare_multi skips it. */
 SGH_API int sgh_conv_geom_init_grouped(sgh_conv_geom *g, int N, int C, int H, int W, int K, int R, int S,
                                        int stride_h, int stride_w, int pad_h, int pad_w, int groups);
 
@@ -446,6 +446,10 @@ SGH_API int sgh_conv_geom_init_grouped(sgh_conv_geom *g, int N, int C, int H, in
 /* Scratch bytes the given pass needs for this geometry (CudnnConvHandle::workspace_count,
  * src/model/operation/convolution.cc:560-571). */
 SGH_API size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which);
+/* The least that the pass accepts (dtype 0: fp32 tensors, 1: 16-bit ones), for a handle whose
+ * workspace_byte_limit is below sgh_conv_workspace_bytes[_h]: fp32 forward passes and data gradients
+ * then run without room for partial sums, slower where a launch does not fill the chip. */
+SGH_API size_t sgh_conv_workspace_least_bytes(const sgh_conv_geom *g, int which, int dtype);
 
 /* GpuConvBackwardx (src/model/operation/convolution.cc:634-656; native algorithm
  * src/model/layer/convolution.cc:178-182 + Col2im :224-248):

@@ -156,6 +156,7 @@ SIGNATURES = {
     "sgh_conv_geom_init": (C.c_int, [C.POINTER(ConvGeom)] + [C.c_int] * 11),
     "sgh_conv_geom_init_grouped": (C.c_int, [C.POINTER(ConvGeom)] + [C.c_int] * 12),
     "sgh_conv_workspace_bytes": (sz, [C.POINTER(ConvGeom), C.c_int]),
+    "sgh_conv_workspace_least_bytes": (sz, [C.POINTER(ConvGeom), C.c_int, C.c_int]),
     "sgh_conv_dgrad_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),
     "sgh_conv_dgrad_acc_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),
     "sgh_conv_wgrad_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),

@@ -155,6 +155,7 @@ int sgh_wgrad_fewc_run(const sgh_conv_geom *g, const float *dy, const float *x, 
 bool sgh_dgrad3x3_supported(const sgh_conv_geom *g);
 bool sgh_dgrad3x3_forward_pays(const sgh_conv_geom *g);
 size_t sgh_dgrad3x3_partial_bytes(const sgh_conv_geom *g);  // scratch for split-reduction partial images
+// `partials` may be null: every tile is then one workgroup's, at the price of an uneven last round.
 // `tag` names the profiling record; `bias` (may be NULL) is added per output channel -- the forward
 // convolution runs through this kernel as the data gradient of the channel-swapped problem.
 // `accumulate`: dx += result (the sum in the fixed order result-then-add of the separate "+=").

@@ -496,9 +496,9 @@ size_t sgh_dgrad3x3_partial_bytes(const sgh_conv_geom *g) {
 // `partials` is sgh_dgrad3x3_partial_bytes(g) bytes of scratch (may be NULL when that is 0).
 int sgh_dgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *wt, int KP, float *dx, float *partials,
                      hipStream_t s, const char *tag, const float *bias, bool accumulate) {
-  const D3Plan p = plan(g);
+  D3Plan p = plan(g);
   if (!p.ok) return SGH_EUNSUPPORTED;
-  if (p.sk_wgs > 0 && !partials) return SGH_EWORKSPACE;
+  if (!partials) p.dp_tiles = p.tiles, p.sk_units = 0, p.sk_wgs = 0;   // no room for shared tiles
   D3Args a;
   a.dy = dy;
   a.wt = wt;

@@ -889,10 +889,11 @@ GroupPlan group_plan(const sgh_conv_geom *g, size_t elem) {
 // `sub(sg, which, a, b, bias, out, workspace, ws_bytes)` runs one dense pass; T is the element type.
 template <typename T, typename Sub>
 int conv_grouped(const sgh_conv_geom *g, int which, const T *a, const T *b, const T *bias, T *out, void *workspace,
-                 size_t ws_bytes, size_t sub_ws, hipStream_t s, Sub sub) {
+                 size_t ws_bytes, size_t sub_least, hipStream_t s, Sub sub) {
   if (!conv_ok(g) || !a || !b || !out) return SGH_EINVAL;
   GroupPlan p = group_plan(g, sizeof(T));
-  if (!workspace || ws_bytes < p.x_bytes + p.y_bytes + sub_ws) return SGH_EWORKSPACE;
+  if (!workspace || ws_bytes < p.x_bytes + p.y_bytes + sub_least) return SGH_EWORKSPACE;
+  const size_t sub_ws = ws_bytes - p.x_bytes - p.y_bytes;
   char *w = static_cast<char *>(workspace);
   T *xg = reinterpret_cast<T *>(w), *yg = reinterpret_cast<T *>(w + p.x_bytes);
   void *inner = w + p.x_bytes + p.y_bytes;
@@ -979,8 +980,8 @@ int conv_grouped_f32(const sgh_conv_geom *g, int which, const float *a, const fl
   const int rc = sgh_group_conv_run(g, which, 0, a, b, bias, out, workspace, ws_bytes, sgh_stream_of(stream));
   if (rc != SGH_EUNSUPPORTED) return rc;
   GroupPlan p = group_plan(g, sizeof(float));
-  const size_t sub_ws = sgh_conv_workspace_bytes(&p.sg, which);
-  return conv_grouped<float>(g, which, a, b, bias, out, workspace, ws_bytes, sub_ws, sgh_stream_of(stream),
+  const size_t sub_least = sgh_conv_workspace_least_bytes(&p.sg, which, 0);
+  return conv_grouped<float>(g, which, a, b, bias, out, workspace, ws_bytes, sub_least, sgh_stream_of(stream),
                              [&](sgh_conv_geom *sg, int wh, const float *a_, const float *b_, const float *bias_,
                                  float *out_, void *ws, size_t wsb) {
                                return conv_dense_f32(sg, wh, a_, b_, bias_, out_, ws, wsb, stream);
@@ -1026,12 +1027,25 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   }
 }
 
+// The partial sums of the shared-tile kernel are the part of a workspace that a pass can do without
+static size_t least_bytes_f32(const sgh_conv_geom *g, int which) {
+  const size_t full = sgh_conv_workspace_bytes(g, which);
+  if (full == 0) return 0;
+  sgh_conv_geom gt;
+  if (which == SGH_CONV_FWD && fwd_as_dgrad(g, &gt)) {
+    const size_t wt = size_t(g->R) * g->S * round_up(g->C, BK) * g->K * sizeof(float), fewc = sgh_fwd_fewc_workspace_bytes(g);
+    return wt > fewc ? wt : fewc;
+  }
+  if (which == SGH_CONV_DGRAD && dgrad_path(g) == kDgradTile3x3) return full - sgh_dgrad3x3_partial_bytes(g);
+  return full;
+}
+
 // `prelaid`: the workspace already holds this layer's re-laid weights (sgh_conv_dgrad_prepare_multi)
 static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, float *dx, void *workspace,
                       size_t ws_bytes, void *stream, bool accumulate, bool prelaid) {
   if (!conv_ok(g) || !dy || !W || !dx) return SGH_EINVAL;
-  const size_t need = sgh_conv_workspace_bytes(g, SGH_CONV_DGRAD);
-  if (need && (!workspace || ws_bytes < need)) return SGH_EWORKSPACE;
+  const size_t full = sgh_conv_workspace_bytes(g, SGH_CONV_DGRAD), least = least_bytes_f32(g, SGH_CONV_DGRAD);
+  if (least && (!workspace || ws_bytes < least)) return SGH_EWORKSPACE;
   hipStream_t s = sgh_stream_of(stream);
   const int RS = g->R * g->S, KP = round_up(g->K, BK);
   const DgradPath path = dgrad_path(g);
@@ -1095,6 +1109,7 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
     float *partials = reinterpret_cast<float *>(static_cast<char *>(workspace) +
                                                 align256(size_t(RS) * KP * g->C * sizeof(float)) +
                                                 align256(sizeof(DgClsTable)));
+    if (ws_bytes < full) partials = nullptr;
     rc = sgh_dgrad3x3_run(g, dy, Wt, KP, dx, partials, s, "conv_dgrad/k_dgrad3x3", nullptr, accumulate);
   } else if (path == kDgradClasses) {
     float *Wc = static_cast<float *>(workspace);
@@ -1324,7 +1339,7 @@ int sgh_conv_dgrad_prepare_multi(const sgh_conv_prepare_item *items, int count, 
       const DgradPath path = dgrad_path(g);
       if (path != kDgradTile3x3 && path != kDgradGather) continue;   // the other kernels read W as it is or re-lay it their own way
       it.A = round_up(g->K, BK), it.B = g->C;
-      need = sgh_conv_workspace_bytes(g, SGH_CONV_DGRAD);
+      need = least_bytes_f32(g, SGH_CONV_DGRAD);
     } else {
       if (sgh_env().conv16_off || !sgh_conv16_dgrad_relayout_dims(g, &it.A, &it.B)) continue;
       need = sgh_conv16_workspace_bytes(g, SGH_CONV_DGRAD);
@@ -1363,8 +1378,8 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
   if (!conv_ok(g) || !x || !W || !y) return SGH_EINVAL;
   if (g->groups > 1) return conv_grouped_f32(g, SGH_CONV_FWD, x, W, bias, y, workspace, ws_bytes, stream);
   sgh_prelaid_clear_if_overlap(g, workspace, ws_bytes);
-  const size_t need = sgh_conv_workspace_bytes(g, SGH_CONV_FWD);
-  if (!workspace || ws_bytes < need) return SGH_EWORKSPACE;
+  const size_t full = sgh_conv_workspace_bytes(g, SGH_CONV_FWD);
+  if (!workspace || ws_bytes < least_bytes_f32(g, SGH_CONV_FWD)) return SGH_EWORKSPACE;
   hipStream_t s = sgh_stream_of(stream);
   float *Wt = static_cast<float *>(workspace);
   const int RS = g->R * g->S, CP = round_up(g->C, BK);
@@ -1378,13 +1393,14 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
   }
   sgh_conv_geom gt;
   if (fwd_as_dgrad(g, &gt)) {
-    // 3x3 stride 1 pad 1: the shared-tile kernel on the channel-swapped problem with reversed taps
+    // stride 1 with "same" padding, 3x3 or 5x5: the shared-tile kernel on the channel-swapped problem with reversed taps
     const long total = long(RS) * CP * g->K;
     long blocks = (total + NT - 1) / NT;
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(k_weight_relayout, dim3(int(blocks)), dim3(NT), 0, s, W, Wt, g->K, g->C, RS, CP, 2);
     float *partials = reinterpret_cast<float *>(static_cast<char *>(workspace) +
                                                 align256(size_t(RS) * CP * g->K * sizeof(float)));
+    if (ws_bytes < full) partials = nullptr;
     const int rc3 = sgh_dgrad3x3_run(&gt, x, Wt, CP, y, partials, s, "conv_fwd/k_dgrad3x3", bias, false);
     sgh_prof_stop(s);
     return rc3;
@@ -1562,7 +1578,8 @@ namespace {
 
 struct HalfPlan {
   size_t a_elems, b_elems, out_elems, inner;  // the two inputs, the output, the fp32 pass's workspace
-  size_t total() const { return align256(a_elems * 4) + align256(b_elems * 4) + align256(out_elems * 4) + inner; }
+  size_t copies() const { return align256(a_elems * 4) + align256(b_elems * 4) + align256(out_elems * 4); }
+  size_t total() const { return copies() + inner; }
 };
 
 inline HalfPlan half_plan(const sgh_conv_geom *g, int which) {
@@ -1588,8 +1605,8 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
                                       sgh_stream_of(stream));
     if (rc != SGH_EUNSUPPORTED) return rc;
     GroupPlan p = group_plan(g, sizeof(uint16_t));
-    const size_t sub_ws = sgh_conv_workspace_bytes_h(&p.sg, which);
-    return conv_grouped<uint16_t>(g, which, a, b, bias, out, workspace, ws_bytes, sub_ws, sgh_stream_of(stream),
+    const size_t sub_least = sgh_conv_workspace_least_bytes(&p.sg, which, 1);
+    return conv_grouped<uint16_t>(g, which, a, b, bias, out, workspace, ws_bytes, sub_least, sgh_stream_of(stream),
                                   [&](sgh_conv_geom *sg, int wh, const uint16_t *a_, const uint16_t *b_,
                                       const uint16_t *bias_, uint16_t *out_, void *ws, size_t wsb) {
                                     return conv_half(sg, wh, a_, b_, bias_, out_, ws, wsb, stream, in, outc);
@@ -1625,13 +1642,15 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
                               in == sgh_cast_bf16_to_f32, sgh_stream_of(stream));
     if (rc != SGH_EUNSUPPORTED) return rc;
   }
-  const HalfPlan p = half_plan(g, which);
-  if (!workspace || ws_bytes < p.total() + (bias ? align256(size_t(g->K) * 4) : 0)) return SGH_EWORKSPACE;
+  HalfPlan p = half_plan(g, which);
+  const size_t bias_bytes = bias ? align256(size_t(g->K) * 4) : 0;
+  if (workspace && ws_bytes < p.total() + bias_bytes) p.inner = least_bytes_f32(g, which);
+  if (!workspace || ws_bytes < p.total() + bias_bytes) return SGH_EWORKSPACE;
   char *w = static_cast<char *>(workspace);
   float *a32 = reinterpret_cast<float *>(w);
   float *b32 = reinterpret_cast<float *>(w + align256(p.a_elems * 4));
   float *o32 = reinterpret_cast<float *>(w + align256(p.a_elems * 4) + align256(p.b_elems * 4));
-  char *inner = w + align256(p.a_elems * 4) + align256(p.b_elems * 4) + align256(p.out_elems * 4);
+  char *inner = w + p.copies();
   float *bias32 = nullptr;
   int rc = in(a, a32, p.a_elems, stream);
   if (rc == SGH_OK) rc = in(b, b32, p.b_elems, stream);
@@ -1666,6 +1685,21 @@ size_t sgh_conv_workspace_bytes_h(const sgh_conv_geom *g, int which) {
     return p.x_bytes + p.y_bytes + sgh_conv_workspace_bytes_h(&p.sg, which);
   }
   const size_t wide = half_plan(g, which).total() + (which == SGH_CONV_FWD ? align256(size_t(g->K) * 4) : 0);
+  size_t native = sgh_conv16_workspace_bytes(g, which);
+  if (which == SGH_CONV_FWD && sgh_fwd_fewc16_workspace_bytes(g) > native) native = sgh_fwd_fewc16_workspace_bytes(g);
+  return wide > native ? wide : native;
+}
+
+size_t sgh_conv_workspace_least_bytes(const sgh_conv_geom *g, int which, int dtype) {
+  if (!conv_ok(g) || which < 0 || which > 2 || dtype < 0 || dtype > 1) return 0;
+  const size_t full = dtype == 0 ? sgh_conv_workspace_bytes(g, which) : sgh_conv_workspace_bytes_h(g, which);
+  if (g->groups > 1) {
+    if (sgh_group_conv_supported(g, which)) return full;
+    const GroupPlan p = group_plan(g, dtype == 0 ? sizeof(float) : sizeof(uint16_t));
+    return p.x_bytes + p.y_bytes + sgh_conv_workspace_least_bytes(&p.sg, which, dtype);
+  }
+  if (dtype == 0) return least_bytes_f32(g, which);
+  const size_t wide = half_plan(g, which).copies() + least_bytes_f32(g, which) + (which == SGH_CONV_FWD ? align256(size_t(g->K) * 4) : 0);
   size_t native = sgh_conv16_workspace_bytes(g, which);
   if (which == SGH_CONV_FWD && sgh_fwd_fewc16_workspace_bytes(g) > native) native = sgh_fwd_fewc16_workspace_bytes(g);
   return wide > native ? wide : native;

@@ -760,8 +760,11 @@ class CudnnConvHandle(_HasGeometry):
         self.dtype = x.data_type()
         ws_fn = _L().sgh_conv_workspace_bytes if self.dtype == kFloat32 else _L().sgh_conv_workspace_bytes_h
         need = max(ws_fn(C.byref(self.geom), w) for w in (0, 1, 2))
-        if need > workspace_byte_limit:
-            raise SingaHipError("workspace of %d bytes exceeds the limit" % need)
+        if need > workspace_byte_limit:   # the least that every pass accepts, and what else the limit allows
+            least = max(_L().sgh_conv_workspace_least_bytes(C.byref(self.geom), w, int(self.dtype != kFloat32)) for w in (0, 1, 2))
+            need = max(least, int(workspace_byte_limit) // 4 * 4)
+            if least > workspace_byte_limit:
+                raise SingaHipError("workspace of %d bytes exceeds the limit" % least)
         self.workspace_count = need // 4
         self.workspace = Tensor((max(self.workspace_count, 1),), x.device(), kFloat32)
         self.wgrad_workspace = None   # a second one, made when a weight gradient runs on the auxiliary stream

@@ -455,3 +455,27 @@ def test_shared_tile_data_gradient_is_chosen_by_size():
     assert not takes(2, 64, 14, 14, 72, 3, 2) and not takes(2, 48, 14, 14, 64, 3, 2) and not takes(2, 64, 80, 80, 64, 3, 2)
     assert takes(2, 64, 14, 14, 104, 3, 2)          # a longer reduction
     assert takes(32, 48, 64, 64, 24, 3, 2)          # a tile for every CU
+
+
+@pytest.mark.parametrize("geom, before", [
+    # (N, C, H, W, K, R, stride), the largest of the three passes' workspaces before the shared-tile kernel took the layer
+    ((9, 592, 12, 8, 261, 3, 2), 5797120), ((5, 64, 24, 22, 246, 3, 2), 2833920), ((1, 252, 16, 18, 125, 3, 2), 1161472),
+    ((3, 64, 33, 47, 32, 5, 1), None), ((2, 64, 40, 40, 64, 3, 1), None)])
+def test_least_workspace_of_a_convolution(geom, before):
+    """The least workspace is no more than the usual one and (where it is given) than a handle of this layer had to allow before;
+    every pass refuses a byte less (no launch: the check comes first)."""
+    L = _lib.lib()
+    n, c, h, w, k, r, stride = geom
+    g = _lib.ConvGeom()
+    assert L.sgh_conv_geom_init(C.byref(g), n, c, h, w, k, r, r, stride, stride, r // 2, r // 2) == 0
+    full = [L.sgh_conv_workspace_bytes(C.byref(g), q) for q in range(3)]
+    least = [L.sgh_conv_workspace_least_bytes(C.byref(g), q, 0) for q in range(3)]
+    assert all(0 <= a <= b for a, b in zip(least, full)) and least[1] < full[1]
+    assert before is None or max(least) <= before < max(full)
+    for q, name in enumerate(("sgh_conv_fwd_f32", "sgh_conv_dgrad_f32", "sgh_conv_wgrad_f32")):
+        bias = (None,) if q == 0 else ()
+        if least[q]:
+            assert getattr(L, name)(C.byref(g), 4096, 4096, *bias, 4096, 4096, least[q] - 1, None) < 0
+    half = [L.sgh_conv_workspace_least_bytes(C.byref(g), q, 1) for q in range(3)]
+    assert all(a <= L.sgh_conv_workspace_bytes_h(C.byref(g), q) for q, a in enumerate(half))
+    assert L.sgh_conv_workspace_least_bytes(C.byref(g), 3, 0) == 0 and L.sgh_conv_workspace_least_bytes(C.byref(g), 0, 2) == 0

@@ -1027,3 +1027,32 @@ def test_few_channel_data_gradient_rounding(singa, dev, case):
         want[:, :, rows[:, None], cols[None, :]] += np.einsum("nkpq,kc->ncpq", dy[:, :, prow, qcol].astype(np.float64), w[:, :, i, j].astype(np.float64))
     got = singa.GpuConvBackwardx(singa.from_numpy(dy, dev), wd, xd, h).to_numpy()
     assert nl2(got, want) < 2.0 ** -24 / np.sqrt(3) * np.sqrt((K + R * R) / 2)
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+@pytest.mark.parametrize("case", [(3, 64, 10, 10, 104, 3, 2, 1), (2, 36, 20, 22, 60, 5, 1, 1), (2, 80, 18, 18, 80, 3, 1, 2)])
+def test_convolution_within_a_workspace_limit(singa, dev, kind, case):
+    """A handle whose limit lies below the usual workspace (no room for partial sums; 60 and 40 channels also send 16-bit tensors
+    through the fp32 kernels) runs all passes, and refuses a limit below the least."""
+    N, C, H, W, K, R, stride, groups = case
+    print("limited workspace", kind, case, flush=True)
+    r = rng(sum(case))
+    dt, tol = (singa.kFloat32, 1e-5) if kind == "f32" else (singa.kBFloat16, 1e-2)
+    to = lambda a: singa.from_numpy(a.astype(np.float32), dev).AsType(dt)
+    back = lambda t: t.AsType(singa.kFloat32).to_numpy()
+    xt, wt, bt = to(randn(r, N, C, H, W)), to(randn(r, K, C // groups, R, R) * np.sqrt(2.0 * groups / (C * R * R))), to(randn(r, K))
+    make = lambda **kw: singa.CudnnConvHandle(xt, (R, R), (stride, stride), (R // 2, R // 2), C, K, True, groups, **kw)
+    free = make()
+    least = max(singa._L().sgh_conv_workspace_least_bytes(free.geom, q, int(kind != "f32")) for q in range(3))
+    usual = free.workspace.MemSize()
+    assert least < usual
+    tight, between = make(workspace_byte_limit=least), make(workspace_byte_limit=(least + usual) // 2)
+    assert tight.workspace.MemSize() == least and least <= between.workspace.MemSize() < usual
+    with pytest.raises(singa.SingaHipError):
+        make(workspace_byte_limit=least - 1)
+    dyt = to(randn(r, N, K, free.conv_height, free.conv_width))
+    passes = lambda h: [back(t) for t in (singa.GpuConvForward(xt, wt, bt, h), singa.GpuConvBackwardx(dyt, wt, xt, h), singa.GpuConvBackwardW(dyt, xt, wt, h))]
+    want = passes(free)
+    for h in (tight, between):
+        for got, ref in zip(passes(h), want):
+            assert nl2(got, ref) < tol
