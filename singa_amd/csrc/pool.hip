@@ -266,13 +266,14 @@ __global__ __launch_bounds__(kBlock) void k_pool_max_fwd_strip(const typename S:
   float top = best_of(r0.a, r0.b, r0.c).m;
 #pragma unroll
   for (int k = 0; k < kStrip; ++k) {
+    if (k >= g.rows) break;
     const Row3<S, GROUP> rm(v[2 * k + 1], g, s, h0 + 2 * k + 1), rb(v[2 * k + 2], g, s, h0 + 2 * k + 2);
     const float mid = best_of(rm.a, rm.b, rm.c).m, bot = best_of(rb.a, rb.b, rb.c).m;
     float best = top;
     if (mid > best) best = mid;
     if (bot > best) best = bot;
     top = bot;
-    if (s.makes && k < g.rows && s.p0 + k < g.P) S::st(out + size_t(k) * g.Q, best);
+    if (s.makes && s.p0 + k < g.P) S::st(out + size_t(k) * g.Q, best);
   }
 }
 
@@ -309,19 +310,20 @@ __global__ __launch_bounds__(kBlock) void k_pool_max_bwd_strip(const typename S:
   float dy_p = 0.f, ndy_p = 0.f;
 #pragma unroll
   for (int k = 0; k <= kStrip; ++k) {
+    if (k > g.rows) break;
     const Row3<S, GROUP> rm(v[2 * k + 1], g, s, h0 + 2 * k + 1), rb(v[2 * k + 2], g, s, h0 + 2 * k + 2);
     const RowBest mid = best_of(rm.a, rm.b, rm.c), bot = best_of(rb.a, rb.b, rb.c);
     float best = top.m;
     int code = top.k;
     if (mid.m > best) best = mid.m, code = 3 + mid.k;
     if (bot.m > best) code = 6 + bot.k;
-    if (!s.inside || s.p0 + k >= g.P || k > g.rows) code = 64;
+    if (!s.inside || s.p0 + k >= g.P) code = 64;
     top = bot;
     const float dyv = d[k];
     int ncode = __shfl_down(code, 1, GROUP);
     const float ndy = __shfl_down(dyv, 1, GROUP);
     if (last) ncode = 64;
-    if (k > 0 && k <= g.rows && s.makes && s.p0 + k - 1 < g.P) {
+    if (k > 0 && s.makes && s.p0 + k - 1 < g.P) {
       // block row p0 + k - 1: windows (.., q), (.., q + 1), then the two below, in that order
       const float o00 = 0.f + (code_p == 4 ? dy_p : 0.f);
       const float o01 = (0.f + (code_p == 5 ? dy_p : 0.f)) + (ncode_p == 3 ? ndy_p : 0.f);
@@ -743,9 +745,15 @@ inline bool strip_plan(const sgh_pool_geom *g, int esize, StripG *s) {
   if (x >= (size_t(1) << 31)) return false;   // (32-bit byte offsets)
   const int group = strip_group(g->Q);
   s->H = g->H, s->W = g->W, s->P = g->P, s->Q = g->Q;
-  s->strips = (g->P + kStrip - 1) / kStrip;
-  s->rows = (g->P + s->strips - 1) / s->strips;
   s->chunks = g->Q <= group ? 1 : (g->Q + group - 3) / (group - 2);
+  // rows: the more, the fewer are computed twice; but a strip is one chain of shuffles, so no more than leave every CU two
+  // wavefronts.  Backward against the kernels before, 500 shapes: with strips of seven throughout 1.20 times as fast below
+  // 100 000 elements and 1.47 below a million, 19 of 262 slower, down to 0.75 (4.0 -> 5.0 us); with this rule 1.44 and 1.70,
+  // two slower.  With one or four wavefronts per CU 1.42 / 1.57 and 1.34 / 1.71.
+  const long fill = long(g->N) * g->C * s->chunks * g->P * group / 64 / (2 * sgh_num_cus());
+  const int most = fill < 1 ? 1 : fill > kStrip ? kStrip : int(fill);
+  s->strips = (g->P + most - 1) / most;
+  s->rows = (g->P + s->strips - 1) / s->strips;
   s->units = int(size_t(g->N) * g->C * s->strips * s->chunks);   // (fewer than dx elements)
   s->x_bytes = unsigned(x);
   s->y_bytes = unsigned(size_t(g->N) * g->C * g->P * g->Q * esize);

@@ -847,6 +847,8 @@ def test_shared_tile_convolution_edges(singa, dev, case):
     # strips of 16, 32 and 64 lanes at and around the width they hold, odd rows and columns, several chunks per row
     (2, 3, 15, 31, 3), (3, 2, 9, 32, 3), (2, 2, 16, 33, 3), (1, 3, 29, 63, 3), (2, 1, 14, 66, 3), (1, 2, 31, 127, 3),
     (1, 1, 17, 129, 3), (1, 2, 7, 251, 3), (5, 7, 1, 2, 3), (4, 3, 2, 3, 3), (50, 9, 5, 7, 3), (1, 1, 43, 5, 3),
+    # strips of four, five and seven rows (small tensors are cut into strips of one)
+    (40, 90, 15, 31, 3), (16, 64, 43, 5, 3), (60, 64, 14, 33, 3),
     # 2 x 2: odd last rows and columns belong to no window, more blocks than one step of the grid covers, one window
     (3, 5, 8, 8, 2), (2, 3, 7, 9, 2), (2, 2, 6, 5, 2), (1, 2, 2, 2, 2), (1, 1, 3, 2, 2), (3, 100, 45, 37, 2),
 ])
