@@ -507,6 +507,19 @@ inline size_t chip_workspace_bytes(int C, int G) { return size_t(C) * size_t(G) 
 constexpr int kFwdWords = 4;
 inline size_t chip_fwd_workspace_bytes(int C, int G) { return size_t(C) * size_t(G) * kFwdWords * sizeof(unsigned long long); }
 
+// The value of the lane R before this one, around its row of 16 lanes (no LDS access, unlike a shuffle)
+template <int R>
+__device__ __forceinline__ float row_rotated(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + R, 0xF, 0xF, false));
+}
+template <int R>
+__device__ __forceinline__ double row_rotated(double v) {
+  const unsigned long long bits = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(bits)), 0x120 + R, 0xF, 0xF, false));
+  const unsigned hi = unsigned(__builtin_amdgcn_update_dpp(0, int(unsigned(bits >> 32)), 0x120 + R, 0xF, 0xF, false));
+  return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
+}
+
 // Sums of two values over the NT threads of a workgroup.  The rounding errors of the first levels of the tree average out
 // over its many sums, those of the last ones do not: from sums of eight lanes on it is in double.  With fp32 throughout and one
 // slice where there were two to eight, a channel's mean came out up to 2.7 times as far from the exact one.
@@ -515,10 +528,12 @@ template <int NT>
 __device__ __forceinline__ void chip_block_sums(float a, float b, double *red, double *A, double *B) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int o = 32; o >= 8; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+  for (int o = 32; o >= 16; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+  a += row_rotated<8>(a), b += row_rotated<8>(b);
   double da = a, db = b;
-#pragma unroll
-  for (int o = 4; o > 0; o >>= 1) da += __shfl_xor(da, o, 64), db += __shfl_xor(db, o, 64);
+  da += row_rotated<4>(da), db += row_rotated<4>(db);
+  da += row_rotated<2>(da), db += row_rotated<2>(db);
+  da += row_rotated<1>(da), db += row_rotated<1>(db);
   if (lane == 0) red[2 * wave] = da, red[2 * wave + 1] = db;
   __syncthreads();
   da = 0, db = 0;
@@ -533,8 +548,12 @@ __device__ __forceinline__ void chip_block_sums(float a, float b, double *red, d
 __device__ __forceinline__ void chip_totals(double a, double b, double *total, double *A, double *B) {
   const int t = threadIdx.x;
   if (t < kChipMaxG) {
+    a += row_rotated<8>(a), b += row_rotated<8>(b);
+    a += row_rotated<4>(a), b += row_rotated<4>(b);
+    a += row_rotated<2>(a), b += row_rotated<2>(b);
+    a += row_rotated<1>(a), b += row_rotated<1>(b);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+    for (int o = 32; o >= 16; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
     if ((t & 63) == 0) total[t >> 5] = a, total[(t >> 5) + 1] = b;
   }
   __syncthreads();
@@ -560,6 +579,22 @@ inline bool chip_slices_fit(int G, int C, int nt) {
   const long slots = long(sgh_num_cus()) * (nt == 512 ? 2 : 1);
   const bool xcd_runs = G <= 16 && C >= 8;
   return xcd_runs ? long(G) <= slots / 8 : long(G) <= slots;
+}
+
+// Whole rounds: as many slices as still fit into the rounds of (2 workgroups x CUs) that G slices of C channels need; with a run
+// of channels per XCD a round is what the XCD with most channels holds.  (A round more costs more than the thinner slices
+// save -- the workgroups of a channel wait for each other: two workgroups for every CU rounded up made 600 of 100 channels.
+// Backward, bfloat16 30 x 100 x 32 x 32 17.6 -> 10.6 us, 50 x 72 x 57 x 43 22.9 -> 14.9, fp32 32 x 48 x 56 x 56 16.5 -> 11.8;
+// forward 50 x 72 x 57 x 43 22.1 -> 12.7, 64 x 300 x 8 x 8 in one workgroup per channel 11.6 -> 5.6.  Without the XCDs in the
+// count 35 channels of 14 slices made 70 workgroups for the 64 places of an XCD: fp32 4 x 35 x 69 x 29
+// forward 12.0 -> 7.6 us, bfloat16 125 x 73 x 5 x 9 10.1 -> 6.5.)
+inline long chip_fill(long G, int C) {
+  const long slots = 2L * sgh_num_cus(), share = slots / 8, run = (C + 7) / 8;
+  const long rounds = C >= 8 && G <= 16 ? (run * G + share - 1) / share : (long(C) * G + slots - 1) / slots;
+  long fill = rounds * slots / C;
+  if (C >= 8 && fill <= 16) fill = rounds * share / run;
+  if (fill > kChipMaxG) fill = kChipMaxG;
+  return fill > G ? fill : G;
 }
 
 template <class S>
@@ -596,14 +631,7 @@ inline ChipPlan chip_plan(int N, int C, int HW) {
   }
   // a channel that fits one workgroup and a channel for every CU: nothing is exchanged
   const bool whole_channels = G == 1 && C >= sgh_num_cus();
-  // whole rounds: as many slices as still fit into the rounds of (2 workgroups x CUs) that this many need.  (A round more
-  // costs more than the thinner slices save -- the workgroups of a channel wait for each other: two workgroups for every CU
-  // rounded up, as it was, made 600 of 100 channels.  bfloat16 30 x 100 x 32 x 32 17.6 -> 10.6 us, 50 x 72 x 57 x 43
-  // 22.9 -> 14.9, fp32 32 x 48 x 56 x 56 16.5 -> 11.8)
-  const long slots = 2L * sgh_num_cus(), rounds = (long(C) * G + slots - 1) / slots;
-  long fill = rounds * slots / C;
-  if (fill > kChipMaxG) fill = kChipMaxG;
-  if (fill > G && !whole_channels) G = fill;
+  if (!whole_channels) G = chip_fill(G, C);
   while (G > 1 && (TV + G - 1) / G < 64) --G;
   if (G > kChipMaxG || G < 1) return p;
   p.vpg = int((TV + G - 1) / G);
@@ -902,11 +930,7 @@ inline ChipPlan chip_fwd_plan(int N, int C, int HW, bool two) {
   const long TV = long(N) * ((HW + S::VEC - 1) / S::VEC);
   const long per_wg = 512L * chip_fwd_nv<S>(two);
   long G = (TV + per_wg - 1) / per_wg;
-  const long slots = 2L * sgh_num_cus(), rounds = (long(C) * G + slots - 1) / slots;
-  // whole rounds, as in chip_plan (50 x 72 x 57 x 43 22.1 -> 12.7 us, 64 x 300 x 8 x 8 in one workgroup per channel 11.6 -> 5.6)
-  long fill = rounds * slots / C;
-  if (fill > kChipMaxG) fill = kChipMaxG;
-  if (fill > G) G = fill;
+  G = chip_fill(G, C);
   while (G > 1 && (TV + G - 1) / G < 64) --G;
   if (G > kChipMaxG || G < 1) return p;
   p.vpg = int((TV + G - 1) / G);

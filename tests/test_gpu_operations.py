@@ -1058,3 +1058,28 @@ def test_convolution_within_a_workspace_limit(singa, dev, kind, case):
     for h in (tight, between):
         for got, ref in zip(passes(h), want):
             assert nl2(got, ref) < tol
+
+
+@pytest.mark.parametrize("shape", [(4, 35, 69, 29), (125, 73, 5, 9), (102, 41, 16, 112), (9, 7, 40, 41), (3, 129, 30, 30)])
+def test_bn_slice_counts_around_the_xcds(singa, dev, shape):
+    """Channel counts that leave the XCDs unequal runs of channels (and fewer than eight channels): forward and backward against
+    the oracle."""
+    print("bn slices", shape, flush=True)
+    r = rng(sum(shape))
+    C = shape[1]
+    x, dy = (randn(r, *shape) * 1.5 + 0.3).astype(np.float32), randn(r, *shape)
+    xd = singa.from_numpy(x, dev)
+    h = singa.CudnnBatchNormHandle(0.9, xd)
+    gamma, beta = (randn(r, C) * 0.2 + 1).astype(np.float32), randn(r, C)
+    gd, bd = singa.from_numpy(gamma, dev), singa.from_numpy(beta, dev)
+    y, mean, inv = singa.GpuBatchNormForwardTraining(h, xd, gd, bd, singa.from_numpy(np.zeros(C, np.float32), dev), singa.from_numpy(np.ones(C, np.float32), dev))
+    x64, d64 = x.astype(np.float64), dy.astype(np.float64)
+    S = lambda v: v[None, :, None, None]
+    m, i = x64.mean((0, 2, 3)), 1 / np.sqrt(x64.var((0, 2, 3)) + 1e-5)
+    xh = (x64 - S(m)) * S(i)
+    assert nl2(y.to_numpy(), xh * S(gamma) + S(beta)) < 1e-6
+    dx, dg, db = singa.GpuBatchNormBackward(h, singa.from_numpy(dy, dev), xd, gd, mean, inv)
+    n = x.size // C
+    want = S(gamma * i) * (d64 - S(d64.sum((0, 2, 3))) / n - xh * S((d64 * xh).sum((0, 2, 3))) / n)
+    assert nl2(dx.to_numpy(), want) < 1e-6
+    assert nl2(dg.to_numpy(), (d64 * xh).sum((0, 2, 3))) < 1e-5 and nl2(db.to_numpy(), d64.sum((0, 2, 3))) < 1e-5
