@@ -716,16 +716,12 @@ def AddRow(v, m):
 
 # ------------------------------------------------------------------------------------ operations
 
-class _HasGeometry(object):
-    """A handle with a geometry structure, `geom`, that calls get the address of: asked for each time, because a copied or
-    unpickled handle and one whose `geom` was replaced have a structure of their own."""
-
-    @property
-    def geom_ptr(self):
-        return C.addressof(self.geom)
+# A handle's geometry goes to the library by address.  The address is asked for at every call: a copied or unpickled handle,
+# and one whose `geom` was replaced, has a structure of its own.
+_address = C.addressof
 
 
-class CudnnConvHandle(_HasGeometry):
+class CudnnConvHandle(object):
     """Geometry + workspace of a convolution on the GPU device.  Same constructor arguments and
     public fields as the reference's handle (src/model/operation/convolution.h:43-129; fields read
     from Python: src/api/model_operation.i:37-54)."""
@@ -783,7 +779,7 @@ def GpuConvForward(x, W, b, h):
     y = _empty(Tensor, h.dy_shape, x.device(), x.data_type())
     bias = b.ptr if (h.bias_term and b is not None) else None
     fn, name = _fn("conv_fwd", x)
-    check(fn(h.geom_ptr, x.ptr, W.ptr, bias, y.ptr, h.workspace.ptr, h.workspace.MemSize(),
+    check(fn(_address(h.geom), x.ptr, W.ptr, bias, y.ptr, h.workspace.ptr, h.workspace.MemSize(),
              x.device().stream), name)
     return y
 
@@ -795,7 +791,7 @@ def GpuConvBackwardxAccumulate(dy, W, x, h, dx):
     h._check_dy(dy)
     _same(dx, x)
     if dy.data_type() == kFloat32:   # (on 16-bit tensors the kernel's read-modify-write loses to the separate add)
-        rc = _L().sgh_conv_dgrad_acc_f32(h.geom_ptr, dy.ptr, W.ptr, dx.ptr, h.workspace.ptr,
+        rc = _L().sgh_conv_dgrad_acc_f32(_address(h.geom), dy.ptr, W.ptr, dx.ptr, h.workspace.ptr,
                                          h.workspace.MemSize(), dy.device().stream)
         if rc != _lib.SGH_EUNSUPPORTED:
             check(rc, "sgh_conv_dgrad_acc_f32")
@@ -808,7 +804,7 @@ def GpuConvBackwardx(dy, W, x, h):
     h._check_dy(dy)
     dx = _like(x)
     fn, name = _fn("conv_dgrad", dy)
-    check(fn(h.geom_ptr, dy.ptr, W.ptr, dx.ptr, h.workspace.ptr, h.workspace.MemSize(),
+    check(fn(_address(h.geom), dy.ptr, W.ptr, dx.ptr, h.workspace.ptr, h.workspace.MemSize(),
              dy.device().stream), name)
     return dx
 
@@ -832,7 +828,7 @@ def GpuConvBackwardW(dy, x, W, h, stream=None, out=None):
             h.wgrad_workspace = Tensor(((max(need, 4) + 3) // 4,), dy.device(), kFloat32)
         ws = h.wgrad_workspace
         dy.device().UsedOn(stream, dy, x, dW, ws)
-    check(fn(h.geom_ptr, dy.ptr, x.ptr, dW.ptr, ws.ptr, ws.MemSize(),
+    check(fn(_address(h.geom), dy.ptr, x.ptr, dW.ptr, ws.ptr, ws.MemSize(),
              dy.device().stream if stream is None else stream), name)
     return dW
 
@@ -847,7 +843,7 @@ def GpuConvBackwardWb(dy, x, W, b, h):
     h._check_x(x)
     dW, db = _like(W), _like(b)
     ws = h.workspace
-    check(_L().sgh_conv_wgrad_bias_f32(h.geom_ptr, dy.ptr, x.ptr, dW.ptr, db.ptr, ws.ptr, ws.MemSize(),
+    check(_L().sgh_conv_wgrad_bias_f32(_address(h.geom), dy.ptr, x.ptr, dW.ptr, db.ptr, ws.ptr, ws.MemSize(),
                                        dy.device().stream), "sgh_conv_wgrad_bias_f32")
     return dW, db
 
@@ -883,7 +879,7 @@ def GpuConvBackwardb(dy, b, h):
     h._check_dy(dy)
     db = _like(b)
     fn, name = _fn("conv_bgrad", dy)
-    check(fn(h.geom_ptr, dy.ptr, db.ptr, dy.device().stream), name)
+    check(fn(_address(h.geom), dy.ptr, db.ptr, dy.device().stream), name)
     return db
 
 
@@ -993,7 +989,7 @@ def GpuBatchNormReLUBackward(h, dy, x, scale, bias, mean, var):
     return [dx, ds, db]
 
 
-class CudnnPoolingHandle(_HasGeometry):
+class CudnnPoolingHandle(object):
     """``CudnnPoolingHandle(x, kernel, stride, padding, is_max)``
     (src/model/operation/pooling.h:40-91)."""
 
@@ -1016,7 +1012,7 @@ class CudnnPoolingHandle(_HasGeometry):
 def GpuPoolingForward(h, x):
     y = _empty(Tensor, h.dy_shape, x.device(), x.data_type())
     fn, name = _fn("pool_fwd", x)
-    check(fn(h.geom_ptr, x.ptr, y.ptr, x.device().stream), name)
+    check(fn(_address(h.geom), x.ptr, y.ptr, x.device().stream), name)
     return y
 
 
@@ -1027,5 +1023,5 @@ def GpuPoolingBackward(h, dy, x, y):
         raise SingaHipError("dy and x differ in data type")
     dx = _like(x)
     fn, name = _fn("pool_bwd", x)
-    check(fn(h.geom_ptr, dy.ptr, x.ptr, y.ptr if y is not None else None, dx.ptr, dy.device().stream), name)
+    check(fn(_address(h.geom), dy.ptr, x.ptr, y.ptr if y is not None else None, dx.ptr, dy.device().stream), name)
     return dx

@@ -422,21 +422,29 @@ assert type(like) is singa.Tensor and like.shape() == [3, 5] and like.ptr == 30,
     subprocess.run([sys.executable, "-c", program, stub], check=True, cwd=ROOT, timeout=60)
 
 
-def test_copied_handles_pass_their_own_geometry():
+def test_copied_handles_pass_their_own_geometry(monkeypatch):
     """A pooling handle that was copied, pickled or given another geometry structure calls with the structure it holds."""
     import copy
     import pickle
 
-    from singa_amd import _native, singa_wrap as singa
-    x = singa.from_device_pointer(4096, (2, 3, 8, 8), object(), singa.kFloat32)
+    from singa_amd import singa_wrap as singa
+
+    class Device(object):
+        stream = None
+
+    passed = []
+    x = singa.from_device_pointer(4096, (2, 3, 8, 8), Device(), singa.kFloat32)
+    monkeypatch.setattr(singa, "_fn", lambda name, t: (lambda geom, *rest: passed.append(geom) or 0, name))
+    monkeypatch.setattr(singa, "_empty", lambda *a: x)
     h = singa.CudnnPoolingHandle(x, (3, 3), (2, 2), (1, 1), True)
-    other = copy.deepcopy(h)
-    assert other.geom_ptr == C.addressof(other.geom) != h.geom_ptr
-    loaded = pickle.loads(pickle.dumps(h))
-    assert loaded.geom_ptr == C.addressof(loaded.geom) and loaded.geom.P == h.geom.P
+    other, loaded = copy.deepcopy(h), pickle.loads(pickle.dumps(h))
+    for handle in (h, other, loaded):
+        singa.GpuPoolingForward(handle, x)
+    assert passed == [C.addressof(v.geom) for v in (h, other, loaded)] and len(set(passed)) == 3
     h.geom = other.geom
-    assert h.geom_ptr == other.geom_ptr
-    assert _native.sgh_pool_fwd_f32(loaded.geom_ptr, None, None, None) < 0   # (null tensors are refused)
+    singa.GpuPoolingForward(h, x)
+    assert passed[-1] == C.addressof(other.geom)
+
 
 
 def test_shared_tile_data_gradient_is_chosen_by_size():
