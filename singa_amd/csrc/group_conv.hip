@@ -62,7 +62,7 @@ __device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsr
                                              int planes_end, int vrow0) {
   const int total = planes * a.VR * a.VC;
   constexpr int U = 4;
-  bool odd = false;
+  float zero = 0.f;   // until it has been multiplied with an infinity or a NaN
   for (int i0 = threadIdx.x; i0 < total; i0 += GT * U) {
     float v[U];
 #pragma unroll
@@ -82,11 +82,11 @@ __device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsr
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      odd = odd || !isfinite(v[u]);
+      zero = fmaf(v[u], 0.f, zero);
       if (i0 + u * GT < total) lds[i0 + u * GT] = v[u];
     }
   }
-  return odd;
+  return zero != 0.f;
 }
 
 // The zeros that pad the image, and in the data gradient those between its rows, are multiplied like everything else; that
@@ -153,20 +153,16 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
               if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP) acc[(i - r) / T] = fmaf(w[r * R + s], v, acc[(i - r) / T]);
           }
         }
-      } else {
+      } else {   // (in loops: this path is small rather than fast)
         const int y0 = p0 + st * STRIP - a.padh, x0 = q - a.padw;
 #pragma unroll
-        for (int i = 0; i < STRIP - 1 + R; ++i) {
-          const int yy = y0 + i, y = a.d_dil.div(yy < 0 ? 0 : yy);
-          const bool row = yy >= 0 && y < a.SH && y * a.dil == yy;
-#pragma unroll
-          for (int s = 0; s < R; ++s) {
-            const int xx = x0 + s, x = a.d_dil.div(xx < 0 ? 0 : xx);
-            const bool there = row && xx >= 0 && x < a.SW && x * a.dil == xx;
-            const float v = im[i * a.VC + s];
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-              if (i >= r && i - r < STRIP) acc[i - r] = there ? fmaf(w[r * R + s], v, acc[i - r]) : acc[i - r];
+        for (int o = 0; o < STRIP; ++o) {
+#pragma unroll 1
+          for (int k = 0; k < RS; ++k) {
+            const int r = k / R, s = k - r * R, yy = y0 + o + r, xx = x0 + s;
+            const int y = a.d_dil.div(yy < 0 ? 0 : yy), x = a.d_dil.div(xx < 0 ? 0 : xx);
+            const bool there = yy >= 0 && y < a.SH && y * a.dil == yy && xx >= 0 && x < a.SW && x * a.dil == xx;
+            if (there) acc[o] = fmaf(wf[k], im[(o + r) * a.VC + s], acc[o]);
           }
         }
       }
@@ -231,16 +227,13 @@ __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__re
             }
           }
         } else {
+#pragma unroll 1
+          for (int o = 0; o < STRIP && p + o < pe; ++o) {
+            const float dd = ld_elem<S>(ys, (((n0 + ul) * K + k) * a.DH + p + o) * a.DW + q, true);
 #pragma unroll
-          for (int i = 0; i < (STRIP - 1) * T + R; ++i) {
+            for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int s = 0; s < R; ++s) {
-              const float v = im[i * a.VC + s];
-#pragma unroll
-              for (int r = 0; r < R; ++r)
-                if (i >= r && (i - r) % T == 0 && (i - r) / T < STRIP)
-                  acc[r * R + s] = p + (i - r) / T < pe ? fmaf(d[(i - r) / T], v, acc[r * R + s]) : acc[r * R + s];
-            }
+              for (int s = 0; s < R; ++s) acc[r * R + s] = fmaf(dd, im[(o * T + r) * a.VC + s], acc[r * R + s]);
           }
         }
       }
