@@ -1141,7 +1141,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
     const int ev = g->W >= 7 ? 8 : 4, QO = (g->H * g->W + ev - 1) / ev;
     const int KP = (g->K + KC - 1) / KC * KC;
     // The tile with the least work for a CU: the tiles that fall to it, one after the other or two at a time where their LDS
-    // fits twice, and twice the smallest tile's products (ten fifths) per such turn for staging and stores.  Over 1000 layers
+    // fits twice, and 2.4 times the smallest tile's products (twelve fifths) per such turn for staging and stores.  Over 1000 layers
     // of 8 to 640 channels the choice is 1.317 times as fast as the tap-by-tap kernel and the tiles before this one, two
     // layers slower than 0.95; the largest tile that gives three quarters of the CUs a workgroup made 1.29, 13 slower, down to
     // 0.63 where the smallest tile just missed a single turn: bfloat16 12 x 208 x 56 x 63 -> 62 25.2 us with 171 tiles of
@@ -1156,7 +1156,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
       const long groups = images * QO < sp / ev + 2 * images ? images * QO : sp / ev + 2 * images;
       if (G + 1024 >= (long(1) << 31) || groups > (ev == 8 ? 64 : 128) || lds > size_t(160) * 1024) continue;
       const long load = ((G + mt - 1) / mt * mt_c + sgh_num_cus() - 1) / sgh_num_cus();
-      const long turns = lds <= size_t(80) * 1024 ? (load + 1) / 2 : load, cost = load * tiles[i][3] + 10 * turns;
+      const long turns = lds <= size_t(80) * 1024 ? (load + 1) / 2 : load, cost = load * tiles[i][3] + 12 * turns;
       if (p.slab != 0 && cost >= least) continue;
       least = cost;
       p.slab = tiles[i][0];
