@@ -13,7 +13,7 @@ constexpr int BT = 1024, BU = 8;
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
-// A piece of 16 bytes (8 or 2 for short vector classes) at element alignment
+// A piece of 16 bytes, or one element of 4 or 2 bytes (planes shorter than a vector), at element alignment
 template <int BYTES>
 struct Piece;
 template <>

@@ -1131,7 +1131,7 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
   }
   for (int cls = st * st; cls < 5; ++cls) p.cls_tile0[cls] = int(tiles);
   // 3x3 / stride 1 / padding 1: the slab kernel, when its slab fits beside the weight tiles in the 160 KB of LDS and its
-  // threads cover the slab's pixel groups.  Groups of 8 pixels at element alignment, of 4 on rows of 3 to 6 (a group
+  // threads cover the slab's pixel groups: rows of 3 to 177 pixels with tiles of 128 positions, to 113 with tiles of 256.  Groups of 8 pixels at element alignment, of 4 on rows of 3 to 6 (a group
   // may end one row and start the next, no more).
   if (fs == 1 && g->R == 3 && g->S == 3 && st == 1 && g->pad_h == 1 && g->pad_w == 1 && !sgh_env().slab16_off &&
       g->W >= 3 && g->H * g->W >= (g->W >= 7 ? 8 : 4)) {

@@ -19,8 +19,10 @@
 // wavefronts per SIMD) share a CU and one's staging work and barriers overlap the other's MFMAs.
 //
 // The row pitch of the slab is the row's own length, Q + 2 o, and a channel gets 256, 512 or 1024 floats, the smallest that
-// holds the rows a tile touches: any plane width up to about 140 fits, 7 x 7 planes take half the LDS that a pitch of 16
-// took, and a tile's reads step through the banks almost contiguously.
+// holds the rows a tile touches: 7 x 7 planes take half the LDS that a pitch of 16 took, and a tile's reads step through the
+// banks almost contiguously.  Square planes fit up to a width of 168 (3x3, 128-pixel tiles; 126 with the 256-pixel tiles of up
+// to 32 channels), 101 gradient columns at stride 2, 89 with 5x5 filters (74 with up to 32 channels); wider ones run the
+// kernels of igemm.hip.
 #include <stdlib.h>
 
 #include "common.h"
@@ -436,8 +438,9 @@ inline D3Plan plan(const sgh_conv_geom *g) {
   // Work balance.  Whole multiples of the CU count of tiles run one tile per workgroup; the
   // remaining tiles (all of them when there are fewer tiles than CUs) are cut into (tile, chunk)
   // units and dealt evenly to one workgroup per CU (two per CU measured slower: twice the
-  // partial tiles to write and sum), so that no CU is left with a whole extra tile while others idle.  Tiles shared between workgroups are finished by
-  // k_dgrad3x3_fixup in a fixed order: results stay run-to-run identical.
+  // partial tiles to write and sum), so that no CU is left with a whole extra tile while others
+  // idle.  Tiles shared between workgroups are finished by k_dgrad3x3_fixup in a fixed order:
+  // results stay run-to-run identical.
   const int cus = sgh_num_cus();
   p.ctiles = (g->C + p.bm - 1) / p.bm;
   const long tiles = long(p.ctiles) * ((long(g->N) * g->P * g->Q + p.bn - 1) / p.bn);

@@ -9,9 +9,8 @@
 // transposed) a thread copies one octet with a 16-byte load; with the row index contiguous (A transposed,
 // B not transposed) it loads eight rows of one k with a 16-byte load and writes them as eight 2-byte LDS
 // stores; pointers, pitches or edges that do not allow the 16-byte access fall back to single elements.
-// The reduction is not split: results are run-to-run identical.
-//
-// Problems with few output tiles take the second kernel of this file.
+// This kernel does not split the reduction.  Problems with few output tiles take the second kernel of this file, which splits it
+// over the wavefronts of a workgroup and adds their sums in a fixed order: results are run-to-run identical either way.
 #include <hip/hip_runtime.h>
 
 #include "common.h"

@@ -145,6 +145,8 @@ void launch(int tile, int waves, const float *A, int lda, const float *B, int ld
 //   1000 x 2048 x 512 NT     27 / 31            so the line lies at three tiles per CU
 // Wavefronts: 16 pay from a reduction of 1024 on (512 x 1024 x 2048 NN: 28 / 25 / 24 us with 4 / 8 / 16), and with few
 // indices per wavefront the sum of the partial tiles costs more than it saves (784 x 1000 x 128 NN: 6.1 / 6.0 / 7.1).
+// Reductions of 1 to 128 take it as well: 4.2 us on either kernel at 128 x 1000 x 16, 4.7 / 4.8 at 1024 x 1024 x 16, 4.7 / 4.2
+// at 2048 x 512 x 4 and 5.6 / 4.4 at 512 x 512 x 64.
 static bool plan(bool nt, int M, int N, int K, int *tile, int *waves) {
   const long t32 = long((M + 31) / 32) * ((N + 31) / 32), cus = sgh_num_cus();
   if (t32 > (nt ? 3 : 8) * cus) return false;

@@ -402,7 +402,8 @@ PyMemberDef tensor_members[] = {{"_shape", T_OBJECT, offsetof(Tensor, shape), 0,
                                 {nullptr, 0, 0, 0, nullptr}};
 PyGetSetDef tensor_getset[] = {{"ptr", tensor_ptr, nullptr, "device address", nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMethodDef tensor_methods[] = {
-    {"shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(tensor_shape)), METH_FASTCALL | METH_KEYWORDS, "extents, or one of them"},
+    {"shape", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(tensor_shape)), METH_FASTCALL | METH_KEYWORDS,
+     "extents, or one of them"},
     {"Size", tensor_size, METH_NOARGS, "number of elements"},
     {"MemSize", tensor_memsize, METH_NOARGS, "bytes"},
     {"nDim", tensor_ndim, METH_NOARGS, "number of dimensions"},
@@ -452,7 +453,8 @@ PyObject *fork_(PyObject *, PyObject *h) {
   return PyLong_FromVoidPtr(aux);
 }
 
-#define SGH_CALL(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call<Entry_##name>::call)), METH_FASTCALL, nullptr},
+#define SGH_CALL(name) \
+  {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(Call<Entry_##name>::call)), METH_FASTCALL, nullptr},
 #define SGH_CALL3(name) SGH_CALL(name##_f32) SGH_CALL(name##_f16) SGH_CALL(name##_bf16)
 
 PyMethodDef methods[] = {

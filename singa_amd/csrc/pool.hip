@@ -126,8 +126,9 @@ __global__ __launch_bounds__(kBlock) void k_pool_max_bwd(const typename S::elem 
 // into chunks that overlap by one lane on either side.
 //
 // The kernels that the odd sizes ran before staged elements one by one in LDS (backward) or gave every output its own nine
-// loads (forward): bfloat16 50 x 72 x 57 x 43, 40.7 + 18.8 us; here 17.6 + 9.2.  Backward of the residual networks' stem (N x 64 x 112 x 112)
-// against rows staged in LDS as whole vectors: bfloat16 N = 64 65.8 -> 53.0, 128 125 -> 107, fp32 N = 64 82.3 -> 82.8.
+// loads (forward): bfloat16 50 x 72 x 57 x 43, 40.7 + 18.8 us; here 17.6 + 9.2.  Backward of the residual networks' stem
+// (N x 64 x 112 x 112) against rows staged in LDS as whole vectors: bfloat16 N = 64 65.8 -> 53.0, 128 125 -> 107, fp32 N = 64
+// 82.3 -> 82.8.
 constexpr int kStrip = 7;
 constexpr float kLowest = -3.402823466e38f;
 
@@ -810,12 +811,16 @@ int pool_fwd(const sgh_pool_geom *g, const typename S::elem *x, typename S::elem
   StripG sg;
   QuadG qg;
   if (g->is_max && g->kernel_h == 3 && g->kernel_w == 3 && g->stride_h == 2 && g->stride_w == 2 && g->pad_h == 1 &&
-      g->pad_w == 1 && g->H % 2 == 0 && g->W % 2 == 0 && g->Q % S::VEC == 0 && sgh_aligned16(x) && sgh_aligned16(y) && (esize == 2 || total <= kStripFwdMin))
+      g->pad_w == 1 && g->H % 2 == 0 && g->W % 2 == 0 && g->Q % S::VEC == 0 && sgh_aligned16(x) && sgh_aligned16(y) &&
+      (esize == 2 || total <= kStripFwdMin))
     hipLaunchKernelGGL(k_pool_max_fwd_3x3s2<S>, dim3(grid_for(total / S::VEC)), dim3(kBlock), 0, sgh_stream_of(stream), x, y,
                        g->H, g->W, total / S::VEC);
   else if (g->is_max && strip_plan(g, esize, &sg)) {
     const int group = strip_group(g->Q);
-    auto kern = group == 8 ? k_pool_max_fwd_strip<S, 8> : group == 16 ? k_pool_max_fwd_strip<S, 16> : group == 32 ? k_pool_max_fwd_strip<S, 32> : k_pool_max_fwd_strip<S, 64>;
+    auto kern = group == 8    ? k_pool_max_fwd_strip<S, 8>
+                : group == 16 ? k_pool_max_fwd_strip<S, 16>
+                : group == 32 ? k_pool_max_fwd_strip<S, 32>
+                              : k_pool_max_fwd_strip<S, 64>;
     hipLaunchKernelGGL(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, sg);
   } else if (quad_plan(g, esize, false, &qg)) {
     auto kern = g->is_max ? k_pool_quad_fwd<S, true> : k_pool_quad_fwd<S, false>;
@@ -861,7 +866,10 @@ int pool_bwd(const sgh_pool_geom *g, const typename S::elem *dy, const typename 
   QuadG qg;
   if (g->is_max && strip_plan(g, esize, &sg)) {
     const int group = strip_group(g->Q);
-    auto kern = group == 8 ? k_pool_max_bwd_strip<S, 8> : group == 16 ? k_pool_max_bwd_strip<S, 16> : group == 32 ? k_pool_max_bwd_strip<S, 32> : k_pool_max_bwd_strip<S, 64>;
+    auto kern = group == 8    ? k_pool_max_bwd_strip<S, 8>
+                : group == 16 ? k_pool_max_bwd_strip<S, 16>
+                : group == 32 ? k_pool_max_bwd_strip<S, 32>
+                              : k_pool_max_bwd_strip<S, 64>;
     SGH_LAUNCH_TIMED(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), dy, x, dx, sg);
   } else if (quad_plan(g, esize, true, &qg)) {
     auto kern = g->is_max ? k_pool_quad_bwd<S, true> : k_pool_quad_bwd<S, false>;

@@ -1026,7 +1026,8 @@ def test_few_channel_data_gradient_rounding(singa, dev, case):
     dy = randn(r, N, K, P, Q)
     want = np.zeros((N, C, H, W))
     for i, j, prow, qcol, rows, cols in _windows(x, R, stride, p, P, Q):
-        want[:, :, rows[:, None], cols[None, :]] += np.einsum("nkpq,kc->ncpq", dy[:, :, prow, qcol].astype(np.float64), w[:, :, i, j].astype(np.float64))
+        tap = np.einsum("nkpq,kc->ncpq", dy[:, :, prow, qcol].astype(np.float64), w[:, :, i, j].astype(np.float64))
+        want[:, :, rows[:, None], cols[None, :]] += tap
     got = singa.GpuConvBackwardx(singa.from_numpy(dy, dev), wd, xd, h).to_numpy()
     assert nl2(got, want) < 2.0 ** -24 / np.sqrt(3) * np.sqrt((K + R * R) / 2)
 
@@ -1053,7 +1054,8 @@ def test_convolution_within_a_workspace_limit(singa, dev, kind, case):
     with pytest.raises(singa.SingaHipError):
         make(workspace_byte_limit=least - 1)
     dyt = to(randn(r, N, K, free.conv_height, free.conv_width))
-    passes = lambda h: [back(t) for t in (singa.GpuConvForward(xt, wt, bt, h), singa.GpuConvBackwardx(dyt, wt, xt, h), singa.GpuConvBackwardW(dyt, xt, wt, h))]
+    passes = lambda h: [back(t) for t in (singa.GpuConvForward(xt, wt, bt, h), singa.GpuConvBackwardx(dyt, wt, xt, h),
+                                          singa.GpuConvBackwardW(dyt, xt, wt, h))]
     want = passes(free)
     for h in (tight, between):
         for got, ref in zip(passes(h), want):
@@ -1072,7 +1074,8 @@ def test_bn_slice_counts_around_the_xcds(singa, dev, shape):
     h = singa.CudnnBatchNormHandle(0.9, xd)
     gamma, beta = (randn(r, C) * 0.2 + 1).astype(np.float32), randn(r, C)
     gd, bd = singa.from_numpy(gamma, dev), singa.from_numpy(beta, dev)
-    y, mean, inv = singa.GpuBatchNormForwardTraining(h, xd, gd, bd, singa.from_numpy(np.zeros(C, np.float32), dev), singa.from_numpy(np.ones(C, np.float32), dev))
+    running = [singa.from_numpy(v, dev) for v in (np.zeros(C, np.float32), np.ones(C, np.float32))]
+    y, mean, inv = singa.GpuBatchNormForwardTraining(h, xd, gd, bd, *running)
     x64, d64 = x.astype(np.float64), dy.astype(np.float64)
     S = lambda v: v[None, :, None, None]
     m, i = x64.mean((0, 2, 3)), 1 / np.sqrt(x64.var((0, 2, 3)) + 1e-5)
