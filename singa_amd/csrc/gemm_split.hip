@@ -147,18 +147,26 @@ void launch(int tile, int waves, const float *A, int lda, const float *B, int ld
 // indices per wavefront the sum of the partial tiles costs more than it saves (784 x 1000 x 128 NN: 6.1 / 6.0 / 7.1).
 // Reductions of 1 to 128 take it as well: 4.2 us on either kernel at 128 x 1000 x 16, 4.7 / 4.8 at 1024 x 1024 x 16, 4.7 / 4.2
 // at 2048 x 512 x 4 and 5.6 / 4.4 at 512 x 512 x 64.
-static bool plan(bool nt, int M, int N, int K, int *tile, int *waves) {
+//   Beyond five and a half tiles per CU long reductions go back to the tiled kernel: NN 421 x 3758 x 1172 63 / 74, 1809 x 947 x
+// 1833 96 / 109, TT 848 x 2072 x 2733 137 / 175 against 30 / 22 at 1879 x 625 x 529 and 33 / 33 at 773 x 1988 x 585; with A alone
+// transposed it holds on to reductions of 2000 (1672 x 925 x 2032 104 / 79; 503 x 3847 x 2373 124 / 131).
+//   With both reductions contiguous four wavefronts do from one tile per CU on, eight before: 160 problems, reductions of 256 to
+// 4096, against the kernels before; from one tile per CU on 0.91 to 1.08 times as fast with the wavefronts of the other cases and
+// 1.01 to 1.11 with four (392 x 677 x 3084: 41.8 us before, 55.6, 42); below, 2048 and up, 1.20 with sixteen and 1.22 with eight.
+static bool plan(bool ta, bool tb, int M, int N, int K, int *tile, int *waves) {
+  const bool nt = !ta && tb;
   const long t32 = long((M + 31) / 32) * ((N + 31) / 32), cus = sgh_num_cus();
-  if (t32 > (nt ? 3 : 8) * cus) return false;
+  if (t32 > (nt ? 3 : 8) * cus || (2 * t32 > 11 * cus && K > (ta && !tb ? 2048 : 640))) return false;
   *tile = 2 * t32 < cus ? 16 : 32;
   *waves = K < 256 ? 4 : K < 1024 || *tile == 16 ? 8 : 16;
+  if (nt && *tile == 32 && K >= 256) *waves = t32 >= cus ? 4 : 8;
   return (M + *tile - 1) / *tile <= 65535;
 }
 
 int sgh_gemm_split_run(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
                        float beta, float *C, int ldc, hipStream_t s) {
   int tile, waves;
-  if (!plan(!transA && transB, M, N, K, &tile, &waves)) return SGH_EUNSUPPORTED;
+  if (!plan(transA, transB, M, N, K, &tile, &waves)) return SGH_EUNSUPPORTED;
   if (!transA && transB) launch<true, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
   else if (!transA) launch<true, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
   else if (transB) launch<false, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);

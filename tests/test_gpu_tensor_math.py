@@ -554,10 +554,11 @@ def test_int_float_casts(singa, dev):
 
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 33, 7), (17, 15, 250), (33, 100, 257), (128, 10, 1031), (1, 300, 64),
-                                   (400, 333, 70), (415, 401, 255), (417, 349, 1033)])
+                                   (400, 333, 70), (415, 401, 255), (417, 349, 1033), (512, 513, 260), (1500, 1000, 644)])
 def test_gemm_split_reduction_edges(singa, dev, kind, M, N, K):
     """Mult at the edges of the kernels that split the reduction over a workgroup's wavefronts: tiles of 16 and of 32 (from 128
-    tiles of 32 on), 4, 8 and 16 wavefronts, reductions that end inside a group or leave wavefronts without work, odd matrix
+    tiles of 32 on, with both reductions contiguous four wavefronts from 256 on; long ones beyond 1408 tiles are the tiled kernel's
+    unless A alone is transposed), 4, 8 and 16 wavefronts, reductions that end inside a group or leave wavefronts without work, odd matrix
     edges, all four transposes.  Bound: K products in fp32, |error| <= K 2^-24 sum |a b| (+ one rounding of the result)."""
     print("gemm split", kind, M, N, K, flush=True)
     r = rng(M + 3 * N + 7 * K)
