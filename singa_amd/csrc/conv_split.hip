@@ -1,0 +1,523 @@
+// fp32 convolutions of stride 1 with "same" padding (3x3, 5x5), forward and data gradient, on the bfloat16 matrix
+// instructions without giving up fp32 operands: every fp32 value is the exact sum of three bfloat16 values
+//
+//   x = x0 + x1 + x2,   x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)      (8 + 8 + 8 bits of significand)
+//
+// and a product of two of them is the sum of nine exact products, of which the six with weights down to 2^-16 are formed
+// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0); the three left out are below 2^-25 of the product, half an ulp of fp32.
+// v_mfma_f32_32x32x16_bf16 multiplies 16 x as much per cycle as v_mfma_f32_32x32x2_f32, so six of them are 2.67 times as
+// fast, with fp32 accumulators either way.
+//
+//   out[n][c][h][w] = sum_{k,r,s} in[n][k][h + r - o][w + s - o] * Wf[c][k][r][s],   o = (R - 1) / 2
+//
+// forward: Wf = W; data gradient: Wf[c][k][r][s] = W[k][c][R - 1 - r][R - 1 - s].
+//
+// GEMM view: M = output channels, N = consecutive pixels of the flattened (n, h, w) index, reduction = (k, tap) in chunks of
+// 16 input channels.  Per chunk a workgroup stages the input rows its pixels touch, split, as [octet of channels][slab
+// position][part][8 channels]: 48 bytes per position, one operand fragment of a tap is three ds_read_b128 at an offset that
+// is the tap's alone.  A value is fetched and split once per chunk for all R * R taps.  Rows are addressed in a "virtual row"
+// space in which every image owns P + 2 o rows, so a tile may straddle images and the padding is materialised as zeros.
+// The weights are split and laid out in fragment order by a kernel of their own and go from L2 straight to registers, two
+// taps ahead: no LDS, no barrier per tap.
+//
+// 256 threads = 4 wavefronts, two workgroups per CU (at most 80 KB of LDS, 256 registers): while one stages and waits at its
+// barriers the other one's matrix instructions run.
+//
+// Infinities, NaNs and values within half a bfloat16 ulp of the largest float: a part that overflows makes products of
+// infinity with zero, so a result that comes out non-finite is computed again from the fp32 values (`redo`), term by term.
+#include "common.h"
+#include "conv_split.h"
+
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+constexpr int NT = 512, NW = NT / 64, KC = 16;
+constexpr int kOOB = int(0x80000000u);
+constexpr int kMaxSlab = 1024;        // positions of a slab (96 KB; up to 853 of them leave room for a second workgroup)
+constexpr int kPos = 48;              // bytes of a slab position: three parts of eight channels
+constexpr int kFrag = 3 * 1024;       // bytes of a 32-row weight fragment: three parts x 64 lanes x 16 bytes
+
+__device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
+}
+
+__device__ __forceinline__ unsigned pack2(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, bf16x2));
+}
+__device__ __forceinline__ float lo_f(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float hi_f(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// Eight fp32 values -> the three parts of each, packed
+__device__ __forceinline__ void split8(const float (&v)[8], v4u (&part)[3]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = v[2 * i], b = v[2 * i + 1];
+    const unsigned p0 = pack2(a, b);
+    const float ra = a - lo_f(p0), rb = b - hi_f(p0);
+    const unsigned p1 = pack2(ra, rb);
+    part[0][i] = p0, part[1][i] = p1, part[2][i] = pack2(ra - lo_f(p1), rb - hi_f(p1));
+  }
+}
+
+__device__ __forceinline__ v16f mfma(v4u a, v4u b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
+
+struct ScArgs {
+  const float *in;
+  const uint16_t *wt;     // weight fragments [chunk][tap][32-row block][part][lane][8]
+  const float *bias;      // per output channel (NULL: none)
+  float *out;
+  float *partials;        // [workgroup][BM * BN]
+  int accumulate;         // out += result
+  int dgrad;
+  int N, C, K, P, Q;      // in is N x K x P x Q, out N x C x P x Q
+  int cblocks;            // 32-row blocks of the weight fragments
+  int pitch, slab;        // LDS row pitch and positions of the slab (rows * pitch)
+  int total_pix, nchunks;
+  // Workgroups [0, dp_tiles) take one whole tile each; workgroup dp_tiles + r * share + i takes part i of the chunks of tile
+  // dp_tiles + r.  A workgroup's slot of `partials` holds what it leaves for k_conv_split_fixup, or the first half of its sum.
+  int ctiles, dp_tiles, share, halves;
+  int xcd_runs;
+  unsigned in_bytes, wt_bytes;
+};
+
+__device__ __forceinline__ int whole_tile_of(const ScArgs &a, int w) {   // see dgrad3x3.hip: runs of eight tiles per XCD
+  if (!a.xcd_runs) return w;
+  const int x = w & 7, j = w >> 3;
+  return (((j >> 3) << 3) + x) * 8 + (j & 7);
+}
+
+// One result from the fp32 values: channel c at (n, h, w), chunks [ch0, ch1).  Taps in the padding multiply a zero in the
+// forward pass (which makes a NaN of an infinite weight) and do not exist in the data gradient.
+__device__ float redo(const ScArgs &a, int R, int c, int n, int h, int w, int ch0, int ch1) {
+  const int o = (R - 1) / 2, k1 = min(a.K, ch1 * KC);
+  float s = 0.f;
+  for (int k = ch0 * KC; k < k1 && s == s; ++k)   // (a NaN stays one)
+    for (int tap = 0; tap < R * R; ++tap) {
+      const int hh = h + tap / R - o, ww = w + tap % R - o;
+      const bool in = unsigned(hh) < unsigned(a.P) && unsigned(ww) < unsigned(a.Q);
+      if (!in && a.dgrad) continue;
+      const float x = in ? a.in[((size_t(n) * a.K + k) * a.P + hh) * a.Q + ww] : 0.f;
+      const uint16_t *f = a.wt + (size_t((k / KC) * (R * R) + tap) * a.cblocks + c / 32) * (kFrag / 2) +
+                          ((k % KC) / 8 * 32 + c % 32) * 8 + k % 8;
+      const float w0 = lo_f(f[0]), w1 = lo_f(f[512]), w2 = lo_f(f[1024]);
+      s = __builtin_fmaf(x, w0 + w1 + w2, s);
+    }
+  return s;
+}
+
+// GM x (NW / GM) wavefronts, each on WM x WN blocks of 32 x 32; ET: slab elements (octet, position) per thread; R: filter size.
+template <int GM, int WM, int WN, int ET, int R>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_split(ScArgs a) {
+  constexpr int GN = NW / GM, BM = GM * WM * 32, BN = GN * WN * 32, TAPS = R * R, O = (R - 1) / 2;
+  constexpr int AD = 2;                       // weight fragments: this tap's and the next one's
+  extern __shared__ __align__(16) char smem[];
+  const int t = threadIdx.x, lane = t & 63, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave / GN, wn = wave % GN;
+  const int PQ = a.P * a.Q, VH = a.P + 2 * O;
+  const rsrc_t rin = make_rsrc(a.in, a.in_bytes), rwt = make_rsrc(a.wt, a.wt_bytes);
+
+  const int rest = int(blockIdx.x) - a.dp_tiles, part = rest < 0 ? 0 : rest % a.share;
+  const bool whole = rest < 0;
+  const int tile = whole ? whole_tile_of(a, int(blockIdx.x)) : a.dp_tiles + rest / a.share;
+  const int ch_begin = whole ? 0 : part * a.nchunks / a.share, ch_end = whole ? a.nchunks : (part + 1) * a.nchunks / a.share;
+  const int c0 = (tile % a.ctiles) * BM, pix0 = (tile / a.ctiles) * BN;
+  const int n_first = pix0 / PQ, h_first = (pix0 - n_first * PQ) / a.Q;
+  const int vbase = n_first * VH + h_first;   // virtual row of the slab's first row
+
+  // ---- slab loader: element e * NT + t = (octet, position); channel k0 + 8 octet + j is the scalar offset j * PQ away
+  int g0[ET];
+#pragma unroll
+  for (int e = 0; e < ET; ++e) {
+    const int idx = e * NT + t, oct = idx >= a.slab, pos = idx - (oct ? a.slab : 0);
+    const int vr = pos / a.pitch, col = pos - vr * a.pitch, v = vbase + vr, n = v / VH;
+    const int p = v - n * VH - O, q = col - O;
+    const bool ok = idx < 2 * a.slab && n < a.N && unsigned(p) < unsigned(a.P) && unsigned(q) < unsigned(a.Q);
+    g0[e] = ok ? (((n * a.K + oct * 8) * a.P + p) * a.Q + q) * 4 : kOOB;
+  }
+  float st[ET][8];
+  // (no branch: behind one, the waits for the weights would have to count on none of these loads and wait for them too.
+  // Channels from `k_end` on read as zero: those beyond K, and all of them when there is no further chunk.)
+  auto load = [&](int ch, int e, int k_end) {
+    const int k0 = ch * KC, valid = k_end - k0 - (e * NT + t >= a.slab ? 8 : 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      st[e][j] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rin, j < valid ? g0[e] : kOOB, (k0 + j) * PQ * 4, 0));
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int e = 0; e < ET; ++e) {
+      v4u part[3];
+      split8(st[e], part);
+      if (e * NT + t < 2 * a.slab) {
+        v4u *d = reinterpret_cast<v4u *>(smem + (e * NT + t) * kPos);
+        d[0] = part[0], d[1] = part[1], d[2] = part[2];
+      }
+    }
+  };
+
+  // ---- this lane's pixels (columns of the B operand)
+  int boff[WN], pixn[WN];
+#pragma unroll
+  for (int j = 0; j < WN; ++j) {
+    const int pix = min(pix0 + (wn * WN + j) * 32 + l32, a.total_pix - 1);   // (a tail lane computes a pixel it does not store)
+    const int pn = pix / PQ, prem = pix - pn * PQ, ph = prem / a.Q, pw = prem - ph * a.Q;
+    boff[j] = ((pn * VH + ph - vbase) * a.pitch + pw + (lane >> 5) * a.slab) * kPos;
+    pixn[j] = pn;
+  }
+
+  v16f acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  // ---- weights: step q = chunk * TAPS + tap reads cblocks fragments at q * cblocks * kFrag, `step_end` steps in all
+  const int step_end = a.nchunks * TAPS, cb = c0 / 32 + wm * WM;
+  v4u wa[AD][WM][3];
+  auto weights = [&](v4u (&dst)[WM][3], int step) {
+    const int base = min(step, step_end - 1) * a.cblocks;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const int off = (base + min(cb + i, a.cblocks - 1)) * kFrag;   // (rows beyond the last block: computed, not stored)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        dst[i][p] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rwt, lane * 16, off + p * 1024, 0));
+    }
+  };
+
+  // operand fragment of block j at a tap
+  v4u b[WN][3];
+  auto fragment = [&](int tap, int j) {
+    const char *p = smem + boff[j] + tap / R * a.pitch * kPos + tap % R * kPos;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) b[j][k] = *reinterpret_cast<const v4u *>(p + k * 16);
+  };
+
+  // Everything a tap needs is requested before the matrix instructions of an earlier one: weights two taps ahead, the next
+  // chunk's slab an element per tap, a block's fragment while the other block is multiplied.  (The scheduling barriers keep
+  // the compiler from moving the requests down to their uses, which it does to save registers.)
+#pragma unroll
+  for (int e = 0; e < ET; ++e) load(ch_begin, e, a.K);
+  weights(wa[0], ch_begin * TAPS);
+  if (AD > 2) weights(wa[1], ch_begin * TAPS + 1);
+  stage();
+  __syncthreads();
+  // Where few workgroups leave each a long reduction, its first half goes through memory: the error of a sum grows with the
+  // square root of the roundings that its longest chain has, six per tap and chunk.
+  const int half_at = a.halves ? (ch_begin + ch_end) / 2 : ch_end;
+  const int slot = whole || a.halves ? int(blockIdx.x) : rest;
+  const rsrc_t rslot = make_rsrc(a.partials + size_t(slot) * (BM * BN), BM * BN * 4);
+  const int slot_off = ((wm * WM * 32 + 4 * (lane >> 5)) * BN + wn * WN * 32 + l32) * 4;
+  auto keep = [&](float r, int off, int row) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, r), rslot, off, row, 0);
+  };
+  auto slot_row = [](int i, int j, int v) { return ((i * 32 + 8 * (v >> 2) + (v & 3)) * BN + j * 32) * 4; };   // (scalar)
+  for (int ch = ch_begin; ch < ch_end; ++ch) {
+    if (ch == half_at) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            keep(acc[i][j][v], slot_off, slot_row(i, j, v));
+            acc[i][j][v] = 0.f;
+          }
+    }
+    const bool more = ch + 1 < ch_end;
+    if (WN > 1) fragment(0, 0);
+#pragma unroll
+    for (int tap = 0; tap < TAPS; ++tap) {
+      const v4u(&w)[WM][3] = wa[tap % AD];
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        if (j == 0) weights(wa[(tap + AD - 1) % AD], ch * TAPS + tap + AD - 1);
+        if (j == WN - 1 && tap < ET) load(ch + 1, tap, more ? a.K : 0);
+        if (WN == 1) fragment(tap, 0);
+        else if (j + 1 < WN) fragment(tap, j + 1);
+        else if (tap + 1 < TAPS) fragment(tap + 1, 0);
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};   // small products first
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+#pragma unroll
+          for (int i = 0; i < WM; ++i) acc[i][j] = mfma(w[i][PA[k]], b[j][PB[k]], acc[i][j]);
+#pragma unroll
+        for (int k = 0; k < 6 * WM; ++k) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x006, 4, 0);
+          __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (TAPS % AD) {   // (the ring continues one place further)
+      static_assert(TAPS % AD == 0 || TAPS % AD == 1, "ring of the weight fragments");
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const v4u x = wa[0][i][p];
+#pragma unroll
+          for (int d = 0; d + 1 < AD; ++d) wa[d][i][p] = wa[d + 1][i][p];
+          wa[AD - 1][i][p] = x;
+        }
+    }
+    __syncthreads();
+    if (more) {
+      stage();
+      __syncthreads();
+    }
+  }
+
+  // ---- store: this lane holds column l32 and rows 8 (v / 4) + 4 (lane / 32) + v % 4 of every 32 x 32 block
+  const int lhalf = lane >> 5;
+  if (half_at < ch_end) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[i][j][v] += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rslot, slot_off, slot_row(i, j, v), 0));
+  }
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][j][v]);
+  auto put = [&](int m, int col, int n, float r) {   // row, column of the tile
+    const int c = c0 + m, pix = pix0 + col;
+    if (c >= a.C || pix >= a.total_pix) return;
+    float *o = a.out + (size_t(n) * a.C + c) * PQ + (pix - n * PQ);
+    if (a.bias) r += a.bias[c];
+    *o = a.accumulate ? *o + r : r;
+  };
+  const bool redone = __any(bad);
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      unsigned mask = 0;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = (wm * WM + i) * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3), col = (wn * WN + j) * 32 + l32;
+        if (redone && !finite(acc[i][j][v])) mask |= 1u << v;
+        else if (whole) put(m, col, pixn[j], acc[i][j][v]);
+        else keep(acc[i][j][v], slot_off, slot_row(i, j, v));
+      }
+      if (redone)
+        for (; mask; mask &= mask - 1) {
+          const int v = __builtin_ctz(mask);
+          const int m = (wm * WM + i) * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3), col = (wn * WN + j) * 32 + l32;
+          if (c0 + m >= a.C || pix0 + col >= a.total_pix) continue;
+          const int rem = pix0 + col - pixn[j] * PQ, h = rem / a.Q;
+          const float r = redo(a, R, c0 + m, pixn[j], h, rem - h * a.Q, ch_begin, ch_end);
+          if (whole) put(m, col, pixn[j], r);
+          else keep(r, (m * BN + col) * 4, 0);
+        }
+    }
+}
+
+// Sums the parts of the tiles that several workgroups shared, in ascending chunk order: the result does not depend on timing
+__global__ __launch_bounds__(256) void k_conv_split_fixup(ScArgs a, int BM, int BN) {
+  const int r = blockIdx.x, TPR = BN / 4;
+  const int tile = a.dp_tiles + r, c0 = (tile % a.ctiles) * BM, pix0 = (tile / a.ctiles) * BN, PQ = a.P * a.Q;
+  const int m = int(blockIdx.y * 256 + threadIdx.x) / TPR, col = int(threadIdx.x) % TPR * 4, c = c0 + m;
+  if (c >= a.C) return;
+  const float *p = a.partials + (size_t(r) * a.share + (a.halves ? a.dp_tiles : 0)) * BM * BN + m * BN + col;
+  v4f s = *reinterpret_cast<const v4f *>(p);
+  for (int i = 1; i < a.share; ++i) s += *reinterpret_cast<const v4f *>(p + size_t(i) * BM * BN);
+  const float bb = a.bias ? a.bias[c] : 0.f;
+  int pix = pix0 + col, pn = pix / PQ, prem = pix - pn * PQ;
+  if ((PQ & 3) == 0 && pix + 3 < a.total_pix) {   // the four pixels lie in one image, 16-byte aligned
+    v4f *o = reinterpret_cast<v4f *>(a.out + (size_t(pn) * a.C + c) * PQ + prem);
+    *o = a.accumulate ? *o + (s + bb) : s + bb;
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j, ++pix) {
+    if (pix >= a.total_pix) break;
+    float *o = a.out + (size_t(pn) * a.C + c) * PQ + prem;
+    *o = a.accumulate ? *o + (s[j] + bb) : s[j] + bb;
+    if (++prem == PQ) prem = 0, ++pn;
+  }
+}
+
+struct ScPlan {
+  bool ok;
+  int r, gm, wm, wn, et, bm, bn, pitch, rows, slab, nchunks, cblocks;
+  int ctiles, tiles, dp_tiles, share, wgs;
+  bool halves;
+};
+
+ScPlan plan(const sgh_conv_geom *g) {
+  ScPlan p{};
+  if ((g->R != 3 && g->R != 5) || g->S != g->R || g->stride_h != 1 || g->stride_w != 1) return p;
+  const int o = (g->R - 1) / 2;
+  if (g->pad_h != o || g->pad_w != o || g->C < 16 || g->K < 8) return p;
+  const size_t lim = size_t(1) << 31;
+  if (size_t(g->N) * g->K * g->P * g->Q * 4 >= lim || size_t(g->N) * g->C * g->P * g->Q * 4 >= lim) return p;
+  if (size_t(g->N) * (g->P + 2 * o) >= lim / 64) return p;
+  p.r = g->R;
+  p.pitch = g->Q + 2 * o;
+  p.nchunks = (g->K + KC - 1) / KC;
+  p.cblocks = (g->C + 31) / 32;
+  if (size_t(p.nchunks) * p.r * p.r * p.cblocks * kFrag >= lim) return p;
+  const int cus = sgh_num_cus();
+  const long pixels = long(g->N) * g->P * g->Q;
+  // Tile: 128 x 128, 64 x 256, 64 x 128 or 32 x 256 (a wavefront holds 32 x 64 of the first two, 32 x 32 of the others), the
+  // least rows counting those beyond C, with 32-row tiles a quarter dearer.  64 rows take 256 pixels from two fifths more
+  // tiles than CUs on; below, tiles of half the size leave fewer CUs idle (64 channels of 56 x 56: N = 64 94 against 105 us,
+  // N = 32 58 against 57, N = 8 32 against 29; 96 channels of 20 x 20: 51 on 32 rows, 57 on 128; 200 channels: 42 on 128, 54 on 32).
+  auto rows_of = [&](int bm) { return (g->C + bm - 1) / bm * bm; };
+  const int r128 = rows_of(128), r64 = rows_of(64), r32 = rows_of(32);
+  auto take = [&](int gm, int wn) {
+    p.gm = gm, p.wm = 1, p.wn = wn, p.bm = gm * 32, p.bn = NW / gm * wn * 32;
+    // virtual rows a tile can touch: its pixel rows, the halo rows, and the zero rows of every image boundary it crosses
+    p.rows = (p.bn + g->Q - 2) / g->Q + 1 + 2 * o + 2 * o * ((p.bn - 1) / (g->P * g->Q) + 1);
+    return long(p.rows) * p.pitch <= kMaxSlab;
+  };
+  bool fits = false;
+  // (too few chunks to give every CU one: small tiles.  204 filters over 14 channels, 10 x 2 tiles: 16.5 -> 13 us)
+  if (p.r == 3 && r128 == r64 && 4 * r128 <= 5 * r32 && r128 / 128 * ((pixels + 127) / 128) * p.nchunks >= cus) fits = take(4, 2);
+  if (!fits && 4 * r64 <= 5 * r32)
+    fits = (5 * (r64 / 64) * ((pixels + 255) / 256) >= 7 * cus && take(2, 2)) || take(2, 1);
+  if (!fits && !take(1, 1)) return p;
+  p.slab = p.rows * p.pitch;
+  p.et = (2 * p.slab + NT - 1) / NT;
+  p.ctiles = (g->C + p.bm - 1) / p.bm;
+  const long tiles = long(p.ctiles) * ((pixels + p.bn - 1) / p.bn);
+  if (tiles >= (long(1) << 30)) return p;
+  p.tiles = int(tiles);
+  // Whole multiples of the CU count of tiles are one workgroup's each; the chunks of a remaining tile are dealt evenly to as
+  // many workgroups as leave every CU at most one of them.  (Two per CU, or runs of chunks that cross tiles: more partial
+  // tiles to write and sum, 64 images of 512 channels 7 x 7 93 against 92 / 101 us, of 128 channels 28 x 28 91 against 100 / 99.)
+  p.dp_tiles = int(tiles / cus * cus);
+  const int rest = p.tiles - p.dp_tiles;
+  p.share = rest ? cus / rest : 1;
+  if (p.share > p.nchunks) p.share = p.nchunks;
+  if (p.share <= 1) p.share = 1, p.dp_tiles = p.tiles;
+  p.wgs = p.dp_tiles + (p.tiles - p.dp_tiles) * p.share;
+  // (both halves through memory: 256 channels of 14 x 14, N = 64, error against float64 7.2e-7 -> 5.1e-7 of the result; with
+  // more workgroups than this the fp32 matrix instructions sum in one chain as well, and theirs is the larger error)
+  p.halves = p.wgs <= 2 * cus && p.nchunks / p.share >= 3;
+  p.ok = true;
+  return p;
+}
+
+template <int GM, int WM, int WN, int ET, int R>
+int launch(const ScArgs &a, const ScPlan &p, hipStream_t s) {
+  auto kern = k_conv_split<GM, WM, WN, ET, R>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
+        hipSuccess)
+      return SGH_EUNSUPPORTED;
+    attr_set = true;
+  }
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(p.wgs)), dim3(NT), size_t(p.slab) * 2 * kPos, s, a);
+  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+}
+
+inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Weight fragments [chunk][tap][32-row block][part][lane][8]: one workgroup per (chunk, block).  Destination rows c are the
+// output channels, k the reduction; the source is W[c][k][tap] (forward) or W[k][c][last - tap] (data gradient).
+__global__ __launch_bounds__(256) void k_conv_split_weights(const float *__restrict__ W, uint16_t *__restrict__ wt, int C, int K,
+                                                           int RS, int cblocks, int dgrad, int taps) {
+  __shared__ float buf[kSplitWeightLds];
+  sgh_conv_split_weights_block(W, wt, C, K, RS, cblocks, dgrad, int(blockIdx.x), taps, buf);
+}
+
+}  // namespace
+
+bool sgh_conv_split_supported(const sgh_conv_geom *g) { return plan(g).ok && !sgh_env().conv_split_off; }
+
+size_t sgh_conv_split_weight_bytes(const sgh_conv_geom *g) {
+  const ScPlan p = plan(g);
+  return p.ok ? size_t(p.nchunks) * p.r * p.r * p.cblocks * kFrag : 0;
+}
+
+size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g) {
+  const ScPlan p = plan(g);
+  const int slots = p.halves ? p.wgs : p.wgs - p.dp_tiles;
+  return p.ok ? align256(sgh_conv_split_weight_bytes(g)) + size_t(slots) * p.bm * p.bn * sizeof(float) : 0;
+}
+
+int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps) {
+  const ScPlan p = plan(g);
+  const int pairs = p.nchunks * p.cblocks;
+  *cblocks = p.cblocks;
+  *taps = pairs >= sgh_num_cus() ? kSplitTaps : kSplitTapsFew;
+  return p.ok ? pairs * ((g->R * g->S + *taps - 1) / *taps) : 0;
+}
+
+int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspace, bool dgrad, hipStream_t s) {
+  int cblocks, taps;
+  const int blocks = sgh_conv_split_weight_blocks(g, &cblocks, &taps);
+  if (!blocks) return SGH_EUNSUPPORTED;
+  hipLaunchKernelGGL(k_conv_split_weights, dim3(unsigned(blocks)), dim3(256), 0, s, W, static_cast<uint16_t *>(workspace), g->C,
+                     g->K, g->R * g->S, cblocks, dgrad ? 1 : 0, taps);
+  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+}
+
+int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, float *out, void *workspace, hipStream_t s, const char *tag,
+                       bool dgrad, const float *bias, bool accumulate) {
+  const ScPlan p = plan(g);
+  if (!p.ok) return SGH_EUNSUPPORTED;
+  ScArgs a;
+  a.in = in;
+  a.wt = static_cast<const uint16_t *>(workspace);
+  a.bias = bias;
+  a.out = out;
+  a.partials = reinterpret_cast<float *>(static_cast<char *>(workspace) + align256(sgh_conv_split_weight_bytes(g)));
+  a.accumulate = accumulate ? 1 : 0;
+  a.dgrad = dgrad ? 1 : 0;
+  a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
+  a.cblocks = p.cblocks, a.pitch = p.pitch, a.slab = p.slab;
+  a.total_pix = g->N * g->P * g->Q, a.nchunks = p.nchunks;
+  a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share, a.halves = p.halves;
+  a.xcd_runs = p.dp_tiles % 64 == 0 && !sgh_env().conv_xcd_off;
+  a.in_bytes = unsigned(size_t(g->N) * g->K * g->P * g->Q * 4);
+  a.wt_bytes = unsigned(sgh_conv_split_weight_bytes(g));
+  int rc = SGH_EUNSUPPORTED;
+  sgh_prof_kernel_begin(tag, 2.0 * g->N * g->K * g->P * g->Q * g->C * p.r * p.r);
+#define SC_CASE(GM_, WM_, WN_, ET_, R_) \
+  if (p.gm == GM_ && p.wm == WM_ && p.wn == WN_ && p.et == ET_ && p.r == R_) rc = launch<GM_, WM_, WN_, ET_, R_>(a, p, s);
+#define SC_CASES(GM_, WM_, WN_, R_) \
+  SC_CASE(GM_, WM_, WN_, 1, R_) SC_CASE(GM_, WM_, WN_, 2, R_) SC_CASE(GM_, WM_, WN_, 3, R_) SC_CASE(GM_, WM_, WN_, 4, R_)
+  SC_CASES(4, 1, 2, 3)
+  SC_CASES(2, 1, 2, 3)
+  SC_CASES(2, 1, 1, 3)
+  SC_CASES(1, 1, 1, 3)
+  SC_CASES(2, 1, 2, 5)
+  SC_CASES(2, 1, 1, 5)
+  SC_CASES(1, 1, 1, 5)
+#undef SC_CASES
+#undef SC_CASE
+  sgh_prof_kernel_end(s);
+  if (rc != SGH_OK) return rc;
+  if (p.share > 1) {
+    hipLaunchKernelGGL(k_conv_split_fixup, dim3(unsigned(p.tiles - p.dp_tiles), unsigned(p.bm * p.bn / 1024)), dim3(256), 0, s, a,
+                       p.bm, p.bn);
+    if (hipGetLastError() != hipSuccess) return SGH_EINVAL;
+  }
+  return SGH_OK;
+}

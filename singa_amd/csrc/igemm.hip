@@ -25,6 +25,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "conv_split.h"
 
 namespace {
 
@@ -858,6 +859,20 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
   return sgh_dgrad3x3_forward_pays(gt);
 }
 
+// The same problem for the split kernel (conv_split.hip), where that one takes it
+inline bool fwd_as_split(const sgh_conv_geom *g, sgh_conv_geom *gt) {
+  if (g->stride_h != 1 || g->stride_w != 1) return false;
+  *gt = *g;
+  gt->C = g->K;
+  gt->K = g->C;
+  return sgh_conv_split_supported(gt);
+}
+
+inline bool dgrad_as_split(const sgh_conv_geom *g) {
+  const DgradPath path = dgrad_path(g);
+  return path != kDgradFewC && path != kDgradPointwise && path != kDgradColumns && sgh_conv_split_supported(g);
+}
+
 }  // namespace
 
 // ---- grouped convolution (cudnnSetConvolutionGroupCount in the reference, src/model/operation/convolution.cc
@@ -990,7 +1005,8 @@ int conv_grouped_f32(const sgh_conv_geom *g, int which, const float *a, const fl
 
 }  // namespace
 
-size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
+// without the split kernel, which runs where the workspace holds its weights and partial sums as well
+static size_t plain_workspace_bytes(const sgh_conv_geom *g, int which) {
   if (!conv_ok(g)) return 0;
   if (g->groups > 1) {
     if (which < 0 || which > 2) return 0;
@@ -1027,9 +1043,19 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   }
 }
 
+size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
+  const size_t plain = plain_workspace_bytes(g, which);
+  if (!conv_ok(g) || g->groups > 1) return plain;
+  sgh_conv_geom gt;
+  size_t split = 0;
+  if (which == SGH_CONV_FWD && fwd_as_split(g, &gt)) split = sgh_conv_split_workspace_bytes(&gt);
+  if (which == SGH_CONV_DGRAD && dgrad_as_split(g)) split = sgh_conv_split_workspace_bytes(g);
+  return split > plain ? split : plain;
+}
+
 // The partial sums of the shared-tile kernel are the part of a workspace that a pass can do without
 static size_t least_bytes_f32(const sgh_conv_geom *g, int which) {
-  const size_t full = sgh_conv_workspace_bytes(g, which);
+  const size_t full = plain_workspace_bytes(g, which);
   if (full == 0) return 0;
   sgh_conv_geom gt;
   if (which == SGH_CONV_FWD && fwd_as_dgrad(g, &gt)) {
@@ -1040,11 +1066,16 @@ static size_t least_bytes_f32(const sgh_conv_geom *g, int which) {
   return full;
 }
 
+// Which of the two layouts of the weights a data gradient with this workspace works on
+static bool dgrad_splits(const sgh_conv_geom *g, size_t ws_bytes) {
+  return dgrad_as_split(g) && ws_bytes >= sgh_conv_split_workspace_bytes(g);
+}
+
 // `prelaid`: the workspace already holds this layer's re-laid weights (sgh_conv_dgrad_prepare_multi)
 static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, float *dx, void *workspace,
                       size_t ws_bytes, void *stream, bool accumulate, bool prelaid) {
   if (!conv_ok(g) || !dy || !W || !dx) return SGH_EINVAL;
-  const size_t full = sgh_conv_workspace_bytes(g, SGH_CONV_DGRAD), least = least_bytes_f32(g, SGH_CONV_DGRAD);
+  const size_t full = plain_workspace_bytes(g, SGH_CONV_DGRAD), least = least_bytes_f32(g, SGH_CONV_DGRAD);
   if (least && (!workspace || ws_bytes < least)) return SGH_EWORKSPACE;
   hipStream_t s = sgh_stream_of(stream);
   const int RS = g->R * g->S, KP = round_up(g->K, BK);
@@ -1099,6 +1130,9 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
       if (blocks > cap) blocks = cap;
       hipLaunchKernelGGL(k_col2im_gather, dim3(int(blocks)), dim3(NT), 0, s, dcol, dx, to_g(g), total);
     }
+  } else if (dgrad_splits(g, ws_bytes)) {
+    if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
+    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
   } else if (path == kDgradTile3x3) {
     float *Wt = static_cast<float *>(workspace);
     const long total = long(RS) * KP * g->C;
@@ -1192,9 +1226,10 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
 }
 
 // The note of a prepare call is read once: whether it held or not, this pass leaves none behind.
-static bool take_prelaid(sgh_conv_geom *g, int dtype, const void *W, const void *workspace) {
+static bool take_prelaid(sgh_conv_geom *g, int dtype, const void *W, const void *workspace, size_t ws_bytes) {
   if (!g) return false;
-  const bool ok = sgh_prelaid_valid(g, dtype, W, workspace);
+  bool ok = sgh_prelaid_valid(g, dtype, W, workspace);
+  if (ok && dtype == 0) ok = dgrad_splits(g, g->prelaid_ws_bytes) == dgrad_splits(g, ws_bytes);
   sgh_prelaid_clear(g);
   return ok;
 }
@@ -1203,7 +1238,7 @@ int sgh_conv_dgrad_f32(sgh_conv_geom *g, const float *dy, const float *W, float 
                        size_t ws_bytes, void *stream) {
   if (g && conv_ok(g) && g->groups > 1)
     return conv_grouped_f32(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream);
-  const bool prelaid = take_prelaid(g, 0, W, workspace);
+  const bool prelaid = take_prelaid(g, 0, W, workspace, ws_bytes);
   return conv_dgrad(g, dy, W, dx, workspace, ws_bytes, stream, false, prelaid);
 }
 
@@ -1221,6 +1256,7 @@ struct RelayoutTable {
     const void *W;
     void *Wt;
     int K, C, RS, A, B;   // destination [tap][A][B]: fp32 A = KP (k), B = C;  16-bit A = CP (c), B = KP (k)
+    int cblocks, taps;    // cblocks > 0: the fragments of conv_split.hip instead
   } it[kMaxRelayouts];
 };
 
@@ -1231,8 +1267,8 @@ constexpr int kRelayoutPerBlock = NT * 8, kRelayoutTile = 32, kRelayoutMaxTaps =
 extern "C++" {
 template <class T>
 __device__ __forceinline__ void relayout_tile(const T *__restrict__ W, T *__restrict__ Wt, int K, int C, int RS, int A,
-                                              int B, bool k_fastest, int tile) {
-  __shared__ T lds[kRelayoutTile][kRelayoutTile * kRelayoutMaxTaps + 1];
+                                              int B, bool k_fastest, int tile,
+                                              T (&lds)[kRelayoutTile][kRelayoutTile * kRelayoutMaxTaps + 1]) {
   // destination [tap][A][B]; k_fastest: (A, B) = (c, k), else (k, c)
   const int kdim = k_fastest ? B : A, cdim = k_fastest ? A : B;
   const int ctiles = (cdim + kRelayoutTile - 1) / kRelayoutTile;
@@ -1285,8 +1321,16 @@ __global__ __launch_bounds__(NT) void k_weight_relayout_multi(const RelayoutTabl
   const int blk = int(blockIdx.x) - t.block0[lo];
   const T *W = static_cast<const T *>(t.it[lo].W);
   T *Wt = static_cast<T *>(t.it[lo].Wt);
+  __shared__ T lds[kRelayoutTile][kRelayoutTile * kRelayoutMaxTaps + 1];
+  if constexpr (sizeof(T) == 4) {
+    static_assert(sizeof(lds) >= kSplitWeightLds * sizeof(float), "room for the fragments of a block");
+    if (t.it[lo].cblocks) {
+      sgh_conv_split_weights_block(W, reinterpret_cast<uint16_t *>(Wt), C, K, RS, t.it[lo].cblocks, 1, blk, t.it[lo].taps, &lds[0][0]);
+      return;
+    }
+  }
   if (RS <= kRelayoutMaxTaps) {
-    relayout_tile<T>(W, Wt, K, C, RS, A, B, k_fastest, blk);
+    relayout_tile<T>(W, Wt, K, C, RS, A, B, k_fastest, blk, lds);
     return;
   }
   // large filters: element by element
@@ -1337,7 +1381,7 @@ int sgh_conv_dgrad_prepare_multi(const sgh_conv_prepare_item *items, int count, 
     size_t need;
     if (dtype == 0) {
       const DgradPath path = dgrad_path(g);
-      if (path != kDgradTile3x3 && path != kDgradGather) continue;   // the other kernels read W as it is or re-lay it their own way
+      if (path != kDgradTile3x3 && path != kDgradGather && !dgrad_splits(g, items[i].ws_bytes)) continue;   // the other kernels read W as it is or re-lay it their own way
       it.A = round_up(g->K, BK), it.B = g->C;
       need = least_bytes_f32(g, SGH_CONV_DGRAD);
     } else {
@@ -1346,7 +1390,9 @@ int sgh_conv_dgrad_prepare_multi(const sgh_conv_prepare_item *items, int count, 
     }
     if (!items[i].workspace || items[i].ws_bytes < need) return SGH_EWORKSPACE;
     const long total = long(it.RS) * it.A * it.B;
-    const long blocks = it.RS <= kRelayoutMaxTaps
+    const bool split = dtype == 0 && dgrad_splits(g, items[i].ws_bytes);
+    const long blocks = split ? sgh_conv_split_weight_blocks(g, &it.cblocks, &it.taps)
+                        : it.RS <= kRelayoutMaxTaps
                             ? long((it.A + kRelayoutTile - 1) / kRelayoutTile) * ((it.B + kRelayoutTile - 1) / kRelayoutTile)
                             : (total + kRelayoutPerBlock - 1) / kRelayoutPerBlock;
     if (t.count == kMaxRelayouts || long(t.block0[t.count]) + blocks >= (long(1) << 30)) {
@@ -1369,7 +1415,7 @@ int sgh_conv_dgrad_acc_supported(const sgh_conv_geom *g) {
 int sgh_conv_dgrad_acc_f32(sgh_conv_geom *g, const float *dy, const float *W, float *dx, void *workspace,
                            size_t ws_bytes, void *stream) {
   if (g && conv_ok(g) && !sgh_conv_dgrad_acc_supported(g)) return SGH_EUNSUPPORTED;   // (the note stays for the fallback call)
-  const bool prelaid = take_prelaid(g, 0, W, workspace);
+  const bool prelaid = take_prelaid(g, 0, W, workspace, ws_bytes);
   return conv_dgrad(g, dy, W, dx, workspace, ws_bytes, stream, true, prelaid);
 }
 
@@ -1378,7 +1424,7 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
   if (!conv_ok(g) || !x || !W || !y) return SGH_EINVAL;
   if (g->groups > 1) return conv_grouped_f32(g, SGH_CONV_FWD, x, W, bias, y, workspace, ws_bytes, stream);
   sgh_prelaid_clear_if_overlap(g, workspace, ws_bytes);
-  const size_t full = sgh_conv_workspace_bytes(g, SGH_CONV_FWD);
+  const size_t full = plain_workspace_bytes(g, SGH_CONV_FWD);
   if (!workspace || ws_bytes < least_bytes_f32(g, SGH_CONV_FWD)) return SGH_EWORKSPACE;
   hipStream_t s = sgh_stream_of(stream);
   float *Wt = static_cast<float *>(workspace);
@@ -1392,6 +1438,12 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
     }
   }
   sgh_conv_geom gt;
+  if (fwd_as_split(g, &gt) && ws_bytes >= sgh_conv_split_workspace_bytes(&gt)) {
+    int rcs = sgh_conv_split_weights(&gt, W, workspace, false, s);
+    if (rcs == SGH_OK) rcs = sgh_conv_split_run(&gt, x, y, workspace, s, "conv_fwd/k_conv_split", false, bias, false);
+    sgh_prof_stop(s);
+    return rcs;
+  }
   if (fwd_as_dgrad(g, &gt)) {
     // stride 1 with "same" padding, 3x3 or 5x5: the shared-tile kernel on the channel-swapped problem with reversed taps
     const long total = long(RS) * CP * g->K;
@@ -1613,7 +1665,7 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
                                   });
   }
   bool prelaid = false;
-  if (which == SGH_CONV_DGRAD) prelaid = take_prelaid(g, in == sgh_cast_bf16_to_f32 ? 2 : 1, b, workspace);
+  if (which == SGH_CONV_DGRAD) prelaid = take_prelaid(g, in == sgh_cast_bf16_to_f32 ? 2 : 1, b, workspace, ws_bytes);
   else sgh_prelaid_clear_if_overlap(g, workspace, ws_bytes);
   // the gradients and the forward pass (strides 1 and 2) run on the 16-bit matrix instructions where
   // conv16.hip covers the geometry; everything else computes in fp32 on widened copies

@@ -1086,3 +1086,69 @@ def test_bn_slice_counts_around_the_xcds(singa, dev, shape):
     want = S(gamma * i) * (d64 - S(d64.sum((0, 2, 3))) / n - xh * S((d64 * xh).sum((0, 2, 3))) / n)
     assert nl2(dx.to_numpy(), want) < 1e-6
     assert nl2(dg.to_numpy(), (d64 * xh).sum((0, 2, 3))) < 1e-5 and nl2(db.to_numpy(), d64.sum((0, 2, 3))) < 1e-5
+
+
+# sizes at the edges of the split-operand kernel (conv_split.hip): channel and pixel remainders of its four tiles, reductions of
+# part of a chunk, tiles shared between workgroups, halves of a sum through memory, rows too wide for its slab
+SPLIT_CASES = [
+    # n, c, h, w, k, r
+    (2, 8, 7, 9, 16, 3), (3, 17, 6, 5, 33, 3), (1, 16, 16, 16, 32, 3), (5, 24, 13, 11, 31, 3),     # 32-row tiles
+    (4, 33, 16, 16, 64, 3), (2, 64, 8, 16, 63, 3), (9, 40, 17, 19, 64, 3), (90, 64, 40, 40, 64, 3),   # 64 rows, 128 and 256 pixels
+    (2, 48, 9, 8, 128, 3), (3, 129, 14, 14, 127, 3), (1, 512, 7, 7, 256, 3), (33, 128, 28, 28, 129, 3),   # 128 rows, shared, halves
+    (2, 96, 20, 20, 96, 3), (1, 20, 3, 300, 40, 3), (1, 32, 2, 112, 64, 3), (7, 32, 1, 4, 64, 3),   # planes of extreme shape
+    (2, 9, 12, 10, 32, 5), (3, 32, 16, 16, 64, 5), (1, 70, 5, 4, 100, 5), (40, 32, 16, 16, 33, 5),
+]
+
+
+def split_reference(x, w, b, dy, r):
+    import torch
+    import torch.nn.functional as F
+    t = lambda a: torch.from_numpy(np.asarray(a, np.float64))
+    y = F.conv2d(t(x), t(w), t(b), padding=r // 2)
+    dx = F.conv_transpose2d(t(dy), t(w), padding=r // 2)
+    return y.numpy(), dx.numpy()
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r", SPLIT_CASES)
+def test_conv_split_operands(singa, dev, n, c, h, w, k, r):
+    """Forward and data gradient of stride 1 and "same" padding against float64.  Bounds: an fp32 sum of `terms` products is
+    off by at most terms * 2^-23 of the sum of their magnitudes in any order (six matrix instructions per 16 channels and tap
+    round less often than once per term), and by about sqrt(terms) * 2^-24 of the result in the 2-norm; twice that is allowed."""
+    rg = rng(n * 7 + c + k)
+    x, W, b, dy = randn(rg, n, c, h, w), randn(rg, k, c, r, r), randn(rg, k), randn(rg, n, k, h, w)
+    want = split_reference(x, W, b, dy, r)
+    size = split_reference(np.abs(x), np.abs(W), np.abs(b), np.abs(dy), r)
+    xd, wd, bd, dyd = (singa.from_numpy(a, dev) for a in (x, W, b, dy))
+    hd = singa.CudnnConvHandle(xd, (r, r), (1, 1), (r // 2, r // 2), c, k, True)
+    got = (singa.GpuConvForward(xd, wd, bd, hd).to_numpy(), singa.GpuConvBackwardx(dyd, wd, xd, hd).to_numpy())
+    for g, ref, mag, terms in zip(got, want, size, (c * r * r + 1, k * r * r)):
+        assert np.all(np.abs(g - ref) <= terms * 2.0 ** -23 * mag)
+        assert nl2(g, ref) < 2 * (terms + 16) ** 0.5 * 2.0 ** -24
+    singa.GpuConvPrepareBackward([(wd, hd)])
+    assert_bit_equal(singa.GpuConvBackwardx(dyd, wd, xd, hd).to_numpy(), got[1], "prepared weights")
+
+
+@pytest.mark.parametrize("where", ["x", "w"])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.4e38])
+@pytest.mark.parametrize("n,c,h,w,k", [(2, 24, 9, 10, 40), (1, 300, 6, 6, 130), (30, 64, 20, 20, 64)])
+def test_conv_split_operands_non_finite(singa, dev, n, c, h, w, k, where, bad):
+    """Infinities, NaNs and values whose bfloat16 rounding is infinite reach exactly the results that their products reach."""
+    rg = rng(5)
+    x, W, b, dy = randn(rg, n, c, h, w), randn(rg, k, c, 3, 3) * np.float32(0.01), randn(rg, k), randn(rg, n, k, h, w)
+    if where == "x":
+        x[-1, c // 2, 0, w - 1] = bad
+        dy[0, k - 1, h // 2, 1] = bad
+    else:
+        W[k - 1, c // 3, 1, 2] = bad
+        if bad == np.float32(3.4e38):   # (products stay in range)
+            x *= np.float32(0.01)
+            dy *= np.float32(0.01)
+    with np.errstate(all="ignore"):
+        want = [a.astype(np.float32) for a in split_reference(x, W, b, dy, 3)]
+    xd, wd, bd, dyd = (singa.from_numpy(a, dev) for a in (x, W, b, dy))
+    hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, True)
+    got = (singa.GpuConvForward(xd, wd, bd, hd).to_numpy(), singa.GpuConvBackwardx(dyd, wd, xd, hd).to_numpy())
+    for g, ref in zip(got, want):
+        assert np.array_equal(np.isnan(g), np.isnan(ref)) and np.array_equal(np.isposinf(g), np.isposinf(ref))
+        fin = np.isfinite(ref) & np.isfinite(g)
+        np.testing.assert_allclose(g[fin], ref[fin], rtol=1e-4, atol=1e-4)
