@@ -1114,6 +1114,9 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
       rc = launch_igemm<64, 64, DenseLoader<64, false>, PixelGatherLoader<64, false>, DilateStore, false, false, false, 2, 4>(
           la, lb, st, g->C, Ncols, g->K, 1, chunks, s, "conv_dgrad/k_igemm", conv_flops(g));
     }
+  } else if (dgrad_splits(g, ws_bytes)) {
+    if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
+    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
   } else if (path == kDgradColumns) {
     float *dcol = static_cast<float *>(workspace);
     const int CRS = g->C * RS, Ncols = g->N * g->P * g->Q;
@@ -1130,9 +1133,6 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
       if (blocks > cap) blocks = cap;
       hipLaunchKernelGGL(k_col2im_gather, dim3(int(blocks)), dim3(NT), 0, s, dcol, dx, to_g(g), total);
     }
-  } else if (dgrad_splits(g, ws_bytes)) {
-    if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
-    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
   } else if (path == kDgradTile3x3) {
     float *Wt = static_cast<float *>(workspace);
     const long total = long(RS) * KP * g->C;

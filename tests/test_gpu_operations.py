@@ -1095,6 +1095,7 @@ SPLIT_CASES = [
     (2, 8, 7, 9, 16, 3), (3, 17, 6, 5, 33, 3), (1, 16, 16, 16, 32, 3), (5, 24, 13, 11, 31, 3),     # 32-row tiles
     (4, 33, 16, 16, 64, 3), (2, 64, 8, 16, 63, 3), (9, 40, 17, 19, 64, 3), (90, 64, 40, 40, 64, 3),   # 64 rows, 128 and 256 pixels
     (2, 48, 9, 8, 128, 3), (3, 129, 14, 14, 127, 3), (1, 512, 7, 7, 256, 3), (33, 128, 28, 28, 129, 3),   # 128 rows, shared, halves
+    (5, 30, 13, 12, 5, 3), (40, 100, 16, 18, 1, 3), (6, 24, 21, 18, 4, 5),   # fewer filters than a tile has rows
     (2, 96, 20, 20, 96, 3), (1, 20, 3, 300, 40, 3), (1, 32, 2, 112, 64, 3), (7, 32, 1, 4, 64, 3),   # planes of extreme shape
     (2, 9, 12, 10, 32, 5), (3, 32, 16, 16, 64, 5), (1, 70, 5, 4, 100, 5), (40, 32, 16, 16, 33, 5),
 ]
