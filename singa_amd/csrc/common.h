@@ -144,6 +144,11 @@ size_t sgh_wgrad3x3_workspace_bytes(const sgh_conv_geom *g);
 int sgh_wgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace,
                      size_t ws_bytes, hipStream_t s);
 
+// fp32 3x3 stride-1 pad-1 weight gradient on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
+// take; the caller checks that the workspace has them.
+size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);
+int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s);
+
 // Weight gradient for few input channels and a large filter (C*R*S in 65..160: the 7x7 stem),
 // wgrad_fewc.hip.  Same conventions as the 3x3 kernel above.
 size_t sgh_wgrad_fewc_workspace_bytes(const sgh_conv_geom *g);

@@ -1050,6 +1050,7 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   size_t split = 0;
   if (which == SGH_CONV_FWD && fwd_as_split(g, &gt)) split = sgh_conv_split_workspace_bytes(&gt);
   if (which == SGH_CONV_DGRAD && dgrad_as_split(g)) split = sgh_conv_split_workspace_bytes(g);
+  if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g);
   return split > plain ? split : plain;
 }
 
@@ -1497,6 +1498,12 @@ static int bgrad_launch(const sgh_conv_geom *g, const float *dy, float *db, hipS
   return sgh_conv_bgrad_run(g, dy, db, 0, s);
 }
 
+// The octet kernel runs where the workspace holds its partial images
+static bool wgrad_by_octets(const sgh_conv_geom *g, const void *workspace, size_t ws_bytes) {
+  const size_t need = sgh_wgrad_oct_workspace_bytes(g);
+  return need && workspace && ws_bytes >= need;
+}
+
 // `db` (may be null): the bias gradient as well.  In the generic kernel it rides along as one more column
 // of the x operand (a column of ones) whenever the last column tile has a spare column; the shared-tile
 // and few-channel kernels are followed by the reduction kernel of sgh_conv_bgrad_f32.
@@ -1508,6 +1515,12 @@ static int conv_wgrad(sgh_conv_geom *g, const float *dy, const float *x, float *
     return rc == SGH_OK && db ? bgrad_launch(g, dy, db, sgh_stream_of(stream)) : rc;
   }
   sgh_prelaid_clear_if_overlap(g, workspace, ws_bytes);
+  if (wgrad_by_octets(g, workspace, ws_bytes)) {
+    sgh_prof_start("conv_wgrad_op", conv_flops(g), sgh_stream_of(stream));
+    const int rco = sgh_wgrad_oct_run(g, dy, x, dW, workspace, sgh_stream_of(stream));
+    sgh_prof_stop(sgh_stream_of(stream));
+    return rco == SGH_OK && db ? bgrad_launch(g, dy, db, sgh_stream_of(stream)) : rco;
+  }
   if (sgh_wgrad3x3_workspace_bytes(g)) {  // 3x3, stride 1 or 2: shared-input-tile kernel
     sgh_prof_start("conv_wgrad_op", conv_flops(g), sgh_stream_of(stream));
     const int rc3 = sgh_wgrad3x3_run(g, dy, x, dW, workspace, ws_bytes, sgh_stream_of(stream));
@@ -1527,7 +1540,7 @@ static int conv_wgrad(sgh_conv_geom *g, const float *dy, const float *x, float *
     return rcp == SGH_OK && db ? bgrad_launch(g, dy, db, sgh_stream_of(stream)) : rcp;
   }
   const WgradPlan p = plan_wgrad(g);
-  const size_t need = sgh_conv_workspace_bytes(g, SGH_CONV_WGRAD);
+  const size_t need = plain_workspace_bytes(g, SGH_CONV_WGRAD);
   if (need && (!workspace || ws_bytes < need)) return SGH_EWORKSPACE;
   hipStream_t s = sgh_stream_of(stream);
   const int CRS = g->C * g->R * g->S, PQ = g->P * g->Q;

@@ -1,0 +1,460 @@
+// fp32 weight gradient of 3x3 convolutions of stride 1 and padding 1 on the bfloat16 matrix instructions: three parts per value,
+// six products (conv_split.hip says why that is fp32 arithmetic).
+//
+//   dW[k][c][r][s] = sum_{n,p,q} dy[n][k][p][q] * x[n][c][p + r - 1][q + s - 1]
+//
+// The reduction runs over pixels: a matrix operand holds octets of eight consecutive pixels of a row.  An octet of dy meets the
+// x octets of three rows as they are (s = 1) and shifted by one pixel (s = 0, 2): a lane reads the aligned octet and the
+// neighbour dword on either side and forms both shifts with funnel shifts, so x is staged once for all nine taps.
+//
+// A workgroup owns 64 x 64 (k, c) pairs and all nine taps: a wavefront 32 x 32 pairs, 144 accumulators.  Its 512 threads are two
+// groups of 2 x 2 wavefronts, each walking half of the workgroup's rows with LDS of its own; the sums meet in LDS at the end, so
+// that one partial image per CU goes through memory.  A group walks a strip of up to 32 columns down the images, in "virtual"
+// rows (an image is its P rows and a row of zeros): per iteration RPI new rows of dy and of x are fetched into registers while
+// the previous ones are multiplied, then split and written; x rows live in a ring of RPI + 2.  Rows of OCS octets: the columns
+// beyond Q are zeros on both sides.
+//
+// The sums of the workgroups of a (k, c) tile are added in ascending order by k_wgrad_oct_reduce.
+#include "common.h"
+
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+constexpr int NT = 512, GT = 256;   // threads of a workgroup, of a group
+constexpr int PARTS = 3;
+constexpr int kOOB = int(0x80000000u);
+constexpr int kChain = 400;          // roundings of an accumulator (plan)
+constexpr int kAcc = 9 * 16 * 64;   // accumulators of a wavefront
+
+__device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
+}
+
+__device__ __forceinline__ v16f mfma(v4u a, v4u b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ unsigned pack2(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, bf16x2));
+}
+__device__ __forceinline__ float lo_f(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float hi_f(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
+
+struct WoArgs {
+  const float *dy, *x;
+  float *partial;   // [split][tile][wavefront][accumulator][lane]
+  int N, C, K, P, Q;
+  int ktiles, tiles, splits, strips, iters, per_split;   // iterations of a strip, of a workgroup
+  unsigned dy_bytes, x_bytes;
+};
+
+// Eight elements of a tensor row as they come from memory
+struct Octet {
+  v4u raw[2];
+  int nv;   // valid elements
+  // elements [off, off + nv) of the tensor; nothing beyond its last byte is touched
+  __device__ __forceinline__ void load(rsrc_t r, unsigned bytes, int off, int nv_) {
+    nv = nv_;
+    const int at = nv > 0 ? off * 4 : kOOB;
+    const bool tail = nv > 0 && unsigned(at) + 32 > bytes;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      raw[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, tail ? kOOB : at, 16 * i, 0));
+    if (__any(tail)) {
+      if (tail) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j / 4][j % 4] = __builtin_amdgcn_raw_buffer_load_b32(r, j < nv ? at + 4 * j : kOOB, 0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void parts(v4u (&out)[PARTS]) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned ua = raw[i / 2][2 * i % 4], ub = raw[i / 2][2 * i % 4 + 1];
+      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) : 0.f;
+      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) : 0.f;
+      const unsigned p0 = pack2(a, b);
+      const float ra = a - lo_f(p0), rb = b - hi_f(p0);
+      const unsigned p1 = pack2(ra, rb);
+      out[0][i] = p0, out[1][i] = p1, out[2][i] = pack2(ra - lo_f(p1), rb - hi_f(p1));
+    }
+  }
+};
+
+// One sum term by term: virtual rows [v0, v1), columns [q0, q1)
+__device__ float redo(const WoArgs &a, int k, int c, int tap, int v0, int v1, int q0, int q1) {
+  float sum = 0.f;
+  for (int v = v0; v < v1 && sum == sum; ++v) {
+    const int n = v / (a.P + 1), p = v - n * (a.P + 1);
+    if (p >= a.P || n >= a.N) continue;
+    const int h = p + tap / 3 - 1;
+    for (int q = q0; q < q1; ++q) {
+      const int w = q + tap % 3 - 1;
+      const bool in = unsigned(h) < unsigned(a.P) && unsigned(w) < unsigned(a.Q);
+      const float xv = in ? a.x[((size_t(n) * a.C + c) * a.P + h) * a.Q + w] : 0.f;
+      sum = __builtin_fmaf(a.dy[((size_t(n) * a.K + k) * a.P + p) * a.Q + q], xv, sum);
+    }
+  }
+  return sum;
+}
+
+template <int OCS, int RPI>
+struct Shape {
+  static constexpr int OPI = OCS * RPI, RING = RPI + 2;
+  static constexpr int XP = OCS == 4 ? 7 : OCS == 1 ? 3 : 5;   // 16-byte units of a channel's x row: the octets, a dword on either side, odd
+  static constexpr int XPART = 64 * XP * 16, XROW = PARTS * XPART;
+  static constexpr int DYO = (PARTS * 64 + 4) * 16;            // an octet of dy; four units of padding spread the writes over the banks
+  static constexpr int GROUP = RING * XROW + OPI * DYO;
+  static constexpr int LDS = 2 * GROUP > kAcc * 16 ? 2 * GROUP : kAcc * 16;
+  static_assert(OPI % 2 == 0 && LDS <= 160 * 1024, "");
+};
+
+template <int OCS, int RPI>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_wgrad_oct(WoArgs a) {
+  typedef Shape<OCS, RPI> S;
+  constexpr int OPI = S::OPI, RING = S::RING;
+  constexpr int TASKS = (OPI * 64 + GT - 1) / GT, EDGES = OCS >= 3 ? (RPI * 128 + GT - 1) / GT : 0;
+  extern __shared__ __align__(16) char smem[];
+  const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = wave >> 2, w4 = wave & 3, wm = w4 >> 1, wn = w4 & 1;
+  const int tg = t & (GT - 1);
+  char *const xs = smem + group * S::GROUP, *const dys = xs + RING * S::XROW;
+  // (the tiles of a split read the same rows: they go to one XCD, as in conv16.hip)
+  int tile, split;
+  if ((a.splits & 7) == 0) {
+    const int slot = int(blockIdx.x) >> 3;
+    tile = slot % a.tiles, split = slot / a.tiles * 8 + (int(blockIdx.x) & 7);
+  } else {
+    tile = int(blockIdx.x) % a.tiles, split = int(blockIdx.x) / a.tiles;
+  }
+  const int k0 = tile % a.ktiles * 64, c0 = tile / a.ktiles * 64;
+  const int strip = split % a.strips, q0 = strip * OCS * 8;
+  const int first = split / a.strips * a.per_split, last = min(a.iters, first + a.per_split);
+  const int mine = (a.per_split + 1) / 2;                    // iterations of a group (a last one may be empty)
+  const int it0 = first + group * mine, it1 = min(last, it0 + mine);
+  const int VP = a.P + 1;
+  const rsrc_t rdy = make_rsrc(a.dy, a.dy_bytes), rx = make_rsrc(a.x, a.x_bytes);
+
+  for (int i = tg; i < RING * S::XROW / 16; i += GT) reinterpret_cast<v4u *>(xs)[i] = v4u{0u, 0u, 0u, 0u};
+
+  // ---- staging.  A task is an octet of a channel: o = task % OPI (row o / OCS, octet o % OCS), channel task / OPI
+  auto row_of = [&](int v, int &n, int &p) {
+    n = v < 0 ? -1 : v / VP, p = v < 0 ? a.P : v - n * VP;
+  };
+  auto count = [&](int n, int p, int c, int channels, int q) {   // valid elements of the octet at column q
+    return p < a.P && n >= 0 && n < a.N && c < channels ? max(0, min(8, a.Q - q)) : 0;
+  };
+  auto put_x = [&](const Octet &o, int slot, int c, int oc) {
+    v4u part[PARTS];
+    o.parts(part);
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+      *reinterpret_cast<v4u *>(xs + slot * S::XROW + i * S::XPART + (c * S::XP + 1 + oc) * 16) = part[i];
+  };
+  // the element left (side 0) and right (side 1) of the strip
+  auto edge_off = [&](int n, int p, int c, int side) {
+    const int q = side ? q0 + 8 * OCS : q0 - 1;
+    const bool ok = p < a.P && n >= 0 && n < a.N && c0 + c < a.C && q >= 0 && q < a.Q;
+    return ok ? (((n * a.C + c0 + c) * a.P + p) * a.Q + q) * 4 : kOOB;
+  };
+  auto edge_get = [&](int off) -> unsigned { return __builtin_amdgcn_raw_buffer_load_b32(rx, off, 0, 0); };
+  auto put_edge = [&](unsigned raw, int slot, int c, int side) {
+    const float v = __builtin_bit_cast(float, raw);
+    const unsigned p0 = pack2(v, 0.f);
+    const float r = v - lo_f(p0);
+    const unsigned p1 = pack2(r, 0.f);
+    const uint16_t part[PARTS] = {uint16_t(p0), uint16_t(p1), uint16_t(pack2(r - lo_f(p1), 0.f))};
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+      *reinterpret_cast<uint16_t *>(xs + slot * S::XROW + i * S::XPART + c * S::XP * 16 + (side ? 16 + OCS * 16 : 14)) = part[i];
+  };
+
+  int dn[TASKS], dp[TASKS], xn[TASKS], xp[TASKS];   // (image, row) of this thread's next octets
+  int en[EDGES ? EDGES : 1], ep[EDGES ? EDGES : 1];
+#pragma unroll
+  for (int e = 0; e < TASKS; ++e) {
+    const int rr = (e * GT + tg) % OPI / OCS;
+    row_of(it0 * RPI + rr, dn[e], dp[e]);
+    row_of(it0 * RPI + 1 + rr, xn[e], xp[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < EDGES; ++e) row_of(it0 * RPI + 1 + (e * GT + tg) / 128, en[e], ep[e]);
+
+  Octet sd[TASKS], sx[TASKS];
+  unsigned se[EDGES ? EDGES : 1];
+  auto step_row = [&](int &n, int &p) {
+    p += RPI;
+    if (p >= VP) p -= VP, ++n;
+  };
+  auto load = [&]() {   // dy rows [v0, v0 + RPI) and x rows [v0 + 1, v0 + RPI] of an iteration, then on to the next one
+#pragma unroll
+    for (int e = 0; e < TASKS; ++e) {
+      const int i = e * GT + tg, o = i % OPI, ch = i / OPI, q = q0 + o % OCS * 8;
+      sd[e].load(rdy, a.dy_bytes, ((dn[e] * a.K + k0 + ch) * a.P + dp[e]) * a.Q + q, ch < 64 ? count(dn[e], dp[e], k0 + ch, a.K, q) : 0);
+      sx[e].load(rx, a.x_bytes, ((xn[e] * a.C + c0 + ch) * a.P + xp[e]) * a.Q + q, ch < 64 ? count(xn[e], xp[e], c0 + ch, a.C, q) : 0);
+      step_row(dn[e], dp[e]), step_row(xn[e], xp[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < EDGES; ++e) {
+      const int i = e * GT + tg;
+      se[e] = edge_get(edge_off(en[e], ep[e], i >> 1 & 63, i & 1));
+      step_row(en[e], ep[e]);
+    }
+  };
+  // The second group sums -dy x: the accumulating instructions round towards minus infinity on average, by 2^-26 of the sum,
+  // which over hundreds of partial sums would outweigh their random errors (64 channels of 56 x 56, N = 64: 6.0e-7 from float64
+  // with one sign, 3.2e-7 with two)
+  const unsigned sign = group ? 0x80008000u : 0u;
+  auto slot_of = [](int base, int j) { return base + j < RING ? base + j : base + j - RING; };
+  auto stage = [&](int base) {   // base: the ring slot of row v0 - 1
+#pragma unroll
+    for (int e = 0; e < TASKS; ++e) {
+      const int i = e * GT + tg, o = i % OPI, ch = i / OPI;
+      v4u part[PARTS];
+      sd[e].parts(part);
+      if (OPI * 64 % GT == 0 || ch < 64) {
+#pragma unroll
+        for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + ch) * 16) = part[j] ^ sign;
+        put_x(sx[e], slot_of(base, 2 + o / OCS), ch, o % OCS);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EDGES; ++e) {
+      const int i = e * GT + tg;
+      if (RPI * 128 % GT == 0 || i < RPI * 128) put_edge(se[e], slot_of(base, 2 + i / 128), i >> 1 & 63, i & 1);
+    }
+  };
+
+  v16f acc[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+
+  // rows v0 - 1 and v0, then the first iteration's own
+  int base = it0 * RPI % RING;
+  __syncthreads();   // (the zeros are in place)
+  for (int i = tg; i < 2 * OCS * 64; i += GT) {
+    const int oc = i % OCS, c = i / OCS & 63, j = i / (OCS * 64), q = q0 + oc * 8;
+    int n, p;
+    row_of(it0 * RPI - 1 + j, n, p);
+    Octet o;
+    o.load(rx, a.x_bytes, ((n * a.C + c0 + c) * a.P + p) * a.Q + q, count(n, p, c0 + c, a.C, q));
+    put_x(o, slot_of(base, j), c, oc);
+  }
+  if (EDGES) {
+    const int j = tg >> 7, c = tg >> 1 & 63;
+    int n, p;
+    row_of(it0 * RPI - 1 + j, n, p);
+    put_edge(edge_get(edge_off(n, p, c, tg & 1)), slot_of(base, j), c, tg & 1);
+  }
+  load();
+  stage(base);
+  __syncthreads();
+
+  const char *const da = dys + half * S::DYO + (wm * 32 + l32) * 16;
+  const char *const xb = xs + (wn * 32 + l32) * S::XP * 16 + 12;
+  for (int i = 0; i < mine; ++i) {
+    const bool more = i + 1 < mine;
+    if (more) load();
+    if (it0 + i < it1) {
+      struct Raw {
+        v4u d;
+        unsigned l, r;
+      };
+      // unit u = (step, row r, part): the octet and its neighbours; a unit's are read while the one before is multiplied
+      constexpr int UNITS = OPI / 2 * 3 * PARTS;
+      constexpr int ORDER[PARTS] = {0, 2, 1};   // (nine, three, six products)
+      auto read = [&](int u) {
+        const int s = u / (3 * PARTS), r = u / PARTS % 3, p = ORDER[u % PARTS];
+        const int oa = 2 * s, ob = 2 * s + 1;
+        const int ja = slot_of(base, oa / OCS + r) * S::XROW + oa % OCS * 16;
+        const int jb = slot_of(base, ob / OCS + r) * S::XROW + ob % OCS * 16;
+        const char *at = xb + (half ? jb : ja) + p * S::XPART;
+        Raw w;
+        w.l = *reinterpret_cast<const unsigned *>(at);
+        w.d = *reinterpret_cast<const v4u *>(at + 4);
+        w.r = *reinterpret_cast<const unsigned *>(at + 20);
+        return w;
+      };
+      v4u A[2][PARTS];
+      auto read_a = [&](int s) {
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) A[s & 1][p] = *reinterpret_cast<const v4u *>(da + 2 * s * S::DYO + p * 1024);
+      };
+      read_a(0);
+      Raw next = read(0);
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) {
+        const int s = u / (3 * PARTS), r = u / PARTS % 3, p = ORDER[u % PARTS];
+        const Raw w = next;
+        if (u + 1 < UNITS) next = read(u + 1);
+        if (u % (3 * PARTS) == 0 && s + 1 < OPI / 2) read_a(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        v4u sh[3];
+        sh[1] = w.d;
+        const unsigned m1 = __builtin_amdgcn_alignbit(w.d[1], w.d[0], 16), m2 = __builtin_amdgcn_alignbit(w.d[2], w.d[1], 16),
+                       m3 = __builtin_amdgcn_alignbit(w.d[3], w.d[2], 16);
+        sh[0] = v4u{__builtin_amdgcn_alignbit(w.d[0], w.l, 16), m1, m2, m3};
+        sh[2] = v4u{m1, m2, m3, __builtin_amdgcn_alignbit(w.r, w.d[3], 16)};
+#pragma unroll
+        for (int q = PARTS - 1 - p; q >= 0; --q)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) acc[r * 3 + c] = mfma(A[s & 1][q], sh[c], acc[r * 3 + c]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+    if (more) {
+      base = slot_of(base, RPI);
+      stage(base);
+      __syncthreads();
+    }
+  }
+
+  // ---- the two groups' sums, then this workgroup's partial image
+  float *const ex = reinterpret_cast<float *>(smem) + w4 * kAcc + lane;
+  if (group) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) ex[(i * 16 + v) * 64] = acc[i][v];
+  }
+  __syncthreads();
+  if (group) return;
+  const rsrc_t rp = make_rsrc(a.partial + (size_t(split) * a.tiles + tile) * 4 * kAcc, 4 * kAcc * 4);
+  const int po = (w4 * kAcc + lane) * 4;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    unsigned mask = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float s = acc[i][v] - ex[(i * 16 + v) * 64];
+      if (!finite(s)) mask |= 1u << v;
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po, (i * 16 + v) * 256, 0);
+    }
+    for (; mask; mask &= mask - 1) {
+      const int v = __builtin_ctz(mask), k = k0 + wm * 32 + 8 * (v >> 2) + 4 * half + (v & 3), c = c0 + wn * 32 + l32;
+      if (k >= a.K || c >= a.C) continue;
+      const float s = redo(a, k, c, i, first * RPI, last * RPI, q0, min(a.Q, q0 + 8 * OCS));
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po + (i * 16 + v) * 256, 0, 0);
+    }
+  }
+}
+
+// dW from the partial images: a row of 64 lanes is one accumulator of a wavefront, ZL threads share its splits
+template <int ZL>
+__global__ __launch_bounds__(64 * ZL) void k_wgrad_oct_reduce(WoArgs a, float *__restrict__ dW) {
+  __shared__ double sums[ZL][64];
+  const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
+  const int row = blockIdx.x, accum = row % 144, w4 = row / 144 % 4, tile = row / 576;
+  const size_t image = size_t(a.tiles) * 4 * kAcc;
+  const float *p = a.partial + size_t(row) * 64 + lane;
+  double s = 0;   // (in fp32 256 images add a tenth to the error of their sums)
+#pragma unroll 8
+  for (int i = z; i < a.splits; i += ZL) s += p[i * image];
+  if (ZL > 1) {
+    sums[z][lane] = s;
+    __syncthreads();
+    if (z) return;
+#pragma unroll
+    for (int i = 1; i < ZL; ++i) s += sums[i][lane];
+  }
+  const int tap = accum / 16, v = accum % 16;
+  const int k = tile % a.ktiles * 64 + (w4 >> 1) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+  const int c = tile / a.ktiles * 64 + (w4 & 1) * 32 + (lane & 31);
+  if (k >= a.K || c >= a.C) return;
+  dW[(size_t(k) * a.C + c) * 9 + tap] = float(s);
+}
+
+struct WoPlan {
+  bool ok;
+  int ocs, rpi, ktiles, tiles, splits, strips, iters, per_split;
+};
+
+WoPlan plan(const sgh_conv_geom *g) {
+  WoPlan p{};
+  if (g->R != 3 || g->S != 3 || g->stride_h != 1 || g->stride_w != 1 || g->pad_h != 1 || g->pad_w != 1) return p;
+  const size_t pixels = size_t(g->N) * g->P * g->Q, lim = size_t(1) << 29;
+  if (pixels * g->C >= lim || pixels * g->K >= lim) return p;
+  // Few channels leave the 64 columns of a tile empty (their nine taps are columns to the fp32 kernels: 3, 11 and 25 of 64
+  // channels 0.6 times as fast, 39 and more 1.1 to 2.4 times), and below 0.4 G products a launch is not worth its partial
+  // images (0.14 to 0.3 G: 0.94 to 1.0 times, and the shorter chains of the fp32 kernel are the more exact ones).
+  if (20 * g->C < 11 * 64 * ((g->C + 63) / 64) || double(pixels) * g->K * g->C * 9 < 7e8) return p;
+  const int oc = (g->Q + 7) / 8;
+  p.strips = (oc + 3) / 4;
+  p.ocs = (oc + p.strips - 1) / p.strips;
+  p.rpi = p.ocs == 4 ? 1 : p.ocs == 1 ? 4 : 2;
+  if (g->P + 1 < p.rpi || size_t(g->N) * (g->P + 1) >= (size_t(1) << 30)) return p;
+  p.iters = int((size_t(g->N) * (g->P + 1) + p.rpi - 1) / p.rpi);
+  p.ktiles = (g->K + 63) / 64;
+  const long tiles = long(p.ktiles) * ((g->C + 63) / 64);
+  if (tiles > 65536) return p;
+  p.tiles = int(tiles);
+  const int cus = sgh_num_cus();
+  // One workgroup per CU; more rounds of them where an accumulator would take more than kChain products' roundings (the error of
+  // a chain grows with its square root: 14 images of 154 and 670 channels, 37 x 27, 5.1e-7 from float64 in one round).
+  const long most = p.iters / 4 > 0 ? p.iters / 4 : 1;   // (two iterations for either group)
+  for (long rounds = 1;; ++rounds) {
+    long sp = rounds * cus / (tiles * p.strips);
+    if (sp > most) sp = most;
+    if (sp < 1) sp = 1;
+    p.per_split = int((p.iters + sp - 1) / sp);
+    if (sp == most || rounds == 8 || (p.per_split + 1) / 2 * (p.ocs * p.rpi / 2) * 6 <= kChain) break;
+  }
+  p.splits = (p.iters + p.per_split - 1) / p.per_split * p.strips;
+  p.ok = true;
+  return p;
+}
+
+template <int OCS, int RPI>
+int launch(const WoArgs &a, hipStream_t s) {
+  auto kern = k_wgrad_oct<OCS, RPI>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
+        hipSuccess)
+      return SGH_EUNSUPPORTED;
+    attr_set = true;
+  }
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.splits)), dim3(NT), (Shape<OCS, RPI>::LDS), s, a);
+  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+}
+
+}  // namespace
+
+size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g) {
+  const WoPlan p = plan(g);
+  return p.ok && !sgh_env().conv_split_off ? size_t(p.splits) * p.tiles * 4 * kAcc * sizeof(float) : 0;
+}
+
+int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s) {
+  const WoPlan p = plan(g);
+  if (!p.ok) return SGH_EUNSUPPORTED;
+  WoArgs a;
+  a.dy = dy, a.x = x, a.partial = static_cast<float *>(workspace);
+  a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
+  a.ktiles = p.ktiles, a.tiles = p.tiles, a.splits = p.splits, a.strips = p.strips, a.iters = p.iters, a.per_split = p.per_split;
+  const size_t pixels = size_t(g->N) * g->P * g->Q;
+  a.dy_bytes = unsigned(pixels * g->K * 4), a.x_bytes = unsigned(pixels * g->C * 4);
+  sgh_prof_kernel_begin("conv_wgrad/k_wgrad_oct", 2.0 * pixels * g->K * g->C * 9);
+  const int rc = p.ocs == 4   ? launch<4, 1>(a, s)
+                 : p.ocs == 3 ? launch<3, 2>(a, s)
+                 : p.ocs == 2 ? launch<2, 2>(a, s)
+                              : launch<1, 4>(a, s);
+  sgh_prof_kernel_end(s);
+  if (rc != SGH_OK) return rc;
+  // (threads per accumulator: as many as leave each a few images)
+  const dim3 grid(unsigned(a.tiles * 576));
+  if (a.splits >= 64) hipLaunchKernelGGL(k_wgrad_oct_reduce<16>, grid, dim3(1024), 0, s, a, dW);
+  else if (a.splits >= 8) hipLaunchKernelGGL(k_wgrad_oct_reduce<4>, grid, dim3(256), 0, s, a, dW);
+  else hipLaunchKernelGGL(k_wgrad_oct_reduce<1>, grid, dim3(64), 0, s, a, dW);
+  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+}

@@ -1153,3 +1153,62 @@ def test_conv_split_operands_non_finite(singa, dev, n, c, h, w, k, where, bad):
         assert np.array_equal(np.isnan(g), np.isnan(ref)) and np.array_equal(np.isposinf(g), np.isposinf(ref))
         fin = np.isfinite(ref) & np.isfinite(g)
         np.testing.assert_allclose(g[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+# sizes of the split-operand weight gradient (wgrad_oct.hip): rows of one to four octets and of several strips, ragged octets and
+# channels, rows that do not divide the iterations, and (few products) its neighbours
+WGRAD_OCTET_CASES = [
+    # n, c, h, w, k
+    (64, 64, 14, 7, 130), (70, 129, 7, 8, 150), (40, 70, 13, 9, 257), (30, 64, 17, 16, 200), (9, 100, 25, 17, 230),
+    (11, 64, 21, 24, 260), (10, 65, 30, 25, 170), (5, 128, 31, 32, 130), (3, 64, 33, 41, 400), (2, 64, 56, 56, 300), (1, 257, 30, 111, 130),
+    (4, 12, 20, 20, 64), (2, 300, 3, 64, 300), (600, 64, 2, 6, 400),
+]
+
+
+@pytest.mark.parametrize("n,c,h,w,k", WGRAD_OCTET_CASES)
+def test_conv_wgrad_octets(singa, dev, n, c, h, w, k):
+    """Against float64: in any order the error of `terms` products is at most terms * 2^-23 of the sum of their magnitudes, and
+    about sqrt(terms) * 2^-24 of the result in the 2-norm (twice that is allowed); the last row and column of the tensors count."""
+    import torch
+    rg = rng(n + 3 * c + k)
+    x, dy = randn(rg, n, c, h, w), randn(rg, n, k, h, w)
+    xd, dyd, wd = singa.from_numpy(x, dev), singa.from_numpy(dy, dev), singa.from_numpy(np.zeros((k, c, 3, 3), np.float32), dev)
+    hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, False)
+    got = singa.GpuConvBackwardW(dyd, xd, wd, hd).to_numpy()
+    pad = lambda a: np.pad(a.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    for absolute in (False, True):
+        xp, d = pad(np.abs(x) if absolute else x), (np.abs(dy) if absolute else dy).astype(np.float64)
+        d2 = torch.from_numpy(d.transpose(1, 0, 2, 3).reshape(k, -1).copy())
+        ref = np.stack([(d2 @ torch.from_numpy(xp[:, :, r:r + h, s:s + w].transpose(0, 2, 3, 1).reshape(-1, c).copy())).numpy()
+                        for r in range(3) for s in range(3)], -1).reshape(k, c, 3, 3)
+        if absolute:
+            assert np.all(np.abs(got - want) <= n * h * w * 2.0 ** -23 * ref)
+        else:
+            want = ref
+            assert nl2(got, want) < 2 * (n * h * w) ** 0.5 * 2.0 ** -24
+    again = singa.GpuConvBackwardW(dyd, xd, wd, hd).to_numpy()
+    assert_bit_equal(again, got, "partial images in a fixed order")
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.4e38])
+def test_conv_wgrad_octets_non_finite(singa, dev, bad):
+    """Non-finite values (and those whose bfloat16 rounding is infinite) reach the weights whose products they are in, the
+    products with padding among them (zeros: NaN), and no others."""
+    n, c, h, w, k = 12, 70, 20, 30, 140
+    rg = rng(8)
+    x, dy = randn(rg, n, c, h, w), randn(rg, n, k, h, w)
+    x *= np.float32(1e-3)
+    dy *= np.float32(1e-3)
+    x[3, 5, 7, 29] = bad
+    dy[11, 139, 19, 4] = bad
+    xd, dyd, wd = singa.from_numpy(x, dev), singa.from_numpy(dy, dev), singa.from_numpy(np.zeros((k, c, 3, 3), np.float32), dev)
+    hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, False)
+    got = singa.GpuConvBackwardW(dyd, xd, wd, hd).to_numpy()
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    with np.errstate(all="ignore"):
+        d2 = dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(k, -1)
+        want = np.stack([np.einsum("kp,pc->kc", d2, xp[:, :, r:r + h, s:s + w].transpose(0, 2, 3, 1).reshape(-1, c))
+                         for r in range(3) for s in range(3)], -1).reshape(k, c, 3, 3).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    fin = np.isfinite(want) & np.isfinite(got)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-5)
