@@ -148,6 +148,11 @@ int sgh_wgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *x, fl
 // take; the caller checks that the workspace has them.
 size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);
 int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s);
+// The same of 16-bit tensors, stride 1 or 2 (wgrad_oct16.hip)
+size_t sgh_wgrad_oct16_workspace_bytes(const sgh_conv_geom *g);
+double sgh_wgrad_oct16_us(const sgh_conv_geom *g);   // its expected time
+int sgh_wgrad_oct16_run(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace, bool bf16,
+                        hipStream_t s);
 
 // Weight gradient for few input channels and a large filter (C*R*S in 65..160: the 7x7 stem),
 // wgrad_fewc.hip.  Same conventions as the 3x3 kernel above.
@@ -189,6 +194,7 @@ int sgh_pw_dgrad_run(const sgh_conv_geom *g, const float *dy, const float *W, fl
 // *_workspace_bytes is 0 and the run functions return SGH_EUNSUPPORTED for geometries they do not
 // cover (strides above 2, K not a multiple of 8 for the data gradient, tensors of 2^31 elements).
 size_t sgh_conv16_workspace_bytes(const sgh_conv_geom *g, int which);
+size_t sgh_conv16_wgrad_full_bytes(const sgh_conv_geom *g);
 int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace,
                      size_t ws_bytes, bool bf16, hipStream_t s);
 int sgh_conv16_dgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, uint16_t *dx, void *workspace,

@@ -1040,6 +1040,7 @@ struct W16Plan {
   int bm, stride, mtiles, ntiles, chunks, splits, cps;
   sgh_conv_geom f;  // the geometry the kernel sees (1x1 stride-1 layers: image plane as one row)
   int QO;
+  double walk, reduce;   // chunks of a workgroup times rounds, the split reduction, both in chunk times
 };
 
 // `shared`: the launch shares the chip with another stream's kernels (it runs on a device's auxiliary stream
@@ -1083,10 +1084,29 @@ W16Plan wplan(const sgh_conv_geom *g, bool shared) {
     const int s2 = s >= 8 ? s : (p.chunks + cps - 1) / cps;
     const long rounds = (long(tiles) * s2 + slots - 1) / slots;
     const double cost = double(rounds * (cps + 2)) + s2 * reduce_chunks_per_split;  // (+2: prologue, epilogue)
-    if (best < 0 || cost < best) best = cost, p.cps = cps, p.splits = s2;
+    if (best < 0 || cost < best)
+      best = cost, p.cps = cps, p.splits = s2, p.walk = double(rounds * (cps + 2)), p.reduce = s2 * reduce_chunks_per_split;
   }
   p.ok = true;
   return p;
+}
+
+// 3x3 layers of padding 1 take the octet kernel (wgrad_oct16.hip) where it is expected to be a tenth faster.  Microseconds of
+// either, fitted to 170 layers drawn over 1..128 images, 3..1024 channels, planes of 7..112 and both strides (the octet kernel's
+// to 9 per cent, this one's to 10; sgh_wgrad_oct16_us has the other side).  A chunk costs more where the chip is full, where
+// stride 2 fetches twice the bytes, and less on the 64-row tile.  Few channels, few pixels and tiles that are mostly empty stay
+// here: 8 x 59 x 59 to 12 filters 11 against 25 us; 128 images of 512 channels, 7 x 7, leave: 107 against 59 us.
+bool octets_pay(const sgh_conv_geom *g, size_t *workspace) {
+  const size_t need = sgh_wgrad_oct16_workspace_bytes(g);
+  if (!need) return false;
+  const W16Plan p = wplan(g, false);
+  if (!p.ok) return false;
+  const double full = double(p.mtiles) * p.ntiles * p.splits / (2 * sgh_num_cus());
+  const double chunk = 0.76 + 0.65 * (full < 1 ? full : 1) + (p.stride == 2 ? 0.35 : 0.0) + (g->Q <= 8 ? 0.09 : 0.0) -
+                       (p.bm == 64 ? 0.41 : 0.0);
+  if (7 + p.walk * chunk + 2.5 * p.reduce < 1.1 * sgh_wgrad_oct16_us(g)) return false;
+  *workspace = need;
+  return true;
 }
 
 struct D16Plan {
@@ -1297,12 +1317,21 @@ size_t sgh_conv16_workspace_bytes(const sgh_conv_geom *g, int which) {
   return 0;
 }
 
+// The workspace with which sgh_conv16_wgrad takes its fastest kernel; with sgh_conv16_workspace_bytes it runs
+size_t sgh_conv16_wgrad_full_bytes(const sgh_conv_geom *g) {
+  const size_t least = sgh_conv16_workspace_bytes(g, SGH_CONV_WGRAD);
+  size_t octets;
+  return least && octets_pay(g, &octets) && octets > least ? octets : least;
+}
+
 int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace,
                      size_t ws_bytes, bool bf16, hipStream_t s) {
   const int mode = g_wgrad16_split_mode.load(std::memory_order_relaxed);
   const W16Plan p = wplan(g, mode < 0 ? sgh_stream_is_aux(s) : mode != 0);
   if (!p.ok) return SGH_EUNSUPPORTED;
   if (!workspace || ws_bytes < sgh_conv16_workspace_bytes(g, SGH_CONV_WGRAD)) return SGH_EWORKSPACE;
+  size_t octets;
+  if (octets_pay(g, &octets) && ws_bytes >= octets) return sgh_wgrad_oct16_run(g, dy, x, dW, workspace, bf16, s);
   W16Args a{};
   a.dy = dy, a.x = x, a.partial = static_cast<float *>(workspace);
   a.N = p.f.N, a.C = p.f.C, a.H = p.f.H, a.W = p.f.W, a.K = p.f.K, a.P = p.f.P, a.Q = p.f.Q;

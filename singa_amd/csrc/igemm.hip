@@ -1752,6 +1752,7 @@ size_t sgh_conv_workspace_bytes_h(const sgh_conv_geom *g, int which) {
   const size_t wide = half_plan(g, which).total() + (which == SGH_CONV_FWD ? align256(size_t(g->K) * 4) : 0);
   size_t native = sgh_conv16_workspace_bytes(g, which);
   if (which == SGH_CONV_FWD && sgh_fwd_fewc16_workspace_bytes(g) > native) native = sgh_fwd_fewc16_workspace_bytes(g);
+  if (which == SGH_CONV_WGRAD) native = sgh_conv16_wgrad_full_bytes(g);
   return wide > native ? wide : native;
 }
 

@@ -968,6 +968,79 @@ def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
             assert nl2(got[part], want[part]) < bound
 
 
+# layers that the octet weight gradient (wgrad_oct16.hip) takes: rows of one to four octets and of several strips, whole and ragged
+# octets and channels, odd and even planes of stride 2, rows that do not divide the iterations; and two that it does not take
+WGRAD_OCTET16_CASES = [
+    # N, C, H, W, K, stride
+    (26, 568, 59, 8, 43, 1), (77, 464, 61, 6, 22, 1), (50, 512, 7, 7, 130, 1), (55, 600, 36, 9, 26, 1), (23, 601, 56, 13, 28, 1),
+    (53, 640, 20, 24, 18, 1), (50, 548, 26, 17, 24, 1), (29, 324, 64, 42, 11, 1), (13, 516, 25, 32, 56, 1), (75, 113, 58, 57, 10, 1),
+    (6, 955, 27, 24, 146, 1), (64, 64, 56, 56, 64, 1),
+    (54, 233, 51, 12, 142, 2), (95, 172, 66, 5, 172, 2), (7, 895, 22, 23, 540, 2), (41, 60, 65, 18, 388, 2), (94, 536, 30, 17, 42, 2),
+    (41, 345, 65, 50, 24, 2), (34, 253, 21, 49, 135, 2), (64, 468, 60, 77, 8, 2), (128, 128, 57, 56, 128, 2),
+    (3, 65, 6, 20, 40, 1), (5, 100, 49, 48, 230, 2),
+]
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("case", WGRAD_OCTET16_CASES)
+def test_conv_wgrad_octets_16bit(singa, dev, kind, case):
+    """Against float64 on the stored values: one rounding of the result (2^-12 or 2^-9 of it in the mean, at most 2^-11 or 2^-8)
+    and fp32 sums; single weights within that of the sum of their terms' magnitudes."""
+    import torch
+    from util import nl2
+    N, C, H, W, K, st = case
+    print("octets", kind, case, flush=True)
+    r = rng(sum(case) + 6)
+    xt, x = _to(singa, dev, r.standard_normal((N, C, H, W)).astype(np.float32), kind)
+    wt, _ = _to(singa, dev, np.zeros((K, C, 3, 3), np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (3, 3), (st, st), (1, 1), C, K, False)
+    P, Q = (H - 1) // st + 1, (W - 1) // st + 1
+    dyt, dy = _to(singa, dev, r.standard_normal((N, K, P, Q)).astype(np.float32), kind)
+    dw = singa.GpuConvBackwardW(dyt, xt, wt, h).to_numpy()
+
+    def product(x, dy):
+        xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 2), (1, 2)))
+        d2 = torch.from_numpy(dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(K, -1).copy())
+        taps = [d2 @ torch.from_numpy(xp[:, :, i:i + st * P:st, j:j + st * Q:st].transpose(0, 2, 3, 1).reshape(-1, C).copy())
+                for i in range(3) for j in range(3)]
+        return torch.stack(taps, -1).numpy().reshape(K, C, 3, 3)
+
+    want, most = product(x, dy), product(np.abs(x), np.abs(dy))
+    unit = 2.0 ** (-11 if kind == "f16" else -8)
+    assert nl2(dw, want) < unit
+    assert np.all(np.abs(dw - want) <= unit * np.abs(want) + N * P * Q * 2.0 ** -23 * most + 2.0 ** -25)
+    _same_bits(singa.GpuConvBackwardW(dyt, xt, wt, h).to_numpy(), dw, "partial images in a fixed order")
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_conv_wgrad_octets_16bit_non_finite(singa, dev, kind, stride, bad):
+    """Non-finite values reach the weights whose products they are in, those with the padding among them, and no others."""
+    import torch
+    N, C, H, W, K = (23, 601, 56, 13, 28) if stride == 1 else (54, 233, 51, 11, 155)
+    r = rng(9)
+    P, Q = (H - 1) // stride + 1, (W - 1) // stride + 1
+    x, dy = r.standard_normal((N, C, H, W)).astype(np.float32), r.standard_normal((N, K, P, Q)).astype(np.float32)
+    x[3, 5, H - 1, W - 1] = bad
+    x[4, 6, 0, 0] = bad
+    dy[11, 27, P - 1, 4] = bad
+    xt, x = _to(singa, dev, x, kind)
+    dyt, dy = _to(singa, dev, dy, kind)
+    wt, _ = _to(singa, dev, np.zeros((K, C, 3, 3), np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (3, 3), (stride, stride), (1, 1), C, K, False)
+    got = singa.GpuConvBackwardW(dyt, xt, wt, h).to_numpy()
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 2), (1, 2)))
+    with np.errstate(all="ignore"):
+        d2 = torch.from_numpy(dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(K, -1).copy())
+        want = torch.stack([d2 @ torch.from_numpy(xp[:, :, i:i + stride * P:stride, j:j + stride * Q:stride].transpose(0, 2, 3, 1)
+                                                  .reshape(-1, C).copy()) for i in range(3) for j in range(3)], -1)
+        want = want.numpy().reshape(K, C, 3, 3)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-2, atol=1e-1)
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 @pytest.mark.parametrize("case", [(2, 64, 16, 24, 40), (3, 40, 12, 20, 24), (2, 72, 14, 14, 136), (2, 16, 9, 11, 8), (1, 16, 4, 10, 64),
                                   (1, 64, 7, 4, 16)])
