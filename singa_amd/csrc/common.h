@@ -144,6 +144,9 @@ size_t sgh_wgrad3x3_workspace_bytes(const sgh_conv_geom *g);
 int sgh_wgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace,
                      size_t ws_bytes, hipStream_t s);
 
+// fp32 forward over fewer than eight input channels (fwd_few.hip); SGH_EUNSUPPORTED for geometries it does not take
+int sgh_fwd_few_run(const sgh_conv_geom *g, const float *x, const float *W, const float *bias, float *y, hipStream_t s);
+
 // fp32 3x3 stride-1 pad-1 weight gradient on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
 // take; the caller checks that the workspace has them.
 size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);

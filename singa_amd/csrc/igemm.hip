@@ -1438,6 +1438,13 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
       return rcf;
     }
   }
+  {
+    const int rcf = sgh_fwd_few_run(g, x, W, bias, y, s);
+    if (rcf != SGH_EUNSUPPORTED) {
+      sgh_prof_stop(s);
+      return rcf;
+    }
+  }
   sgh_conv_geom gt;
   if (fwd_as_split(g, &gt) && ws_bytes >= sgh_conv_split_workspace_bytes(&gt)) {
     int rcs = sgh_conv_split_weights(&gt, W, workspace, false, s);

@@ -1212,3 +1212,41 @@ def test_conv_wgrad_octets_non_finite(singa, dev, bad):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
     fin = np.isfinite(want) & np.isfinite(got)
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-5)
+
+
+# sizes of the few-channel forward kernel (fwd_few.hip): one to seven channels, tiles that cross images, ragged blocks of pixels and
+# filters, strides and paddings, planes smaller than the window, rows of the most pixels
+FWD_FEW_CASES = [
+    # n, c, h, w, k, r, stride, pad
+    (5, 3, 32, 32, 32, 5, 1, 2), (3, 1, 28, 28, 33, 5, 1, 2), (2, 7, 9, 11, 65, 7, 1, 3), (40, 3, 7, 7, 8, 3, 1, 1), (7, 2, 5, 6, 100, 3, 2, 1),
+    (2, 3, 65, 64, 64, 7, 2, 3), (1, 4, 112, 256, 24, 3, 1, 1), (1, 6, 30, 31, 31, 5, 2, 0), (9, 5, 3, 2, 40, 3, 3, 2), (300, 3, 4, 4, 130, 5, 1, 2),
+    (1, 3, 1, 1, 1, 7, 1, 3), (2, 3, 40, 300, 16, 3, 1, 1),
+]
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,st,pad", FWD_FEW_CASES)
+def test_conv_forward_few_channels(singa, dev, n, c, h, w, k, r, st, pad):
+    """Against float64: `terms` products in any order are within terms * 2^-23 of the sum of their magnitudes and within about
+    sqrt(terms) * 2^-24 in the 2-norm (twice that is allowed); non-finite values reach the windows that they are in, no others."""
+    import torch
+    rg = rng(n + 3 * c + k + r)
+    x, W, b = randn(rg, n, c, h, w), randn(rg, k, c, r, r), randn(rg, k)
+    terms = c * r * r + 1
+    conv = lambda x, W, b: torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(W).double(),
+                                                      torch.from_numpy(b).double(), st, pad).numpy()
+
+    def run(x, bias):
+        xd, wd, bd = singa.from_numpy(x, dev), singa.from_numpy(W, dev), singa.from_numpy(b, dev)
+        return singa.GpuConvForward(xd, wd, bd if bias else None,
+                                    singa.CudnnConvHandle(xd, (r, r), (st, st), (pad, pad), c, k, bias)).to_numpy()
+
+    for bias in (True, False):
+        bb = b if bias else 0 * b
+        got, want, most = run(x, bias), conv(x, W, bb), conv(np.abs(x), np.abs(W), np.abs(bb))
+        assert np.all(np.abs(got - want) <= terms * 2.0 ** -23 * most)
+        assert nl2(got, want) < 2 * terms ** 0.5 * 2.0 ** -24
+    x[n // 2, c - 1, h // 2, w // 2] = np.inf
+    x[0, 0, 0, w - 1] = np.nan
+    got = run(x, False)
+    hit = conv((~np.isfinite(x)).astype(np.float32), np.ones_like(W), 0 * b) > 0
+    assert np.array_equal(~np.isfinite(got), hit)
