@@ -349,29 +349,37 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   }
 }
 
-// dW from the partial images: a row of 64 lanes is one accumulator of a wavefront, ZL threads share its splits
+// dW from the partial images, in ascending order.  A workgroup takes four accumulator registers of a wavefront (16 bytes a lane:
+// 4 bytes a lane and one register a workgroup read the 38 MB of a layer in 12 us, this in 9) and nine taps: stretches of 288
+// weights; ZL threads share the images of a sum, ZL workgroups the taps.
 template <int ZL>
-__global__ __launch_bounds__(64 * ZL) void k_wgrad_oct_reduce(WoArgs a, float *__restrict__ dW) {
-  __shared__ double sums[ZL][64];
-  const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
-  const int row = blockIdx.x, accum = row % 144, w4 = row / 144 % 4, tile = row / 576;
+__global__ __launch_bounds__(576) void k_wgrad_oct_reduce(WoArgs a, float *__restrict__ dW) {
+  constexpr int TAPS = 9 / ZL;   // taps of a workgroup
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  __shared__ double sums[ZL][TAPS][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, z = wave / TAPS, ti = wave % TAPS;
+  const int tap0 = int(blockIdx.x) % ZL * TAPS, b = int(blockIdx.x) / ZL, v = b % 4 * 4, w4 = b / 4 % 4, tile = b / 16;
   const size_t image = size_t(a.tiles) * 4 * kAcc;
-  const float *p = a.partial + size_t(row) * 64 + lane;
-  double s = 0;   // (in fp32 256 images add a tenth to the error of their sums)
-#pragma unroll 8
-  for (int i = z; i < a.splits; i += ZL) s += p[i * image];
-  if (ZL > 1) {
-    sums[z][lane] = s;
-    __syncthreads();
-    if (z) return;
+  const float *p = a.partial + (size_t(tile) * 4 + w4) * kAcc + ((tap0 + ti) * 16 + v) * 64 + lane * 4;
+  double s[4] = {0, 0, 0, 0};   // (in fp32 256 images add a tenth to the error of their sums)
+#pragma unroll 4
+  for (int i = z; i < a.splits; i += ZL) {
+    const v4f x = *reinterpret_cast<const v4f *>(p + i * image);
 #pragma unroll
-    for (int i = 1; i < ZL; ++i) s += sums[i][lane];
+    for (int d = 0; d < 4; ++d) s[d] += x[d];
   }
-  const int tap = accum / 16, v = accum % 16;
-  const int k = tile % a.ktiles * 64 + (w4 >> 1) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-  const int c = tile / a.ktiles * 64 + (w4 & 1) * 32 + (lane & 31);
-  if (k >= a.K || c >= a.C) return;
-  dW[(size_t(k) * a.C + c) * 9 + tap] = float(s);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) sums[z][ti][lane * 4 + d] = s[d];
+  __syncthreads();
+  for (int e = threadIdx.x; e < TAPS * 256; e += 576) {
+    const int l = e / TAPS, tj = e % TAPS;   // l: register, lane of an accumulator
+    double r = sums[0][tj][l];
+#pragma unroll
+    for (int i = 1; i < ZL; ++i) r += sums[i][tj][l];
+    const int k = tile % a.ktiles * 64 + (w4 >> 1) * 32 + 2 * v + 4 * (l >> 5 & 1) + (l >> 6);
+    const int c = tile / a.ktiles * 64 + (w4 & 1) * 32 + (l & 31);
+    if (k < a.K && c < a.C) dW[(size_t(k) * a.C + c) * 9 + tap0 + tj] = float(r);
+  }
 }
 
 struct WoPlan {
@@ -452,9 +460,9 @@ int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, f
   sgh_prof_kernel_end(s);
   if (rc != SGH_OK) return rc;
   // (threads per accumulator: as many as leave each a few images)
-  const dim3 grid(unsigned(a.tiles * 576));
-  if (a.splits >= 64) hipLaunchKernelGGL(k_wgrad_oct_reduce<16>, grid, dim3(1024), 0, s, a, dW);
-  else if (a.splits >= 8) hipLaunchKernelGGL(k_wgrad_oct_reduce<4>, grid, dim3(256), 0, s, a, dW);
-  else hipLaunchKernelGGL(k_wgrad_oct_reduce<1>, grid, dim3(64), 0, s, a, dW);
+  const unsigned blocks = unsigned(a.tiles) * 16;
+  if (a.splits >= 24) hipLaunchKernelGGL(k_wgrad_oct_reduce<9>, dim3(blocks * 9), dim3(576), 0, s, a, dW);
+  else if (a.splits >= 6) hipLaunchKernelGGL(k_wgrad_oct_reduce<3>, dim3(blocks * 3), dim3(576), 0, s, a, dW);
+  else hipLaunchKernelGGL(k_wgrad_oct_reduce<1>, dim3(blocks), dim3(576), 0, s, a, dW);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
