@@ -15,6 +15,11 @@
 // beyond Q are zeros on both sides.
 //
 // The sums of the workgroups of a (k, c) tile are added in ascending order by k_wgrad_oct_reduce.
+//
+// 64 images, with the reduction, k_wgrad3x3 before and this: 64 channels of 56 x 56 164 -> 103 us, 128 of 28 x 28 146 -> 104,
+// 256 of 14 x 14 146 -> 97, 512 of 7 x 7 143 -> 101; 130 drawn layers 1.5 times as fast, 0.9 times the error against float64.
+// The matrix instructions are busy for 62 per cent of the cycles and the clock falls to 1.8 GHz under them: letting the groups take
+// turns, one multiplying while the other stages, gave 1 to 3 per cent and spilled the rows of three octets.
 #include "common.h"
 
 namespace {
@@ -88,18 +93,22 @@ struct Octet {
   }
 };
 
-// One sum term by term: virtual rows [v0, v1), columns [q0, q1)
-__device__ float redo(const WoArgs &a, int k, int c, int tap, int v0, int v1, int q0, int q1) {
+// One sum term by term: virtual rows [v0, v1), columns [q0, q1).  A NaN of dy makes one of the filter's sums of every tap and
+// channel, a NaN of x of every filter's at this tap and channel; `seen` tells the caller (bit 0: dy, bit 1: x), which need not
+// look for it again (a diverged network has little else: 144 searches a lane took 0.8 ms)
+__device__ float redo(const WoArgs &a, int k, int c, int tap, int v0, int v1, int q0, int q1, unsigned &seen) {
   float sum = 0.f;
   for (int v = v0; v < v1 && sum == sum; ++v) {
     const int n = v / (a.P + 1), p = v - n * (a.P + 1);
     if (p >= a.P || n >= a.N) continue;
     const int h = p + tap / 3 - 1;
-    for (int q = q0; q < q1; ++q) {
+    for (int q = q0; q < q1 && sum == sum; ++q) {
       const int w = q + tap % 3 - 1;
       const bool in = unsigned(h) < unsigned(a.P) && unsigned(w) < unsigned(a.Q);
       const float xv = in ? a.x[((size_t(n) * a.C + c) * a.P + h) * a.Q + w] : 0.f;
-      sum = __builtin_fmaf(a.dy[((size_t(n) * a.K + k) * a.P + p) * a.Q + q], xv, sum);
+      const float d = a.dy[((size_t(n) * a.K + k) * a.P + p) * a.Q + q];
+      seen |= (d != d ? 1u : 0u) | (xv != xv ? 2u : 0u);
+      sum = __builtin_fmaf(d, xv, sum);
     }
   }
   return sum;
@@ -331,9 +340,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (group) return;
   const rsrc_t rp = make_rsrc(a.partial + (size_t(split) * a.tiles + tile) * 4 * kAcc, 4 * kAcc * 4);
   const int po = (w4 * kAcc + lane) * 4;
+  unsigned nan_k = 0;   // accumulator registers whose filter has met a NaN of dy
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
     unsigned mask = 0;
+    bool nan_x = false;   // this tap has met a NaN of x
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const float s = acc[i][v] - ex[(i * 16 + v) * 64];
@@ -343,7 +354,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     for (; mask; mask &= mask - 1) {
       const int v = __builtin_ctz(mask), k = k0 + wm * 32 + 8 * (v >> 2) + 4 * half + (v & 3), c = c0 + wn * 32 + l32;
       if (k >= a.K || c >= a.C) continue;
-      const float s = redo(a, k, c, i, first * RPI, last * RPI, q0, min(a.Q, q0 + 8 * OCS));
+      float s = __builtin_nanf("");
+      if (!nan_x && !(nan_k >> v & 1)) {
+        unsigned seen = 0;
+        s = redo(a, k, c, i, first * RPI, last * RPI, q0, min(a.Q, q0 + 8 * OCS), seen);
+        nan_k |= (seen & 1) << v, nan_x = seen & 2;
+      }
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po + (i * 16 + v) * 256, 0, 0);
     }
   }
