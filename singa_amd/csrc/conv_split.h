@@ -22,7 +22,7 @@ constexpr int kSplitTaps = 9, kSplitTapsFew = 3;
 
 // One (chunk of 16 channels k, block of 32 channels c) of the weight fragments [chunk][tap][block][part][lane][8], by 256
 // threads: the source runs are contiguous, the fragments too, LDS turns one into the other.
-// (w0, w1, w2) sum to w exactly; an infinite w is (w, 0, 0), so that the sum stays what w was.
+// (w0, w1, w2) sum to w exactly; an infinite w is (w, 0, 0), so that the sum stays what w was.  Odd taps are negated.
 __device__ __forceinline__ void sgh_conv_split_weights_block(const float *__restrict__ W, uint16_t *__restrict__ wt, int C, int K,
                                                              int RS, int cblocks, int dgrad, int blk, int taps, float *buf) {
   const int groups = (RS + taps - 1) / taps, group = blk % groups;
@@ -54,7 +54,7 @@ __device__ __forceinline__ void sgh_conv_split_weights_block(const float *__rest
       uint16_t part[3][8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float w = src[j * 9];
+        const float w = q % RS & 1 ? -src[j * 9] : src[j * 9];
         auto up = [](uint16_t b) { return __builtin_bit_cast(float, unsigned(b) << 16); };
         auto down = [](float f) { return __builtin_bit_cast(uint16_t, __bf16(f)); };
         const bool big = !(__builtin_fabsf(w) < 3.38e38f);   // rounds to infinity, is infinite or NaN

@@ -1,12 +1,20 @@
 // fp32 convolutions of stride 1 with "same" padding (3x3, 5x5), forward and data gradient, on the bfloat16 matrix
-// instructions without giving up fp32 operands: every fp32 value is the exact sum of three bfloat16 values
+// instructions without giving up fp32 operands (the splitting of G. Henry, P. Tang, A. Heinecke, "Leveraging the bfloat16
+// artificial intelligence datatype for higher-precision computations", 2019): a fp32 value is the sum of three bfloat16 values
 //
 //   x = x0 + x1 + x2,   x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)      (8 + 8 + 8 bits of significand)
 //
 // and a product of two of them is the sum of nine exact products, of which the six with weights down to 2^-16 are formed
-// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0); the three left out are below 2^-25 of the product, half an ulp of fp32.
+// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0).  The three left out come to 2^-24 of the product at most, 2^-29 in the mean.
 // v_mfma_f32_32x32x16_bf16 multiplies 16 x as much per cycle as v_mfma_f32_32x32x2_f32, so six of them are 2.67 times as
 // fast, with fp32 accumulators either way.
+//
+// What decides the error of a convolution is how often its sum is rounded: the fp32 instructions do that once per product, the
+// bfloat16 ones once per eight, six times over.  So the six products of a tap and 16 channels are summed on their own, the
+// small ones first, and that sum is added to the accumulator with one rounding to nearest.  (All on the accumulator: 1.05 to 1.2
+// times the error of the fp32 instructions behind a ReLU, whose zeros cost those nothing.)  The matrix instructions round towards
+// minus infinity on average; the weights of every other tap are negated, and their sums subtracted, so that this does not add
+// up (900 channels: a mean error of 2e-7 of the results with one sign, 2e-8 with two).
 //
 //   out[n][c][h][w] = sum_{k,r,s} in[n][k][h + r - o][w + s - o] * Wf[c][k][r][s],   o = (R - 1) / 2
 //
@@ -23,9 +31,10 @@
 // 512 threads = 8 wavefronts of at most 128 registers, two workgroups per CU where the slab takes no more than 80 KB of LDS: while
 // one stages and waits at its barriers the other one's matrix instructions run.
 //
-// 64 images, forward pass, the kernel on fp32 instructions (dgrad3x3.hip) before and this: 64 channels of 56 x 56 131 -> 82 us,
-// 128 of 28 x 28 129 -> 85, 256 of 14 x 14 137 -> 82, 512 of 7 x 7 138 -> 92; 270 drawn layers 2.1 times as fast, none slower than
-// 0.96, with 0.7 times the error against float64 (1.03 at most).
+// 64 images, whole calls, on fp32 instructions (dgrad3x3.hip) and here: 64 channels of 56 x 56 forward 143 -> 97 us, data gradient
+// 131 -> 90; 128 of 28 x 28 139 -> 94, 128 -> 90; 256 of 14 x 14 145 -> 97, 136 -> 91; 512 of 7 x 7 156 -> 106, 137 -> 100.  The error
+// against float64 is 0.15 to 0.6 times that of the fp32 instructions, 0.9 at most, on normal, on rectified and on positive
+// operands; an addition of 16 results per six products costs 4 to 8 per cent of the time.
 //
 // Infinities, NaNs and values within half a bfloat16 ulp of the largest float: a part that overflows makes products of
 // infinity with zero, so a result that comes out non-finite is computed again from the fp32 values (`redo`), term by term.
@@ -89,8 +98,8 @@ struct ScArgs {
   int pitch, slab;        // LDS row pitch and positions of the slab (rows * pitch)
   int total_pix, nchunks;
   // Workgroups [0, dp_tiles) take one whole tile each; workgroup dp_tiles + r * share + i takes part i of the chunks of tile
-  // dp_tiles + r.  A workgroup's slot of `partials` holds what it leaves for k_conv_split_fixup, or the first half of its sum.
-  int ctiles, dp_tiles, share, halves;
+  // dp_tiles + r.  Its slot of `partials` holds what it leaves for k_conv_split_fixup.
+  int ctiles, dp_tiles, share;
   int xcd_runs;
   unsigned in_bytes, wt_bytes;
 };
@@ -117,7 +126,7 @@ __device__ float redo(const ScArgs &a, int R, int c, int n, int h, int w, int ch
       const uint16_t *f = a.wt + (size_t((k / KC) * (R * R) + tap) * a.cblocks + c / 32) * (kFrag / 2) +
                           ((k % KC) / 8 * 32 + c % 32) * 8 + k % 8;
       const float w0 = lo_f(f[0]), w1 = lo_f(f[512]), w2 = lo_f(f[1024]);
-      s = __builtin_fmaf(x, w0 + w1 + w2, s);
+      s = __builtin_fmaf(x, tap & 1 ? -(w0 + w1 + w2) : w0 + w1 + w2, s);
     }
   return s;
 }
@@ -127,6 +136,7 @@ template <int GM, int WM, int WN, int ET, int R>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_split(ScArgs a) {
   constexpr int GN = NW / GM, BM = GM * WM * 32, BN = GN * WN * 32, TAPS = R * R, O = (R - 1) / 2;
   constexpr int AD = 2;                       // weight fragments: this tap's and the next one's
+  constexpr int EARLY = WN > 1 && ET > 3 ? 3 : ET;   // elements requested under the products (registers); the others after them
   extern __shared__ __align__(16) char smem[];
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave / GN, wn = wave % GN;
@@ -206,11 +216,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   };
 
   // operand fragment of block j at a tap
-  v4u b[WN][3];
+  v4u b[3];
   auto fragment = [&](int tap, int j) {
     const char *p = smem + boff[j] + tap / R * a.pitch * kPos + tap % R * kPos;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) b[j][k] = *reinterpret_cast<const v4u *>(p + k * 16);
+    for (int k = 0; k < 3; ++k) b[k] = *reinterpret_cast<const v4u *>(p + k * 16);
   };
 
   // Everything a tap needs is requested before the matrix instructions of an earlier one: weights two taps ahead, the next
@@ -222,55 +232,45 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   if (AD > 2) weights(wa[1], ch_begin * TAPS + 1);
   stage();
   __syncthreads();
-  // Where few workgroups leave each a long reduction, its first half goes through memory: the error of a sum grows with the
-  // square root of the roundings that its longest chain has, six per tap and chunk.
-  const int half_at = a.halves ? (ch_begin + ch_end) / 2 : ch_end;
-  const int slot = whole || a.halves ? int(blockIdx.x) : rest;
-  const rsrc_t rslot = make_rsrc(a.partials + size_t(slot) * (BM * BN), BM * BN * 4);
+  const rsrc_t rslot = make_rsrc(a.partials + size_t(whole ? 0 : rest) * (BM * BN), BM * BN * 4);
   const int slot_off = ((wm * WM * 32 + 4 * (lane >> 5)) * BN + wn * WN * 32 + l32) * 4;
   auto keep = [&](float r, int off, int row) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, r), rslot, off, row, 0);
   };
   auto slot_row = [](int i, int j, int v) { return ((i * 32 + 8 * (v >> 2) + (v & 3)) * BN + j * 32) * 4; };   // (scalar)
   for (int ch = ch_begin; ch < ch_end; ++ch) {
-    if (ch == half_at) {
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            keep(acc[i][j][v], slot_off, slot_row(i, j, v));
-            acc[i][j][v] = 0.f;
-          }
-    }
     const bool more = ch + 1 < ch_end;
-    if (WN > 1) fragment(0, 0);
+    fragment(0, 0);
 #pragma unroll
     for (int tap = 0; tap < TAPS; ++tap) {
       const v4u(&w)[WM][3] = wa[tap % AD];
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
         if (j == 0) weights(wa[(tap + AD - 1) % AD], ch * TAPS + tap + AD - 1);
-        if (j == WN - 1 && tap < ET) load(ch + 1, tap, more ? a.K : 0);
-        if (WN == 1) fragment(tap, 0);
-        else if (j + 1 < WN) fragment(tap, j + 1);
-        else if (tap + 1 < TAPS) fragment(tap + 1, 0);
+        if (j == WN - 1 && tap < EARLY) load(ch + 1, tap, more ? a.K : 0);
         constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};   // small products first
+        v16f sum[WM];
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) sum[i][v] = 0.f;
 #pragma unroll
         for (int k = 0; k < 6; ++k)
 #pragma unroll
-          for (int i = 0; i < WM; ++i) acc[i][j] = mfma(w[i][PA[k]], b[j][PB[k]], acc[i][j]);
+          for (int i = 0; i < WM; ++i) sum[i] = mfma(w[i][PA[k]], b[PB[k]], sum[i]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + 1 < WN) fragment(tap, j + 1);
+        else if (tap + 1 < TAPS) fragment(tap + 1, 0);
 #pragma unroll
-        for (int k = 0; k < 6 * WM; ++k) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x006, 4, 0);
-          __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        for (int i = 0; i < WM; ++i) {
+          acc[i][j] = tap % 2 ? acc[i][j] - sum[i] : acc[i][j] + sum[i];
+          asm volatile("" : "+v"(acc[i][j]));   // (here, not when all taps' sums are there)
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+#pragma unroll
+    for (int e = EARLY; e < ET; ++e) load(ch + 1, e, more ? a.K : 0);
     if (TAPS % AD) {   // (the ring continues one place further)
       static_assert(TAPS % AD == 0 || TAPS % AD == 1, "ring of the weight fragments");
 #pragma unroll
@@ -292,15 +292,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 
   // ---- store: this lane holds column l32 and rows 8 (v / 4) + 4 (lane / 32) + v % 4 of every 32 x 32 block
   const int lhalf = lane >> 5;
-  if (half_at < ch_end) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          acc[i][j][v] += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rslot, slot_off, slot_row(i, j, v), 0));
-  }
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < WM; ++i)
@@ -349,7 +340,7 @@ __global__ __launch_bounds__(256) void k_conv_split_fixup(ScArgs a, int BM, int 
   const int tile = a.dp_tiles + r, c0 = (tile % a.ctiles) * BM, pix0 = (tile / a.ctiles) * BN, PQ = a.P * a.Q;
   const int m = int(blockIdx.y * 256 + threadIdx.x) / TPR, col = int(threadIdx.x) % TPR * 4, c = c0 + m;
   if (c >= a.C) return;
-  const float *p = a.partials + (size_t(r) * a.share + (a.halves ? a.dp_tiles : 0)) * BM * BN + m * BN + col;
+  const float *p = a.partials + size_t(r) * a.share * BM * BN + m * BN + col;
   v4f s = *reinterpret_cast<const v4f *>(p);
   for (int i = 1; i < a.share; ++i) s += *reinterpret_cast<const v4f *>(p + size_t(i) * BM * BN);
   const float bb = a.bias ? a.bias[c] : 0.f;
@@ -372,7 +363,6 @@ struct ScPlan {
   bool ok;
   int r, gm, wm, wn, et, bm, bn, pitch, rows, slab, nchunks, cblocks;
   int ctiles, tiles, dp_tiles, share, wgs;
-  bool halves;
 };
 
 ScPlan plan(const sgh_conv_geom *g) {
@@ -426,9 +416,6 @@ ScPlan plan(const sgh_conv_geom *g) {
   if (p.share > p.nchunks) p.share = p.nchunks;
   if (p.share <= 1) p.share = 1, p.dp_tiles = p.tiles;
   p.wgs = p.dp_tiles + (p.tiles - p.dp_tiles) * p.share;
-  // (both halves through memory: 256 channels of 14 x 14, N = 64, error against float64 7.2e-7 -> 5.1e-7 of the result; with
-  // more workgroups than this the fp32 matrix instructions sum in one chain as well, and theirs is the larger error)
-  p.halves = p.wgs <= 2 * cus && p.nchunks / p.share >= 3;
   p.ok = true;
   return p;
 }
@@ -468,8 +455,7 @@ size_t sgh_conv_split_weight_bytes(const sgh_conv_geom *g) {
 
 size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g) {
   const ScPlan p = plan(g);
-  const int slots = p.halves ? p.wgs : p.wgs - p.dp_tiles;
-  return p.ok ? align256(sgh_conv_split_weight_bytes(g)) + size_t(slots) * p.bm * p.bn * sizeof(float) : 0;
+  return p.ok ? align256(sgh_conv_split_weight_bytes(g)) + size_t(p.wgs - p.dp_tiles) * p.bm * p.bn * sizeof(float) : 0;
 }
 
 int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps) {
@@ -504,7 +490,7 @@ int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, float *out, void
   a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
   a.cblocks = p.cblocks, a.pitch = p.pitch, a.slab = p.slab;
   a.total_pix = g->N * g->P * g->Q, a.nchunks = p.nchunks;
-  a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share, a.halves = p.halves;
+  a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share;
   a.xcd_runs = p.dp_tiles % 64 == 0 && !sgh_env().conv_xcd_off;
   a.in_bytes = unsigned(size_t(g->N) * g->K * g->P * g->Q * 4);
   a.wt_bytes = unsigned(sgh_conv_split_weight_bytes(g));
