@@ -16,10 +16,10 @@
 //
 // The sums of the workgroups of a (k, c) tile are added in ascending order by k_wgrad_oct_reduce.
 //
-// 64 images, with the reduction, k_wgrad3x3 before and this: 64 channels of 56 x 56 164 -> 103 us, 128 of 28 x 28 146 -> 104,
-// 256 of 14 x 14 146 -> 97, 512 of 7 x 7 143 -> 101; 130 drawn layers 1.5 times as fast, 0.9 times the error against float64.
-// The matrix instructions are busy for 62 per cent of the cycles and the clock falls to 1.8 GHz under them: letting the groups take
-// turns, one multiplying while the other stages, gave 1 to 3 per cent and spilled the rows of three octets.
+// 64 images, whole calls, k_wgrad3x3 and this: 64 channels of 56 x 56 153 -> 105 us, 128 of 28 x 28 133 -> 102, 256 of 14 x 14
+// 134 -> 101, 512 of 7 x 7 137 -> 108, with 0.25 to 0.75 times the error against float64.  A tap's six products are summed on their
+// own and added to the accumulator once; without that the error is up to 1.5 times that of the fp32 instructions behind a
+// ReLU (whose zeros cost those no rounding), and the kernel 7 per cent faster.
 #include "common.h"
 
 namespace {
@@ -34,7 +34,6 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr int NT = 512, GT = 256;   // threads of a workgroup, of a group
 constexpr int PARTS = 3;
 constexpr int kOOB = int(0x80000000u);
-constexpr int kChain = 400;          // roundings of an accumulator (plan)
 constexpr int kAcc = 9 * 16 * 64;   // accumulators of a wavefront
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
@@ -217,9 +216,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       step_row(en[e], ep[e]);
     }
   };
-  // The second group sums -dy x: the accumulating instructions round towards minus infinity on average, by 2^-26 of the sum,
-  // which over hundreds of partial sums would outweigh their random errors (64 channels of 56 x 56, N = 64: 6.0e-7 from float64
-  // with one sign, 3.2e-7 with two)
+  // Every other step's dy is negated, and the other ones in the second group, and what they give is subtracted: the matrix
+  // instructions round towards minus infinity on average, which adds up over a sum (1024 channels of 14 x 14, forward pass:
+  // 2e-7 of the mean magnitude with one sign, 2e-8 with two)
   const unsigned sign = group ? 0x80008000u : 0u;
   auto slot_of = [](int base, int j) { return base + j < RING ? base + j : base + j - RING; };
   auto stage = [&](int base) {   // base: the ring slot of row v0 - 1
@@ -230,7 +229,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       sd[e].parts(part);
       if (OPI * 64 % GT == 0 || ch < 64) {
 #pragma unroll
-        for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + ch) * 16) = part[j] ^ sign;
+        for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + ch) * 16) = part[j] ^ (o & 2 ? ~sign & 0x80008000u : sign);
         put_x(sx[e], slot_of(base, 2 + o / OCS), ch, o % OCS);
       }
     }
@@ -278,12 +277,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         v4u d;
         unsigned l, r;
       };
-      // unit u = (step, row r, part): the octet and its neighbours; a unit's are read while the one before is multiplied
-      constexpr int UNITS = OPI / 2 * 3 * PARTS;
-      constexpr int ORDER[PARTS] = {0, 2, 1};   // (nine, three, six products)
-      auto read = [&](int u) {
-        const int s = u / (3 * PARTS), r = u / PARTS % 3, p = ORDER[u % PARTS];
-        const int oa = 2 * s, ob = 2 * s + 1;
+      // unit u = (step, row r of the filter): the three parts of the octet and its neighbours, three taps.  A tap's six products
+      // are summed on their own, the small ones first, and the sum is added to the accumulator: one rounding there for 16
+      // pixels instead of six or more.  A part of the next unit is read as soon as the last tap has taken its own.
+      constexpr int UNITS = OPI / 2 * 3;
+      auto read = [&](int u, int p) {
+        const int s = u / 3, r = u % 3, oa = 2 * s, ob = 2 * s + 1;
         const int ja = slot_of(base, oa / OCS + r) * S::XROW + oa % OCS * 16;
         const int jb = slot_of(base, ob / OCS + r) * S::XROW + ob % OCS * 16;
         const char *at = xb + (half ? jb : ja) + p * S::XPART;
@@ -293,31 +292,43 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         w.r = *reinterpret_cast<const unsigned *>(at + 20);
         return w;
       };
-      v4u A[2][PARTS];
+      v4u A[PARTS];
       auto read_a = [&](int s) {
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) A[s & 1][p] = *reinterpret_cast<const v4u *>(da + 2 * s * S::DYO + p * 1024);
+        for (int p = PARTS - 1; p >= 0; --p) A[p] = *reinterpret_cast<const v4u *>(da + 2 * s * S::DYO + p * 1024);
       };
+      Raw w[PARTS];
       read_a(0);
-      Raw next = read(0);
+#pragma unroll
+      for (int p = PARTS - 1; p >= 0; --p) w[p] = read(0, p);
 #pragma unroll
       for (int u = 0; u < UNITS; ++u) {
-        const int s = u / (3 * PARTS), r = u / PARTS % 3, p = ORDER[u % PARTS];
-        const Raw w = next;
-        if (u + 1 < UNITS) next = read(u + 1);
-        if (u % (3 * PARTS) == 0 && s + 1 < OPI / 2) read_a(s + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        v4u sh[3];
-        sh[1] = w.d;
-        const unsigned m1 = __builtin_amdgcn_alignbit(w.d[1], w.d[0], 16), m2 = __builtin_amdgcn_alignbit(w.d[2], w.d[1], 16),
-                       m3 = __builtin_amdgcn_alignbit(w.d[3], w.d[2], 16);
-        sh[0] = v4u{__builtin_amdgcn_alignbit(w.d[0], w.l, 16), m1, m2, m3};
-        sh[2] = v4u{m1, m2, m3, __builtin_amdgcn_alignbit(w.r, w.d[3], 16)};
+        const int s = u / 3, r = u % 3;
 #pragma unroll
-        for (int q = PARTS - 1 - p; q >= 0; --q)
+        for (int c = 0; c < 3; ++c) {
+          v16f sum;
 #pragma unroll
-          for (int c = 0; c < 3; ++c) acc[r * 3 + c] = mfma(A[s & 1][q], sh[c], acc[r * 3 + c]);
-        __builtin_amdgcn_sched_barrier(0);
+          for (int v = 0; v < 16; ++v) sum[v] = 0.f;
+#pragma unroll
+          for (int p = PARTS - 1; p >= 0; --p) {
+            const v4u d = w[p].d;
+            v4u x = d;
+            if (c != 1) {
+              const unsigned m1 = __builtin_amdgcn_alignbit(d[1], d[0], 16), m2 = __builtin_amdgcn_alignbit(d[2], d[1], 16),
+                             m3 = __builtin_amdgcn_alignbit(d[3], d[2], 16);
+              if (c == 0) x = v4u{__builtin_amdgcn_alignbit(d[0], w[p].l, 16), m1, m2, m3};
+              else x = v4u{m1, m2, m3, __builtin_amdgcn_alignbit(w[p].r, d[3], 16)};
+            }
+            if (c == 2 && u + 1 < UNITS) w[p] = read(u + 1, p);
+#pragma unroll
+            for (int q = PARTS - 1 - p; q >= 0; --q) sum = mfma(A[q], x, sum);
+          }
+          if (r == 2 && c == 2 && s + 1 < OPI / 2) read_a(s + 1);
+          v16f &total = acc[r * 3 + c];
+          total = s % 2 ? total - sum : total + sum;
+          asm volatile("" : "+v"(total));   // (here, not when all taps' sums are there)
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
     __syncthreads();
@@ -415,6 +426,7 @@ WoPlan plan(const sgh_conv_geom *g) {
   const int oc = (g->Q + 7) / 8;
   p.strips = (oc + 3) / 4;
   p.ocs = (oc + p.strips - 1) / p.strips;
+  if (p.ocs == 3) p.ocs = 4;   // (two rows of three octets do not fit the registers: 64 images, 96 channels of 20 x 22 109 against 102 us)
   p.rpi = p.ocs == 4 ? 1 : p.ocs == 1 ? 4 : 2;
   if (g->P + 1 < p.rpi || size_t(g->N) * (g->P + 1) >= (size_t(1) << 30)) return p;
   p.iters = int((size_t(g->N) * (g->P + 1) + p.rpi - 1) / p.rpi);
@@ -423,16 +435,12 @@ WoPlan plan(const sgh_conv_geom *g) {
   if (tiles > 65536) return p;
   p.tiles = int(tiles);
   const int cus = sgh_num_cus();
-  // One workgroup per CU; more rounds of them where an accumulator would take more than kChain products' roundings (the error of
-  // a chain grows with its square root: 14 images of 154 and 670 channels, 37 x 27, 5.1e-7 from float64 in one round).
-  const long most = p.iters / 4 > 0 ? p.iters / 4 : 1;   // (two iterations for either group)
-  for (long rounds = 1;; ++rounds) {
-    long sp = rounds * cus / (tiles * p.strips);
-    if (sp > most) sp = most;
-    if (sp < 1) sp = 1;
-    p.per_split = int((p.iters + sp - 1) / sp);
-    if (sp == most || rounds == 8 || (p.per_split + 1) / 2 * (p.ocs * p.rpi / 2) * 6 <= kChain) break;
-  }
+  // one workgroup per CU, two iterations at least for either of its groups
+  const long most = p.iters / 4 > 0 ? p.iters / 4 : 1;
+  long sp = cus / (tiles * p.strips);
+  if (sp > most) sp = most;
+  if (sp < 1) sp = 1;
+  p.per_split = int((p.iters + sp - 1) / sp);
   p.splits = (p.iters + p.per_split - 1) / p.per_split * p.strips;
   p.ok = true;
   return p;
@@ -470,7 +478,6 @@ int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, f
   a.dy_bytes = unsigned(pixels * g->K * 4), a.x_bytes = unsigned(pixels * g->C * 4);
   sgh_prof_kernel_begin("conv_wgrad/k_wgrad_oct", 2.0 * pixels * g->K * g->C * 9);
   const int rc = p.ocs == 4   ? launch<4, 1>(a, s)
-                 : p.ocs == 3 ? launch<3, 2>(a, s)
                  : p.ocs == 2 ? launch<2, 2>(a, s)
                               : launch<1, 4>(a, s);
   sgh_prof_kernel_end(s);

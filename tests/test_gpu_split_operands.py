@@ -94,3 +94,31 @@ def test_conv_split_error_of_an_fp32_chain(singa, dev, n, c, h, w, k, r, kind):
     for got, (want, chain) in ((fwd[0], conv64(x, W)), (dgrad[0], conv64(dy, Wt))):
         print(kind, "error %.2e, of a chain %.2e" % (nl2(got, want), nl2(chain, want)))
         assert nl2(got, want) < 0.45 * nl2(chain, want)
+
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive"])
+@pytest.mark.parametrize("n,c,h,w,k", [(20, 512, 7, 7, 200), (13, 256, 10, 10, 256), (20, 100, 21, 20, 260), (8, 128, 25, 29, 140), (6, 64, 48, 40, 180)])
+def test_conv_wgrad_octets_error_of_fp32_chains(singa, dev, n, c, h, w, k, kind):
+    """The same for the weight gradient, whose pixels are summed in twice as many stretches as there are partial images (one per
+    CU): against chains of fp32 multiply-adds over as many stretches, on the first filters and channels."""
+    import torch
+    x, W, dy = operands(kind, n + c + k, n, c, h, w, k, 3)
+    got, names = passes(singa, dev, x, W, dy)[2]
+    assert names == {"k_wgrad_oct"}
+    few = 16
+    strips = (w + 31) // 32
+    stretches = 2 * (256 // (((k + 63) // 64) * ((c + 63) // 64) * strips))
+    xp = torch.nn.functional.pad(torch.from_numpy(x[:, :few]), (1, 1, 1, 1))
+    taps = torch.stack([xp[:, :, i:i + h, j:j + w].permute(1, 0, 2, 3).reshape(few, -1) for i in range(3) for j in range(3)], 1)
+    d = torch.from_numpy(dy[:, :few]).permute(1, 0, 2, 3).reshape(few, -1)
+    want = torch.einsum("kp,ctp->kct", d.double(), taps.double()).reshape(few, few, 3, 3).numpy()
+    length = -(-d.shape[1] // stretches)
+    total = torch.zeros(few, few, 9, dtype=torch.float64)
+    pad = stretches * length - d.shape[1]
+    d, taps = (torch.nn.functional.pad(t, (0, pad)).unflatten(-1, (stretches, length)) for t in (d, taps))
+    acc = torch.zeros(few, few, 9, stretches)
+    for i in range(length):
+        acc = fma32(acc, d[:, None, None, :, i], taps[None, :, :, :, i])
+    chain = acc.double().sum(-1).float().reshape(few, few, 3, 3).numpy()
+    mine = got[:few, :few]
+    print(kind, "error %.2e, of chains %.2e" % (nl2(mine, want), nl2(chain, want)))
+    assert nl2(mine, want) < nl2(chain, want)   # (short chains: the rounding of the result is most of either error)
