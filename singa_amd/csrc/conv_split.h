@@ -11,8 +11,9 @@ size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g);   // weight fragm
 int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspace, bool dgrad, hipStream_t s);
 // the same as a batch item: workgroups of sgh_conv_split_weights_block
 int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps);
-int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, float *out, void *workspace, hipStream_t s, const char *tag,
-                       bool dgrad, const float *bias, bool accumulate);
+// `W`: the same weights again, for what the fragments cannot hold
+int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s,
+                       const char *tag, bool dgrad, const float *bias, bool accumulate);
 
 constexpr int kSplitWeightLds = 512 * 9;   // floats of LDS that a workgroup below needs
 

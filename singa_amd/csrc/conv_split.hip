@@ -5,7 +5,7 @@
 //   x = x0 + x1 + x2,   x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)      (8 + 8 + 8 bits of significand)
 //
 // and a product of two of them is the sum of nine exact products, of which the six with weights down to 2^-16 are formed
-// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0).  The three left out come to 2^-24 of the product at most, 2^-29 in the mean.
+// (x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0).  The three left out come to 2^-24 of the product at most, 2^-28 in the mean.
 // v_mfma_f32_32x32x16_bf16 multiplies 16 x as much per cycle as v_mfma_f32_32x32x2_f32, so six of them are 2.67 times as
 // fast, with fp32 accumulators either way.
 //
@@ -37,7 +37,8 @@
 // operands; an addition of 16 results per six products costs 4 to 8 per cent of the time.
 //
 // Infinities, NaNs and values within half a bfloat16 ulp of the largest float: a part that overflows makes products of
-// infinity with zero, so a result that comes out non-finite is computed again from the fp32 values (`redo`), term by term.
+// infinity with zero, so a tile with a result that comes out non-finite is formed again by its workgroup on the fp32 matrix
+// instructions, whatever the values are.
 #include "common.h"
 #include "conv_split.h"
 
@@ -87,6 +88,8 @@ __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __
 
 struct ScArgs {
   const float *in;
+  const float *W;         // the weights, W[c * w_c + k * w_k + tap]; the data gradient takes the taps in reverse
+  int w_c, w_k;
   const uint16_t *wt;     // weight fragments [chunk][tap][32-row block][part][lane][8]
   const float *bias;      // per output channel (NULL: none)
   float *out;
@@ -108,27 +111,6 @@ __device__ __forceinline__ int whole_tile_of(const ScArgs &a, int w) {   // see 
   if (!a.xcd_runs) return w;
   const int x = w & 7, j = w >> 3;
   return (((j >> 3) << 3) + x) * 8 + (j & 7);
-}
-
-// One result from the fp32 values: channel c at (n, h, w), chunks [ch0, ch1).  Taps in the padding multiply a zero in the
-// forward pass (which makes a NaN of an infinite weight) and do not exist in the data gradient.
-// A NaN of the input makes one of every channel's result there: `nan_in` tells the caller, which need not look for it again.
-__device__ float redo(const ScArgs &a, int R, int c, int n, int h, int w, int ch0, int ch1, bool &nan_in) {
-  const int o = (R - 1) / 2, k1 = min(a.K, ch1 * KC);
-  float s = 0.f;
-  for (int k = ch0 * KC; k < k1 && s == s; ++k)   // (a NaN stays one)
-    for (int tap = 0; tap < R * R && s == s; ++tap) {
-      const int hh = h + tap / R - o, ww = w + tap % R - o;
-      const bool in = unsigned(hh) < unsigned(a.P) && unsigned(ww) < unsigned(a.Q);
-      if (!in && a.dgrad) continue;
-      const float x = in ? a.in[((size_t(n) * a.K + k) * a.P + hh) * a.Q + ww] : 0.f;
-      nan_in |= x != x;
-      const uint16_t *f = a.wt + (size_t((k / KC) * (R * R) + tap) * a.cblocks + c / 32) * (kFrag / 2) +
-                          ((k % KC) / 8 * 32 + c % 32) * 8 + k % 8;
-      const float w0 = lo_f(f[0]), w1 = lo_f(f[512]), w2 = lo_f(f[1024]);
-      s = __builtin_fmaf(x, tap & 1 ? -(w0 + w1 + w2) : w0 + w1 + w2, s);
-    }
-  return s;
 }
 
 // GM x (NW / GM) wavefronts, each on WM x WN blocks of 32 x 32; ET: slab elements (octet, position) per thread; R: filter size.
@@ -306,32 +288,103 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     if (a.bias) r += a.bias[c];
     *o = a.accumulate ? *o + r : r;
   };
-  const bool redone = __any(bad);
+  // (the slab is free after the last chunk's barrier)
+  int *const again = reinterpret_cast<int *>(smem);
+  if (t == 0) *again = 0;
+  __syncthreads();
+  if (__any(bad) && lane == 0) *again = 1;
+  __syncthreads();
+  if (*again) {
+    // The tile from the fp32 values, on the fp32 instructions: the slab as [channel][position], the weights from where they are,
+    // step k of a tap over channels k and 8 + k.  Taps in the padding multiply a zero in the forward pass (which makes a NaN of an
+    // infinite weight) and do not exist in the data gradient, where an infinite or NaN weight is multiplied pixel by pixel.
+    // (Everything is derived anew from opaque copies: what the loop above holds in registers for this, it spills.)
+    static_assert(WM == 1, "");
+    float *const xs = reinterpret_cast<float *>(smem);
+    int tt = threadIdx.x, P = a.P, Q = a.Q, slab = a.slab, pitch = a.pitch;
+    asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q), "+s"(slab), "+s"(pitch));
+    const int half = tt >> 5 & 1, column = tt & 31, c = min(c0 + wm * 32 + column, a.C - 1), vh = P + 2 * O;
+    int ph[WN], pw[WN], base[WN];   // this lane's pixels: row, column, place in the slab of channel 8 half
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int pix = min(pix0 + (wn * WN + j) * 32 + column, a.total_pix - 1), n = pix / (P * Q), rem = pix - n * P * Q;
+      ph[j] = rem / Q, pw[j] = rem - ph[j] * Q;
+      base[j] = (n * vh + ph[j] - vbase) * pitch + pw[j] + half * 8 * slab;
+    }
+    bool number = true;   // not every result of this wavefront is a NaN yet (in a diverged network they soon are)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[0][j][v] = 0.f;
+    for (int ch = ch_begin; ch < ch_end; ++ch) {
+      __syncthreads();
+#pragma unroll 1
+      for (int i = tt; i < 2 * slab; i += NT) {
+        const int oct = i >= slab, pos = i - (oct ? slab : 0), vr = pos / pitch, q = pos - vr * pitch - O, v = vbase + vr, n = v / vh;
+        const int p = v - n * vh - O, k0 = ch * KC + oct * 8;
+        const bool in = n < a.N && unsigned(p) < unsigned(P) && unsigned(q) < unsigned(Q);
+        const float *const src = a.in + ((size_t(n) * a.K + k0) * P + p) * Q + q;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) xs[(oct * 8 + k) * slab + pos] = in && k0 + k < a.K ? src[size_t(k) * P * Q] : 0.f;
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int i = 0; i < TAPS && number; ++i) {
+        // (the middle tap first: it is inside the image everywhere, so a layer of NaN weights ends here)
+        const int tap = (i + TAPS / 2) % TAPS;
+        const bool apart = a.dgrad && i;
+        const float *const wp = a.W + size_t(c) * a.w_c + (a.dgrad ? TAPS - 1 - tap : tap);
+        const int k0 = ch * KC + half * 8;
+        float w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = k0 + k < a.K ? wp[size_t(k0 + k) * a.w_k] : 0.f;
+        const float *const xt = xs + tap / R * pitch + tap % R;
+        if (apart) {
+#pragma unroll 1
+          for (int k = 0; k < 8; ++k) {
+            float wk = w[0];
+#pragma unroll
+            for (int u = 1; u < 8; ++u) wk = k == u ? w[u] : wk;
+            for (unsigned long long m = __ballot(!finite(wk)); m; m &= m - 1) {
+              const int from = __builtin_ctzll(m), row = from & 31;
+              const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wk), from));
+#pragma unroll
+              for (int j = 0; j < WN; ++j) {
+                const bool in = unsigned(ph[j] + tap / R - O) < unsigned(P) && unsigned(pw[j] + tap % R - O) < unsigned(Q);
+                const float x = xt[base[j] + ((from >> 5) - half) * 8 * slab + k * slab];
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                  if (v == (row >> 3) * 4 + (row & 3) && in && half == (row >> 2 & 1)) acc[0][j][v] = __builtin_fmaf(f, x, acc[0][j][v]);
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const float f = apart && !finite(w[k]) ? 0.f : w[k];
+#pragma unroll
+          for (int j = 0; j < WN; ++j)
+            acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f, xt[base[j] + k * slab], acc[0][j], 0, 0, 0);
+        }
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) any |= acc[0][j][v] == acc[0][j][v];
+        number = __any(any);
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      unsigned mask = 0;
+    for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int m = (wm * WM + i) * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3), col = (wn * WN + j) * 32 + l32;
-        if (redone && !finite(acc[i][j][v])) mask |= 1u << v;
-        else if (whole) put(m, col, pixn[j], acc[i][j][v]);
+        if (whole) put(m, col, pixn[j], acc[i][j][v]);
         else keep(acc[i][j][v], slot_off, slot_row(i, j, v));
       }
-      if (redone) {
-        bool nan_in = false;
-        for (; mask; mask &= mask - 1) {
-          const int v = __builtin_ctz(mask);
-          const int m = (wm * WM + i) * 32 + 8 * (v >> 2) + 4 * lhalf + (v & 3), col = (wn * WN + j) * 32 + l32;
-          if (c0 + m >= a.C || pix0 + col >= a.total_pix) continue;
-          const int rem = pix0 + col - pixn[j] * PQ, h = rem / a.Q;
-          const float r = nan_in ? __builtin_nanf("") : redo(a, R, c0 + m, pixn[j], h, rem - h * a.Q, ch_begin, ch_end, nan_in);
-          if (whole) put(m, col, pixn[j], r);
-          else keep(r, (m * BN + col) * 4, 0);
-        }
-      }
-    }
 }
 
 // Sums the parts of the tiles that several workgroups shared, in ascending chunk order: the result does not depend on timing
@@ -475,12 +528,14 @@ int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspa
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 
-int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, float *out, void *workspace, hipStream_t s, const char *tag,
+int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s, const char *tag,
                        bool dgrad, const float *bias, bool accumulate) {
   const ScPlan p = plan(g);
   if (!p.ok) return SGH_EUNSUPPORTED;
   ScArgs a;
   a.in = in;
+  a.W = W;
+  a.w_c = (dgrad ? 1 : g->K) * p.r * p.r, a.w_k = (dgrad ? g->C : 1) * p.r * p.r;
   a.wt = static_cast<const uint16_t *>(workspace);
   a.bias = bias;
   a.out = out;

@@ -1117,7 +1117,7 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
     }
   } else if (dgrad_splits(g, ws_bytes)) {
     if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
-    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
+    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
   } else if (path == kDgradColumns) {
     float *dcol = static_cast<float *>(workspace);
     const int CRS = g->C * RS, Ncols = g->N * g->P * g->Q;
@@ -1448,7 +1448,7 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
   sgh_conv_geom gt;
   if (fwd_as_split(g, &gt) && ws_bytes >= sgh_conv_split_workspace_bytes(&gt)) {
     int rcs = sgh_conv_split_weights(&gt, W, workspace, false, s);
-    if (rcs == SGH_OK) rcs = sgh_conv_split_run(&gt, x, y, workspace, s, "conv_fwd/k_conv_split", false, bias, false);
+    if (rcs == SGH_OK) rcs = sgh_conv_split_run(&gt, x, W, y, workspace, s, "conv_fwd/k_conv_split", false, bias, false);
     sgh_prof_stop(s);
     return rcs;
   }

@@ -122,3 +122,76 @@ def test_conv_wgrad_octets_error_of_fp32_chains(singa, dev, n, c, h, w, k, kind)
     mine = got[:few, :few]
     print(kind, "error %.2e, of chains %.2e" % (nl2(mine, want), nl2(chain, want)))
     assert nl2(mine, want) < nl2(chain, want)   # (short chains: the rounding of the result is most of either error)
+
+
+def seconds(dev, call):
+    """The least of three runs of `call` on an idle device"""
+    import time
+    call()
+    best = 1e9
+    for _ in range(3):
+        dev.Sync()
+        t = time.perf_counter()
+        call()
+        dev.Sync()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan", "nan weights", "inf weights"])
+def test_conv_split_time_of_non_finite_operands(singa, dev, what):
+    """Results that are not finite take a second pass over their tile on the fp32 instructions, 2.7 times the first one, and no search
+    per result: eight times the time of ordinary operands at most (a term-by-term search took 100 to 250 times)."""
+    n, c, h, w, k = 32, 256, 14, 14, 256
+    x, W, dy = operands("normal", 3, n, c, h, w, k, 3)
+
+    def times(x, W, dy):
+        xd, wd, dyd = (singa.from_numpy(a, dev) for a in (x, W, dy))
+        hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, False)
+        return seconds(dev, lambda: singa.GpuConvForward(xd, wd, None, hd)), seconds(dev, lambda: singa.GpuConvBackwardx(dyd, wd, xd, hd))
+
+    plain = times(x, W, dy)
+    value = np.float32(np.nan if "nan" in what else np.inf)
+    if what == "one inf":
+        x[:, 0, 7, 7] = value
+        dy[:, 0, 7, 7] = value
+    elif what == "overflow":
+        x, W, dy = x * np.float32(1e30), W * np.float32(1e10), dy * np.float32(1e30)
+    elif "weights" in what:
+        W[:] = value
+    else:
+        x[:] = value
+        dy[:] = value
+    for got, ordinary in zip(times(x, W, dy), plain):
+        print(what, "%.1f us, ordinary operands %.1f" % (got * 1e6, ordinary * 1e6))
+        assert got < 8 * ordinary
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r", [(2, 24, 9, 10, 40, 3), (1, 300, 6, 6, 130, 3), (30, 64, 20, 20, 64, 3), (2, 20, 9, 7, 40, 5)])
+@pytest.mark.parametrize("where", ["x", "w", "both"])
+def test_conv_split_infinities_and_nans(singa, dev, n, c, h, w, k, r, where):
+    """+inf, -inf and NaN reach exactly the results that their products reach, with the sign that those have, and the finite
+    results next to them stay what they were; an infinite weight meets the padding in the forward pass (a NaN) and not in the
+    data gradient."""
+    import torch
+    x, W, dy = operands("normal", 11, n, c, h, w, k, r)
+    if where != "w":
+        for t in (x, dy):
+            t[0, 1, 0, w - 1], t[-1, 2, h // 2, 1], t[0, 3, h - 1, 0] = -np.inf, np.inf, np.nan
+    if where != "x":
+        W[k - 1, c // 3, r // 2, 0], W[0, 0, 0, 0], W[k // 2, c - 1, r - 1, r - 1], W[1, 1, r // 2, r // 2] = -np.inf, np.inf, np.nan, -np.inf
+    fwd, dgrad, _ = passes(singa, dev, x, W, dy)
+    with np.errstate(all="ignore"):
+        t = lambda a: torch.from_numpy(a.astype(np.float64))
+        xp = torch.nn.functional.pad(t(x), (r // 2,) * 4)
+        want = [sum(torch.einsum("kc,nchw->nkhw", t(W[:, :, i, j].copy()), xp[:, :, i:i + h, j:j + w]) for i in range(r) for j in range(r))]
+        dx = torch.zeros(n, c, h + r - 1, w + r - 1, dtype=torch.float64)
+        for i in range(r):
+            for j in range(r):
+                dx[:, :, i:i + h, j:j + w] += torch.einsum("kc,nkhw->nchw", t(W[:, :, i, j].copy()), t(dy))
+        want.append(dx[:, :, r // 2:r // 2 + h, r // 2:r // 2 + w])
+    for (got, _), ref in zip((fwd, dgrad), (a.numpy().astype(np.float32) for a in want)):
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
+        fin = np.isfinite(ref)
+        np.testing.assert_allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
