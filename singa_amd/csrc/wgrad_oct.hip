@@ -92,27 +92,6 @@ struct Octet {
   }
 };
 
-// One sum term by term: virtual rows [v0, v1), columns [q0, q1).  A NaN of dy makes one of the filter's sums of every tap and
-// channel, a NaN of x of every filter's at this tap and channel; `seen` tells the caller (bit 0: dy, bit 1: x), which need not
-// look for it again (a diverged network has little else: 144 searches a lane took 0.8 ms)
-__device__ float redo(const WoArgs &a, int k, int c, int tap, int v0, int v1, int q0, int q1, unsigned &seen) {
-  float sum = 0.f;
-  for (int v = v0; v < v1 && sum == sum; ++v) {
-    const int n = v / (a.P + 1), p = v - n * (a.P + 1);
-    if (p >= a.P || n >= a.N) continue;
-    const int h = p + tap / 3 - 1;
-    for (int q = q0; q < q1 && sum == sum; ++q) {
-      const int w = q + tap % 3 - 1;
-      const bool in = unsigned(h) < unsigned(a.P) && unsigned(w) < unsigned(a.Q);
-      const float xv = in ? a.x[((size_t(n) * a.C + c) * a.P + h) * a.Q + w] : 0.f;
-      const float d = a.dy[((size_t(n) * a.K + k) * a.P + p) * a.Q + q];
-      seen |= (d != d ? 1u : 0u) | (xv != xv ? 2u : 0u);
-      sum = __builtin_fmaf(d, xv, sum);
-    }
-  }
-  return sum;
-}
-
 template <int OCS, int RPI>
 struct Shape {
   static constexpr int OPI = OCS * RPI, RING = RPI + 2;
@@ -339,6 +318,81 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
   }
 
+  // ---- sums that are not finite: an infinity or a value near the largest float has parts whose products are NaN, and a zero of
+  // the virtual rows and columns has met one.  All of the workgroup's sums are formed again on the fp32 instructions, a row at a
+  // time, whatever the values are: 2.7 times the products' time.  (LDS is free.  Everything is derived anew from opaque copies:
+  // what the loop above holds in registers for this, it spills.)
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][v]);
+  int *const again = reinterpret_cast<int *>(smem);
+  if (t == 0) *again = 0;
+  __syncthreads();
+  if (__any(bad) && lane == 0) *again = 1;
+  __syncthreads();
+  if (*again) {
+    constexpr int COLS = 8 * OCS, YP = COLS + 1, XW = COLS + 2, XF = COLS + 3;   // odd pitches
+    static_assert((64 * YP + 192 * XF) * 4 <= S::GROUP, "");
+    int tt = threadIdx.x, P = a.P, Q = a.Q;
+    asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q));
+    const int th = tt >> 5 & 1, row = wm * 32 + (tt & 31), col = wn * 32 + (tt & 31);
+    float *const ys = reinterpret_cast<float *>(smem + group * S::GROUP), *const xr = ys + 64 * YP;
+    unsigned valid = 0;   // accumulator registers that hold a filter
+#pragma unroll
+    for (int v = 0; v < 16; ++v) valid |= unsigned(k0 + wm * 32 + 8 * (v >> 2) + 4 * th + (v & 3) < a.K && c0 + col < a.C) << v;
+    bool number = true;   // not every sum of this wavefront is a NaN yet (in a diverged network they soon are)
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+    for (int i = 0; i < mine * RPI; ++i) {
+      const int v = it0 * RPI + i, n = v / (P + 1), p = v - n * (P + 1);
+      const bool live = v < it1 * RPI && n < a.N && p < P;
+      __syncthreads();
+      if (live) {
+        for (int e = tt & (GT - 1); e < 64 * COLS; e += GT) {
+          const int ch = e / COLS, q = e % COLS;
+          ys[ch * YP + q] = k0 + ch < a.K && q0 + q < Q ? a.dy[((n * a.K + k0 + ch) * P + p) * Q + q0 + q] : 0.f;
+        }
+        for (int e = tt & (GT - 1); e < 192 * XW; e += GT) {
+          const int ch = e / XW % 64, h = p + e / (XW * 64) - 1, w = q0 + e % XW - 1;
+          const bool in = c0 + ch < a.C && unsigned(h) < unsigned(P) && unsigned(w) < unsigned(Q);
+          xr[e / XW * XF + e % XW] = in ? a.x[((n * a.C + c0 + ch) * P + h) * Q + w] : 0.f;
+        }
+      }
+      __syncthreads();
+      if (live && number) {
+#pragma unroll 1
+        for (int u = 0; u < COLS; u += 2) {
+          const float d = ys[row * YP + u + th];
+          const bool in = q0 + u + th < Q;   // (beyond the row dy's zeros must meet zeros)
+#pragma unroll
+          for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const float xv = xr[(r * 64 + col) * XF + u + th + c];
+              acc[r * 3 + c] = __builtin_amdgcn_mfma_f32_32x32x2f32(d, in ? xv : 0.f, acc[r * 3 + c], 0, 0, 0);
+            }
+        }
+        bool any = false;
+#pragma unroll
+        for (int c = 0; c < 9; ++c)
+#pragma unroll
+          for (int u = 0; u < 16; ++u) any |= acc[c][u] == acc[c][u] && (valid >> u & 1);
+        number = __any(any);
+      }
+    }
+    if (group) {   // (as the loop above leaves it)
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][v] = -acc[i][v];
+    }
+    __syncthreads();
+  }
+
   // ---- the two groups' sums, then this workgroup's partial image
   float *const ex = reinterpret_cast<float *>(smem) + w4 * kAcc + lane;
   if (group) {
@@ -351,29 +405,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (group) return;
   const rsrc_t rp = make_rsrc(a.partial + (size_t(split) * a.tiles + tile) * 4 * kAcc, 4 * kAcc * 4);
   const int po = (w4 * kAcc + lane) * 4;
-  unsigned nan_k = 0;   // accumulator registers whose filter has met a NaN of dy
 #pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    unsigned mask = 0;
-    bool nan_x = false;   // this tap has met a NaN of x
+  for (int i = 0; i < 9; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float s = acc[i][v] - ex[(i * 16 + v) * 64];
-      if (!finite(s)) mask |= 1u << v;
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po, (i * 16 + v) * 256, 0);
-    }
-    for (; mask; mask &= mask - 1) {
-      const int v = __builtin_ctz(mask), k = k0 + wm * 32 + 8 * (v >> 2) + 4 * half + (v & 3), c = c0 + wn * 32 + l32;
-      if (k >= a.K || c >= a.C) continue;
-      float s = __builtin_nanf("");
-      if (!nan_x && !(nan_k >> v & 1)) {
-        unsigned seen = 0;
-        s = redo(a, k, c, i, first * RPI, last * RPI, q0, min(a.Q, q0 + 8 * OCS), seen);
-        nan_k |= (seen & 1) << v, nan_x = seen & 2;
-      }
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po + (i * 16 + v) * 256, 0, 0);
-    }
-  }
+    for (int v = 0; v < 16; ++v)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][v] - ex[(i * 16 + v) * 64]), rp, po, (i * 16 + v) * 256, 0);
 }
 
 // dW from the partial images, in ascending order.  A workgroup takes four accumulator registers of a wavefront (16 bytes a lane:

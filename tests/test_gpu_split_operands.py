@@ -195,3 +195,74 @@ def test_conv_split_infinities_and_nans(singa, dev, n, c, h, w, k, r, where):
         assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
         fin = np.isfinite(ref)
         np.testing.assert_allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+# rows of one, two, four and (three) four octets, several strips, ragged channels; each takes the octet kernel
+WGRAD_OCTET_LAYERS = [(20, 512, 7, 7, 200), (24, 257, 9, 8, 190), (40, 100, 13, 13, 250), (13, 130, 20, 21, 120), (14, 100, 20, 30, 140), (6, 64, 37, 41, 210)]
+
+
+def wgrad64(x, dy):
+    """float64 weight gradient of 3x3, stride 1, padding 1"""
+    import torch
+    n, c, h, w = x.shape
+    xp = torch.nn.functional.pad(torch.from_numpy(x).double(), (1, 1, 1, 1))
+    d = torch.from_numpy(dy).double().permute(1, 0, 2, 3).reshape(dy.shape[1], -1).contiguous()
+    taps = [d @ xp[:, :, i:i + h, j:j + w].permute(0, 2, 3, 1).reshape(-1, c) for i in range(3) for j in range(3)]
+    return torch.stack(taps, -1).reshape(dy.shape[1], c, 3, 3).numpy()
+
+
+@pytest.mark.parametrize("n,c,h,w,k", WGRAD_OCTET_LAYERS)
+def test_conv_wgrad_octets_values(singa, dev, n, c, h, w, k):
+    """Against float64: within terms * 2^-23 of the sum of the terms' magnitudes, and closer than a sixteenth of the roundings of
+    chains of fp32 additions (0.5 * sqrt(terms) * 2^-24, and the rounding of the result); the same bits again."""
+    x, W, dy = operands("normal", n + c + k, n, c, h, w, k, 3)
+    got, names = passes(singa, dev, x, W, dy)[2]
+    assert names == {"k_wgrad_oct"}
+    want = wgrad64(x, dy)
+    assert np.all(np.abs(got - want) <= n * h * w * 2.0 ** -23 * wgrad64(np.abs(x), np.abs(dy)))
+    assert nl2(got, want) < (0.5 * (n * h * w) ** 0.5 + 1) * 2.0 ** -24
+    again, _ = passes(singa, dev, x, W, dy)[2]
+    assert np.array_equal(again, got)
+
+
+@pytest.mark.parametrize("n,c,h,w,k", WGRAD_OCTET_LAYERS)
+def test_conv_wgrad_octets_infinities_and_nans(singa, dev, n, c, h, w, k):
+    """+inf, -inf and NaN, also in the first and last rows and columns, reach exactly the weights that their products reach, those
+    with the padding among them (zeros: NaN), with the sign that those have."""
+    x, W, dy = operands("normal", 13, n, c, h, w, k, 3)
+    x[n // 2, 5, h - 1, w - 1], x[1, 6, 0, 0], x[2, 7, h // 2, 1], x[0, c - 1, 0, w - 1] = -np.inf, np.inf, np.nan, np.inf
+    dy[n - 1, k - 1, h - 1, 4], dy[0, 3, 1, w - 1], dy[3, 4, 2, 2] = np.inf, -np.inf, np.nan
+    got, names = passes(singa, dev, x, W, dy)[2]
+    assert names == {"k_wgrad_oct"}
+    with np.errstate(all="ignore"):
+        want = wgrad64(x, dy).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan"])
+def test_conv_wgrad_octets_time_of_non_finite_operands(singa, dev, what):
+    """As the forward pass and the data gradient: no search per result."""
+    n, c, h, w, k = 32, 256, 14, 14, 256
+    x, W, dy = operands("normal", 3, n, c, h, w, k, 3)
+
+    def time(x, dy):
+        xd, wd, dyd = (singa.from_numpy(a, dev) for a in (x, W, dy))
+        hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, False)
+        assert kernels_of(dev, lambda: singa.GpuConvBackwardW(dyd, xd, wd, hd))[1] == {"k_wgrad_oct"}
+        return seconds(dev, lambda: singa.GpuConvBackwardW(dyd, xd, wd, hd))
+
+    plain = time(x, dy)
+    value = np.float32(np.nan if what == "nan" else np.inf)
+    if what == "one inf":
+        dy[:, 0, 7, 7] = value
+    elif what == "overflow":
+        x, dy = x * np.float32(1e30), dy * np.float32(1e30)
+    else:
+        x[:] = value
+        dy[:] = value
+    got = time(x, dy)
+    print(what, "%.1f us, ordinary operands %.1f" % (got * 1e6, plain * 1e6))
+    assert got < 8 * plain
