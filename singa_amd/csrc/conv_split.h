@@ -15,6 +15,11 @@ int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps
 int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s,
                        const char *tag, bool dgrad, const float *bias, bool accumulate);
 
+// Operands are multiplied by this before they are split, results by the square of its inverse: three bfloat16 values hold 24 bits
+// of a number from 2^-110 on, and with this all bits of every fp32 number down to the smallest subnormal one.  What comes out
+// beyond 2^96 is formed again anyway.
+constexpr float kSplitScale = 65536.f, kSplitUnscale = 1.f / kSplitScale / kSplitScale;
+
 constexpr int kSplitWeightLds = 512 * 9;   // floats of LDS that a workgroup below needs
 
 // Taps that a workgroup below handles: all of a small filter once that many workgroups fill the chip, else a third of them (64 to
@@ -23,7 +28,7 @@ constexpr int kSplitTaps = 9, kSplitTapsFew = 3;
 
 // One (chunk of 16 channels k, block of 32 channels c) of the weight fragments [chunk][tap][block][part][lane][8], by 256
 // threads: the source runs are contiguous, the fragments too, LDS turns one into the other.
-// (w0, w1, w2) sum to w exactly; an infinite w is (w, 0, 0), so that the sum stays what w was.  Odd taps are negated.
+// w0 + w1 + w2 is kSplitScale w, or not finite where that does not fit; odd taps are negated.
 __device__ __forceinline__ void sgh_conv_split_weights_block(const float *__restrict__ W, uint16_t *__restrict__ wt, int C, int K,
                                                              int RS, int cblocks, int dgrad, int blk, int taps, float *buf) {
   const int groups = (RS + taps - 1) / taps, group = blk % groups;
@@ -55,15 +60,11 @@ __device__ __forceinline__ void sgh_conv_split_weights_block(const float *__rest
       uint16_t part[3][8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float w = q % RS & 1 ? -src[j * 9] : src[j * 9];
+        const float w = (q % RS & 1 ? -kSplitScale : kSplitScale) * src[j * 9];
         auto up = [](uint16_t b) { return __builtin_bit_cast(float, unsigned(b) << 16); };
         auto down = [](float f) { return __builtin_bit_cast(uint16_t, __bf16(f)); };
-        const bool big = !(__builtin_fabsf(w) < 3.38e38f);   // rounds to infinity, is infinite or NaN
-        const bool fin = __builtin_fabsf(w) < __builtin_inff();
-        const uint16_t p0 = big && fin ? uint16_t(__builtin_bit_cast(unsigned, w) >> 16) : down(w);
-        const float r = big && !fin ? 0.f : w - up(p0);
-        const uint16_t p1 = down(r);
-        part[0][j] = p0, part[1][j] = p1, part[2][j] = down(r - up(p1));
+        const uint16_t p0 = down(w), p1 = down(w - up(p0));
+        part[0][j] = p0, part[1][j] = p1, part[2][j] = down(w - up(p0) - up(p1));
       }
       uint16_t *dst = wt + (size_t(q) * cblocks + cb) * 1536 + lane * 8;
 #pragma unroll

@@ -1,6 +1,7 @@
 // fp32 convolutions of stride 1 with "same" padding (3x3, 5x5), forward and data gradient, on the bfloat16 matrix
 // instructions without giving up fp32 operands (the splitting of G. Henry, P. Tang, A. Heinecke, "Leveraging the bfloat16
-// artificial intelligence datatype for higher-precision computations", 2019): a fp32 value is the sum of three bfloat16 values
+// artificial intelligence datatype for higher-precision computations", 2019): a fp32 value, times 2^16 so that this holds for
+// the smallest ones too, is the sum of three bfloat16 values
 //
 //   x = x0 + x1 + x2,   x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)      (8 + 8 + 8 bits of significand)
 //
@@ -36,8 +37,7 @@
 // against float64 is 0.15 to 0.6 times that of the fp32 instructions, 0.9 at most, on normal, on rectified and on positive
 // operands; an addition of 16 results per six products costs 4 to 8 per cent of the time.
 //
-// Infinities, NaNs and values within half a bfloat16 ulp of the largest float: a part that overflows makes products of
-// infinity with zero, so a tile with a result that comes out non-finite is formed again by its workgroup on the fp32 matrix
+// Infinities, NaNs and values and results too large for the scale (2^112, 2^96): parts that overflow make NaNs, so a tile with a result that comes out non-finite is formed again by its workgroup on the fp32 matrix
 // instructions, whatever the values are.
 #include "common.h"
 #include "conv_split.h"
@@ -72,7 +72,7 @@ __device__ __forceinline__ float hi_f(unsigned p) { return __builtin_bit_cast(fl
 __device__ __forceinline__ void split8(const float (&v)[8], v4u (&part)[3]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float a = v[2 * i], b = v[2 * i + 1];
+    const float a = v[2 * i] * kSplitScale, b = v[2 * i + 1] * kSplitScale;
     const unsigned p0 = pack2(a, b);
     const float ra = a - lo_f(p0), rb = b - hi_f(p0);
     const unsigned p1 = pack2(ra, rb);
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][j][v]);
+      for (int v = 0; v < 16; ++v) acc[i][j][v] *= kSplitUnscale, bad |= !finite(acc[i][j][v]);
   auto put = [&](int m, int col, int n, float r) {   // row, column of the tile
     const int c = c0 + m, pix = pix0 + col;
     if (c >= a.C || pix >= a.total_pix) return;

@@ -21,6 +21,7 @@
 // own and added to the accumulator once; without that the error is up to 1.5 times that of the fp32 instructions behind a
 // ReLU (whose zeros cost those no rounding), and the kernel 7 per cent faster.
 #include "common.h"
+#include "conv_split.h"
 
 namespace {
 
@@ -82,8 +83,8 @@ struct Octet {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const unsigned ua = raw[i / 2][2 * i % 4], ub = raw[i / 2][2 * i % 4 + 1];
-      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) : 0.f;
-      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) : 0.f;
+      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) * kSplitScale : 0.f;
+      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) * kSplitScale : 0.f;
       const unsigned p0 = pack2(a, b);
       const float ra = a - lo_f(p0), rb = b - hi_f(p0);
       const unsigned p1 = pack2(ra, rb);
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   };
   auto edge_get = [&](int off) -> unsigned { return __builtin_amdgcn_raw_buffer_load_b32(rx, off, 0, 0); };
   auto put_edge = [&](unsigned raw, int slot, int c, int side) {
-    const float v = __builtin_bit_cast(float, raw);
+    const float v = __builtin_bit_cast(float, raw) * kSplitScale;
     const unsigned p0 = pack2(v, 0.f);
     const float r = v - lo_f(p0);
     const unsigned p1 = pack2(r, 0.f);
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
   }
 
-  // ---- sums that are not finite: an infinity or a value near the largest float has parts whose products are NaN, and a zero of
+  // ---- sums that are not finite: an infinity or a value too large for the scale has parts whose products are NaN, and a zero of
   // the virtual rows and columns has met one.  All of the workgroup's sums are formed again on the fp32 instructions, a row at a
   // time, whatever the values are: 2.7 times the products' time.  (LDS is free.  Everything is derived anew from opaque copies:
   // what the loop above holds in registers for this, it spills.)
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
   for (int i = 0; i < 9; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][v]);
+    for (int v = 0; v < 16; ++v) acc[i][v] *= kSplitUnscale, bad |= !finite(acc[i][v]);
   int *const again = reinterpret_cast<int *>(smem);
   if (t == 0) *again = 0;
   __syncthreads();

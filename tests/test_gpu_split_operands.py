@@ -266,3 +266,22 @@ def test_conv_wgrad_octets_time_of_non_finite_operands(singa, dev, what):
     got = time(x, dy)
     print(what, "%.1f us, ordinary operands %.1f" % (got * 1e6, plain * 1e6))
     assert got < 8 * plain
+
+
+@pytest.mark.parametrize("small,large", [(2.0 ** -116, 1.0), (2.0 ** -124, 2.0 ** 40), (2.0 ** -132, 2.0 ** 60), (1.0, 2.0 ** -116)])
+def test_conv_split_operands_of_any_magnitude(singa, dev, small, large):
+    """Inputs and gradients (or weights) of small magnitude, down to subnormal ones, at the error that ordinary magnitudes have: on
+    three bfloat16 values alone the last bits of a number below 2^-110 are lost."""
+    n, c, h, w, k = 14, 100, 20, 30, 140
+    x, W, dy = operands("normal", 5, n, c, h, w, k, 3)
+    x, W, dy = x * np.float32(small), W * np.float32(large), dy * np.float32(small)
+    (y, ky), (dx, kx), _ = passes(singa, dev, x, W, dy)
+    assert ky == {"k_conv_split"} and kx == {"k_conv_split"}
+    import torch
+    t = lambda a: torch.from_numpy(a).double()
+    assert nl2(y, torch.nn.functional.conv2d(t(x), t(W), padding=1).numpy()) < 3e-7
+    assert nl2(dx, torch.nn.functional.conv_transpose2d(t(dy), t(W), padding=1).numpy()) < 3e-7
+    for a, b in ((x, dy / np.float32(small) * np.float32(large)), (x / np.float32(small) * np.float32(large), dy)):
+        dw, kw = passes(singa, dev, a, W, b)[2]
+        assert kw == {"k_wgrad_oct"}
+        assert nl2(dw, wgrad64(a, b)) < 3e-7
