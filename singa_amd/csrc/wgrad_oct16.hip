@@ -49,12 +49,6 @@ __device__ __forceinline__ v16f mfma(v4u a, v4u b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-template <bool BF16>
-__device__ __forceinline__ float widen(uint16_t v) {
-  if constexpr (BF16) return __builtin_bit_cast(float, unsigned(v) << 16);
-  else return float(__builtin_bit_cast(_Float16, v));
-}
-
 __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
 
 struct Wo16Args {
@@ -89,28 +83,6 @@ __device__ __forceinline__ v4u load8(rsrc_t r, unsigned bytes, unsigned off, int
     }
   }
   return v;
-}
-
-// One sum term by term: virtual rows [v0, v1), columns [q0, q1).  A NaN of dy makes one of the filter's sums of every tap and
-// channel, a NaN of x of every filter's at this tap and channel; `seen` tells the caller (bit 0: dy, bit 1: x), which need not
-// look for it again (a diverged network has little else: 144 searches a lane took 0.8 ms)
-template <int ST, bool BF16>
-__device__ float redo(const Wo16Args &a, int k, int c, int tap, int v0, int v1, int q0, int q1, unsigned &seen) {
-  float sum = 0.f;
-  for (int v = v0; v < v1 && sum == sum; ++v) {
-    const int n = v / (a.P + 1), p = v - n * (a.P + 1);
-    if (p >= a.P || n >= a.N) continue;
-    const int h = ST * p + tap / 3 - 1;
-    for (int q = q0; q < q1 && sum == sum; ++q) {
-      const int w = ST * q + tap % 3 - 1;
-      const bool in = unsigned(h) < unsigned(a.H) && unsigned(w) < unsigned(a.W);
-      const float xv = in ? widen<BF16>(a.x[((size_t(n) * a.C + c) * a.H + h) * a.W + w]) : 0.f;
-      const float d = widen<BF16>(a.dy[((size_t(n) * a.K + k) * a.P + p) * a.Q + q]);
-      seen |= (d != d ? 1u : 0u) | (xv != xv ? 2u : 0u);
-      sum = __builtin_fmaf(d, xv, sum);
-    }
-  }
-  return sum;
 }
 
 template <int ST, int OCS, int RPI>
@@ -438,6 +410,90 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     __syncthreads();
   }
 
+  // ---- sums that are not finite: a zero of the virtual rows and columns may have met an infinity or a NaN.  All of the
+  // workgroup's sums are formed again, a row at a time, with every tap's octets in LDS on their own and zero where dy's are no
+  // pixels: three to four times the time of the loop above, whatever the values are.  (LDS is free.  Everything is derived anew from opaque
+  // copies: what the loop above holds in registers for this, it spills.)
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) bad |= !finite(acc[i][v]);
+  int *const again = reinterpret_cast<int *>(smem);
+  if (t == 0) *again = 0;
+  __syncthreads();
+  if (__any(bad) && lane == 0) *again = 1;
+  __syncthreads();
+  if (*again) {
+    static_assert(10 * 64 * OCS * 16 <= S::LDS / 2, "");
+    int tt = threadIdx.x, P = a.P, Q = a.Q, H = a.H, W = a.W;
+    asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q), "+s"(H), "+s"(W));
+    const int th = tt >> 5 & 1, row = wm * 32 + (tt & 31), col = wn * 32 + (tt & 31);
+    v4u *const ys = reinterpret_cast<v4u *>(smem + group * (S::LDS / 2)), *const xt = ys + 64 * OCS;   // [channel][octet], [tap][channel][octet]
+    unsigned valid = 0;   // accumulator registers that hold a filter
+#pragma unroll
+    for (int v = 0; v < 16; ++v) valid |= unsigned(k0 + wm * 32 + 8 * (v >> 2) + 4 * th + (v & 3) < a.K && c0 + col < a.C) << v;
+    bool number = true;   // not every sum of this wavefront is a NaN yet (in a diverged network they soon are)
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+    for (int i = 0; i < mine * RPI; ++i) {
+      const int v = it0 * RPI + i, n = v / (P + 1), p = v - n * (P + 1);
+      const bool live = v < it1 * RPI && n < a.N && p < P;
+      __syncthreads();
+      if (live) {
+        for (int e = tt & (GT - 1); e < 10 * 64 * OCS; e += GT) {
+          const int tap = e / (64 * OCS) - 1, ch = e / OCS % 64, q = q0 + e % OCS * 8;   // tap -1: dy
+          const bool of_dy = tap < 0;
+          const int h = of_dy ? p : ST * p + tap / 3 - 1, w0 = of_dy ? q : ST * q + tap % 3 - 1, step = of_dy ? 1 : ST;
+          const int width = of_dy ? Q : W, height = of_dy ? P : H, channels = of_dy ? a.K : a.C, channel = (of_dy ? k0 : c0) + ch;
+          // the first n pixels count, the very first not where it is left of the image: then all come from a column further on
+          const int n8 = min(min(8, Q - q), (width - w0 + step - 1) / step), left = w0 < 0, at = w0 + left;
+          const bool in = channel < channels && unsigned(h) < unsigned(height);
+          const unsigned off = unsigned(((n * channels + channel) * height + h) * width + at) * 2;
+          v4u raw[ST];
+#pragma unroll
+          for (int u = 0; u < ST; ++u)
+            raw[u] = of_dy ? load8(rdy, a.dy_bytes, off, in && !u ? width - at : 0) : load8(rx, a.x_bytes, off + 16 * u, in ? width - at - 8 * u : 0);
+          v4u o = raw[0];
+          if (step == 2) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const v4u &r = raw[ST == 2 ? u / 2 : 0];
+              o[u] = __builtin_amdgcn_perm(r[2 * u % 4 + 1], r[2 * u % 4], left ? 0x07060302 : 0x05040100);
+            }
+          }
+          if (left) o = v4u{o[0] << 16, __builtin_amdgcn_alignbit(o[1], o[0], 16), __builtin_amdgcn_alignbit(o[2], o[1], 16),
+                            __builtin_amdgcn_alignbit(o[3], o[2], 16)};
+          o = in ? o & keep_first(n8) : v4u{0u, 0u, 0u, 0u};
+          ys[e] = o;
+        }
+      }
+      __syncthreads();
+      if (live && number) {
+#pragma unroll 1
+        for (int o = 0; o < OCS; o += 2) {
+          const bool there = o + th < OCS;
+          const int at = there ? o + th : o;
+          const v4u d = there ? ys[row * OCS + at] : v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int c = 0; c < 9; ++c) {
+            const v4u x = xt[(c * 64 + col) * OCS + at];
+            acc[c] = mfma<BF16>(d, there ? x : v4u{0u, 0u, 0u, 0u}, acc[c]);
+          }
+        }
+        bool any = false;
+#pragma unroll
+        for (int c = 0; c < 9; ++c)
+#pragma unroll
+          for (int u = 0; u < 16; ++u) any |= acc[c][u] == acc[c][u] && (valid >> u & 1);
+        number = __any(any);
+      }
+    }
+    __syncthreads();
+  }
+
   // ---- the two groups' sums, then this workgroup's partial image
   float *const ex = reinterpret_cast<float *>(smem) + w4 * kAcc + lane;
   if (group) {
@@ -450,30 +506,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (group) return;
   const rsrc_t rp = make_rsrc(a.partial + (size_t(range * a.strips + strip) * a.tiles + tile) * 4 * kAcc, 4 * kAcc * 4);
   const int po = (w4 * kAcc + lane) * 4;
-  unsigned nan_k = 0;   // accumulator registers whose filter has met a NaN of dy
 #pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    unsigned mask = 0;
-    bool nan_x = false;   // this tap has met a NaN of x
+  for (int i = 0; i < 9; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float s = acc[i][v] + ex[(i * 16 + v) * 64];
-      if (!finite(s)) mask |= 1u << v;
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po, (i * 16 + v) * 256, 0);
-    }
-    // a zero beside the image's own padding (the virtual row, the columns beyond Q) may have met an infinity or a NaN
-    for (; mask; mask &= mask - 1) {
-      const int v = __builtin_ctz(mask), k = k0 + wm * 32 + 8 * (v >> 2) + 4 * half + (v & 3), c = c0 + wn * 32 + l32;
-      if (k >= a.K || c >= a.C) continue;
-      float s = __builtin_nanf("");
-      if (!nan_x && !(nan_k >> v & 1)) {
-        unsigned seen = 0;
-        s = redo<ST, BF16>(a, k, c, i, first * RPI, last * RPI, q0, min(a.Q, q0 + 8 * OCS), seen);
-        nan_k |= (seen & 1) << v, nan_x = seen & 2;
-      }
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s), rp, po + (i * 16 + v) * 256, 0, 0);
-    }
-  }
+    for (int v = 0; v < 16; ++v)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][v] + ex[(i * 16 + v) * 64]), rp, po, (i * 16 + v) * 256, 0);
 }
 
 // dW from the partial images, summed in ascending order.  A workgroup takes four accumulator registers of a wavefront (16 bytes

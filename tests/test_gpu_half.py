@@ -1041,6 +1041,75 @@ def test_conv_wgrad_octets_16bit_non_finite(singa, dev, kind, stride, bad):
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-2, atol=1e-1)
 
 
+def _octet_layer(singa, dev, kind, case, spoil=None):
+    """x, dy as stored, and the weight gradient as a call; asserts that the octet kernel runs it"""
+    from util import kernels_of
+    N, C, H, W, K, st = case
+    r = rng(sum(case))
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    dy = r.standard_normal((N, K, (H - 1) // st + 1, (W - 1) // st + 1)).astype(np.float32)
+    if spoil:
+        spoil(x, dy)
+    (xt, x), (dyt, dy) = _to(singa, dev, x, kind), _to(singa, dev, dy, kind)
+    wt, _ = _to(singa, dev, np.zeros((K, C, 3, 3), np.float32), kind)
+    h = singa.CudnnConvHandle(xt, (3, 3), (st, st), (1, 1), C, K, False)
+    call = lambda: singa.GpuConvBackwardW(dyt, xt, wt, h)
+    assert kernels_of(dev, call)[1] == {"k_wgrad_oct16"}
+    return x, dy, call
+
+
+# one, two, three and four octets, several strips, planes of both parities
+WGRAD_OCTET16_LAYERS = [(26, 568, 59, 8, 43, 1), (100, 400, 7, 8, 300, 1), (23, 601, 56, 13, 28, 1), (53, 640, 20, 24, 18, 1), (13, 516, 25, 32, 56, 1),
+                        (29, 324, 64, 42, 11, 1), (54, 233, 51, 11, 155, 2), (94, 536, 30, 17, 42, 2), (41, 345, 65, 50, 24, 2), (64, 468, 60, 77, 8, 2),
+                        (128, 128, 57, 56, 128, 2)]
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("case", WGRAD_OCTET16_LAYERS)
+def test_conv_wgrad_octets_16bit_infinities_and_nans(singa, dev, kind, case):
+    """+inf, -inf and NaN, also in the first and last rows and columns, reach exactly the weights that their products reach, those
+    with the padding among them (zeros: NaN), with the sign that those have; all other weights are the ordinary ones."""
+    import torch
+    N, C, H, W, K, st = case
+    P, Q = (H - 1) // st + 1, (W - 1) // st + 1
+
+    def spoil(x, dy):
+        x[N // 2, 5, H - 1, W - 1], x[1, 6, 0, 0], x[2, 7, H // 2, 1], x[0, C - 1, 0, W - 1] = -np.inf, np.inf, np.nan, np.inf
+        dy[N - 1, K - 1, P - 1, 2], dy[0, 3, 1, Q - 1], dy[3, 4, 2, 2] = np.inf, -np.inf, np.nan
+
+    x, dy, call = _octet_layer(singa, dev, kind, case, spoil)
+    got = call().to_numpy()
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 2), (1, 2)))
+    with np.errstate(all="ignore"):
+        d2 = torch.from_numpy(dy.astype(np.float64).transpose(1, 0, 2, 3).reshape(K, -1).copy())
+        want = torch.stack([d2 @ torch.from_numpy(xp[:, :, i:i + st * P:st, j:j + st * Q:st].transpose(0, 2, 3, 1).reshape(-1, C).copy())
+                            for i in range(3) for j in range(3)], -1).numpy().reshape(K, C, 3, 3)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    assert np.linalg.norm(got[fin] - want[fin]) < 2.0 ** (-11 if kind == "f16" else -8) * np.linalg.norm(want[fin])
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("what", ["inf", "one inf", "nan"])
+def test_conv_wgrad_octets_16bit_time_of_non_finite_operands(singa, dev, kind, stride, what):
+    """Sums that are not finite take a second pass over the workgroup's rows on the same instructions, and no search per sum: eight
+    times the time of ordinary operands at most (a term-by-term search took 50 to 100 times)."""
+    from util import seconds
+    case = (128, 256, 14, 14, 256, 1) if stride == 1 else (128, 128, 56, 57, 128, 2)
+
+    def spoil(x, dy):
+        if what == "one inf":
+            dy[:, 0, 3, 3] = np.inf
+        else:
+            x[:] = dy[:] = np.float32(what)
+
+    plain, got = (seconds(dev, _octet_layer(singa, dev, kind, case, f)[2]) for f in (None, spoil))
+    print(what, "%.1f us, ordinary operands %.1f" % (got * 1e6, plain * 1e6))
+    assert got < 8 * plain
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 @pytest.mark.parametrize("case", [(2, 64, 16, 24, 40), (3, 40, 12, 20, 24), (2, 72, 14, 14, 136), (2, 16, 9, 11, 8), (1, 16, 4, 10, 64),
                                   (1, 64, 7, 4, 16)])

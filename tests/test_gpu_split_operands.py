@@ -1,11 +1,9 @@
 """The fp32 convolutions on split operands (conv_split.hip, wgrad_oct.hip) against what fp32 instructions would give: the error of
 their sums over the operands that networks have."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
-from util import nl2, randn, rng
+from util import kernels_of, nl2, randn, rng, seconds
 
 pytestmark = pytest.mark.gpu
 
@@ -14,27 +12,6 @@ pytestmark = pytest.mark.gpu
 def singa():
     from singa_amd import singa_wrap
     return singa_wrap
-
-
-def kernels_of(dev, call):
-    """(result of `call`, names of the kernels that it was timed on)"""
-    from singa_amd import _lib
-    lib, n, buf = _lib.lib(), C.c_int(), C.create_string_buffer(64)
-    dev.Sync()
-    lib.sgh_prof_clear()
-    _lib.check(lib.sgh_prof_enable(1), "sgh_prof_enable")
-    try:
-        out = call()
-        dev.Sync()
-        _lib.check(lib.sgh_prof_count(C.byref(n)), "sgh_prof_count")
-        names, ms, work = set(), C.c_float(), C.c_double()
-        for i in range(n.value):
-            _lib.check(lib.sgh_prof_get(i, buf, 64, C.byref(ms), C.byref(work)), "sgh_prof_get")
-            names.update(buf.value.decode().split("/")[1:])   # ("class/kernel"; the record of a whole entry point has no kernel)
-    finally:
-        lib.sgh_prof_enable(0)
-        lib.sgh_prof_clear()
-    return out, names
 
 
 def operands(kind, seed, n, c, h, w, k, r):
@@ -122,20 +99,6 @@ def test_conv_wgrad_octets_error_of_fp32_chains(singa, dev, n, c, h, w, k, kind)
     mine = got[:few, :few]
     print(kind, "error %.2e, of chains %.2e" % (nl2(mine, want), nl2(chain, want)))
     assert nl2(mine, want) < nl2(chain, want)   # (short chains: the rounding of the result is most of either error)
-
-
-def seconds(dev, call):
-    """The least of three runs of `call` on an idle device"""
-    import time
-    call()
-    best = 1e9
-    for _ in range(3):
-        dev.Sync()
-        t = time.perf_counter()
-        call()
-        dev.Sync()
-        best = min(best, time.perf_counter() - t)
-    return best
 
 
 @pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan", "nan weights", "inf weights"])

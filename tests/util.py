@@ -37,3 +37,39 @@ def assert_bit_equal(a, b, what=""):
     same = (bits(a) == bits(b)) | ((a == 0) & (b == 0))
     assert bool(np.all(same)), "%s: %d of %d elements differ, first at %s" % (
         what, int((~same).sum()), a.size, np.argwhere(~same)[:3].tolist())
+
+
+def kernels_of(dev, call):
+    """(result of `call`, names of the kernels that it was timed on)"""
+    import ctypes as C
+    from singa_amd import _lib
+    lib, n, buf = _lib.lib(), C.c_int(), C.create_string_buffer(64)
+    dev.Sync()
+    lib.sgh_prof_clear()
+    _lib.check(lib.sgh_prof_enable(1), "sgh_prof_enable")
+    try:
+        out = call()
+        dev.Sync()
+        _lib.check(lib.sgh_prof_count(C.byref(n)), "sgh_prof_count")
+        names, ms, work = set(), C.c_float(), C.c_double()
+        for i in range(n.value):
+            _lib.check(lib.sgh_prof_get(i, buf, 64, C.byref(ms), C.byref(work)), "sgh_prof_get")
+            names.update(buf.value.decode().split("/")[1:])   # ("class/kernel"; the record of a whole entry point has no kernel)
+    finally:
+        lib.sgh_prof_enable(0)
+        lib.sgh_prof_clear()
+    return out, names
+
+
+def seconds(dev, call):
+    """The least of three runs of `call` on an idle device"""
+    import time
+    call()
+    best = 1e9
+    for _ in range(3):
+        dev.Sync()
+        t = time.perf_counter()
+        call()
+        dev.Sync()
+        best = min(best, time.perf_counter() - t)
+    return best
