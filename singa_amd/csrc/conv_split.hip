@@ -311,13 +311,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
       ph[j] = rem / Q, pw[j] = rem - ph[j] * Q;
       base[j] = (n * vh + ph[j] - vbase) * pitch + pw[j] + half * 8 * slab;
     }
-    bool number = true;   // not every result of this wavefront is a NaN yet (in a diverged network they soon are)
+    // not every result of this wavefront, of the workgroup is a NaN yet (in a diverged network they soon are)
+    bool number = true;
+    int *const numbers = reinterpret_cast<int *>(smem + 2 * a.slab * kPos);   // the last chunk that left one
+    if (tt == 0) *numbers = ch_begin - 1;
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[0][j][v] = 0.f;
     for (int ch = ch_begin; ch < ch_end; ++ch) {
       __syncthreads();
+      if (*numbers < ch - 1) break;
 #pragma unroll 1
       for (int i = tt; i < 2 * slab; i += NT) {
         const int oct = i >= slab, pos = i - (oct ? slab : 0), vr = pos / pitch, q = pos - vr * pitch - O, v = vbase + vr, n = v / vh;
@@ -373,6 +377,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
           for (int v = 0; v < 16; ++v) any |= acc[0][j][v] == acc[0][j][v];
         number = __any(any);
       }
+      if (number && lane == 0) *numbers = ch;
     }
   }
 #pragma unroll
@@ -483,7 +488,7 @@ int launch(const ScArgs &a, const ScPlan &p, hipStream_t s) {
       return SGH_EUNSUPPORTED;
     attr_set = true;
   }
-  SGH_LAUNCH_TIMED(kern, dim3(unsigned(p.wgs)), dim3(NT), size_t(p.slab) * 2 * kPos, s, a);
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(p.wgs)), dim3(NT), size_t(p.slab) * 2 * kPos + 16, s, a);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 

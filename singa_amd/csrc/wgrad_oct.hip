@@ -101,7 +101,7 @@ struct Shape {
   static constexpr int DYO = (PARTS * 64 + 4) * 16;            // an octet of dy; four units of padding spread the writes over the banks
   static constexpr int GROUP = RING * XROW + OPI * DYO;
   static constexpr int LDS = 2 * GROUP > kAcc * 16 ? 2 * GROUP : kAcc * 16;
-  static_assert(OPI % 2 == 0 && LDS <= 160 * 1024, "");
+  static_assert(OPI % 2 == 0 && LDS + 16 <= 160 * 1024, "");
 };
 
 template <int OCS, int RPI>
@@ -343,7 +343,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     unsigned valid = 0;   // accumulator registers that hold a filter
 #pragma unroll
     for (int v = 0; v < 16; ++v) valid |= unsigned(k0 + wm * 32 + 8 * (v >> 2) + 4 * th + (v & 3) < a.K && c0 + col < a.C) << v;
-    bool number = true;   // not every sum of this wavefront is a NaN yet (in a diverged network they soon are)
+    // not every sum of this wavefront, of the workgroup is a NaN yet (in a diverged network they soon are)
+    bool number = true;
+    int *const numbers = reinterpret_cast<int *>(smem + S::LDS);   // the last row that left one
+    if (tt == 0) *numbers = -1;
 #pragma unroll
     for (int i = 0; i < 9; ++i)
 #pragma unroll
@@ -352,6 +355,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       const int v = it0 * RPI + i, n = v / (P + 1), p = v - n * (P + 1);
       const bool live = v < it1 * RPI && n < a.N && p < P;
       __syncthreads();
+      if (*numbers < i - 1) break;
       if (live) {
         for (int e = tt & (GT - 1); e < 64 * COLS; e += GT) {
           const int ch = e / COLS, q = e % COLS;
@@ -384,6 +388,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           for (int u = 0; u < 16; ++u) any |= acc[c][u] == acc[c][u] && (valid >> u & 1);
         number = __any(any);
       }
+      if (number && lane == 0) *numbers = i;
     }
     if (group) {   // (as the loop above leaves it)
 #pragma unroll
@@ -493,7 +498,7 @@ int launch(const WoArgs &a, hipStream_t s) {
       return SGH_EUNSUPPORTED;
     attr_set = true;
   }
-  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.splits)), dim3(NT), (Shape<OCS, RPI>::LDS), s, a);
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.splits)), dim3(NT), (Shape<OCS, RPI>::LDS + 16), s, a);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 

@@ -97,7 +97,7 @@ struct Shape {
   static constexpr int DYO = 65 * 16, DYB = OPI * DYO;               // an octet of dy, a buffer of them
   static constexpr int GROUP = RING * XV + 2 * DYB;
   static constexpr int LDS = 2 * GROUP > kAcc * 16 ? 2 * GROUP : kAcc * 16;
-  static_assert(OPI % 2 == 0 && XP % 2 == 1 && LDS <= 160 * 1024, "");
+  static_assert(OPI % 2 == 0 && XP % 2 == 1 && LDS + 16 <= 160 * 1024, "");
 };
 
 template <int ST, int OCS, int RPI, bool BF16>
@@ -433,7 +433,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     unsigned valid = 0;   // accumulator registers that hold a filter
 #pragma unroll
     for (int v = 0; v < 16; ++v) valid |= unsigned(k0 + wm * 32 + 8 * (v >> 2) + 4 * th + (v & 3) < a.K && c0 + col < a.C) << v;
-    bool number = true;   // not every sum of this wavefront is a NaN yet (in a diverged network they soon are)
+    // not every sum of this wavefront, of the workgroup is a NaN yet (in a diverged network they soon are)
+    bool number = true;
+    int *const numbers = reinterpret_cast<int *>(smem + S::LDS);   // the last row that left one
+    if (tt == 0) *numbers = -1;
 #pragma unroll
     for (int i = 0; i < 9; ++i)
 #pragma unroll
@@ -442,6 +445,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       const int v = it0 * RPI + i, n = v / (P + 1), p = v - n * (P + 1);
       const bool live = v < it1 * RPI && n < a.N && p < P;
       __syncthreads();
+      if (*numbers < i - 1) break;
       if (live) {
         for (int e = tt & (GT - 1); e < 10 * 64 * OCS; e += GT) {
           const int tap = e / (64 * OCS) - 1, ch = e / OCS % 64, q = q0 + e % OCS * 8;   // tap -1: dy
@@ -490,6 +494,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           for (int u = 0; u < 16; ++u) any |= acc[c][u] == acc[c][u] && (valid >> u & 1);
         number = __any(any);
       }
+      if (number && lane == 0) *numbers = i;
     }
     __syncthreads();
   }
@@ -586,7 +591,7 @@ int launch(const Wo16Args &a, hipStream_t s) {
       return SGH_EUNSUPPORTED;
     attr_set = true;
   }
-  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.strips * a.ranges)), dim3(NT), (Shape<ST, OCS, RPI>::LDS), s, a);
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.strips * a.ranges)), dim3(NT), (Shape<ST, OCS, RPI>::LDS + 16), s, a);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 
