@@ -1250,3 +1250,41 @@ def test_conv_forward_few_channels(singa, dev, n, c, h, w, k, r, st, pad):
     got = run(x, False)
     hit = conv((~np.isfinite(x)).astype(np.float32), np.ones_like(W), 0 * b) > 0
     assert np.array_equal(~np.isfinite(got), hit)
+
+
+# the 64-filter blocks of the few-channel forward kernel, which layers of many pixels take: whole and ragged blocks and rows of pixels
+FWD_FEW_WIDE_CASES = [
+    # n, c, h, w, k, r, stride, pad
+    (128, 3, 32, 32, 65, 3, 1, 1), (128, 3, 32, 32, 64, 5, 1, 2), (90, 5, 29, 31, 70, 7, 1, 3), (40, 7, 57, 56, 100, 3, 1, 1),
+    (64, 1, 90, 95, 64, 3, 2, 1), (33, 2, 60, 250, 40, 5, 1, 2),
+]
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,st,pad", FWD_FEW_WIDE_CASES)
+def test_conv_forward_few_channels_wide_blocks(singa, dev, n, c, h, w, k, r, st, pad):
+    """As above, where the rule takes 64 filters to a workgroup (a tile for every CU)."""
+    import torch
+    from util import kernels_of
+    p, q = (h + 2 * pad - r) // st + 1, (w + 2 * pad - r) // st + 1
+    assert k > 32 and -(-n * p * q // 256) * -(-k // 64) >= 256   # (the card's CUs)
+    rg = rng(n + 3 * c + k + r)
+    x, W, b = randn(rg, n, c, h, w), randn(rg, k, c, r, r), randn(rg, k)
+    terms = c * r * r + 1
+    conv = lambda x, W, b: torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(W).double(),
+                                                      torch.from_numpy(b).double(), st, pad).numpy()
+
+    def run(x, bias):
+        xd, wd, bd = singa.from_numpy(x, dev), singa.from_numpy(W, dev), singa.from_numpy(b, dev)
+        hd = singa.CudnnConvHandle(xd, (r, r), (st, st), (pad, pad), c, k, bias)
+        out, names = kernels_of(dev, lambda: singa.GpuConvForward(xd, wd, bd if bias else None, hd).to_numpy())
+        assert names == {"k_fwd_few"}
+        return out
+
+    got, want, most = run(x, True), conv(x, W, b), conv(np.abs(x), np.abs(W), np.abs(b))
+    assert np.all(np.abs(got - want) <= terms * 2.0 ** -23 * most)
+    assert nl2(got, want) < 2 * terms ** 0.5 * 2.0 ** -24
+    x[n // 2, c - 1, h // 2, w // 2] = np.inf
+    x[0, 0, 0, w - 1] = np.nan
+    got = run(x, False)
+    hit = conv((~np.isfinite(x)).astype(np.float32), np.ones_like(W), 0 * b) > 0
+    assert np.array_equal(~np.isfinite(got), hit)

@@ -248,3 +248,55 @@ def test_conv_split_operands_of_any_magnitude(singa, dev, small, large):
         dw, kw = passes(singa, dev, a, W, b)[2]
         assert kw == {"k_wgrad_oct"}
         assert nl2(dw, wgrad64(a, b)) < 3e-7
+
+
+def test_conv_split_weights_prepared_for_another_workspace(singa, dev):
+    """The size of the workspace decides whether the split kernel runs: weights laid out for a call with one size are not taken by a
+    call with another, and either call gives what it gives without preparation."""
+    import ctypes as C
+
+    from singa_amd import _lib
+    lib = _lib.lib()
+    n, c, h, w, k = 2, 64, 20, 22, 96
+    x, W, dy = operands("normal", 4, n, c, h, w, k, 3)
+    xd, wd, dyd, dxd = (singa.from_numpy(a, dev) for a in (x, W, dy, np.zeros_like(x)))
+    hd = singa.CudnnConvHandle(xd, (3, 3), (1, 1), (1, 1), c, k, False)
+    g = hd.geom
+    full = lib.sgh_conv_workspace_bytes(C.byref(g), _lib.SGH_CONV_DGRAD)
+    space = singa.from_numpy(np.zeros(full // 4 + 64, np.float32), dev)
+
+    def dgrad(size):
+        dxd.CopyFloatDataFromHostPtr(np.full_like(x, 7))
+        (rc, out), names = kernels_of(dev, lambda: (lib.sgh_conv_dgrad_f32(C.byref(g), dyd.ptr, wd.ptr, dxd.ptr, space.ptr, size, dev.stream),
+                                                    dxd.to_numpy()))
+        assert rc == 0
+        return out, names
+
+    def prepare(size):
+        item = (_lib.ConvPrepareItem * 1)()
+        item[0].g, item[0].W, item[0].workspace, item[0].ws_bytes = C.pointer(g), wd.ptr, space.ptr, size
+        assert lib.sgh_conv_dgrad_prepare_multi(item, 1, 0, dev.stream) == 0
+
+    plain = full
+    while dgrad(plain)[1] == {"k_conv_split"}:   # (a size that is too little for it and enough for the fp32 kernel)
+        plain //= 2
+    want = {size: dgrad(size) for size in (full, plain)}
+    assert want[full][1] == {"k_conv_split"} and want[plain][1] == {"k_dgrad3x3"}
+    for prepared in (full, plain):
+        for called in (full, plain):
+            prepare(prepared)
+            got, names = dgrad(called)
+            assert names == want[called][1] and np.array_equal(got, want[called][0]), (prepared, called)
+
+
+def test_conv_wgrad_octets_workspace_is_an_image_per_cu(dev):
+    """The partial images of the octet kernel: one for each of the card's 256 CUs at most, however many pixels there are."""
+    import ctypes as C
+
+    from singa_amd import _lib
+    lib, cus = _lib.lib(), 256
+    for n, c, h, w, k in WGRAD_OCTET_LAYERS + [(37, 71, 106, 112, 132), (64, 154, 37, 27, 670), (128, 64, 112, 112, 64)]:
+        g = _lib.ConvGeom()
+        assert lib.sgh_conv_geom_init(C.byref(g), n, c, h, w, k, 3, 3, 1, 1, 1, 1) == 0
+        tiles = ((k + 63) // 64) * ((c + 63) // 64) * ((w + 31) // 32)
+        assert lib.sgh_conv_workspace_bytes(C.byref(g), _lib.SGH_CONV_WGRAD) <= max(cus, tiles) * 64 * 64 * 9 * 4
