@@ -9,11 +9,13 @@ synthetic seeded inputs whose forward activations are already resident in HBM.
 
 Prints ONE JSON line: the whole-job images/s (mean over the timed steps; median and minimum of the
 per-step HIP event times as extra keys) plus
-  roofline     -- the dominant kernel family (fp32 MFMA conv dgrad + wgrad kernels):
+  roofline     -- the dominant kernel family (conv dgrad + wgrad kernels on matrix instructions):
                   algorithmic FLOPs / measured kernel time (HIP events on the kernels' stream),
-                  against the MI355X fp32 matrix peak; `traffic` = HBM bytes per step of the same
-                  launches, read from the rocprofv3 counter summary under profiles/ when that
-                  summary was taken on the kernels this run launched (null otherwise);
+                  against the MI355X fp32 matrix peak (the kernels on split operands form six
+                  bfloat16 products for an fp32 one: `peak_split` is their ceiling); `traffic` =
+                  HBM bytes per step of the same launches, read from the rocprofv3 counter summary
+                  under profiles/ when that summary was taken on the kernels this run launched
+                  (null otherwise);
   hbm_kernels  -- the bandwidth-bound kernel families: algorithmic bytes / measured time against
                   the HBM3E peak;
   cpu_baseline -- the CPU oracle replaying the same tape on the host cores, on a bounded sample
@@ -277,12 +279,13 @@ def main():
     workload_key = "%s N=%d %s%s" % (args.config, args.batch, args.storage, " no-fusion" if args.no_fusion else "")
     roofline = {
         "bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
+        "peak_split": None if half else round(PEAK_16BIT_MFMA_TFLOPS / 6, 1),
         "frac": round(achieved / peak, 4),
         "traffic": traffic_from_profile(workload_key, kernels),
         "traffic_unit": "HBM bytes per step over the same launches (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated on a "
                         "streaming kernel; from profiles/%s, null when that summary covers other kernels or another workload)"
                         % os.path.basename(TRAFFIC_PROFILE),
-        "kernel": "%s MFMA conv dgrad + wgrad kernels (%s; %d launches/step)"
+        "kernel": "%s conv dgrad + wgrad kernels on matrix instructions (%s; %d launches/step)"
                   % ("16-bit" if half else "fp32", ", ".join(kernels), launches // prof_steps),
         "flop_per_step": flop / prof_steps, "kernel_ms_per_step": round(ms / prof_steps, 4),
         "timing": "HIP events attached to each dispatch (the kernel's own start and end) in %d extra steps with all "

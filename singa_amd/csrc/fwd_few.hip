@@ -135,7 +135,7 @@ struct FfPlan {
 
 FfPlan plan(const sgh_conv_geom *g) {
   FfPlan p{};
-  if (g->groups > 1 || g->C < 1 || g->C >= 8 || g->R != g->S || (g->R != 3 && g->R != 5 && g->R != 7)) return p;
+  if (sgh_env().fwd_fewc_off || g->groups > 1 || g->C < 1 || g->C >= 8 || g->R != g->S || (g->R != 3 && g->R != 5 && g->R != 7)) return p;
   if (g->stride_h != g->stride_w || g->Q > kPixels || g->P < 1 || g->Q < 1) return p;
   const size_t lim = size_t(1) << 31;
   const size_t vh = size_t(g->P) * g->stride_h + g->R - 1;

@@ -11,8 +11,8 @@
 // groups of 2 x 2 wavefronts, each walking half of the workgroup's rows with LDS of its own; the sums meet in LDS at the end, so
 // that one partial image per CU goes through memory.  A group walks a strip of up to 32 columns down the images, in "virtual"
 // rows (an image is its P rows and a row of zeros): per iteration RPI new rows of dy and of x are fetched into registers while
-// the previous ones are multiplied, then split and written; x rows live in a ring of RPI + 2.  Rows of OCS octets: the columns
-// beyond Q are zeros on both sides.
+// the previous ones are multiplied, then split and written; x rows live in a ring of RPI + 2.  Rows of OCS octets (one, two or
+// four): the columns beyond Q are zeros on both sides.
 //
 // The sums of the workgroups of a (k, c) tile are added in ascending order by k_wgrad_oct_reduce.
 //
@@ -462,8 +462,8 @@ WoPlan plan(const sgh_conv_geom *g) {
   const size_t pixels = size_t(g->N) * g->P * g->Q, lim = size_t(1) << 29;
   if (pixels * g->C >= lim || pixels * g->K >= lim) return p;
   // Few channels leave the 64 columns of a tile empty (their nine taps are columns to the fp32 kernels: 3, 11 and 25 of 64
-  // channels 0.6 times as fast, 39 and more 1.1 to 2.4 times), and below 0.4 G products a launch is not worth its partial
-  // images (0.14 to 0.3 G: 0.94 to 1.0 times, and the shorter chains of the fp32 kernel are the more exact ones).
+  // channels 0.6 times as fast, 39 and more 1.1 to 2.4 times).  Below 0.7 G products a launch is short beside its partial images:
+  // 0.13 to 0.67 G, 55 layers, 0.9 to 1.5 times as fast, and the rule that would tell those apart is not there.
   if (20 * g->C < 11 * 64 * ((g->C + 63) / 64) || double(pixels) * g->K * g->C * 9 < 7e8) return p;
   const int oc = (g->Q + 7) / 8;
   p.strips = (oc + 3) / 4;

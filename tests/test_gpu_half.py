@@ -969,7 +969,7 @@ def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
 
 
 # layers that the octet weight gradient (wgrad_oct16.hip) takes: rows of one to four octets and of several strips, whole and ragged
-# octets and channels, odd and even planes of stride 2, rows that do not divide the iterations; and two that it does not take
+# octets and channels, odd and even planes of stride 2, rows that do not divide the iterations; and three that it does not take (50 x 512 x 7 x 7, 3 x 65 and 5 x 100)
 WGRAD_OCTET16_CASES = [
     # N, C, H, W, K, stride
     (26, 568, 59, 8, 43, 1), (77, 464, 61, 6, 22, 1), (50, 512, 7, 7, 130, 1), (55, 600, 36, 9, 26, 1), (23, 601, 56, 13, 28, 1),
@@ -1037,6 +1037,7 @@ def test_conv_wgrad_octets_16bit_non_finite(singa, dev, kind, stride, bad):
                                                   .reshape(-1, C).copy()) for i in range(3) for j in range(3)], -1)
         want = want.numpy().reshape(K, C, 3, 3)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
     fin = np.isfinite(want)
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-2, atol=1e-1)
 

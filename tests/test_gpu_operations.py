@@ -1151,12 +1151,14 @@ def test_conv_split_operands_non_finite(singa, dev, n, c, h, w, k, where, bad):
     got = (singa.GpuConvForward(xd, wd, bd, hd).to_numpy(), singa.GpuConvBackwardx(dyd, wd, xd, hd).to_numpy())
     for g, ref in zip(got, want):
         assert np.array_equal(np.isnan(g), np.isnan(ref)) and np.array_equal(np.isposinf(g), np.isposinf(ref))
+        assert np.array_equal(np.isneginf(g), np.isneginf(ref))
         fin = np.isfinite(ref) & np.isfinite(g)
         np.testing.assert_allclose(g[fin], ref[fin], rtol=1e-4, atol=1e-4)
 
 
-# sizes of the split-operand weight gradient (wgrad_oct.hip): rows of one to four octets and of several strips, ragged octets and
-# channels, rows that do not divide the iterations, and (few products) its neighbours
+# sizes around the split-operand weight gradient (wgrad_oct.hip): rows of two to four octets and of several strips, ragged octets
+# and channels, rows that do not divide the iterations, and layers that the rule leaves to its neighbours (all of at most eight
+# columns among them; test_gpu_split_operands.py has such that it takes)
 WGRAD_OCTET_CASES = [
     # n, c, h, w, k
     (64, 64, 14, 7, 130), (70, 129, 7, 8, 150), (40, 70, 13, 9, 257), (30, 64, 17, 16, 200), (9, 100, 25, 17, 230),
@@ -1193,7 +1195,8 @@ def test_conv_wgrad_octets(singa, dev, n, c, h, w, k):
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.4e38])
 def test_conv_wgrad_octets_non_finite(singa, dev, bad):
     """Non-finite values (and those whose bfloat16 rounding is infinite) reach the weights whose products they are in, the
-    products with padding among them (zeros: NaN), and no others."""
+    products with padding among them (zeros: NaN), and no others.  (Of a layer that the rule leaves to the fp32 instructions;
+    test_gpu_split_operands.py has the others.)"""
     n, c, h, w, k = 12, 70, 20, 30, 140
     rg = rng(8)
     x, dy = randn(rg, n, c, h, w), randn(rg, n, k, h, w)
@@ -1210,6 +1213,7 @@ def test_conv_wgrad_octets_non_finite(singa, dev, bad):
         want = np.stack([np.einsum("kp,pc->kc", d2, xp[:, :, r:r + h, s:s + w].transpose(0, 2, 3, 1).reshape(-1, c))
                          for r in range(3) for s in range(3)], -1).reshape(k, c, 3, 3).astype(np.float32)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
     fin = np.isfinite(want) & np.isfinite(got)
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-5)
 
