@@ -4,6 +4,7 @@
 #define SINGA_AMD_CSRC_CONV_SPLIT_H_
 
 #include "common.h"
+#include "split_parts.h"
 
 bool sgh_conv_split_supported(const sgh_conv_geom *g);
 size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g);   // weight fragments, then the partial tiles
@@ -14,11 +15,6 @@ int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps
 // `W`: the same weights again, for what the fragments cannot hold
 int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s,
                        const char *tag, bool dgrad, const float *bias, bool accumulate);
-
-// Operands are multiplied by this before they are split, results by the square of its inverse: three bfloat16 values hold 24 bits
-// of a number from 2^-110 on, and with this all bits of every fp32 number down to the smallest subnormal one.  What comes out
-// beyond 2^96 is formed again anyway.
-constexpr float kSplitScale = 65536.f, kSplitUnscale = 1.f / kSplitScale / kSplitScale;
 
 constexpr int kSplitWeightLds = 512 * 9;   // floats of LDS that a workgroup below needs
 
@@ -60,11 +56,8 @@ __device__ __forceinline__ void sgh_conv_split_weights_block(const float *__rest
       uint16_t part[3][8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float w = (q % RS & 1 ? -kSplitScale : kSplitScale) * src[j * 9];
-        auto up = [](uint16_t b) { return __builtin_bit_cast(float, unsigned(b) << 16); };
-        auto down = [](float f) { return __builtin_bit_cast(uint16_t, __bf16(f)); };
-        const uint16_t p0 = down(w), p1 = down(w - up(p0));
-        part[0][j] = p0, part[1][j] = p1, part[2][j] = down(w - up(p0) - up(p1));
+        const Parts w = split2(q % RS & 1 ? -src[j * 9] : src[j * 9], 0.f);
+        part[0][j] = uint16_t(w.p[0]), part[1][j] = uint16_t(w.p[1]), part[2][j] = uint16_t(w.p[2]);
       }
       uint16_t *dst = wt + (size_t(q) * cblocks + cb) * 1536 + lane * 8;
 #pragma unroll

@@ -44,13 +44,7 @@
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int NT = 512, NW = NT / 64, KC = 16;
 constexpr int kOOB = int(0x80000000u);
@@ -62,29 +56,14 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
 }
 
-__device__ __forceinline__ unsigned pack2(float a, float b) {
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, bf16x2));
-}
-__device__ __forceinline__ float lo_f(unsigned p) { return __builtin_bit_cast(float, p << 16); }
-__device__ __forceinline__ float hi_f(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
-
 // Eight fp32 values -> the three parts of each, packed
 __device__ __forceinline__ void split8(const float (&v)[8], v4u (&part)[3]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float a = v[2 * i] * kSplitScale, b = v[2 * i + 1] * kSplitScale;
-    const unsigned p0 = pack2(a, b);
-    const float ra = a - lo_f(p0), rb = b - hi_f(p0);
-    const unsigned p1 = pack2(ra, rb);
-    part[0][i] = p0, part[1][i] = p1, part[2][i] = pack2(ra - lo_f(p1), rb - hi_f(p1));
+    const Parts s = split2(v[2 * i], v[2 * i + 1]);
+    part[0][i] = s.p[0], part[1][i] = s.p[1], part[2][i] = s.p[2];
   }
 }
-
-__device__ __forceinline__ v16f mfma(v4u a, v4u b, v16f c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
 
 struct ScArgs {
   const float *in;

@@ -21,16 +21,9 @@
 // own and added to the accumulator once; without that the error is up to 1.5 times that of the fp32 instructions behind a
 // ReLU (whose zeros cost those no rounding), and the kernel 7 per cent faster.
 #include "common.h"
-#include "conv_split.h"
+#include "split_parts.h"
 
 namespace {
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int NT = 512, GT = 256;   // threads of a workgroup, of a group
 constexpr int PARTS = 3;
@@ -40,17 +33,6 @@ constexpr int kAcc = 9 * 16 * 64;   // accumulators of a wavefront
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
 }
-
-__device__ __forceinline__ v16f mfma(v4u a, v4u b, v16f c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ unsigned pack2(float a, float b) {
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, bf16x2));
-}
-__device__ __forceinline__ float lo_f(unsigned p) { return __builtin_bit_cast(float, p << 16); }
-__device__ __forceinline__ float hi_f(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
-__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
 
 struct WoArgs {
   const float *dy, *x;
@@ -83,12 +65,10 @@ struct Octet {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const unsigned ua = raw[i / 2][2 * i % 4], ub = raw[i / 2][2 * i % 4 + 1];
-      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) * kSplitScale : 0.f;
-      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) * kSplitScale : 0.f;
-      const unsigned p0 = pack2(a, b);
-      const float ra = a - lo_f(p0), rb = b - hi_f(p0);
-      const unsigned p1 = pack2(ra, rb);
-      out[0][i] = p0, out[1][i] = p1, out[2][i] = pack2(ra - lo_f(p1), rb - hi_f(p1));
+      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) : 0.f;
+      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) : 0.f;
+      const Parts s = split2(a, b);
+      out[0][i] = s.p[0], out[1][i] = s.p[1], out[2][i] = s.p[2];
     }
   }
 };
@@ -154,11 +134,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   };
   auto edge_get = [&](int off) -> unsigned { return __builtin_amdgcn_raw_buffer_load_b32(rx, off, 0, 0); };
   auto put_edge = [&](unsigned raw, int slot, int c, int side) {
-    const float v = __builtin_bit_cast(float, raw) * kSplitScale;
-    const unsigned p0 = pack2(v, 0.f);
-    const float r = v - lo_f(p0);
-    const unsigned p1 = pack2(r, 0.f);
-    const uint16_t part[PARTS] = {uint16_t(p0), uint16_t(p1), uint16_t(pack2(r - lo_f(p1), 0.f))};
+    const Parts s = split2(__builtin_bit_cast(float, raw), 0.f);
+    const uint16_t part[PARTS] = {uint16_t(s.p[0]), uint16_t(s.p[1]), uint16_t(s.p[2])};
 #pragma unroll
     for (int i = 0; i < PARTS; ++i)
       *reinterpret_cast<uint16_t *>(xs + slot * S::XROW + i * S::XPART + c * S::XP * 16 + (side ? 16 + OCS * 16 : 14)) = part[i];
