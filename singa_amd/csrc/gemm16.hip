@@ -2,16 +2,19 @@
 // accumulation on v_mfma_f32_32x32x16_{f16,bf16} and one rounding at the store -- the Linear layers of
 // a half model (the reference calls cublasHgemm: src/core/tensor/tensor_math_cuda.h:1163-1187).
 //
-// A workgroup of four wavefronts owns a 64 x 64 tile of C, a wavefront a 32 x 32 quarter.  Both matrix
+// Three kernels; none splits the reduction over workgroups and every sum is taken in a fixed order: results are run-to-run
+// identical.  k_gemm16_tile (many output tiles) and k_gemm16_split (few) do the work; k_gemm16 is left with what neither can
+// address: operands of 2 GB and more, and fewer than eight rows, columns or reduction indices against many of the others.
+//
+// k_gemm16: a workgroup of four wavefronts owns a 64 x 64 tile of C, a wavefront a 32 x 32 quarter.  Both matrix
 // operands want, per lane, eight consecutive reduction indices of one tile row, so both LDS tiles are
-// [row][k] with k contiguous (pitch 32 + 8 halves: 16-byte reads without bank conflicts).  How a tile is
-// staged depends on which index is contiguous in memory: with k contiguous (A not transposed, B
-// transposed) a thread copies one octet with a 16-byte load; with the row index contiguous (A transposed,
-// B not transposed) it loads eight rows of one k with a 16-byte load and writes them as eight 2-byte LDS
+// [row][k] with k contiguous (pitch 32 + 8 halves: 16-byte reads without bank conflicts).  With k contiguous in memory
+// a thread copies one octet with a 16-byte load; with the row index contiguous
+// it loads eight rows of one k with a 16-byte load and writes them as eight 2-byte LDS
 // stores; pointers, pitches or edges that do not allow the 16-byte access fall back to single elements.
-// This kernel does not split the reduction.  Problems with few output tiles take the second kernel of this file, which splits it
-// over the wavefronts of a workgroup and adds their sums in a fixed order: results are run-to-run identical either way.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "storage.h"
@@ -272,12 +275,255 @@ void launch_split(int tile, int waves, const uint16_t *A, int lda, const uint16_
 #undef SGH_SPLIT_CASE
 }
 
-// Whether the split kernel takes the problem, its tile and the wavefronts that share one.  Measured in binary16 (us, tiled
-// kernel / 32-wide / 16-wide tiles, 8 wavefronts; NN = neither operand transposed, NT = B transposed):
-//   256 x 1000 x 2048 NN    42 / 10.2 / 19        128 x 10 x 4096 NN    133 / 13.5 / 8.9
-//   1024 x 1024 x 1024 NN   23 / 17.3, NT 16.9 / 16.9    four 32-wide tiles per CU;
-//   1000 x 2048 x 512 NN    14.5 / 17.2                  eight: the tiled kernel loads half the bytes per product
-// 16-wide tiles win while 32-wide ones leave half of the CUs without a workgroup; four wavefronts are enough for short
+// ---- many output tiles -----------------------------------------------------------------------------------------------
+// A workgroup of four wavefronts owns a BT x BT tile of C (BT = 64 or 128, a wavefront a quarter).  Chunks of 64 reduction
+// indices go through two register sets (requested two chunks ahead) into two LDS buffers, one barrier per chunk.
+// A tile is kept in LDS as it lies in memory: [row][k] where the reduction index is the contiguous one (16-byte reads are the
+// fragments), [k][row] where the row is (ds_read_b64_tr_b16 hands a lane four k of its row).  Either way a load is 16 bytes of
+// one line of the matrix at any element alignment.  Rows come in octets, the last of which ends with the matrix and overlaps its
+// neighbour (nothing is read beyond an operand, no masks); reduction indices beyond K are zeros: whole lines where k is a line,
+// else the last octet ends with K too and is shifted down.
+//   Bound by the serial phases of a chunk (request, 16 KB to LDS, 32 KB from it, 64 matrix instructions: 0.33 us with a CU to
+// itself), not by the loads: four register sets instead of two were 5-10 % slower.  So several workgroups per CU, or two groups of
+// four wavefronts that take alternate chunks and add their sums in order.  bfloat16, before (k_gemm16 or k_gemm16_split) -> now, us:
+// 256 x 2048 x 1000 NT 9.8 -> 6.7, 2048 x 1000 x 256 TN 12.1 -> 5.6, 1024^3 NN 16.8 -> 7.0, 1001 x 2049 x 333 NN 31.8 -> 9.4, 1500^3 NT
+// 169 -> 23, 2048 x 4096 x 1200 NT 71 -> 30 (670 TFLOP/s).  An empty launch is 3.7 of each.
+constexpr int TK = 64, NOT_THERE = int(0x80000000u);
+
+template <bool KC, int BT>
+struct Panel {
+  static constexpr int N = BT / 32;   // 16-byte loads of a thread and chunk
+  rsrc_t r;
+  int off[KC ? N : 1];   // byte offset of the thread's loads at reduction index 0 (rows apart) / of its first line
+  int ld2, K, k;         // pitch in bytes; the thread's own reduction index in a chunk
+  u32x4 v[2][N];
+  __device__ __forceinline__ void init(const uint16_t *p, int ld, unsigned bytes, int row0, int rows, int K_) {
+    const int t = threadIdx.x & 255;
+    r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p), 0, bytes, 0x00020000);
+    ld2 = ld * 2, K = K_;
+    if constexpr (KC) {
+      k = (t & 7) * 8;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const int row = row0 + 32 * j + (t >> 3), base = min(row & ~7, rows - 8);
+        off[j] = (base + (row & 7)) * ld2 + k * 2;
+      }
+    } else {
+      k = t / (BT / 8);
+      off[0] = k * ld2 + min(row0 + (t % (BT / 8)) * 8, rows - 8) * 2;
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void request(int k0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if constexpr (KC) {
+        const int over = k0 + k + 8 - K;   // beyond K: the octet that ends with K, or nothing
+        v[S][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, over >= 8 ? NOT_THERE : off[j] + 2 * (k0 - max(over, 0)), 0, 0));
+      } else {
+        constexpr int LINES = 256 / (BT / 8);
+        v[S][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, k0 + k + LINES * j < K ? off[0] + LINES * j * ld2 : NOT_THERE, k0 * ld2, 0));
+      }
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void stage(uint16_t *tile, int k0) {
+    const int t = threadIdx.x & 255;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if constexpr (KC) {
+        const int row = 32 * j + (t >> 3);
+        u32x4 w = v[S][j];
+        if (k0 + TK > K) {   // (uniform: the last chunk)
+          const int over = k0 + k + 8 - K;
+          if (over > 0 && over < 8) {
+            if (over & 4) w = u32x4{w[2], w[3], 0u, 0u};
+            if (over & 2) w = u32x4{w[1], w[2], w[3], 0u};
+            if (over & 1)
+              w = u32x4{__builtin_amdgcn_alignbyte(w[1], w[0], 2), __builtin_amdgcn_alignbyte(w[2], w[1], 2),
+                        __builtin_amdgcn_alignbyte(w[3], w[2], 2), w[3] >> 16};
+          }
+        }
+        *reinterpret_cast<u32x4 *>(tile + row * TK + (((t & 7) ^ ((row >> 1) & 7)) * 8)) = w;
+      } else {
+        const int line = k + 256 / (BT / 8) * j, oct = t % (BT / 8);
+        *reinterpret_cast<u32x4 *>(tile + line * BT + (oct ^ (BT == 64 ? (line & 2) << 1 : (line & 3) << 2)) * 8) = v[S][j];
+      }
+    }
+  }
+  // fragments of 32-row tile `tile32` for matrix steps k2 and k2 + 1 (16 reduction indices each)
+  static __device__ __forceinline__ void fragments(const uint16_t *tile, int tile32, int k2, u32x4 (&f)[2]) {
+    const int lane = threadIdx.x & 63, lh = lane >> 5;
+    if constexpr (KC) {
+      const int row = 32 * tile32 + (lane & 31);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        f[s] = *reinterpret_cast<const u32x4 *>(tile + row * TK + (((2 * (k2 + s) + lh) ^ ((row >> 1) & 7)) * 8));
+    } else {
+      typedef __attribute__((address_space(3))) const uint16_t lds_u16;
+      const int line = (lane >> 2) & 3, oct = 4 * tile32 + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+      const unsigned a = unsigned(size_t((lds_u16 *)(tile + (16 * k2 + 8 * lh + line) * BT +
+                                                     (oct ^ (BT == 64 ? (line & 2) << 1 : line << 2)) * 8 + (lane & 1) * 4)));
+      u32x2 q[4];
+      // (one block with its own wait: the builtin waits for every load under way)
+      if constexpr (BT == 64)
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %4 offset:512\n\t"
+            "ds_read_b64_tr_b16 %2, %4 offset:2048\n\tds_read_b64_tr_b16 %3, %4 offset:2560\n\ts_waitcnt lgkmcnt(0)"
+            : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3]) : "v"(a) : "memory");
+      else
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %4 offset:1024\n\t"
+            "ds_read_b64_tr_b16 %2, %4 offset:4096\n\tds_read_b64_tr_b16 %3, %4 offset:5120\n\ts_waitcnt lgkmcnt(0)"
+            : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3]) : "v"(a) : "memory");
+#pragma unroll
+      for (int s = 0; s < 2; ++s) f[s] = u32x4{q[2 * s][0], q[2 * s][1], q[2 * s + 1][0], q[2 * s + 1][1]};
+    }
+  }
+};
+
+template <bool BF16, bool AK, bool BKc, int BT, int KS>
+__global__ __launch_bounds__(256 * KS) void k_gemm16_tile(const uint16_t *__restrict__ A, int lda, unsigned a_bytes,
+                                                     const uint16_t *__restrict__ B, int ldb, unsigned b_bytes,
+                                                     uint16_t *__restrict__ C, int ldc, int M, int N, int K, int mtiles, int tiles,
+                                                     float alpha, float beta) {
+  constexpr int TM = BT / 64, HALF = BT * TK, OP = BT + 8;
+  static_assert(OP * BT <= 4 * HALF && 2 * BT * BT <= 4 * HALF, "");
+  __shared__ __align__(16) uint16_t lds_all[KS][2][2 * HALF];
+  // workgroup w runs on XCD w % 8: an XCD takes neighbouring tiles, which share their panels in its L2
+  const int per = (tiles + 7) >> 3, l = (int(blockIdx.x) & 7) * per + (int(blockIdx.x) >> 3);
+  if ((int(blockIdx.x) >> 3) >= per || l >= tiles) return;
+  const int m0 = (l % mtiles) * BT, n0 = (l / mtiles) * BT;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = (wave >> 1) & 1, wn = wave & 1;
+  const int group = wave >> 2;   // of four wavefronts: chunks group, group + KS, ...
+  uint16_t (*const lds)[2 * HALF] = lds_all[group];
+  Panel<AK, BT> pa;
+  Panel<BKc, BT> pb;
+  pa.init(A, lda, a_bytes, m0, M, K);
+  pb.init(B, ldb, b_bytes, n0, N, K);
+  f32x16 acc[TM][TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  auto multiply = [&](const uint16_t *st) {
+#pragma unroll
+    for (int k2 = 0; k2 < TK / 16; k2 += 2) {
+      u32x4 fa[TM][2], fb[TM][2];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) Panel<AK, BT>::fragments(st, wm * TM + i, k2, fa[i]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) Panel<BKc, BT>::fragments(st + HALF, wn * TM + i, k2, fb[i]);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) acc[i][j] = mfma16<BF16>(fb[j][s], fa[i][s], acc[i][j]);   // rows: n, columns: m
+    }
+  };
+  const int rounds = (K + KS * TK - 1) / (KS * TK), kg = group * TK;
+  auto at = [&](int c) { return c * (KS * TK) + kg; };   // first reduction index of the group's chunk c (beyond K: zeros)
+  auto request = [&](auto SET, int c) {
+    constexpr int S = decltype(SET)::value;
+    pa.template request<S>(at(c)), pb.template request<S>(at(c));
+  };
+  auto stage = [&](auto SET, int c) {
+    constexpr int S = decltype(SET)::value;
+    pa.template stage<S>(lds[S], at(c)), pb.template stage<S>(lds[S] + HALF, at(c));
+  };
+  // chunk c of the group: request what takes its registers, multiply, hand the next one to the other buffer; false at the end
+  auto step = [&](auto SET, int c) {
+    constexpr int S = decltype(SET)::value;
+    __syncthreads();
+    request(SET, c + 2);
+    multiply(lds[S]);
+    if (c + 1 >= rounds) return false;
+    stage(std::integral_constant<int, S ^ 1>{}, c + 1);
+    return true;
+  };
+  typedef std::integral_constant<int, 0> Set0;
+  typedef std::integral_constant<int, 1> Set1;
+  request(Set0{}, 0);
+  request(Set1{}, 1);
+  stage(Set0{}, 0);
+  for (int c = 0; step(Set0{}, c) && step(Set1{}, c + 1); c += 2) {
+  }
+  if constexpr (KS > 1) {   // the groups' sums in their order
+    static_assert(BT == 64, "");
+    __syncthreads();
+    float *const part = reinterpret_cast<float *>(lds_all[group]) + (wave & 3) * 1024;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[v * 64 + lane] = acc[0][0][v];
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int g = 1; g < KS; ++g)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[0][0][v] += reinterpret_cast<const float *>(lds_all[g])[(wave & 3) * 1024 + v * 64 + lane];
+    }
+  }
+  // the tile leaves through LDS as [m][n] rows of octets; a lane holds four neighbouring n of one m
+  __syncthreads();
+  uint16_t *const o = lds_all[0][0];
+  if (group == 0)
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; v += 4) {
+        const int row = (wm * TM + i) * 32 + (lane & 31), col = (wn * TM + j) * 32 + 2 * v + 4 * (lane >> 5);
+        const int gm = min((m0 + row) & ~7, M - 8) + (row & 7), gn = min((n0 + col) & ~7, N - 8) + (col & 7);
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = alpha * acc[i][j][v + e];
+        }
+        if (beta != 0.f) {   // (an element of two octets is stored by the first of them only, below)
+          const uint16_t *c = C + size_t(gm) * ldc + gn;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] += beta * (BF16 ? sgh_bf16_to_f32(c[e]) : sgh_f16_to_f32(c[e]));
+        }
+        const u32x2 q = BF16 ? u32x2{sgh_pack2_bf16(x[0], x[1]), sgh_pack2_bf16(x[2], x[3])}
+                             : u32x2{sgh_pack2_f16(x[0], x[1]), sgh_pack2_f16(x[2], x[3])};
+        *reinterpret_cast<u32x2 *>(o + row * OP + col) = q;
+      }
+  __syncthreads();
+  constexpr int OCT = BT / 8, STEP = 256 * KS / OCT;
+#pragma unroll
+  for (int row = t / OCT; row < BT; row += STEP) {
+    const int go = n0 + (t % OCT) * 8;
+    const int gm = min((m0 + row) & ~7, M - 8) + (row & 7), gn = min(go, N - 8);
+    if (gm < ((m0 + row) & ~7) || go >= N) continue;   // (the row or the whole octet belongs to its neighbour)
+    uint16_t *dst = C + size_t(gm) * ldc + gn;
+    const uint16_t *src = o + row * OP + (t % OCT) * 8;
+    if (beta == 0.f || gn == go) __builtin_memcpy(dst, src, 16);
+    else
+      for (int e = go - gn; e < 8; ++e) dst[e] = src[e];
+  }
+}
+
+template <bool BF16, bool AK, bool BKc>
+void launch_tile(int bt, int ks, const uint16_t *A, int lda, const uint16_t *B, int ldb, uint16_t *C, int ldc, int M, int N, int K,
+                 float alpha, float beta, hipStream_t s) {
+  const unsigned ab = unsigned((size_t(AK ? M - 1 : K - 1) * lda + (AK ? K : M)) * 2);
+  const unsigned bb = unsigned((size_t(BKc ? N - 1 : K - 1) * ldb + (BKc ? K : N)) * 2);
+  const int mt = (M + bt - 1) / bt, tiles = mt * ((N + bt - 1) / bt);
+  const dim3 grid(unsigned((tiles + 7) / 8 * 8));
+#define SGH_TILE_CASE(BT_, KS_)                                                                                                     \
+  hipLaunchKernelGGL((k_gemm16_tile<BF16, AK, BKc, BT_, KS_>), grid, dim3(256 * KS_), 0, s, A, lda, ab, B, ldb, bb, C, ldc, M, N,   \
+                     K, mt, tiles, alpha, beta)
+  if (bt == 128) SGH_TILE_CASE(128, 1);
+  else if (ks == 2) SGH_TILE_CASE(64, 2);
+  else SGH_TILE_CASE(64, 1);
+#undef SGH_TILE_CASE
+}
+
+// The split kernel's tile and the wavefronts that share one, and whether it can take the problem at all.  16-wide tiles win while
+// 32-wide ones leave half of the CUs without a workgroup (128 x 10 x 4096 NN 8.7 / 13.5 us); four wavefronts are enough for short
 // reductions (784 x 1000 x 128: 5.0 / 5.1 us with 4 / 8), 16 gain nothing over 8 (512 x 1024 x 2048: 17.6 / 17.5).
 bool split_plan(int M, int N, int K, int *tile, int *waves) {
   const long t32 = long((M + 31) / 32) * ((N + 31) / 32), cus = sgh_num_cus();
@@ -285,6 +531,27 @@ bool split_plan(int M, int N, int K, int *tile, int *waves) {
   *tile = 2 * t32 < cus ? 16 : 32;
   *waves = K < 256 ? 4 : 8;
   return (M + *tile - 1) / *tile <= 65535;
+}
+
+// Whether the tiled kernel is the better one where both can run.  Beyond one 32-wide tile per CU it is (us, split / tiled, bfloat16:
+// 512 x 1024 x 2048 NN 16.8 / 10.2, 1024^3 NN 16.5 / 7.0, 48 x 6256 x 2536 NT 23.5 / 13.9), below where there is much to do (2000 x
+// 100 x 2000 NN, 504 000 tiles times indices, 10.5 / 10.1; but 20 x 8000 x 1000 NT, 250 000, 5.1 / 6.4 and 8 x 1608 x 2824 NT,
+// 144 000, 4.9 / 12.6); with rows at odd elements the split kernel's loads take several times as long, and the line lies lower
+// (807 x 211 x 6728 NN 79 / 35, 220 x 927 x 1271 NN, 258 000, 18.5 / 9.5, 116 x 181 x 5879 NN, 141 000, 43 / 32, but 87 x 133 x 2207
+// NT, 33 000, 12.3 / 13.8).
+bool tile_pays(int M, int N, int K, bool odd) {
+  const long t32 = long((M + 31) / 32) * ((N + 31) / 32);
+  return t32 > sgh_num_cus() || t32 * K > (odd ? 120000 : 400000);
+}
+
+// The tiled kernel's tile and groups.  128-wide tiles (half the loads per product) once they give every CU one and the reduction
+// is long enough to matter (64 / 128: 2048 x 4096 x 1200 NT 46 / 30 us, 512 tiles; 700 x 6000 x 700 NT 18.5 / 17.7, 282; 1500^3 23.5 /
+// 24.9, 144; 2232 x 2280 x 40 TN 6.4 / 7.1).  Two groups halve the chain of a workgroup that has its CU to itself (1024^3 8.4 / 7.0 with
+// 256 tiles, 700 x 700 x 6000 39 / 31 with 121; 1813 x 597 x 964 11.8 / 12.1 with 290); four gain nothing more (6.9, 31.3).
+void tile_plan(int M, int N, int K, int *bt, int *ks) {
+  const long t64 = long((M + 63) / 64) * ((N + 63) / 64), t128 = long((M + 127) / 128) * ((N + 127) / 128), cus = sgh_num_cus();
+  *bt = t128 > cus && K >= 256 ? 128 : 64;
+  *ks = t64 <= cus && K > 2 * TK ? 2 : 1;
 }
 
 template <bool BF16>
@@ -301,9 +568,21 @@ int gemm16(int transA, int transB, int M, int N, int K, float alpha, const uint1
   if (grid.y > 65535u) return SGH_EUNSUPPORTED;
   hipStream_t st = sgh_stream_of(stream);
   sgh_prof_scope prof("gemm16", 2.0 * M * N * K, st);
-  int tile, waves;
-  if (K > 0 && split_plan(M, N, K, &tile, &waves) && size_t(transA ? K : M) * lda < (size_t(1) << 30) &&
-      size_t(transB ? N : K) * ldb < (size_t(1) << 30)) {   // (operands addressed with 32-bit byte offsets)
+  int tile, waves, bt, ks;
+  const bool small = K > 0 && size_t(transA ? K : M) * lda < (size_t(1) << 30) &&
+                     size_t(transB ? N : K) * ldb < (size_t(1) << 30);   // operands addressed with 32-bit byte offsets
+  const bool split = small && split_plan(M, N, K, &tile, &waves), octets = M >= 8 && N >= 8 && K >= 8;
+  const bool odd = ((lda | ldb) & 1) || ((transA ? M : 0) & 1) || ((transB ? 0 : N) & 1);
+  if (small && octets && !(split && !tile_pays(M, N, K, odd))) {
+    tile_plan(M, N, K, &bt, &ks);
+    if (!transA && transB) launch_tile<BF16, true, true>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
+    else if (!transA) launch_tile<BF16, true, false>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
+    else if (transB) launch_tile<BF16, false, true>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
+    else launch_tile<BF16, false, false>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
+    SGH_LAUNCH_CHECK();
+    return SGH_OK;
+  }
+  if (split) {
     if (!transA && transB) launch_split<BF16, true, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
     else if (!transA) launch_split<BF16, true, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
     else if (transB) launch_split<BF16, false, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);

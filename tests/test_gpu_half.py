@@ -186,6 +186,38 @@ def test_gemm_16bit(singa, dev, kind, M, N, K):
     _same_bits(singa.Mult(et, bt).to_numpy(), singa.Mult(et, bt).to_numpy(), "run to run")
 
 
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1100, 265, 9), (1032, 264, 64), (1031, 270, 65), (265, 1030, 131), (520, 523, 198), (519, 525, 260),
+                                   (513, 770, 127), (2049, 2183, 257)])
+def test_gemm_16bit_tile_edges(singa, dev, kind, M, N, K):
+    """The tiled kernel (more than 256 tiles of 32 x 32): edges that end inside an octet of rows, reductions that end inside an octet,
+    a chunk or leave the second group without one, one group (more than 256 tiles of 64, or at most 128 indices) and two, 128-wide tiles
+    (more than 256 of them); beta and pitches, where an element of two octets must be written once.  Exact: small whole numbers."""
+    from singa_amd import _lib
+    print("gemm tile", kind, M, N, K, flush=True)
+    r = rng(M + N + K)
+    fn = {"f16": _lib.lib().sgh_gemm_f16, "bf16": _lib.lib().sgh_gemm_bf16}[kind]
+    dt = {"f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+
+    def to(rows, cols, pad):   # one leading element and `pad` at the end of a row: any alignment of pointers and rows
+        a = r.integers(-2, 3, size=(rows, cols + pad)).astype(np.float32)
+        t = singa.from_numpy(np.concatenate([[np.float32(0)], a.ravel()]), dev).AsType(dt)
+        return t, t.ptr + 2, a[:, :cols].astype(np.float64)
+    for tA, tB in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        pad = int(r.integers(0, 4))
+        at, ap, a = to(K if tA else M, M if tA else K, pad)
+        bt, bp, b = to(N if tB else K, K if tB else N, pad)
+        ct, cp, c = to(M, N, pad)
+        want = (a.T if tA else a) @ (b.T if tB else b)
+        lda, ldb = (M if tA else K) + pad, (K if tB else N) + pad
+        for beta in (0.0, -1.0):
+            out = ct.Clone()
+            _lib.check(fn(tA, tB, M, N, K, 1.0, ap, lda, bp, ldb, beta, out.ptr + 2, N + pad, dev.stream), "sgh_gemm")
+            want_c = singa.from_numpy((want + beta * c).astype(np.float32), dev).AsType(dt).AsType(singa.kFloat32).to_numpy()
+            got = out.AsType(singa.kFloat32).to_numpy()[1:].reshape(M, N + pad)
+            assert np.array_equal(got[:, :N], want_c), (tA, tB, beta, np.argwhere(got[:, :N] != want_c)[:4])
+            assert np.array_equal(got[:, N:], ct.AsType(singa.kFloat32).to_numpy()[1:].reshape(M, N + pad)[:, N:])
+
 def test_gemm_16bit_alpha_beta_and_pitches(singa, dev):
     """The C ABI directly: alpha / beta in fp32, row pitches larger than the rows, unaligned pointers
     (the element-wise staging path) against float64."""
