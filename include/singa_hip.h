@@ -204,6 +204,9 @@ SGH_API int sgh_softmax_ce_label_errors(void *stream, int *count);
 SGH_API int sgh_softmax_fwd_f32(const float *x, float *p, size_t batch, size_t dim, void *stream);
 SGH_API int sgh_cross_entropy_fwd_f32(const float *p, const int32_t *t, float *loss, size_t batch,
                                       size_t dim, int int_target, void *stream);
+/* Both in one launch: p = softmax(x), loss = cross entropy of p (the bits of the two calls). */
+SGH_API int sgh_softmax_ce_fwd_f32(const float *x, const int32_t *t, float *p, float *loss, size_t batch, size_t dim,
+                                   int int_target, void *stream);
 
 /* Transform<float, Lang> (src/core/tensor/tensor_math_cpp.h:685-689, CUDA tensor_math_cuda.h:284-300):
  * the dense row-major copy of a strided view -- transposed, sliced or broadcast (stride 0, as
@@ -390,6 +393,18 @@ SGH_API int sgh_sgd_momentum_master_bf16(float *p_master, const uint16_t *g, flo
 SGH_API int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const float *A,
                          int lda, const float *B, int ldb, float beta, float *C, int ldc,
                          void *stream);
+/* A dense layer with what surrounds its products, in one launch where the GEMM's split kernel takes the problem (the bits of
+ * the separate calls either way): y[rows][out] = x[rows][in] W[in][out] + bias, then ReLU if `relu`; bias may be NULL
+ * (autograd.Linear forward, python/singa/autograd.py:596-612, :680-695, :420-431). */
+SGH_API int sgh_linear_fwd_f32(const float *x, const float *W, const float *bias, float *y, int rows, int in, int out,
+                               int relu, void *stream);
+/* dx = dy W^T, kept where gate[rows][in] > 0 and zero elsewhere if `gate` is not NULL: the layer's data gradient and the backward
+ * of the ReLU in front of it (python/singa/autograd.py:613-623, :432-439). */
+SGH_API int sgh_linear_bwd_x_f32(const float *dy, const float *W, const float *gate, float *dx, int rows, int in, int out,
+                                 void *stream);
+/* dW = x^T dy and db[out] = the column sums of dy (python/singa/autograd.py:613-623, :696-709). */
+SGH_API int sgh_linear_bwd_wb_f32(const float *x, const float *dy, float *dW, float *db, int rows, int in, int out,
+                                  void *stream);
 /* GEMM<half, Lang> (cublasHgemm in the reference, src/core/tensor/tensor_math_cuda.h:1163-1187): the
  * Linear layers of a half model.  A, B, C are binary16 (bfloat16); products of the stored values are
  * accumulated in fp32 on the 16-bit matrix instructions (v_mfma_f32_32x32x16), alpha and beta apply in

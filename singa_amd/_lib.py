@@ -151,6 +151,10 @@ SIGNATURES = {
                                                C.c_int, vp]),
     "sgh_gemm_f32": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, vp, C.c_int,
                                vp, C.c_int, C.c_float, vp, C.c_int, vp]),
+    "sgh_linear_fwd_f32": (C.c_int, [vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, C.c_int, vp]),
+    "sgh_linear_bwd_x_f32": (C.c_int, [vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, vp]),
+    "sgh_linear_bwd_wb_f32": (C.c_int, [vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, vp]),
+    "sgh_softmax_ce_fwd_f32": (C.c_int, [vp, vp, vp, vp, sz, sz, C.c_int, vp]),
     "sgh_sum_rows_f32": (C.c_int, [vp, vp, C.c_int, C.c_int, vp]),
     "sgh_add_row_f32": (C.c_int, [vp, vp, C.c_int, C.c_int, vp]),
     "sgh_conv_geom_init": (C.c_int, [C.POINTER(ConvGeom)] + [C.c_int] * 11),

@@ -123,10 +123,20 @@ struct sgh_prof_kernel_scope {
       hipLaunchKernelGGL(kern, grid, block, lds, stream, __VA_ARGS__);                                           \
   } while (0)
 
+// What a dense layer does around its products, in the launch that computes them: C[m][n] = gate[m][n] > 0 ? relu(r + bias[n]) : 0
+// with the result r (each part if its pointer or flag is set; gate dense, pitch N), and colsum[n] = sum of op(B)'s column n, rows in
+// ascending order.  The bits of the separate calls.  (A launch that waits for the one before it costs 2.5-4 us whatever it does: a step of
+// an MLP of 784-1000-10 over 128 rows, sixteen launches 70.8 us, nine 47.4.)
+struct sgh_gemm_around {
+  const float *bias = nullptr, *gate = nullptr;
+  float *colsum = nullptr;
+  int relu = 0;
+};
+
 // fp32 GEMM with few output tiles, the reduction split over a workgroup's wavefronts (gemm_split.hip); arguments of
-// sgh_gemm_f32, checked by it, K > 0.  SGH_EUNSUPPORTED where the tiled kernel is the better one.
+// sgh_gemm_f32, checked by it, K > 0.  SGH_EUNSUPPORTED where the tiled kernel is the better one.  colsum: B not transposed.
 int sgh_gemm_split_run(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-                       float beta, float *C, int ldc, hipStream_t s);
+                       float beta, float *C, int ldc, const sgh_gemm_around &around, hipStream_t s);
 
 // Grouped convolutions with few channels per group (group_conv.hip), all three passes and types (dtype 0 fp32, 1 binary16,
 // 2 bfloat16): (a, b, out) = (x, W, y), (dy, W, dx), (dy, x, dW).  SGH_EUNSUPPORTED for every other geometry.

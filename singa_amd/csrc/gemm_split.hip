@@ -62,11 +62,36 @@ struct Mfma<16> {
   static __device__ __forceinline__ int row(int v, int h) { return 4 * h + v; }
 };
 
+// out[n] = sum over the rows of m[row][n], in ascending order, of the T columns from n0 on: 32 loads in flight per column
+template <int T>
+__device__ __forceinline__ void sum_columns(const float *__restrict__ m, int ld, int rows, int cols, int n0, float *__restrict__ out) {
+  const int j = n0 + int(threadIdx.x);
+  if (threadIdx.x >= T || j >= cols) return;
+  constexpr int U = 32;
+  float s = 0.f;
+  int i = 0;
+  for (; i + U <= rows; i += U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = m[size_t(i + u) * ld + j];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += v[u];
+  }
+  for (; i < rows; ++i) s += m[size_t(i) * ld + j];
+  out[j] = s;
+}
+
 template <bool AK, bool BKc, int T, int W>
 __global__ __launch_bounds__(W * 64) void k_gemm_split(const float *__restrict__ A, int lda, unsigned a_bytes,
                                                        const float *__restrict__ B, int ldb, unsigned b_bytes,
                                                        float *__restrict__ C, long ldc, int M, int N, int K, int kq, float alpha,
-                                                       float beta) {
+                                                       float beta, sgh_gemm_around around) {
+  if constexpr (!BKc) {
+    if (around.colsum && blockIdx.y == gridDim.y - 1) {   // (a row of workgroups of its own, beside the tiles)
+      sum_columns<T>(B, ldb, K, N, blockIdx.x * T, around.colsum);
+      return;
+    }
+  }
   __shared__ float part[W][T * T];
   constexpr int G = 4 * (64 / T);   // reduction indices of a group: four per lane
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, i = lane % T, h = lane / T;
@@ -109,21 +134,25 @@ __global__ __launch_bounds__(W * 64) void k_gemm_split(const float *__restrict__
     const int row = e / T, col = e % T;
     if (m0 + row < M && n0 + col < N) {
       float *p = C + size_t(m0 + row) * ldc + n0 + col;
-      *p = beta == 0.f ? alpha * v : alpha * v + beta * *p;
+      float r = beta == 0.f ? alpha * v : alpha * v + beta * *p;
+      if (around.bias) r += around.bias[n0 + col];
+      if (around.relu) r = r >= 0.f ? r : 0.f;
+      if (around.gate) r = around.gate[size_t(m0 + row) * N + n0 + col] > 0.f ? r : 0.f;
+      *p = r;
     }
   }
 }
 
 template <bool AK, bool BKc>
 void launch(int tile, int waves, const float *A, int lda, const float *B, int ldb, float *C, int ldc, int M, int N, int K, float alpha,
-            float beta, hipStream_t s) {
+            float beta, const sgh_gemm_around &around, hipStream_t s) {
   const int G = 256 / tile, kq = ((K + waves - 1) / waves + G - 1) / G * G;
   const unsigned ab = unsigned((size_t(AK ? M - 1 : K - 1) * lda + (AK ? K : M)) * 4);
   const unsigned bb = unsigned((size_t(BKc ? N - 1 : K - 1) * ldb + (BKc ? K : N)) * 4);
-  const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile);
+  const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile + (around.colsum ? 1 : 0));
 #define SGH_SPLIT_CASE(T_, W_)                                                                                                     \
   hipLaunchKernelGGL((k_gemm_split<AK, BKc, T_, W_>), grid, dim3(W_ * 64), 0, s, A, lda, ab, B, ldb, bb, C, long(ldc), M, N, K, kq, \
-                     alpha, beta)
+                     alpha, beta, around)
   if (tile == 16 && waves == 8) SGH_SPLIT_CASE(16, 8);
   else if (tile == 16) SGH_SPLIT_CASE(16, 4);
   else if (waves == 16) SGH_SPLIT_CASE(32, 16);
@@ -160,16 +189,16 @@ static bool plan(bool ta, bool tb, int M, int N, int K, int *tile, int *waves) {
   *tile = 2 * t32 < cus ? 16 : 32;
   *waves = K < 256 ? 4 : K < 1024 || *tile == 16 ? 8 : 16;
   if (nt && *tile == 32 && K >= 256) *waves = t32 >= cus ? 4 : 8;
-  return (M + *tile - 1) / *tile <= 65535;
+  return (M + *tile - 1) / *tile < 65535;   // (one more row of workgroups sums columns)
 }
 
 int sgh_gemm_split_run(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-                       float beta, float *C, int ldc, hipStream_t s) {
+                       float beta, float *C, int ldc, const sgh_gemm_around &around, hipStream_t s) {
   int tile, waves;
   if (!plan(transA, transB, M, N, K, &tile, &waves)) return SGH_EUNSUPPORTED;
-  if (!transA && transB) launch<true, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
-  else if (!transA) launch<true, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
-  else if (transB) launch<false, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
-  else launch<false, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, s);
+  if (!transA && transB) launch<true, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, around, s);
+  else if (!transA) launch<true, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, around, s);
+  else if (transB) launch<false, true>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, around, s);
+  else launch<false, false>(tile, waves, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, around, s);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }

@@ -1615,8 +1615,10 @@ int sgh_conv_bgrad_f32(const sgh_conv_geom *g, const float *dy, float *db, void 
   return sgh_conv_bgrad_run(g, dy, db, 0, sgh_stream_of(stream));
 }
 
-int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B,
-                 int ldb, float beta, float *C, int ldc, void *stream) {
+// sgh_gemm_f32 with what surrounds it; `around_done` says whether that was part of the launch (else it is the caller's to do)
+static int gemm_around(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+                       float beta, float *C, int ldc, const sgh_gemm_around &around, bool *around_done, void *stream) {
+  *around_done = false;
   if (M < 0 || N < 0 || K < 0) return SGH_EINVAL;
   if (M == 0 || N == 0) return SGH_OK;
   if (!C || ldc < N) return SGH_EINVAL;
@@ -1631,7 +1633,8 @@ int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const
   const long b_rs = transB ? ldb : 1, b_ks = transB ? 1 : ldb;  // B(k, n) addressed as (n, k)
   int rc;
   sgh_prof_start("gemm", 2.0 * M * N * K, s);
-  rc = K > 0 ? sgh_gemm_split_run(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s) : SGH_EUNSUPPORTED;
+  rc = K > 0 ? sgh_gemm_split_run(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, around, s) : SGH_EUNSUPPORTED;
+  *around_done = rc == SGH_OK;
   if (rc != SGH_EUNSUPPORTED) {   // (few output tiles)
   } else if (!transA && transB) rc = gemm_pick<true, true>(M, N, K, alpha, A, a_rs, a_ks, B, b_rs, b_ks, beta, C, ldc, s);
   else if (!transA && !transB) rc = gemm_pick<true, false>(M, N, K, alpha, A, a_rs, a_ks, B, b_rs, b_ks, beta, C, ldc, s);
@@ -1641,6 +1644,41 @@ int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const
   return rc;
 }
 
+int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B,
+                 int ldb, float beta, float *C, int ldc, void *stream) {
+  bool done;
+  return gemm_around(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, sgh_gemm_around{}, &done, stream);
+}
+
+int sgh_linear_fwd_f32(const float *x, const float *W, const float *bias, float *y, int rows, int in, int out, int relu,
+                       void *stream) {
+  sgh_gemm_around around;
+  around.bias = bias, around.relu = relu != 0;
+  bool done = false;
+  int rc = gemm_around(0, 0, rows, out, in, 1.f, x, in, W, out, 0.f, y, out, around, &done, stream);
+  if (rc == SGH_OK && !done && bias) rc = sgh_add_row_f32(bias, y, rows, out, stream);
+  if (rc == SGH_OK && !done && relu) rc = sgh_relu_fwd_f32(y, y, size_t(rows) * out, stream);
+  return rc;
+}
+
+int sgh_linear_bwd_x_f32(const float *dy, const float *W, const float *gate, float *dx, int rows, int in, int out, void *stream) {
+  sgh_gemm_around around;
+  around.gate = gate;
+  bool done = false;
+  int rc = gemm_around(0, 1, rows, in, out, 1.f, dy, out, W, out, 0.f, dx, in, around, &done, stream);
+  if (rc == SGH_OK && !done && gate) rc = sgh_relu_bwd_f32(dx, gate, dx, size_t(rows) * in, stream);
+  return rc;
+}
+
+int sgh_linear_bwd_wb_f32(const float *x, const float *dy, float *dW, float *db, int rows, int in, int out, void *stream) {
+  if (!db) return SGH_EINVAL;
+  sgh_gemm_around around;
+  around.colsum = db;
+  bool done = false;
+  int rc = gemm_around(1, 0, in, out, rows, 1.f, x, in, dy, out, 0.f, dW, out, around, &done, stream);
+  if (rc == SGH_OK && !done) rc = sgh_sum_rows_f32(dy, db, rows, out, stream);
+  return rc;
+}
 
 // ---- 16-bit storage (binary16 / bfloat16) --------------------------------------------------
 // The tensors are converted to fp32 in the workspace, the fp32 kernels above do the arithmetic

@@ -69,6 +69,7 @@ struct EntryOf {
   ONE(sgh_div_f32) ONE(sgh_add_scalar_f32) ONE(sgh_mult_scalar_f32) ONE(sgh_clamp_f32) ONE(sgh_cast_f32_to_f16)                 \
   ONE(sgh_cast_f16_to_f32) ONE(sgh_cast_f32_to_bf16) ONE(sgh_cast_bf16_to_f32) ONE(sgh_cast_f32_to_i32)                         \
   ONE(sgh_cast_i32_to_f32) ALL(sgh_softmax_ce_bwd) ONE(sgh_softmax_fwd_f32) ONE(sgh_cross_entropy_fwd_f32) ALL(sgh_gemm)        \
+  ONE(sgh_linear_fwd_f32) ONE(sgh_linear_bwd_x_f32) ONE(sgh_linear_bwd_wb_f32) ONE(sgh_softmax_ce_fwd_f32)                       \
   ONE(sgh_sum_rows_f32) ONE(sgh_add_row_f32) ONE(sgh_row_max_f32) ONE(sgh_row_max_zero_seeded_f32) ONE(sgh_dot_f32)             \
   ONE(sgh_sum_all_f32) ALL(sgh_sgd_momentum) ONE(sgh_sgd_momentum_multi_f32) ONE(sgh_sgd_momentum_multi_mixed)                  \
   ONE(sgh_sgd_momentum_master_f16) ONE(sgh_sgd_momentum_master_bf16) ALL(sgh_conv_fwd) ALL(sgh_conv_dgrad) ALL(sgh_conv_wgrad)  \

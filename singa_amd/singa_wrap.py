@@ -571,6 +571,17 @@ def CrossEntropyFwd(p, t):
     return loss
 
 
+def SoftMaxCrossEntropyFwd(x, t):
+    """(``SoftMax(x)``, ``CrossEntropyFwd`` of it and `t`) by one launch; the bits of the two calls."""
+    _need_f32("SoftMax", x)
+    batch, dim, int_target = _ce_dims(x, t)
+    p = _like(x)
+    loss = _empty(Tensor, (batch,), x.device(), kFloat32)
+    check(_L().sgh_softmax_ce_fwd_f32(x.ptr, t.ptr, p.ptr, loss.ptr, batch, dim, int(int_target), x.device().stream),
+          "sgh_softmax_ce_fwd_f32")
+    return p, loss
+
+
 def SoftmaxCrossEntropyBwd(p, t, scale=1.0):
     """``singa.SoftmaxCrossEntropyBwd(p, t)`` (src/core/tensor/tensor.cc:1717-1721): returns a new
     tensor.  ``scale`` (not in the reference signature) fuses the ``dx /= N`` that follows it."""
@@ -707,6 +718,46 @@ def Sum(t, axis):
     out = _empty(Tensor, (t.shape(1),), t.device(), kFloat32)
     check(_L().sgh_sum_rows_f32(t.ptr, out.ptr, t.shape(0), t.shape(1), t.device().stream), "sgh_sum_rows_f32")
     return out
+
+
+def _linear_dims(what, W, rows_tensors, extents, vector=None):
+    """The checks that ``Mult`` and the row functions make on a dense layer's tensors, all plain fp32 matrices."""
+    for t in (W,) + rows_tensors:
+        if len(t._shape) != 2 or t._transposed or t._dtype != kFloat32:
+            raise SingaHipError("%s: fp32 matrices that are not transposed are expected" % what)
+    for t, e in zip(rows_tensors, extents):
+        if t._shape != (rows_tensors[0]._shape[0], e):
+            raise SingaHipError("%s: shape mismatch %s" % (what, t.shape()))
+    if vector is not None and (vector._dtype != kFloat32 or vector.Size() != W._shape[1]):
+        raise SingaHipError("%s: the bias does not match" % what)
+
+
+def LinearForward(x, W, b, relu=False):
+    """``AddRow(b, Mult(x, W))``, behind a ReLU if `relu`, in one launch for the sizes whose product takes one; the bits of
+    the separate calls."""
+    _linear_dims("LinearForward", W, (x,), W._shape[:1], b)
+    y = _empty(Tensor, (x._shape[0], W._shape[1]), x._dev, kFloat32)
+    check(_L().sgh_linear_fwd_f32(x.ptr, W.ptr, b.ptr, y.ptr, x._shape[0], W._shape[0], W._shape[1], int(relu), x._dev.stream),
+          "sgh_linear_fwd_f32")
+    return y
+
+
+def LinearBackwardx(dy, W, gate=None):
+    """``Mult(dy, W^T)``, with `gate` followed by ``ReLUBackward(_, gate)``, as ``LinearForward``."""
+    _linear_dims("LinearBackwardx", W, (dy,) if gate is None else (dy, gate), (W._shape[1], W._shape[0]))
+    dx = _empty(Tensor, (dy._shape[0], W._shape[0]), dy._dev, kFloat32)
+    check(_L().sgh_linear_bwd_x_f32(dy.ptr, W.ptr, gate.ptr if gate is not None else None, dx.ptr, dy._shape[0], W._shape[0],
+                                    W._shape[1], dy._dev.stream), "sgh_linear_bwd_x_f32")
+    return dx
+
+
+def LinearBackwardWb(dy, x, W, b):
+    """(``Mult(x^T, dy)``, ``Sum(dy, 0)``) of the layer with weights `W` and bias `b`, as ``LinearForward``."""
+    _linear_dims("LinearBackwardWb", W, (dy, x), (W._shape[1], W._shape[0]), b)
+    dW, db = _like(W), _like(b)
+    check(_L().sgh_linear_bwd_wb_f32(x.ptr, dy.ptr, dW.ptr, db.ptr, dy._shape[0], W._shape[0], W._shape[1], dy._dev.stream),
+          "sgh_linear_bwd_wb_f32")
+    return dW, db
 
 
 def AddRow(v, m):

@@ -99,6 +99,22 @@ class HipOps(object):
     def ce_fwd(self, p, t):
         return singa.CrossEntropyFwd(p, t)
 
+    # cross-op fusion the tape permits: a dense layer's products with its bias, the ReLU next to it and the column sums of
+    # its bias gradient; softmax with its loss
+    fuse_linear = True
+
+    def linear_fwd(self, x, W, b, relu):
+        return singa.LinearForward(x, W, b, relu)
+
+    def linear_bwd_x(self, dy, W, gate):
+        return singa.LinearBackwardx(dy, W, gate)
+
+    def linear_bwd_wb(self, dy, x, W, b):
+        return singa.LinearBackwardWb(dy, x, W, b)
+
+    def softmax_ce_fwd(self, x, t):
+        return singa.SoftMaxCrossEntropyFwd(x, t)
+
     # backward
     def softmax_ce_bwd(self, p, t, batch):
         # SoftmaxCrossEntropyBwd followed by "dx /= N" (python/singa/autograd.py:1319-1322), fused
@@ -208,12 +224,13 @@ class HipOps(object):
             self.dev.Join()    # the update (and any reader of a weight gradient) comes after the last of them
             self._aux = None
 
-    fusions = ("fuse_bn_relu", "fuse_dgrad_add", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward")   # what set_fusion(True) turns on
+    fusions = ("fuse_bn_relu", "fuse_dgrad_add", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
+               "fuse_linear")   # what set_fusion(True) turns on
 
     def set_fusion(self, on):
         """All of this implementation's cross-op fusions on, or the reference's op-per-op tape."""
         for f in ("fuse_bn_relu", "fuse_dgrad_add", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad",
-                  "fuse_forward"):
+                  "fuse_forward", "fuse_linear"):
             setattr(self, f, bool(on) and f in self.fusions)
 
     def accumulate(self, a, b):
@@ -255,7 +272,8 @@ class HalfHipOps(HipOps):
     # scattered 2-byte stores make a read-modify-write epilogue slower than the separate add)
     fuse_dgrad_add = False
     fuse_add_relu = True
-    fusions = ("fuse_bn_relu", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward")
+    fusions = ("fuse_bn_relu", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
+               "fuse_linear")
 
     def __init__(self, dev, dtype):
         HipOps.__init__(self, dev)
@@ -478,9 +496,31 @@ class Linear(_Layer):
 
     def fwd(self, x):
         self.x = x
+        if getattr(self.ops, "fuse_linear", False):
+            return self.ops.linear_fwd(x, self.W, self.b, False)
         return self.ops.add_bias(self.ops.matmul(x, self.W), self.b)
 
-    def bwd(self, dy, grads):
+    def fwd_through_relu(self, relu, x):
+        """Forward of ``relu(self(x))``; fused, the ReLU keeps its output, as in BatchNorm.fwd_through_relu."""
+        if not getattr(self.ops, "fuse_linear", False):
+            return relu.fwd(self.fwd(x))
+        self.x = x
+        relu.x = self.ops.linear_fwd(x, self.W, self.b, True)
+        return relu.x
+
+    def bwd_behind_relu(self, relu, dy, grads):
+        """Backward of ``self(relu(_))``, the data gradient gated as it is computed where the ops implementation offers it."""
+        if not getattr(self.ops, "fuse_linear", False):
+            return relu.bwd(self.bwd(dy, grads), grads)
+        return self.bwd(dy, grads, relu.x)
+
+    def bwd(self, dy, grads, gate=None):
+        if getattr(self.ops, "fuse_linear", False):
+            dx = self.ops.linear_bwd_x(dy, self.W, gate)
+            dW, db = self.ops.linear_bwd_wb(dy, self.x, self.W, self.b)
+            grads(self.name + ".b", self.b, db)
+            grads(self.name + ".W", self.W, dW)
+            return dx
         # tape order: AddBias.backward (db) first, then Matmul.backward (autograd.py:613-623, :696-709)
         grads(self.name + ".b", self.b, self.ops.sum0(dy))
         dx, dW = self.ops.matmul_bwd(dy, self.x, self.W)
@@ -642,15 +682,18 @@ class Net(object):
         i = 0
         while i < len(self.layers):
             l = self.layers[i]
-            if isinstance(l, BatchNorm) and i + 1 < len(self.layers) and isinstance(self.layers[i + 1], ReLU):
-                x = l.fwd_through_relu(self.layers[i + 1], x)   # the stem's conv -> BatchNorm -> ReLU
+            if isinstance(l, (BatchNorm, Linear)) and i + 1 < len(self.layers) and isinstance(self.layers[i + 1], ReLU):
+                x = l.fwd_through_relu(self.layers[i + 1], x)   # the stem's conv -> BatchNorm -> ReLU, a hidden dense layer
                 i += 2
             else:
                 x = l.fwd(x)
                 i += 1
         self.logits = x
-        self.p = self.ops.softmax(x)
         self.t = labels
+        if getattr(self.ops, "fuse_linear", False):
+            self.p, loss = self.ops.softmax_ce_fwd(x, labels)
+            return loss
+        self.p = self.ops.softmax(x)
         return self.ops.ce_fwd(self.p, labels)
 
     def backward_and_update(self, keep_grads=False, fused_update=False):
@@ -679,6 +722,9 @@ class Net(object):
             while i < len(rev):
                 if isinstance(rev[i], ReLU) and i + 1 < len(rev) and isinstance(rev[i + 1], BatchNorm):
                     dy = rev[i + 1].bwd_through_relu(rev[i], _summed(ops, dy), grads)   # the stem's conv -> BatchNorm -> ReLU
+                    i += 2
+                elif isinstance(rev[i], Linear) and i + 1 < len(rev) and isinstance(rev[i + 1], ReLU):
+                    dy = rev[i].bwd_behind_relu(rev[i + 1], _summed(ops, dy), grads)
                     i += 2
                 else:
                     if not isinstance(rev[i], (BasicBlock, Bottleneck)):

@@ -578,3 +578,49 @@ def test_gemm_split_reduction_edges(singa, dev, kind, M, N, K):
             g = (got if kind == "f32" else got.AsType(singa.kFloat32)).to_numpy().astype(np.float64)
             bound = K * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + ulp * np.abs(a @ b) + (1e-7 if kind == "f16" else 0.0)
             assert np.all(np.abs(g - a @ b) <= bound), (tA, tB, float(np.max(np.abs(g - a @ b) - bound)))
+
+
+@pytest.mark.parametrize("rows,inner,out", [(1, 1, 1), (3, 5, 7), (128, 784, 1000), (33, 4096, 10), (129, 33, 31), (1000, 70, 4160)])
+def test_linear_calls_store_the_bits_of_the_separate_ones(singa, dev, rows, inner, out):
+    """LinearForward / LinearBackwardx / LinearBackwardWb against Mult, AddRow, ReLU, ReLUBackward and Sum: 16- and 32-wide
+    tiles, edges inside a tile, and (the last) a problem that the split kernel leaves to the tiled one; infinities and NaNs too."""
+    r = rng(rows + inner + out)
+    x, W, b, dy, gate = randn(r, rows, inner), randn(r, inner, out), randn(r, out), randn(r, rows, out), randn(r, rows, inner)
+    x[rows // 2, 0], dy[rows - 1, out // 2], gate[0, inner - 1] = np.inf, np.nan, np.nan
+    x, W, b, dy, gate = (singa.from_numpy(a, dev) for a in (x, W, b, dy, gate))
+    y = singa.Mult(x, W)
+    singa.AddRow(b, y)
+    same = lambda a, e, what: np.testing.assert_array_equal(a.to_numpy().view(np.uint32), e.to_numpy().view(np.uint32), what)
+    same(singa.LinearForward(x, W, b), y, "y")
+    same(singa.LinearForward(x, W, b, True), singa.ReLU(y), "relu(y)")
+    dx = singa.Mult(dy, singa.DefaultTranspose(W))
+    same(singa.LinearBackwardx(dy, W), dx, "dx")
+    same(singa.LinearBackwardx(dy, W, gate), singa.ReLUBackward(dx, gate), "gated dx")
+    dW, db = singa.LinearBackwardWb(dy, x, W, b)
+    same(dW, singa.Mult(singa.DefaultTranspose(x), dy), "dW")
+    same(db, singa.Sum(dy, 0), "db")
+    with pytest.raises(singa.SingaHipError):
+        singa.LinearForward(dy if out != inner else W.T(), W, b)
+
+
+@pytest.mark.parametrize("dim", [1, 10, 255, 257, 2048, 2049, 5000])
+def test_softmax_with_its_loss_stores_the_bits_of_the_separate_calls(singa, dev, dim):
+    """Rows held in registers (up to 2048 values) and longer ones; whole-number targets, one of them out of range, and rows
+    of target values; p against float64."""
+    r = rng(dim)
+    x = (4 * randn(r, 7, dim)).astype(np.float32)
+    xt = singa.from_numpy(x, dev)
+    e = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+    for t in (r.integers(0, dim, 7), r.integers(0, 3, (7, dim)) + 1)[:1 if dim == 1 else 2]:   # (7 x 1 is a whole-number target)
+        t = t.astype(np.int32)
+        if t.ndim == 1:
+            t[3] = dim
+        tt = singa.Tensor(t.shape, dev, singa.kInt)
+        tt.CopyIntDataFromHostPtr(t)
+        singa.LabelErrors(dev)
+        p, loss = singa.SoftMaxCrossEntropyFwd(xt, tt)
+        assert singa.LabelErrors(dev) == (1 if t.ndim == 1 else 0)
+        assert_bit_equal(p.to_numpy(), singa.SoftMax(xt).to_numpy(), "p")
+        assert_bit_equal(loss.to_numpy(), singa.CrossEntropyFwd(p, tt).to_numpy(), "loss")
+        # expf to 2 ulp of its value, its argument to half an ulp, sum of dim terms in a tree, one division
+        assert np.max(np.abs(p.to_numpy() / (e / e.sum(1, keepdims=True)) - 1)) < (40 + np.log2(dim + 1)) * 2.0 ** -24
