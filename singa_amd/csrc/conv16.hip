@@ -35,6 +35,7 @@
 
 #include "common.h"
 #include "pw16.h"
+#include "wgrad_pw16.h"
 #include "storage.h"
 
 namespace {
@@ -1109,6 +1110,10 @@ bool octets_pay(const sgh_conv_geom *g, size_t *workspace) {
   return true;
 }
 
+size_t pw_wgrad_bytes(const sgh_conv_geom *g, const sgh_wgrad_pw16_plan &p) {
+  return p.parts > 1 ? align256(size_t(p.parts) * g->K * g->C * sizeof(float)) : 0;
+}
+
 struct D16Plan {
   bool ok;
   bool pixk;   // several taps: the kernel reads a pixel-major copy of the gradient (k_pixel_major16)
@@ -1222,6 +1227,20 @@ D16Plan dplan(const sgh_conv_geom *real, int fs = 1) {
   return p;
 }
 
+// dW from `splits` partial images of n elements
+int sum_partials(const float *partial, int splits, size_t n, uint16_t *dW, bool bf16, hipStream_t s) {
+  if (n / 64 >= size_t(2 * sgh_num_cus()) || splits < 16) {
+    const dim3 grid(unsigned((n + 63) / 64));
+    if (bf16) hipLaunchKernelGGL((k_wgrad16_reduce<64, true>), grid, dim3(256), 0, s, partial, splits, n, dW);
+    else hipLaunchKernelGGL((k_wgrad16_reduce<64, false>), grid, dim3(256), 0, s, partial, splits, n, dW);
+  } else {  // few elements, many splits: more z-lanes
+    const dim3 grid(unsigned((n + 15) / 16));
+    if (bf16) hipLaunchKernelGGL((k_wgrad16_reduce<16, true>), grid, dim3(256), 0, s, partial, splits, n, dW);
+    else hipLaunchKernelGGL((k_wgrad16_reduce<16, false>), grid, dim3(256), 0, s, partial, splits, n, dW);
+  }
+  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+}
+
 template <int BM, int STRIDE, bool BF16>
 int launch_w(const W16Args &a, const W16Plan &p, hipStream_t s) {
   auto kern = k_wgrad16<BM, STRIDE, BF16>;
@@ -1320,8 +1339,11 @@ size_t sgh_conv16_workspace_bytes(const sgh_conv_geom *g, int which) {
 // The workspace with which sgh_conv16_wgrad takes its fastest kernel; with sgh_conv16_workspace_bytes it runs
 size_t sgh_conv16_wgrad_full_bytes(const sgh_conv_geom *g) {
   const size_t least = sgh_conv16_workspace_bytes(g, SGH_CONV_WGRAD);
-  size_t octets;
-  return least && octets_pay(g, &octets) && octets > least ? octets : least;
+  if (!least) return 0;
+  size_t octets = 0;
+  if (const sgh_wgrad_pw16_plan q = sgh_wgrad_pw16_plan_of(g); q.ok) octets = pw_wgrad_bytes(g, q);
+  else octets_pay(g, &octets);
+  return octets > least ? octets : least;
 }
 
 int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace,
@@ -1330,6 +1352,13 @@ int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t 
   const W16Plan p = wplan(g, mode < 0 ? sgh_stream_is_aux(s) : mode != 0);
   if (!p.ok) return SGH_EUNSUPPORTED;
   if (!workspace || ws_bytes < sgh_conv16_workspace_bytes(g, SGH_CONV_WGRAD)) return SGH_EWORKSPACE;
+  if (const sgh_wgrad_pw16_plan q = sgh_wgrad_pw16_plan_of(g); q.ok && ws_bytes >= pw_wgrad_bytes(g, q)) {
+    float *partial = static_cast<float *>(workspace);
+    sgh_prof_kernel_begin("conv_wgrad16/k_wgrad_pw16", 2.0 * g->N * g->K * g->P * g->Q * double(g->C));
+    const int rc = sgh_wgrad_pw16_run(g, q, dy, x, partial, dW, bf16, s);
+    sgh_prof_kernel_end(s);
+    return rc != SGH_OK || q.parts == 1 ? rc : sum_partials(partial, q.parts, size_t(g->K) * g->C, dW, bf16, s);
+  }
   size_t octets;
   if (octets_pay(g, &octets) && ws_bytes >= octets) return sgh_wgrad_oct16_run(g, dy, x, dW, workspace, bf16, s);
   W16Args a{};
@@ -1351,17 +1380,7 @@ int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t 
   }
   sgh_prof_kernel_end(s);
   if (rc != SGH_OK) return rc;
-  const size_t n = size_t(g->K) * a.CRS;
-  if (n / 64 >= size_t(2 * sgh_num_cus()) || p.splits < 16) {
-    const dim3 grid(unsigned((n + 63) / 64));
-    if (bf16) hipLaunchKernelGGL((k_wgrad16_reduce<64, true>), grid, dim3(256), 0, s, a.partial, p.splits, n, dW);
-    else hipLaunchKernelGGL((k_wgrad16_reduce<64, false>), grid, dim3(256), 0, s, a.partial, p.splits, n, dW);
-  } else {  // few elements, many splits: more z-lanes
-    const dim3 grid(unsigned((n + 15) / 16));
-    if (bf16) hipLaunchKernelGGL((k_wgrad16_reduce<16, true>), grid, dim3(256), 0, s, a.partial, p.splits, n, dW);
-    else hipLaunchKernelGGL((k_wgrad16_reduce<16, false>), grid, dim3(256), 0, s, a.partial, p.splits, n, dW);
-  }
-  return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
+  return sum_partials(a.partial, p.splits, size_t(g->K) * a.CRS, dW, bf16, s);
 }
 
 namespace {

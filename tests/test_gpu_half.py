@@ -682,6 +682,36 @@ def _grad16_cases(count, seed):
 
 
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("N,C,H,W,K", [(1, 1, 2, 4, 1), (3, 65, 3, 3, 63), (2, 64, 5, 7, 66), (5, 33, 7, 7, 129), (9, 130, 6, 6, 200),
+                                       (4, 17, 9, 11, 600), (21, 64, 24, 24, 256), (30, 300, 13, 10, 520), (128, 256, 14, 14, 256)])
+def test_pointwise_weight_gradient_16bit_edges(singa, dev, kind, N, C, H, W, K):
+    """1x1 weight gradients on k_wgrad_pw16: planes that end inside an octet by every remainder, batches that end inside a chunk, edges
+    of the tiles of 64 and 128, one part and several, an odd number of chunks.  Exact: whole numbers whose sums fit 24 bits, one rounding.
+    An infinity in the pixels that two octets share counts once."""
+    from util import kernels_of
+    print("pointwise wgrad", kind, N, C, H, W, K, flush=True)
+    r = rng(N + C + H + W + K)
+    x, dy = r.integers(-2, 3, (N, C, H, W)).astype(np.float32), r.integers(-2, 3, (N, K, H, W)).astype(np.float32)
+    dt = {"f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+    to = lambda a: singa.from_numpy(a.astype(np.float32), dev).AsType(dt)
+    back = lambda t: t.AsType(singa.kFloat32).to_numpy()
+    wt = to(np.zeros((K, C, 1, 1)))
+
+    def run(x):
+        xt, dyt = to(x), to(dy)
+        h = singa.CudnnConvHandle(xt, (1, 1), (1, 1), (0, 0), C, K, False)
+        dW, names = kernels_of(dev, lambda: singa.GpuConvBackwardW(dyt, xt, wt, h))
+        assert names == {"k_wgrad_pw16"}, names
+        return back(dW)[:, :, 0, 0]
+    want = np.einsum("nkp,ncp->kc", dy.reshape(N, K, -1).astype(np.float64), x.reshape(N, C, -1).astype(np.float64))
+    assert np.array_equal(run(x), back(to(want)))
+    x[N - 1, C - 1, H - 1, W - 2] = np.inf
+    got = run(x)
+    assert np.array_equal(got[:, :C - 1], back(to(want))[:, :C - 1])
+    at = dy[N - 1, :, H - 1, W - 2]
+    assert np.array_equal(np.isnan(got[:, C - 1]), at == 0) and np.array_equal(np.sign(got[at != 0, C - 1]), np.sign(at[at != 0]))
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
 @pytest.mark.parametrize("case", _grad16_cases(40, 777) + [
     (2, 64, 56, 56, 64, 3, 3, (1, 1), (1, 1)),      # ResNet stage-1 3x3
     (2, 256, 14, 14, 64, 1, 1, (1, 1), (0, 0)),     # bottleneck reduce: plane of 196 = 24.5 octets
