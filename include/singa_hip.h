@@ -479,6 +479,15 @@ SGH_API int sgh_conv_dgrad_f32(sgh_conv_geom *g, const float *dy, const float *W
  * K a multiple of 16); SGH_EUNSUPPORTED otherwise, with dx untouched. */
 SGH_API int sgh_conv_dgrad_acc_f32(sgh_conv_geom *g, const float *dy, const float *W,
                                    float *dx, void *workspace, size_t ws_bytes, void *stream);
+/* dx = ReLUBackward(data gradient + add, x): the input gradient of a residual block whose input x is a ReLU's output, summed with
+ * the gradient `add` of its other branch and gated (python/singa/autograd.py:204, :432-439).  The bits of the separate calls
+ * (sgh_conv_dgrad_*, sgh_relu_bwd_add_*); one launch for 1x1 layers of stride 1.  add and x are not dx. */
+SGH_API int sgh_conv_dgrad_add_relu_f16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W,
+                                        const uint16_t *add, const uint16_t *x, uint16_t *dx,
+                                        void *workspace, size_t ws_bytes, void *stream);
+SGH_API int sgh_conv_dgrad_add_relu_bf16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W,
+                                         const uint16_t *add, const uint16_t *x, uint16_t *dx,
+                                         void *workspace, size_t ws_bytes, void *stream);
 /* 1 if sgh_conv_dgrad_acc_f32 covers this geometry, else 0: a caller that has to schedule the
  * fallback (data gradient + Add) itself asks before it submits anything. */
 SGH_API int sgh_conv_dgrad_acc_supported(const sgh_conv_geom *g);

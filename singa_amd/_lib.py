@@ -162,6 +162,8 @@ SIGNATURES = {
     "sgh_conv_workspace_bytes": (sz, [C.POINTER(ConvGeom), C.c_int]),
     "sgh_conv_workspace_least_bytes": (sz, [C.POINTER(ConvGeom), C.c_int, C.c_int]),
     "sgh_conv_dgrad_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),
+    "sgh_conv_dgrad_add_relu_f16": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, vp, vp, sz, vp]),
+    "sgh_conv_dgrad_add_relu_bf16": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, vp, vp, sz, vp]),
     "sgh_conv_dgrad_acc_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),
     "sgh_conv_wgrad_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, sz, vp]),
     "sgh_conv_wgrad_bias_f32": (C.c_int, [C.POINTER(ConvGeom), vp, vp, vp, vp, vp, sz, vp]),

@@ -210,8 +210,12 @@ size_t sgh_conv16_workspace_bytes(const sgh_conv_geom *g, int which);
 size_t sgh_conv16_wgrad_full_bytes(const sgh_conv_geom *g);
 int sgh_conv16_wgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace,
                      size_t ws_bytes, bool bf16, hipStream_t s);
+struct sgh_dgrad_tail {   // dx = gate > 0 ? the data gradient as it would be stored + add : 0
+  const uint16_t *add, *gate;
+  bool done;              // set by a kernel that did it; else it is the caller's to do
+};
 int sgh_conv16_dgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, uint16_t *dx, void *workspace,
-                     size_t ws_bytes, bool bf16, hipStream_t s, bool prelaid);
+                     size_t ws_bytes, bool bf16, hipStream_t s, bool prelaid, sgh_dgrad_tail *tail);
 // Data-gradient weight re-layout of conv16.hip as a batch item: false when the geometry is not covered;
 // otherwise the destination layout [tap][CP][KP] (sgh_conv16_dgrad skips its re-layout when told that the
 // workspace already holds it).

@@ -1389,7 +1389,7 @@ namespace {
 // geometry *fwd_of, W is that convolution's weight tensor and `bias` its bias (or null)
 int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t *dy, const uint16_t *W,
             const uint16_t *bias, uint16_t *dx, void *workspace, size_t ws_bytes, bool bf16, hipStream_t s, int fs = 1,
-            bool prelaid = false) {
+            bool prelaid = false, sgh_dgrad_tail *tail = nullptr) {
   const D16Plan p = dplan(g, fs);
   if (!p.ok) return SGH_EUNSUPPORTED;
   const int RS = g->R * g->S;
@@ -1451,6 +1451,7 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     b.QO = (b.HW + 7) / 8, b.octets = g->N * b.QO, b.mtiles = p.mtiles, b.ptiles = p.tiles;
     b.a_bytes = unsigned((as_is ? size_t(g->C) * g->K : nw) * 2);
     b.src_bytes = unsigned(size_t(g->N) * g->K * b.HW * 2);
+    if (tail) b.add = tail->add, b.gate = tail->gate, tail->done = true;
     sgh_prof_kernel_begin(fwd_of ? "conv_fwd16/k_pw16" : "conv_dgrad16/k_pw16", 2.0 * g->N * g->K * b.HW * double(g->C));
     const int rc = sgh_pw16_launch(b, p.bm, bf16, s);
     sgh_prof_kernel_end(s);
@@ -1493,8 +1494,8 @@ bool sgh_conv16_dgrad_relayout_dims(const sgh_conv_geom *g, int *CP, int *KP) {
 }
 
 int sgh_conv16_dgrad(const sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, uint16_t *dx, void *workspace,
-                     size_t ws_bytes, bool bf16, hipStream_t s, bool prelaid) {
-  return run_d16(g, nullptr, dy, W, nullptr, dx, workspace, ws_bytes, bf16, s, 1, prelaid);
+                     size_t ws_bytes, bool bf16, hipStream_t s, bool prelaid, sgh_dgrad_tail *tail) {
+  return run_d16(g, nullptr, dy, W, nullptr, dx, workspace, ws_bytes, bf16, s, 1, prelaid, tail);
 }
 
 int sgh_conv16_fwd(const sgh_conv_geom *g, const uint16_t *x, const uint16_t *W, const uint16_t *bias, uint16_t *y,

@@ -1708,7 +1708,8 @@ typedef int (*cast_out_fn)(const float *, uint16_t *, size_t, void *);
 
 // which: SGH_CONV_*; (a, b) are the pass's two tensor inputs in the order of its fp32 entry point
 int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b, const uint16_t *bias,
-              uint16_t *out, void *workspace, size_t ws_bytes, void *stream, cast_in_fn in, cast_out_fn outc) {
+              uint16_t *out, void *workspace, size_t ws_bytes, void *stream, cast_in_fn in, cast_out_fn outc,
+              sgh_dgrad_tail *tail = nullptr) {
   if (!conv_ok(g) || !a || !b || !out) return SGH_EINVAL;
   if (g->groups > 1) {
     const int rc = sgh_group_conv_run(g, which, in == sgh_cast_bf16_to_f32 ? 2 : 1, a, b, bias, out, workspace, ws_bytes,
@@ -1735,7 +1736,7 @@ int conv_half(sgh_conv_geom *g, int which, const uint16_t *a, const uint16_t *b,
   if (sgh_conv16_workspace_bytes(g, which) != 0 && !sgh_env().conv16_off) {
     const bool bf16 = in == sgh_cast_bf16_to_f32;
     hipStream_t s = sgh_stream_of(stream);
-    const int rc = which == SGH_CONV_DGRAD   ? sgh_conv16_dgrad(g, a, b, out, workspace, ws_bytes, bf16, s, prelaid)
+    const int rc = which == SGH_CONV_DGRAD   ? sgh_conv16_dgrad(g, a, b, out, workspace, ws_bytes, bf16, s, prelaid, tail)
                    : which == SGH_CONV_WGRAD ? sgh_conv16_wgrad(g, a, b, out, workspace, ws_bytes, bf16, s)
                                              : sgh_conv16_fwd(g, a, b, bias, out, workspace, ws_bytes, bf16, s);
     if (rc != SGH_EUNSUPPORTED) return rc;
@@ -1825,6 +1826,22 @@ int sgh_conv_dgrad_bf16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W,
                         size_t ws_bytes, void *stream) {
   return conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_bf16_to_f32,
                    sgh_cast_f32_to_bf16);
+}
+int sgh_conv_dgrad_add_relu_f16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, const uint16_t *add, const uint16_t *x,
+                                uint16_t *dx, void *workspace, size_t ws_bytes, void *stream) {
+  if (!conv_ok(g) || !add || !x) return SGH_EINVAL;
+  sgh_dgrad_tail tail{add, x, false};
+  const int rc = conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_f16_to_f32,
+                           sgh_cast_f32_to_f16, &tail);
+  return rc != SGH_OK || tail.done ? rc : sgh_relu_bwd_add_f16(dx, add, x, dx, size_t(g->N) * g->C * g->H * g->W, stream);
+}
+int sgh_conv_dgrad_add_relu_bf16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, const uint16_t *add, const uint16_t *x,
+                                 uint16_t *dx, void *workspace, size_t ws_bytes, void *stream) {
+  if (!conv_ok(g) || !add || !x) return SGH_EINVAL;
+  sgh_dgrad_tail tail{add, x, false};
+  const int rc = conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_bf16_to_f32,
+                           sgh_cast_f32_to_bf16, &tail);
+  return rc != SGH_OK || tail.done ? rc : sgh_relu_bwd_add_bf16(dx, add, x, dx, size_t(g->N) * g->C * g->H * g->W, stream);
 }
 int sgh_conv_wgrad_f16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *x, uint16_t *dW, void *workspace,
                        size_t ws_bytes, void *stream) {

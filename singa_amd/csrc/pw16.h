@@ -10,6 +10,7 @@ struct sgh_pw16_args {
   const uint16_t *src;   // [N][K][HW]
   uint16_t *out;         // [N][M][HW]
   const uint16_t *bias;  // per output channel, or null
+  const uint16_t *add, *gate;   // out = gate > 0 ? stored result + add : 0, both laid out as out; or null
   int M, K, HW, lda;     // K and lda: multiples of 8, HW >= 8
   int QO, octets;        // octets of a plane (the last one overlaps its neighbour), of the batch
   int mtiles, ptiles;

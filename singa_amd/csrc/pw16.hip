@@ -240,15 +240,53 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         *reinterpret_cast<u32x2 *>(lds + row * OP + (wn * TN + j) * 32 + 2 * v + 4 * lh) = o;
       }
   }
-  __syncthreads();
   const int g = t & 15, go = pt * 16 + g;
-  if (go >= a.octets) return;
   const int n = go / a.QO, p = go - n * a.QO;
-  uint16_t *out = a.out + (size_t(n) * a.M + m0) * a.HW + min(8 * p, a.HW - 8);
+  const size_t first = (size_t(n) * a.M + m0) * a.HW + min(8 * p, a.HW - 8);
+  // A residual block's input gradient: the sum with its other branch and the ReLU in front of the block.  Two reads here instead of
+  // a pass of its own that reads three tensors and writes one (ResNet-50, 128 images: 0.85 of 13.2 ms of kernel time).  Both are
+  // requested before the tile is complete.
+  if (a.add) {
+    u32x4 va[BM / 32], vg[BM / 32];
+#pragma unroll
+    for (int i = 0; i < BM / 32; ++i) {
+      const int row = (t >> 4) + 32 * i;
+      if (go < a.octets && m0 + row < a.M) {
+        __builtin_memcpy(&va[i], a.add + first + size_t(row) * a.HW, 16);
+        __builtin_memcpy(&vg[i], a.gate + first + size_t(row) * a.HW, 16);
+      }
+    }
+    __syncthreads();
+    if (go >= a.octets) return;
+#pragma unroll
+    for (int i = 0; i < BM / 32; ++i) {
+      const int row = (t >> 4) + 32 * i;
+      if (m0 + row >= a.M) continue;
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(lds + row * OP + 8 * g);
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float r[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          auto value = [&](const u32x4 &w) {
+            const uint16_t b = uint16_t(w[e] >> (16 * k));
+            return BF16 ? sgh_bf16_to_f32(b) : sgh_f16_to_f32(b);
+          };
+          r[k] = value(vg[i]) > 0.f ? value(v) + value(va[i]) : 0.f;
+        }
+        o[e] = BF16 ? sgh_pack2_bf16(r[0], r[1]) : sgh_pack2_f16(r[0], r[1]);
+      }
+      __builtin_memcpy(a.out + first + size_t(row) * a.HW, &o, 16);
+    }
+    return;
+  }
+  __syncthreads();
+  if (go >= a.octets) return;
 #pragma unroll
   for (int i = 0; i < BM / 32; ++i) {
     const int row = (t >> 4) + 32 * i;
-    if (m0 + row < a.M) __builtin_memcpy(out + size_t(row) * a.HW, lds + row * OP + 8 * g, 16);
+    if (m0 + row < a.M) __builtin_memcpy(a.out + first + size_t(row) * a.HW, lds + row * OP + 8 * g, 16);
   }
 }
 

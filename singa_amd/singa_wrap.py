@@ -851,6 +851,20 @@ def GpuConvBackwardxAccumulate(dy, W, x, h, dx):
     return dx
 
 
+def GpuConvBackwardxAddReLU(dy, W, x, h, add):
+    """``ReLUBackwardSum(GpuConvBackwardx(dy, W, x, h), add, x)``, bit for bit: what a residual block whose input ``x`` is the
+    output of a ReLU hands to the layer in front of that ReLU (16-bit 1x1 layers of stride 1: in one launch)."""
+    if dy.data_type() == kFloat32:
+        return ReLUBackwardSum(GpuConvBackwardx(dy, W, x, h), add, x)
+    h._check_dy(dy)
+    _same(add, x)
+    dx = _like(x)
+    fn, name = _fn("conv_dgrad_add_relu", dy)
+    check(fn(_address(h.geom), dy.ptr, W.ptr, add.ptr, x.ptr, dx.ptr, h.workspace.ptr, h.workspace.MemSize(), dy.device().stream),
+          name)
+    return dx
+
+
 def GpuConvBackwardx(dy, W, x, h):
     h._check_dy(dy)
     dx = _like(x)

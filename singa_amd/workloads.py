@@ -200,6 +200,12 @@ class HipOps(object):
     def relu_bwd_add(self, dy0, dy1, x):
         return singa.ReLUBackwardSum(dy0, dy1, x)
 
+    # ... or, where the next block is a residual one as well, adds and gates in the data gradient that yields the last summand
+    fuse_dgrad_relu = False
+
+    def conv_bwd_x_add_relu(self, dy, W, x, h, add):
+        return singa.GpuConvBackwardxAddReLU(dy, W, x, h, add)
+
     # batching the tape permits: the weights do not change during a backward pass, so the re-layouts
     # that the data gradients need are done by one launch before the first backward op
     batch_relayout = True
@@ -230,7 +236,7 @@ class HipOps(object):
     def set_fusion(self, on):
         """All of this implementation's cross-op fusions on, or the reference's op-per-op tape."""
         for f in ("fuse_bn_relu", "fuse_dgrad_add", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad",
-                  "fuse_forward", "fuse_linear"):
+                  "fuse_forward", "fuse_linear", "fuse_dgrad_relu"):
             setattr(self, f, bool(on) and f in self.fusions)
 
     def accumulate(self, a, b):
@@ -272,8 +278,9 @@ class HalfHipOps(HipOps):
     # scattered 2-byte stores make a read-modify-write epilogue slower than the separate add)
     fuse_dgrad_add = False
     fuse_add_relu = True
+    fuse_dgrad_relu = True
     fusions = ("fuse_bn_relu", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
-               "fuse_linear")
+               "fuse_linear", "fuse_dgrad_relu")
 
     def __init__(self, dev, dtype):
         HipOps.__init__(self, dev)
@@ -323,10 +330,11 @@ class Conv(_Layer):
         self.x = x
         return self.ops.conv_fwd(x, self.W, self.b, self.h)
 
-    def bwd(self, dy, grads, add_into=None):
+    def bwd(self, dy, grads, add_into=None, gated_sum_with=None):
         """`add_into`: a gradient of this convolution's input that arrived earlier over another
         branch; the data gradient is added into that tensor (ops implementations with
-        ``fuse_dgrad_add``), which is returned."""
+        ``fuse_dgrad_add``), which is returned.  `gated_sum_with`: likewise, and the input is a ReLU's output: the
+        gradient in front of that ReLU is returned (``fuse_dgrad_relu``)."""
         # A weight gradient that goes to the auxiliary stream is enqueued first, so that it starts beside
         # this layer's data gradient instead of behind it (it has a workspace of its own there).
         early = getattr(self.ops, "_aux", None) is not None
@@ -336,6 +344,8 @@ class Conv(_Layer):
         # _Conv2d.backward: dx is always computed, even for the network input (autograd.py:1695-1697)
         if add_into is not None:
             dx = self.ops.conv_bwd_x_acc(dy, self.W, self.x, self.h, add_into)
+        elif gated_sum_with is not None:
+            dx = self.ops.conv_bwd_x_add_relu(dy, self.W, self.x, self.h, gated_sum_with)
         else:
             dx = self.ops.conv_bwd_x(dy, self.W, self.x, self.h)
         if not early:
@@ -418,6 +428,13 @@ class _Sum:
 
     def __init__(self, a, b):
         self.a, self.b = a, b
+
+
+class _Gated:
+    """A gradient that has been through the ReLU backward of the block it goes to."""
+
+    def __init__(self, t):
+        self.t = t
 
 
 def _summed(ops, dy):
@@ -615,8 +632,9 @@ class Bottleneck(_Layer):
             residual = self.ds_bn.fwd(self.ds_conv.fwd(x))
         return self.bn3.fwd_add_relu(self.relu3, out, residual)
 
-    def bwd(self, dy, grads):
-        d_add = self.relu3.bwd(dy, grads)
+    def bwd(self, dy, grads, behind_block=False):
+        """`behind_block`: this block's input is the ReLU output of another Bottleneck."""
+        d_add = dy.t if isinstance(dy, _Gated) else self.relu3.bwd(dy, grads)
         if self.ds_conv is not None:   # the stack pops the residual branch first, as in BasicBlock
             d_res = self.ds_conv.bwd(self.ds_bn.bwd(d_add, grads), grads)
         else:
@@ -626,6 +644,8 @@ class Bottleneck(_Layer):
         d = self.bn1.bwd_through_relu(self.relu1, d, grads)
         if getattr(self.ops, "fuse_dgrad_add", False):
             return self.conv1.bwd(d, grads, add_into=d_res)
+        if behind_block and getattr(self.ops, "fuse_dgrad_relu", False):
+            return _Gated(self.conv1.bwd(d, grads, gated_sum_with=d_res))
         d_main = self.conv1.bwd(d, grads)
         if getattr(self.ops, "fuse_add_relu", False):
             return _Sum(d_main, d_res)
@@ -729,7 +749,10 @@ class Net(object):
                 else:
                     if not isinstance(rev[i], (BasicBlock, Bottleneck)):
                         dy = _summed(ops, dy)
-                    dy = rev[i].bwd(dy, grads)
+                    if isinstance(rev[i], Bottleneck):
+                        dy = rev[i].bwd(dy, grads, behind_block=i + 1 < len(rev) and isinstance(rev[i + 1], Bottleneck))
+                    else:
+                        dy = rev[i].bwd(dy, grads)
                     i += 1
             dy = _summed(ops, dy)
         finally:

@@ -712,6 +712,30 @@ def test_pointwise_weight_gradient_16bit_edges(singa, dev, kind, N, C, H, W, K):
     assert np.array_equal(np.isnan(got[:, C - 1]), at == 0) and np.array_equal(np.sign(got[at != 0, C - 1]), np.sign(at[at != 0]))
 
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("N,C,H,W,K,R,stride", [(2, 64, 8, 9, 64, 1, 1), (3, 300, 7, 7, 72, 1, 1), (40, 130, 14, 14, 64, 1, 1), (70, 256, 28, 28, 64, 1, 1),
+                                                (5, 70, 5, 5, 40, 1, 1), (2, 64, 8, 8, 64, 3, 1), (2, 64, 8, 8, 64, 1, 2), (2, 8, 6, 6, 12, 1, 1)])
+def test_data_gradient_with_sum_and_gate(singa, dev, kind, N, C, H, W, K, R, stride):
+    """GpuConvBackwardxAddReLU stores the bits of GpuConvBackwardx and ReLUBackwardSum: tiles of 64, 128 and 256 channels, planes
+    whose last octet overlaps, and layers of the other kernels, where it is those two calls; NaNs and infinities in every operand."""
+    r = rng(N + C + H + K)
+    dt = {"f16": singa.kFloat16, "bf16": singa.kBFloat16}[kind]
+    to = lambda *s: singa.from_numpy(r.standard_normal(s).astype(np.float32), dev).AsType(dt)
+
+    def bad(*s):
+        a = r.standard_normal(s).astype(np.float32)
+        a.ravel()[r.integers(0, a.size, 5)] = [np.nan, np.inf, -np.inf, 0.0, -0.0]
+        return singa.from_numpy(a, dev).AsType(dt)
+    x, add, w = bad(N, C, H, W), bad(N, C, H, W), to(K, C, R, R)
+    h = singa.CudnnConvHandle(x, (R, R), (stride, stride), (R // 2, R // 2), C, K, False)
+    dy = bad(N, K, h.conv_height, h.conv_width)
+    back = lambda t: t.AsType(singa.kFloat32).to_numpy()   # (exact)
+    want = back(singa.ReLUBackwardSum(singa.GpuConvBackwardx(dy, w, x, h), add, x))
+    got = back(singa.GpuConvBackwardxAddReLU(dy, w, x, h, add))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got.view(np.uint32)[~np.isnan(want)], want.view(np.uint32)[~np.isnan(want)])
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
 @pytest.mark.parametrize("case", _grad16_cases(40, 777) + [
     (2, 64, 56, 56, 64, 3, 3, (1, 1), (1, 1)),      # ResNet stage-1 3x3
     (2, 256, 14, 14, 64, 1, 1, (1, 1), (0, 0)),     # bottleneck reduce: plane of 196 = 24.5 octets
