@@ -156,17 +156,28 @@ class HipOps(object):
     # are held back and go to the auxiliary stream `graph_wgrad_group` layers at a time, behind ONE fork
     # (groups of 6 to 10: 5.44 ms; ResNet-50 in 16 bits 9.70 against 9.89 ms).
     graph_wgrad_group = 8
+    # A fork costs the host 10 us, a launch 5, and a 16-bit network over a few images is bound by them: there the weight gradients
+    # of layers of up to `small_wgrad_bytes` (x and dy) are held back for groups of `small_wgrad_group` behind one fork.  ResNet-50
+    # step, groups of 1 / 2 / 4, 16 MB: 8 images 3.34 / 2.95 / 2.83 ms, 21 of 192 pixels 3.34 / 3.28 / 3.30, 128 12.38 / 12.35 / 12.37.  (In
+    # fp32 the weight gradients are long and better started at once: ResNet-18 over 8 images 2.09 / 2.15 / 2.20.)
+    small_wgrad_group, small_wgrad_bytes = 1, 16 << 20
     _deferred = ()
 
     def conv_bwd_w(self, dy, x, W, h):
         if self._aux is not None:
-            if self.dev.graph_enabled() and self.graph_wgrad_group > 1:
+            group = self.small_wgrad_group if x.MemSize() + dy.MemSize() <= self.small_wgrad_bytes else 1
+            if self.dev.graph_enabled():
+                group = self.graph_wgrad_group
+            if group > 1:
                 dW = singa.Tensor(W.shape(), W.device(), W.data_type())
                 self._deferred = list(self._deferred) + [(dy, x, W, h, dW)]
-                if len(self._deferred) >= self.graph_wgrad_group:
+                if len(self._deferred) >= group:
                     self._flush_deferred()
                 return dW
-            self._aux = self.dev.Fork()    # (everything enqueued so far, i.e. the producer of dy, comes first)
+            if self._deferred:
+                self._flush_deferred()     # (forks as well)
+            else:
+                self._aux = self.dev.Fork()    # (everything enqueued so far, i.e. the producer of dy, comes first)
             # (the tensors it touches are announced to the pool there: nothing is kept alive here)
             return singa.GpuConvBackwardW(dy, x, W, h, stream=self._aux)
         return singa.GpuConvBackwardW(dy, x, W, h)
@@ -279,6 +290,7 @@ class HalfHipOps(HipOps):
     fuse_dgrad_add = False
     fuse_add_relu = True
     fuse_dgrad_relu = True
+    small_wgrad_group = 4
     fusions = ("fuse_bn_relu", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
                "fuse_linear", "fuse_dgrad_relu")
 
