@@ -240,7 +240,8 @@ def main():
     reference_tape = None
     if not (args.no_fusion or args.with_forward or args.no_reference_tape):
         saved = {f: getattr(hip, f) for f in ("fuse_bn_relu", "fuse_dgrad_add", "fuse_add_relu", "fuse_wgrad_bias",
-                                              "batch_relayout", "overlap_wgrad", "fuse_forward", "fuse_linear", "fuse_dgrad_relu")}
+                                              "batch_relayout", "overlap_wgrad", "fuse_forward", "fuse_linear", "fuse_dgrad_relu",
+                                              "fuse_pool_relu")}
         hip.set_fusion(False)
         net.sgd.op_by_op = True     # SGD.apply's own tensor ops, three launches per parameter
         ref_steps = max(3, min(args.steps, 10))

@@ -731,6 +731,10 @@ SGH_API int sgh_pool_geom_init(sgh_pool_geom *g, int N, int C, int H, int W, int
  * row-major window order wins (src/model/layer/pooling.cc:189-196); avg: count-exclude-padding
  * (pooling.cc:70-72, :172). */
 SGH_API int sgh_pool_fwd_f32(const sgh_pool_geom *g, const float *x, float *y, void *stream);
+/* A ReLU and the max pooling behind it in one pass each way (2x2, stride 2, no padding; SGH_EUNSUPPORTED otherwise, nothing
+ * written): y = pool(relu(x)); dx = ReLUBackward(PoolingBackward(dy, relu(x), y), x).  The bits of the separate calls. */
+SGH_API int sgh_pool_relu_fwd_f32(const sgh_pool_geom *g, const float *x, float *y, void *stream);
+SGH_API int sgh_pool_relu_bwd_f32(const sgh_pool_geom *g, const float *dy, const float *x, float *dx, void *stream);
 /* GpuPoolingBackward (src/model/operation/pooling.cc:207-226), same (dy, x, y) arguments.
  * Max: dy[n,c,p,q] is routed to the first-maximum position of its window (recomputed from x;
  * y is accepted for signature parity and may be NULL), contributions of overlapping windows

@@ -211,6 +211,8 @@ SIGNATURES = {
     "sgh_bn_bwd_bf16": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, vp, sz, vp]),
     "sgh_pool_geom_init": (C.c_int, [C.POINTER(PoolGeom)] + [C.c_int] * 11),
     "sgh_pool_fwd_f32": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp]),
+    "sgh_pool_relu_fwd_f32": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp]),
+    "sgh_pool_relu_bwd_f32": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp, vp]),
     "sgh_pool_bwd_f32": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp, vp, vp]),
     "sgh_pool_fwd_f16": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp]),
     "sgh_pool_fwd_bf16": (C.c_int, [C.POINTER(PoolGeom), vp, vp, vp]),

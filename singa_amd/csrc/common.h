@@ -157,6 +157,10 @@ int sgh_wgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *x, fl
 // fp32 forward over fewer than eight input channels (fwd_few.hip); SGH_EUNSUPPORTED for geometries it does not take
 int sgh_fwd_few_run(const sgh_conv_geom *g, const float *x, const float *W, const float *bias, float *y, hipStream_t s);
 
+// fp32 data gradient, at most four input channels, 3x3 and 5x5 of stride 1 (dgrad_few.hip); no workspace
+bool sgh_dgrad_few_supported(const sgh_conv_geom *g);
+int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, float *dx, hipStream_t s);
+
 // fp32 3x3 stride-1 pad-1 weight gradient on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
 // take; the caller checks that the workspace has them.
 size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);

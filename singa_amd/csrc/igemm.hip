@@ -1118,6 +1118,8 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
   } else if (dgrad_splits(g, ws_bytes)) {
     if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
     if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
+  } else if (path == kDgradColumns && sgh_dgrad_few_supported(g)) {
+    rc = sgh_dgrad_few_run(g, dy, W, dx, s);
   } else if (path == kDgradColumns) {
     float *dcol = static_cast<float *>(workspace);
     const int CRS = g->C * RS, Ncols = g->N * g->P * g->Q;

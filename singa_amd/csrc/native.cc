@@ -75,7 +75,8 @@ struct EntryOf {
   ONE(sgh_sgd_momentum_master_f16) ONE(sgh_sgd_momentum_master_bf16) ALL(sgh_conv_fwd) ALL(sgh_conv_dgrad) ALL(sgh_conv_wgrad)  \
   ALL(sgh_conv_bgrad) ONE(sgh_conv_dgrad_acc_f32) ONE(sgh_conv_dgrad_add_relu_f16) ONE(sgh_conv_dgrad_add_relu_bf16)               \
   ONE(sgh_conv_wgrad_bias_f32) ALL(sgh_bn_fwd_train) ALL(sgh_bn_relu_fwd_train) \
-  ALL(sgh_bn_add_relu_fwd_train) ALL(sgh_bn_fwd_infer) ALL(sgh_bn_bwd) ALL(sgh_bn_relu_bwd) ALL(sgh_pool_fwd) ALL(sgh_pool_bwd)
+  ALL(sgh_bn_add_relu_fwd_train) ALL(sgh_bn_fwd_infer) ALL(sgh_bn_bwd) ALL(sgh_bn_relu_bwd) ALL(sgh_pool_fwd) ALL(sgh_pool_bwd) \
+  ONE(sgh_pool_relu_fwd_f32) ONE(sgh_pool_relu_bwd_f32)
 SGH_CALLS(SGH_ENTRY, SGH_ENTRY3)
 SGH_ENTRY(sgh_malloc)
 SGH_ENTRY(sgh_free)

@@ -351,10 +351,22 @@ struct QuadG {
   sgh_fastdiv d_bw, d_bh;
 };
 
-template <class S, bool MAX>
+// kQuadReluMax: x is the input of a ReLU in front of the pooling layer; the ReLU is applied as x is read, and its gate as the gradient
+// is stored: the bits of the two layers one after the other, without the rectified tensor and its gradient (fp32 128 x 32 x 32 x 32, forward
+// and backward: 5.5 + 4.7 + 6.7 + 7.2 us of kernels, 4.5 + 7 here).
+enum { kQuadMean, kQuadMax, kQuadReluMax };
+
+template <class S>
+__device__ __forceinline__ void rectify(Pair<S> &t, Pair<S> &b) {
+  t.lo = t.lo >= 0.f ? t.lo : 0.f, t.hi = t.hi >= 0.f ? t.hi : 0.f;
+  b.lo = b.lo >= 0.f ? b.lo : 0.f, b.hi = b.hi >= 0.f ? b.hi : 0.f;
+}
+
+template <class S, int MODE>
 __global__ __launch_bounds__(kBlock) void k_pool_quad_fwd(const typename S::elem *__restrict__ x, typename S::elem *__restrict__ y,
                                                          const QuadG g) {
   typedef typename S::elem elem;
+  constexpr bool MAX = MODE != kQuadMean;
   const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, g.x_bytes, 0x00020000);
   constexpr int U = 4;
   for (int i0 = int(blockIdx.x) * kBlock * U + int(threadIdx.x); i0 < g.total; i0 += int(gridDim.x) * kBlock * U) {
@@ -373,6 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_pool_quad_fwd(const typename S::elem
       float v;
       if (MAX) {
         v = kLowest;
+        if constexpr (MODE == kQuadReluMax) rectify<S>(t[u], b[u]);
         if (t[u].lo > v) v = t[u].lo;
         if (t[u].hi > v) v = t[u].hi;
         if (b[u].lo > v) v = b[u].lo;
@@ -385,10 +398,11 @@ __global__ __launch_bounds__(kBlock) void k_pool_quad_fwd(const typename S::elem
   }
 }
 
-template <class S, bool MAX>
+template <class S, int MODE>
 __global__ __launch_bounds__(kBlock) void k_pool_quad_bwd(const typename S::elem *__restrict__ dy, const typename S::elem *__restrict__ x,
                                                          typename S::elem *__restrict__ dx, const QuadG g, int BH, unsigned y_bytes) {
   typedef typename S::elem elem;
+  constexpr bool MAX = MODE != kQuadMean;
   const rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(x), 0, MAX ? g.x_bytes : 0, 0x00020000);
   const rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(const_cast<elem *>(dy), 0, y_bytes, 0x00020000);
   constexpr int U = 4;
@@ -416,12 +430,17 @@ __global__ __launch_bounds__(kBlock) void k_pool_quad_bwd(const typename S::elem
       if (MAX) {
         float v = kLowest;
         int k = -1;
+        bool open[4] = {true, true, true, true};
+        if constexpr (MODE == kQuadReluMax) {
+          open[0] = t[u].lo > 0.f, open[1] = t[u].hi > 0.f, open[2] = b[u].lo > 0.f, open[3] = b[u].hi > 0.f;
+          rectify<S>(t[u], b[u]);
+        }
         if (t[u].lo > v) v = t[u].lo, k = 0;
         if (t[u].hi > v) v = t[u].hi, k = 1;
         if (b[u].lo > v) v = b[u].lo, k = 2;
         if (b[u].hi > v) k = 3;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = 0.f + (k == e ? d[u] : 0.f);   // (a block without a window read d = 0)
+        for (int e = 0; e < 4; ++e) o[e] = open[e] ? 0.f + (k == e ? d[u] : 0.f) : 0.f;   // (a block without a window read d = 0)
       } else {
         o[0] = o[1] = o[2] = o[3] = 0.f + d[u] / 4.f;
       }
@@ -823,7 +842,7 @@ int pool_fwd(const sgh_pool_geom *g, const typename S::elem *x, typename S::elem
                               : k_pool_max_fwd_strip<S, 64>;
     hipLaunchKernelGGL(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, sg);
   } else if (quad_plan(g, esize, false, &qg)) {
-    auto kern = g->is_max ? k_pool_quad_fwd<S, true> : k_pool_quad_fwd<S, false>;
+    auto kern = g->is_max ? k_pool_quad_fwd<S, kQuadMax> : k_pool_quad_fwd<S, kQuadMean>;
     hipLaunchKernelGGL(kern, dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, qg);
   } else if (g->is_max)
     hipLaunchKernelGGL(k_pool_max_fwd<S>, dim3(grid_for(total)), dim3(kBlock), 0, sgh_stream_of(stream), x, y, to_g(g),
@@ -872,7 +891,7 @@ int pool_bwd(const sgh_pool_geom *g, const typename S::elem *dy, const typename 
                               : k_pool_max_bwd_strip<S, 64>;
     SGH_LAUNCH_TIMED(kern, dim3(strip_blocks(sg)), dim3(kBlock), 0, sgh_stream_of(stream), dy, x, dx, sg);
   } else if (quad_plan(g, esize, true, &qg)) {
-    auto kern = g->is_max ? k_pool_quad_bwd<S, true> : k_pool_quad_bwd<S, false>;
+    auto kern = g->is_max ? k_pool_quad_bwd<S, kQuadMax> : k_pool_quad_bwd<S, kQuadMean>;
     SGH_LAUNCH_TIMED(kern, dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0, sgh_stream_of(stream), dy, x, dx, qg,
                      (g->H + 1) / 2, unsigned(size_t(g->N) * g->C * g->P * g->Q * esize));
   } else if (g->is_max) {
@@ -949,6 +968,24 @@ int sgh_pool_fwd_f16(const sgh_pool_geom *g, const uint16_t *x, uint16_t *y, voi
 }
 int sgh_pool_fwd_bf16(const sgh_pool_geom *g, const uint16_t *x, uint16_t *y, void *stream) {
   return pool_fwd<StBF16>(g, x, y, stream);
+}
+int sgh_pool_relu_fwd_f32(const sgh_pool_geom *g, const float *x, float *y, void *stream) {
+  if (!geom_ok(g) || !x || !y) return SGH_EINVAL;
+  QuadG qg;
+  if (!g->is_max || !quad_plan(g, 4, false, &qg)) return SGH_EUNSUPPORTED;
+  hipLaunchKernelGGL((k_pool_quad_fwd<StF32, kQuadReluMax>), dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0,
+                     sgh_stream_of(stream), x, y, qg);
+  SGH_LAUNCH_CHECK();
+  return SGH_OK;
+}
+int sgh_pool_relu_bwd_f32(const sgh_pool_geom *g, const float *dy, const float *x, float *dx, void *stream) {
+  if (!geom_ok(g) || !dy || !x || !dx) return SGH_EINVAL;
+  QuadG qg;
+  if (!g->is_max || !quad_plan(g, 4, true, &qg)) return SGH_EUNSUPPORTED;
+  hipLaunchKernelGGL((k_pool_quad_bwd<StF32, kQuadReluMax>), dim3(grid_for((size_t(qg.total) + 3) / 4)), dim3(kBlock), 0,
+                     sgh_stream_of(stream), dy, x, dx, qg, (g->H + 1) / 2, unsigned(size_t(g->N) * g->C * g->P * g->Q * 4));
+  SGH_LAUNCH_CHECK();
+  return SGH_OK;
 }
 int sgh_pool_bwd_f32(const sgh_pool_geom *g, const float *dy, const float *x, const float *y, float *dx,
                      void *stream) {

@@ -1081,6 +1081,32 @@ def GpuPoolingForward(h, x):
     return y
 
 
+def GpuPoolingReLUForward(h, x):
+    """``GpuPoolingForward(h, ReLU(x))``, for 2x2 maxima of stride 2 in one launch; the bits of the two calls."""
+    if x.data_type() == kFloat32:
+        y = _empty(Tensor, h.dy_shape, x.device(), kFloat32)
+        rc = _L().sgh_pool_relu_fwd_f32(_address(h.geom), x.ptr, y.ptr, x.device().stream)
+        if rc != _lib.SGH_EUNSUPPORTED:
+            check(rc, "sgh_pool_relu_fwd_f32")
+            return y
+    return GpuPoolingForward(h, ReLU(x))
+
+
+def GpuPoolingReLUBackward(h, dy, x, y):
+    """``ReLUBackward(GpuPoolingBackward(h, dy, ReLU(x), y), x)``, as ``GpuPoolingReLUForward``."""
+    if dy._shape != h.dy_shape:
+        raise SingaHipError("dy shape does not match the handle")
+    if dy.data_type() != x.data_type():
+        raise SingaHipError("dy and x differ in data type")
+    if x.data_type() == kFloat32:
+        dx = _like(x)
+        rc = _L().sgh_pool_relu_bwd_f32(_address(h.geom), dy.ptr, x.ptr, dx.ptr, dy.device().stream)
+        if rc != _lib.SGH_EUNSUPPORTED:
+            check(rc, "sgh_pool_relu_bwd_f32")
+            return dx
+    return ReLUBackward(GpuPoolingBackward(h, dy, ReLU(x), y), x)
+
+
 def GpuPoolingBackward(h, dy, x, y):
     if dy._shape != h.dy_shape:
         raise SingaHipError("dy shape does not match the handle")

@@ -80,6 +80,15 @@ class HipOps(object):
     def pool_fwd(self, h, x):
         return singa.GpuPoolingForward(h, x)
 
+    # cross-op fusion the tape permits: a ReLU with the 2x2 max pooling behind it
+    fuse_pool_relu = True
+
+    def pool_relu_fwd(self, h, x):
+        return singa.GpuPoolingReLUForward(h, x)
+
+    def pool_relu_bwd(self, h, dy, x, y):
+        return singa.GpuPoolingReLUBackward(h, dy, x, y)
+
     def relu(self, x):
         return singa.ReLU(x)
 
@@ -242,12 +251,12 @@ class HipOps(object):
             self._aux = None
 
     fusions = ("fuse_bn_relu", "fuse_dgrad_add", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
-               "fuse_linear")   # what set_fusion(True) turns on
+               "fuse_linear", "fuse_pool_relu")   # what set_fusion(True) turns on
 
     def set_fusion(self, on):
         """All of this implementation's cross-op fusions on, or the reference's op-per-op tape."""
         for f in ("fuse_bn_relu", "fuse_dgrad_add", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad",
-                  "fuse_forward", "fuse_linear", "fuse_dgrad_relu"):
+                  "fuse_forward", "fuse_linear", "fuse_dgrad_relu", "fuse_pool_relu"):
             setattr(self, f, bool(on) and f in self.fusions)
 
     def accumulate(self, a, b):
@@ -291,6 +300,7 @@ class HalfHipOps(HipOps):
     fuse_add_relu = True
     fuse_dgrad_relu = True
     small_wgrad_group = 4
+    fuse_pool_relu = False
     fusions = ("fuse_bn_relu", "fuse_add_relu", "fuse_wgrad_bias", "batch_relayout", "overlap_wgrad", "fuse_forward",
                "fuse_linear", "fuse_dgrad_relu")
 
@@ -485,6 +495,25 @@ class Pool(_Layer):
         self.x = x
         self.y = self.ops.pool_fwd(self.h, x)
         return self.y
+
+    def _takes_relu(self):
+        return getattr(self.ops, "fuse_pool_relu", False) and self.cfg == ((2, 2), (2, 2), (0, 0), True)
+
+    def fwd_of_relu(self, relu, x):
+        """Forward of ``self(relu(x))``, in one pass where the ops implementation offers it; both layers then keep x."""
+        if not self._takes_relu():
+            return self.fwd(relu.fwd(x))
+        if self.h is None:
+            self.h = self.ops.pool_handle(x, *self.cfg)
+        self.x = relu.x = x
+        self.y = self.ops.pool_relu_fwd(self.h, x)
+        return self.y
+
+    def bwd_through_relu(self, relu, dy, grads):
+        """Backward of ``self(relu(_))``.  (Whether x has been through the ReLU or not, its maxima and its gate are the same.)"""
+        if not self._takes_relu():
+            return relu.bwd(self.bwd(dy, grads), grads)
+        return self.ops.pool_relu_bwd(self.h, dy, self.x, self.y)
 
     def bwd(self, dy, grads):
         return self.ops.pool_bwd(self.h, dy, self.x, self.y)
@@ -717,6 +746,9 @@ class Net(object):
             if isinstance(l, (BatchNorm, Linear)) and i + 1 < len(self.layers) and isinstance(self.layers[i + 1], ReLU):
                 x = l.fwd_through_relu(self.layers[i + 1], x)   # the stem's conv -> BatchNorm -> ReLU, a hidden dense layer
                 i += 2
+            elif isinstance(l, ReLU) and i + 1 < len(self.layers) and isinstance(self.layers[i + 1], Pool):
+                x = self.layers[i + 1].fwd_of_relu(l, x)
+                i += 2
             else:
                 x = l.fwd(x)
                 i += 1
@@ -754,6 +786,9 @@ class Net(object):
             while i < len(rev):
                 if isinstance(rev[i], ReLU) and i + 1 < len(rev) and isinstance(rev[i + 1], BatchNorm):
                     dy = rev[i + 1].bwd_through_relu(rev[i], _summed(ops, dy), grads)   # the stem's conv -> BatchNorm -> ReLU
+                    i += 2
+                elif isinstance(rev[i], Pool) and i + 1 < len(rev) and isinstance(rev[i + 1], ReLU) and rev[i]._takes_relu():
+                    dy = rev[i].bwd_through_relu(rev[i + 1], _summed(ops, dy), grads)
                     i += 2
                 elif isinstance(rev[i], Linear) and i + 1 < len(rev) and isinstance(rev[i + 1], ReLU):
                     dy = rev[i].bwd_behind_relu(rev[i + 1], _summed(ops, dy), grads)

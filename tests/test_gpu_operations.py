@@ -1292,3 +1292,54 @@ def test_conv_forward_few_channels_wide_blocks(singa, dev, n, c, h, w, k, r, st,
     got = run(x, False)
     hit = conv((~np.isfinite(x)).astype(np.float32), np.ones_like(W), 0 * b) > 0
     assert np.array_equal(~np.isfinite(got), hit)
+
+
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, 1, 3, 1), (3, 3, 8, 32, 5, 5, 2), (2, 3, 9, 33, 32, 5, 2), (2, 2, 31, 65, 7, 3, 1), (3, 4, 17, 40, 9, 5, 0),
+                                  (2, 4, 12, 29, 3, 3, 2), (128, 3, 32, 32, 32, 5, 2)])
+@pytest.mark.parametrize("bad", [0.0, np.inf, np.nan])
+def test_data_gradient_with_few_input_channels(singa, dev, case, bad):
+    """One to four input channels, 3x3 and 5x5 of stride 1 on the vector ALUs: edges of the tiles of 8 x 32, paddings, fewer filters
+    than wavefronts.  Bound: K R^2 products, |error| <= (R^2 + K / 4 + 4) 2^-24 sum |dy w|.  An infinity or NaN of a filter reaches the
+    pixels that it is multiplied with and no others."""
+    N, C, H, W, K, R, pad = case
+    print("few input channels", case, bad, flush=True)
+    r = rng(sum(case))
+    w = randn(r, K, C, R, R)
+    if bad != 0.0:
+        w[K - 1, 0, 0, R - 1] = w[0, C - 1, R - 1, 0] = bad
+    x = singa.from_numpy(np.zeros((N, C, H, W), np.float32), dev)
+    h = singa.CudnnConvHandle(x, (R, R), (1, 1), (pad, pad), C, K, False)
+    dy = randn(r, N, K, h.conv_height, h.conv_width)
+    got = singa.GpuConvBackwardx(singa.from_numpy(dy, dev), singa.from_numpy(w, dev), x, h).to_numpy()
+    want, size = np.zeros((N, C, H + 2 * pad, W + 2 * pad)), np.zeros((N, C, H + 2 * pad, W + 2 * pad))
+    with np.errstate(invalid="ignore"):
+        for i in range(R):
+            for j in range(R):
+                t = dy[:, :, None].astype(np.float64) * w[None, :, :, i, j, None, None]
+                want[:, :, i:i + dy.shape[2], j:j + dy.shape[3]] += t.sum(1)
+                size[:, :, i:i + dy.shape[2], j:j + dy.shape[3]] += np.abs(t).sum(1)
+    cut = slice(pad, pad + H), slice(pad, pad + W)
+    want, size = want[:, :, cut[0], cut[1]], size[:, :, cut[0], cut[1]]
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), ok)
+    assert np.all(np.abs(got[ok] - want[ok]) <= (R * R + K / 4 + 4) * 2.0 ** -24 * size[ok])
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 8, 8), (3, 5, 7, 9), (1, 1, 2, 2), (40, 16, 33, 30)])
+def test_pooling_through_relu_stores_the_bits_of_the_two_layers(singa, dev, shape):
+    """GpuPoolingReLUForward / Backward against ReLU and pooling: 2x2 maxima in one launch (even and odd planes), other windows by the
+    two calls; ties, zeros of either sign, infinities and NaNs."""
+    r = rng(sum(shape))
+    x = np.round(randn(r, *shape) * 2) / 2
+    x.ravel()[r.integers(0, x.size, 6)] = [np.nan, np.inf, -np.inf, -0.0, 0.0, np.nan]
+    xd = singa.from_numpy(x.astype(np.float32), dev)
+    for kernel, stride, pad, is_max in (((2, 2), (2, 2), (0, 0), True), ((2, 2), (1, 1), (0, 0), True), ((2, 2), (2, 2), (0, 0), False)):
+        h = singa.CudnnPoolingHandle(xd, kernel, stride, pad, is_max)
+        a = singa.ReLU(xd)
+        z = singa.GpuPoolingForward(h, a)
+        got = singa.GpuPoolingReLUForward(h, xd)
+        np.testing.assert_array_equal(got.to_numpy().view(np.uint32), z.to_numpy().view(np.uint32))
+        dz = singa.from_numpy(randn(r, *z.shape()), dev)
+        want = singa.ReLUBackward(singa.GpuPoolingBackward(h, dz, a, z), xd).to_numpy()
+        np.testing.assert_array_equal(singa.GpuPoolingReLUBackward(h, dz, xd, z).to_numpy().view(np.uint32), want.view(np.uint32))
+
