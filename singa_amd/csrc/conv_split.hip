@@ -19,6 +19,8 @@
 //
 //   out[n][c][h][w] = sum_{k,r,s} in[n][k][h + r - o][w + s - o] * Wf[c][k][r][s],   o = (R - 1) / 2
 //
+// (forward passes of 3x3 and stride 2 as well: in[n][k][2 h + r - o][2 w + s - o])
+//
 // forward: Wf = W; data gradient: Wf[c][k][r][s] = W[k][c][R - 1 - r][R - 1 - s].
 //
 // GEMM view: M = output channels, N = consecutive pixels of the flattened (n, h, w) index, reduction = (k, tap) in chunks of
@@ -31,6 +33,11 @@
 //
 // 512 threads = 8 wavefronts of at most 128 registers, two workgroups per CU where the slab takes no more than 80 KB of LDS: while
 // one stages and waits at its barriers the other one's matrix instructions run.
+//
+// Stride 2, whole forward calls, the generic kernel (igemm.hip) and here: 64 images of 64 channels, 56 x 56, to 128 125 -> 103 us, of 128,
+// 28 x 28, to 256 163 -> 69, of 256, 14 x 14, to 512 169 -> 77; 13 of 256, 10 x 10, to 512 108 -> 33 (48 workgroups before); the error
+// 0.12 to 0.35 times, and over 34 drawn layers none slower than 0.97.  The tiles are the ones of stride 1; a wavefront of two blocks with
+// three slab elements a thread, ten registers spilled, is faster than one block (28 x 28: 69 / 75, 14 x 14: 77 / 92).
 //
 // 64 images, whole calls, on fp32 instructions (dgrad3x3.hip) and here: 64 channels of 56 x 56 forward 143 -> 97 us, data gradient
 // 131 -> 90; 128 of 28 x 28 139 -> 94, 128 -> 90; 256 of 14 x 14 145 -> 97, 136 -> 91; 512 of 7 x 7 156 -> 106, 137 -> 100.  The error
@@ -75,7 +82,8 @@ struct ScArgs {
   float *partials;        // [workgroup][BM * BN]
   int accumulate;         // out += result
   int dgrad;
-  int N, C, K, P, Q;      // in is N x K x P x Q, out N x C x P x Q
+  int N, C, K, P, Q;      // in is N x K x IH x IW, out N x C x P x Q
+  int IH, IW, plane;      // P and Q at stride 1; bytes of IH x IW
   int cblocks;            // 32-row blocks of the weight fragments
   int pitch, slab;        // LDS row pitch and positions of the slab (rows * pitch)
   int total_pix, nchunks;
@@ -92,8 +100,21 @@ __device__ __forceinline__ int whole_tile_of(const ScArgs &a, int w) {   // see 
   return (((j >> 3) << 3) + x) * 8 + (j & 7);
 }
 
-// GM x (NW / GM) wavefronts, each on WM x WN blocks of 32 x 32; ET: slab elements (octet, position) per thread; R: filter size.
-template <int GM, int WM, int WN, int ET, int R>
+// Column of the input at place `at` of a slab row, from the left padding on, and the other way round.  At stride 2 the even columns come
+// first, then the odd ones, so that neighbouring pixels read neighbouring places for every tap.
+template <int ST>
+__device__ __forceinline__ int column_at(int at, int pitch) {
+  const int even = (pitch + 1) >> 1;
+  return ST == 1 ? at : at < even ? 2 * at : 2 * (at - even) + 1;
+}
+template <int ST>
+__device__ __forceinline__ int place_of(int column, int pitch) {
+  return ST == 1 ? column : (column & 1) * ((pitch + 1) >> 1) + (column >> 1);
+}
+
+// GM x (NW / GM) wavefronts, each on WM x WN blocks of 32 x 32; ET: slab elements (octet, position) per thread; R: filter size;
+// ST: stride (2: forward passes only).
+template <int GM, int WM, int WN, int ET, int R, int ST>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_split(ScArgs a) {
   constexpr int GN = NW / GM, BM = GM * WM * 32, BN = GN * WN * 32, TAPS = R * R, O = (R - 1) / 2;
   constexpr int AD = 2;                       // weight fragments: this tap's and the next one's
@@ -101,7 +122,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   extern __shared__ __align__(16) char smem[];
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave / GN, wn = wave % GN;
-  const int PQ = a.P * a.Q, VH = a.P + 2 * O;
+  const int PQ = a.P * a.Q, IH = ST == 1 ? a.P : a.IH, IW = ST == 1 ? a.Q : a.IW, VH = IH + 2 * O;
   const rsrc_t rin = make_rsrc(a.in, a.in_bytes), rwt = make_rsrc(a.wt, a.wt_bytes);
 
   const int rest = int(blockIdx.x) - a.dp_tiles, part = rest < 0 ? 0 : rest % a.share;
@@ -110,17 +131,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   const int ch_begin = whole ? 0 : part * a.nchunks / a.share, ch_end = whole ? a.nchunks : (part + 1) * a.nchunks / a.share;
   const int c0 = (tile % a.ctiles) * BM, pix0 = (tile / a.ctiles) * BN;
   const int n_first = pix0 / PQ, h_first = (pix0 - n_first * PQ) / a.Q;
-  const int vbase = n_first * VH + h_first;   // virtual row of the slab's first row
+  const int vbase = n_first * VH + h_first * ST;   // virtual row of the slab's first row
 
-  // ---- slab loader: element e * NT + t = (octet, position); channel k0 + 8 octet + j is the scalar offset j * PQ away
+  // ---- slab loader: element e * NT + t = (octet, position); channel k0 + 8 octet + j is the scalar offset j * IH * IW away
   int g0[ET];
 #pragma unroll
   for (int e = 0; e < ET; ++e) {
     const int idx = e * NT + t, oct = idx >= a.slab, pos = idx - (oct ? a.slab : 0);
-    const int vr = pos / a.pitch, col = pos - vr * a.pitch, v = vbase + vr, n = v / VH;
+    const int vr = pos / a.pitch, col = column_at<ST>(pos - vr * a.pitch, a.pitch), v = vbase + vr, n = v / VH;
     const int p = v - n * VH - O, q = col - O;
-    const bool ok = idx < 2 * a.slab && n < a.N && unsigned(p) < unsigned(a.P) && unsigned(q) < unsigned(a.Q);
-    g0[e] = ok ? (((n * a.K + oct * 8) * a.P + p) * a.Q + q) * 4 : kOOB;
+    const bool ok = idx < 2 * a.slab && n < a.N && unsigned(p) < unsigned(IH) && unsigned(q) < unsigned(IW);
+    g0[e] = ok ? (((n * a.K + oct * 8) * IH + p) * IW + q) * 4 : kOOB;
   }
   float st[ET][8];
   // (no branch: behind one, the waits for the weights would have to count on none of these loads and wait for them too.
@@ -130,7 +151,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       st[e][j] = __builtin_bit_cast(
-          float, __builtin_amdgcn_raw_buffer_load_b32(rin, j < valid ? g0[e] : kOOB, (k0 + j) * PQ * 4, 0));
+          float, __builtin_amdgcn_raw_buffer_load_b32(rin, j < valid ? g0[e] : kOOB, ST == 1 ? (k0 + j) * PQ * 4 : (k0 + j) * a.plane, 0));
   };
   auto stage = [&]() {
 #pragma unroll
@@ -150,7 +171,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   for (int j = 0; j < WN; ++j) {
     const int pix = min(pix0 + (wn * WN + j) * 32 + l32, a.total_pix - 1);   // (a tail lane computes a pixel it does not store)
     const int pn = pix / PQ, prem = pix - pn * PQ, ph = prem / a.Q, pw = prem - ph * a.Q;
-    boff[j] = ((pn * VH + ph - vbase) * a.pitch + pw + (lane >> 5) * a.slab) * kPos;
+    boff[j] = ((pn * VH + ph * ST - vbase) * a.pitch + pw + (lane >> 5) * a.slab) * kPos;   // (place_of an even column: pw)
     pixn[j] = pn;
   }
 
@@ -179,7 +200,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
   // operand fragment of block j at a tap
   v4u b[3];
   auto fragment = [&](int tap, int j) {
-    const char *p = smem + boff[j] + tap / R * a.pitch * kPos + tap % R * kPos;
+    const char *p = smem + boff[j] + (tap / R * a.pitch + place_of<ST>(tap % R, a.pitch)) * kPos;
 #pragma unroll
     for (int k = 0; k < 3; ++k) b[k] = *reinterpret_cast<const v4u *>(p + k * 16);
   };
@@ -280,15 +301,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     // (Everything is derived anew from opaque copies: what the loop above holds in registers for this, it spills.)
     static_assert(WM == 1, "");
     float *const xs = reinterpret_cast<float *>(smem);
-    int tt = threadIdx.x, P = a.P, Q = a.Q, slab = a.slab, pitch = a.pitch;
+    int tt = threadIdx.x, P = IH, Q = IW, slab = a.slab, pitch = a.pitch;   // (of the input)
     asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q), "+s"(slab), "+s"(pitch));
     const int half = tt >> 5 & 1, column = tt & 31, c = min(c0 + wm * 32 + column, a.C - 1), vh = P + 2 * O;
     int ph[WN], pw[WN], base[WN];   // this lane's pixels: row, column, place in the slab of channel 8 half
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
-      const int pix = min(pix0 + (wn * WN + j) * 32 + column, a.total_pix - 1), n = pix / (P * Q), rem = pix - n * P * Q;
-      ph[j] = rem / Q, pw[j] = rem - ph[j] * Q;
-      base[j] = (n * vh + ph[j] - vbase) * pitch + pw[j] + half * 8 * slab;
+      const int pix = min(pix0 + (wn * WN + j) * 32 + column, a.total_pix - 1), pq = ST == 1 ? P * Q : PQ, qq = ST == 1 ? Q : a.Q, n = pix / pq, rem = pix - n * pq;
+      ph[j] = rem / qq, pw[j] = rem - ph[j] * qq;
+      base[j] = (n * vh + ph[j] * ST - vbase) * pitch + pw[j] + half * 8 * slab;
     }
     // not every result of this wavefront, of the workgroup is a NaN yet (in a diverged network they soon are)
     bool number = true;
@@ -303,7 +324,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
       if (*numbers < ch - 1) break;
 #pragma unroll 1
       for (int i = tt; i < 2 * slab; i += NT) {
-        const int oct = i >= slab, pos = i - (oct ? slab : 0), vr = pos / pitch, q = pos - vr * pitch - O, v = vbase + vr, n = v / vh;
+        const int oct = i >= slab, pos = i - (oct ? slab : 0), vr = pos / pitch, q = column_at<ST>(pos - vr * pitch, pitch) - O, v = vbase + vr, n = v / vh;
         const int p = v - n * vh - O, k0 = ch * KC + oct * 8;
         const bool in = n < a.N && unsigned(p) < unsigned(P) && unsigned(q) < unsigned(Q);
         const float *const src = a.in + ((size_t(n) * a.K + k0) * P + p) * Q + q;
@@ -321,7 +342,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         float w[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) w[k] = k0 + k < a.K ? wp[size_t(k0 + k) * a.w_k] : 0.f;
-        const float *const xt = xs + tap / R * pitch + tap % R;
+        const float *const xt = xs + tap / R * pitch + place_of<ST>(tap % R, pitch);
         if (apart) {
 #pragma unroll 1
           for (int k = 0; k < 8; ++k) {
@@ -398,23 +419,25 @@ __global__ __launch_bounds__(256) void k_conv_split_fixup(ScArgs a, int BM, int 
 
 struct ScPlan {
   bool ok;
-  int r, gm, wm, wn, et, bm, bn, pitch, rows, slab, nchunks, cblocks;
+  int r, st, gm, wm, wn, et, bm, bn, ih, iw, pitch, rows, slab, nchunks, cblocks;
   int ctiles, tiles, dp_tiles, share, wgs;
 };
 
 ScPlan plan(const sgh_conv_geom *g) {
   ScPlan p{};
-  if ((g->R != 3 && g->R != 5) || g->S != g->R || g->stride_h != 1 || g->stride_w != 1) return p;
+  // (stride 2: the geometry of a forward pass with its channels swapped)
+  if ((g->R != 3 && g->R != 5) || g->S != g->R || g->stride_h != g->stride_w || g->stride_h < 1 || g->stride_h > (g->R == 3 ? 2 : 1)) return p;
   const int o = (g->R - 1) / 2;
+  p.st = g->stride_h, p.ih = p.st == 1 ? g->P : g->H, p.iw = p.st == 1 ? g->Q : g->W;
   if (g->pad_h != o || g->pad_w != o) return p;
   // (below eight channels the padded reduction rounds more often than the fp32 instructions do on the few products there are:
   // 5x5 over 3 channels 1.5e-7 -> 2.0e-7 from float64)
   if (g->K < 8) return p;
   const size_t lim = size_t(1) << 31;
-  if (size_t(g->N) * g->K * g->P * g->Q * 4 >= lim || size_t(g->N) * g->C * g->P * g->Q * 4 >= lim) return p;
-  if (size_t(g->N) * (g->P + 2 * o) >= lim / 64) return p;
+  if (size_t(g->N) * g->K * p.ih * p.iw * 4 >= lim || size_t(g->N) * g->C * g->P * g->Q * 4 >= lim) return p;
+  if (size_t(g->N) * (p.ih + 2 * o) >= lim / 64) return p;
   p.r = g->R;
-  p.pitch = g->Q + 2 * o;
+  p.pitch = (g->Q - 1) * p.st + p.r;
   p.nchunks = (g->K + KC - 1) / KC;
   p.cblocks = (g->C + 31) / 32;
   if (size_t(p.nchunks) * p.r * p.r * p.cblocks * kFrag >= lim) return p;
@@ -429,8 +452,22 @@ ScPlan plan(const sgh_conv_geom *g) {
   auto take = [&](int gm, int wn) {
     p.gm = gm, p.wm = 1, p.wn = wn, p.bm = gm * 32, p.bn = NW / gm * wn * 32;
     // virtual rows a tile can touch: its pixel rows, the halo rows, and the zero rows of every image boundary it crosses
-    p.rows = (p.bn + g->Q - 2) / g->Q + 1 + 2 * o + 2 * o * ((p.bn - 1) / (g->P * g->Q) + 1);
-    return long(p.rows) * p.pitch <= kMaxSlab;
+    const int vh = p.ih + 2 * o, pq = g->P * g->Q;
+    p.rows = (p.bn + g->Q - 2) / g->Q * p.st + p.r + (vh - g->P * p.st) * ((p.bn - 1) / pq + 1);
+    int a = pq, b = p.bn;   // the distinct places in an image where a tile begins, if they are few: not the bound but what it is
+    while (b) {
+      const int m = a % b;
+      a = b, b = m;
+    }
+    if (p.st > 1 && pq / a <= 256) {
+      p.rows = 0;
+      for (int first = 0; first < pq; first += a) {
+        const int last = first + p.bn - 1;
+        const int rows = last / pq * vh + last % pq / g->Q * p.st + p.r - first / g->Q * p.st;
+        if (rows > p.rows) p.rows = rows;
+      }
+    }
+    return long(p.rows) * p.pitch <= (p.st > 1 && wn > 1 ? 3 * NT / 2 : kMaxSlab);   // (four elements per thread: spills)
   };
   bool fits = false;
   // (too few chunks to give every CU one: small tiles.  204 filters over 14 channels, 10 x 2 tiles: 16.5 -> 13 us)
@@ -440,6 +477,7 @@ ScPlan plan(const sgh_conv_geom *g) {
   if (!fits && !take(1, 1)) return p;
   p.slab = p.rows * p.pitch;
   p.et = (2 * p.slab + NT - 1) / NT;
+  if (p.st > 1 && p.et < 2) p.et = 2;   // (a kernel less)
   p.ctiles = (g->C + p.bm - 1) / p.bm;
   const long tiles = long(p.ctiles) * ((pixels + p.bn - 1) / p.bn);
   if (tiles >= (long(1) << 30)) return p;
@@ -457,9 +495,9 @@ ScPlan plan(const sgh_conv_geom *g) {
   return p;
 }
 
-template <int GM, int WM, int WN, int ET, int R>
+template <int GM, int WM, int WN, int ET, int R, int ST>
 int launch(const ScArgs &a, const ScPlan &p, hipStream_t s) {
-  auto kern = k_conv_split<GM, WM, WN, ET, R>;
+  auto kern = k_conv_split<GM, WM, WN, ET, R, ST>;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
@@ -527,18 +565,23 @@ int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, 
   a.accumulate = accumulate ? 1 : 0;
   a.dgrad = dgrad ? 1 : 0;
   a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
+  a.IH = p.ih, a.IW = p.iw, a.plane = p.ih * p.iw * 4;
   a.cblocks = p.cblocks, a.pitch = p.pitch, a.slab = p.slab;
   a.total_pix = g->N * g->P * g->Q, a.nchunks = p.nchunks;
   a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share;
   a.xcd_runs = p.dp_tiles % 64 == 0 && !sgh_env().conv_xcd_off;
-  a.in_bytes = unsigned(size_t(g->N) * g->K * g->P * g->Q * 4);
+  a.in_bytes = unsigned(size_t(g->N) * g->K * p.ih * p.iw * 4);
   a.wt_bytes = unsigned(sgh_conv_split_weight_bytes(g));
   int rc = SGH_EUNSUPPORTED;
   sgh_prof_kernel_begin(tag, 2.0 * g->N * g->K * g->P * g->Q * g->C * p.r * p.r);
-#define SC_CASE(GM_, WM_, WN_, ET_, R_) \
-  if (p.gm == GM_ && p.wm == WM_ && p.wn == WN_ && p.et == ET_ && p.r == R_) rc = launch<GM_, WM_, WN_, ET_, R_>(a, p, s);
+#define SC_CASE(GM_, WM_, WN_, ET_, R_, ST_) \
+  if (p.gm == GM_ && p.wm == WM_ && p.wn == WN_ && p.et == ET_ && p.r == R_ && p.st == ST_) rc = launch<GM_, WM_, WN_, ET_, R_, ST_>(a, p, s);
 #define SC_CASES(GM_, WM_, WN_, R_) \
-  SC_CASE(GM_, WM_, WN_, 1, R_) SC_CASE(GM_, WM_, WN_, 2, R_) SC_CASE(GM_, WM_, WN_, 3, R_) SC_CASE(GM_, WM_, WN_, 4, R_)
+  SC_CASE(GM_, WM_, WN_, 1, R_, 1) SC_CASE(GM_, WM_, WN_, 2, R_, 1) SC_CASE(GM_, WM_, WN_, 3, R_, 1) SC_CASE(GM_, WM_, WN_, 4, R_, 1)
+#define SC_CASES2(GM_, WM_, WN_) SC_CASE(GM_, WM_, WN_, 2, 3, 2) SC_CASE(GM_, WM_, WN_, 3, 3, 2)
+  SC_CASES2(4, 1, 2)   // (256 pixels of stride 2 are more than 1024 places: no such tiles)
+  SC_CASES2(2, 1, 1)
+  SC_CASE(2, 1, 1, 4, 3, 2)
   SC_CASES(4, 1, 2, 3)
   SC_CASES(2, 1, 2, 3)
   SC_CASES(2, 1, 1, 3)
@@ -546,6 +589,7 @@ int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, 
   SC_CASES(2, 1, 2, 5)
   SC_CASES(2, 1, 1, 5)
   SC_CASES(1, 1, 1, 5)
+#undef SC_CASES2
 #undef SC_CASES
 #undef SC_CASE
   sgh_prof_kernel_end(s);

@@ -861,7 +861,6 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
 
 // The same problem for the split kernel (conv_split.hip), where that one takes it
 inline bool fwd_as_split(const sgh_conv_geom *g, sgh_conv_geom *gt) {
-  if (g->stride_h != 1 || g->stride_w != 1) return false;
   *gt = *g;
   gt->C = g->K;
   gt->K = g->C;
@@ -869,6 +868,7 @@ inline bool fwd_as_split(const sgh_conv_geom *g, sgh_conv_geom *gt) {
 }
 
 inline bool dgrad_as_split(const sgh_conv_geom *g) {
+  if (g->stride_h != 1 || g->stride_w != 1) return false;
   const DgradPath path = dgrad_path(g);
   return path != kDgradFewC && path != kDgradPointwise && path != kDgradColumns && sgh_conv_split_supported(g);
 }

@@ -101,6 +101,34 @@ def test_conv_wgrad_octets_error_of_fp32_chains(singa, dev, n, c, h, w, k, kind)
     assert nl2(mine, want) < nl2(chain, want)   # (short chains: the rounding of the result is most of either error)
 
 
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive"])
+@pytest.mark.parametrize("n,c,h,w,k", [(1, 8, 7, 7, 64), (3, 20, 9, 12, 130), (30, 64, 14, 14, 64), (2, 40, 57, 43, 60), (70, 33, 8, 8, 300), (2, 64, 30, 62, 128)])
+def test_conv_split_forward_of_stride_two(singa, dev, n, c, h, w, k, kind):
+    """3x3 forward passes of stride 2 and padding 1: odd and even planes, tiles over many images, every tile size, against float64, no
+    further off than the fp32 chain; an infinity in x and one in a filter reach the results that they do in a zero-padded image."""
+    import torch
+    x, W, _ = operands(kind, n + c + h, n, c, h, w, k, 3)
+    b = randn(rng(k), k)
+    hd = singa.CudnnConvHandle(singa.from_numpy(x, dev), (3, 3), (2, 2), (1, 1), c, k, True)
+    run = lambda x, W: kernels_of(dev, lambda: singa.GpuConvForward(*(singa.from_numpy(a, dev) for a in (x, W, b)), hd).to_numpy())
+    conv = lambda x, W: (torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(W).double(), stride=2, padding=1)
+                         + torch.from_numpy(b).double()[:, None, None]).numpy()
+    got, names = run(x, W)
+    assert names == {"k_conv_split"}, names
+    m = min(n, 3)   # (the chain of a few images is as good as that of all)
+    want, chain = conv64(x[:m], W)
+    want, chain = want[:, :, ::2, ::2], chain[:, :, ::2, ::2]
+    off = got - conv(x, W)
+    assert nl2(got[:m] - b[:, None, None].astype(np.float64), want) <= 1.1 * nl2(chain, want) + 2.0 ** -24
+    assert np.all(np.abs(off) <= 2.0 ** -24 * (9 * c + 40) * (np.abs(want).max() + np.abs(b).max()))
+    x[n - 1, c - 1, h - 1, w // 2] = np.inf
+    W[k - 1, 0, 0, 2] = np.inf
+    got, want = run(x, W)[0], conv(x, W)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(np.isnan(got), np.isnan(want))
+    ok = np.isfinite(want)
+    assert np.all(np.abs(got[ok] - want[ok]) <= 2.0 ** -24 * (9 * c + 40) * (np.abs(want[ok]).max() + np.abs(b).max()))
+
+
 @pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan", "nan weights", "inf weights"])
 def test_conv_split_time_of_non_finite_operands(singa, dev, what):
     """Results that are not finite take a second pass over their tile on the fp32 instructions, 2.7 times the first one, and no search
