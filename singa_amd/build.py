@@ -19,7 +19,7 @@ SOURCES = [
     "runtime.hip", "eltwise.hip", "pool.hip", "batchnorm.hip", "igemm.hip", "wgrad3x3.hip", "conv16.hip",
     "wgrad_fewc.hip", "dgrad3x3.hip", "dgrad_fewc.hip", "half.hip", "tensor_fns.hip", "pointwise.hip",
     "fwd_fewc16.hip", "fwd_fewc.hip", "gemm16.hip", "bgrad.hip", "group_conv.hip", "gemm_split.hip", "pw16.hip", "conv_split.hip", "wgrad_oct.hip",
-    "wgrad_oct16.hip", "wgrad_pw16.hip", "fwd_few.hip", "dgrad_few.hip",
+    "wgrad_oct16.hip", "wgrad_pw16.hip", "fwd_few.hip", "dgrad_few.hip", "dgrad_split2.hip",
 ]
 
 # Packed-FP32 VALU ops are disabled for every device code object of this library.

@@ -534,17 +534,15 @@ size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g) {
 }
 
 int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps) {
-  const ScPlan p = plan(g);
-  const int pairs = p.nchunks * p.cblocks;
-  *cblocks = p.cblocks;
+  *cblocks = (g->C + 31) / 32;
+  const int pairs = (g->K + KC - 1) / KC * *cblocks;
   *taps = pairs >= sgh_num_cus() ? kSplitTaps : kSplitTapsFew;
-  return p.ok ? pairs * ((g->R * g->S + *taps - 1) / *taps) : 0;
+  return pairs * ((g->R * g->S + *taps - 1) / *taps);
 }
 
 int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspace, bool dgrad, hipStream_t s) {
   int cblocks, taps;
   const int blocks = sgh_conv_split_weight_blocks(g, &cblocks, &taps);
-  if (!blocks) return SGH_EUNSUPPORTED;
   hipLaunchKernelGGL(k_conv_split_weights, dim3(unsigned(blocks)), dim3(256), 0, s, W, static_cast<uint16_t *>(workspace), g->C,
                      g->K, g->R * g->S, cblocks, dgrad ? 1 : 0, taps);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;

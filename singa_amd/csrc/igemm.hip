@@ -26,6 +26,7 @@
 
 #include "common.h"
 #include "conv_split.h"
+#include "dgrad_split2.h"
 
 namespace {
 
@@ -867,10 +868,15 @@ inline bool fwd_as_split(const sgh_conv_geom *g, sgh_conv_geom *gt) {
   return sgh_conv_split_supported(gt);
 }
 
+// (stride 1: conv_split.hip, stride 2: dgrad_split2.hip)
 inline bool dgrad_as_split(const sgh_conv_geom *g) {
-  if (g->stride_h != 1 || g->stride_w != 1) return false;
   const DgradPath path = dgrad_path(g);
-  return path != kDgradFewC && path != kDgradPointwise && path != kDgradColumns && sgh_conv_split_supported(g);
+  if (path == kDgradFewC || path == kDgradPointwise || path == kDgradColumns) return false;
+  return g->stride_h == 1 && g->stride_w == 1 ? sgh_conv_split_supported(g) : sgh_dgrad_split2_supported(g);
+}
+
+inline size_t dgrad_split_bytes(const sgh_conv_geom *g) {
+  return g->stride_h == 1 ? sgh_conv_split_workspace_bytes(g) : sgh_dgrad_split2_workspace_bytes(g);
 }
 
 }  // namespace
@@ -1049,7 +1055,7 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   sgh_conv_geom gt;
   size_t split = 0;
   if (which == SGH_CONV_FWD && fwd_as_split(g, &gt)) split = sgh_conv_split_workspace_bytes(&gt);
-  if (which == SGH_CONV_DGRAD && dgrad_as_split(g)) split = sgh_conv_split_workspace_bytes(g);
+  if (which == SGH_CONV_DGRAD && dgrad_as_split(g)) split = dgrad_split_bytes(g);
   if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g);
   return split > plain ? split : plain;
 }
@@ -1069,7 +1075,7 @@ static size_t least_bytes_f32(const sgh_conv_geom *g, int which) {
 
 // Which of the two layouts of the weights a data gradient with this workspace works on
 static bool dgrad_splits(const sgh_conv_geom *g, size_t ws_bytes) {
-  return dgrad_as_split(g) && ws_bytes >= sgh_conv_split_workspace_bytes(g);
+  return dgrad_as_split(g) && ws_bytes >= dgrad_split_bytes(g);
 }
 
 // `prelaid`: the workspace already holds this layer's re-laid weights (sgh_conv_dgrad_prepare_multi)
@@ -1117,7 +1123,9 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
     }
   } else if (dgrad_splits(g, ws_bytes)) {
     if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
-    if (rc == SGH_OK) rc = sgh_conv_split_run(g, dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate);
+    if (rc == SGH_OK)
+      rc = g->stride_h == 1 ? sgh_conv_split_run(g, dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate)
+                            : sgh_dgrad_split2_run(g, dy, W, dx, workspace, s, accumulate);
   } else if (path == kDgradColumns && sgh_dgrad_few_supported(g)) {
     rc = sgh_dgrad_few_run(g, dy, W, dx, s);
   } else if (path == kDgradColumns) {

@@ -129,6 +129,84 @@ def test_conv_split_forward_of_stride_two(singa, dev, n, c, h, w, k, kind):
     assert np.all(np.abs(got[ok] - want[ok]) <= 2.0 ** -24 * (9 * c + 40) * (np.abs(want[ok]).max() + np.abs(b).max()))
 
 
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive"])
+@pytest.mark.parametrize("n,c,h,w,k", [(4, 64, 14, 14, 64), (2, 128, 9, 11, 130), (70, 33, 7, 8, 8), (1, 100, 58, 120, 72), (1, 100, 6, 256, 72),
+                                       (1, 64, 8, 219, 64), (44, 64, 56, 56, 48), (300, 200, 5, 3, 16)])
+def test_data_gradient_of_stride_two_on_split_operands(singa, dev, n, c, h, w, k, kind):
+    """3x3 data gradients of stride 2 and padding 1: odd and even planes, tiles over many images, either tile, whole and shared, every
+    slab, against float64 and no further off than the fp32 chain; onto a gradient that is there already, the sum of the two; an infinity
+    in dy and one in a filter reach the results that they do where a tap outside dy does not exist."""
+    import torch
+    x, W, _ = operands(kind, n + c + h, n, c, h, w, k, 3)
+    dy = operands(kind, n + k, n, k, (h + 1) // 2, (w + 1) // 2, 1, 1)[0]
+    there = randn(rng(c), n, c, h, w)
+    xd = singa.from_numpy(x, dev)
+    hd = singa.CudnnConvHandle(xd, (3, 3), (2, 2), (1, 1), c, k, False)
+    onto = lambda dy, W: singa.GpuConvBackwardxAccumulate(singa.from_numpy(dy, dev), singa.from_numpy(W, dev), xd, hd, singa.from_numpy(there, dev))
+    run = lambda dy, W: kernels_of(dev, lambda: singa.GpuConvBackwardx(singa.from_numpy(dy, dev), singa.from_numpy(W, dev), xd, hd).to_numpy())
+    grad = lambda dy, W: torch.nn.functional.conv_transpose2d(torch.from_numpy(dy).double(), torch.from_numpy(W).double(), stride=2, padding=1,
+                                                              output_padding=(1 - h % 2, 1 - w % 2)).numpy()
+    got, names = run(dy, W)
+    assert names == {"k_dgrad_split2"}, names
+    assert np.array_equal(onto(dy, W).to_numpy(), there + got)
+    m = min(n, 3)   # (the chain of a few images is as good as that of all)
+    apart = np.zeros((m, k, h, w), np.float32)
+    apart[:, :, ::2, ::2] = dy[:m]
+    want, chain = conv64(apart, np.ascontiguousarray(W.transpose(1, 0, 2, 3)[:, :, ::-1, ::-1]))
+    print(kind, "error %.2e, of a chain %.2e" % (nl2(got[:m], want), nl2(chain, want)))
+    assert nl2(got[:m], want) <= 1.1 * nl2(chain, want) + 2.0 ** -24   # (half an ulp of a result: one channel has one product)
+    bound = lambda want: 2.0 ** -24 * (4 * k + 40) * np.abs(want).max()   # (four taps at most, a rounding each of what is no larger)
+    assert np.all(np.abs(got - grad(dy, W)) <= bound(want) + 2.0 ** -24 * (4 * k + 40))
+    dy[n - 1, k - 1, -1, -1] = np.inf
+    W[k - 1, 0, 0, 2], W[0, c - 1, 0, 0] = np.inf, -np.inf
+    got, want = run(dy, W)[0], grad(dy, W)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.array_equal(np.isnan(got), np.isnan(want))
+    ok = np.isfinite(want)
+    assert np.all(np.abs(got[ok] - want[ok]) <= bound(want[ok]) + 2.0 ** -24 * (4 * k + 40))
+
+
+def test_data_gradient_of_stride_two_by_workspace_and_size(singa, dev):
+    """The split kernel runs where the workspace holds its partial tiles and where the reduction is worth the split; weights laid out for
+    a call with one size of workspace are not taken by a call with another."""
+    import ctypes as C
+
+    from singa_amd import _lib
+    lib = _lib.lib()
+    for (n, c, h, w, k), least in (((4, 64, 20, 22, 96), "k_dgrad3x3"), ((4, 64, 21, 22, 96), "k_igemm"), ((5, 131, 9, 11, 31), None), ((2, 64, 20, 22, 40), None)):
+        x, W, _ = operands("normal", 4, n, c, h, w, k, 3)
+        dy = randn(rng(5), n, k, (h + 1) // 2, (w + 1) // 2)
+        xd, wd, dyd, dxd = (singa.from_numpy(a, dev) for a in (x, W, dy, np.zeros_like(x)))
+        hd = singa.CudnnConvHandle(xd, (3, 3), (2, 2), (1, 1), c, k, False)
+        g = hd.geom
+        full = lib.sgh_conv_workspace_bytes(C.byref(g), _lib.SGH_CONV_DGRAD)
+        space = singa.from_numpy(np.zeros(full // 4 + 64, np.float32), dev)
+
+        def dgrad(size):
+            (rc, out), names = kernels_of(dev, lambda: (lib.sgh_conv_dgrad_f32(C.byref(g), dyd.ptr, wd.ptr, dxd.ptr, space.ptr, size, dev.stream),
+                                                        dxd.to_numpy()))
+            return (out, names) if rc == 0 else (None, rc)
+
+        def prepare(size):
+            item = (_lib.ConvPrepareItem * 1)()
+            item[0].g, item[0].W, item[0].workspace, item[0].ws_bytes = C.pointer(g), wd.ptr, space.ptr, size
+            assert lib.sgh_conv_dgrad_prepare_multi(item, 1, 0, dev.stream) == 0
+
+        if least is None:
+            assert dgrad(full)[1] in ({"k_dgrad3x3"}, {"k_igemm"})
+            continue
+        less = full
+        while dgrad(less)[1] == {"k_dgrad_split2"}:   # (a size that is too little for it and enough for the fp32 kernel)
+            less = less * 9 // 10
+        want = {size: dgrad(size) for size in (full, less)}
+        assert want[full][1] == {"k_dgrad_split2"} and want[less][1] == {least}, (want[less][1], least)
+        assert nl2(want[full][0], want[less][0]) < 1e-6
+        for prepared in (full, less):
+            for called in (full, less):
+                prepare(prepared)
+                got, names = dgrad(called)
+                assert names == want[called][1] and np.array_equal(got, want[called][0]), (prepared, called)
+
+
 @pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan", "nan weights", "inf weights"])
 def test_conv_split_time_of_non_finite_operands(singa, dev, what):
     """Results that are not finite take a second pass over their tile on the fp32 instructions, 2.7 times the first one, and no search
