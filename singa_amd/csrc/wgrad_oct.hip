@@ -1,4 +1,4 @@
-// fp32 weight gradient of 3x3 convolutions of stride 1 and padding 1 on the bfloat16 matrix instructions: three parts per value,
+// fp32 weight gradient of 3x3 convolutions of stride 1 or 2 and padding 1 on the bfloat16 matrix instructions: three parts per value,
 // six products (conv_split.hip says why that is fp32 arithmetic).
 //
 //   dW[k][c][r][s] = sum_{n,p,q} dy[n][k][p][q] * x[n][c][p + r - 1][q + s - 1]
@@ -13,6 +13,13 @@
 // rows (an image is its P rows and a row of zeros): per iteration RPI new rows of dy and of x are fetched into registers while
 // the previous ones are multiplied, then split and written; x rows live in a ring of RPI + 2.  Rows of OCS octets (one, two or
 // four): the columns beyond Q are zeros on both sides.
+//
+// Stride 2: the octet's columns 2 q + s - 1 of x are kept apart, the odd ones (s = 2 as they are, s = 0 shifted by one pixel) and the
+// even ones (s = 1), and two rows of x come in for one of dy.  That is four times the LDS per pixel, so the strips are half as wide and
+// an iteration half as long.  64 images, whole calls, k_wgrad3x3 and this: 64 channels of 56 x 56 to 128 95 -> 85 us, 128 of 28 x 28 to
+// 256 95 -> 85, 256 of 14 x 14 to 512 90 -> 89; what that kernel leaves to the generic one: 45 images of 224, 50 x 59, to 213
+// 542 -> 314, 17 of 109, 96 x 112, to 268 606 -> 298; 0.3 to 0.45 times the error.  (128 x 32 pairs, with iterations as long as at stride 1:
+// eleven registers spilled, 88 to 93 us.)
 //
 // The sums of the workgroups of a (k, c) tile are added in ascending order by k_wgrad_oct_reduce.
 //
@@ -37,58 +44,69 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
 struct WoArgs {
   const float *dy, *x;
   float *partial;   // [split][tile][wavefront][accumulator][lane]
-  int N, C, K, P, Q;
+  int N, C, K, P, Q, H, W;
   int ktiles, tiles, splits, strips, iters, per_split;   // iterations of a strip, of a workgroup
   unsigned dy_bytes, x_bytes;
 };
 
-// Eight elements of a tensor row as they come from memory
-struct Octet {
-  v4u raw[2];
+// E elements of a tensor row as they come from memory: eight, or the sixteen that an octet of dy meets at stride 2
+template <int E>
+struct Run {
+  v4u raw[E / 4];
   int nv;   // valid elements
   // elements [off, off + nv) of the tensor; nothing beyond its last byte is touched
   __device__ __forceinline__ void load(rsrc_t r, unsigned bytes, int off, int nv_) {
     nv = nv_;
     const int at = nv > 0 ? off * 4 : kOOB;
-    const bool tail = nv > 0 && unsigned(at) + 32 > bytes;
+    const bool tail = nv > 0 && unsigned(at) + E * 4 > bytes;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < E / 4; ++i)
       raw[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, tail ? kOOB : at, 16 * i, 0));
     if (__any(tail)) {
       if (tail) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) raw[j / 4][j % 4] = __builtin_amdgcn_raw_buffer_load_b32(r, j < nv ? at + 4 * j : kOOB, 0, 0);
+        for (int j = 0; j < E; ++j) raw[j / 4][j % 4] = __builtin_amdgcn_raw_buffer_load_b32(r, j < nv ? at + 4 * j : kOOB, 0, 0);
       }
     }
   }
-  __device__ __forceinline__ void parts(v4u (&out)[PARTS]) const {
+  // an octet from element `from` on, every E / 8
+  __device__ __forceinline__ void parts(v4u (&out)[PARTS], int from = 0) const {
+    constexpr int EVERY = E / 8;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const unsigned ua = raw[i / 2][2 * i % 4], ub = raw[i / 2][2 * i % 4 + 1];
-      const float a = 2 * i < nv ? __builtin_bit_cast(float, ua) : 0.f;
-      const float b = 2 * i + 1 < nv ? __builtin_bit_cast(float, ub) : 0.f;
+      const int ia = from + 2 * i * EVERY, ib = ia + EVERY;
+      const unsigned ua = raw[ia / 4][ia % 4], ub = raw[ib / 4][ib % 4];
+      const float a = ia < nv ? __builtin_bit_cast(float, ua) : 0.f;
+      const float b = ib < nv ? __builtin_bit_cast(float, ub) : 0.f;
       const Parts s = split2(a, b);
       out[0][i] = s.p[0], out[1][i] = s.p[1], out[2][i] = s.p[2];
     }
   }
 };
 
-template <int OCS, int RPI>
+template <int OCS, int RPI, int ST>
 struct Shape {
-  static constexpr int OPI = OCS * RPI, RING = RPI + 2;
-  static constexpr int XP = OCS == 4 ? 7 : OCS == 1 ? 3 : 5;   // 16-byte units of a channel's x row: the octets, a dword on either side, odd
+  static constexpr int OPI = OCS * RPI, RING = ST == 1 ? RPI + 2 : 2 * RPI + 1;
+  // 16-byte units of a channel's x row: the octets, a dword on either side, odd
+  // (stride 2: a dword, the octets of the odd columns, those of the even ones)
+  static constexpr int XP = ST == 2 ? 2 * OCS + 1 : OCS == 4 ? 7 : OCS == 1 ? 3 : 5;
   static constexpr int XPART = 64 * XP * 16, XROW = PARTS * XPART;
   static constexpr int DYO = (PARTS * 64 + 4) * 16;            // an octet of dy; four units of padding spread the writes over the banks
   static constexpr int GROUP = RING * XROW + OPI * DYO;
   static constexpr int LDS = 2 * GROUP > kAcc * 16 ? 2 * GROUP : kAcc * 16;
-  static_assert(OPI % 2 == 0 && LDS + 16 <= 160 * 1024, "");
+  static_assert(OPI * ST == 4 && LDS + 16 <= 160 * 1024, "");
 };
 
-template <int OCS, int RPI>
+template <int OCS, int RPI, int ST>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_wgrad_oct(WoArgs a) {
-  typedef Shape<OCS, RPI> S;
-  constexpr int OPI = S::OPI, RING = S::RING;
-  constexpr int TASKS = (OPI * 64 + GT - 1) / GT, EDGES = OCS >= 3 ? (RPI * 128 + GT - 1) / GT : 0;
+  typedef Shape<OCS, RPI, ST> S;
+  typedef Run<8> Octet;
+  typedef Run<8 * ST> XRun;
+  constexpr int OPI = S::OPI, RING = S::RING, XO = 4;
+  static_assert(ST * OPI == XO && XO * 64 == GT, "an octet of x, or a run of sixteen, per thread; of dy one for all or half of them");
+  // elements beside the strip: on either side, or (stride 2) on the left of twice as many rows
+  constexpr int EDGE = RPI * 128, EDGES = OCS >= 4 / ST ? 1 : 0;
+  static_assert(EDGES * EDGE <= GT, "");
   extern __shared__ __align__(16) char smem[];
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = wave >> 2, w4 = wave & 3, wm = w4 >> 1, wn = w4 & 1;
@@ -107,7 +125,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   const int first = split / a.strips * a.per_split, last = min(a.iters, first + a.per_split);
   const int mine = (a.per_split + 1) / 2;                    // iterations of a group (a last one may be empty)
   const int it0 = first + group * mine, it1 = min(last, it0 + mine);
-  const int VP = a.P + 1;
+  const int VP = a.P + 1, H = ST == 1 ? a.P : a.H, W = ST == 1 ? a.Q : a.W, VX = VP * ST;
   const rsrc_t rdy = make_rsrc(a.dy, a.dy_bytes), rx = make_rsrc(a.x, a.x_bytes);
 
   for (int i = tg; i < RING * S::XROW / 16; i += GT) reinterpret_cast<v4u *>(xs)[i] = v4u{0u, 0u, 0u, 0u};
@@ -119,18 +137,27 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   auto count = [&](int n, int p, int c, int channels, int q) {   // valid elements of the octet at column q
     return p < a.P && n >= 0 && n < a.N && c < channels ? max(0, min(8, a.Q - q)) : 0;
   };
-  auto put_x = [&](const Octet &o, int slot, int c, int oc) {
+  auto row_of_x = [&](int v, int &n, int &p) {
+    n = v < 0 ? -1 : v / VX, p = v < 0 ? H : v - n * VX;
+  };
+  auto count_x = [&](int n, int p, int c, int q) {
+    return p < H && n >= 0 && n < a.N && c < a.C ? max(0, min(8 * ST, W - q * ST)) : 0;
+  };
+  auto put_x = [&](const XRun &o, int slot, int c, int oc) {
     v4u part[PARTS];
-    o.parts(part);
 #pragma unroll
-    for (int i = 0; i < PARTS; ++i)
-      *reinterpret_cast<v4u *>(xs + slot * S::XROW + i * S::XPART + (c * S::XP + 1 + oc) * 16) = part[i];
+    for (int odd = ST - 1; odd >= 0; --odd) {
+      o.parts(part, odd);
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i)
+        *reinterpret_cast<v4u *>(xs + slot * S::XROW + i * S::XPART + (c * S::XP + 1 + oc + (ST == 2 && !odd ? OCS : 0)) * 16) = part[i];
+    }
   };
   // the element left (side 0) and right (side 1) of the strip
   auto edge_off = [&](int n, int p, int c, int side) {
-    const int q = side ? q0 + 8 * OCS : q0 - 1;
-    const bool ok = p < a.P && n >= 0 && n < a.N && c0 + c < a.C && q >= 0 && q < a.Q;
-    return ok ? (((n * a.C + c0 + c) * a.P + p) * a.Q + q) * 4 : kOOB;
+    const int q = side ? q0 + 8 * OCS : q0 * ST - 1;
+    const bool ok = p < H && n >= 0 && n < a.N && c0 + c < a.C && q >= 0 && q < W;
+    return ok ? (((n * a.C + c0 + c) * H + p) * W + q) * 4 : kOOB;
   };
   auto edge_get = [&](int off) -> unsigned { return __builtin_amdgcn_raw_buffer_load_b32(rx, off, 0, 0); };
   auto put_edge = [&](unsigned raw, int slot, int c, int side) {
@@ -141,36 +168,35 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       *reinterpret_cast<uint16_t *>(xs + slot * S::XROW + i * S::XPART + c * S::XP * 16 + (side ? 16 + OCS * 16 : 14)) = part[i];
   };
 
-  int dn[TASKS], dp[TASKS], xn[TASKS], xp[TASKS];   // (image, row) of this thread's next octets
-  int en[EDGES ? EDGES : 1], ep[EDGES ? EDGES : 1];
-#pragma unroll
-  for (int e = 0; e < TASKS; ++e) {
-    const int rr = (e * GT + tg) % OPI / OCS;
-    row_of(it0 * RPI + rr, dn[e], dp[e]);
-    row_of(it0 * RPI + 1 + rr, xn[e], xp[e]);
-  }
-#pragma unroll
-  for (int e = 0; e < EDGES; ++e) row_of(it0 * RPI + 1 + (e * GT + tg) / 128, en[e], ep[e]);
+  int dn, dp, xn, xp, en, ep;   // (image, row) of this thread's next octets and edge
+  const int v0 = it0 * RPI;
+  // this thread's element of the edges: its row among the new ones, channel, side
+  const int edge_row = ST == 1 ? tg >> 7 : tg >> 6, edge_channel = ST == 1 ? tg >> 1 & 63 : tg & 63, edge_side = ST == 1 ? tg & 1 : 0;
+  const int first_x = ST == 1 ? v0 + 1 : 2 * v0;
+  row_of(v0 + tg % OPI / OCS, dn, dp);
+  row_of_x(first_x + tg % XO / OCS, xn, xp);
+  row_of_x(first_x + edge_row, en, ep);
 
-  Octet sd[TASKS], sx[TASKS];
-  unsigned se[EDGES ? EDGES : 1];
+  Octet sd;
+  XRun sx;
+  unsigned se;
   auto step_row = [&](int &n, int &p) {
     p += RPI;
     if (p >= VP) p -= VP, ++n;
   };
-  auto load = [&]() {   // dy rows [v0, v0 + RPI) and x rows [v0 + 1, v0 + RPI] of an iteration, then on to the next one
-#pragma unroll
-    for (int e = 0; e < TASKS; ++e) {
-      const int i = e * GT + tg, o = i % OPI, ch = i / OPI, q = q0 + o % OCS * 8;
-      sd[e].load(rdy, a.dy_bytes, ((dn[e] * a.K + k0 + ch) * a.P + dp[e]) * a.Q + q, ch < 64 ? count(dn[e], dp[e], k0 + ch, a.K, q) : 0);
-      sx[e].load(rx, a.x_bytes, ((xn[e] * a.C + c0 + ch) * a.P + xp[e]) * a.Q + q, ch < 64 ? count(xn[e], xp[e], c0 + ch, a.C, q) : 0);
-      step_row(dn[e], dp[e]), step_row(xn[e], xp[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < EDGES; ++e) {
-      const int i = e * GT + tg;
-      se[e] = edge_get(edge_off(en[e], ep[e], i >> 1 & 63, i & 1));
-      step_row(en[e], ep[e]);
+  auto step_row_x = [&](int &n, int &p) {
+    p += RPI * ST;
+    if (p >= VX) p -= VX, ++n;
+  };
+  // dy rows [v0, v0 + RPI) and x rows [v0 + 1, v0 + RPI], or [2 v0, 2 (v0 + RPI)), of an iteration, then on to the next one
+  auto load = [&]() {
+    const int k = tg / OPI, c = tg / XO, q = q0 + tg % OCS * 8;
+    sd.load(rdy, a.dy_bytes, ((dn * a.K + k0 + k) * a.P + dp) * a.Q + q, k < 64 ? count(dn, dp, k0 + k, a.K, q) : 0);
+    sx.load(rx, a.x_bytes, ((xn * a.C + c0 + c) * H + xp) * W + q * ST, count_x(xn, xp, c0 + c, q));
+    step_row(dn, dp), step_row_x(xn, xp);
+    if (EDGES) {
+      se = edge_get(edge_off(en, ep, edge_channel, edge_side));
+      step_row_x(en, ep);
     }
   };
   // Every other step's dy is negated, and the other ones in the second group, and what they give is subtracted: the matrix
@@ -178,23 +204,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   // 2e-7 of the mean magnitude with one sign, 2e-8 with two)
   const unsigned sign = group ? 0x80008000u : 0u;
   auto slot_of = [](int base, int j) { return base + j < RING ? base + j : base + j - RING; };
-  auto stage = [&](int base) {   // base: the ring slot of row v0 - 1
+  auto stage = [&](int base) {   // base: the ring slot of row v0 - 1, or 2 v0 - 1
+    const int o = tg % OPI, k = tg / OPI;
+    v4u part[PARTS];
+    sd.parts(part);
+    if (ST == 1 || k < 64) {
 #pragma unroll
-    for (int e = 0; e < TASKS; ++e) {
-      const int i = e * GT + tg, o = i % OPI, ch = i / OPI;
-      v4u part[PARTS];
-      sd[e].parts(part);
-      if (OPI * 64 % GT == 0 || ch < 64) {
-#pragma unroll
-        for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + ch) * 16) = part[j] ^ (o & 2 ? ~sign & 0x80008000u : sign);
-        put_x(sx[e], slot_of(base, 2 + o / OCS), ch, o % OCS);
-      }
+      for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + k) * 16) = part[j] ^ (o & 2 ? ~sign & 0x80008000u : sign);
     }
-#pragma unroll
-    for (int e = 0; e < EDGES; ++e) {
-      const int i = e * GT + tg;
-      if (RPI * 128 % GT == 0 || i < RPI * 128) put_edge(se[e], slot_of(base, 2 + i / 128), i >> 1 & 63, i & 1);
-    }
+    put_x(sx, slot_of(base, 3 - ST + tg % XO / OCS), tg / XO, tg % OCS);
+    if (EDGES && (EDGE % GT == 0 || tg < EDGE)) put_edge(se, slot_of(base, 3 - ST + edge_row), edge_channel, edge_side);
   };
 
   v16f acc[9];
@@ -203,22 +222,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
 
-  // rows v0 - 1 and v0, then the first iteration's own
-  int base = it0 * RPI % RING;
+  // rows v0 - 1 and v0, or row 2 v0 - 1, then the first iteration's own
+  constexpr int AHEAD = 3 - ST;
+  int base = v0 % RING;
   __syncthreads();   // (the zeros are in place)
-  for (int i = tg; i < 2 * OCS * 64; i += GT) {
+  for (int i = tg; i < AHEAD * OCS * 64; i += GT) {
     const int oc = i % OCS, c = i / OCS & 63, j = i / (OCS * 64), q = q0 + oc * 8;
     int n, p;
-    row_of(it0 * RPI - 1 + j, n, p);
-    Octet o;
-    o.load(rx, a.x_bytes, ((n * a.C + c0 + c) * a.P + p) * a.Q + q, count(n, p, c0 + c, a.C, q));
+    row_of_x(v0 * ST - 1 + j, n, p);
+    XRun o;
+    o.load(rx, a.x_bytes, ((n * a.C + c0 + c) * H + p) * W + q * ST, count_x(n, p, c0 + c, q));
     put_x(o, slot_of(base, j), c, oc);
   }
-  if (EDGES) {
-    const int j = tg >> 7, c = tg >> 1 & 63;
+  if (EDGES && edge_row < AHEAD) {
     int n, p;
-    row_of(it0 * RPI - 1 + j, n, p);
-    put_edge(edge_get(edge_off(n, p, c, tg & 1)), slot_of(base, j), c, tg & 1);
+    row_of_x(v0 * ST - 1 + edge_row, n, p);
+    put_edge(edge_get(edge_off(n, p, edge_channel, edge_side)), slot_of(base, edge_row), edge_channel, edge_side);
   }
   load();
   stage(base);
@@ -231,7 +250,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     if (more) load();
     if (it0 + i < it1) {
       struct Raw {
-        v4u d;
+        v4u d, e;        // (stride 2: of the odd columns and of the even ones)
         unsigned l, r;
       };
       // unit u = (step, row r of the filter): the three parts of the octet and its neighbours, three taps.  A tap's six products
@@ -240,13 +259,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       constexpr int UNITS = OPI / 2 * 3;
       auto read = [&](int u, int p) {
         const int s = u / 3, r = u % 3, oa = 2 * s, ob = 2 * s + 1;
-        const int ja = slot_of(base, oa / OCS + r) * S::XROW + oa % OCS * 16;
-        const int jb = slot_of(base, ob / OCS + r) * S::XROW + ob % OCS * 16;
+        const int ja = slot_of(base, oa / OCS * ST + r) * S::XROW + oa % OCS * 16;
+        const int jb = slot_of(base, ob / OCS * ST + r) * S::XROW + ob % OCS * 16;
         const char *at = xb + (half ? jb : ja) + p * S::XPART;
         Raw w;
         w.l = *reinterpret_cast<const unsigned *>(at);
         w.d = *reinterpret_cast<const v4u *>(at + 4);
-        w.r = *reinterpret_cast<const unsigned *>(at + 20);
+        if (ST == 1) w.r = *reinterpret_cast<const unsigned *>(at + 20);
+        else w.e = *reinterpret_cast<const v4u *>(at + 4 + OCS * 16);
         return w;
       };
       v4u A[PARTS];
@@ -269,8 +289,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
           for (int p = PARTS - 1; p >= 0; --p) {
             const v4u d = w[p].d;
-            v4u x = d;
-            if (c != 1) {
+            v4u x = ST == 2 && c == 1 ? w[p].e : d;   // (stride 2: columns 2 q - 1, 2 q, 2 q + 1)
+            if (ST == 1 ? c != 1 : c == 0) {
               const unsigned m1 = __builtin_amdgcn_alignbit(d[1], d[0], 16), m2 = __builtin_amdgcn_alignbit(d[2], d[1], 16),
                              m3 = __builtin_amdgcn_alignbit(d[3], d[2], 16);
               if (c == 0) x = v4u{__builtin_amdgcn_alignbit(d[0], w[p].l, 16), m1, m2, m3};
@@ -290,7 +310,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
     __syncthreads();
     if (more) {
-      base = slot_of(base, RPI);
+      base = slot_of(base, RPI * ST);
       stage(base);
       __syncthreads();
     }
@@ -311,10 +331,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   if (__any(bad) && lane == 0) *again = 1;
   __syncthreads();
   if (*again) {
-    constexpr int COLS = 8 * OCS, YP = COLS + 1, XW = COLS + 2, XF = COLS + 3;   // odd pitches
+    constexpr int COLS = 8 * OCS, YP = COLS + 1, XW = ST == 1 ? COLS + 2 : 2 * COLS + 1, XF = XW | 1;   // odd pitches
     static_assert((64 * YP + 192 * XF) * 4 <= S::GROUP, "");
-    int tt = threadIdx.x, P = a.P, Q = a.Q;
-    asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q));
+    int tt = threadIdx.x, P = a.P, Q = a.Q, H = ST == 1 ? P : a.H, W = ST == 1 ? Q : a.W;
+    asm volatile("" : "+v"(tt), "+s"(P), "+s"(Q), "+s"(H), "+s"(W));
     const int th = tt >> 5 & 1, row = wm * 32 + (tt & 31), col = wn * 32 + (tt & 31);
     float *const ys = reinterpret_cast<float *>(smem + group * S::GROUP), *const xr = ys + 64 * YP;
     unsigned valid = 0;   // accumulator registers that hold a filter
@@ -339,9 +359,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           ys[ch * YP + q] = k0 + ch < a.K && q0 + q < Q ? a.dy[((n * a.K + k0 + ch) * P + p) * Q + q0 + q] : 0.f;
         }
         for (int e = tt & (GT - 1); e < 192 * XW; e += GT) {
-          const int ch = e / XW % 64, h = p + e / (XW * 64) - 1, w = q0 + e % XW - 1;
-          const bool in = c0 + ch < a.C && unsigned(h) < unsigned(P) && unsigned(w) < unsigned(Q);
-          xr[e / XW * XF + e % XW] = in ? a.x[((n * a.C + c0 + ch) * P + h) * Q + w] : 0.f;
+          const int ch = e / XW % 64, h = p * ST + e / (XW * 64) - 1, w = q0 * ST + e % XW - 1;
+          const bool in = c0 + ch < a.C && unsigned(h) < unsigned(H) && unsigned(w) < unsigned(W);
+          xr[e / XW * XF + e % XW] = in ? a.x[((n * a.C + c0 + ch) * H + h) * W + w] : 0.f;
         }
       }
       __syncthreads();
@@ -354,7 +374,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           for (int r = 0; r < 3; ++r)
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-              const float xv = xr[(r * 64 + col) * XF + u + th + c];
+              const float xv = xr[(r * 64 + col) * XF + (u + th) * ST + c];
               acc[r * 3 + c] = __builtin_amdgcn_mfma_f32_32x32x2f32(d, in ? xv : 0.f, acc[r * 3 + c], 0, 0, 0);
             }
         }
@@ -430,23 +450,25 @@ __global__ __launch_bounds__(576) void k_wgrad_oct_reduce(WoArgs a, float *__res
 
 struct WoPlan {
   bool ok;
-  int ocs, rpi, ktiles, tiles, splits, strips, iters, per_split;
+  int st, ocs, rpi, ktiles, tiles, splits, strips, iters, per_split;
 };
 
 WoPlan plan(const sgh_conv_geom *g) {
   WoPlan p{};
-  if (g->R != 3 || g->S != 3 || g->stride_h != 1 || g->stride_w != 1 || g->pad_h != 1 || g->pad_w != 1) return p;
+  p.st = g->stride_h;
+  if (g->R != 3 || g->S != 3 || p.st < 1 || p.st > 2 || g->stride_w != p.st || g->pad_h != 1 || g->pad_w != 1) return p;
+  if (g->P != (g->H + p.st - 1) / p.st || g->Q != (g->W + p.st - 1) / p.st) return p;
   const size_t pixels = size_t(g->N) * g->P * g->Q, lim = size_t(1) << 29;
-  if (pixels * g->C >= lim || pixels * g->K >= lim) return p;
+  if (size_t(g->N) * g->H * g->W * g->C >= lim || pixels * g->K >= lim) return p;
   // Few channels leave the 64 columns of a tile empty (their nine taps are columns to the fp32 kernels: 3, 11 and 25 of 64
   // channels 0.6 times as fast, 39 and more 1.1 to 2.4 times).  Below 0.7 G products a launch is short beside its partial images:
   // 0.13 to 0.67 G, 55 layers, 0.9 to 1.5 times as fast, and the rule that would tell those apart is not there.
   if (20 * g->C < 11 * 64 * ((g->C + 63) / 64) || double(pixels) * g->K * g->C * 9 < 7e8) return p;
-  const int oc = (g->Q + 7) / 8;
-  p.strips = (oc + 3) / 4;
+  const int oc = (g->Q + 7) / 8, widest = 4 / p.st;   // (stride 2: twice the columns of x)
+  p.strips = (oc + widest - 1) / widest;
   p.ocs = (oc + p.strips - 1) / p.strips;
   if (p.ocs == 3) p.ocs = 4;   // (two rows of three octets do not fit the registers: 64 images, 96 channels of 20 x 22 109 against 102 us)
-  p.rpi = p.ocs == 4 ? 1 : p.ocs == 1 ? 4 : 2;
+  p.rpi = widest / p.ocs;
   if (g->P + 1 < p.rpi || size_t(g->N) * (g->P + 1) >= (size_t(1) << 30)) return p;
   p.iters = int((size_t(g->N) * (g->P + 1) + p.rpi - 1) / p.rpi);
   p.ktiles = (g->K + 63) / 64;
@@ -465,9 +487,9 @@ WoPlan plan(const sgh_conv_geom *g) {
   return p;
 }
 
-template <int OCS, int RPI>
+template <int OCS, int RPI, int ST>
 int launch(const WoArgs &a, hipStream_t s) {
-  auto kern = k_wgrad_oct<OCS, RPI>;
+  auto kern = k_wgrad_oct<OCS, RPI, ST>;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
@@ -475,7 +497,7 @@ int launch(const WoArgs &a, hipStream_t s) {
       return SGH_EUNSUPPORTED;
     attr_set = true;
   }
-  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.splits)), dim3(NT), (Shape<OCS, RPI>::LDS + 16), s, a);
+  SGH_LAUNCH_TIMED(kern, dim3(unsigned(a.tiles * a.splits)), dim3(NT), (Shape<OCS, RPI, ST>::LDS + 16), s, a);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 
@@ -491,14 +513,14 @@ int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, f
   if (!p.ok) return SGH_EUNSUPPORTED;
   WoArgs a;
   a.dy = dy, a.x = x, a.partial = static_cast<float *>(workspace);
-  a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
+  a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q, a.H = g->H, a.W = g->W;
   a.ktiles = p.ktiles, a.tiles = p.tiles, a.splits = p.splits, a.strips = p.strips, a.iters = p.iters, a.per_split = p.per_split;
   const size_t pixels = size_t(g->N) * g->P * g->Q;
-  a.dy_bytes = unsigned(pixels * g->K * 4), a.x_bytes = unsigned(pixels * g->C * 4);
+  a.dy_bytes = unsigned(pixels * g->K * 4), a.x_bytes = unsigned(size_t(g->N) * g->H * g->W * g->C * 4);
   sgh_prof_kernel_begin("conv_wgrad/k_wgrad_oct", 2.0 * pixels * g->K * g->C * 9);
-  const int rc = p.ocs == 4   ? launch<4, 1>(a, s)
-                 : p.ocs == 2 ? launch<2, 2>(a, s)
-                              : launch<1, 4>(a, s);
+  const int rc = p.ocs == 4   ? launch<4, 1, 1>(a, s)
+                 : p.ocs == 2 ? (p.st == 1 ? launch<2, 2, 1>(a, s) : launch<2, 1, 2>(a, s))
+                              : (p.st == 1 ? launch<1, 4, 1>(a, s) : launch<1, 2, 2>(a, s));
   sgh_prof_kernel_end(s);
   if (rc != SGH_OK) return rc;
   // (threads per accumulator: as many as leave each a few images)

@@ -311,6 +311,42 @@ def test_conv_wgrad_octets_infinities_and_nans(singa, dev, n, c, h, w, k):
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("n,c,h,w,k", [(30, 256, 14, 13, 256), (40, 150, 22, 31, 96), (20, 100, 41, 40, 260), (8, 128, 50, 57, 140), (6, 62, 97, 120, 80)])
+def test_weight_gradient_of_stride_two_by_octets(singa, dev, n, c, h, w, k):
+    """3x3 weight gradients of stride 2 and padding 1, one strip and several, odd and even planes, against float64: within terms * 2^-23 of
+    the sum of the terms' magnitudes, and closer than a sixteenth of the roundings of chains of fp32 additions (0.5 * sqrt(terms) * 2^-24, and
+    the rounding of the result); infinities and NaNs reach the weights that their products reach, those with the padding among them."""
+    import torch
+    x, W, _ = operands("normal", n + c + k, n, c, h, w, k, 3)
+    P, Q = (h + 1) // 2, (w + 1) // 2
+    dy = randn(rng(n), n, k, P, Q)
+    terms = n * P * Q
+    hd = singa.CudnnConvHandle(singa.from_numpy(x, dev), (3, 3), (2, 2), (1, 1), c, k, False)
+    run = lambda x, dy: kernels_of(dev, lambda: singa.GpuConvBackwardW(*(singa.from_numpy(a, dev) for a in (dy, x, W)), hd).to_numpy())
+
+    def grad(x, dy):
+        xp = torch.nn.functional.pad(torch.from_numpy(x).double(), (1, 2, 1, 2))
+        d = torch.from_numpy(dy).double().permute(1, 0, 2, 3).reshape(k, -1).contiguous()
+        taps = [d @ xp[:, :, i:i + 2 * P:2, j:j + 2 * Q:2].permute(0, 2, 3, 1).reshape(-1, c) for i in range(3) for j in range(3)]
+        return torch.stack(taps, -1).reshape(k, c, 3, 3).numpy()
+
+    got, names = run(x, dy)
+    assert names == {"k_wgrad_oct"}, names
+    want = grad(x, dy)
+    assert np.all(np.abs(got - want) <= terms * 2.0 ** -23 * grad(np.abs(x), np.abs(dy)))
+    assert nl2(got, want) < (0.5 * terms ** 0.5 + 1) * 2.0 ** -24
+    assert np.array_equal(run(x, dy)[0], got)
+    x[n // 2, 5, h - 1, w - 1], x[1, 6, 0, 0], x[2, 7, h // 2, 1], x[0, c - 1, 0, w - 1] = -np.inf, np.inf, np.nan, np.inf
+    dy[n - 1, k - 1, P - 1, 4], dy[0, 3, 1, Q - 1], dy[3, 4, 2, 2] = np.inf, -np.inf, np.nan
+    got = run(x, dy)[0]
+    with np.errstate(all="ignore"):
+        want = grad(x, dy).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan"])
 def test_conv_wgrad_octets_time_of_non_finite_operands(singa, dev, what):
     """As the forward pass and the data gradient: no search per result."""
