@@ -28,13 +28,13 @@
 // position][part][8 channels]: 48 bytes per position, one operand fragment of a tap is three ds_read_b128 at an offset that
 // is the tap's alone.  A value is fetched and split once per chunk for all R * R taps.  Rows are addressed in a "virtual row"
 // space in which every image owns P + 2 o rows, so a tile may straddle images and the padding is materialised as zeros.
-// The weights are split and laid out in fragment order by a kernel of their own and go from L2 straight to registers, two
-// taps ahead: no LDS, no barrier per tap.
+// The weights are split and laid out in fragment order by a kernel of their own and go from L2 straight to registers, a tap or two
+// ahead: no LDS, no barrier per tap.
 //
 // 512 threads = 8 wavefronts of at most 128 registers, two workgroups per CU where the slab takes no more than 80 KB of LDS: while
 // one stages and waits at its barriers the other one's matrix instructions run.
 //
-// Stride 2, whole forward calls, the generic kernel (igemm.hip) and here: 64 images of 64 channels, 56 x 56, to 128 125 -> 103 us, of 128,
+// Stride 2, whole forward calls, the generic kernel (igemm.hip) and here: 64 images of 64 channels, 56 x 56, to 128 125 -> 99 us, of 128,
 // 28 x 28, to 256 163 -> 69, of 256, 14 x 14, to 512 169 -> 77; 13 of 256, 10 x 10, to 512 108 -> 33 (48 workgroups before); the error
 // 0.12 to 0.35 times, and over 34 drawn layers none slower than 0.97.  The tiles are the ones of stride 1; a wavefront of two blocks with
 // three slab elements a thread, ten registers spilled, is faster than one block (28 x 28: 69 / 75, 14 x 14: 77 / 92).
@@ -117,7 +117,9 @@ __device__ __forceinline__ int place_of(int column, int pitch) {
 template <int GM, int WM, int WN, int ET, int R, int ST>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_split(ScArgs a) {
   constexpr int GN = NW / GM, BM = GM * WM * 32, BN = GN * WN * 32, TAPS = R * R, O = (R - 1) / 2;
-  constexpr int AD = 2;                       // weight fragments: this tap's and the next one's
+  // Weight fragments: this tap's and the next one's, or the next two's where a wavefront has six products per tap and not twelve to cover
+  // the loads (5x5 onto 64 channels, 128 images of 16 x 16: 29.3 -> 26.8 us, onto 32 35.2 -> 33.4; 64 channels, 8 x 56 x 56: 25.4 -> 23.6)
+  constexpr int AD = WN == 1 ? 3 : 2;
   constexpr int EARLY = WN > 1 && ET > 3 ? 3 : ET;   // elements requested under the products (registers); the others after them
   extern __shared__ __align__(16) char smem[];
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31;
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     for (int k = 0; k < 3; ++k) b[k] = *reinterpret_cast<const v4u *>(p + k * 16);
   };
 
-  // Everything a tap needs is requested before the matrix instructions of an earlier one: weights two taps ahead, the next
+  // Everything a tap needs is requested before the matrix instructions of an earlier one: weights AD - 1 taps ahead, the next
   // chunk's slab an element per tap, a block's fragment while the other block is multiplied.  (The scheduling barriers keep
   // the compiler from moving the requests down to their uses, which it does to save registers.)
 #pragma unroll
