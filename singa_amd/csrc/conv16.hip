@@ -931,7 +931,12 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
   const int brow = (wp * TP * 32 + l32 + a.Wp + 1) * PITCH + half * 32 + lh * 8;
   // step = 9 * kc + tap; PAR = step & 1 names the weight tile buffer in LDS that the step reads and the
   // register set that it loads
-  auto step = [&](int kc, auto tapc, auto parc) {
+  // (`tail`: the last chunk holds channels beyond K; of this group's matrix steps only the first `left` are not all zeros.  37 images
+  // of 31 x 45, 72 and 136 channels: forward and data gradient 75 -> 69 us together.  A layer of one chunk keeps them all: with a second
+  // copy of its loop it takes 168 registers instead of 116)
+  const int left = max(0, (a.K - (nkc - 1) * KC - half * 32 + 15) / 16);
+  auto step = [&](int kc, auto tapc, auto parc, auto tailc) {
+    constexpr bool TAIL = decltype(tailc)::value;
     constexpr int TAP = decltype(tapc)::value, PAR = decltype(parc)::value, R_ = TAP / 3, S_ = TAP % 3;
     const uint16_t *const slab = (MULTI && (kc & 1)) ? slab1 : slab0;
     uint16_t *const slab_next = (MULTI && (kc & 1)) ? slab0 : slab1;
@@ -941,6 +946,7 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
     const uint16_t *Bs = slab + brow + ((1 - R_) * a.Wp + (1 - S_)) * PITCH;
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
+      if (TAIL && j >= left) break;
       u32x4 av[TC], bv[TP];
 #pragma unroll
       for (int i = 0; i < TC; ++i) av[i] = *reinterpret_cast<const u32x4 *>(As + i * 32 * PITCH + 16 * j);
@@ -956,24 +962,29 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
     if (MULTI && TAP == 8) stage_pixels(slab_next, EV / 2, EV / 2);
     __syncthreads();
   };
-  auto chunk = [&](int kc, auto parc) {
+  auto chunk = [&](int kc, auto parc, auto tail) {
     constexpr int P = decltype(parc)::value;
     typedef std::integral_constant<int, P> P0;
     typedef std::integral_constant<int, P ^ 1> P1;
-    step(kc, std::integral_constant<int, 0>{}, P0{});
-    step(kc, std::integral_constant<int, 1>{}, P1{});
-    step(kc, std::integral_constant<int, 2>{}, P0{});
-    step(kc, std::integral_constant<int, 3>{}, P1{});
-    step(kc, std::integral_constant<int, 4>{}, P0{});
-    step(kc, std::integral_constant<int, 5>{}, P1{});
-    step(kc, std::integral_constant<int, 6>{}, P0{});
-    step(kc, std::integral_constant<int, 7>{}, P1{});
-    step(kc, std::integral_constant<int, 8>{}, P0{});
+    step(kc, std::integral_constant<int, 0>{}, P0{}, tail);
+    step(kc, std::integral_constant<int, 1>{}, P1{}, tail);
+    step(kc, std::integral_constant<int, 2>{}, P0{}, tail);
+    step(kc, std::integral_constant<int, 3>{}, P1{}, tail);
+    step(kc, std::integral_constant<int, 4>{}, P0{}, tail);
+    step(kc, std::integral_constant<int, 5>{}, P1{}, tail);
+    step(kc, std::integral_constant<int, 6>{}, P0{}, tail);
+    step(kc, std::integral_constant<int, 7>{}, P1{}, tail);
+    step(kc, std::integral_constant<int, 8>{}, P0{}, tail);
   };
-  for (int kc = 0; kc < nkc; kc += 2) {
-    chunk(kc, std::integral_constant<int, 0>{});
-    if (!MULTI || kc + 1 >= nkc) break;
-    chunk(kc + 1, std::integral_constant<int, 1>{});
+  const int nfull = MULTI && left < KS ? nkc - 1 : nkc;
+  for (int kc = 0; kc < nfull; kc += 2) {
+    chunk(kc, std::integral_constant<int, 0>{}, std::false_type{});
+    if (!MULTI || kc + 1 >= nfull) break;
+    chunk(kc + 1, std::integral_constant<int, 1>{}, std::false_type{});
+  }
+  if (MULTI && nfull < nkc) {
+    if (nfull & 1) chunk(nfull, std::integral_constant<int, 1>{}, std::true_type{});
+    else chunk(nfull, std::integral_constant<int, 0>{}, std::true_type{});
   }
 
   // SPLIT: the two groups' sums meet in LDS, one channel block at a time: a wavefront hands over the position

@@ -1054,6 +1054,33 @@ def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
             assert nl2(got[part], want[part]) < bound
 
 
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("K", [80, 88, 104, 112, 120, 144, 160, 184])
+@pytest.mark.parametrize("N,C,H,W", [(3, 64, 9, 14), (60, 72, 28, 30)])
+def test_conv_3x3_16bit_partial_last_chunk(singa, dev, kind, K, N, C, H, W):
+    """A reduction whose last chunk of 64 channels is partly empty: the matrix steps that would multiply only zeros are left out, so
+    the results have the bits that they have with those channels there and zero; a forward pass and a data gradient."""
+    r = rng(K + C)
+    full = (K + 63) // 64 * 64
+    pad = lambda a, axis: np.concatenate([a, np.zeros(a.shape[:axis] + (full - K,) + a.shape[axis + 1:], np.float32)], axis)
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, C, 3, 3)) * 0.05).astype(np.float32)
+    dy = r.standard_normal((N, K, H, W)).astype(np.float32)
+
+    def dgrad(w, dy):
+        k = len(w)
+        xt, wt, dyt = (_to(singa, dev, a, kind)[0] for a in (x, w, dy))
+        return singa.GpuConvBackwardx(dyt, wt, xt, singa.CudnnConvHandle(xt, (3, 3), (1, 1), (1, 1), C, k, False)).to_numpy()
+
+    def forward(w, dy):   # (the reduction over dy's channels)
+        k = len(w)
+        dyt, wt = (_to(singa, dev, a, kind)[0] for a in (dy, np.ascontiguousarray(w.transpose(1, 0, 2, 3))))
+        return singa.GpuConvForward(dyt, wt, None, singa.CudnnConvHandle(dyt, (3, 3), (1, 1), (1, 1), k, C, False)).to_numpy()
+
+    for f in (dgrad, forward):
+        _same_bits(f(w, dy), f(pad(w, 0), pad(dy, 1)), f.__name__)
+
+
 # layers that the octet weight gradient (wgrad_oct16.hip) takes: rows of one to four octets and of several strips, whole and ragged
 # octets and channels, odd and even planes of stride 2, rows that do not divide the iterations; and three that it does not take (50 x 512 x 7 x 7, 3 x 65 and 5 x 100)
 WGRAD_OCTET16_CASES = [
