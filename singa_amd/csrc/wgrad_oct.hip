@@ -201,16 +201,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   };
   // Every other step's dy is negated, and the other ones in the second group, and what they give is subtracted: the matrix
   // instructions round towards minus infinity on average, which adds up over a sum (1024 channels of 14 x 14, forward pass:
-  // 2e-7 of the mean magnitude with one sign, 2e-8 with two)
-  const unsigned sign = group ? 0x80008000u : 0u;
+  // 2e-7 of the mean magnitude with one sign, 2e-8 with two).  Stride 2, where an iteration is one step: every other iteration's, and
+  // the other way round in every other split, which often is the same rows of another image (64 images, 64 channels of 56 x 56 to 128:
+  // the groups alone left 4.0e-8)
+  const bool turned = (group != 0) != (ST == 2 && (split / a.strips & 1));
+  const unsigned sign = turned ? 0x80008000u : 0u;
   auto slot_of = [](int base, int j) { return base + j < RING ? base + j : base + j - RING; };
-  auto stage = [&](int base) {   // base: the ring slot of row v0 - 1, or 2 v0 - 1
+  auto stage = [&](int base, int i) {   // of iteration i; base: the ring slot of row v0 - 1, or 2 v0 - 1
     const int o = tg % OPI, k = tg / OPI;
     v4u part[PARTS];
     sd.parts(part);
     if (ST == 1 || k < 64) {
 #pragma unroll
-      for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + k) * 16) = part[j] ^ (o & 2 ? ~sign & 0x80008000u : sign);
+      for (int j = 0; j < PARTS; ++j) *reinterpret_cast<v4u *>(dys + o * S::DYO + (j * 64 + k) * 16) = part[j] ^ ((ST == 1 ? o & 2 : i & 1) ? ~sign & 0x80008000u : sign);
     }
     put_x(sx, slot_of(base, 3 - ST + tg % XO / OCS), tg / XO, tg % OCS);
     if (EDGES && (EDGE % GT == 0 || tg < EDGE)) put_edge(se, slot_of(base, 3 - ST + edge_row), edge_channel, edge_side);
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     put_edge(edge_get(edge_off(n, p, edge_channel, edge_side)), slot_of(base, edge_row), edge_channel, edge_side);
   }
   load();
-  stage(base);
+  stage(base, 0);
   __syncthreads();
 
   const char *const da = dys + half * S::DYO + (wm * 32 + l32) * 16;
@@ -249,6 +252,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const bool more = i + 1 < mine;
     if (more) load();
     if (it0 + i < it1) {
+      [[maybe_unused]] const float turn = i & 1 ? -1.f : 1.f;
       struct Raw {
         v4u d, e;        // (stride 2: of the odd columns and of the even ones)
         unsigned l, r;
@@ -302,7 +306,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           }
           if (r == 2 && c == 2 && s + 1 < OPI / 2) read_a(s + 1);
           v16f &total = acc[r * 3 + c];
-          total = s % 2 ? total - sum : total + sum;
+          if constexpr (ST == 1) total = s % 2 ? total - sum : total + sum;
+          else
+#pragma unroll
+            for (int v = 0; v < 16; ++v) total[v] = __builtin_fmaf(sum[v], turn, total[v]);
           asm volatile("" : "+v"(total));   // (here, not when all taps' sums are there)
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -311,7 +318,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     __syncthreads();
     if (more) {
       base = slot_of(base, RPI * ST);
-      stage(base);
+      stage(base, i + 1);
       __syncthreads();
     }
   }
@@ -387,7 +394,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       }
       if (number && lane == 0) *numbers = i;
     }
-    if (group) {   // (as the loop above leaves it)
+    if (turned) {   // (as the loop above leaves it)
 #pragma unroll
       for (int i = 0; i < 9; ++i)
 #pragma unroll
@@ -412,7 +419,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   for (int i = 0; i < 9; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][v] - ex[(i * 16 + v) * 64]), rp, po, (i * 16 + v) * 256, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][v] - ex[(i * 16 + v) * 64]) ^ (sign & 0x80000000u), rp, po, (i * 16 + v) * 256, 0);
 }
 
 // dW from the partial images, in ascending order.  A workgroup takes four accumulator registers of a wavefront (16 bytes a lane:
