@@ -1462,10 +1462,11 @@ int run_d16(const sgh_conv_geom *g, const sgh_conv_geom *fwd_of, const uint16_t 
     b.QO = (b.HW + 7) / 8, b.octets = g->N * b.QO, b.mtiles = p.mtiles, b.ptiles = p.tiles;
     b.a_bytes = unsigned((as_is ? size_t(g->C) * g->K : nw) * 2);
     b.src_bytes = unsigned(size_t(g->N) * g->K * b.HW * 2);
-    if (tail) b.add = tail->add, b.gate = tail->gate, tail->done = true;
+    if (tail) b.add = tail->add, b.gate = tail->gate;
     sgh_prof_kernel_begin(fwd_of ? "conv_fwd16/k_pw16" : "conv_dgrad16/k_pw16", 2.0 * g->N * g->K * b.HW * double(g->C));
     const int rc = sgh_pw16_launch(b, p.bm, bf16, s);
     sgh_prof_kernel_end(s);
+    if (tail) tail->done = rc == SGH_OK;
     return rc;
   }
   D16Args a{};
