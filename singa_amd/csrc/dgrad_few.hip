@@ -135,8 +135,9 @@ __global__ __launch_bounds__(NT) void k_dgrad_few(Args a) {
 // drawn layers none of up to 67 filters is slower (50 x 3 x 42 x 53 to 140 43.8 / 39.6, 3 x 3 x 102 x 102 to 62 17.6 / 16.6), beyond, few
 // images are: 1 x 3 x 61 x 77, 5x5 to 79 23.0 / 26.5, 3 x 4 x 32 x 30 to 167 22.9 / 35.3, 13 x 4 x 32 x 22 to 964 84 / 222.
 bool sgh_dgrad_few_supported(const sgh_conv_geom *g) {
-  const size_t lim = size_t(1) << 31;
-  return g->C <= 4 && g->K <= 64 && g->R == g->S && (g->R == 3 || g->R == 5) && g->stride_h == 1 && g->stride_w == 1 && g->pad_h == g->pad_w &&
+  const size_t lim = size_t(1) << 31, wgs = size_t(g->N) * ((g->H + TH - 1) / TH) * ((g->W + TW - 1) / TW);
+  return wgs < size_t(1) << 24 &&   // (a launch holds less than 2^32 threads)
+         g->C <= 4 && g->K <= 64 && g->R == g->S && (g->R == 3 || g->R == 5) && g->stride_h == 1 && g->stride_w == 1 && g->pad_h == g->pad_w &&
          g->pad_h < g->R && size_t(g->N) * g->K * g->P * g->Q * 4 < lim && size_t(g->N) * g->C * g->H * g->W * 4 < lim;
 }
 

@@ -18,3 +18,16 @@ answer([run(), refused])
 """)
     assert fused[-1] == "k_pw16", fused
     assert "k_pw16" not in refused and "relu_bwd_add" in refused[-1], refused
+
+
+def test_data_gradient_of_too_many_tiny_planes_is_unsupported():
+    """A workgroup per 8 x 32 pixels of an image: 2^24 planes of one pixel are more than a launch can hold (2^32 threads).  They are left
+    to the column GEMM, which says that its grid does not hold them either; one plane less is launched."""
+    most, beyond = recorded("""
+def run(n):
+    g = conv(n, 1, 1, 1, 1, 3, 3, 1, 1, 1, 1)
+    need = max(lib.sgh_conv_workspace_bytes(C.byref(g), _lib.SGH_CONV_DGRAD), 9 << 26)
+    return lib.sgh_conv_dgrad_f32(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, need, None) == _lib.SGH_EUNSUPPORTED, kernels()
+answer([run((1 << 24) - 1), run(1 << 24)])
+""")
+    assert most == [False, ["k_dgrad_few"]] and beyond == [True, []], (most, beyond)
