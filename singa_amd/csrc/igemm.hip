@@ -1031,7 +1031,7 @@ static size_t plain_workspace_bytes(const sgh_conv_geom *g, int which) {
     case SGH_CONV_DGRAD:
       if (dgrad_path(g) == kDgradFewC) return sgh_dgrad_fewc_workspace_bytes(g);
       if (dgrad_path(g) == kDgradPointwise) return 0;
-      if (dgrad_path(g) == kDgradColumns) return RS * g->C * size_t(g->N) * g->P * g->Q * sizeof(float);
+      if (dgrad_path(g) == kDgradColumns) return sgh_dgrad_few_supported(g) ? 0 : RS * g->C * size_t(g->N) * g->P * g->Q * sizeof(float);
       return align256(RS * round_up(g->K, BK) * g->C * sizeof(float)) + align256(sizeof(DgClsTable)) +
              sgh_dgrad3x3_partial_bytes(g);
     case SGH_CONV_WGRAD: {

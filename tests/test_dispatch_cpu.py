@@ -31,3 +31,26 @@ def run(n):
 answer([run((1 << 24) - 1), run(1 << 24)])
 """)
     assert most == [False, ["k_dgrad_few"]] and beyond == [True, []], (most, beyond)
+
+
+def test_data_gradient_with_few_input_channels_takes_no_workspace():
+    """Layers of k_dgrad_few write no columns: no workspace is asked for, in fp32 none is needed, and the 16-bit passes, which widen
+    into theirs, need no more than that; one filter more than it takes, and the columns are there."""
+    few, few16, columns = recorded("""
+which = _lib.SGH_CONV_DGRAD
+g, wider = conv(128, 3, 32, 32, 64, 5, 5, 1, 1, 2, 2), conv(128, 3, 32, 32, 65, 5, 5, 1, 1, 2, 2)
+least = lib.sgh_conv_workspace_least_bytes(C.byref(g), which, 0)
+rc = lib.sgh_conv_dgrad_f32(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, None, 0, None)
+few = [lib.sgh_conv_workspace_bytes(C.byref(g), which), least, rc, kernels()]
+need = lib.sgh_conv_workspace_bytes_h(C.byref(g), which)
+rc = lib.sgh_conv_dgrad_bf16(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, need, None)
+few16 = [need, rc, kernels()]
+need = lib.sgh_conv_workspace_bytes(C.byref(wider), which)
+rc = lib.sgh_conv_dgrad_f32(C.byref(wider), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, need, None)
+columns = [need, rc, kernels(), lib.sgh_conv_dgrad_f32(C.byref(wider), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, need - 4, None) == -2]
+answer([few, few16, columns])
+""")
+    assert few == [0, 0, 0, ["k_dgrad_few"]], few
+    tensors = 4 * (128 * 64 * 32 * 32 + 64 * 3 * 25 + 128 * 3 * 32 * 32)   # dy, W and dx in fp32
+    assert few16[1] == 0 and few16[2].count("k_dgrad_few") == 1 and few16[0] <= tensors + 4096, few16
+    assert columns == [4 * 25 * 3 * 128 * 32 * 32, 0, ["k_igemm", "k_col2im_gather"], True], columns
