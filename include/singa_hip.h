@@ -399,7 +399,7 @@ SGH_API int sgh_gemm_f32(int transA, int transB, int M, int N, int K, float alph
 SGH_API int sgh_linear_fwd_f32(const float *x, const float *W, const float *bias, float *y, int rows, int in, int out,
                                int relu, void *stream);
 /* dx = dy W^T, kept where gate[rows][in] > 0 and zero elsewhere if `gate` is not NULL: the layer's data gradient and the backward
- * of the ReLU in front of it (python/singa/autograd.py:613-623, :432-439). */
+ * of the ReLU in front of it (python/singa/autograd.py:613-623, :432-439).  gate may not overlap dx (SGH_EINVAL). */
 SGH_API int sgh_linear_bwd_x_f32(const float *dy, const float *W, const float *gate, float *dx, int rows, int in, int out,
                                  void *stream);
 /* dW = x^T dy and db[out] = the column sums of dy (python/singa/autograd.py:613-623, :696-709). */
@@ -481,7 +481,8 @@ SGH_API int sgh_conv_dgrad_acc_f32(sgh_conv_geom *g, const float *dy, const floa
                                    float *dx, void *workspace, size_t ws_bytes, void *stream);
 /* dx = ReLUBackward(data gradient + add, x): the input gradient of a residual block whose input x is a ReLU's output, summed with
  * the gradient `add` of its other branch and gated (python/singa/autograd.py:204, :432-439).  The bits of the separate calls
- * (sgh_conv_dgrad_*, sgh_relu_bwd_add_*); one launch for 1x1 layers of stride 1.  add and x are not dx. */
+ * (sgh_conv_dgrad_*, sgh_relu_bwd_add_*); one launch for 1x1 layers of stride 1.  add and x may not
+ * overlap dx (SGH_EINVAL). */
 SGH_API int sgh_conv_dgrad_add_relu_f16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W,
                                         const uint16_t *add, const uint16_t *x, uint16_t *dx,
                                         void *workspace, size_t ws_bytes, void *stream);

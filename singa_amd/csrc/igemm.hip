@@ -1671,7 +1671,14 @@ int sgh_linear_fwd_f32(const float *x, const float *W, const float *bias, float 
   return rc;
 }
 
+// Whether two tensors of `bytes` each share memory
+static bool overlap(const void *a, const void *b, size_t bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return (x < y ? y - x : x - y) < bytes;
+}
+
 int sgh_linear_bwd_x_f32(const float *dy, const float *W, const float *gate, float *dx, int rows, int in, int out, void *stream) {
+  if (gate && rows > 0 && in > 0 && overlap(gate, dx, size_t(rows) * in * sizeof(float))) return SGH_EINVAL;
   sgh_gemm_around around;
   around.gate = gate;
   bool done = false;
@@ -1837,9 +1844,13 @@ int sgh_conv_dgrad_bf16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W,
   return conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_bf16_to_f32,
                    sgh_cast_f32_to_bf16);
 }
+static bool tail_refused(const sgh_conv_geom *g, const uint16_t *add, const uint16_t *x, const uint16_t *dx) {
+  const size_t bytes = size_t(g->N) * g->C * g->H * g->W * sizeof(uint16_t);
+  return !add || !x || overlap(add, dx, bytes) || overlap(x, dx, bytes);
+}
 int sgh_conv_dgrad_add_relu_f16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, const uint16_t *add, const uint16_t *x,
                                 uint16_t *dx, void *workspace, size_t ws_bytes, void *stream) {
-  if (!conv_ok(g) || !add || !x) return SGH_EINVAL;
+  if (!conv_ok(g) || tail_refused(g, add, x, dx)) return SGH_EINVAL;
   sgh_dgrad_tail tail{add, x, false};
   const int rc = conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_f16_to_f32,
                            sgh_cast_f32_to_f16, &tail);
@@ -1847,7 +1858,7 @@ int sgh_conv_dgrad_add_relu_f16(sgh_conv_geom *g, const uint16_t *dy, const uint
 }
 int sgh_conv_dgrad_add_relu_bf16(sgh_conv_geom *g, const uint16_t *dy, const uint16_t *W, const uint16_t *add, const uint16_t *x,
                                  uint16_t *dx, void *workspace, size_t ws_bytes, void *stream) {
-  if (!conv_ok(g) || !add || !x) return SGH_EINVAL;
+  if (!conv_ok(g) || tail_refused(g, add, x, dx)) return SGH_EINVAL;
   sgh_dgrad_tail tail{add, x, false};
   const int rc = conv_half(g, SGH_CONV_DGRAD, dy, W, nullptr, dx, workspace, ws_bytes, stream, sgh_cast_bf16_to_f32,
                            sgh_cast_f32_to_bf16, &tail);

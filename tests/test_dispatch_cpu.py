@@ -54,3 +54,29 @@ answer([few, few16, columns])
     tensors = 4 * (128 * 64 * 32 * 32 + 64 * 3 * 25 + 128 * 3 * 32 * 32)   # dy, W and dx in fp32
     assert few16[1] == 0 and few16[2].count("k_dgrad_few") == 1 and few16[0] <= tensors + 4096, few16
     assert columns == [4 * 25 * 3 * 128 * 32 * 32, 0, ["k_igemm", "k_col2im_gather"], True], columns
+
+
+def test_gates_and_sums_that_overlap_the_result_are_refused():
+    """The other branch's gradient, the gate and the result of sgh_conv_dgrad_add_relu_*, the gate and the result of
+    sgh_linear_bwd_x_f32: read after parts of the result have been written.  Shared or overlapping they are refused and nothing is launched;
+    side by side they are taken."""
+    refused, taken = recorded("""
+bytes_ = 2 * 64 * 9 * 9 * 2
+g = conv(2, 64, 9, 9, 64, 1, 1, 1, 1, 0, 0)
+need = lib.sgh_conv_workspace_bytes_h(C.byref(g), _lib.SGH_CONV_DGRAD)
+def block(fn, add, x, dx):
+    return fn(C.byref(g), SPACE, 2 * SPACE, add, x, dx, 6 * SPACE, need, None), len(kernels())
+A, X, D = 3 * SPACE, 4 * SPACE, 5 * SPACE
+refused, taken = [], []
+for fn in (lib.sgh_conv_dgrad_add_relu_f16, lib.sgh_conv_dgrad_add_relu_bf16):
+    refused += [block(fn, D, X, D), block(fn, A, D, D), block(fn, D + bytes_ - 2, X, D), block(fn, A, D - bytes_ + 2, D)]
+    taken += [block(fn, D + bytes_, X, D), block(fn, A, D - bytes_, D), block(fn, A, A, D)]
+for rows, inner, out in ((33, 70, 50), (3000, 700, 800)):
+    linear = lambda gate, dx: (lib.sgh_linear_bwd_x_f32(SPACE, 2 * SPACE, gate, dx, rows, inner, out, None), len(kernels()))
+    bytes_ = rows * inner * 4
+    refused += [linear(D, D), linear(D + bytes_ - 4, D), linear(D - bytes_ + 4, D)]
+    taken += [linear(D + bytes_, D), linear(None, D)]
+answer([refused, taken])
+""")
+    assert all(r == [-1, 0] for r in refused), refused
+    assert all(rc == 0 and n > 0 for rc, n in taken), taken
