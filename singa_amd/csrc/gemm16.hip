@@ -533,15 +533,22 @@ bool split_plan(int M, int N, int K, int *tile, int *waves) {
   return (M + *tile - 1) / *tile <= 65535;
 }
 
-// Whether the tiled kernel is the better one where both can run.  Beyond one 32-wide tile per CU it is (us, split / tiled, bfloat16:
-// 512 x 1024 x 2048 NN 16.8 / 10.2, 1024^3 NN 16.5 / 7.0, 48 x 6256 x 2536 NT 23.5 / 13.9), below where there is much to do (2000 x
-// 100 x 2000 NN, 504 000 tiles times indices, 10.5 / 10.1; but 20 x 8000 x 1000 NT, 250 000, 5.1 / 6.4 and 8 x 1608 x 2824 NT,
-// 144 000, 4.9 / 12.6); with rows at odd elements the split kernel's loads take several times as long, and the line lies lower
-// (807 x 211 x 6728 NN 79 / 35, 220 x 927 x 1271 NN, 258 000, 18.5 / 9.5, 116 x 181 x 5879 NN, 141 000, 43 / 32, but 87 x 133 x 2207
-// NT, 33 000, 12.3 / 13.8).
-bool tile_pays(int M, int N, int K, bool odd) {
-  const long t32 = long((M + 31) / 32) * ((N + 31) / 32);
-  return t32 > sgh_num_cus() || t32 * K > (odd ? 120000 : 400000);
+// Whether the tiled kernel is the better one where both can run.  The lines lie where the fewest of 1500 products lose to the other
+// kernel (drawn over 8..4096 rows and columns, 8..8192 indices, all four layouts, replayed from a graph; us, split / tiled):
+//   More than one 32-wide tile per CU: the tiled one, unless the reduction is short beside a launch (1024^3 NN 16.5 / 7.0, 512 x 1024 x
+// 2048 NN 16.8 / 10.2; 504 x 904 x 104 NT 3.3 / 3.6, 44 x 5002 x 49 NT 3.0 / 3.7; with rows at odd elements 129 x 1648 x 587 TT 12.1 / 6.4).
+//   Fewer: 64-wide tiles leave most of the CUs without a workgroup, and the split kernel is the better one however long the reduction is
+// (256 x 1000 x 2048 NN 10.0 / 11.0, 472 x 54 x 5911 NN 21.1 / 30.3, 208 x 744 x 4304 NT 12.8 / 17.6, 974 x 36 x 6700 NN 13.4 / 29.1), except
+// with rows at odd elements, where its loads take several times as long (780 x 213 x 4336 NN 82 / 26, 180 tiles x 2984 NN 2.6 times, 128 x 1657
+// TT 1.8 times; but 54 tiles x 3323 NN 13.4 / 18.4, 25 x 1795 NT 0.8 times).  A transposed and B not, both walk along their rows and odd
+// ones cost little (231 x 791 x 695 5.4 / 6.8, 1643 x 69 x 7633 36 / 43).
+// 59 of the 1500 are more than 5 per cent from the better kernel, 0.6 per cent at the geometric mean.
+bool tile_pays(bool ta, bool tb, int M, int N, int K, int lda, int ldb) {
+  const long t32 = long((M + 31) / 32) * ((N + 31) / 32), cus = sgh_num_cus(), work = t32 * K;
+  const bool odd = (lda | ldb) & 1;
+  if (t32 > cus) return work > (odd ? 30000 : 100000);
+  if (!odd || (ta && !tb)) return false;
+  return !ta && !tb && (ldb & 1) ? work > 30000 : 4 * t32 >= cus && work > 100000;
 }
 
 // The tiled kernel's tile and groups.  128-wide tiles (half the loads per product) once they give every CU one and the reduction
@@ -572,8 +579,7 @@ int gemm16(int transA, int transB, int M, int N, int K, float alpha, const uint1
   const bool small = K > 0 && size_t(transA ? K : M) * lda < (size_t(1) << 30) &&
                      size_t(transB ? N : K) * ldb < (size_t(1) << 30);   // operands addressed with 32-bit byte offsets
   const bool split = small && split_plan(M, N, K, &tile, &waves), octets = M >= 8 && N >= 8 && K >= 8;
-  const bool odd = ((lda | ldb) & 1) || ((transA ? M : 0) & 1) || ((transB ? 0 : N) & 1);
-  if (small && octets && !(split && !tile_pays(M, N, K, odd))) {
+  if (small && octets && !(split && !tile_pays(transA, transB, M, N, K, lda, ldb))) {
     tile_plan(M, N, K, &bt, &ks);
     if (!transA && transB) launch_tile<BF16, true, true>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
     else if (!transA) launch_tile<BF16, true, false>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);

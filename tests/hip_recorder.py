@@ -53,7 +53,7 @@ const char *recorder_take() { static std::string out; out = noted; noted.clear()
 
 PREAMBLE = """
 import ctypes as C, json, sys
-sys.path.insert(0, %r)
+sys.path[:0] = [%r, %r]
 recorder = C.CDLL(%r, mode=C.RTLD_GLOBAL)
 recorder.recorder_take.restype = C.c_char_p
 from singa_amd import _lib
@@ -92,7 +92,7 @@ def recorded(code):
         with open(src, "w") as f:
             f.write(SOURCE)
         subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", src, "-o", so])
-        body = PREAMBLE % (ROOT, so) + "\ndef answer(v):\n    print('ANSWER ' + json.dumps(v), flush=True)\n\n" + code
+        body = PREAMBLE % (ROOT, os.path.join(ROOT, "tests"), so) + "\ndef answer(v):\n    print('ANSWER ' + json.dumps(v), flush=True)\n\n" + code
         p = subprocess.run([sys.executable, "-c", body], stdout=subprocess.PIPE, stderr=subprocess.PIPE, timeout=120, cwd=ROOT)
         lines = [l for l in p.stdout.decode().splitlines() if l.startswith("ANSWER ")]
         assert p.returncode == 0 and lines, p.stderr.decode()[-3000:]

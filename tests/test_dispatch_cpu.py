@@ -80,3 +80,26 @@ answer([refused, taken])
 """)
     assert all(r == [-1, 0] for r in refused), refused
     assert all(rc == 0 and n > 0 for rc, n in taken), taken
+
+
+def test_which_16bit_gemm_takes_a_product():
+    """Few tiles and a long reduction stay with the split kernel (64-wide tiles would leave most CUs idle), as do many tiles with hardly
+    any reduction; many tiles with some, and odd rows, go to the tiled one.  (M, N, K, layouts): measured on both."""
+    split = [(256, 1000, 2048, "NN"), (256, 1000, 2048, "NT"), (472, 54, 5911, "NN"), (208, 744, 4304, "NT"), (840, 88, 6296, "NT"),
+             (974, 36, 6700, "NN"), (44, 5002, 49, "NT"), (1357, 337, 9, "NT"), (1643, 69, 7633, "TN"), (231, 791, 695, "TN"),
+             (857, 62, 3323, "NN")]
+    tiled = [(512, 1024, 2048, "NN"), (1024, 1024, 1024, "NN"), (48, 6256, 2536, "NT"), (780, 213, 4336, "NN"), (807, 211, 6728, "NN"),
+             (161, 621, 2303, "TT"), (129, 1648, 587, "TT"), (700, 6000, 700, "NT")]
+    got = recorded("""
+def kernel(M, N, K, layout, pad=0):
+    tA, tB = layout[0] == "T", layout[1] == "T"
+    lda, ldb = (M if tA else K) + pad, (K if tB else N) + pad
+    assert lib.sgh_gemm_bf16(tA, tB, M, N, K, 1.0, SPACE, lda, 2 * SPACE, ldb, 0.0, 3 * SPACE, N, None) == 0
+    return kernels()
+from test_gpu_half import TILE_EDGES
+answer([[kernel(*p) for p in %r], [kernel(*p) for p in %r],
+        [kernel(*p, a + b, pad) for p in TILE_EDGES for a in "NT" for b in "NT" for pad in range(4)]])
+""" % (split, tiled))
+    for products, kernels, name in zip((split, tiled, None), got, ("k_gemm16_split", "k_gemm16_tile", "k_gemm16_tile")):
+        wrong = [(p, k) for p, k in zip(products or kernels, kernels) if k != [name]]
+        assert not wrong, (name, wrong)

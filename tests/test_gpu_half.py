@@ -186,9 +186,14 @@ def test_gemm_16bit(singa, dev, kind, M, N, K):
     _same_bits(singa.Mult(et, bt).to_numpy(), singa.Mult(et, bt).to_numpy(), "run to run")
 
 
+# products that the tiled 16-bit GEMM takes, whatever the layouts and pitches (test_dispatch_cpu.py)
+TILE_EDGES = [(1100, 1065, 9), (1032, 1064, 64), (1031, 1070, 65), (1030, 1041, 128), (1000, 1001, 131), (520, 523, 390), (519, 525, 352),
+              (265, 1030, 450), (513, 770, 257), (2049, 2183, 257)]
+
+
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
-@pytest.mark.parametrize("M,N,K", [(1100, 265, 9), (1032, 264, 64), (1031, 270, 65), (265, 1030, 131), (520, 523, 198), (519, 525, 260),
-                                   (513, 770, 127), (2049, 2183, 257)])
+@pytest.mark.parametrize("M,N,K", TILE_EDGES + [(1100, 265, 9), (1032, 264, 64), (1031, 270, 65), (265, 1030, 131), (520, 523, 198),
+                                                (519, 525, 260), (513, 770, 127)])   # (the last: either kernel, by layout and pitch)
 def test_gemm_16bit_tile_edges(singa, dev, kind, M, N, K):
     """The tiled kernel (more than 256 tiles of 32 x 32): edges that end inside an octet of rows, reductions that end inside an octet,
     a chunk or leave the second group without one, one group (more than 256 tiles of 64, or at most 128 indices) and two, 128-wide tiles
