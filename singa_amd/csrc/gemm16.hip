@@ -4,7 +4,7 @@
 //
 // Three kernels; none splits the reduction over workgroups and every sum is taken in a fixed order: results are run-to-run
 // identical.  k_gemm16_tile (many output tiles) and k_gemm16_split (few) do the work; k_gemm16 is left with what neither can
-// address: operands of 2 GB and more, and fewer than eight rows, columns or reduction indices against many of the others.
+// address: operands of 2 GB and more, 2^24 tiles, and fewer than eight rows, columns or reduction indices against many of the others.
 //
 // k_gemm16: a workgroup of four wavefronts owns a 64 x 64 tile of C, a wavefront a 32 x 32 quarter.  Both matrix
 // operands want, per lane, eight consecutive reduction indices of one tile row, so both LDS tiles are
@@ -555,10 +555,12 @@ bool tile_pays(bool ta, bool tb, int M, int N, int K, int lda, int ldb) {
 // is long enough to matter (64 / 128: 2048 x 4096 x 1200 NT 46 / 30 us, 512 tiles; 700 x 6000 x 700 NT 18.5 / 17.7, 282; 1500^3 23.5 /
 // 24.9, 144; 2232 x 2280 x 40 TN 6.4 / 7.1).  Two groups halve the chain of a workgroup that has its CU to itself (1024^3 8.4 / 7.0 with
 // 256 tiles, 700 x 700 x 6000 39 / 31 with 121; 1813 x 597 x 964 11.8 / 12.1 with 290); four gain nothing more (6.9, 31.3).
-void tile_plan(int M, int N, int K, int *bt, int *ks) {
+// False where the workgroups are more than a launch holds (2^32 threads).
+bool tile_plan(int M, int N, int K, int *bt, int *ks) {
   const long t64 = long((M + 63) / 64) * ((N + 63) / 64), t128 = long((M + 127) / 128) * ((N + 127) / 128), cus = sgh_num_cus();
   *bt = t128 > cus && K >= 256 ? 128 : 64;
   *ks = t64 <= cus && K > 2 * TK ? 2 : 1;
+  return (*bt == 128 ? t128 : t64) <= (long(1) << 24) - 8;
 }
 
 template <bool BF16>
@@ -579,8 +581,7 @@ int gemm16(int transA, int transB, int M, int N, int K, float alpha, const uint1
   const bool small = K > 0 && size_t(transA ? K : M) * lda < (size_t(1) << 30) &&
                      size_t(transB ? N : K) * ldb < (size_t(1) << 30);   // operands addressed with 32-bit byte offsets
   const bool split = small && split_plan(M, N, K, &tile, &waves), octets = M >= 8 && N >= 8 && K >= 8;
-  if (small && octets && !(split && !tile_pays(transA, transB, M, N, K, lda, ldb))) {
-    tile_plan(M, N, K, &bt, &ks);
+  if (small && octets && !(split && !tile_pays(transA, transB, M, N, K, lda, ldb)) && tile_plan(M, N, K, &bt, &ks)) {
     if (!transA && transB) launch_tile<BF16, true, true>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
     else if (!transA) launch_tile<BF16, true, false>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);
     else if (transB) launch_tile<BF16, false, true>(bt, ks, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, st);

@@ -103,3 +103,15 @@ answer([[kernel(*p) for p in %r], [kernel(*p) for p in %r],
     for products, kernels, name in zip((split, tiled, None), got, ("k_gemm16_split", "k_gemm16_tile", "k_gemm16_tile")):
         wrong = [(p, k) for p, k in zip(products or kernels, kernels) if k != [name]]
         assert not wrong, (name, wrong)
+
+
+def test_16bit_gemm_of_more_tiles_than_a_launch_holds():
+    """The tiled kernel's workgroups are counted in one dimension, 2^24 of 256 threads at most: a short product of 2^18 x 2^18 goes to the
+    kernel with two, as do extents below eight; a row of tiles less is tiled."""
+    got = recorded("""
+def kernel(M, N, K):
+    assert lib.sgh_gemm_f16(0, 0, M, N, K, 1.0, SPACE, K, 2 * SPACE, N, 0.0, 3 * SPACE, N, None) == 0
+    return kernels()
+answer([kernel(1 << 18, 1 << 18, 8), kernel((1 << 18) - 64, 1 << 18, 8), kernel(1 << 18, 4, 8)])
+""")
+    assert got == [["k_gemm16"], ["k_gemm16_tile"], ["k_gemm16"]], got
