@@ -57,6 +57,33 @@ def test_fused_update_equals_per_parameter_update(dev):
         assert np.array_equal(a, b)
 
 
+def test_dense_layers_take_transposed_views(dev):
+    """A network's input, or a layer's weights in a forward and a backward pass, may be a transposed view of what lies in memory: the same
+    products as those of the op-by-op tape, bit for bit, and those of a dense copy to rounding."""
+    from singa_amd import singa_wrap as singa
+    hip = wl.HipOps(dev)
+    x, labels = wl.make_inputs("mlp", 20)
+    view = lambda a: singa.DefaultTranspose(hip.from_numpy(np.ascontiguousarray(a.T)))
+
+    def step(fused, x_view, w_view):
+        hip.set_fusion(fused)
+        net = wl.build("mlp", hip)
+        if w_view:
+            net.layers[2].W = view(net.layers[2].W.to_numpy())
+        loss = net.forward(view(x) if x_view else hip.from_numpy(x), hip.from_numpy(labels)).to_numpy()
+        grads = {}
+        dy = net.layers[2].bwd_behind_relu(net.layers[1], hip.softmax_ce_bwd(net.p, net.t, net.batch), lambda n, p, g: grads.update({n: g.to_numpy()}))
+        dy = net.layers[0].bwd(dy, lambda n, p, g: grads.update({n: g.to_numpy()}))
+        return dict(grads, loss=loss, dx=dy.to_numpy())
+
+    dense = step(True, False, False)
+    for x_view, w_view in ((True, False), (False, True), (True, True)):
+        got, want = step(True, x_view, w_view), step(False, x_view, w_view)
+        for k in dense:
+            assert np.array_equal(got[k], want[k]), k
+            assert nl2(got[k], dense[k]) < 1e-5, k
+
+
 def test_resnet18_full_batch_properties(dev):
     """ResNet-18 at the benchmark's full size (N=64, 224x224) is beyond the CPU oracle inside a
     test; parity at that size is checked through properties that do not depend on size:
