@@ -934,7 +934,7 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
   // (`tail`: the last chunk holds channels beyond K; of this group's matrix steps only the first `left` are not all zeros.  37 images
   // of 31 x 45, 72 and 136 channels: forward and data gradient 75 -> 69 us together.  A layer of one chunk keeps them all: with a second
   // copy of its loop it takes 168 registers instead of 116)
-  const int left = max(0, (a.K - (nkc - 1) * KC - half * 32 + 15) / 16);
+  const int last_steps = (a.K - (nkc - 1) * KC + 15) / 16, left = max(0, last_steps - half * KS);
   auto step = [&](int kc, auto tapc, auto parc, auto tailc) {
     constexpr bool TAIL = decltype(tailc)::value;
     constexpr int TAP = decltype(tapc)::value, PAR = decltype(parc)::value, R_ = TAP / 3, S_ = TAP % 3;
@@ -976,7 +976,9 @@ __global__ __launch_bounds__(NT) void k_dgrad16_slab(S16Args a) {
     step(kc, std::integral_constant<int, 7>{}, P1{}, tail);
     step(kc, std::integral_constant<int, 8>{}, P0{}, tail);
   };
-  const int nfull = MULTI && left < KS ? nkc - 1 : nkc;
+  // (both groups run the same copy of the loop: its barriers are the whole workgroup's, so a group without zeros of its own takes the tail
+  // with the other one)
+  const int nfull = MULTI && last_steps < KC / 16 ? nkc - 1 : nkc;
   for (int kc = 0; kc < nfull; kc += 2) {
     chunk(kc, std::integral_constant<int, 0>{}, std::false_type{});
     if (!MULTI || kc + 1 >= nfull) break;

@@ -1065,6 +1065,7 @@ def test_conv_3x3_16bit_any_plane(singa, dev, kind, case):
 def test_conv_3x3_16bit_partial_last_chunk(singa, dev, kind, K, N, C, H, W):
     """A reduction whose last chunk of 64 channels is partly empty: the matrix steps that would multiply only zeros are left out, so
     the results have the bits that they have with those channels there and zero; a forward pass and a data gradient."""
+    from util import kernels_of
     r = rng(K + C)
     full = (K + 63) // 64 * 64
     pad = lambda a, axis: np.concatenate([a, np.zeros(a.shape[:axis] + (full - K,) + a.shape[axis + 1:], np.float32)], axis)
@@ -1075,15 +1076,19 @@ def test_conv_3x3_16bit_partial_last_chunk(singa, dev, kind, K, N, C, H, W):
     def dgrad(w, dy):
         k = len(w)
         xt, wt, dyt = (_to(singa, dev, a, kind)[0] for a in (x, w, dy))
-        return singa.GpuConvBackwardx(dyt, wt, xt, singa.CudnnConvHandle(xt, (3, 3), (1, 1), (1, 1), C, k, False)).to_numpy()
+        h = singa.CudnnConvHandle(xt, (3, 3), (1, 1), (1, 1), C, k, False)
+        return kernels_of(dev, lambda: singa.GpuConvBackwardx(dyt, wt, xt, h).to_numpy())
 
     def forward(w, dy):   # (the reduction over dy's channels)
         k = len(w)
         dyt, wt = (_to(singa, dev, a, kind)[0] for a in (dy, np.ascontiguousarray(w.transpose(1, 0, 2, 3))))
-        return singa.GpuConvForward(dyt, wt, None, singa.CudnnConvHandle(dyt, (3, 3), (1, 1), (1, 1), k, C, False)).to_numpy()
+        h = singa.CudnnConvHandle(dyt, (3, 3), (1, 1), (1, 1), k, C, False)
+        return kernels_of(dev, lambda: singa.GpuConvForward(dyt, wt, None, h).to_numpy())
 
     for f in (dgrad, forward):
-        _same_bits(f(w, dy), f(pad(w, 0), pad(dy, 1)), f.__name__)
+        (got, names), (want, full_names) = f(w, dy), f(pad(w, 0), pad(dy, 1))
+        assert names == full_names == {"k_dgrad16_slab"}, (names, full_names)
+        _same_bits(got, want, f.__name__)
 
 
 # layers that the octet weight gradient (wgrad_oct16.hip) takes: rows of one to four octets and of several strips, whole and ragged
