@@ -1,20 +1,27 @@
-// fp32 convolutions on split operands (conv_split.hip): stride 1, "same" padding, 3x3 and 5x5.  `g` is the geometry of the
-// data gradient: K channels of `in` are gathered onto C channels of `out`; a forward pass hands in the channel-swapped one.
+// fp32 convolutions on split operands (conv_split.hip): "same" padding, 3x3 and 5x5 of stride 1 and forward passes of 3x3 and stride 2.
+// `g` is the geometry of the data gradient: K channels of `in` are gathered onto C channels of `out`; a forward pass hands in the
+// channel-swapped one.
 #ifndef SINGA_AMD_CSRC_CONV_SPLIT_H_
 #define SINGA_AMD_CSRC_CONV_SPLIT_H_
 
 #include "common.h"
 #include "split_parts.h"
 
-bool sgh_conv_split_supported(const sgh_conv_geom *g);
-size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g);   // weight fragments, then the partial tiles
+// How the layer runs; made once per call (stride 2: a microsecond of host time)
+struct sgh_conv_split_plan {
+  bool ok;   // false: a layer for other kernels
+  int r, st, gm, wm, wn, et, bm, bn, ih, iw, pitch, rows, slab, nchunks, cblocks;
+  int ctiles, tiles, dp_tiles, share, wgs;
+  size_t weight_bytes, bytes;   // of the workspace: the weight fragments, and with the partial tiles behind them
+};
+sgh_conv_split_plan sgh_conv_split_plan_of(const sgh_conv_geom *g);
 // the weight fragments of `g` into the front of `workspace`, from W[C][K][R][S] or (dgrad) W[K][C][R][S]
 int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspace, bool dgrad, hipStream_t s);
 // the same as a batch item: workgroups of sgh_conv_split_weights_block
 int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps);
 // `W`: the same weights again, for what the fragments cannot hold
-int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s,
-                       const char *tag, bool dgrad, const float *bias, bool accumulate);
+int sgh_conv_split_run(const sgh_conv_geom *g, const sgh_conv_split_plan &p, const float *in, const float *W, float *out, void *workspace,
+                       hipStream_t s, const char *tag, bool dgrad, const float *bias, bool accumulate);
 
 constexpr int kSplitWeightLds = 512 * 9;   // floats of LDS that a workgroup below needs
 

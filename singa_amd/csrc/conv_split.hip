@@ -1,5 +1,5 @@
-// fp32 convolutions of stride 1 with "same" padding (3x3, 5x5), forward and data gradient, on the bfloat16 matrix
-// instructions without giving up fp32 operands (the splitting of G. Henry, P. Tang, A. Heinecke, "Leveraging the bfloat16
+// fp32 convolutions of stride 1 with "same" padding (3x3, 5x5), forward and data gradient, and 3x3 forward passes of stride 2, on the
+// bfloat16 matrix instructions without giving up fp32 operands (the splitting of G. Henry, P. Tang, A. Heinecke, "Leveraging the bfloat16
 // artificial intelligence datatype for higher-precision computations", 2019): a fp32 value, times 2^16 so that this holds for
 // the smallest ones too, is the sum of three bfloat16 values
 //
@@ -419,14 +419,13 @@ __global__ __launch_bounds__(256) void k_conv_split_fixup(ScArgs a, int BM, int 
   }
 }
 
-struct ScPlan {
-  bool ok;
-  int r, st, gm, wm, wn, et, bm, bn, ih, iw, pitch, rows, slab, nchunks, cblocks;
-  int ctiles, tiles, dp_tiles, share, wgs;
-};
+inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
-ScPlan plan(const sgh_conv_geom *g) {
-  ScPlan p{};
+}  // namespace
+
+sgh_conv_split_plan sgh_conv_split_plan_of(const sgh_conv_geom *g) {
+  sgh_conv_split_plan p{};
+  if (sgh_env().conv_split_off) return p;
   // (stride 2: the geometry of a forward pass with its channels swapped)
   if ((g->R != 3 && g->R != 5) || g->S != g->R || g->stride_h != g->stride_w || g->stride_h < 1 || g->stride_h > (g->R == 3 ? 2 : 1)) return p;
   const int o = (g->R - 1) / 2;
@@ -493,12 +492,16 @@ ScPlan plan(const sgh_conv_geom *g) {
   if (p.share > p.nchunks) p.share = p.nchunks;
   if (p.share <= 1) p.share = 1, p.dp_tiles = p.tiles;
   p.wgs = p.dp_tiles + (p.tiles - p.dp_tiles) * p.share;
+  p.weight_bytes = size_t(p.nchunks) * p.r * p.r * p.cblocks * kFrag;
+  p.bytes = align256(p.weight_bytes) + size_t(p.wgs - p.dp_tiles) * p.bm * p.bn * sizeof(float);
   p.ok = true;
   return p;
 }
 
+namespace {
+
 template <int GM, int WM, int WN, int ET, int R, int ST>
-int launch(const ScArgs &a, const ScPlan &p, hipStream_t s) {
+int launch(const ScArgs &a, const sgh_conv_split_plan &p, hipStream_t s) {
   auto kern = k_conv_split<GM, WM, WN, ET, R, ST>;
   static bool attr_set = false;
   if (!attr_set) {
@@ -511,8 +514,6 @@ int launch(const ScArgs &a, const ScPlan &p, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 
-inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
-
 // Weight fragments [chunk][tap][32-row block][part][lane][8]: one workgroup per (chunk, block).  Destination rows c are the
 // output channels, k the reduction; the source is W[c][k][tap] (forward) or W[k][c][last - tap] (data gradient).
 __global__ __launch_bounds__(256) void k_conv_split_weights(const float *__restrict__ W, uint16_t *__restrict__ wt, int C, int K,
@@ -522,18 +523,6 @@ __global__ __launch_bounds__(256) void k_conv_split_weights(const float *__restr
 }
 
 }  // namespace
-
-bool sgh_conv_split_supported(const sgh_conv_geom *g) { return plan(g).ok && !sgh_env().conv_split_off; }
-
-size_t sgh_conv_split_weight_bytes(const sgh_conv_geom *g) {
-  const ScPlan p = plan(g);
-  return p.ok ? size_t(p.nchunks) * p.r * p.r * p.cblocks * kFrag : 0;
-}
-
-size_t sgh_conv_split_workspace_bytes(const sgh_conv_geom *g) {
-  const ScPlan p = plan(g);
-  return p.ok ? align256(sgh_conv_split_weight_bytes(g)) + size_t(p.wgs - p.dp_tiles) * p.bm * p.bn * sizeof(float) : 0;
-}
 
 int sgh_conv_split_weight_blocks(const sgh_conv_geom *g, int *cblocks, int *taps) {
   *cblocks = (g->C + 31) / 32;
@@ -550,9 +539,8 @@ int sgh_conv_split_weights(const sgh_conv_geom *g, const float *W, void *workspa
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
 
-int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, float *out, void *workspace, hipStream_t s, const char *tag,
-                       bool dgrad, const float *bias, bool accumulate) {
-  const ScPlan p = plan(g);
+int sgh_conv_split_run(const sgh_conv_geom *g, const sgh_conv_split_plan &p, const float *in, const float *W, float *out, void *workspace,
+                       hipStream_t s, const char *tag, bool dgrad, const float *bias, bool accumulate) {
   if (!p.ok) return SGH_EUNSUPPORTED;
   ScArgs a;
   a.in = in;
@@ -561,7 +549,7 @@ int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, 
   a.wt = static_cast<const uint16_t *>(workspace);
   a.bias = bias;
   a.out = out;
-  a.partials = reinterpret_cast<float *>(static_cast<char *>(workspace) + align256(sgh_conv_split_weight_bytes(g)));
+  a.partials = reinterpret_cast<float *>(static_cast<char *>(workspace) + align256(p.weight_bytes));
   a.accumulate = accumulate ? 1 : 0;
   a.dgrad = dgrad ? 1 : 0;
   a.N = g->N, a.C = g->C, a.K = g->K, a.P = g->P, a.Q = g->Q;
@@ -571,7 +559,7 @@ int sgh_conv_split_run(const sgh_conv_geom *g, const float *in, const float *W, 
   a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share;
   a.xcd_runs = p.dp_tiles % 64 == 0 && !sgh_env().conv_xcd_off;
   a.in_bytes = unsigned(size_t(g->N) * g->K * p.ih * p.iw * 4);
-  a.wt_bytes = unsigned(sgh_conv_split_weight_bytes(g));
+  a.wt_bytes = unsigned(p.weight_bytes);
   int rc = SGH_EUNSUPPORTED;
   sgh_prof_kernel_begin(tag, 2.0 * g->N * g->K * g->P * g->Q * g->C * p.r * p.r);
 #define SC_CASE(GM_, WM_, WN_, ET_, R_, ST_) \

@@ -861,22 +861,22 @@ inline bool fwd_as_dgrad(const sgh_conv_geom *g, sgh_conv_geom *gt) {
 }
 
 // The same problem for the split kernel (conv_split.hip), where that one takes it
-inline bool fwd_as_split(const sgh_conv_geom *g, sgh_conv_geom *gt) {
+inline sgh_conv_split_plan fwd_split_plan(const sgh_conv_geom *g, sgh_conv_geom *gt) {
   *gt = *g;
   gt->C = g->K;
   gt->K = g->C;
-  return sgh_conv_split_supported(gt);
+  return sgh_conv_split_plan_of(gt);
 }
 
-// (stride 1: conv_split.hip, stride 2: dgrad_split2.hip)
-inline bool dgrad_as_split(const sgh_conv_geom *g) {
-  const DgradPath path = dgrad_path(g);
-  if (path == kDgradFewC || path == kDgradPointwise || path == kDgradColumns) return false;
-  return g->stride_h == 1 && g->stride_w == 1 ? sgh_conv_split_supported(g) : sgh_dgrad_split2_supported(g);
-}
-
+// The workspace of a data gradient on split operands (stride 1: conv_split.hip, stride 2: dgrad_split2.hip), 0 for the other layers
 inline size_t dgrad_split_bytes(const sgh_conv_geom *g) {
-  return g->stride_h == 1 ? sgh_conv_split_workspace_bytes(g) : sgh_dgrad_split2_workspace_bytes(g);
+  const DgradPath path = dgrad_path(g);
+  if (path == kDgradFewC || path == kDgradPointwise || path == kDgradColumns) return 0;
+  if (g->stride_h == 1 && g->stride_w == 1) {
+    const sgh_conv_split_plan p = sgh_conv_split_plan_of(g);
+    return p.ok ? p.bytes : 0;
+  }
+  return sgh_dgrad_split2_supported(g) ? sgh_dgrad_split2_workspace_bytes(g) : 0;
 }
 
 }  // namespace
@@ -1054,8 +1054,11 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   if (!conv_ok(g) || g->groups > 1) return plain;
   sgh_conv_geom gt;
   size_t split = 0;
-  if (which == SGH_CONV_FWD && fwd_as_split(g, &gt)) split = sgh_conv_split_workspace_bytes(&gt);
-  if (which == SGH_CONV_DGRAD && dgrad_as_split(g)) split = dgrad_split_bytes(g);
+  if (which == SGH_CONV_FWD) {
+    const sgh_conv_split_plan p = fwd_split_plan(g, &gt);
+    split = p.ok ? p.bytes : 0;
+  }
+  if (which == SGH_CONV_DGRAD) split = dgrad_split_bytes(g);
   if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g);
   return split > plain ? split : plain;
 }
@@ -1075,7 +1078,8 @@ static size_t least_bytes_f32(const sgh_conv_geom *g, int which) {
 
 // Which of the two layouts of the weights a data gradient with this workspace works on
 static bool dgrad_splits(const sgh_conv_geom *g, size_t ws_bytes) {
-  return dgrad_as_split(g) && ws_bytes >= dgrad_split_bytes(g);
+  const size_t bytes = dgrad_split_bytes(g);
+  return bytes && ws_bytes >= bytes;
 }
 
 // `prelaid`: the workspace already holds this layer's re-laid weights (sgh_conv_dgrad_prepare_multi)
@@ -1124,7 +1128,8 @@ static int conv_dgrad(const sgh_conv_geom *g, const float *dy, const float *W, f
   } else if (dgrad_splits(g, ws_bytes)) {
     if (!prelaid) rc = sgh_conv_split_weights(g, W, workspace, true, s);
     if (rc == SGH_OK)
-      rc = g->stride_h == 1 ? sgh_conv_split_run(g, dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr, accumulate)
+      rc = g->stride_h == 1 ? sgh_conv_split_run(g, sgh_conv_split_plan_of(g), dy, W, dx, workspace, s, "conv_dgrad/k_conv_split", true, nullptr,
+                                                 accumulate)
                             : sgh_dgrad_split2_run(g, dy, W, dx, workspace, s, accumulate);
   } else if (path == kDgradColumns && sgh_dgrad_few_supported(g)) {
     rc = sgh_dgrad_few_run(g, dy, W, dx, s);
@@ -1456,9 +1461,9 @@ int sgh_conv_fwd_f32(sgh_conv_geom *g, const float *x, const float *W, const flo
     }
   }
   sgh_conv_geom gt;
-  if (fwd_as_split(g, &gt) && ws_bytes >= sgh_conv_split_workspace_bytes(&gt)) {
+  if (const sgh_conv_split_plan p = fwd_split_plan(g, &gt); p.ok && ws_bytes >= p.bytes) {
     int rcs = sgh_conv_split_weights(&gt, W, workspace, false, s);
-    if (rcs == SGH_OK) rcs = sgh_conv_split_run(&gt, x, W, y, workspace, s, "conv_fwd/k_conv_split", false, bias, false);
+    if (rcs == SGH_OK) rcs = sgh_conv_split_run(&gt, p, x, W, y, workspace, s, "conv_fwd/k_conv_split", false, bias, false);
     sgh_prof_stop(s);
     return rcs;
   }

@@ -72,7 +72,8 @@ def launched():
 def kernels():
     '''the kernels' plain names, in order'''
     import re
-    return [re.search(r"\\d+(k_[a-z0-9_]+?)(?=I|E|v|P|$)", n).group(1) if re.search(r"\\d+k_", n) else n for n, _, _ in launched()]
+    found = [(re.search(r"\\d(k_[a-z0-9_]+)", n), n) for n, _, _ in launched()]   # (a name ends at the I, E or P of the mangling)
+    return [m.group(1) if m else n for m, n in found]
 
 
 def conv(*dims):
