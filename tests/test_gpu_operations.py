@@ -1295,12 +1295,13 @@ def test_conv_forward_few_channels_wide_blocks(singa, dev, n, c, h, w, k, r, st,
 
 
 @pytest.mark.parametrize("case", [(1, 1, 1, 1, 1, 3, 1), (3, 3, 8, 32, 5, 5, 2), (2, 3, 9, 33, 32, 5, 2), (2, 2, 31, 65, 7, 3, 1), (3, 4, 17, 40, 9, 5, 0),
-                                  (2, 4, 12, 29, 3, 3, 2), (128, 3, 32, 32, 32, 5, 2)])
+                                  (2, 4, 12, 29, 3, 3, 2), (128, 3, 32, 32, 32, 5, 2), (2, 3, 19, 34, 64, 5, 2), (2, 3, 19, 34, 65, 5, 2)])
 @pytest.mark.parametrize("bad", [0.0, np.inf, np.nan])
 def test_data_gradient_with_few_input_channels(singa, dev, case, bad):
-    """One to four input channels, 3x3 and 5x5 of stride 1 on the vector ALUs: edges of the tiles of 8 x 32, paddings, fewer filters
-    than wavefronts.  Bound: K R^2 products, |error| <= (R^2 + K / 4 + 4) 2^-24 sum |dy w|.  An infinity or NaN of a filter reaches the
-    pixels that it is multiplied with and no others."""
+    """One to four input channels, 3x3 and 5x5 of stride 1, on the vector ALUs up to 64 filters: edges of the tiles of 8 x 32, paddings,
+    fewer filters than wavefronts.  Bound: K R^2 products, |error| <= (R^2 + K / 4 + 4) 2^-24 sum |dy w|; the column GEMM beyond 64
+    filters sums all of them in a chain.  An infinity or NaN of a filter reaches the pixels that it is multiplied with and no others."""
+    from util import kernels_of
     N, C, H, W, K, R, pad = case
     print("few input channels", case, bad, flush=True)
     r = rng(sum(case))
@@ -1310,7 +1311,8 @@ def test_data_gradient_with_few_input_channels(singa, dev, case, bad):
     x = singa.from_numpy(np.zeros((N, C, H, W), np.float32), dev)
     h = singa.CudnnConvHandle(x, (R, R), (1, 1), (pad, pad), C, K, False)
     dy = randn(r, N, K, h.conv_height, h.conv_width)
-    got = singa.GpuConvBackwardx(singa.from_numpy(dy, dev), singa.from_numpy(w, dev), x, h).to_numpy()
+    got, names = kernels_of(dev, lambda: singa.GpuConvBackwardx(singa.from_numpy(dy, dev), singa.from_numpy(w, dev), x, h).to_numpy())
+    assert names == ({"k_dgrad_few"} if K <= 64 else {"k_igemm"}), names
     want, size = np.zeros((N, C, H + 2 * pad, W + 2 * pad)), np.zeros((N, C, H + 2 * pad, W + 2 * pad))
     with np.errstate(invalid="ignore"):
         for i in range(R):
@@ -1322,7 +1324,7 @@ def test_data_gradient_with_few_input_channels(singa, dev, case, bad):
     want, size = want[:, :, cut[0], cut[1]], size[:, :, cut[0], cut[1]]
     ok = np.isfinite(want)
     assert np.array_equal(np.isfinite(got), ok)
-    assert np.all(np.abs(got[ok] - want[ok]) <= (R * R + K / 4 + 4) * 2.0 ** -24 * size[ok])
+    assert np.all(np.abs(got[ok] - want[ok]) <= (R * R + (K / 4 if K <= 64 else K) + 4) * 2.0 ** -24 * size[ok])
 
 
 @pytest.mark.parametrize("shape", [(2, 3, 8, 8), (3, 5, 7, 9), (1, 1, 2, 2), (40, 16, 33, 30)])
