@@ -397,6 +397,40 @@ def test_conv_wgrad_octets_time_of_non_finite_operands(singa, dev, what):
     assert got < 8 * plain
 
 
+@pytest.mark.parametrize("what", ["inf", "one inf", "overflow", "nan", "inf weights"])
+def test_strided_layers_time_of_non_finite_operands(singa, dev, what):
+    """The three passes of a 3x3 layer of stride 2: a second pass over the tiles with results that are not finite, and no search per
+    result."""
+    n, c, h, w, k = 32, 128, 28, 28, 256
+    x, W, _ = operands("normal", 3, n, c, h, w, k, 3)
+    dy = operands("normal", 4, n, k, h // 2, w // 2, 1, 1)[0]
+    kernels = ["k_conv_split", "k_dgrad_split2", "k_wgrad_oct"]
+
+    def times(x, W, dy):
+        xd, wd, dyd = (singa.from_numpy(a, dev) for a in (x, W, dy))
+        hd = singa.CudnnConvHandle(xd, (3, 3), (2, 2), (1, 1), c, k, False)
+        calls = [lambda: singa.GpuConvForward(xd, wd, None, hd), lambda: singa.GpuConvBackwardx(dyd, wd, xd, hd),
+                 lambda: singa.GpuConvBackwardW(dyd, xd, wd, hd)]
+        assert [kernels_of(dev, f)[1] for f in calls] == [{name} for name in kernels]
+        return [seconds(dev, f) for f in calls]
+
+    plain = times(x, W, dy)
+    value = np.float32(np.nan if what == "nan" else np.inf)
+    if what == "one inf":
+        x[:, 0, 7, 7] = value
+        dy[:, 0, 7, 7] = value
+    elif what == "overflow":
+        x, W, dy = x * np.float32(1e30), W * np.float32(1e10), dy * np.float32(1e30)
+    elif what == "inf weights":
+        W[:] = value
+    else:
+        x[:] = value
+        dy[:] = value
+    for name, got, ordinary in zip(kernels, times(x, W, dy), plain):
+        print(name, what, "%.1f us, ordinary operands %.1f" % (got * 1e6, ordinary * 1e6))
+        assert got < 8 * ordinary
+
+
 @pytest.mark.parametrize("small,large", [(2.0 ** -116, 1.0), (2.0 ** -124, 2.0 ** 40), (2.0 ** -132, 2.0 ** 60), (1.0, 2.0 ** -116)])
 def test_conv_split_operands_of_any_magnitude(singa, dev, small, large):
     """Inputs and gradients (or weights) of small magnitude, down to subnormal ones, at the error that ordinary magnitudes have: on
