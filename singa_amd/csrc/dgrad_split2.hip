@@ -24,6 +24,8 @@
 //
 // Neither the taps of a class nor their signs change within a chunk, so the one that the matrix instructions' rounding needs (it
 // leans towards minus infinity) changes from chunk to chunk: in odd ones dy goes negated into the slab and the sums are subtracted.
+#include <atomic>
+
 #include "common.h"
 #include "dgrad_split2.h"
 
@@ -31,7 +33,7 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int NT = 512, NW = NT / 64, KC = 16, R = 3, TAPS = 9;
+constexpr int NT = 512, NW = NT / 64, KC = 16, TAPS = 9;
 constexpr int kOOB = int(0x80000000u);
 constexpr int kPos = 48;              // bytes of a slab position: three parts of eight channels
 constexpr int kFrag = 3 * 1024;       // bytes of a 32-row weight fragment: three parts x 64 lanes x 16 bytes
@@ -393,11 +395,11 @@ S2Plan plan(const sgh_conv_geom *g) {
 template <int GM, int ET>
 int launch(const S2Args &a, const S2Plan &p, hipStream_t s) {
   auto kern = k_dgrad_split2<GM, ET>;
-  static bool attr_set = false;
-  if (!attr_set) {
+  static std::atomic<bool> allowed{false};   // (host threads may come here at once)
+  if (!allowed.load(std::memory_order_relaxed)) {
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
       return SGH_EUNSUPPORTED;
-    attr_set = true;
+    allowed.store(true, std::memory_order_relaxed);
   }
   SGH_LAUNCH_TIMED(kern, dim3(unsigned(p.wgs)), dim3(NT), size_t(p.slab) * 4 * kPos, s, a);
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
