@@ -12,7 +12,8 @@ per-step HIP event times as extra keys) plus
   roofline     -- the dominant kernel family (conv dgrad + wgrad kernels on matrix instructions):
                   algorithmic FLOPs / measured kernel time (HIP events on the kernels' stream),
                   against the MI355X fp32 matrix peak (the kernels on split operands form six
-                  bfloat16 products for an fp32 one: `peak_split` is their ceiling); `traffic` =
+                  bfloat16 products for an fp32 one: `peak_split` is their ceiling, and
+                  `frac_of_each_kernels_peak` takes every kernel against its own); `traffic` =
                   HBM bytes per step of the same launches, read from the rocprofv3 counter summary
                   under profiles/ when that summary was taken on the kernels this run launched
                   (null otherwise);
@@ -35,6 +36,7 @@ if ROOT not in sys.path:
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_16BIT_MFMA_TFLOPS = 2500.0   # dense fp16 / bf16 matrix peak
 PEAK_HBM_GBS = 8000.0
+SPLIT_KERNELS = ("k_conv_split", "k_dgrad_split2", "k_wgrad_oct")   # six bfloat16 products for an fp32 one
 # HBM bytes the conv dgrad/wgrad MFMA launches of one step move (fetched + written) come from two
 # rocprofv3 --pmc runs of this script (FETCH_SIZE, WRITE_SIZE), summarised in this file together with the
 # workload and the kernels the figure covers; it is quoted only for a run that launched exactly those kernels.
@@ -54,12 +56,13 @@ def collect_prof(lib):
         if rc != 0:
             raise RuntimeError("sgh_prof_get rc=%d" % rc)
         cls, _, kern = buf.value.decode().partition("/")
-        d = out.setdefault(cls, {"launches": 0, "ms": 0.0, "work": 0.0, "kernels": set()})
+        d = out.setdefault(cls, {"launches": 0, "ms": 0.0, "work": 0.0, "kernels": set(), "work_of": {}})
         d["launches"] += 1
         d["ms"] += ms.value
         d["work"] += work.value
         if kern:
             d["kernels"].add(kern)
+            d["work_of"][kern] = d["work_of"].get(kern, 0.0) + work.value
     return out
 
 
@@ -277,11 +280,14 @@ def main():
     kernels = sorted(set().union(*[v["kernels"] for v in conv.values()])) if conv else []
     achieved = flop / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
     peak = PEAK_16BIT_MFMA_TFLOPS if half else PEAK_FP32_MFMA_TFLOPS
+    # the time that the products take at the peak of the instructions that form them, over the kernels' time
+    at_peak = sum(w / (PEAK_16BIT_MFMA_TFLOPS / 6 if not half and k in SPLIT_KERNELS else peak)
+                  for v in conv.values() for k, w in v["work_of"].items()) * 1e-9
     workload_key = "%s N=%d %s%s" % (args.config, args.batch, args.storage, " no-fusion" if args.no_fusion else "")
     roofline = {
         "bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
         "peak_split": None if half else round(PEAK_16BIT_MFMA_TFLOPS / 6, 1),
-        "frac": round(achieved / peak, 4),
+        "frac": round(achieved / peak, 4), "frac_of_each_kernels_peak": round(at_peak / ms, 4) if ms > 0 else 0.0,
         "traffic": traffic_from_profile(workload_key, kernels),
         "traffic_unit": "HBM bytes per step over the same launches (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated on a "
                         "streaming kernel; from profiles/%s, null when that summary covers other kernels or another workload)"

@@ -161,7 +161,7 @@ int sgh_fwd_few_run(const sgh_conv_geom *g, const float *x, const float *W, cons
 bool sgh_dgrad_few_supported(const sgh_conv_geom *g);
 int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, float *dx, hipStream_t s);
 
-// fp32 3x3 stride-1 pad-1 weight gradient on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
+// fp32 3x3 pad-1 weight gradient, stride 1 or 2, on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
 // take; the caller checks that the workspace has them.
 size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);
 int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s);

@@ -841,7 +841,7 @@ def GpuConvBackwardxAccumulate(dy, W, x, h, dx):
     gradient where the kernel supports it, otherwise the two separate steps."""
     h._check_dy(dy)
     _same(dx, x)
-    if dy.data_type() == kFloat32:   # (on 16-bit tensors the kernel's read-modify-write loses to the separate add)
+    if dy.data_type() == kFloat32:   # (16-bit tensors: GpuConvBackwardxAddReLU)
         rc = _L().sgh_conv_dgrad_acc_f32(_address(h.geom), dy.ptr, W.ptr, dx.ptr, h.workspace.ptr,
                                          h.workspace.MemSize(), dy.device().stream)
         if rc != _lib.SGH_EUNSUPPORTED:

@@ -303,8 +303,8 @@ class HalfHipOps(HipOps):
     (binary16 or bfloat16), BatchNorm parameters / statistics and the classifier head stay fp32,
     16-bit weights are updated through fp32 master copies."""
 
-    # the residual "+=": folded into the next ReLU backward (the 16-bit data-gradient kernel's
-    # scattered 2-byte stores make a read-modify-write epilogue slower than the separate add)
+    # the residual "+=": with the ReLU gate behind it in the store of the 1x1 data gradient, which goes out in 16-byte rows, or folded into the
+    # next ReLU backward (onto the gradient that is there, element by element, it was slower than the separate add)
     fuse_dgrad_add = False
     fuse_add_relu = True
     fuse_dgrad_relu = True
