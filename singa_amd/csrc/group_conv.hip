@@ -81,12 +81,13 @@ __device__ __forceinline__ rsrc_t buffer_of(const typename S::elem *p, unsigned 
 
 // Source rows of `planes` consecutive planes (first plane `plane0`, those from `planes_end` on are zero) into LDS as
 // [plane][VR][VC]; row 0 of the virtual image is virtual row `vrow0`.  Returns whether this thread met an infinity or a NaN.
-template <class S>
+// (QUADS: loads of four columns in flight, 0 if a.QN is never set)
+template <class S, int QUADS>
 __device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsrc_t src, int plane0, int planes, int plane_step,
                                              int planes_end, int vrow0) {
-  constexpr int U = 4;
   float zero = 0.f;   // until it has been multiplied with an infinity or a NaN
-  if (a.QN) {
+  if constexpr (QUADS > 0) if (a.QN) {
+    constexpr int U = QUADS;
     // four columns per load (the last four of a row overlap the ones before): 2 700 values of three 28 x 28 planes are one round
     // of loads, where one value per load and two divisions each were three (depthwise 3x3 on
     // 32 x 96 x 28 x 28: 9.4 -> 8.0 us a pass)
@@ -120,6 +121,7 @@ __device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsr
     }
     return zero != 0.f;
   }
+  constexpr int U = 4;
   const int total = planes * a.VR * a.VC;
   for (int i0 = threadIdx.x; i0 < total; i0 += GT * U) {
     float v[U];
@@ -152,8 +154,9 @@ __device__ __forceinline__ bool stage_planes(float *lds, const GroupArgs &a, rsr
 // zero-padded image does; the data gradient has no padding in its definition, and with such a filter in LDS (`odd`) the
 // positions that hold no gradient are left out one by one.
 
-// R: filter height and width; T: output stride
-template <class S, int R, int T>
+// R: filter height and width; T: output stride; QUADS: see stage_planes (a 1x1 data gradient of stride 2, which has nothing else to do, takes
+// 14.3 us without that code in it and 16.4 with it: 53 images, 40 filters of 18 x 14 onto 48 channels, eight groups)
+template <class S, int R, int T, int QUADS>
 __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__restrict__ src, const typename S::elem *__restrict__ W,
                                                    const typename S::elem *__restrict__ bias, typename S::elem *__restrict__ dst,
                                                    const GroupArgs a) {
@@ -167,7 +170,7 @@ __global__ __launch_bounds__(GT) void k_group_conv(const typename S::elem *__res
   const int u0 = int(blockIdx.x) * a.UB, p0 = int(blockIdx.y) * a.TP;
   const int ub = a.units - u0 < a.UB ? a.units - u0 : a.UB;
   float *image = lds, *filt = lds + a.UB * a.cs * a.VR * a.VC;
-  stage_planes<S>(image, a, buffer_of<S>(src, a.src_bytes), u0 * a.cs, a.UB * a.cs, 1, ub * a.cs, p0 * T);
+  stage_planes<S, QUADS>(image, a, buffer_of<S>(src, a.src_bytes), u0 * a.cs, a.UB * a.cs, 1, ub * a.cs, p0 * T);
   // filters as [unit][destination channel][source channel][tap]
   const int nf = ub * a.cd * a.cs * RS;
   for (int i = threadIdx.x; i < nf; i += GT) {
@@ -275,14 +278,20 @@ __global__ __launch_bounds__(GT) void k_group_wgrad(const typename S::elem *__re
         for (int o = 0; o < STRIP; ++o) w.d[o] = ld_elem<S>(ys, w.first + o * a.DW, it < items && w.p + o < pe);
         return w;
       };
-      Item next = request(threadIdx.x);   // before x, not behind the barrier, and one item ahead from there on: 12 -> 10.2 us
+      // Up to 3x3 dy is requested before x, not behind the barrier, and one item ahead from there on: 12 -> 10.2 us.  With 25 sums and
+      // more that costs the registers of one or two wavefronts per SIMD, as do four loads of four columns in flight with 25: 5x5 on
+      // 28 x 91 x 25 x 27 17.1 us as here, 22.3 with both.
+      constexpr bool AHEAD = R <= 3;
+      [[maybe_unused]] Item next;
+      if constexpr (AHEAD) next = request(threadIdx.x);
       __syncthreads();   // (the previous tile has been read)
-      if (stage_planes<S>(lds, a, xs, n0 * C + g * a.cs + cl, a.UB, C, ub, p0 * T)) odd = 1;
+      if (stage_planes<S, R == 5 ? 2 : 4>(lds, a, xs, n0 * C + g * a.cs + cl, a.UB, C, ub, p0 * T)) odd = 1;
       __syncthreads();
       const bool select = odd != 0;
       for (int it = threadIdx.x; it < items; it += GT) {
-        const Item w = next;
-        next = request(it + GT);
+        Item w;
+        if constexpr (AHEAD) w = next, next = request(it + GT);
+        else w = request(it);
         const float *im = lds + w.image;
         if (!select) {
 #pragma unroll
@@ -425,7 +434,10 @@ void launch(const Plan &p, const sgh_conv_geom *g, int which, const void *a, con
   E *eo = static_cast<E *>(out);
   if (which != SGH_CONV_WGRAD) {
     const dim3 grid((p.a.units + p.a.UB - 1) / p.a.UB, (p.a.DH + p.a.TP - 1) / p.a.TP);
-    hipLaunchKernelGGL((k_group_conv<S, R, T>), grid, dim3(GT), p.lds, s, ea, eb, static_cast<const E *>(bias), eo, p.a);
+    auto kern = k_group_conv<S, R, T, 4>;
+    if constexpr (R == 1)
+      if (!p.a.QN) kern = k_group_conv<S, R, T, 0>;
+    hipLaunchKernelGGL(kern, grid, dim3(GT), p.lds, s, ea, eb, static_cast<const E *>(bias), eo, p.a);
     return;
   }
   const int pairs = g->K * p.a.cs, n = pairs * R * R;
