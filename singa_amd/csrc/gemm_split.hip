@@ -81,12 +81,13 @@ __device__ __forceinline__ void sum_columns(const float *__restrict__ m, int ld,
   out[j] = s;
 }
 
-template <bool AK, bool BKc, int T, int W>
+// (AROUND: `around` is not empty.  Its tests in the plain product's store cost every fp32 GEMM 0.2 to 0.5 us)
+template <bool AK, bool BKc, int T, int W, bool AROUND>
 __global__ __launch_bounds__(W * 64) void k_gemm_split(const float *__restrict__ A, int lda, unsigned a_bytes,
                                                        const float *__restrict__ B, int ldb, unsigned b_bytes,
                                                        float *__restrict__ C, long ldc, int M, int N, int K, int kq, float alpha,
                                                        float beta, sgh_gemm_around around) {
-  if constexpr (!BKc) {
+  if constexpr (AROUND && !BKc) {
     if (around.colsum && blockIdx.y == gridDim.y - 1) {   // (a row of workgroups of its own, beside the tiles)
       sum_columns<T>(B, ldb, K, N, blockIdx.x * T, around.colsum);
       return;
@@ -135,9 +136,11 @@ __global__ __launch_bounds__(W * 64) void k_gemm_split(const float *__restrict__
     if (m0 + row < M && n0 + col < N) {
       float *p = C + size_t(m0 + row) * ldc + n0 + col;
       float r = beta == 0.f ? alpha * v : alpha * v + beta * *p;
-      if (around.bias) r += around.bias[n0 + col];
-      if (around.relu) r = r >= 0.f ? r : 0.f;
-      if (around.gate) r = around.gate[size_t(m0 + row) * N + n0 + col] > 0.f ? r : 0.f;
+      if constexpr (AROUND) {
+        if (around.bias) r += around.bias[n0 + col];
+        if (around.relu) r = r >= 0.f ? r : 0.f;
+        if (around.gate) r = around.gate[size_t(m0 + row) * N + n0 + col] > 0.f ? r : 0.f;
+      }
       *p = r;
     }
   }
@@ -150,14 +153,21 @@ void launch(int tile, int waves, const float *A, int lda, const float *B, int ld
   const unsigned ab = unsigned((size_t(AK ? M - 1 : K - 1) * lda + (AK ? K : M)) * 4);
   const unsigned bb = unsigned((size_t(BKc ? N - 1 : K - 1) * ldb + (BKc ? K : N)) * 4);
   const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile + (around.colsum ? 1 : 0));
-#define SGH_SPLIT_CASE(T_, W_)                                                                                                     \
-  hipLaunchKernelGGL((k_gemm_split<AK, BKc, T_, W_>), grid, dim3(W_ * 64), 0, s, A, lda, ab, B, ldb, bb, C, long(ldc), M, N, K, kq, \
-                     alpha, beta, around)
+  const bool plain = !around.bias && !around.gate && !around.colsum && !around.relu;
+#define SGH_SPLIT_KERNEL(T_, W_, AROUND_)                                                                                           \
+  hipLaunchKernelGGL((k_gemm_split<AK, BKc, T_, W_, AROUND_>), grid, dim3(W_ * 64), 0, s, A, lda, ab, B, ldb, bb, C, long(ldc), M,  \
+                     N, K, kq, alpha, beta, around)
+#define SGH_SPLIT_CASE(T_, W_)                                \
+  do {                                                        \
+    if (plain) SGH_SPLIT_KERNEL(T_, W_, false);               \
+    else if constexpr (AK || !BKc) SGH_SPLIT_KERNEL(T_, W_, true);   /* (no layer has both operands transposed) */ \
+  } while (0)
   if (tile == 16 && waves == 8) SGH_SPLIT_CASE(16, 8);
   else if (tile == 16) SGH_SPLIT_CASE(16, 4);
   else if (waves == 16) SGH_SPLIT_CASE(32, 16);
   else if (waves == 8) SGH_SPLIT_CASE(32, 8);
   else SGH_SPLIT_CASE(32, 4);
+#undef SGH_SPLIT_KERNEL
 #undef SGH_SPLIT_CASE
 }
 
