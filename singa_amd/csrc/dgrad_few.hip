@@ -2,11 +2,11 @@
 //   dx[n][c][h][w] = sum_k sum_{r,s} dy[n][k][h + pad - r][w + pad - s] * W[k][c][r][s]
 // On matrix tiles such a layer fills 4 of 32 rows; as one GEMM into columns and a gather (igemm.hip) it writes and reads a matrix of
 // R * S times dx: 128 images of 3 channels of 32 x 32, 5x5 to 32 filters, 32 + 18 us.  Its products are few enough for the vector ALUs.
-//   A workgroup of four wavefronts owns 8 x 32 pixels of an image, all channels; wavefront v takes the filters v, v + 4, ...: it stages
+//   A workgroup of four or eight wavefronts owns 8 x 32 pixels of an image, all channels; wavefront v of n takes the filters v, v + n, ...: it stages
 // its own 12 x 36 pixels of dy[n][k] in LDS (the next filter's on their way in registers, no barrier), a lane computes four neighbouring
 // pixels of every channel, 300 products on 40 values from LDS, with the filter in scalar registers.  A filter's taps are summed on their
 // own and added to the lane's sums with one rounding, and the wavefronts' sums are added in order.
-// Bound by the vector ALUs and, where a CU has few workgroups, by the chain of a filter (LDS, scalar loads, 144 to 300 products: 0.85 us).
+// Bound by the vector ALUs and, where a CU has few workgroups, by the chain of a filter (LDS, scalar loads, 144 to 400 products: 0.6 to 1.1 us).
 // That layer 43.8 -> 18.3 us, 67 x 1 x 30 x 36, 5x5 to 17 26.7 -> 8.2, 111 x 2 x 47 x 37, 3x3 to 191 74 -> 64; error 0.5 to 1.0 times.
 // The data gradient has no padding in its definition: with an infinity or a NaN in the filter the taps that fall outside dy are left out
 // one by one.
@@ -14,7 +14,7 @@
 
 namespace {
 
-constexpr int TH = 8, TW = 32, NT = 256;   // a lane: row lane / 8, columns 4 (lane % 8) .. + 3
+constexpr int TH = 8, TW = 32;   // a lane: row lane / 8, columns 4 (lane % 8) .. + 3
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
@@ -25,11 +25,11 @@ struct Args {
   unsigned dy_bytes;
 };
 
-template <int C, int R>
-__global__ __launch_bounds__(NT) void k_dgrad_few(Args a) {
+template <int C, int R, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void k_dgrad_few(Args a) {
   constexpr int VR = TH + R - 1, VC = TW + R - 1, PITCH = (VC + 3) & ~3, E = (VR * VC + 63) / 64, RS = R * R;
-  __shared__ __align__(16) float tiles[4][VR * PITCH + 4];
-  __shared__ float sums[3][C * 4][64];
+  __shared__ __align__(16) float tiles[WAVES][VR * PITCH + 4];
+  __shared__ float sums[WAVES - 1][C * 4][64];
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int strip = int(blockIdx.x) % a.strips, rest = int(blockIdx.x) / a.strips, band = rest % a.bands, n = rest / a.bands;
   const int h0 = band * TH, w0 = strip * TW;
@@ -56,10 +56,10 @@ __global__ __launch_bounds__(NT) void k_dgrad_few(Args a) {
   for (int c = 0; c < C; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int row = lane >> 3, col = 4 * (lane & 7);
   request(wave);
-  for (int k = wave; k < a.K; k += 4) {
+  for (int k = wave; k < a.K; k += WAVES) {
 #pragma unroll
     for (int e = 0; e < E; ++e) tile[at[e]] = next[e];
-    request(k + 4);
+    request(k + WAVES);
     const float *w = a.W + size_t(k) * C * RS;   // (uniform)
     // x * 0 is not zero for an infinity or a NaN
     float zero = 0.f;
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(NT) void k_dgrad_few(Args a) {
     for (int e = 0; e < 4; ++e) {
       float v = acc[c][e];
 #pragma unroll
-      for (int w = 0; w < 3; ++w) v += sums[w][c * 4 + e][lane];
+      for (int w = 0; w < WAVES - 1; ++w) v += sums[w][c * 4 + e][lane];
       if (w0 + col + e < a.Wd) out[e] = v;
     }
   }
@@ -131,9 +131,9 @@ __global__ __launch_bounds__(NT) void k_dgrad_few(Args a) {
 
 }  // namespace
 
-// Up to 64 filters: the columns' reduction runs on the matrix instructions, here a wavefront walks a quarter of the filters one by one.  Over 34
-// drawn layers none of up to 67 filters is slower (50 x 3 x 42 x 53 to 140 43.8 / 39.6, 3 x 3 x 102 x 102 to 62 17.6 / 16.6), beyond, few
-// images are: 1 x 3 x 61 x 77, 5x5 to 79 23.0 / 26.5, 3 x 4 x 32 x 30 to 167 22.9 / 35.3, 13 x 4 x 32 x 22 to 964 84 / 222.
+// Up to 64 filters: the columns' reduction runs on the matrix instructions, here a wavefront walks its share of the filters one by one.  Beyond,
+// few images are slower on four wavefronts: 1 x 3 x 61 x 77, 5x5 to 79 23.0 / 26.5, 3 x 4 x 32 x 30 to 167 22.9 / 35.3, 13 x 4 x 32 x 22 to 964
+// 84 / 222.
 bool sgh_dgrad_few_supported(const sgh_conv_geom *g) {
   const size_t lim = size_t(1) << 31, wgs = size_t(g->N) * ((g->H + TH - 1) / TH) * ((g->W + TW - 1) / TW);
   return wgs < size_t(1) << 24 &&   // (a launch holds less than 2^32 threads)
@@ -146,9 +146,20 @@ int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, f
          unsigned(size_t(g->N) * g->K * g->P * g->Q * 4)};
   const dim3 grid(unsigned(g->N) * unsigned(a.bands) * unsigned(a.strips));
   sgh_prof_kernel_scope prof("conv_dgrad/k_dgrad_few", 2.0 * g->N * g->K * g->P * g->Q * double(g->C) * g->R * g->S, s);
-#define SGH_FEW(C_) \
-  if (g->R == 3) SGH_LAUNCH_TIMED((k_dgrad_few<C_, 3>), grid, dim3(NT), 0, s, a); \
-  else SGH_LAUNCH_TIMED((k_dgrad_few<C_, 5>), grid, dim3(NT), 0, s, a)
+  const long wgs = long(grid.x), cus = sgh_num_cus();
+  // Eight wavefronts halve the chain of a workgroup that has its CU to itself, or shares it with one or two: us in columns / on four / eight, 5x5,
+  // 2 x 4 x 16 x 13 to 64 (bfloat16) 27.5 / 34.5 / 25.6, 5 x 4 x 21 x 21 to 61 21.1 / 23.9 / 19.4, 16 x 4 x 17 x 17 to 63 30.3 / 35.2 / 27.4; with
+  // four, 73 of 500 layers of 40 to 64 filters were slower than in columns.  Beyond, the vector ALUs are busy either way (15 x 4 x 57 x 78, 3x3 to
+  // 10 5.9 / 6.7, 13 x 3 x 96 x 112 to 44 16.3 / 17.6).
+  const bool eight = (wgs <= cus && g->K > 8) || (wgs <= (g->R == 5 ? 3 : 2) * cus && g->K > 24);
+#define SGH_FEW_KERNEL(C_, R_)                                                             \
+  do {                                                                                     \
+    if (eight) SGH_LAUNCH_TIMED((k_dgrad_few<C_, R_, 8>), grid, dim3(512), 0, s, a);       \
+    else SGH_LAUNCH_TIMED((k_dgrad_few<C_, R_, 4>), grid, dim3(256), 0, s, a);             \
+  } while (0)
+#define SGH_FEW(C_)                  \
+  if (g->R == 3) SGH_FEW_KERNEL(C_, 3); \
+  else SGH_FEW_KERNEL(C_, 5)
   switch (g->C) {
     case 1: SGH_FEW(1); break;
     case 2: SGH_FEW(2); break;
@@ -156,5 +167,6 @@ int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, f
     default: SGH_FEW(4); break;
   }
 #undef SGH_FEW
+#undef SGH_FEW_KERNEL
   return hipGetLastError() == hipSuccess ? SGH_OK : SGH_EINVAL;
 }
