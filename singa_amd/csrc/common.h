@@ -162,9 +162,10 @@ bool sgh_dgrad_few_supported(const sgh_conv_geom *g);
 int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, float *dx, hipStream_t s);
 
 // fp32 3x3 pad-1 weight gradient, stride 1 or 2, on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
-// take; the caller checks that the workspace has them.
-size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g);
-int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s);
+// take; the caller checks that the workspace has the least of them.  (More of it: more, shorter workgroups where that is faster.)
+size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g, bool least);
+int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, size_t ws_bytes,
+                      hipStream_t s);
 // The same of 16-bit tensors, stride 1 or 2 (wgrad_oct16.hip)
 size_t sgh_wgrad_oct16_workspace_bytes(const sgh_conv_geom *g);
 double sgh_wgrad_oct16_us(const sgh_conv_geom *g);   // its expected time

@@ -1059,7 +1059,7 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
     split = p.ok ? p.bytes : 0;
   }
   if (which == SGH_CONV_DGRAD) split = dgrad_split_bytes(g);
-  if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g);
+  if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g, false);
   return split > plain ? split : plain;
 }
 
@@ -1522,7 +1522,7 @@ static int bgrad_launch(const sgh_conv_geom *g, const float *dy, float *db, hipS
 
 // The octet kernel runs where the workspace holds its partial images
 static bool wgrad_by_octets(const sgh_conv_geom *g, const void *workspace, size_t ws_bytes) {
-  const size_t need = sgh_wgrad_oct_workspace_bytes(g);
+  const size_t need = sgh_wgrad_oct_workspace_bytes(g, true);
   return need && workspace && ws_bytes >= need;
 }
 
@@ -1539,7 +1539,7 @@ static int conv_wgrad(sgh_conv_geom *g, const float *dy, const float *x, float *
   sgh_prelaid_clear_if_overlap(g, workspace, ws_bytes);
   if (wgrad_by_octets(g, workspace, ws_bytes)) {
     sgh_prof_start("conv_wgrad_op", conv_flops(g), sgh_stream_of(stream));
-    const int rco = sgh_wgrad_oct_run(g, dy, x, dW, workspace, sgh_stream_of(stream));
+    const int rco = sgh_wgrad_oct_run(g, dy, x, dW, workspace, ws_bytes, sgh_stream_of(stream));
     sgh_prof_stop(sgh_stream_of(stream));
     return rco == SGH_OK && db ? bgrad_launch(g, dy, db, sgh_stream_of(stream)) : rco;
   }

@@ -460,7 +460,10 @@ struct WoPlan {
   int st, ocs, rpi, ktiles, tiles, splits, strips, iters, per_split;
 };
 
-WoPlan plan(const sgh_conv_geom *g) {
+size_t image_bytes(const WoPlan &p) { return size_t(p.splits) * p.tiles * 4 * kAcc * sizeof(float); }
+
+// `room`: bytes for the partial images
+WoPlan plan(const sgh_conv_geom *g, size_t room) {
   WoPlan p{};
   p.st = g->stride_h;
   if (g->R != 3 || g->S != 3 || p.st < 1 || p.st > 2 || g->stride_w != p.st || g->pad_h != 1 || g->pad_w != 1) return p;
@@ -485,11 +488,31 @@ WoPlan plan(const sgh_conv_geom *g) {
   const int cus = sgh_num_cus();
   // one workgroup per CU, two iterations at least for either of its groups
   const long most = p.iters / 4 > 0 ? p.iters / 4 : 1;
-  long sp = cus / (tiles * p.strips);
-  if (sp > most) sp = most;
-  if (sp < 1) sp = 1;
-  p.per_split = int((p.iters + sp - 1) / sp);
-  p.splits = (p.iters + p.per_split - 1) / p.per_split * p.strips;
+  auto split = [&](long sp) {
+    if (sp > most) sp = most;
+    if (sp < 1) sp = 1;
+    p.per_split = int((p.iters + sp - 1) / sp);
+    p.splits = (p.iters + p.per_split - 1) / p.per_split * p.strips;
+  };
+  const long one = cus / (tiles * p.strips);
+  split(one);
+  // Stride 2, more than a quarter as many tiles and strips as CUs: one to three splits of them leave up to half of the CUs idle in their only or
+  // last round.  Up to three rounds of shorter workgroups do not, if there is room for their images: 35 images, 654 channels of 31 x 36 to 344,
+  // 132 workgroups 1017 us, 660 of them 661 (k_wgrad3x3 766); 7 of 811, 73 x 70, to 488 980 -> 751 (the generic kernel 887); 4 of 299, 88 x 107,
+  // to 417 344 -> 258.  (us, fitted over 96 layers: 3.6 for an iteration of either group, 0.06 for an image written and summed.)
+  if (p.st == 2 && one < 4) {
+    auto us = [&] {
+      const long wgs = tiles * p.splits;
+      return double((wgs + cus - 1) / cus) * ((p.per_split + 1) / 2) * 3.6 + 0.06 * double(wgs);
+    };
+    WoPlan best = p;
+    double least = us();
+    for (long sp = one + 1; sp * tiles * p.strips <= 3l * cus && sp <= most; ++sp) {
+      split(sp);
+      if (us() < least && image_bytes(p) <= room) least = us(), best = p;
+    }
+    p = best;
+  }
   p.ok = true;
   return p;
 }
@@ -510,13 +533,14 @@ int launch(const WoArgs &a, hipStream_t s) {
 
 }  // namespace
 
-size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g) {
-  const WoPlan p = plan(g);
-  return p.ok && !sgh_env().conv_split_off ? size_t(p.splits) * p.tiles * 4 * kAcc * sizeof(float) : 0;
+size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g, bool least) {
+  const WoPlan p = plan(g, least ? 0 : size_t(-1));
+  return p.ok && !sgh_env().conv_split_off ? image_bytes(p) : 0;
 }
 
-int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, hipStream_t s) {
-  const WoPlan p = plan(g);
+int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, size_t ws_bytes,
+                      hipStream_t s) {
+  const WoPlan p = plan(g, ws_bytes);
   if (!p.ok) return SGH_EUNSUPPORTED;
   WoArgs a;
   a.dy = dy, a.x = x, a.partial = static_cast<float *>(workspace);

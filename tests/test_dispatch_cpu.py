@@ -138,3 +138,39 @@ plain, strided = call(1), call(2)
 answer([min(time_of(strided) for _ in range(15)) / min(time_of(plain) for _ in range(15)) for _ in range(5)])
 """)
     assert min(ratios) < 2.5, ratios
+
+
+def test_strided_weight_gradients_fill_the_chip_where_their_workspace_allows():
+    """132 tiles and strips of a layer of stride 2 are 132 workgroups on 256 CUs, or, with room for their partial images, more and shorter
+    ones; a workspace for the 132 still runs them, less is refused (the fp32 kernel wants more).  Layers of few tiles have the workgroups
+    that they had."""
+    full, least, less, few = recorded("""
+which = _lib.SGH_CONV_WGRAD
+def run(g, size):
+    if lib.sgh_conv_wgrad_f32(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, size, None) == -2:   # SGH_EWORKSPACE
+        return None
+    (name, grid, _), *_rest = launched()
+    return "k_wgrad_oct" in name, grid[0]
+g = conv(35, 654, 31, 36, 344, 3, 3, 2, 2, 1, 1)
+image = 9 * 64 * 64 * 4
+few = conv(64, 64, 56, 56, 128, 3, 3, 2, 2, 1, 1)
+answer([run(g, lib.sgh_conv_workspace_bytes(C.byref(g), which)) + (lib.sgh_conv_workspace_bytes(C.byref(g), which) // image,),
+        run(g, 132 * image), run(g, 132 * image - 4), run(few, lib.sgh_conv_workspace_bytes(C.byref(few), which))])
+""")
+    assert full[0] and full[1] == full[2] and 400 < full[1] <= 768, full
+    assert least == [True, 132], least
+    assert less is None and few == [True, 256], (less, few)
+
+
+def test_wavefronts_of_data_gradients_onto_few_channels():
+    """Eight where a workgroup has its CU to itself, or nearly, and filters for them; four where the chip is full."""
+    got = recorded("""
+def threads(n, c, h, w, k, r):
+    g = conv(n, c, h, w, k, r, r, 1, 1, r // 2, r // 2)
+    assert lib.sgh_conv_dgrad_f32(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, None, 0, None) == 0
+    (_, _, t), = launched()
+    return t
+answer([threads(2, 4, 16, 13, 64, 5), threads(16, 4, 17, 17, 63, 5), threads(128, 3, 32, 32, 32, 5), threads(1, 3, 8, 8, 8, 3),
+        threads(15, 4, 57, 78, 10, 3), threads(13, 3, 96, 112, 44, 3), threads(128, 4, 112, 112, 64, 5)])
+""")
+    assert got == [512, 512, 512, 256, 256, 256, 256], got

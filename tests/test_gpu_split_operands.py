@@ -311,7 +311,8 @@ def test_conv_wgrad_octets_infinities_and_nans(singa, dev, n, c, h, w, k):
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-3)
 
 
-@pytest.mark.parametrize("n,c,h,w,k", [(30, 256, 14, 13, 256), (40, 150, 22, 31, 96), (20, 100, 41, 40, 260), (8, 128, 50, 57, 140), (6, 62, 97, 120, 80)])
+@pytest.mark.parametrize("n,c,h,w,k", [(30, 256, 14, 13, 256), (40, 150, 22, 31, 96), (20, 100, 41, 40, 260), (8, 128, 50, 57, 140), (6, 62, 97, 120, 80),
+                                       (20, 520, 17, 34, 500)])   # (the last: 144 tiles and strips, split over three rounds of workgroups)
 def test_weight_gradient_of_stride_two_by_octets(singa, dev, n, c, h, w, k):
     """3x3 weight gradients of stride 2 and padding 1, one strip and several, odd and even planes, against float64: within terms * 2^-23 of
     the sum of the terms' magnitudes, and closer than a sixteenth of the roundings of chains of fp32 additions (0.5 * sqrt(terms) * 2^-24, and
