@@ -151,6 +151,7 @@ int sgh_conv_bgrad_run(const sgh_conv_geom *g, const void *dy, void *db, int dty
 // 3x3 (stride 1 or 2) weight gradient with a shared LDS input tile (wgrad3x3.hip).  *_run returns
 // SGH_EUNSUPPORTED for geometries it does not cover; *_workspace_bytes is 0 for those.
 size_t sgh_wgrad3x3_workspace_bytes(const sgh_conv_geom *g);
+double sgh_wgrad3x3_us(const sgh_conv_geom *g);
 int sgh_wgrad3x3_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace,
                      size_t ws_bytes, hipStream_t s);
 
@@ -164,6 +165,7 @@ int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, f
 // fp32 3x3 pad-1 weight gradient, stride 1 or 2, on split operands (wgrad_oct.hip).  *_workspace_bytes is 0 for geometries it does not
 // take; the caller checks that the workspace has the least of them.  (More of it: more, shorter workgroups where that is faster.)
 size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g, bool least);
+double sgh_wgrad_oct_us(const sgh_conv_geom *g);   // its expected time, stride 2
 int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, size_t ws_bytes,
                       hipStream_t s);
 // The same of 16-bit tensors, stride 1 or 2 (wgrad_oct16.hip)

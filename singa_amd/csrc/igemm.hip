@@ -24,6 +24,8 @@
 // perform im2col on the fly: no column matrix is ever materialised.
 #include <stdlib.h>
 
+#include <cmath>
+
 #include "common.h"
 #include "conv_split.h"
 #include "dgrad_split2.h"
@@ -1049,6 +1051,24 @@ static size_t plain_workspace_bytes(const sgh_conv_geom *g, int which) {
   }
 }
 
+// Whether the octet kernel takes the weight gradient of a layer where it can: always at stride 1.  At stride 2 it is 1.5 times as fast as
+// the fp32 kernels in the mean, with less error, but an octet half beyond a row of few pixels, or tiles half empty, is work for
+// nothing: 98 images, 84 channels of 16 x 17, to 380 93 us, 68 on k_wgrad3x3; 90 of 731, 8 x 7, to 904 334, 290 on the generic kernel; 69 of 42,
+// 89 x 67, to 116 161, 140.  The expected times tell those from the rest to 10 per cent (5 of 190 drawn layers).
+static bool octets_pay(const sgh_conv_geom *g) {
+  if (!sgh_wgrad_oct_workspace_bytes(g, true)) return false;
+  if (g->stride_h == 1) return true;
+  double other = sgh_wgrad3x3_us(g);
+  if (other == 0) {
+    const WgradPlan p = plan_wgrad(g);
+    const int CRS = g->C * 9;
+    const double wgs = double((g->K + p.bm - 1) / p.bm) * ((CRS + p.bn - 1) / p.bn) * p.splits, cus = sgh_num_cus();
+    other = 12 + p.chunks_per_split * std::ceil(wgs / cus) * 1.55 * p.bm * p.bn / 16384 +
+            (p.splits > 1 ? double(p.splits) * g->K * CRS / 1e6 : 0);
+  }
+  return 0.9 * sgh_wgrad_oct_us(g) <= other;
+}
+
 size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
   const size_t plain = plain_workspace_bytes(g, which);
   if (!conv_ok(g) || g->groups > 1) return plain;
@@ -1059,7 +1079,7 @@ size_t sgh_conv_workspace_bytes(const sgh_conv_geom *g, int which) {
     split = p.ok ? p.bytes : 0;
   }
   if (which == SGH_CONV_DGRAD) split = dgrad_split_bytes(g);
-  if (which == SGH_CONV_WGRAD) split = sgh_wgrad_oct_workspace_bytes(g, false);
+  if (which == SGH_CONV_WGRAD && octets_pay(g)) split = sgh_wgrad_oct_workspace_bytes(g, false);
   return split > plain ? split : plain;
 }
 
@@ -1522,8 +1542,7 @@ static int bgrad_launch(const sgh_conv_geom *g, const float *dy, float *db, hipS
 
 // The octet kernel runs where the workspace holds its partial images
 static bool wgrad_by_octets(const sgh_conv_geom *g, const void *workspace, size_t ws_bytes) {
-  const size_t need = sgh_wgrad_oct_workspace_bytes(g, true);
-  return need && workspace && ws_bytes >= need;
+  return workspace && octets_pay(g) && ws_bytes >= sgh_wgrad_oct_workspace_bytes(g, true);
 }
 
 // `db` (may be null): the bias gradient as well.  In the generic kernel it rides along as one more column

@@ -460,6 +460,12 @@ struct WoPlan {
   int st, ocs, rpi, ktiles, tiles, splits, strips, iters, per_split;
 };
 
+// Expected us of a plan of stride 2 (fitted over 96 layers): 3.6 for an iteration of either group, 0.06 for an image written and summed
+double expected_us(const WoPlan &p) {
+  const long wgs = long(p.tiles) * p.splits, cus = sgh_num_cus();
+  return 6 + double((wgs + cus - 1) / cus) * ((p.per_split + 1) / 2) * 3.6 + 0.06 * double(wgs);
+}
+
 size_t image_bytes(const WoPlan &p) { return size_t(p.splits) * p.tiles * 4 * kAcc * sizeof(float); }
 
 // `room`: bytes for the partial images
@@ -499,17 +505,13 @@ WoPlan plan(const sgh_conv_geom *g, size_t room) {
   // Stride 2, more than a quarter as many tiles and strips as CUs: one to three splits of them leave up to half of the CUs idle in their only or
   // last round.  Up to three rounds of shorter workgroups do not, if there is room for their images: 35 images, 654 channels of 31 x 36 to 344,
   // 132 workgroups 1017 us, 660 of them 661 (k_wgrad3x3 766); 7 of 811, 73 x 70, to 488 980 -> 751 (the generic kernel 887); 4 of 299, 88 x 107,
-  // to 417 344 -> 258.  (us, fitted over 96 layers: 3.6 for an iteration of either group, 0.06 for an image written and summed.)
+  // to 417 344 -> 258.
   if (p.st == 2 && one < 4) {
-    auto us = [&] {
-      const long wgs = tiles * p.splits;
-      return double((wgs + cus - 1) / cus) * ((p.per_split + 1) / 2) * 3.6 + 0.06 * double(wgs);
-    };
     WoPlan best = p;
-    double least = us();
+    double least = expected_us(p);
     for (long sp = one + 1; sp * tiles * p.strips <= 3l * cus && sp <= most; ++sp) {
       split(sp);
-      if (us() < least && image_bytes(p) <= room) least = us(), best = p;
+      if (const double us = expected_us(p); us < least && image_bytes(p) <= room) least = us, best = p;
     }
     p = best;
   }
@@ -537,6 +539,8 @@ size_t sgh_wgrad_oct_workspace_bytes(const sgh_conv_geom *g, bool least) {
   const WoPlan p = plan(g, least ? 0 : size_t(-1));
   return p.ok && !sgh_env().conv_split_off ? image_bytes(p) : 0;
 }
+
+double sgh_wgrad_oct_us(const sgh_conv_geom *g) { return expected_us(plan(g, size_t(-1))); }
 
 int sgh_wgrad_oct_run(const sgh_conv_geom *g, const float *dy, const float *x, float *dW, void *workspace, size_t ws_bytes,
                       hipStream_t s) {

@@ -162,6 +162,29 @@ answer([run(g, lib.sgh_conv_workspace_bytes(C.byref(g), which)) + (lib.sgh_conv_
     assert less is None and few == [True, 256], (less, few)
 
 
+def test_which_kernels_take_strided_layers():
+    """3x3 gradients of stride 2 that the fp32 kernels do in less time stay there: data gradients of few, short tiles with odd rows, weight
+    gradients whose octets or tiles are half empty.  (n, c, h, w, k): measured on both."""
+    fp32_dgrad = [(2, 360, 14, 17, 14), (7, 69, 12, 9, 9), (30, 252, 17, 13, 56), (12, 477, 12, 13, 71)]
+    split_dgrad = [(6, 59, 10, 13, 11), (2, 717, 46, 43, 9), (2, 263, 55, 42, 8), (2, 593, 8, 7, 51), (64, 64, 56, 56, 128)]
+    fp32_wgrad = [(98, 84, 16, 17, 380), (90, 731, 8, 7, 904), (69, 42, 89, 67, 116)]
+    split_wgrad = [(35, 654, 31, 36, 344), (7, 811, 73, 70, 488), (122, 319, 20, 15, 356), (64, 256, 14, 14, 512)]
+    got = recorded("""
+def names(which, layers):
+    out = []
+    for n, c, h, w, k in layers:
+        g = conv(n, c, h, w, k, 3, 3, 2, 2, 1, 1)
+        need = lib.sgh_conv_workspace_bytes(C.byref(g), which)
+        fn = (None, lib.sgh_conv_dgrad_f32, lib.sgh_conv_wgrad_f32)[which]
+        assert fn(C.byref(g), SPACE, 2 * SPACE, 3 * SPACE, 4 * SPACE, need, None) == 0
+        out.append(kernels())
+    return out
+answer([names(1, %r), names(1, %r), names(2, %r), names(2, %r)])
+""" % (fp32_dgrad, split_dgrad, fp32_wgrad, split_wgrad))
+    assert not any("k_dgrad_split2" in k for k in got[0]) and all("k_dgrad_split2" in k for k in got[1]), got[:2]
+    assert not any("k_wgrad_oct" in k for k in got[2]) and all("k_wgrad_oct" in k for k in got[3]), got[2:]
+
+
 def test_wavefronts_of_data_gradients_onto_few_channels():
     """Eight where a workgroup has its CU to itself, or nearly, and filters for them; four where the chip is full."""
     got = recorded("""
