@@ -112,23 +112,33 @@ class HipOps(object):
     # its bias gradient; softmax with its loss
     fuse_linear = True
 
-    # (a network's input or a layer's weights may be a transposed view: the products take it as it lies, the fused calls do not)
+    # (a network's input or a layer's weights may be a transposed view: the products take it as it lies, the fused calls refuse it.  Asking
+    # the tensors first took 0.3 of the 47.5 us of an MLP's step)
     def linear_fwd(self, x, W, b, relu):
-        if x.transpose() or W.transpose():
-            y = self.add_bias(self.matmul(x, W), b)
-            return self.relu(y) if relu else y
-        return singa.LinearForward(x, W, b, relu)
+        try:
+            return singa.LinearForward(x, W, b, relu)
+        except singa.SingaHipError:
+            if not (x.transpose() or W.transpose()):
+                raise
+        y = self.add_bias(self.matmul(x, W), b)
+        return self.relu(y) if relu else y
 
     def linear_bwd_x(self, dy, W, gate):
-        if W.transpose():
-            dx = singa.Mult(dy, singa.DefaultTranspose(W))
-            return dx if gate is None else self.relu_bwd(dx, gate)
-        return singa.LinearBackwardx(dy, W, gate)
+        try:
+            return singa.LinearBackwardx(dy, W, gate)
+        except singa.SingaHipError:
+            if not W.transpose():
+                raise
+        dx = singa.Mult(dy, singa.DefaultTranspose(W))
+        return dx if gate is None else self.relu_bwd(dx, gate)
 
     def linear_bwd_wb(self, dy, x, W, b):
-        if x.transpose() or W.transpose():
-            return singa.Mult(singa.DefaultTranspose(x), dy), self.sum0(dy)
-        return singa.LinearBackwardWb(dy, x, W, b)
+        try:
+            return singa.LinearBackwardWb(dy, x, W, b)
+        except singa.SingaHipError:
+            if not (x.transpose() or W.transpose()):
+                raise
+        return singa.Mult(singa.DefaultTranspose(x), dy), self.sum0(dy)
 
     def softmax_ce_fwd(self, x, t):
         return singa.SoftMaxCrossEntropyFwd(x, t)
