@@ -150,8 +150,9 @@ int sgh_dgrad_few_run(const sgh_conv_geom *g, const float *dy, const float *W, f
   // Eight wavefronts halve the chain of a workgroup that has its CU to itself, or shares it with one or two: us in columns / on four / eight, 5x5,
   // 2 x 4 x 16 x 13 to 64 (bfloat16) 27.5 / 34.5 / 25.6, 5 x 4 x 21 x 21 to 61 21.1 / 23.9 / 19.4, 16 x 4 x 17 x 17 to 63 30.3 / 35.2 / 27.4; with
   // four, 73 of 500 layers of 40 to 64 filters were slower than in columns.  Beyond, the vector ALUs are busy either way (15 x 4 x 57 x 78, 3x3 to
-  // 10 5.9 / 6.7, 13 x 3 x 96 x 112 to 44 16.3 / 17.6).
-  const bool eight = (wgs <= cus && g->K > 8) || (wgs <= (g->R == 5 ? 3 : 2) * cus && g->K > 24);
+  // 10 5.9 / 6.7, 13 x 3 x 96 x 112 to 44 16.3 / 17.6), and beside another stream's kernels four leave those more room (the small CNN's step, 512
+  // workgroups, 32 filters: alone 16.2 / 15.3, the step 278.6 / 280.2).
+  const bool eight = (wgs <= cus && g->K > 8) || (wgs <= (g->R == 5 ? 3 : 2) * cus && g->K > 32);
 #define SGH_FEW_KERNEL(C_, R_)                                                             \
   do {                                                                                     \
     if (eight) SGH_LAUNCH_TIMED((k_dgrad_few<C_, R_, 8>), grid, dim3(512), 0, s, a);       \
