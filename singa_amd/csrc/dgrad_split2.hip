@@ -381,12 +381,6 @@ S2Plan plan(const sgh_conv_geom *g) {
   // (two or three chunks, few tiles: their sums cost what the split saves.  31 channels onto 5 x 131 of 9 x 11 15.6 us on fp32
   // instructions, 18.0 here; 38 onto 2 x 407 of 8 x 9 17.9 / 18.5; 35 onto 3 x 506 of 46 x 62, 136 tiles, 40 / 23)
   if ((p.nchunks == 2 || p.nchunks == 3) && 2 * tiles < cus) return p;
-  // (rows of an odd number of results go out in single floats, which costs few and short tiles more than they save.  One chunk: 14 onto
-  // 2 x 360 of 14 x 17 11.8 / 18.1, 9 onto 7 x 69 of 12 x 9 11.6 / 14.2, but 11 onto 6 x 59 of 10 x 13 16.5 / 14.8, 9 onto 2 x 717 of 46 x 43,
-  // 96 tiles, 18.6 / 16.6; in even rows 8 onto 2 x 263 of 55 x 42 15.9 / 13.6.  Four or five: 56 onto 30 x 252 of 17 x 13 25.1 / 36.0, 71 onto
-  // 12 x 477 of 12 x 13 23.5 / 28.8, but 51 onto 2 x 593 of 8 x 7, five tiles, 19.7 / 18.3)
-  if (g->W % 2 && p.nchunks == 1 && g->C > 64 && 5 * tiles < cus) return p;
-  if (g->W % 2 && (p.nchunks == 4 || p.nchunks == 5) && g->C > 128 && tiles >= 16 && 2 * tiles < cus) return p;
   p.tiles = int(tiles);
   p.dp_tiles = int(tiles / cus * cus);
   const int rest = p.tiles - p.dp_tiles;
