@@ -25,6 +25,7 @@
 // Neither the taps of a class nor their signs change within a chunk, so the one that the matrix instructions' rounding needs (it
 // leans towards minus infinity) changes from chunk to chunk: in odd ones dy goes negated into the slab and the sums are subtracted.
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
 #include "dgrad_split2.h"
@@ -32,6 +33,7 @@
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
 constexpr int NT = 512, NW = NT / 64, KC = 16, TAPS = 9;
 constexpr int kOOB = int(0x80000000u);
@@ -58,29 +60,28 @@ struct S2Args {
   // Workgroups [0, dp_tiles) take one whole tile each; workgroup dp_tiles + r * share + i takes part i of the chunks of tile
   // dp_tiles + r.
   int ctiles, dp_tiles, share;
-  unsigned dy_bytes, wt_bytes;
+  unsigned dy_bytes, wt_bytes, dx_bytes;
 };
 
-// The 2 x 2 results of pixel (p, q); `o` is the plane of dx.  Images of odd height or width have no last odd row or column.
+// The 2 x 2 results of pixel (p, q) for the second pass; `o` is the plane of dx.  Images of odd height or width have no last odd row or
+// column.
 __device__ __forceinline__ void put(const S2Args &a, float *o, int p, int q, float r00, float r01, float r10, float r11) {
+  typedef v2f pair __attribute__((aligned(4)));
   o += size_t(2 * p) * a.Wd + 2 * q;
   const bool below = 2 * p + 1 < a.H;
-  if (!(a.Wd & 1)) {
+  if (2 * q + 1 < a.Wd) {
     v2f r0{r00, r01}, r1{r10, r11};
-    v2f *const o0 = reinterpret_cast<v2f *>(o), *const o1 = reinterpret_cast<v2f *>(o + a.Wd);
+    pair *const o0 = reinterpret_cast<pair *>(o), *const o1 = reinterpret_cast<pair *>(o + a.Wd);
     if (a.accumulate) {
       r0 += *o0;
       if (below) r1 += *o1;
     }
     *o0 = r0;
     if (below) *o1 = r1;
-    return;
+  } else {
+    o[0] = a.accumulate ? o[0] + r00 : r00;
+    if (below) o[a.Wd] = a.accumulate ? o[a.Wd] + r10 : r10;
   }
-  const bool beside = 2 * q + 1 < a.Wd;
-  o[0] = a.accumulate ? o[0] + r00 : r00;
-  if (beside) o[1] = a.accumulate ? o[1] + r01 : r01;
-  if (below) o[a.Wd] = a.accumulate ? o[a.Wd] + r10 : r10;
-  if (below && beside) o[a.Wd + 1] = a.accumulate ? o[a.Wd + 1] + r11 : r11;
 }
 
 // GM x (NW / GM) wavefronts, each on 32 channels x 32 pixels of all four classes; ET: slab elements (octet, position) per thread
@@ -300,14 +301,63 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   asm volatile("" : "+v"(tt));
   const int row0 = wm * 32 + (tt >> 3 & 4), col = wn * 32 + (tt & 31);
   if (whole) {
+    // A lane's places in the plane of its first channel, those that do not exist out of range; the other channels are scalar offsets away.
+    // Results go out in pairs of a row, at any element's address: what a CU's stores cost is their number (rows of an odd number in single
+    // floats: 14 filters onto 2 x 360 of 14 x 17 15.0 us, so 9.6, as of 14 x 18).  The last column of such a row goes
+    // out with its left neighbour's result, which is the neighbouring lane's and is stored there as well.
     int n, p, q;
     pixel(col, n, p, q);
-    if (pix0 + col >= a.total_pix) return;
+    const rsrc_t rdx = make_rsrc(a.dx, a.dx_bytes);
+    const int plane = a.H * a.Wd * 4, at = int((unsigned(n * a.C + c0 + row0) * a.H * a.Wd + 2 * p * a.Wd + 2 * q) * 4u);
+    const bool there = pix0 + col < a.total_pix, below = 2 * p + 1 < a.H, beside = 2 * q + 1 < a.Wd, alone = !beside && (q == 0 || (tt & 31) == 0);
+    const int first = there && !alone ? (beside ? at : at - 4) : kOOB, second = there && !alone && below ? first + a.Wd * 4 : kOOB;
+    const int left = a.C - c0 - row0;   // channels from this lane's first one on
+    auto out = [&](auto acc_c, auto odd_c) {
+      constexpr bool ACC = decltype(acc_c)::value, ODD = decltype(odd_c)::value;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int c = c0 + row0 + 8 * (v >> 2) + (v & 3);
-      if (c < a.C) put(a, a.dx + (size_t(n) * a.C + c) * a.H * a.Wd, p, q, acc[0][v], acc[1][v], acc[2][v], acc[3][v]);
-    }
+      for (int v0 = 0; v0 < 16; v0 += 4) {
+        v2f r[4][2];
+        // (the sum in the fixed order result, then what is there; all of it is requested before the first sum is stored)
+        if constexpr (ACC)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+              r[v][k] = __builtin_bit_cast(
+                  v2f, __builtin_amdgcn_raw_buffer_load_b64(rdx, 2 * v0 + v < left ? (k ? second : first) : kOOB, (2 * v0 + v) * plane, 0));
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            v2f w{acc[2 * k][v0 + v], acc[2 * k + 1][v0 + v]};
+            if constexpr (ODD) {
+              const float own = w[1];   // (a cast of the vector's element itself would take its first)
+              constexpr int WAVE_SHR1 = 0x138;
+              const float l = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, own), WAVE_SHR1, 0xf, 0xf, true));
+              w = beside ? w : v2f{l, w[0]};
+            }
+            if constexpr (ACC) w += r[v][k];
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, w), rdx, 2 * v0 + v < left ? (k ? second : first) : kOOB,
+                                                  (2 * v0 + v) * plane, 0);
+          }
+      }
+      if constexpr (ODD)
+        if (__any(alone && there)) {   // (the tile begins with the last column, or it is the only one)
+          const int single = alone && there ? at : kOOB, under = alone && there && below ? at + a.Wd * 4 : kOOB;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              const int rel = 8 * (v >> 2) + (v & 3), off = rel < left ? (k ? under : single) : kOOB;
+              float w = acc[2 * k][v];
+              if constexpr (ACC) w += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdx, off, rel * plane, 0));
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, w), rdx, off, rel * plane, 0);
+            }
+        }
+    };
+    const bool odd = a.Wd & 1;
+    if (a.accumulate) odd ? out(std::true_type{}, std::true_type{}) : out(std::true_type{}, std::false_type{});
+    else odd ? out(std::false_type{}, std::true_type{}) : out(std::false_type{}, std::false_type{});
     return;
   }
   const rsrc_t rslot = make_rsrc(a.partials + size_t(rest) * (4 * BM * BN), 4 * BM * BN * 4);
@@ -430,6 +480,7 @@ int sgh_dgrad_split2_run(const sgh_conv_geom *g, const float *dy, const float *W
   a.cblocks = p.cblocks, a.pitch = p.pitch, a.slab = p.slab, a.total_pix = g->N * g->P * g->Q, a.nchunks = p.nchunks;
   a.ctiles = p.ctiles, a.dp_tiles = p.dp_tiles, a.share = p.share;
   a.dy_bytes = unsigned(size_t(g->N) * g->K * g->P * g->Q * 4), a.wt_bytes = unsigned(weight_bytes(p));
+  a.dx_bytes = unsigned(size_t(g->N) * g->C * g->H * g->W * 4);
   int rc = SGH_EUNSUPPORTED;
   sgh_prof_kernel_begin("conv_dgrad/k_dgrad_split2", 2.0 * g->N * g->K * g->P * g->Q * g->C * TAPS);
 #define S2_CASE(GM_, ET_) \

@@ -131,7 +131,8 @@ def test_conv_split_forward_of_stride_two(singa, dev, n, c, h, w, k, kind):
 
 @pytest.mark.parametrize("kind", ["normal", "relu", "positive"])
 @pytest.mark.parametrize("n,c,h,w,k", [(4, 64, 14, 14, 64), (2, 128, 9, 11, 130), (70, 33, 7, 8, 8), (1, 100, 58, 120, 72), (1, 100, 6, 256, 72),
-                                       (1, 64, 8, 219, 64), (44, 64, 56, 56, 48), (300, 200, 5, 3, 16)])
+                                       (1, 64, 8, 219, 64), (44, 64, 56, 56, 48), (300, 200, 5, 3, 16), (40, 70, 9, 1, 16), (41, 64, 11, 5, 130),
+                                       (7, 300, 9, 13, 8)])   # (odd rows: single columns, tiles that begin with the last one)
 def test_data_gradient_of_stride_two_on_split_operands(singa, dev, n, c, h, w, k, kind):
     """3x3 data gradients of stride 2 and padding 1: odd and even planes, tiles over many images, either tile, whole and shared, every
     slab, against float64 and no further off than the fp32 chain; onto a gradient that is there already, the sum of the two; an infinity
