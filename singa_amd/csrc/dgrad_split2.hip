@@ -316,6 +316,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       constexpr bool ACC = decltype(acc_c)::value, ODD = decltype(odd_c)::value;
 #pragma unroll
       for (int v0 = 0; v0 < 16; v0 += 4) {
+        if (2 * v0 >= a.C - c0 - wm * 32) break;   // (rows without a channel, of the whole wavefront)
         v2f r[4][2];
         // (the sum in the fixed order result, then what is there; all of it is requested before the first sum is stored)
         if constexpr (ACC)
